@@ -296,7 +296,7 @@ def instrument(clock: KernelClock, cfg):
     costs = {"embed_bigram_norm": io, "add_scalar_norm": io, "scalar_norm": io, "polynorm": io, "gate_heads": io,
              "token_shift": io, "wkv_decay": io, "wkv_recurrence": wkv, "rotary_interleaved": io, "latent_kv_store": io,
              "latent_attention": latent, "moe_route": io, "moe_align": io, "moe_grouped_gemm": grouped, "moe_glu": io,
-             "moe_combine": io, "rmsnorm": io, "fused_add_rmsnorm": io, "silu_and_mul": io, "rotary_embedding": io,
+             "moe_grouped_glu": grouped, "moe_combine": io, "rmsnorm": io, "fused_add_rmsnorm": io, "silu_and_mul": io, "rotary_embedding": io,
              "extend_attention": llama_extend, "decode_attention": llama_extend, "linear": gemm,
              "embed_scale": embed, "norm_shift": io, "stream_add": io, "qkv_rotary_store": io, "pool_blocks": io,
              "window_attention": window, "small_linear_f32": small, "causal_conv_silu": io, "mamba2_scan": scan,

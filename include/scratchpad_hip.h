@@ -490,6 +490,13 @@ SP_API int sp_moe_align(int32_t* offsets, int32_t* order, int32_t* place, const 
 SP_API int sp_moe_grouped_gemm(void* out, const void* a, const void* w, const int32_t* offsets, const int32_t* order,
                                int row_div, int pairs, int n, int k, int experts, int64_t a_stride, int64_t out_stride,
                                int act, int dtype, void* stream);
+/* the gated form: w [experts, 2 ff, k] holds each expert's gate rows, then its up rows, and out [pairs, ff] is the activation of
+ * the two sums, each rounded to `dtype` first: act 0 = sp_silu_and_mul's, 1 = sp_moe_glu's (limit, alpha) - bit for bit the
+ * plain product followed by that call.  SP_ERR_UNSUPPORTED (nothing is launched) for fp32, k no multiple of 32, or rows of a
+ * that are not 16-byte aligned.                                                                                         */
+SP_API int sp_moe_grouped_glu(void* out, const void* a, const void* w, const int32_t* offsets, const int32_t* order,
+                              int row_div, int pairs, int ff, int k, int experts, int64_t a_stride, int64_t out_stride,
+                              int act, float limit, float alpha, int dtype, void* stream);
 /* out[p, f] = g * sigmoid(alpha g) * (u + 1), g = min(gu[p, f], limit), u = clamp(gu[p, ff + f], -limit, limit) */
 SP_API int sp_moe_glu(void* out, const void* gu, int64_t pairs, int ff, float limit, float alpha, int dtype, void* stream);
 /* out[t] = sum over k < top, in that order, of weights[t, k] * z[place[t * top + k]] */

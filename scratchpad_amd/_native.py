@@ -123,6 +123,7 @@ SIGNATURES = {
     "sp_moe_route": (_i32, [_vp, _vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _vp]),
     "sp_moe_align": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _vp]),
     "sp_moe_grouped_gemm": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i64, _i64, _i32, _i32, _vp]),
+    "sp_moe_grouped_glu": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i64, _i64, _i32, _f32, _f32, _i32, _vp]),
     "sp_moe_glu": (_i32, [_vp, _vp, _i64, _i32, _f32, _f32, _i32, _vp]),
     "sp_moe_combine": (_i32, [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i64, _i32, _vp]),
     # ---- ABI 11
@@ -1301,6 +1302,24 @@ def moe_grouped_gemm(a: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, pa
     _check(load().sp_moe_grouped_gemm(out.data_ptr(), a.data_ptr(), w.data_ptr(), offsets.data_ptr(), _ptr(order), row_div,
                                       pairs, N, K, E, a.stride(0), out.stride(0), {"none": 0, "relu2": 1}[act], _dt(a), _stream()),
            "sp_moe_grouped_gemm")
+    return out
+
+
+def moe_grouped_glu(a: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, pairs: int, order: Optional[torch.Tensor],
+                    row_div: int, act: str, limit: float = 0.0, alpha: float = 0.0) -> Optional[torch.Tensor]:
+    """out [pairs, ff]: ``moe_grouped_gemm`` with w [E, 2 ff, K] and its gated activation in one launch, bit for bit the two
+    calls; act "silu" (silu_and_mul) or "clamped" (moe_glu).  None: not a form of the fused kernel (fp32, rows that are not
+    16-byte aligned, K no multiple of 32) - the caller runs the two steps."""
+    _mat(a, "a")
+    if w.dim() != 3 or not w.is_contiguous() or w.dtype != a.dtype or w.shape[2] != a.shape[1] or w.shape[1] % 2:
+        raise RuntimeError("moe_grouped_glu: w [E, 2 ff, K] contiguous of a's dtype")
+    E, n, K = w.shape
+    if a.dtype == torch.float32 or K % 32 or a.stride(0) % 8 or a.data_ptr() % 16 or w.data_ptr() % 16:
+        return None
+    out = torch.empty((pairs, n // 2), dtype=a.dtype, device=a.device)
+    _check(load().sp_moe_grouped_glu(out.data_ptr(), a.data_ptr(), w.data_ptr(), offsets.data_ptr(), _ptr(order), row_div, pairs,
+                                     n // 2, K, E, a.stride(0), out.stride(0), {"silu": 0, "clamped": 1}[act], limit, alpha,
+                                     _dt(a), _stream()), "sp_moe_grouped_glu")
     return out
 
 

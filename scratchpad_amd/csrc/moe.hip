@@ -5,6 +5,8 @@
 // a fixed order, so a token's result does not depend on which other tokens share the step.
 #include "seq_batch.h"
 
+#include <type_traits>
+
 namespace sp {
 namespace {
 
@@ -256,12 +258,14 @@ moe_grouped_gemm_kernel(void* out, const void* a, const void* w, const int32_t* 
 }
 
 // ---- the same product on the matrix cores (16-bit types, K a multiple of 32, 16-byte aligned rows) -------------------
-// Tiles of 128 rows x 64 columns, 4 waves of 32 x 64 each: per k-step of 32 a wave loads 2 row fragments and 4 weight
-// fragments (16 bytes per lane, straight from global memory: the 4 waves of a workgroup share the weight fragments
-// through the cache) and issues 8 MFMAs.  v_mfma_f32_16x16x32: lane (r16 = lane & 15, q = lane >> 4) holds 8 k-values of
-// row r16 of each operand and receives D[4 q + r][r16], r < 4 - with the weights as the first operand a lane ends up
-// with 4 neighbouring output columns of ONE row.  A wave whose 32 rows lie past the expert's rows leaves at once, so a
-// decode step (a few rows per expert) streams every chosen expert's weights once and does little else.
+// v_mfma_f32_16x16x32: lane (r16 = lane & 15, q = lane >> 4) holds 8 k-values of row r16 of each operand and receives
+// D[4 q + r][r16], r < 4 - with the weights as the first operand a lane ends up with 4 neighbouring output columns of ONE
+// row.  Both kernels below add the k-steps of 32 in ascending order into one accumulator, so an output element has the same
+// bits whichever of them - and whichever tile height - computes it: a token's result does not depend on the step's size.
+//
+// ACT: 0 the product, 1 max(., 0)^2 of the fp32 sum; 2 and 3 take w [E, 2 N, K] (gate rows, then up rows), keep the two sums
+// of an output column in one lane and store the activation of the ROUNDED sums - bit for bit the plain product followed by
+// sp_silu_and_mul (2) or sp_moe_glu (3), without the [P, 2 N] round trip and the launch.
 typedef float f32x4_q __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_q __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_q __attribute__((ext_vector_type(8)));
@@ -276,73 +280,298 @@ __device__ __forceinline__ f32x4_q mfma_q<f16_tag>(const u32x4& a, const u32x4& 
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_q, a), __builtin_bit_cast(f16x8_q, b), c, 0, 0, 0);
 }
 
-constexpr int QM = 128, QN = 64;
+struct GroupedArgs {
+  char* out;
+  const char* a;
+  const char* w;
+  const int32_t* offsets;
+  const int32_t* order;
+  int row_div, N, K, E;              // N: output columns
+  int64_t a_stride, out_stride;      // elements
+  int vec_out;                       // 8-byte stores of 4 columns are aligned and inside a row
+  float limit, alpha;                // ACT 3
+};
+
+// a * b rounded to fp32 before anything else happens to it: a product that is then rounded to fp16 would otherwise become one
+// v_fma_mixlo_f16, which rounds once - in one kernel and perhaps not in the next
+__device__ __forceinline__ float mul_f32(float a, float b) {
+  float r = a * b;
+  asm("" : "+v"(r));
+  return r;
+}
+
+// (shared by the separate launch and the fused epilogue, which agree bit for bit)
+__device__ __forceinline__ float moe_glu_f32(float g, float u, float limit, float alpha) {
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  return mul_f32(g / (1.f + expf(-alpha * g)), u + 1.f);
+}
+
+template <typename Tag, int ACT>
+__device__ __forceinline__ float grouped_act(float v, float up, const GroupedArgs& p) {
+  typedef Elem<Tag> El;
+  if constexpr (ACT == 1) return gemm_act(v, 1);
+  if constexpr (ACT == 2) return mul_f32(El::round(silu_ref(El::round(v))), El::round(up));
+  if constexpr (ACT == 3) return moe_glu_f32(El::round(v), El::round(up), p.limit, p.alpha);
+  return v;
+}
 
 template <typename Tag>
-__global__ void __launch_bounds__(256)
-moe_grouped_mfma_kernel(void* out, const void* a, const void* w, const int32_t* offsets, const int32_t* order, int row_div,
-                        int N, int K, int E, int64_t a_stride, int64_t out_stride, int act) {
+__device__ __forceinline__ void store4(const GroupedArgs& p, int64_t pos, int n, const float* v) {
   typedef Elem<Tag> El;
-  int tile = blockIdx.x, e = 0, row0 = 0, rows_end = 0;
-  for (; e < E; ++e) {
-    const int lo = offsets[e], hi = offsets[e + 1];
-    const int tiles = (hi - lo + QM - 1) / QM;
-    if (tile < tiles) {
-      row0 = lo + tile * QM;
-      rows_end = hi;
-      break;
+  if (p.vec_out && n + 4 <= p.N) {
+    const float f[8] = {v[0], v[1], v[2], v[3], 0.f, 0.f, 0.f, 0.f};
+    const u32x4 w = pack16<Tag>(f);
+    *(u32x2*)(p.out + (pos * p.out_stride + n) * 2) = u32x2{w[0], w[1]};
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (n + r < p.N) El::store(p.out, pos * p.out_stride + n + r, v[r]);
+}
+
+// Row tiles of `bm` rows, expert after expert (a tile never spans two): the expert, first row and end of tile `tile`, found by
+// a wave with one load per lane and a scan (E <= 64: one round).  False past the last tile.  `total`: all tiles, if asked for.
+__device__ __forceinline__ int wave_inclusive(int v, int lane) {
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int o = __shfl_up(v, off, 64);
+    if (lane >= off) v += o;
+  }
+  return v;
+}
+__device__ __forceinline__ int grouped_tiles(const int32_t* offsets, int E, int bm, int lane) {
+  int run = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane;
+    int v = e < E ? (offsets[e + 1] - offsets[e] + bm - 1) / bm : 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    run += v;
+  }
+  return run;
+}
+__device__ __forceinline__ bool grouped_tile(const int32_t* offsets, int E, int bm, int tile, int lane, int& e_out, int& row0,
+                                             int& rows_end) {
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane;
+    const int lo = e < E ? offsets[e] : 0, hi = e < E ? offsets[e + 1] : 0;
+    const int tiles = (hi - lo + bm - 1) / bm, incl = wave_inclusive(tiles, lane);
+    const uint64_t hit = __ballot(tile < incl);
+    if (hit) {
+      const int l = __ffsll((unsigned long long)hit) - 1;
+      e_out = e0 + l;
+      row0 = __builtin_amdgcn_readfirstlane(__shfl(lo, l, 64) + (tile - __shfl(incl - tiles, l, 64)) * bm);
+      rows_end = __builtin_amdgcn_readfirstlane(__shfl(hi, l, 64));
+      return true;
     }
-    tile -= tiles;
+    tile -= __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
   }
-  if (e >= E) return;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
-  if (row0 + 32 * wave >= rows_end) return;                       // (no workgroup barrier in this kernel)
-  const int n0 = blockIdx.y * QN;
-  const char* xp[2];
-  bool xv[2];
+  return false;
+}
+
+// Steps with many rows per expert: BM rows x 128 weight rows per workgroup, k in steps of 64.  Both operands go to LDS by
+// direct loads (16 bytes per lane, no registers on the way), one step ahead of the MFMAs, in two buffers; a step costs one
+// barrier.  LDS rows are 128 bytes whose eight 16-byte chunks are permuted by the row's number (the SOURCE address is
+// permuted: a direct load writes lane after lane), so the 16 rows of a fragment read meet no bank twice in a phase.
+// Four waves: BM 128 as 2 x 2 of 64 x 64, smaller tiles as 1 x 4 of BM x 32.  The tiles of a row block lie next to each
+// other in one XCD's share of the grid (block b runs on XCD b mod 8), so an XCD's L2 sees each row of `a` once.
+constexpr int kGroupedBN = 128, kGroupedBK = 64;
+
+template <typename Tag, int BM, int ACT>
+__global__ void __launch_bounds__(256, 2) moe_grouped_tile_kernel(GroupedArgs p) {
+  constexpr bool GLU = ACT >= 2;
+  constexpr int WN = BM == 128 ? 2 : 4, CPW = kGroupedBN / WN, FM = (BM == 128 ? 64 : BM) / 16, FN = CPW / 16;
+  constexpr int OUT_N = GLU ? kGroupedBN / 2 : kGroupedBN;
+  constexpr int LA = BM / 32, LB = kGroupedBN / 32;              // direct loads per wave and step
+  constexpr int kBuf = (BM + kGroupedBN) * 128;
+  __shared__ __attribute__((aligned(16))) char lds0[kBuf];
+  __shared__ __attribute__((aligned(16))) char lds1[kBuf];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+  const int ntiles = (p.N + OUT_N - 1) / OUT_N;
+  const int total = grouped_tiles(p.offsets, p.E, BM, lane) * ntiles, share = (total + 7) / 8;
+  const int idx = (int)(blockIdx.x >> 3), at = (int)(blockIdx.x & 7) * share + idx;
+  if (idx >= share || at >= total) return;
+  int e = 0, row0 = 0, rows_end = 0;
+  if (!grouped_tile(p.offsets, p.E, BM, at / ntiles, lane, e, row0, rows_end)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  const int n0 = (at % ntiles) * OUT_N;
+  const int wm = wave / WN, wn = wave % WN;
+  const int wrows = GLU ? 2 * p.N : p.N;
+  // sources of this wave's direct loads: lane -> row lane / 8 of the 8 rows of a load, chunk lane % 8 of LDS
+  const int chunk = (lane & 7) ^ (lane >> 3);
+  const char* src[LA + LB];
 #pragma unroll
-  for (int f = 0; f < 2; ++f) {
-    const int pos = row0 + 32 * wave + 16 * f + r16;
-    xv[f] = pos < rows_end;
-    const int64_t arow = xv[f] ? (order ? order[pos] / row_div : pos) : 0;
-    xp[f] = (const char*)a + (arow * a_stride + 8 * q) * 2;
+  for (int i = 0; i < LA; ++i) {
+    const int pos = min(row0 + (wave * LA + i) * 8 + (lane >> 3), rows_end - 1);      // rows past the end: never stored
+    const int64_t arow = p.order ? p.order[pos] / p.row_div : pos;
+    src[i] = p.a + arow * p.a_stride * 2 + chunk * 16;
   }
-  const char* wbase = (const char*)w + (int64_t)e * N * K * 2;
-  const char* wp[4];
+  const char* wbase = p.w + (int64_t)e * wrows * p.K * 2 + chunk * 16;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int n = min(n0 + 16 * j + r16, N - 1);                  // columns past N are computed and never stored
-    wp[j] = wbase + ((int64_t)n * K + 8 * q) * 2;
+  for (int i = 0; i < LB; ++i) {
+    const int br = (wave * LB + i) * 8 + (lane >> 3);
+    int row;
+    if constexpr (GLU) {
+      const int in = br % CPW, col = n0 + (br / CPW) * (CPW / 2) + in % (CPW / 2);
+      row = min(col, p.N - 1) + (in >= CPW / 2 ? p.N : 0);
+    } else {
+      row = min(n0 + br, p.N - 1);
+    }
+    src[LA + i] = wbase + (int64_t)row * p.K * 2;
   }
-  f32x4_q acc[2][4];
+  const auto stage = [&](char* lds, int k0) {
+    // the last step of a K that is no multiple of 64: chunks past the row's end are read from its start and never used
+    const int back = k0 + chunk * 8 >= p.K ? chunk * 16 : -k0 * 2;
 #pragma unroll
-  for (int f = 0; f < 2; ++f)
+    for (int i = 0; i < LA + LB; ++i) {
+      char* dst = lds + (i < LA ? (wave * LA + i) : (BM / 8 + wave * LB + i - LA)) * 1024;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] - back),
+                                       (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    }
+  };
+  f32x4_q acc[FM][FN];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[f][j] = f32x4_q{0.f, 0.f, 0.f, 0.f};
-  const u32x4 zero = {0u, 0u, 0u, 0u};
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    u32x4 xf[2], wf[4];
+  for (int f = 0; f < FM; ++f)
 #pragma unroll
-    for (int f = 0; f < 2; ++f) xf[f] = xv[f] ? ld16(xp[f] + (int64_t)k0 * 2) : zero;
+    for (int j = 0; j < FN; ++j) acc[f][j] = f32x4_q{0.f, 0.f, 0.f, 0.f};
+  const int arow0 = (wm * (BM == 128 ? 64 : 0) + r16) * 128, brow0 = (BM + wn * CPW + r16) * 128;
+  const auto compute = [&](const char* lds, auto halves) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) wf[j] = ld16(wp[j] + (int64_t)k0 * 2);
+    for (int kk = 0; kk < decltype(halves)::value; ++kk) {
+      const int c = ((kk * 4 + q) ^ (r16 & 7)) * 16;
+      u32x4 xf[FM], wf[FN];
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+      for (int f = 0; f < FM; ++f) xf[f] = ld16(lds + arow0 + f * 2048 + c);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[f][j] = mfma_q<Tag>(wf[j], xf[f], acc[f][j]);
+      for (int j = 0; j < FN; ++j) wf[j] = ld16(lds + brow0 + j * 2048 + c);
+#pragma unroll
+      for (int f = 0; f < FM; ++f)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[f][j] = mfma_q<Tag>(wf[j], xf[f], acc[f][j]);
+    }
+  };
+  const auto ready = [&]() {           // this wave's loads have landed, then everyone's; the other buffer is free
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+  const std::integral_constant<int, 2> whole;
+  const int full = p.K & ~(kGroupedBK - 1);
+  int k0 = 0;
+  stage(lds0, 0);
+  for (; k0 + 2 * kGroupedBK <= full; k0 += 2 * kGroupedBK) {
+    ready();
+    stage(lds1, k0 + kGroupedBK);
+    compute(lds0, whole);
+    ready();
+    if (k0 + 2 * kGroupedBK < p.K) stage(lds0, k0 + 2 * kGroupedBK);
+    compute(lds1, whole);
   }
+  const std::integral_constant<int, 1> half;
+  if (k0 < full) {                     // one more whole step, then perhaps half a one
+    ready();
+    if (full < p.K) stage(lds1, full);
+    compute(lds0, whole);
+    if (full < p.K) {
+      ready();
+      compute(lds1, half);
+    }
+  } else if (full < p.K) {
+    ready();
+    compute(lds0, half);
+  }
+  constexpr int FO = GLU ? FN / 2 : FN;
 #pragma unroll
-  for (int f = 0; f < 2; ++f) {
-    const int pos = row0 + 32 * wave + 16 * f + r16;
+  for (int f = 0; f < FM; ++f) {
+    const int pos = row0 + wm * (BM == 128 ? 64 : 0) + 16 * f + r16;
     if (pos >= rows_end) continue;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < FO; ++j) {
+      float v[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = n0 + 16 * j + 4 * q + r;
-        if (n < N) El::store(out, (int64_t)pos * out_stride + n, gemm_act(acc[f][j][r], act));
-      }
+      for (int r = 0; r < 4; ++r) v[r] = grouped_act<Tag, ACT>(acc[f][j][r], GLU ? acc[f][j + FN - FO][r] : 0.f, p);
+      store4<Tag>(p, pos, n0 + wn * (GLU ? CPW / 2 : CPW) + 16 * j + 4 * q, v);
+    }
   }
+}
+
+// Steps with a few rows per expert (decode): a stream of the chosen experts' weights.  One wave per 16 rows x 32 weight rows
+// (GLU: 16 gate rows and their 16 up rows), operands straight from global memory, kRowsUnroll k-steps of loads in flight.
+// Single waves spread evenly over the 1024 SIMDs whatever the number of chosen experts; nothing is shared between them.
+constexpr int kRowsUnroll = 8;
+
+template <typename Tag, int ACT>
+__global__ void __launch_bounds__(64) moe_grouped_rows_kernel(GroupedArgs p) {
+  constexpr bool GLU = ACT >= 2;
+  const int lane = threadIdx.x, r16 = lane & 15, q = lane >> 4;
+  int e = 0, row0 = 0, rows_end = 0;
+  if (!grouped_tile(p.offsets, p.E, 16, (int)blockIdx.y, lane, e, row0, rows_end)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  const int n0 = blockIdx.x * (GLU ? 16 : 32);
+  const int pos = min(row0 + r16, rows_end - 1);                 // rows past the end: never stored
+  const int64_t arow = p.order ? p.order[pos] / p.row_div : pos;
+  const char* xp = p.a + (arow * p.a_stride + 8 * q) * 2;
+  const char* wbase = p.w + ((int64_t)e * (GLU ? 2 * p.N : p.N) * p.K + 8 * q) * 2;
+  const char* wp[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    wp[j] = wbase + (int64_t)(GLU ? j * p.N + min(n0 + r16, p.N - 1) : min(n0 + 16 * j + r16, p.N - 1)) * p.K * 2;
+  f32x4_q acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  const int ksteps = p.K / 32;
+  int ks = 0;
+  for (; ks + kRowsUnroll <= ksteps; ks += kRowsUnroll) {
+    u32x4 wf[kRowsUnroll][2], xf[kRowsUnroll];
+#pragma unroll
+    for (int u = 0; u < kRowsUnroll; ++u) {
+      wf[u][0] = ld16(wp[0] + (ks + u) * 64);
+      wf[u][1] = ld16(wp[1] + (ks + u) * 64);
+      xf[u] = ld16(xp + (ks + u) * 64);
+    }
+    __builtin_amdgcn_sched_barrier(0);      // all loads of the round first: the scheduler would trade them for registers
+#pragma unroll
+    for (int u = 0; u < kRowsUnroll; ++u) {
+      acc[0] = mfma_q<Tag>(wf[u][0], xf[u], acc[0]);
+      acc[1] = mfma_q<Tag>(wf[u][1], xf[u], acc[1]);
+    }
+  }
+  for (; ks < ksteps; ++ks) {
+    const u32x4 xf = ld16(xp + ks * 64);
+    acc[0] = mfma_q<Tag>(ld16(wp[0] + ks * 64), xf, acc[0]);
+    acc[1] = mfma_q<Tag>(ld16(wp[1] + ks * 64), xf, acc[1]);
+  }
+  if (row0 + r16 >= rows_end) return;
+#pragma unroll
+  for (int j = 0; j < (GLU ? 1 : 2); ++j) {
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = grouped_act<Tag, ACT>(acc[j][r], acc[1][r], p);
+    store4<Tag>(p, row0 + r16, n0 + 16 * j + 4 * q, v);
+  }
+}
+
+// Which kernel: by the mean rows per expert, pairs / experts (the counts themselves are on the device).  Measured at width 2048,
+// 32 experts of ff 1024, top 4, up + down product in us (rows kernel | 64-row tiles | 128-row tiles):
+//   mean rows 1: 60 | 68 | 73     4: 85 | 92 | 94     8: 86 | 92 | 94     16: 104 | 93 | 96     32: 161 | 95 | 99
+//   64: 286 | 103 | 103     96: 410 | 138 | 107     128: 537 | 150 | 157     512: 2038 | 379 | 337
+// (the kernel these replaced, one operand fragment per load and no LDS: 75 at mean 1, 1398 at mean 512)
+template <typename Tag, int ACT>
+int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
+  const int held = pairs < p.E ? pairs : p.E;                    // experts with a row, at most
+  if (pairs <= 10 * (int64_t)p.E) {
+    const int tiles = pairs / 16 + held, per = ACT >= 2 ? 16 : 32;
+    if (tiles > 65535) return SP_ERR_UNSUPPORTED;                // (4096 experts, the most moe_align takes: 6656)
+    moe_grouped_rows_kernel<Tag, ACT><<<dim3((unsigned)((p.N + per - 1) / per), (unsigned)tiles), 64, 0, st>>>(p);
+    SP_LAUNCH_CHECK();
+    return SP_OK;
+  }
+  const int per = ACT >= 2 ? kGroupedBN / 2 : kGroupedBN;
+  const int64_t ntiles = (p.N + per - 1) / per;
+  const int bm = pairs > 56 * (int64_t)p.E ? 128 : 64;
+  const unsigned blocks = (unsigned)(((pairs / bm + held) * ntiles + 7) / 8 * 8);
+  if (bm == 128) moe_grouped_tile_kernel<Tag, 128, ACT><<<dim3(blocks), 256, 0, st>>>(p);
+  else moe_grouped_tile_kernel<Tag, 64, ACT><<<dim3(blocks), 256, 0, st>>>(p);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
 }
 
 // ---- y = g' * sigmoid(alpha g') * (u' + 1), g' = min(g, limit), u' = clamp(u, -limit, limit); gu = [g | u] per row -----
@@ -353,23 +582,60 @@ __global__ void moe_glu_kernel(void* out, const void* gu, int64_t P, int F, floa
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t p = i / F;
     const int f = (int)(i % F);
-    const float g = fminf(El::load(gu, p * 2 * F + f), limit);
-    const float u = fminf(fmaxf(El::load(gu, p * 2 * F + F + f), -limit), limit);
-    El::store(out, i, g / (1.f + expf(-alpha * g)) * (u + 1.f));
+    El::store(out, i, moe_glu_f32(El::load(gu, p * 2 * F + f), El::load(gu, p * 2 * F + F + f), limit, alpha));
   }
 }
 
 // ---- out[t] = sum_k weights[t, k] * z[place[t * top + k]] ----------------------------------------------------------
-template <typename Tag>
-__global__ void moe_combine_kernel(void* out, const void* z, const int32_t* place, const float* weights, int width,
-                                   int top, int64_t out_stride) {
+// A thread holds V neighbouring columns of a token (V = 16 bytes where the rows allow it, else 1): the rows of up to
+// kCombineAhead experts are in flight together, added in the order of k.
+constexpr int kCombineAhead = 4;
+
+template <typename Tag, int V>
+__global__ void __launch_bounds__(kBlock)
+moe_combine_kernel(void* out, const void* z, const int32_t* place, const float* weights, int width, int top,
+                   int64_t out_stride) {
   typedef Elem<Tag> El;
   const int64_t t = blockIdx.x;
-  for (int i = threadIdx.x; i < width; i += blockDim.x) {
-    float acc = 0.f;
-    for (int k = 0; k < top; ++k) acc += weights[t * top + k] * El::load(z, (int64_t)place[t * top + k] * width + i);
-    El::store(out, t * out_stride + i, acc);
+  const int i = (blockIdx.y * kBlock + threadIdx.x) * V;
+  if (i >= width) return;
+  float acc[V];
+#pragma unroll
+  for (int c = 0; c < V; ++c) acc[c] = 0.f;
+  for (int k0 = 0; k0 < top; k0 += kCombineAhead) {
+    const int n = min(top - k0, kCombineAhead);
+    float zv[kCombineAhead][V], w[kCombineAhead];
+#pragma unroll
+    for (int k = 0; k < kCombineAhead; ++k) {
+      const int64_t at = t * top + k0 + min(k, n - 1);
+      w[k] = weights[at];
+      const int64_t row = (int64_t)place[at] * width + i;
+      if constexpr (V == 1) zv[k][0] = El::load(z, row);
+      else unpack16<Tag>(ld16((const char*)z + row * El::kBytes), zv[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < kCombineAhead; ++k)
+      if (k < n) {
+#pragma unroll
+        for (int c = 0; c < V; ++c) acc[c] += w[k] * zv[k][c];
+      }
   }
+  if constexpr (V == 1) El::store(out, t * out_stride + i, acc[0]);
+  else st16((char*)out + (t * out_stride + i) * El::kBytes, pack16<Tag>(acc));
+}
+
+template <typename Tag>
+int launch_combine(void* out, const void* z, const int32_t* place, const float* weights, int64_t T, int width, int top,
+                   int64_t out_stride, hipStream_t st) {
+  constexpr int V = Elem<Tag>::kVec;
+  if (width % V == 0 && out_stride % V == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)z & 15) == 0)
+    moe_combine_kernel<Tag, V><<<dim3((unsigned)T, (unsigned)((width / V + kBlock - 1) / kBlock)), kBlock, 0, st>>>(
+        out, z, place, weights, width, top, out_stride);
+  else
+    moe_combine_kernel<Tag, 1><<<dim3((unsigned)T, (unsigned)((width + kBlock - 1) / kBlock)), kBlock, 0, st>>>(
+        out, z, place, weights, width, top, out_stride);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
 }
 
 }  // namespace
@@ -427,21 +693,34 @@ extern "C" int sp_moe_grouped_gemm(void* out, const void* a, const void* w, cons
   SP_CHECK_ARG(out && a && w && offsets && a_stride >= k && out_stride >= n);
   const bool aligned = k % 32 == 0 && a_stride % 8 == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0;
   if ((dtype == SP_BF16 || dtype == SP_F16) && aligned) {
-    const dim3 grid((unsigned)((pairs + QM - 1) / QM + experts), (unsigned)((n + QN - 1) / QN));
+    const GroupedArgs p{(char*)out, (const char*)a, (const char*)w, offsets, order, row_div, n, k, experts, a_stride, out_stride,
+                        out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0, 0.f, 0.f};
+    hipStream_t st = (hipStream_t)stream;
     if (dtype == SP_BF16)
-      moe_grouped_mfma_kernel<bf16_tag><<<grid, 256, 0, (hipStream_t)stream>>>(out, a, w, offsets, order, row_div, n, k,
-                                                                                experts, a_stride, out_stride, act);
-    else
-      moe_grouped_mfma_kernel<f16_tag><<<grid, 256, 0, (hipStream_t)stream>>>(out, a, w, offsets, order, row_div, n, k,
-                                                                               experts, a_stride, out_stride, act);
-    SP_LAUNCH_CHECK();
-    return SP_OK;
+      return act ? launch_grouped_mfma<bf16_tag, 1>(p, pairs, st) : launch_grouped_mfma<bf16_tag, 0>(p, pairs, st);
+    return act ? launch_grouped_mfma<f16_tag, 1>(p, pairs, st) : launch_grouped_mfma<f16_tag, 0>(p, pairs, st);
   }
   const dim3 grid((unsigned)((pairs + GM - 1) / GM + experts), (unsigned)((n + GN - 1) / GN));
   SP_DISPATCH_DTYPE(dtype, (moe_grouped_gemm_kernel<Tag><<<grid, 256, 0, (hipStream_t)stream>>>(
                                out, a, w, offsets, order, row_div, pairs, n, k, experts, a_stride, out_stride, act)));
   SP_LAUNCH_CHECK();
   return SP_OK;
+}
+
+extern "C" int sp_moe_grouped_glu(void* out, const void* a, const void* w, const int32_t* offsets, const int32_t* order,
+                                  int row_div, int pairs, int ff, int k, int experts, int64_t a_stride, int64_t out_stride,
+                                  int act, float limit, float alpha, int dtype, void* stream) {
+  SP_CHECK_ARG(pairs >= 0 && ff > 0 && k > 0 && experts > 0 && row_div >= 1 && (act == 0 || act == 1));
+  if (pairs == 0) return SP_OK;
+  SP_CHECK_ARG(out && a && w && offsets && a_stride >= k && out_stride >= ff);
+  if (dtype != SP_BF16 && dtype != SP_F16) return SP_ERR_UNSUPPORTED;
+  if (k % 32 || a_stride % 8 || ((uintptr_t)a & 15) || ((uintptr_t)w & 15)) return SP_ERR_UNSUPPORTED;
+  const GroupedArgs p{(char*)out, (const char*)a, (const char*)w, offsets, order, row_div, ff, k, experts, a_stride, out_stride,
+                      out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0, limit, alpha};
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == SP_BF16)
+    return act ? launch_grouped_mfma<bf16_tag, 3>(p, pairs, st) : launch_grouped_mfma<bf16_tag, 2>(p, pairs, st);
+  return act ? launch_grouped_mfma<f16_tag, 3>(p, pairs, st) : launch_grouped_mfma<f16_tag, 2>(p, pairs, st);
 }
 
 extern "C" int sp_moe_glu(void* out, const void* gu, int64_t pairs, int ff, float limit, float alpha, int dtype,
@@ -462,8 +741,6 @@ extern "C" int sp_moe_combine(void* out, const void* z, const int32_t* place, co
   SP_CHECK_ARG(num_tokens >= 0 && width > 0 && top > 0);
   if (num_tokens == 0) return SP_OK;
   SP_CHECK_ARG(out && z && place && weights && out_stride >= width);
-  SP_DISPATCH_DTYPE(dtype, (moe_combine_kernel<Tag><<<dim3((unsigned)num_tokens), kBlock, 0, (hipStream_t)stream>>>(
-                               out, z, place, weights, width, top, out_stride)));
-  SP_LAUNCH_CHECK();
-  return SP_OK;
+  SP_DISPATCH_DTYPE(dtype, return (launch_combine<Tag>(out, z, place, weights, num_tokens, width, top, out_stride,
+                                                       (hipStream_t)stream)));
 }

@@ -41,8 +41,12 @@ class ClampedGluExperts(nn.Module):
         top = ids.shape[1]
         pairs = ids.numel()
         offsets, order, place = _native.moe_align(ids, self.experts)
-        gu = _native.moe_grouped_gemm(x, self.gate_up.data, offsets, pairs, order, top)
-        y = self.activation(gu)
+        act = _FUSED.get(type(self).activation)          # (a subclass with an activation of its own runs it as a step)
+        y = None
+        if act is not None:
+            y = _native.moe_grouped_glu(x, self.gate_up.data, offsets, pairs, order, top, act, self.limit, self.alpha)
+        if y is None:
+            y = self.activation(_native.moe_grouped_gemm(x, self.gate_up.data, offsets, pairs, order, top))
         z = _native.moe_grouped_gemm(y, self.down.data, offsets, pairs)
         return _native.moe_combine(z, place, weights)
 
@@ -94,6 +98,10 @@ class SiluGluExperts(ClampedGluExperts):
 
     def activation(self, gu: torch.Tensor) -> torch.Tensor:
         return _native.silu_and_mul(gu)
+
+
+# activations that the first grouped product can apply in its own launch
+_FUSED = {ClampedGluExperts.activation: "clamped", SiluGluExperts.activation: "silu"}
 
 
 class SoftmaxMoE(nn.Module):

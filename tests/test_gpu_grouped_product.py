@@ -1,0 +1,83 @@
+"""The grouped expert products on the matrix cores at the edges of their tiles (rows per expert around 16, 64 and 128, columns
+and k that end inside a tile, experts without rows, more experts than lanes), against the product in fp32 by torch, and the
+gated form bit for bit against the product followed by its activation."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def grouped_inputs(counts, N, K, dtype, top, seed=0):
+    """rows sorted by expert with the given counts; order holds pairs (token * top + k) in a shuffled order"""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    E, P = len(counts), sum(counts)
+    tokens = (P + top - 1) // top
+    a = torch.randn(tokens, K, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(E, N, K, generator=g, device=DEV) * K ** -0.5).to(dtype)
+    offsets = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device=DEV)
+    order = torch.randperm(tokens * top, generator=g, device=DEV)[:P].to(torch.int32)
+    expert = torch.repeat_interleave(torch.arange(E, device=DEV), torch.tensor(counts, device=DEV))
+    return a, w, offsets, order, expert, P
+
+
+COUNTS = [[1], [0, 3, 0, 17], [16, 0, 15, 33], [63, 64, 65, 1], [127, 128, 129, 257, 0], [300, 2, 140], [3] * 70, [90] * 67 + [0, 1]]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts", COUNTS, ids=lambda c: "-".join(map(str, c[:5])))
+@pytest.mark.parametrize("N,K", [(64, 32), (130, 96), (200, 256)])
+def test_grouped_products(counts, N, K, dtype):
+    from scratchpad_amd import _native
+    top = 3
+    print("grouped", counts[:6], len(counts), N, K, dtype, flush=True)
+    a, w, offsets, order, expert, P = grouped_inputs(counts, N, K, dtype, top)
+    # one rounding of the result plus fp32 sums: half an ulp of the 16-bit type, and K fp32 additions
+    bar = (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) + K * 2.0 ** -23
+    rows = a[(order // top).long()].float()
+    want = torch.cat([rows[expert == e] @ w[e].float().t() for e in range(len(counts))])
+    scale = rows.abs().max() * w.float().abs().sum(-1).max()
+    for got, ref in ((_native.moe_grouped_gemm(a, w, offsets, P, order, top), want),
+                     (_native.moe_grouped_gemm(a, w, offsets, P, order, top, act="relu2"), torch.relu(want) ** 2)):
+        assert ((got.float() - ref).abs() <= 2 * bar * ref.abs() + K * 2.0 ** -22 * scale).all()
+    plain = _native.moe_grouped_gemm(rows.to(dtype), w, offsets, P)
+    assert torch.equal(plain, _native.moe_grouped_gemm(a, w, offsets, P, order, top))
+    # an output row has the same bits whichever tile height computes it: alone, its expert takes the few-rows kernel
+    for e in [e for e, c in enumerate(counts) if c][:3]:
+        at = int(offsets[e])
+        one = torch.zeros_like(offsets)
+        one[e + 1:] = 1
+        assert torch.equal(_native.moe_grouped_gemm(rows[at:at + 1].to(dtype), w, one, 1)[0], plain[at])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts", COUNTS, ids=lambda c: "-".join(map(str, c[:5])))
+@pytest.mark.parametrize("ff,K", [(32, 32), (67, 96), (136, 128)])
+def test_gated_form_is_the_two_steps(counts, ff, K, dtype):
+    from scratchpad_amd import _native
+    a, w, offsets, order, _, P = grouped_inputs(counts, 2 * ff, K, dtype, 2, seed=1)
+    print("gated", counts[:6], ff, K, dtype, flush=True)
+    a = a * 3                                                     # beyond the clamp too
+    gu = _native.moe_grouped_gemm(a, w, offsets, P, order, 2)
+    assert torch.equal(_native.moe_grouped_glu(a, w, offsets, P, order, 2, "silu"), _native.silu_and_mul(gu))
+    assert torch.equal(_native.moe_grouped_glu(a, w, offsets, P, order, 2, "clamped", 2.0, 1.702), _native.moe_glu(gu, 2.0, 1.702))
+
+
+def test_gated_form_leaves_other_shapes_to_the_two_steps():
+    from scratchpad_amd import _native
+    for dtype, K in ((torch.float32, 64), (torch.bfloat16, 40)):
+        a, w, offsets, order, _, P = grouped_inputs([2, 5], 16, K, dtype, 2)
+        assert _native.moe_grouped_glu(a, w, offsets, P, order, 2, "silu") is None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,width,top", [(1, 8, 1), (5, 264, 4), (3, 2056, 6), (9, 37, 5)])
+def test_combine(T, width, top, dtype):
+    from scratchpad_amd import _native
+    g = torch.Generator(device=DEV).manual_seed(2)
+    z = torch.randn(T * top, width, generator=g, device=DEV).to(dtype)
+    place = torch.randperm(T * top, generator=g, device=DEV).to(torch.int32).view(T, top)
+    wt = torch.rand(T, top, generator=g, device=DEV)
+    want = (z.float()[place.long()] * wt[..., None]).sum(1)
+    bar = 2.0 ** -8 if dtype == torch.bfloat16 else top * 2.0 ** -23
+    assert ((_native.moe_combine(z, place.view(-1), wt).float() - want).abs() <= bar * want.abs() + 1e-5).all()
