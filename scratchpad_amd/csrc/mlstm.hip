@@ -8,7 +8,7 @@
 // S, n and m start at ZERO for a sequence (m too: not minus infinity).  One workgroup per (request, head): a column of S
 // lives in the registers of 1, 2 or 4 neighbouring lanes and n is one more column, so a token costs no workgroup barrier
 // and no sum over a wave; tokens are staged through LDS in passes and the per-head norm and gate run as the pass's epilogue.
-#include "seq_batch.h"
+#include "chunk_scan.h"
 
 namespace sp {
 namespace {
@@ -149,12 +149,218 @@ mlstm_scan_kernel(void* out, int64_t out_stride, const void* q, int64_t q_stride
   if (j == 0) mst[0] = m;
 }
 
+// ---- steps of several tokens per request, bf16 rows: 64 tokens at a time (chunk_scan.h) -------------------------------------
+// With F the running sum of the log forget gates inside the chunk, b_s = i_s - F_s and G_t = max(m_0, max_{s <= t} b_s), the
+// running maximum is m_t = F_t + G_t and the weight of token s at t is exp(b_s - G_t) <= 1, that of the old state
+// exp(m_0 - G_t).  The normaliser n . q is a row sum of the weighted tiles plus n_0 . q.
+// One workgroup of Dv / 16 waves per (request, head).  The per-token form is a chain of one token's exponentials, sums and
+// lane exchanges (1.6 us per token: 1546 us at 3001 tokens of 5 requests, 16 heads of 128 x 128); this one takes 140 us there
+// and 568 us for one request of 4096 tokens, 8.9 us per chunk: about 1500 vector instructions per wave at two waves per SIMD
+// (the splits, the weights' exponentials, the epilogue) against 126 MFMAs and 0.5 MB of LDS reads.
+template <int D, int NW>
+struct MlstmLds {
+  typedef ChunkScan<D, NW> C;
+  static constexpr int kN = (C::kBytes + 15) / 16 * 16, kNq = kN + D * 4, kFloor = kNq + kCL * 4, kRed = kFloor + 2 * kCL * 4;
+  static constexpr int kGates = (kRed + NW * kCL * 4 + 7) / 8 * 8;             // double [NW][3][kCL]: F, b and its running maximum of NW chunks
+  static constexpr int kBytes = kGates + NW * 3 * kCL * 8;
+};
+
+template <int D, int NW>
+__global__ void __launch_bounds__(NW * 64)
+mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_stride, const char* k, int64_t k_stride, const char* v,
+                   int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre, const float* norm_w,
+                   float* S_state, int64_t S_stride, float* n_state, int64_t n_stride, float* m_state, int64_t m_stride,
+                   SeqBatch s, int H, float cap, float eps) {
+  typedef Elem<bf16_tag> E;
+  typedef ChunkScan<D, NW> C;
+  typedef MlstmLds<D, NW> L;
+  constexpr int Dv = C::Dv, NT = C::NT;
+  extern __shared__ __attribute__((aligned(16))) char chunk_lds[];
+  const int b = blockIdx.x, h = blockIdx.y;
+  int64_t start, len, prefix;
+  seq_span(s, b, start, len, prefix);
+  if (len <= 0) return;
+  C c(chunk_lds);
+  float* sn = (float*)(chunk_lds + L::kN);
+  float* snq = (float*)(chunk_lds + L::kNq);
+  float* sfloor = (float*)(chunk_lds + L::kFloor);
+  float* red = (float*)(chunk_lds + L::kRed);
+  double* sgate = (double*)(chunk_lds + L::kGates);
+  const bool held = prefix > 0;
+  start = uniform64(start), len = uniform64(len);
+  const int64_t slot = uniform64(load_idx(s.req_pool_indices, b, s.idx64));
+  float* Sst = S_state + slot * S_stride + (int64_t)h * D * Dv;
+  float* nst = n_state + slot * n_stride + (int64_t)h * D;
+  float* mst = m_state + slot * m_stride + h;
+  c.load_state(Sst, held);
+  if (c.tid < D) sn[c.tid] = held ? nst[c.tid] : 0.f;
+  float m = held ? mst[0] : 0.f;                      // (kept by the wave that forms the scalars)
+  const float qscale = 1.f / sqrtf((float)D);
+  q += (start * q_stride + (int64_t)h * D) * 2;
+  k += (start * k_stride + (int64_t)h * D) * 2;
+  v += (start * v_stride + (int64_t)h * Dv) * 2;
+  const char* gb = (const char*)g + (start * g_stride + (int64_t)h * Dv) * 2;
+  char* ob = (char*)out + (start * out_stride + (int64_t)h * Dv) * 2;
+  const int col = c.column();
+  const float nw = norm_w[(int64_t)h * Dv + col];
+  const auto load = [&](int64_t c0) {
+    const int n = (int)(len - c0 < kCL ? len - c0 : kCL);
+    c.load(q + c0 * q_stride * 2, q_stride * 2, k + c0 * k_stride * 2, k_stride * 2, v + c0 * v_stride * 2, v_stride * 2, n);
+  };
+  // F, b and the running maximum of b do not depend on m: the NW waves form those of NW chunks at a time (two scans and five
+  // transcendentals of latency), and a chunk's scalars are a few exponentials more once the chunk before it has fixed m
+  const auto scan_gates = [&](int64_t c0) {
+    const int64_t t = c0 + c.tid;
+    double* to = sgate + c.wave * 3 * kCL + c.lane;
+    const bool live = t < len;
+    const float gi = live ? ipre[(start + t) * H + h] : 0.f, gf = live ? fpre[(start + t) * H + h] : 0.f;
+    const double F = wave_scan_sum(live ? (double)logsigmoid_f(cap * tanhf(gf / cap)) : 0., c.lane);
+    const double bs = live ? (double)(cap * tanhf(gi / cap)) - F : -INFINITY;
+    to[0] = F;
+    to[kCL] = bs;
+    to[2 * kCL] = wave_scan_max(bs, c.lane);
+  };
+  const auto gates = [&](int64_t c0) {                // by the last wave: its share of the tiles is the smallest
+    if (c.wave != NW - 1) return;
+    const double* from = sgate + c0 / kCL % NW * 3 * kCL + c.lane;
+    const double F = from[0], bs = from[kCL], G = fmax((double)m, from[2 * kCL]);
+    const double Gend = __shfl(G, 63, 64), Fend = __shfl(F, 63, 64);
+    ChunkScalars& sc = *c.scalars(c0 / kCL);
+    sc.lt[c.lane] = (float)(Gend - G);                // (relative to the chunk's end: small where the weights are not)
+    sc.ls[c.lane] = (float)(Gend - bs);
+    sc.cs[c.lane] = qscale;
+    sc.a0[c.lane] = expf((float)(m - G)) * qscale;
+    sc.w[c.lane] = expf((float)(bs - Gend));
+    sfloor[(c0 / kCL & 1) * kCL + c.lane] = expf((float)-(F + G));
+    if (c.lane == 0) sc.a_end = expf((float)(m - Gend));
+    m = (float)(Fend + Gend);
+  };
+  load(0);
+  bool zero = !held;
+  for (int64_t c0 = 0; c0 < len; c0 += kCL) {
+    const int n = (int)(len - c0 < kCL ? len - c0 : kCL);
+    c.sc = c.scalars(c0 / kCL);
+    if (c0 / kCL % NW == 0) {
+      scan_gates(c0);
+      __syncthreads();
+      gates(c0);
+    }
+    c.stage();
+    __syncthreads();
+    if (c0 + kCL < len) load(c0 + kCL);
+    c.scores();
+    c.from_state(zero);
+    zero = false;
+    {      // n_0 . q of a token: the lanes of a token share its D channels
+      constexpr int PER = NT / kCL, DP = D / PER;
+      const int t = c.tid / PER, part = c.tid % PER;
+      float d = 0.f;
+#pragma unroll
+      for (int i = 0; i < DP; i += 8) {
+        float f[8];
+        unpack16<bf16_tag>(ld16(chunk_lds + C::kQ + t * C::QROW + (part * DP + i) * 2), f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d += sn[part * DP + i + e] * f[e];
+      }
+      d = lanes_sum<PER>(d);
+      if (part == 0) snq[t] = d;
+    }
+    uint16_t gv[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = 16 * i + 4 * c.q + r;
+        gv[i][r] = *(const uint16_t*)(gb + c0 * g_stride * 2 + (uint32_t)((t < n ? t : n - 1) * (uint32_t)g_stride + col) * 2u);
+      }
+    __syncthreads();
+    c.template weigh<true>();
+    if (c0 + kCL < len && (c0 / kCL + 1) % NW != 0) gates(c0 + kCL);
+    {      // the normaliser's update: the lanes of a channel share the chunk's tokens
+      constexpr int PER = NT / D, TP = kCL / PER;
+      const int d = c.tid / PER, part = c.tid % PER;
+      const ChunkScalars& sc = *c.sc;
+      float x = 0.f;
+#pragma unroll
+      for (int i = 0; i < TP; i += 8) {
+        float f[8];
+        unpack16<bf16_tag>(ld16(chunk_lds + C::kKT + d * C::TROW + (part * TP + i) * 2), f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x += sc.w[part * TP + i + e] * f[e];
+      }
+      x = lanes_sum<PER>(x);
+      if (part == 0) sn[d] = sc.a_end * sn[d] + x;
+    }
+    __syncthreads();
+    c.absorb();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float ss = lanes_sum<16>(c.o[i][r] * c.o[i][r]);
+        if (c.r16 == 0) red[c.wave * kCL + 16 * i + 4 * c.q + r] = ss;
+      }
+    __syncthreads();
+    // lane t of every wave: the division by the normaliser and the RMS of the divided row as one factor
+    float nq = snq[c.lane] * c.sc->a0[c.lane], ss = 0.f;
+    for (int j = 0; j <= c.q; ++j) nq += c.sums()[j * kCL + c.lane];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) ss += red[w * kCL + c.lane];
+    const float den = 1.f / (fmaxf(fabsf(nq), sfloor[(c0 / kCL & 1) * kCL + c.lane]) + 1e-6f);
+    const float factor = den / sqrtf(den * den * ss / (float)Dv + eps);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = 16 * i + 4 * c.q + r;
+        const float gate = bf16_bits_to_f32(gv[i][r]), f = __shfl(factor, t, 64);
+        // (the result is rounded to 16 bits: the hardware's exponential and reciprocal, 1 ulp each, are far below that)
+        if (t < n)
+          E::store(ob + c0 * out_stride * 2 + (uint32_t)(t * (uint32_t)out_stride + col) * 2u, 0,
+                   c.o[i][r] * f * nw * __builtin_amdgcn_rcpf(1.f + __expf(-gate)));
+      }
+  }
+  c.store_state(Sst);
+  if (c.tid < D) nst[c.tid] = sn[c.tid];
+  if (c.tid == (NW - 1) * 64) mst[0] = m;
+}
+
+template <int D, int NW>
+static int launch_mlstm_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                               const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
+                               const float* fpre, const float* norm_w, float* S_state, int64_t S_stride, float* n_state,
+                               int64_t n_stride, float* m_state, int64_t m_stride, const SeqBatch& s, int H, float cap, float eps,
+                               hipStream_t st) {
+  constexpr int bytes = MlstmLds<D, NW>::kBytes;
+  static PerDevice<int> raised;
+  if (!chunk_lds_ready(raised, (const void*)mlstm_chunk_kernel<D, NW>, bytes)) return SP_ERR_LAUNCH;
+  mlstm_chunk_kernel<D, NW><<<dim3((unsigned)s.B, (unsigned)H), NW * 64, bytes, st>>>(
+      out, out_stride, (const char*)q, q_stride, (const char*)k, k_stride, (const char*)v, v_stride, g, g_stride, ipre, fpre,
+      norm_w, S_state, S_stride, n_state, n_stride, m_state, m_stride, s, H, cap, eps);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
+
 template <typename Tag>
 static int launch_mlstm(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
                         const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre,
                         const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride,
                         float* m_state, int64_t m_stride, const SeqBatch& s, int H, int D, int Dv, float cap, float eps,
                         hipStream_t st) {
+  // a step of one token per request stays with the per-token form (one sweep over the state is all there is to do), and so do
+  // the types and head sizes the matrix form is not built for
+  if (std::is_same<Tag, bf16_tag>::value && s.extend_seq_lens && (D == 64 || D == 128) && (Dv == 64 || Dv == 128) &&
+      chunk_aligned(q, q_stride) && chunk_aligned(k, k_stride) && chunk_aligned(v, v_stride) &&
+      g_stride < ((int64_t)1 << 24) && out_stride < ((int64_t)1 << 24)) {
+#define SP_MLSTM_CHUNKS(D_, NW_)                                                                                              \
+  return launch_mlstm_chunks<D_, NW_>(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, norm_w, \
+                                      S_state, S_stride, n_state, n_stride, m_state, m_stride, s, H, cap, eps, st)
+    if (D == 128 && Dv == 128) SP_MLSTM_CHUNKS(128, 8);
+    if (D == 128) SP_MLSTM_CHUNKS(128, 4);
+    if (Dv == 128) SP_MLSTM_CHUNKS(64, 8);
+    SP_MLSTM_CHUNKS(64, 4);
+#undef SP_MLSTM_CHUNKS
+  }
   const dim3 grid((unsigned)s.B, (unsigned)H);
   if ((Dv + 1) * (D > 64 ? 4 : (D > 32 ? 2 : 1)) > 1024) return SP_ERR_UNSUPPORTED;      // vdim 256 with dim > 64
 #define SP_MLSTM(DP)                                                                                                    \
