@@ -130,6 +130,9 @@ SP_API int sp_write_req_to_token(int32_t* req_to_token, int64_t row_stride,
 SP_API int sp_compute_position(int64_t* positions, int32_t* extend_start_loc,
                         const int32_t* extend_prefix_lens, const int32_t* extend_seq_lens,
                         int batch_size, void* stream);
+/* token_req[t] = the request that owns row t of the step: extend_start_loc is the requests' first rows, ascending from 0 */
+SP_API int sp_token_requests(int32_t* token_req, const int32_t* extend_start_loc, int batch_size, int64_t num_tokens,
+                      void* stream);
 SP_API int sp_clamp_position(int64_t* positions, const void* seq_lens, int idx64, int batch_size,
                       void* stream);
 

@@ -66,6 +66,7 @@ SIGNATURES = {
                            _i64, _i32, _vp]),
     "sp_write_req_to_token": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _i32, _vp]),
     "sp_compute_position": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp]),
+    "sp_token_requests": (_i32, [_vp, _vp, _i32, _i64, _vp]),
     "sp_clamp_position": (_i32, [_vp, _vp, _i32, _i32, _vp]),
     "sp_decode_plan_slots": (_i64, [_i32, _i64, _i64, _i32]),
     "sp_decode_attention_workspace_bytes": (_sz, [_i64, _i32, _i32]),
@@ -998,6 +999,17 @@ def linear_relu_square(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 
 # --------------------------------------------------------------------------- per-sequence state, latent attention, experts
+def token_requests(extend_start_loc: torch.Tensor, num_tokens: int) -> torch.Tensor:
+    """int32 [num_tokens]: the request that owns each token row of a step (extend_start_loc int32: the requests' first rows)"""
+    _gpu(extend_start_loc)
+    if extend_start_loc.dtype != torch.int32 or extend_start_loc.dim() != 1 or not extend_start_loc.is_contiguous():
+        raise RuntimeError("extend_start_loc must be a contiguous int32 vector")
+    out = torch.empty(num_tokens, dtype=torch.int32, device=extend_start_loc.device)
+    _check(load().sp_token_requests(out.data_ptr(), extend_start_loc.data_ptr(), extend_start_loc.shape[0], num_tokens, _stream()),
+           "sp_token_requests")
+    return out
+
+
 class SeqParams:
     """The header's SP_SEQ_PARAMS of one step, built once per forward (``from_forward_batch``) and handed to every kernel
     that reads or writes per-request state.  Holds the tensors, so the pointers stay valid while it lives."""
@@ -1027,9 +1039,7 @@ class SeqParams:
     def from_forward_batch(cls, fb) -> "SeqParams":
         if fb.forward_mode.is_decode():
             return cls(fb.req_pool_indices, fb.seq_lens)
-        bs = fb.batch_size
-        token_req = torch.repeat_interleave(torch.arange(bs, dtype=torch.int32, device=fb.extend_seq_lens.device),
-                                            fb.extend_seq_lens.long(), output_size=fb.extend_num_tokens)
+        token_req = token_requests(fb.extend_start_loc, fb.extend_num_tokens)
         return cls(fb.req_pool_indices, fb.seq_lens, fb.extend_seq_lens, fb.extend_prefix_lens, fb.extend_start_loc,
                    token_req)
 

@@ -455,6 +455,21 @@ __global__ __launch_bounds__(kBlock) void compute_position_kernel(
   if (threadIdx.x == 0) extend_start_loc[b] = (int32_t)start;
 }
 
+// the request of every token row: a binary search in the requests' first rows, a thread per row (torch's repeat_interleave took
+// five launches, 22 us of a prompt step whatever its size)
+__global__ void token_request_kernel(int32_t* __restrict__ token_req, const int32_t* __restrict__ start_loc, int batch,
+                                     int64_t tokens) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= tokens) return;
+  int lo = 0, hi = batch - 1;                 // the last request that starts at or before t (one without rows never is: the
+  while (lo < hi) {                           // next one starts where it does, or it starts behind every row)
+    const int mid = (lo + hi + 1) >> 1;
+    if (start_loc[mid] <= t) lo = mid;
+    else hi = mid - 1;
+  }
+  token_req[t] = lo;
+}
+
 // model_executor/forward_info.py:469-471
 __global__ void clamp_position_kernel(int64_t* __restrict__ positions,
                                       const void* __restrict__ seq_lens, int idx64, int n) {
@@ -698,6 +713,17 @@ extern "C" int sp_compute_position(int64_t* positions, int32_t* extend_start_loc
   if (batch_size == 0) return SP_OK;
   compute_position_kernel<<<dim3(batch_size), kBlock, 0, (hipStream_t)stream>>>(
       positions, extend_start_loc, extend_prefix_lens, extend_seq_lens);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
+
+extern "C" int sp_token_requests(int32_t* token_req, const int32_t* extend_start_loc, int batch_size, int64_t num_tokens,
+                                 void* stream) {
+  SP_CHECK_ARG(batch_size >= 0 && num_tokens >= 0 && (num_tokens == 0 || batch_size > 0));
+  if (num_tokens == 0) return SP_OK;
+  SP_CHECK_ARG(token_req && extend_start_loc);
+  token_request_kernel<<<dim3((unsigned)((num_tokens + 255) / 256)), 256, 0, (hipStream_t)stream>>>(
+      token_req, extend_start_loc, batch_size, num_tokens);
   SP_LAUNCH_CHECK();
   return SP_OK;
 }

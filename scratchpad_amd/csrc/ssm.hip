@@ -92,7 +92,8 @@ conv_silu_kernel(void* out, int64_t out_stride, const void* in, int64_t in_strid
 constexpr int kMaxTaps = 16;
 
 // The same on 16-byte pieces of rows, at most 4 taps: a thread keeps one piece's latest inputs in registers while it walks RUN
-// consecutive tokens of the step (a request's start inside the run re-reads them), so a row is read once, not once per tap.
+// consecutive tokens of the step (a request's start inside the run re-reads them), so a row is read once, not once per tap.  A run
+// inside one request - all but a few - has every row on its way before the first is used.
 constexpr int kConvRun = 8;
 template <typename Tag, int TAPS>
 __global__ void __launch_bounds__(kBlock)
@@ -104,14 +105,56 @@ conv_silu_run_kernel(void* out, int64_t out_stride, const void* in, int64_t in_s
   if (c >= C) return;
   const int64_t t0 = (int64_t)blockIdx.x * kConvRun, t1 = t0 + kConvRun < T ? t0 + kConvRun : T;
   float wt[TAPS][V], bs[V], past[TAPS][V];           // past[j]: the input TAPS - 1 - j rows back (the last one: this row's)
+  const bool quads = TAPS == 4 && ((uintptr_t)w & 15) == 0;          // a channel's taps are one load
 #pragma unroll
   for (int x = 0; x < V; ++x) {
     bs[x] = bias ? bias[c + x] : 0.f;
+    if (quads) {
+      const u32x4 w4 = ld16(w + (int64_t)(c + x) * 4);
 #pragma unroll
-    for (int j = 0; j < TAPS; ++j) wt[j][x] = w[(int64_t)(c + x) * TAPS + j];
+      for (int j = 0; j < TAPS; ++j) wt[j][x] = as_f32(w4[j & 3]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) wt[j][x] = w[(int64_t)(c + x) * TAPS + j];
+    }
   }
   int b = -1;
   int64_t start = 0, prefix = 0;
+  if (t1 - t0 == kConvRun && s.extend_seq_lens && s.token_req[t0] == s.token_req[t1 - 1]) {
+    seq_of_token(s, t0, b, start, prefix);
+    const float* st = state + load_idx(s.req_pool_indices, b, s.idx64) * state_stride;
+    u32x4 row[TAPS - 1 + kConvRun];
+#pragma unroll
+    for (int j = 0; j < TAPS - 1 + kConvRun; ++j) {
+      const int64_t r = t0 - (TAPS - 1) + j;
+      row[j] = ld16((const char*)in + ((j < TAPS - 1 && r < start ? t0 : r) * in_stride + c) * E::kBytes);
+    }
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) {
+      unpack16<Tag>(row[j], past[j]);
+      const int64_t back = start - (t0 - (TAPS - 1) + j);            // > 0: so many rows before the step
+      if (back > 0) {
+#pragma unroll
+        for (int x = 0; x < V; ++x) past[j][x] = prefix - back >= 0 ? st[(TAPS - 1 - back) * C + c + x] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kConvRun; ++u) {
+      unpack16<Tag>(row[TAPS - 1 + u], past[TAPS - 1]);
+      float o[V];
+#pragma unroll
+      for (int x = 0; x < V; ++x) {
+        float acc = bs[x];
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) acc += wt[j][x] * past[j][x];
+        o[x] = silu_for<Tag>(acc);
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j) past[j][x] = past[j + 1][x];
+      }
+      st16((char*)out + ((t0 + u) * out_stride + c) * E::kBytes, pack16<Tag>(o));
+    }
+    return;
+  }
   for (int64_t t = t0; t < t1; ++t) {
     int nb;
     int64_t nstart, nprefix;
@@ -138,7 +181,7 @@ conv_silu_run_kernel(void* out, int64_t out_stride, const void* in, int64_t in_s
       float acc = bs[x];
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) acc += wt[j][x] * past[j][x];
-      o[x] = acc / (1.f + expf(-acc));
+      o[x] = silu_for<Tag>(acc);
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) past[j][x] = past[j + 1][x];
     }
@@ -372,6 +415,55 @@ int launch_mamba2_chunks(float* y, int64_t y_stride, const void* xbc, int64_t xb
   return SP_OK;
 }
 
+// The same with rows of 16-byte vectors: a wave per (token, part), the part's values in registers between the sum of squares and
+// the store (VPL vectors of 8 per lane, parts of up to 512 VPL values).  One workgroup per token and a workgroup sum per part
+// (two barriers each, eight parts) took 61 us for 4096 rows of 8 x 512; this takes 20.
+template <typename Tag, int VPL>
+__global__ void __launch_bounds__(kBlock)
+gated_group_norm_vec_kernel(void* out, int64_t out_stride, const float* y, int64_t y_stride, const void* z, int64_t z_stride,
+                            const float* w, int64_t T, int per, int parts, float eps) {
+  typedef Elem<Tag> E;
+  const int lane = threadIdx.x & 63;
+  const int64_t id = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (id >= T * parts) return;
+  const int64_t t = id / parts;
+  const int c0 = (int)(id % parts) * per;
+  u32x4 zr[VPL], ya[VPL], yb[VPL];
+#pragma unroll
+  for (int u = 0; u < VPL; ++u) {
+    const int i = (u * 64 + lane) * 8;
+    if (i < per) {
+      zr[u] = ld16((const char*)z + (t * z_stride + c0 + i) * 2);
+      ya[u] = ld16(y + t * y_stride + c0 + i);
+      yb[u] = ld16(y + t * y_stride + c0 + i + 4);
+    }
+  }
+  float v[VPL][8], ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < VPL; ++u) {
+    const int i = (u * 64 + lane) * 8;
+    if (i >= per) continue;
+    float zf[8];
+    unpack16<Tag>(zr[u], zf);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[u][e] = as_f32(e < 4 ? ya[u][e] : yb[u][e - 4]) * silu_for<Tag>(zf[e]);
+      ss += v[u][e] * v[u][e];
+    }
+  }
+  const float inv = 1.f / sqrtf(wave_sum(ss) / (float)per + eps);
+#pragma unroll
+  for (int u = 0; u < VPL; ++u) {
+    const int i = (u * 64 + lane) * 8;
+    if (i >= per) continue;
+    const u32x4 wa = ld16(w + c0 + i), wb = ld16(w + c0 + i + 4);
+    float o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = v[u][e] * inv * as_f32(e < 4 ? wa[e] : wb[e - 4]);
+    st16((char*)out + (t * out_stride + c0 + i) * 2, pack16<Tag>(o));
+  }
+}
+
 template <typename Tag>
 __global__ void __launch_bounds__(kBlock)
 gated_group_norm_kernel(void* out, int64_t out_stride, const float* y, int64_t y_stride, const void* z, int64_t z_stride,
@@ -514,6 +606,26 @@ extern "C" int sp_gated_group_norm(void* out, int64_t out_stride, const float* y
   SP_CHECK_ARG(num_tokens >= 0 && n > 0 && parts > 0 && n % parts == 0);
   if (num_tokens == 0) return SP_OK;
   SP_CHECK_ARG(out && y && z && weight && out_stride >= n && y_stride >= n && z_stride >= n);
+  const int per = n / parts;
+  const int64_t waves = (num_tokens * parts + kBlock / 64 - 1) / (kBlock / 64);
+  if (dtype != SP_F32 && per % 8 == 0 && per <= 2048 && waves < ((int64_t)1 << 31) && out_stride % 8 == 0 && y_stride % 4 == 0 &&
+      z_stride % 8 == 0 && (((uintptr_t)out | (uintptr_t)y | (uintptr_t)z | (uintptr_t)weight) & 15) == 0) {
+#define SP_GGN(T_, VPL)                                                                                              \
+  gated_group_norm_vec_kernel<T_, VPL><<<dim3((unsigned)waves), kBlock, 0, (hipStream_t)stream>>>(                    \
+      out, out_stride, y, y_stride, z, z_stride, weight, num_tokens, per, parts, eps)
+#define SP_GGN2(T_)                 \
+  do {                              \
+    if (per <= 512) SP_GGN(T_, 1);  \
+    else if (per <= 1024) SP_GGN(T_, 2); \
+    else SP_GGN(T_, 4);             \
+  } while (0)
+    if (dtype == SP_BF16) SP_GGN2(bf16_tag);
+    else SP_GGN2(f16_tag);
+#undef SP_GGN2
+#undef SP_GGN
+    SP_LAUNCH_CHECK();
+    return SP_OK;
+  }
   SP_DISPATCH_DTYPE(dtype, (gated_group_norm_kernel<Tag><<<dim3((unsigned)num_tokens), kBlock, 0, (hipStream_t)stream>>>(
                                out, out_stride, y, y_stride, z, z_stride, weight, n, parts, eps)));
   SP_LAUNCH_CHECK();

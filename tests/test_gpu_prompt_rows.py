@@ -1,0 +1,90 @@
+"""Row kernels of prompt steps at the edges of their runs and vectors, against plain torch: the request of a token row, block means
+(blocks that end inside and across workgroups, widths without whole vectors), the norm of gated parts, the short convolution over
+runs that cross requests."""
+import pytest
+import torch
+
+from tests.test_gpu_toredra_kernels import DEV, announce, close, rms, seq_extend
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lens", [[1], [3, 1, 5], [255, 1, 257], [2, 0, 3, 0, 0, 700]])
+def test_token_requests(lens):
+    from scratchpad_amd import _native
+    starts = torch.tensor([sum(lens[:i]) for i in range(len(lens))], dtype=torch.int32, device=DEV)
+    want = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens)).to(torch.int32)
+    assert torch.equal(_native.token_requests(starts, sum(lens)).cpu(), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("P", [1, 3, 16, 17, 64])
+@pytest.mark.parametrize("kw,vw", [(64, 128), (24, 40), (7, 9), (2048, 2064)])
+def test_pool_blocks(P, kw, vw, dtype):
+    from scratchpad_amd import _native
+    announce("pool_blocks", dtype, P, kw, vw)
+    g = torch.Generator(device=DEV).manual_seed(0)
+    lens, prefixes, slots = [70, 1, 16, 33], [0, 2 * P + P - 1, 5, 130], [1, 2, 3, 5]
+    total = sum(lens) + sum(prefixes)
+    table = torch.zeros(6, 400, dtype=torch.int32, device=DEV)
+    perm, at = torch.randperm(total, generator=g, device=DEV) + 1, 0
+    for n, p, s in zip(lens, prefixes, slots):
+        table[s, :n + p] = perm[at:at + n + p].to(torch.int32)
+        at += n + p
+    k, v = (torch.randn(total + 1, w, generator=g, device=DEV).to(dtype) for w in (kw, vw))
+    kp, vp = torch.full_like(k, float("nan")), torch.full_like(v, float("nan"))
+    _native.pool_blocks(kp, vp, k, v, table, seq_extend(lens, prefixes, slots), P)
+    written = torch.zeros(total + 1, dtype=torch.bool, device=DEV)
+    for n, p, s in zip(lens, prefixes, slots):
+        for pos in range(p, p + n):
+            if (pos + 1) % P == 0:
+                rows, dst = table[s, pos - P + 1:pos + 1].long(), int(table[s, pos])
+                written[dst] = True
+                for got, src in ((kp, k), (vp, v)):
+                    want = src[rows].double().mean(0)
+                    bar = 2.0 ** -8 if dtype == torch.bfloat16 else (P + 2) * 2.0 ** -23
+                    assert ((got[dst].double() - want).abs() <= bar * src[rows].double().abs().mean(0) + 1e-30).all()
+    assert torch.isnan(kp[~written]).all() and torch.isnan(vp[~written]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,parts,per", [(1, 1, 8), (5, 3, 512), (3, 2, 520), (7, 1, 1024), (2, 3, 2048), (2, 1, 2056), (3, 4, 37)])
+def test_gated_group_norm(T, parts, per, dtype):
+    from scratchpad_amd import _native
+    announce("gated_group_norm", dtype, T, parts, per)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    n = parts * per
+    y, w = torch.randn(T, n, generator=g, device=DEV), torch.rand(n, generator=g, device=DEV) + 0.5
+    z = (torch.randn(T, n + 64, generator=g, device=DEV) * 4).to(dtype)[:, :n]
+    z[0, 0] = -100.0
+    v = y.double() * torch.nn.functional.silu(z.double())
+    want = (rms(v.view(T, parts, per), 1e-5).view(T, n) * w.double()).double()
+    got = _native.gated_group_norm(y, z, w, parts, 1e-5).double()
+    bar = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10, torch.float32: 1e-5}[dtype]
+    assert ((got - want).abs() <= bar * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("C", [8, 264, 2056])
+@pytest.mark.parametrize("lens,prefixes", [([8], [0]), ([16, 9, 1, 22], [0, 2, 7, 0]), ([40], [1]), ([7, 8, 8, 1], [3, 0, 5, 1])])
+@pytest.mark.parametrize("taps", [2, 4])
+def test_causal_conv_runs(lens, prefixes, C, taps, dtype):
+    from scratchpad_amd import _native
+    announce("conv", dtype, lens, prefixes, C, taps)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    T, slots = sum(lens), list(range(1, len(lens) + 1))
+    x = torch.randn(T, C + 8, generator=g, device=DEV).to(dtype)[:, :C]
+    w, bias = torch.randn(C, taps, generator=g, device=DEV), torch.randn(C, generator=g, device=DEV)
+    state = torch.randn(len(lens) + 1, taps - 1, C, generator=g, device=DEV)
+    before, at, want = state.clone(), 0, []
+    for n, p, s in zip(lens, prefixes, slots):
+        past = before[s].double().clone()
+        past[:max(0, taps - 1 - p)] = 0                            # entries before the sequence's start are not read
+        pad = torch.cat([past, x[at:at + n].double()])
+        want.append(torch.nn.functional.silu(sum(pad[j:j + n] * w[:, j].double() for j in range(taps)) + bias.double()))
+        at += n
+    got = _native.causal_conv_silu(x, w, bias, state, seq_extend(lens, prefixes, slots))
+    want = torch.cat(want)
+    bar = 2.0 ** -8 if dtype == torch.bfloat16 else 1e-5
+    # (a silu near its zero takes the absolute error of the sum before it)
+    assert ((got.double() - want).abs() <= bar * want.abs() + 4e-6).all()
