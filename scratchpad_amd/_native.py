@@ -160,6 +160,9 @@ SIGNATURES = {
     "sp_lowrank_gate": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _vp]),
     "sp_gated_delta_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i32, _i32,
                                    _i32, _i32, _f32, *_SEQ, _i32, _vp]),
+    "sp_delta_chunk_floats": (_i64, [_i64, _i32, _i32]),
+    "sp_gated_delta_chunks": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64,
+                                     _i32, _i32, _i32, _i32, _f32, *_SEQ, _i32, _vp]),
     # ---- ABI 14
     "sp_post_norm": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _f32, _vp, _vp, _i64, _i64, _i32,
                             _f32, _i32, _vp]),
@@ -1767,6 +1770,24 @@ def lowrank_gate(p: torch.Tensor, w2t: torch.Tensor, bias: Optional[torch.Tensor
     return out
 
 
+# mean tokens per request from which a delta rule's step runs 16 tokens at a time
+DELTA_CHUNK_MIN_TOKENS = 8
+
+
+def _delta_chunks_take(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay, seq: SeqParams, dim: int, vdim: int) -> bool:
+    """the forms sp_gated_delta_chunks / sp_head_delta_chunks are built for"""
+    per = 4 if q.dtype == torch.float32 else 8
+    return (seq.extend_seq_lens is not None and seq.num_tokens >= DELTA_CHUNK_MIN_TOKENS * seq.batch_size and dim in (64, 128)
+            and vdim % 16 == 0 and q.stride(0) % per == 0 and k.stride(0) % per == 0 and q.data_ptr() % 16 == 0
+            and k.data_ptr() % 16 == 0 and (decay is None or decay.data_ptr() % 16 == 0))
+
+
+def _delta_chunk_buffers(seq: SeqParams, heads: int, vdim: int, device):
+    """(prepared matrices, read-outs) fp32 of one launch"""
+    return (torch.empty(load().sp_delta_chunk_floats(seq.num_tokens, seq.batch_size, heads), dtype=torch.float32, device=device),
+            torch.empty(seq.num_tokens * heads * vdim, dtype=torch.float32, device=device))
+
+
 def gated_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bpre: torch.Tensor, decay: torch.Tensor,
                      gate: torch.Tensor, norm_w: torch.Tensor, state: torch.Tensor, seq: SeqParams, heads: int, kv_heads: int,
                      dim: int, vdim: int, eps: float) -> torch.Tensor:
@@ -1781,6 +1802,14 @@ def gated_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bpre: to
             state.shape[1:] != (heads, dim, vdim) or not decay.is_contiguous() or not gate.is_contiguous():
         raise RuntimeError("gated_delta_scan: decay [T, H*D], gate [T, H*Dv], norm_w [Dv], state [slots, H, D, Dv]")
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
+    if _delta_chunks_take(q, k, v, decay, seq, dim, vdim):
+        work, raw = _delta_chunk_buffers(seq, heads, vdim, q.device)
+        _check(load().sp_gated_delta_chunks(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
+                                            v.data_ptr(), v.stride(0), bpre.data_ptr(), bpre.stride(0), decay.data_ptr(),
+                                            gate.data_ptr(), norm_w.data_ptr(), state.data_ptr(), state.stride(0),
+                                            work.data_ptr(), raw.data_ptr(), T, heads, kv_heads, dim, vdim, eps, *seq.args, _dt(q),
+                                            _stream()), "sp_gated_delta_chunks")
+        return out
     _check(load().sp_gated_delta_scan(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                                       v.data_ptr(), v.stride(0), bpre.data_ptr(), bpre.stride(0), decay.data_ptr(),
                                       gate.data_ptr(), norm_w.data_ptr(), state.data_ptr(), state.stride(0), heads, kv_heads,

@@ -1,0 +1,487 @@
+// Delta-rule recurrences with a decay per key channel (or per head), 16 tokens at a time, all of it fp32 on the matrix cores.
+//
+//   S = diag(w_t) S;   u_t = beta_t (v_t - S^T k_t);   S = S + k_t u_t^T;   o_t = S^T q_t        (k, q of the token, S [D, Dv])
+//
+// Over a chunk that starts from S_0, with G_t the product of the decays w_1 .. w_t per channel:
+//   Kd_t = k_t G_t,  Qd_t = q_t G_t,  Ke_s = k_s (w_{s+1} ... w_16)                              (rows of D)
+//   A_ts = beta_t sum_d k_td k_sd (w_{s+1} ... w_t)_d  (s < t),   P_ts = sum_d q_td k_sd (w_{s+1} ... w_t)_d  (s <= t)
+//   U = (I + A)^{-1} diag(beta) (V - Kd S_0),   O = Qd S_0 + P U,   S_16 = diag(G_16) S_0 + Ke^T U
+// so the serial chain is one step of matrix products per 16 tokens.  Every factor is a product of decays, never a quotient: with
+// decays in [0, 1] nothing overflows however strong they are.
+//
+// What does not read the state - A, its inverse, P and the norms of q and k - is formed for all chunks at once
+// (delta_chunk_prepare_kernel, a wave per chunk and head).  delta_chunk_scan_kernel then walks a request's chunks: a wave owns 16
+// columns of S in the accumulator layout of v_mfma_f32_16x16x4_f32 (lane (r16, q): column r16, rows 16 i + 4 q + r), in which the
+// register (i, r) IS the second operand of Kd S and Qd S for the channels 16 i + 4 q + r, and a product's four registers are the
+// second operand of the next one over tokens: the waves of a head share operands through LDS and exchange nothing.  The read-outs
+// go to fp32 rows that a last kernel norms over the head and gates.
+//
+// fp32 MFMAs: 64 multiply-adds per cycle and SIMD against 16 for fp32 vector code, whose sums over a column's lanes and LDS reads
+// per token left the per-token kernels at a quarter of that.  16 heads of 128 x 128 with a decay per channel: 8 requests of 4096
+// tokens together 682 -> 183 us (49 of them the preparation, 21 norm and gate), one request of 4096 tokens 4258 -> 725, 16 requests
+// of 300 tokens 45 -> 33; below 8 tokens per request the per-token kernel is the faster one (1 token: 39 against 51 us).
+//
+// A value that is not finite reaches the other tokens of its chunk too (zero weights times it), not only the later ones.
+#pragma once
+#include "seq_batch.h"
+
+#include <type_traits>
+
+namespace sp {
+
+typedef float f32x4_d __attribute__((ext_vector_type(4)));
+constexpr int kDC = 16;                               // tokens per chunk
+// of a chunk and head, prepared: U's matrix (I + A)^{-1} diag(beta) and P (row major), 1 / |k|, D^(-1/2) / |q|, head decay
+constexpr int kDcT = 0, kDcP = 256, kDcIk = 512, kDcIq = 528, kDcW = 544, kDcFloats = 560;
+
+struct DeltaChunks {
+  const void *q, *k, *v, *bpre;
+  const float* decay;                                 // CHANNEL: [T, H * D]
+  const float *pre, *dt_bias, *A_log;                 // per head: pre [T, >= 2 H] (step sizes, then decays)
+  float *state, *work, *raw;                          // work [chunks, H, kDcFloats], raw [T, H * Dv]
+  int64_t q_stride, k_stride, v_stride, b_stride, pre_stride, state_stride;
+  int64_t T;
+  int H, G, Dv, cols;                                 // cols: columns of a head per workgroup
+};
+
+__device__ __forceinline__ float softplus_dc(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
+
+template <int N>
+__device__ __forceinline__ float group_sum_dc(float v) {
+  v = lanes_sum<(N < 16 ? N : 16)>(v);
+  if constexpr (N >= 32) v += __shfl_xor(v, 16, 64);
+  if constexpr (N >= 64) v += __shfl_xor(v, 32, 64);
+  return v;
+}
+
+// chunks of the requests before `b` (one request per lane and round); all lanes get the sum
+__device__ __forceinline__ int chunks_before(const SeqBatch& s, int b, int lane) {
+  int n = 0;
+  for (int i = lane; i < b; i += 64) n += (s.extend_seq_lens[i] + kDC - 1) / kDC;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+  return n;
+}
+// the request and first token (within it) of chunk `id`; false behind the last
+__device__ __forceinline__ bool chunk_at(const SeqBatch& s, int id, int lane, int& b, int& t0) {
+  for (int b0 = 0; b0 < s.B; b0 += 64) {
+    const int i = b0 + lane;
+    const int n = i < s.B ? (s.extend_seq_lens[i] + kDC - 1) / kDC : 0;
+    int incl = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += o;
+    }
+    const uint64_t hit = __ballot(id < incl);
+    if (hit) {
+      const int l = __ffsll((unsigned long long)hit) - 1;
+      b = __builtin_amdgcn_readfirstlane(b0 + l);
+      t0 = __builtin_amdgcn_readfirstlane((id - __shfl(incl - n, l, 64)) * kDC);
+      return true;
+    }
+    id -= __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
+  }
+  return false;
+}
+
+// One workgroup per (chunk, head), a wave per 32 channels.  A lane sums two columns s of A and P over 4 channels; the decays
+// between s and t build up as t walks on, k, q and w of a token are broadcast reads of LDS that serve both columns.  (One wave for
+// all channels left a CU with five waves, one LDS read in flight each: 50 us for 264 chunks of 16 heads.)
+template <typename Tag, int D, bool CHANNEL>
+__global__ void __launch_bounds__(D * 2) delta_chunk_prepare_kernel(DeltaChunks a, SeqBatch sb) {
+  typedef Elem<Tag> E;
+  constexpr int V = E::kVec, QP = D / V, ROW = D + 4, NW = D / 32, NT = 64 * NW;
+  __shared__ __attribute__((aligned(16))) float sk[kDC][ROW], sq[kDC][ROW], sw[CHANNEL ? kDC : 1][ROW], sA[kDC][kDC + 4];
+  __shared__ float sbeta[kDC], sdec[kDC];
+  static_assert(NW * kDC * (kDC + 1) <= kDC * ROW, "the waves' sums take the place of the rows");
+  float(*skk)[kDC][kDC + 1] = (float(*)[kDC][kDC + 1])&sk[0][0];
+  float(*sqk)[kDC][kDC + 1] = (float(*)[kDC][kDC + 1])&sq[0][0];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = blockIdx.y;
+  int b, c0;
+  if (!chunk_at(sb, (int)blockIdx.x, lane, b, c0)) return;
+  const int64_t row0 = (int64_t)sb.extend_start_loc[b] + c0;
+  const int len = sb.extend_seq_lens[b] - c0, n = len < kDC ? len : kDC;
+  float* work = a.work + ((int64_t)blockIdx.x * a.H + h) * kDcFloats;
+  const int64_t qc = (int64_t)(h / (a.H / a.G)) * D;
+  const float qscale = 1.f / sqrtf((float)D);
+  // unit rows (zeros behind the request's end), QP lanes per row
+  for (int e = tid; e < kDC * QP; e += NT) {
+    const int t = e / QP, i = e % QP * V;
+    float kf[V], qf[V], k2 = 0.f, q2 = 0.f;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    unpack16<Tag>(t < n ? ld16((const char*)a.k + ((row0 + t) * a.k_stride + qc + i) * E::kBytes) : zero, kf);
+    unpack16<Tag>(t < n ? ld16((const char*)a.q + ((row0 + t) * a.q_stride + qc + i) * E::kBytes) : zero, qf);
+#pragma unroll
+    for (int x = 0; x < V; ++x) {
+      k2 += kf[x] * kf[x];
+      q2 += qf[x] * qf[x];
+    }
+    const float ik = 1.f / sqrtf(group_sum_dc<QP>(k2) + 1e-6f), iq = qscale / sqrtf(group_sum_dc<QP>(q2) + 1e-6f);
+#pragma unroll
+    for (int x = 0; x < V; x += 4) {
+      *(f32x4_d*)&sk[t][i + x] = f32x4_d{kf[x] * ik, kf[x + 1] * ik, kf[x + 2] * ik, kf[x + 3] * ik};
+      *(f32x4_d*)&sq[t][i + x] = f32x4_d{qf[x] * iq, qf[x + 1] * iq, qf[x + 2] * iq, qf[x + 3] * iq};
+    }
+    if (e % QP == 0) {
+      work[kDcIk + t] = ik;
+      work[kDcIq + t] = iq;
+    }
+  }
+  if constexpr (CHANNEL) {
+    for (int e = tid * 4; e < kDC * D; e += 4 * NT) {
+      const int t = e / D, i = e % D;
+      *(f32x4_d*)&sw[t][i] = t < n ? *(const f32x4_d*)(a.decay + (row0 + t) * a.H * D + (int64_t)h * D + i) : f32x4_d{1.f, 1.f, 1.f, 1.f};
+    }
+  }
+  if (tid < kDC) {
+    float beta = 0.f, dec = 1.f;
+    if (tid < n) {
+      if constexpr (CHANNEL) {
+        beta = 1.f / (1.f + expf(-E::load(a.bpre, (row0 + tid) * a.b_stride + h)));
+      } else {
+        const float* pre = a.pre + (row0 + tid) * a.pre_stride;
+        beta = 1.f / (1.f + expf(-pre[h]));
+        dec = expf(-expf(a.A_log[h]) * softplus_dc(pre[a.H + h] + a.dt_bias[h]));
+      }
+    }
+    sbeta[tid] = beta;
+    sdec[tid] = dec;
+    if constexpr (!CHANNEL) work[kDcW + tid] = dec;
+  }
+  __syncthreads();
+  // lane (s0, part): columns s0 and s0 + 8 over 4 channels; only rows t >= 8 matter to the second
+  const int s0 = lane & 7, part = lane >> 3, i = wave * 32 + part * 4;
+  f32x4_d rat = *(const f32x4_d*)&sk[s0][i], rat8 = *(const f32x4_d*)&sk[s0 + 8][i];
+  const auto all_parts = [](float v) {
+    v += dpp_f32<0x128>(v);                           // row_ror 8: the other half of the 16 lanes
+    v += __shfl_xor(v, 16, 64);
+    return v + __shfl_xor(v, 32, 64);
+  };
+  float kks[kDC], qks[kDC], kk8s[kDC / 2], qk8s[kDC / 2];
+#pragma unroll
+  for (int t = 0; t < kDC; ++t) {
+    const f32x4_d kt = *(const f32x4_d*)&sk[t][i], qt = *(const f32x4_d*)&sq[t][i];
+    if constexpr (CHANNEL) {
+      const f32x4_d wt = *(const f32x4_d*)&sw[t][i];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) rat[x] *= t >= 8 || t > s0 ? wt[x] : 1.f;
+      if (t > 8) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) rat8[x] *= t > s0 + 8 ? wt[x] : 1.f;
+      }
+    }
+    // (t < s: a number that nobody reads)
+    kks[t] = all_parts((kt[0] * rat[0] + kt[1] * rat[1]) + (kt[2] * rat[2] + kt[3] * rat[3]));
+    qks[t] = all_parts((qt[0] * rat[0] + qt[1] * rat[1]) + (qt[2] * rat[2] + qt[3] * rat[3]));
+    if (t >= 8) {
+      kk8s[t & 7] = all_parts((kt[0] * rat8[0] + kt[1] * rat8[1]) + (kt[2] * rat8[2] + kt[3] * rat8[3]));
+      qk8s[t & 7] = all_parts((qt[0] * rat8[0] + qt[1] * rat8[1]) + (qt[2] * rat8[2] + qt[3] * rat8[3]));
+    }
+  }
+  __syncthreads();                                    // every wave is done with the rows
+  if (part == 0) {
+#pragma unroll
+    for (int t = 0; t < kDC; ++t) {
+      skk[wave][t][s0] = kks[t];
+      sqk[wave][t][s0] = qks[t];
+      skk[wave][t][s0 + 8] = t >= 8 ? kk8s[t & 7] : 0.f;
+      sqk[wave][t][s0 + 8] = t >= 8 ? qk8s[t & 7] : 0.f;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < kDC * kDC; e += NT) {
+    const int t = e / kDC, s = e % kDC;
+    float kk = 0.f, qk = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      kk += skk[w][t][s];
+      qk += sqk[w][t][s];
+    }
+    if constexpr (!CHANNEL) {                         // the decays between s and t as one factor
+      float run = 1.f;
+      for (int j = s + 1; j <= t; ++j) run *= sdec[j];
+      kk *= run;
+      qk *= run;
+    }
+    sA[t][s] = t > s ? sbeta[t] * kk : 0.f;
+    work[kDcP + e] = t >= s ? qk : 0.f;
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  // column s of (I + A)^{-1}: forward substitution
+  const int s = lane & 15;
+  float x[kDC];
+#pragma unroll
+  for (int t = 0; t < kDC; ++t) {
+    float y = t == s ? 1.f : 0.f;
+#pragma unroll
+    for (int j = 0; j < t; ++j) y -= sA[t][j] * x[j];
+    x[t] = y;
+    if (lane < kDC) work[kDcT + t * kDC + s] = y * sbeta[s];
+  }
+}
+
+__device__ __forceinline__ f32x4_d mfma_d(float a, float b, const f32x4_d& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// One workgroup per (request, head, range of the head's columns): a wave per 16 columns runs the products of chunk c while
+// kDcHelpers more waves form the operand rows of chunk c + 1 and have those of chunks c + 2 and c + 3 on their way into LDS; they
+// meet at one barrier per chunk.  (The same waves doing both in turn left the matrix cores idle for two thirds of a chunk: 4.4 us.)
+constexpr int kDcHelpers = 4;
+
+template <typename Tag, int D, bool CHANNEL>
+struct DeltaScanLds {
+  static constexpr int kRow = D + 4;                                                     // floats per operand row
+  static constexpr int kRaw = kDC * D * (2 * Elem<Tag>::kBytes + (CHANNEL ? 4 : 0));     // a chunk's k, q (and decay) rows
+  static constexpr int kOps = (3 * kDC * kRow + D) * 4;                                  // Kd, Qd, Ke, G_end
+  static constexpr int kOp = 3 * kRaw, kWork = kOp + 2 * kOps, kBytes = kWork + 4 * kDcFloats * 4;
+};
+
+template <typename Tag, int D, bool CHANNEL>
+__global__ void __launch_bounds__(768) delta_chunk_scan_kernel(DeltaChunks a, SeqBatch sb) {
+  typedef Elem<Tag> E;
+  typedef DeltaScanLds<Tag, D, CHANNEL> L;
+  constexpr int DT = D / 16, ROW = L::kRow, kRowBytes = D * E::kBytes, HT = kDcHelpers * 64;
+  extern __shared__ __attribute__((aligned(16))) char delta_lds[];
+  const int tid = threadIdx.x, waves = a.cols / 16;    // the first `waves` waves own columns
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, q = lane >> 4;
+  const int b = blockIdx.x, h = blockIdx.y;
+  const int len = __builtin_amdgcn_readfirstlane(sb.extend_seq_lens[b]);
+  if (len <= 0) return;
+  const int64_t start = __builtin_amdgcn_readfirstlane(sb.extend_start_loc[b]);
+  const int64_t qc = (int64_t)(h / (a.H / a.G)) * D;
+  const int chunks = (len + kDC - 1) / kDC;
+  if (wave >= waves) {
+    const int ht = tid - 64 * waves, hw = wave - waves;
+    const float* work = a.work + ((int64_t)chunks_before(sb, b, lane) * a.H + h) * kDcFloats;
+    // a chunk's rows and prepared matrices, straight into LDS: 1 KiB per wave and load (rows past the end repeat the last one)
+    constexpr int LK = kDC * kRowBytes / 1024, LW = CHANNEL ? kDC * D * 4 / 1024 : 0, LM = (kDcFloats * 4 + 1023) / 1024;
+    const auto load = [&](const char* src, char* dst) {
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                       (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    };
+    const auto fetch = [&](int c) {
+      if (c >= chunks) return;
+      const int last = len - c * kDC - 1;              // the chunk's last row (or more)
+      const int64_t row0 = start + c * kDC;
+      char* raw = delta_lds + c % 3 * L::kRaw;
+      for (int u = hw; u < LK; u += kDcHelpers) {
+        const int byte = u * 1024 + lane * 16, t = byte / kRowBytes, x = byte % kRowBytes;
+        const int64_t row = row0 + (t < last ? t : last);
+        load((const char*)a.k + (row * a.k_stride + qc) * E::kBytes + x, raw + u * 1024);
+        load((const char*)a.q + (row * a.q_stride + qc) * E::kBytes + x, raw + (LK + u) * 1024);
+      }
+      for (int u = hw; u < LW; u += kDcHelpers) {
+        const int byte = u * 1024 + lane * 16, t = byte / (D * 4), x = byte % (D * 4);
+        const int64_t row = row0 + (t < last ? t : last);
+        load((const char*)(a.decay + row * a.H * D + (int64_t)h * D) + x, raw + (2 * LK + u) * 1024);
+      }
+      for (int u = hw; u < LM; u += kDcHelpers) {
+        const int byte = u * 1024 + lane * 16;
+        if (byte < kDcFloats * 4)
+          load((const char*)(work + (int64_t)c * a.H * kDcFloats) + byte, delta_lds + L::kWork + (c & 3) * kDcFloats * 4 + u * 1024);
+      }
+    };
+    // operand rows of a chunk: a thread walks a channel forward (Kd, Qd, G_end) or backward (Ke); rows behind the end are zeros
+    const auto operands = [&](int c, auto whole) {
+      const int n = len - c * kDC;
+      const char* raw = delta_lds + c % 3 * L::kRaw;
+      const float* wr = (const float*)(raw + 2 * kDC * kRowBytes);
+      const float* m = (const float*)(delta_lds + L::kWork + (c & 3) * kDcFloats * 4);
+      float* ops = (float*)(delta_lds + L::kOp + (c & 1) * L::kOps);
+      for (int role = ht; role < 2 * D; role += HT) {
+        const int d = role < D ? role : role - D;
+        const bool fwd = role < D;                     // (D is a multiple of 64: whole waves)
+        typename E::storage kr[kDC], qr[kDC];
+        float w[kDC];
+        f32x4_d ik[kDC / 4], iq[kDC / 4];
+#pragma unroll
+        for (int t = 0; t < kDC; ++t) {                // every read on its way before the first is used
+          w[t] = CHANNEL ? wr[t * D + d] : m[kDcW + t];
+          kr[t] = ((const typename E::storage*)raw)[t * D + d];
+          qr[t] = ((const typename E::storage*)(raw + (fwd ? kDC * kRowBytes : 0)))[t * D + d];
+        }
+#pragma unroll
+        for (int x = 0; x < kDC / 4; ++x) {
+          ik[x] = *(const f32x4_d*)&m[kDcIk + 4 * x];
+          iq[x] = *(const f32x4_d*)&m[kDcIq + 4 * x];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float k[kDC];
+#pragma unroll
+        for (int t = 0; t < kDC; ++t) {
+          const bool on = whole || t < n;
+          if (!on) w[t] = 1.f;
+          k[t] = on ? E::load(&kr[t], 0) * ik[t / 4][t % 4] : 0.f;
+        }
+        float g = 1.f;
+        if (fwd) {
+#pragma unroll
+          for (int t = 0; t < kDC; ++t) {
+            g *= w[t];
+            ops[t * ROW + d] = k[t] * g;
+            ops[(kDC + t) * ROW + d] = whole || t < n ? E::load(&qr[t], 0) * iq[t / 4][t % 4] * g : 0.f;
+          }
+          ops[3 * kDC * ROW + d] = g;
+        } else {
+#pragma unroll
+          for (int t = kDC - 1; t >= 0; --t) {
+            ops[(2 * kDC + t) * ROW + d] = k[t] * g;
+            g *= w[t];
+          }
+        }
+      }
+    };
+    const auto form = [&](int c) {
+      if (c >= chunks) return;
+      if (len - c * kDC >= kDC) operands(c, std::true_type());
+      else operands(c, std::false_type());
+    };
+    // loads of one fetch that every helper issues at the least: waiting for all but so many is waiting for the fetch before it
+    constexpr int kLoads = 2 * (LK / kDcHelpers) + LW / kDcHelpers + LM / kDcHelpers;
+    fetch(0);
+    fetch(1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    fetch(2);
+    form(0);
+    lds_barrier();
+    for (int c = 0; c < chunks; ++c) {
+      fetch(c + 3);                                    // (over the rows of chunk c, whose operands are formed)
+      form(c + 1);
+      if (c + 3 < chunks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();                                   // the rows of chunk c + 2 have landed
+    }
+    return;
+  }
+  const bool held = sb.extend_prefix_lens[b] > 0;
+  const int64_t slot = load_idx(sb.req_pool_indices, b, sb.idx64);
+  const int col = blockIdx.z * a.cols + 16 * wave + r16;
+  const bool live = col < a.Dv;                        // (Dv is a multiple of 16: whole waves)
+  float* st = a.state + slot * a.state_stride + (int64_t)h * D * a.Dv + (live ? col : 0);
+  const int64_t vc = (int64_t)h * a.Dv + (live ? col : 0);
+  f32x4_d S[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[i][r] = held && live ? st[(int64_t)(16 * i + 4 * q + r) * a.Dv] : 0.f;
+  float v[4];
+  typename E::storage vn[4];                           // the next chunk's values as they lie in memory
+  const auto fetch_v = [&](int c) {
+    const int last = len - c * kDC - 1;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = 4 * q + r;
+      vn[r] = ((const typename E::storage*)a.v)[(start + c * kDC + (t < last ? t : last)) * a.v_stride + vc];
+    }
+  };
+  fetch_v(0);
+  lds_barrier();
+  lds_barrier();
+  for (int c = 0; c < chunks; ++c) {
+    const int n = len - c * kDC;
+    const float* m = (const float*)(delta_lds + L::kWork + (c & 3) * kDcFloats * 4);
+    const float* ops = (const float*)(delta_lds + L::kOp + (c & 1) * L::kOps);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = 4 * q + r < n ? E::load(&vn[r], 0) : 0.f;
+    if (c + 1 < chunks) fetch_v(c + 1);
+    // the operands of the next products are read while the matrix cores are on the ones before (left to itself the compiler keeps
+    // registers free and waits for each read)
+    f32x4_d kd = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f}, ak[DT], aq[DT], g[DT];
+    float ke[4][DT];
+#pragma unroll
+    for (int i = 0; i < DT; ++i) {
+      ak[i] = *(const f32x4_d*)&ops[r16 * ROW + 16 * i + 4 * q];
+      aq[i] = *(const f32x4_d*)&ops[(kDC + r16) * ROW + 16 * i + 4 * q];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const auto read_state = [&](int i0, int i1) {
+#pragma unroll
+      for (int i = i0; i < i1; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          kd = mfma_d(ak[i][r], S[i][r], kd);
+          o = mfma_d(aq[i][r], S[i][r], o);
+        }
+    };
+    read_state(0, DT / 2);
+    __builtin_amdgcn_sched_barrier(0);
+    const f32x4_d tr = *(const f32x4_d*)&m[kDcT + r16 * kDC + 4 * q], pr = *(const f32x4_d*)&m[kDcP + r16 * kDC + 4 * q];
+#pragma unroll
+    for (int i = 0; i < DT; ++i) g[i] = *(const f32x4_d*)&ops[3 * kDC * ROW + 16 * i + 4 * q];
+    __builtin_amdgcn_sched_barrier(0);
+    read_state(DT / 2, DT);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < DT; ++i) ke[r][i] = ops[(2 * kDC + 4 * q + r) * ROW + 16 * i + r16];
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4_d u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u = mfma_d(tr[r], v[r] - kd[r], u);
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[i][r] *= g[i][r];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+      for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r], S[i]);
+      o = mfma_d(pr[r], u[r], o);
+    }
+    if (live) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * q + r < n) a.raw[(start + c * kDC + 4 * q + r) * (int64_t)a.H * a.Dv + vc] = o[r];
+    }
+    lds_barrier();
+  }
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st[(int64_t)(16 * i + 4 * q + r) * a.Dv] = S[i][r];
+  }
+}
+
+// whether the chunk kernels take a step: several tokens per request, heads of 64 or 128 key channels and whole waves of value
+// channels, rows that can be read 16 bytes at a time
+inline bool delta_chunks_take(const DeltaChunks& a, int D, int dtype, const SeqBatch& s) {
+  const int V = dtype == SP_F32 ? 4 : 8;
+  return s.extend_seq_lens && (D == 64 || D == 128) && a.Dv % 16 == 0 && a.q_stride % V == 0 && a.k_stride % V == 0 &&
+         (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.decay | (uintptr_t)a.work) & 15) == 0;
+}
+
+template <typename Tag, int D, bool CHANNEL>
+int launch_delta_chunks(DeltaChunks a, const SeqBatch& s, hipStream_t st) {
+  const int64_t chunks = a.T / kDC + s.B;              // at most: a request's last chunk may be partial
+  if (chunks >= ((int64_t)1 << 31) || a.H > 65535) return SP_ERR_UNSUPPORTED;
+  delta_chunk_prepare_kernel<Tag, D, CHANNEL><<<dim3((unsigned)chunks, (unsigned)a.H), D * 2, 0, st>>>(a, s);
+  SP_LAUNCH_CHECK();
+  // columns per workgroup: 128 while requests x heads fill the 256 CUs by themselves, fewer (the operand rows are then formed once
+  // per range) until they do
+  a.cols = 128;
+  while (a.cols > 64 && (int64_t)s.B * a.H * ((a.Dv + a.cols - 1) / a.cols) < 256) a.cols /= 2;
+  if (a.cols > a.Dv) a.cols = a.Dv;
+  constexpr int lds = DeltaScanLds<Tag, D, CHANNEL>::kBytes;
+  if (lds > 64 * 1024) {
+    static PerDevice<int> raised;
+    int ok = 0;
+    raised.get(ok, [&](int) {
+      return hipFuncSetAttribute((const void*)delta_chunk_scan_kernel<Tag, D, CHANNEL>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) ==
+             hipSuccess ? 1 : 0;
+    });
+    if (!ok) return SP_ERR_LAUNCH;
+  }
+  delta_chunk_scan_kernel<Tag, D, CHANNEL><<<dim3((unsigned)s.B, (unsigned)a.H, (unsigned)((a.Dv + a.cols - 1) / a.cols)),
+                                             a.cols * 4 + kDcHelpers * 64, lds, st>>>(a, s);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
+
+}  // namespace sp

@@ -17,6 +17,8 @@
 // d = 32 kk + 8 q + 0 .. 7: split in place they ARE the operand of S^T q, the state never passes through LDS.  The 10 lower
 // 16 x 16 tiles of q k^T (and two of zeros) are dealt to the waves and exchanged through LDS.  Two products sum over tokens
 // and take their operands transposed: k and v are also staged as [channel][token], two tokens packed per 4-byte write.
+//
+// A value that is not finite reaches the other tokens of its chunk too (zero weights times it), not only the later ones.
 #pragma once
 #include "seq_batch.h"
 

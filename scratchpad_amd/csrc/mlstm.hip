@@ -242,11 +242,11 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
     c.sc = c.scalars(c0 / kCL);
     if (c0 / kCL % NW == 0) {
       scan_gates(c0);
-      __syncthreads();
+      lds_barrier();
       gates(c0);
     }
     c.stage();
-    __syncthreads();
+    lds_barrier();
     if (c0 + kCL < len) load(c0 + kCL);
     c.scores();
     c.from_state(zero);
@@ -273,7 +273,7 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
         const int t = 16 * i + 4 * c.q + r;
         gv[i][r] = *(const uint16_t*)(gb + c0 * g_stride * 2 + (uint32_t)((t < n ? t : n - 1) * (uint32_t)g_stride + col) * 2u);
       }
-    __syncthreads();
+    lds_barrier();
     c.template weigh<true>();
     if (c0 + kCL < len && (c0 / kCL + 1) % NW != 0) gates(c0 + kCL);
     {      // the normaliser's update: the lanes of a channel share the chunk's tokens
@@ -291,7 +291,7 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
       x = lanes_sum<PER>(x);
       if (part == 0) sn[d] = sc.a_end * sn[d] + x;
     }
-    __syncthreads();
+    lds_barrier();
     c.absorb();
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -300,7 +300,7 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
         const float ss = lanes_sum<16>(c.o[i][r] * c.o[i][r]);
         if (c.r16 == 0) red[c.wave * kCL + 16 * i + 4 * c.q + r] = ss;
       }
-    __syncthreads();
+    lds_barrier();
     // lane t of every wave: the division by the normaliser and the RMS of the divided row as one factor
     float nq = snq[c.lane] * c.sc->a0[c.lane], ss = 0.f;
     for (int j = 0; j <= c.q; ++j) nq += c.sums()[j * kCL + c.lane];

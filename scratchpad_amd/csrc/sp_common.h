@@ -207,6 +207,14 @@ __device__ __forceinline__ u32x4 bf16x8_to_f16x8(const u32x4& v) {
   return o;
 }
 
+// A workgroup barrier for what the waves exchange through LDS only.  __syncthreads() also waits for every global load and store
+// of the wave: rows on their way for the next pass, results on their way out.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // ---- wave reductions ------------------------------------------------------------------------
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

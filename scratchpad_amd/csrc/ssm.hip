@@ -374,7 +374,7 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
     const int n = (int)(len - c0 < kCL ? len - c0 : kCL);
     c.sc = c.scalars(c0 / kCL);
     c.stage();
-    __syncthreads();
+    lds_barrier();
     if (c0 + kCL < len) {
       load(c0 + kCL);
       load_steps(c0 + kCL);
@@ -382,10 +382,10 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
     c.scores();
     c.from_state(zero);
     zero = false;
-    __syncthreads();
+    lds_barrier();
     c.template weigh<false>();
     if (c0 + kCL < len) steps(c0 + kCL);
-    __syncthreads();
+    lds_barrier();
     c.absorb();
     char* yc = (char*)(y + (start + c0) * y_stride + (int64_t)h * Dv);
 #pragma unroll
@@ -397,7 +397,7 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
       for (int r = 0; r < 4; ++r)
         if (t0 + r < n) *(float*)(yc + (uint32_t)((t0 + r) * (uint32_t)y_stride + c.column()) * 4u) = c.o[i][r] + skip * x[r];
     }
-    __syncthreads();
+    lds_barrier();
   }
   c.store_state(st);
 }

@@ -97,3 +97,69 @@ def test_mamba2_chunks(lens, H, G, N, Dv):
         near(y.view(T, H, Dv), want, 2e-5)
     for slot in range(0, n_slots, 2):
         assert torch.isnan(S[slot]).all()
+
+
+DELTA_LENS = [[8], [15, 16, 17], [48, 1, 33, 2], [16, 200, 3]]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lens", DELTA_LENS, ids=lambda l: "-".join(map(str, l)))
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 1, 128, 128), (4, 4, 64, 64), (3, 3, 128, 48), (2, 2, 64, 208)])
+def test_gated_delta_chunks(lens, H, G, D, Dv, dtype):
+    from scratchpad_amd import _native
+    announce("gated delta chunks", dtype, lens, H, G, D, Dv)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    T, slots = sum(lens), slots_of(lens)
+    n_slots = 2 * len(lens) + 1
+    S = torch.full((n_slots, H, D, Dv), float("nan"), device=DEV)
+    ref = {s: torch.zeros(H, D, Dv, dtype=torch.float64, device=DEV) for s in slots}
+    nw = torch.rand(Dv, generator=g, device=DEV) + 0.5
+    for prefixes in ([0] * len(lens), lens):
+        a = torch.randn(T, 2 * G * D + H * Dv + H, generator=g, device=DEV).to(dtype)
+        q, k, v, bp = a.split([G * D, G * D, H * Dv, H], 1)
+        if not _native._delta_chunks_take(q, k, v, None, seq_extend(lens, prefixes, slots), D, Dv):
+            q, k = q.contiguous(), k.contiguous()                # (a product whose width breaks the rows' alignment)
+        decay = torch.rand(T, H * D, generator=g, device=DEV) ** 2
+        decay[torch.rand(T, H * D, generator=g, device=DEV) < 0.05] = 0.0          # a channel forgotten, and one kept, exactly
+        decay[:, 0] = 1.0
+        gate = torch.rand(T, H * Dv, generator=g, device=DEV)
+        seq = seq_extend(lens, prefixes, slots)
+        assert _native._delta_chunks_take(q, k, v, decay, seq, D, Dv)
+        out = _native.gated_delta_scan(q, k, v, bp, decay, gate, nw, S, seq, H, G, D, Dv, 1e-5)
+        unit = lambda x: x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+        kk, qq = (unit(x.double().view(T, G, D)).repeat_interleave(H // G, 1) for x in (k, q))
+        qq, vv, beta = qq * D ** -0.5, v.double().view(T, H, Dv), torch.sigmoid(bp.double())
+        w, want, at = decay.double().view(T, H, D), torch.empty(T, H, Dv, dtype=torch.float64, device=DEV), 0
+        for length, slot in zip(lens, slots):
+            Sr = ref[slot]
+            for t in range(at, at + length):
+                Sr = w[t][:, :, None] * Sr
+                u = beta[t][:, None] * (vv[t] - (Sr * kk[t][:, :, None]).sum(1))
+                Sr = Sr + kk[t][:, :, None] * u[:, None]
+                want[t] = (Sr * qq[t][:, :, None]).sum(1)
+            ref[slot] = Sr
+            at += length
+            near(S[slot], Sr, 2e-5)
+        want = want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-5)
+        want = (want * nw.double()).view(T, H * Dv) * gate.double()
+        bar = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10, torch.float32: 1e-4}[dtype]
+        # (1e-3: a head whose read-out nearly cancels is scaled up by its norm, and the fp32 sums' roundings with it)
+        assert ((out.double() - want).abs() <= bar * want.abs() + 1e-3).all()
+    for slot in range(0, n_slots, 2):
+        assert torch.isnan(S[slot]).all()
+
+
+@pytest.mark.parametrize("T", [64, 129, 700])
+@pytest.mark.parametrize("rank,channels", [(32, 16), (64, 208), (96, 64), (128, 2048)])
+def test_lowrank_gate_of_many_tokens(T, rank, channels):
+    from scratchpad_amd import _native
+    announce("lowrank_gate", T, rank, channels)
+    g = torch.Generator(device=DEV).manual_seed(6)
+    p = torch.randn(T, rank + 8, generator=g, device=DEV).bfloat16()[:, 8:]
+    w2t, bias = torch.randn(rank, channels, generator=g, device=DEV) * rank ** -0.5, torch.randn(channels, generator=g, device=DEV)
+    A = torch.randn(channels // 16, generator=g, device=DEV) * 0.5 - 1
+    z = p.double() @ w2t.double() + bias.double()
+    want = torch.exp(-torch.exp(A.double()).repeat_interleave(16) * torch.nn.functional.softplus(z))
+    # a decay moves by its exponent's error: fp32 sums of `rank` products, a few ulp of exponential and logarithm
+    assert ((_native.lowrank_gate(p, w2t, bias, "decay", A).double() - want).abs() <= 4e-6).all()
+    assert ((_native.lowrank_gate(p, w2t, None, "sigmoid").double() - torch.sigmoid(p.double() @ w2t.double())).abs() <= 2e-6).all()
