@@ -48,15 +48,26 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_vec_kernel(void* out,  // may 
   char* orow = (char*)out + row * o_stride * E::kBytes;
   const int nvec = hidden / V;
   float cache[MAXIT][V];
+  u32x4 xin[MAXIT], rin[MAXIT], win[MAXIT];
   float ss = 0.f;
 #pragma unroll
   for (int it = 0; it < MAXIT; ++it) {
     const int v = threadIdx.x + it * kBlock;
     if (v < nvec) {
-      unpack16<Tag>(ld16(xrow + (int64_t)v * 16), cache[it]);
+      xin[it] = ld16(xrow + (int64_t)v * 16);
+      if (FUSED) rin[it] = ld16(rrow + (int64_t)v * 16);
+      win[it] = ld16((const char*)weight + (int64_t)v * 16);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int it = 0; it < MAXIT; ++it) {
+    const int v = threadIdx.x + it * kBlock;
+    if (v < nvec) {
+      unpack16<Tag>(xin[it], cache[it]);
       if (FUSED) {
         float r[V];
-        unpack16<Tag>(ld16(rrow + (int64_t)v * 16), r);
+        unpack16<Tag>(rin[it], r);
 #pragma unroll
         for (int e = 0; e < V; ++e) cache[it][e] = __fadd_rn(cache[it][e], r[e]);
         st16(rrow + (int64_t)v * 16, pack16<Tag>(cache[it]));
@@ -72,7 +83,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_vec_kernel(void* out,  // may 
     const int v = threadIdx.x + it * kBlock;
     if (v < nvec) {
       float w[V], y[V];
-      unpack16<Tag>(ld16((const char*)weight + (int64_t)v * 16), w);
+      unpack16<Tag>(win[it], w);
 #pragma unroll
       for (int e = 0; e < V; ++e) y[e] = __fmul_rn(E::round(__fmul_rn(cache[it][e], rs)), w[e]);
       st16(orow + (int64_t)v * 16, pack16<Tag>(y));
@@ -117,7 +128,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_scalar_kernel(void* out,  // m
 // ACT 1: gelu_tanh(a) * b, the product of two fp32 values rounded once.
 template <typename Tag, int ACT>
 __device__ __forceinline__ float glu_f32(float a, float b) {
-  if constexpr (ACT == 1) return __fmul_rn(gelu_tanh_f32(a), b);
+  if constexpr (ACT == 1) return mul_f32(gelu_tanh_f32(a), b);
   else return __fmul_rn(Elem<Tag>::round(silu_ref(a)), b);   // sp_common.h
 }
 

@@ -5,17 +5,31 @@
 // 696-760, 423-470, 1033-1155 -> F.linear) and LogitsProcessor._get_logits
 // (nn/layers/logits_processor.py:340-376).  Above 16 rows the library GEMM (hipBLASLt) stays.
 //
-// At M <= 16 the product is a pure stream of the weight matrix (2 flop per weight byte per row):
-// HBM-bound.  hipBLASLt runs these shapes at 2.5-5.0 TB/s of weight bytes (bs 1, Llama-3-8B:
-// o_proj 13.6 us for 33.5 MB, qkv 15.5 us for 50 MB); a kernel shaped for the stream does better:
-//   * one workgroup = 16 output columns (16 rows of W), its 8 waves take the k-steps round-robin,
-//     so at any moment the workgroup reads 512 contiguous bytes of each of its 16 rows;
-//   * per k-step (32 elements) a lane loads 16 B of W and 16 B of x straight into the A / B operand
-//     registers of v_mfma_f32_16x16x32 (rows of W are the A rows, rows of x the B columns) - no LDS
-//     on the way in; x (<= 16 x K, <= 460 KB) is re-read from L2 by every workgroup;
-//   * 8 k-steps of loads are in flight per wave before the first MFMA consumes one;
-//   * the 8 waves' 16x16 partial tiles are summed through LDS in a fixed order (deterministic),
-//     rounded once, and stored.
+// At M <= 16 the product is a pure stream of the weight matrix (2 flop per weight byte per row): HBM-bound.  What decides the
+// rate is how many bytes of each weight row one load covers and how many workgroups share the stream, so there are three forms:
+//   1 row       a wave per weight row: a load covers 1 KB of the row, 4 of them in flight, the products on the vector unit (24
+//               instructions a KB: a quarter of what the stream leaves room for), 2 waves a workgroup
+//   2-4 rows    (few weight rows, or long ones) v_mfma_f32_4x4x4 (16 blocks): lane (b, i) loads 16 B of weight row i at chunk b,
+//               so a load covers 256 B of 4 rows and its two halves are two products; the 16 blocks are 16 partial sums over K.
+//               4 waves share K, 4 or 8 weight rows (columns of out) a workgroup
+//   to 16 rows  v_mfma_f32_16x16x32: 64 B of 16 weight rows a load, x read in the same form (as many bytes out of L2 as weights:
+//               what bounds it from 8 rows on).  A wave's loads in flight lie next to each other in K, so that both halves of a
+//               128-byte line are asked for by one wave
+// Each form sums the partial results of its lanes and waves in a fixed order that M, K and the
+// number of weight rows alone decide.
+// us, cold weights under graph replay, N x K: 1 row / 4 rows / 8 rows; before (the third form for every M, the waves' k-steps
+// interleaved) -> now.  The line between the second and the third form is where their times cross (8 rows: 20.1 and 17.3 at
+// 16384 x 2048, 12.8 and 14.6 at 2048 x 8192), between the first and the second it is the one row itself.
+//   3072 x 2048     5.3 -> 4.6      5.7 -> 5.8      6.1 -> 6.1
+//   2048 x 2048     5.0 -> 3.8      5.3 -> 4.9      5.7 -> 5.8
+//   16384 x 2048   14.5 -> 12.3    15.9 -> 14.8    18.2 -> 17.3
+//   2048 x 8192    13.3 -> 8.2     14.7 -> 10.4    16.2 -> 14.6
+//   6144 x 4096    13.2 -> 9.9     14.4 -> 12.6    16.1 -> 15.6
+//   28672 x 4096   43.7 -> 40.7    47.4 -> 43.0    54.4 -> 50.4
+//   128256 x 2048  89.0 -> 83.1    98.5 -> 90.1   118.0 -> 113.2
+// Tried and slower: x staged in LDS and a persistent loop over weight rows in any of 10 shapes (8 to 40 % slower: the copy and its
+// barrier come before the first product, and the loop's tail is longer than a launch of many small workgroups), 16 products in
+// flight, two weight rows a wave at one row.
 //
 // Epilogue fusion (round 4): with `epilogue` = 1 the weight is the merged gate|up matrix [2 I, K] of LlamaMLP
 // (nn/models/llama/llama.py:62-66) and the output is SiluAndMul (nn/layers/activation.py:21-31) of the projection,
@@ -58,119 +72,260 @@ struct SkinnyArgs {
   int64_t x_stride, w_stride, out_stride;   // elements
 };
 
+// the value a finished sum is stored as (EPI 1 and 3 store glu_value instead)
+template <int EPI>
+__device__ __forceinline__ float plain_value(float s) {
+  if constexpr (EPI == 2) {
+    s = fmaxf(s, 0.f);
+    s *= s;
+  }
+  return s;
+}
+// glu_mul_vec_kernel's arithmetic on the ROUNDED gate and up sums
+template <typename Tag, int EPI>
+__device__ __forceinline__ float glu_value(float gate, float up) {
+  typedef Elem<Tag> E;
+  const float act = EPI == 3 ? gelu_tanh_f32(E::round(gate)) : E::round(silu_ref(E::round(gate)));
+  return mul_f32(act, E::round(up));
+}
+
+// ---- 1 row
+constexpr int kRowWaves = 2, kRowLoads = 4;
+
+template <typename Tag, int EPI>
+__global__ __launch_bounds__(kRowWaves * 64) void gemm_row_kernel(SkinnyArgs a) {
+  typedef Elem<Tag> E;
+  constexpr bool GLU = EPI == 1 || EPI == 3;
+  constexpr int R = GLU ? 2 : 1;                       // a gate row and its up row, or one row
+  const int lane = threadIdx.x & 63, n = blockIdx.x * kRowWaves + (threadIdx.x >> 6);
+  if (n >= a.N) return;                                // no barrier in this kernel
+  const char* wp[R];
+  float acc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    wp[r] = a.w + ((int64_t)r * a.N + n) * a.w_stride * 2;
+    acc[r] = 0.f;
+  }
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  for (int k0 = 0; k0 < a.K; k0 += 512 * kRowLoads) {
+    u32x4 wf[kRowLoads][R], xf[kRowLoads];
+#pragma unroll
+    for (int u = 0; u < kRowLoads; ++u) {
+      const int k = k0 + u * 512 + lane * 8;           // K is a multiple of 8: a lane's 16 bytes are in the row or past it
+      const bool in = k < a.K;
+#pragma unroll
+      for (int r = 0; r < R; ++r) wf[u][r] = in ? ld16(wp[r] + (int64_t)k * 2) : zero;
+      xf[u] = in ? ld16(a.x + (int64_t)k * 2) : zero;
+    }
+    __builtin_amdgcn_sched_barrier(0);                 // all of them on their way before the first is waited for
+#pragma unroll
+    for (int u = 0; u < kRowLoads; ++u) {
+      float xv[8];
+      unpack16<Tag>(xf[u], xv);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float wv[8];
+        unpack16<Tag>(wf[u][r], wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[r] = fmaf(wv[e], xv[e], acc[r]);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
+  if (lane == 0) E::store(a.out, n, GLU ? glu_value<Tag, EPI>(acc[0], acc[R - 1]) : plain_value<EPI>(acc[0]));
+}
+
+// ---- 2-4 rows
+typedef short s16x4_g __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x4_g __attribute__((ext_vector_type(4)));
+
+// lane (b, i): a = weight row i, b = x row i, 8 elements of K; block b of the accumulator += rows . rows^T over those 8
+template <typename Tag>
+__device__ __forceinline__ f32x4_g mfma_quad(const u32x4& a, const u32x4& b, f32x4_g c) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const u32x2 ah = {a[2 * h], a[2 * h + 1]}, bh = {b[2 * h], b[2 * h + 1]};
+    if constexpr (__is_same(Tag, bf16_tag))
+      c = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4_g, ah), __builtin_bit_cast(s16x4_g, bh), c, 0, 0, 0);
+    else
+      c = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4_g, ah), __builtin_bit_cast(f16x4_g, bh), c, 0, 0, 0);
+  }
+  return c;
+}
+
+constexpr int kQuadWaves = 4, kQuadLoads = 4, kQuadRows = 4;
+
+// G groups of 4 weight rows: two where there are enough of them to fill the card (x is read half as often) and for gate and up,
+// else one and twice the length of K in flight.  The order of the sums is the same.
+template <typename Tag, int G, int EPI>
+__global__ __launch_bounds__(kQuadWaves * 64) void gemm_quad_kernel(SkinnyArgs a) {
+  typedef Elem<Tag> E;
+  constexpr bool GLU = EPI == 1 || EPI == 3;
+  static_assert(!GLU || G == 2, "gate rows and the up rows of the same columns");
+  __shared__ float red[kQuadWaves][16 * G];            // [wave][group][weight row 4][x row 4]
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int b = lane >> 2, i = lane & 3;
+  const int n0 = blockIdx.x * (GLU ? 4 : 4 * G);
+  const char* wp[G];                                   // rows past N: row N - 1 again, computed and not stored
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int n = GLU ? g * a.N + min(n0 + i, a.N - 1) : min(n0 + 4 * g + i, a.N - 1);
+    wp[g] = a.w + ((int64_t)n * a.w_stride + 8 * b) * 2;
+  }
+  const bool mrow = i < a.M;
+  const char* xp = a.x + ((int64_t)min(i, a.M - 1) * a.x_stride + 8 * b) * 2;
+  f32x4_g acc[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) acc[g] = f32x4_g{0.f, 0.f, 0.f, 0.f};
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  constexpr int kSpan = 128 * kQuadLoads, kSpans = 2 / G;       // a wave's spans of K: wave, wave + 4, ...; kSpans at a time
+  for (int k0 = wave * kSpan; k0 < a.K; k0 += kSpans * kQuadWaves * kSpan) {
+    u32x4 wf[kSpans * kQuadLoads][G], xf[kSpans * kQuadLoads];
+#pragma unroll
+    for (int u = 0; u < kSpans * kQuadLoads; ++u) {
+      const int k = k0 + (u / kQuadLoads) * kQuadWaves * kSpan + (u % kQuadLoads) * 128;
+      const bool in = k + 8 * b < a.K;
+#pragma unroll
+      for (int g = 0; g < G; ++g) wf[u][g] = in ? ld16(wp[g] + (int64_t)k * 2) : zero;
+      xf[u] = in && mrow ? ld16(xp + (int64_t)k * 2) : zero;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kSpans * kQuadLoads; ++u)
+#pragma unroll
+      for (int g = 0; g < G; ++g) acc[g] = mfma_quad<Tag>(wf[u][g], xf[u], acc[g]);
+  }
+  // lane (b, m): acc[g][r] = block b's part of out[m][row r of group g]
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float s = acc[g][r];
+#pragma unroll
+      for (int step = 4; step < 64; step *= 2) s += __shfl_xor(s, step);
+      if (lane < 4) red[wave][(g * 4 + r) * 4 + lane] = s;
+    }
+  __syncthreads();
+  if (threadIdx.x >= 16 * G) return;
+  float s = 0.f;
+#pragma unroll
+  for (int w = 0; w < kQuadWaves; ++w) s += red[w][lane];
+  const int m = lane & 3, r = (lane >> 2) & 3, g = lane >> 4;
+  if constexpr (GLU) {
+    const float up = __shfl_down(s, 16);
+    if (g == 0 && m < a.M && n0 + r < a.N) E::store(a.out, (int64_t)m * a.out_stride + n0 + r, glu_value<Tag, EPI>(s, up));
+  } else {
+    const int n = n0 + 4 * g + r;
+    if (m < a.M && n < a.N) E::store(a.out, (int64_t)m * a.out_stride + n, plain_value<EPI>(s));
+  }
+}
+
+// ---- 5-16 rows
 constexpr int kSkWaves = 8;
 
-// NB = 16-column blocks per workgroup: one x fragment feeds NB MFMAs (x traffic out of L2 drops to
-// 1/NB of the weight stream).  Measured on MI355X it is SLOWER than NB = 1 wherever N allows it
-// (gate_up 28672x4096 at 1 row: NB 2 53.9 us vs NB 1 44.1 us; LM head 128256x4096: NB 4 206 us vs
-// NB 1 166 us; same sign at 8 rows) - fewer, fatter workgroups lose more than the x reads cost -
-// so launch_skinny always takes NB = 1; the parameter stays for re-measurement.
-// NT (sp_debug_set("skinny_nt", 1); OFF by default): non-temporal weight loads - the weights are read exactly once by
-// exactly one workgroup (MI355X_MICROARCH.md, 'nt-weights').  Measured on this kernel it LOSES: 1 row qkv 14.5 vs 13.6 us,
-// gate_up 46.5 vs 43.3, LM head 186 vs 166; bench.py --bs 1: 4.13 vs 3.98 ms/step (round 3, tools/bench_gemv.py).
+// NT (sp_debug_set("skinny_nt", 1); OFF by default): non-temporal weight loads.  They lose: 1 row qkv 14.5 vs 13.6 us, gate_up
+// 46.5 vs 43.3, LM head 186 vs 166.
 __device__ __forceinline__ u32x4 ld16_nt(const void* p) { return __builtin_nontemporal_load((const u32x4*)p); }
 
-// EPI 1 and 3 (NB = 1 only): a.N = I output columns; the 16 W rows of a workgroup are gate rows n0 .. n0+7 (tile rows 0-7) and
-// up rows I + n0 .. I + n0 + 7 (tile rows 8-15)
-template <typename Tag, int NB, int UNROLL, bool NT, int EPI>
+// EPI 1 and 3: a.N = I output columns; the 16 W rows of a workgroup are gate rows n0 .. n0+7 (tile rows 0-7) and up rows
+// I + n0 .. I + n0 + 7 (tile rows 8-15)
+template <typename Tag, int UNROLL, bool NT, int EPI>
 __global__ __launch_bounds__(kSkWaves * 64) void gemm_skinny_kernel(SkinnyArgs a) {
   typedef Elem<Tag> E;
   constexpr bool GLU = EPI == 1 || EPI == 3;
-  static_assert(!GLU || NB == 1, "the activation-mul epilogue pairs the two halves of one 16-row tile");
-  __shared__ float red[kSkWaves][NB][16 * 17];
+  __shared__ float red[kSkWaves][16 * 17];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r16 = lane & 15, q = lane >> 4;            // operand row / k-quarter of the lane
-  const int n0 = GLU ? blockIdx.x * 8 : blockIdx.x * 16 * NB;
+  const int n0 = GLU ? blockIdx.x * 8 : blockIdx.x * 16;
   const bool mrow = r16 < a.M;
-  const char* wp[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    int n = min(n0 + 16 * nb + r16, a.N - 1);          // clamp: columns past N are computed, never stored
-    if constexpr (GLU) n = (r16 < 8 ? 0 : a.N) + min(n0 + (r16 & 7), a.N - 1);
-    wp[nb] = a.w + ((int64_t)n * a.w_stride + 8 * q) * 2;
-  }
+  int n = min(n0 + r16, a.N - 1);                      // clamp: columns past N are computed, never stored
+  if constexpr (GLU) n = (r16 < 8 ? 0 : a.N) + min(n0 + (r16 & 7), a.N - 1);
+  const char* wp = a.w + ((int64_t)n * a.w_stride + 8 * q) * 2;
   const char* xp = a.x + ((int64_t)min(r16, a.M - 1) * a.x_stride + 8 * q) * 2;
   const int ksteps = a.K / 32;
-  f32x4_g acc[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4_g{0.f, 0.f, 0.f, 0.f};
+  f32x4_g acc = {0.f, 0.f, 0.f, 0.f};
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  // this wave's k-steps: wave, wave + 8, ...; processed in groups of UNROLL with all loads first
-  int ks = wave;
-  for (; ks + (UNROLL - 1) * kSkWaves < ksteps; ks += UNROLL * kSkWaves) {
-    u32x4 wf[UNROLL][NB], xf[UNROLL];
+  // this wave's k-steps: UNROLL in a row, then UNROLL more kSkWaves * UNROLL steps on, all loads of a group first
+  for (int ks = wave * UNROLL; ks < ksteps; ks += UNROLL * kSkWaves) {
+    u32x4 wf[UNROLL], xf[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      const int64_t off = (int64_t)(ks + u * kSkWaves) * 64;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) wf[u][nb] = NT ? ld16_nt(wp[nb] + off) : ld16(wp[nb] + off);
-      xf[u] = mrow ? ld16(xp + off) : zero;
+      const int64_t off = (int64_t)(ks + u) * 64;
+      const bool in = ks + u < ksteps;
+      wf[u] = in ? (NT ? ld16_nt(wp + off) : ld16(wp + off)) : zero;
+      xf[u] = in && mrow ? ld16(xp + off) : zero;
     }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u)
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma_g<Tag>(wf[u][nb], xf[u], acc[nb]);
+    for (int u = 0; u < UNROLL; ++u) acc = mfma_g<Tag>(wf[u], xf[u], acc);
   }
-  for (; ks < ksteps; ks += kSkWaves) {
-    const int64_t off = (int64_t)ks * 64;
-    const u32x4 xf = mrow ? ld16(xp + off) : zero;
+  // acc[r] = partial of out[m = r16][n0 + 4q + r]; sum the waves in wave order
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma_g<Tag>(NT ? ld16_nt(wp[nb] + off) : ld16(wp[nb] + off), xf, acc[nb]);
-  }
-  // acc[nb][r] = partial of out[m = r16][n0 + 16 nb + 4q + r]; sum the waves in wave order
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) red[wave][nb][(4 * q + r) * 17 + r16] = acc[nb][r];
+  for (int r = 0; r < 4; ++r) red[wave][(4 * q + r) * 17 + r16] = acc[r];
   __syncthreads();
-  for (int nb = wave; nb < NB; nb += kSkWaves) {
+  if (wave != 0) return;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int col = 4 * q + r;
-      float s = 0.f;
+  for (int r = 0; r < 4; ++r) {
+    const int col = 4 * q + r;
+    float s = 0.f;
 #pragma unroll
-      for (int w = 0; w < kSkWaves; ++w) s += red[w][nb][col * 17 + r16];
-      if constexpr (GLU) {
-        // tile columns 0-7 are gate sums, 8-15 the up sums of the same output columns: the lanes of the gate half
-        // finish both (same summation order as above) and apply glu_mul_vec_kernel's arithmetic to the ROUNDED sums
-        float su = 0.f;
+    for (int w = 0; w < kSkWaves; ++w) s += red[w][col * 17 + r16];
+    const int no = n0 + col;
+    if constexpr (GLU) {
+      // tile columns 0-7 are gate sums, 8-15 the up sums of the same output columns: the lanes of the gate half finish both
+      // (same summation order as above)
+      float su = 0.f;
 #pragma unroll
-        for (int w = 0; w < kSkWaves; ++w) su += red[w][nb][((col & 7) + 8) * 17 + r16];
-        const int n = n0 + col;
-        if (mrow && q < 2 && n < a.N) {
-          const float act = EPI == 3 ? gelu_tanh_f32(E::round(s)) : E::round(silu_ref(E::round(s)));
-          E::store(a.out, (int64_t)r16 * a.out_stride + n, __fmul_rn(act, E::round(su)));
-        }
-      } else {
-        const int n = n0 + 16 * nb + col;
-        if constexpr (EPI == 2) {
-          s = fmaxf(s, 0.f);
-          s *= s;
-        }
-        if (mrow && n < a.N) E::store(a.out, (int64_t)r16 * a.out_stride + n, s);
-      }
+      for (int w = 0; w < kSkWaves; ++w) su += red[w][((col & 7) + 8) * 17 + r16];
+      if (mrow && q < 2 && no < a.N) E::store(a.out, (int64_t)r16 * a.out_stride + no, glu_value<Tag, EPI>(s, su));
+    } else if (mrow && no < a.N) {
+      E::store(a.out, (int64_t)r16 * a.out_stride + no, plain_value<EPI>(s));
     }
   }
 }
 
 static int g_skinny_nt = 0;     // sp_debug_set("skinny_nt", 0 / 1): A/B switch of the non-temporal weight loads
 void set_skinny_nt(int v) { g_skinny_nt = v; }
-// sp_debug_set("skinny_unroll16", 0 / 1): 16 k-steps of loads in flight per wave where a wave's share is a multiple of
-// 16 (K = 4096: the whole share in ONE round of loads instead of two)
+// sp_debug_set("skinny_unroll16", 0 / 1): 16 k-steps of loads in flight per wave in place of 4
 static int g_skinny_u16 = 0;
 void set_skinny_unroll16(int v) { g_skinny_u16 = v; }
 
+// One group of 4 weight rows up to 2048 rows: 256 workgroups of two groups there (3 rows, K 4096, us: 1024 rows 4.6 one / 6.3 two,
+// 2048 rows 6.3 / 6.9, 2560 rows 7.8 / 8.9, 8192 rows 16.0 / 14.6).
+constexpr int kQuadOneGroup = 2048;
+// 2-4 rows go to the tiles of 16 weight rows where there are more than the one-group form's rows and K is too short for the
+// others' head start (us, 4 rows, tiles / two groups: K 1024, 3072 rows 3.9 / 4.8, 8192 rows 5.8 / 6.5; K 2048, 3072 rows
+// 5.8 / 6.4, 4096 rows 6.3 / 6.4, 6144 rows 9.0 / 7.9; K 4096, 3072 rows 8.7 / 9.6, 5120 rows 14.6 / 12.3).
+static bool few_and_short(int64_t rows, int K) { return rows > kQuadOneGroup && (K <= 1024 || (K <= 2048 && rows <= 4096)); }
+
+template <typename Tag, int EPI>
+static void launch_skinny_as(const SkinnyArgs& a, hipStream_t st) {
+  constexpr bool GLU = EPI == 1 || EPI == 3;
+  if (a.M == 1) {
+    gemm_row_kernel<Tag, EPI><<<dim3((a.N + kRowWaves - 1) / kRowWaves), dim3(kRowWaves * 64), 0, st>>>(a);
+  } else if (a.M <= kQuadRows && !few_and_short(GLU ? 2 * (int64_t)a.N : a.N, a.K)) {
+    if (!GLU && a.N <= kQuadOneGroup) {
+      if constexpr (!GLU) gemm_quad_kernel<Tag, 1, EPI><<<dim3((a.N + 3) / 4), dim3(kQuadWaves * 64), 0, st>>>(a);
+    } else {
+      constexpr int cols = GLU ? 4 : 8;
+      gemm_quad_kernel<Tag, 2, EPI><<<dim3((a.N + cols - 1) / cols), dim3(kQuadWaves * 64), 0, st>>>(a);
+    }
+  } else {
+    constexpr int cols = GLU ? 8 : 16;
+    const dim3 grid((a.N + cols - 1) / cols), block(kSkWaves * 64);
+    if (g_skinny_u16) gemm_skinny_kernel<Tag, 16, false, EPI><<<grid, block, 0, st>>>(a);
+    else if (g_skinny_nt) gemm_skinny_kernel<Tag, 4, true, EPI><<<grid, block, 0, st>>>(a);
+    else gemm_skinny_kernel<Tag, 4, false, EPI><<<grid, block, 0, st>>>(a);
+  }
+}
+
 template <typename Tag>
 static void launch_skinny(const SkinnyArgs& a, int epilogue, hipStream_t st) {
-  const dim3 block(kSkWaves * 64);
-  const bool u16 = g_skinny_u16 && (a.K / 32) % (16 * kSkWaves) == 0;
-  if (epilogue == 1 && u16) gemm_skinny_kernel<Tag, 1, 16, false, 1><<<dim3((a.N + 7) / 8), block, 0, st>>>(a);
-  else if (epilogue == 1) gemm_skinny_kernel<Tag, 1, 8, false, 1><<<dim3((a.N + 7) / 8), block, 0, st>>>(a);
-  else if (epilogue == 3) gemm_skinny_kernel<Tag, 1, 8, false, 3><<<dim3((a.N + 7) / 8), block, 0, st>>>(a);
-  else if (epilogue == 2) gemm_skinny_kernel<Tag, 1, 8, false, 2><<<dim3((a.N + 15) / 16), block, 0, st>>>(a);
-  else if (u16) gemm_skinny_kernel<Tag, 1, 16, false, 0><<<dim3((a.N + 15) / 16), block, 0, st>>>(a);
-  else if (g_skinny_nt) gemm_skinny_kernel<Tag, 1, 8, true, 0><<<dim3((a.N + 15) / 16), block, 0, st>>>(a);
-  else gemm_skinny_kernel<Tag, 1, 8, false, 0><<<dim3((a.N + 15) / 16), block, 0, st>>>(a);
+  if (epilogue == 1) launch_skinny_as<Tag, 1>(a, st);
+  else if (epilogue == 2) launch_skinny_as<Tag, 2>(a, st);
+  else if (epilogue == 3) launch_skinny_as<Tag, 3>(a, st);
+  else launch_skinny_as<Tag, 0>(a, st);
 }
 
 }  // namespace sp

@@ -292,14 +292,6 @@ struct GroupedArgs {
   float limit, alpha;                // ACT 3
 };
 
-// a * b rounded to fp32 before anything else happens to it: a product that is then rounded to fp16 would otherwise become one
-// v_fma_mixlo_f16, which rounds once - in one kernel and perhaps not in the next
-__device__ __forceinline__ float mul_f32(float a, float b) {
-  float r = a * b;
-  asm("" : "+v"(r));
-  return r;
-}
-
 // (shared by the separate launch and the fused epilogue, which agree bit for bit)
 __device__ __forceinline__ float moe_glu_f32(float g, float u, float limit, float alpha) {
   g = fminf(g, limit);

@@ -151,6 +151,14 @@ __device__ __forceinline__ float gelu_tanh_f32(float a) {
   return 0.5f * a * (1.0f + tanhf(0.7978845608028654f * (a + 0.044715f * a * a * a)));
 }
 
+// a * b rounded to fp32 before anything else happens to it: a product that is then rounded to fp16 would otherwise become one
+// v_fma_mixlo_f16, which rounds once - in one kernel and perhaps not in the next
+__device__ __forceinline__ float mul_f32(float a, float b) {
+  float r = a * b;
+  asm("" : "+v"(r));
+  return r;
+}
+
 // z * sigmoid(z) for results that are rounded to 16 bits: the hardware's exponential and reciprocal (1 ulp of fp32 each) in place
 // of the library's exponential and the divide's refinement, a quarter of their instructions.  fp32 results keep the exact form.
 template <typename Tag>
