@@ -728,6 +728,12 @@ SP_API int sp_head_delta_scan(void* out, int64_t out_stride, const void* q, int6
                               int64_t pre_stride, const float* dt_bias, const float* A_log, const float* norm_w, float* state,
                               int64_t state_stride, float* workspace, int64_t num_tokens, int heads, int kv_heads, int dim,
                               int vdim, int ranges, float eps, SP_SEQ_PARAMS, int dtype, void* stream);
+/* The same 16 tokens at a time, as sp_gated_delta_chunks: the same forms, work (sp_delta_chunk_floats) and raw. */
+SP_API int sp_head_delta_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                const void* v, int64_t v_stride, const void* gate, int64_t gate_stride, const float* pre,
+                                int64_t pre_stride, const float* dt_bias, const float* A_log, const float* norm_w, float* state,
+                                int64_t state_stride, float* work, float* raw, int64_t num_tokens, int heads, int kv_heads,
+                                int dim, int vdim, float eps, SP_SEQ_PARAMS, int dtype, void* stream);
 /* out[t, j] = gelu_tanh(x[t, j]) * x[t, d + j], gelu_tanh(z) = z / 2 (1 + tanh(sqrt(2 / pi) (z + 0.044715 z^3))) in fp32, the
  * product rounded once */
 SP_API int sp_gelu_tanh_and_mul(void* out, const void* x, int64_t num_tokens, int d, int64_t x_stride, int64_t out_stride,

@@ -170,6 +170,8 @@ SIGNATURES = {
     "sp_head_linear": (_i32, [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp]),
     "sp_head_delta_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64,
                                   _vp, _i64, _i32, _i32, _i32, _i32, _i32, _f32, *_SEQ, _i32, _vp]),
+    "sp_head_delta_chunks": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64,
+                                    _vp, _vp, _i64, _i32, _i32, _i32, _i32, _f32, *_SEQ, _i32, _vp]),
     "sp_gelu_tanh_and_mul": (_i32, [_vp, _vp, _i64, _i32, _i64, _i64, _i32, _vp]),
 }
 
@@ -1772,12 +1774,17 @@ def lowrank_gate(p: torch.Tensor, w2t: torch.Tensor, bias: Optional[torch.Tensor
 
 # mean tokens per request from which a delta rule's step runs 16 tokens at a time
 DELTA_CHUNK_MIN_TOKENS = 8
+# ... and with one decay per head, whose per-token kernel shares a head's columns out to more workgroups (16 heads of 128 x 128,
+# per-token against chunks, us): 8 requests of 4096 tokens together 364 / 179, one of 4096 2101 / 672, 16 of 300 41 / 33, one of
+# 65 tokens 42 / 27; 16 of 130 20 / 24, 4 of 64 20 / 26.
+HEAD_DELTA_CHUNK_MIN_TOKENS = 18
 
 
 def _delta_chunks_take(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay, seq: SeqParams, dim: int, vdim: int) -> bool:
-    """the forms sp_gated_delta_chunks / sp_head_delta_chunks are built for"""
+    """the forms sp_gated_delta_chunks / sp_head_delta_chunks (decay None) are built for"""
     per = 4 if q.dtype == torch.float32 else 8
-    return (seq.extend_seq_lens is not None and seq.num_tokens >= DELTA_CHUNK_MIN_TOKENS * seq.batch_size and dim in (64, 128)
+    least = HEAD_DELTA_CHUNK_MIN_TOKENS if decay is None else DELTA_CHUNK_MIN_TOKENS
+    return (seq.extend_seq_lens is not None and seq.num_tokens >= least * seq.batch_size and dim in (64, 128)
             and vdim % 16 == 0 and q.stride(0) % per == 0 and k.stride(0) % per == 0 and q.data_ptr() % 16 == 0
             and k.data_ptr() % 16 == 0 and (decay is None or decay.data_ptr() % 16 == 0))
 
@@ -1834,9 +1841,17 @@ def head_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: tor
     if _mat(pre, "pre").dtype != torch.float32 or pre.shape != (T, 2 * heads) or dt_bias.numel() != heads or \
             A_log.numel() != heads or norm_w.numel() != vdim or state.shape[1:] != (heads, dim, vdim):
         raise RuntimeError("head_delta_scan: pre fp32 [T, 2 H], dt_bias / A_log [H], norm_w [Dv], state [slots, H, D, Dv]")
+    out = empty_rows(T, heads * vdim, q.dtype, q.device)
+    if ranges is None and _delta_chunks_take(q, k, v, None, seq, dim, vdim):
+        work, raw = _delta_chunk_buffers(seq, heads, vdim, q.device)
+        _check(load().sp_head_delta_chunks(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
+                                           v.data_ptr(), v.stride(0), gate.data_ptr(), gate.stride(0), pre.data_ptr(),
+                                           pre.stride(0), dt_bias.data_ptr(), A_log.data_ptr(), norm_w.data_ptr(),
+                                           state.data_ptr(), state.stride(0), work.data_ptr(), raw.data_ptr(), T, heads, kv_heads,
+                                           dim, vdim, eps, *seq.args, _dt(q), _stream()), "sp_head_delta_chunks")
+        return out
     if ranges is None:          # decode steps (one token per request) keep the norm and the gate in the scan
         ranges = 1 if T <= seq.batch_size else max(1, min(HEAD_DELTA_WORKGROUPS // max(1, seq.batch_size * heads), vdim // 32))
-    out = empty_rows(T, heads * vdim, q.dtype, q.device)
     ws = torch.empty(T * heads * vdim, dtype=torch.float32, device=q.device) if ranges > 1 else None
     _check(load().sp_head_delta_scan(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                                      v.data_ptr(), v.stride(0), gate.data_ptr(), gate.stride(0), pre.data_ptr(), pre.stride(0),

@@ -20,6 +20,7 @@
 // per token left the per-token kernels at a quarter of that.  16 heads of 128 x 128 with a decay per channel: 8 requests of 4096
 // tokens together 682 -> 183 us (49 of them the preparation, 21 norm and gate), one request of 4096 tokens 4258 -> 725, 16 requests
 // of 300 tokens 45 -> 33; below 8 tokens per request the per-token kernel is the faster one (1 token: 39 against 51 us).
+// With one decay per head: 8 requests 364 -> 179, one request 2101 -> 672, 16 requests of 300 tokens 41 -> 33.
 //
 // A value that is not finite reaches the other tokens of its chunk too (zero weights times it), not only the later ones.
 #pragma once
@@ -485,3 +486,8 @@ int launch_delta_chunks(DeltaChunks a, const SeqBatch& s, hipStream_t st) {
 }
 
 }  // namespace sp
+
+// (weak: both delta rules' sources define it, a library may hold either or both)
+extern "C" __attribute__((weak)) int64_t sp_delta_chunk_floats(int64_t num_tokens, int batch_size, int heads) {
+  return (num_tokens / sp::kDC + batch_size) * heads * sp::kDcFloats;
+}

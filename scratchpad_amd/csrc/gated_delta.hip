@@ -387,10 +387,6 @@ extern "C" int sp_gated_delta_scan(void* out, int64_t out_stride, const void* q,
                                                            vdim, eps, (hipStream_t)stream)));
 }
 
-extern "C" int64_t sp_delta_chunk_floats(int64_t num_tokens, int batch_size, int heads) {
-  return (num_tokens / sp::kDC + batch_size) * heads * sp::kDcFloats;
-}
-
 extern "C" int sp_gated_delta_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k,
                                      int64_t k_stride, const void* v, int64_t v_stride, const void* bpre, int64_t b_stride,
                                      const float* decay, const float* gate, const float* norm_w, float* state,

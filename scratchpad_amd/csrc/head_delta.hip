@@ -15,7 +15,7 @@
 // With one range per head the norm and the gate are the pass's epilogue; where a step brings long portions of few requests,
 // several workgroups share a head and hand fp32 read-outs to head_norm_gate_kernel.  Prompt portions and single decoded
 // tokens take the same path, and the order of every sum depends on the head's sizes only.
-#include "seq_batch.h"
+#include "chunk_delta.h"
 
 namespace sp {
 namespace {
@@ -419,4 +419,35 @@ extern "C" int sp_head_delta_scan(void* out, int64_t out_stride, const void* q, 
   if (dim <= 64) SP_DISPATCH_DTYPE(dtype, return (launch_hd<Tag, 64>(a, s, ranges, vec, num_tokens, st)));
   if (dim <= 128) SP_DISPATCH_DTYPE(dtype, return (launch_hd<Tag, 128>(a, s, ranges, vec, num_tokens, st)));
   SP_DISPATCH_DTYPE(dtype, return (launch_hd<Tag, 256>(a, s, ranges, vec, num_tokens, st)));
+}
+
+extern "C" int sp_head_delta_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k,
+                                    int64_t k_stride, const void* v, int64_t v_stride, const void* gate, int64_t gate_stride,
+                                    const float* pre, int64_t pre_stride, const float* dt_bias, const float* A_log,
+                                    const float* norm_w, float* state, int64_t state_stride, float* work, float* raw,
+                                    int64_t num_tokens, int heads, int kv_heads, int dim, int vdim, float eps, SP_SEQ_PARAMS,
+                                    int dtype, void* stream) {
+  SP_CHECK_ARG(batch_size >= 0 && num_tokens >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && dim > 0 && vdim > 0);
+  if (batch_size == 0 || num_tokens == 0) return SP_OK;
+  SP_CHECK_ARG(out && q && k && v && gate && pre && dt_bias && A_log && norm_w && state && work && raw && req_pool_indices && seq_lens);
+  SP_CHECK_ARG(!extend_seq_lens || (extend_prefix_lens && extend_start_loc));
+  SP_CHECK_ARG(state_stride >= (int64_t)heads * dim * vdim && pre_stride >= 2 * (int64_t)heads);
+  SP_CHECK_ARG(q_stride >= (int64_t)kv_heads * dim && k_stride >= (int64_t)kv_heads * dim);
+  SP_CHECK_ARG(v_stride >= (int64_t)heads * vdim && out_stride >= (int64_t)heads * vdim && gate_stride >= (int64_t)heads * vdim);
+  if (vdim > kHdMaxV || heads > 65535) return SP_ERR_UNSUPPORTED;
+  SEQ_BATCH(s);
+  const DeltaChunks c{q, k, v, nullptr, nullptr, pre, dt_bias, A_log, state, work, raw, q_stride, k_stride, v_stride, 0, pre_stride,
+                      state_stride, num_tokens, heads, kv_heads, vdim, vdim};
+  if (!delta_chunks_take(c, dim, dtype, s)) return SP_ERR_UNSUPPORTED;
+  hipStream_t st = (hipStream_t)stream;
+  int rc = SP_OK;
+  SP_DISPATCH_DTYPE(dtype, rc = (dim == 64 ? launch_delta_chunks<Tag, 64, false>(c, s, st) : launch_delta_chunks<Tag, 128, false>(c, s, st)));
+  if (rc != SP_OK) return rc;
+  const HeadDelta a{out, raw, q, k, v, gate, pre, dt_bias, A_log, norm_w, state, out_stride, q_stride, k_stride, v_stride, gate_stride,
+                    pre_stride, state_stride, heads, kv_heads, dim, vdim, vdim, eps};
+  const int64_t jobs = num_tokens * heads;
+  SP_DISPATCH_DTYPE(dtype, (head_norm_gate_kernel<Tag><<<dim3((unsigned)((jobs + kBlock / 64 - 1) / (kBlock / 64))), kBlock, 0, st>>>(
+                               a, jobs)));
+  SP_LAUNCH_CHECK();
+  return SP_OK;
 }

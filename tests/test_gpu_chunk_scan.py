@@ -163,3 +163,35 @@ def test_lowrank_gate_of_many_tokens(T, rank, channels):
     # a decay moves by its exponent's error: fp32 sums of `rank` products, a few ulp of exponential and logarithm
     assert ((_native.lowrank_gate(p, w2t, bias, "decay", A).double() - want).abs() <= 4e-6).all()
     assert ((_native.lowrank_gate(p, w2t, None, "sigmoid").double() - torch.sigmoid(p.double() @ w2t.double())).abs() <= 2e-6).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lens", [[18], [15, 32, 17], [48, 1, 33, 2], [16, 200, 3]], ids=lambda l: "-".join(map(str, l)))
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 1, 128, 128), (4, 4, 64, 64), (3, 3, 128, 48), (2, 2, 64, 256)])
+def test_head_delta_chunks_against_the_per_token_kernel(lens, H, G, D, Dv, dtype):
+    """Both orders of the same fp32 sums: S within 2e-5 of its largest value, as the channel-gated form is held to, and the normed
+    read-outs within two roundings of the result"""
+    from scratchpad_amd import _native
+    announce("head delta chunks", dtype, lens, H, G, D, Dv)
+    g = torch.Generator(device=DEV).manual_seed(6)
+    T, slots = sum(lens), slots_of(lens)
+    S = torch.full((2 * len(lens) + 1, H, D, Dv), float("nan"), device=DEV)
+    S2 = S.clone()
+    nw, dt_bias, A_log = (torch.rand(n, generator=g, device=DEV) for n in (Dv, H, H))
+    for prefixes in ([0] * len(lens), lens):
+        q, k, v, gate = (torch.randn(T, n, generator=g, device=DEV).to(dtype) for n in (G * D, G * D, H * Dv, H * Dv))
+        pre = torch.randn(T, 2 * H, generator=g, device=DEV)
+        pre[T // 2, H:] = 60.0                                                     # a head forgotten all but exactly
+        seq = seq_extend(lens, prefixes, slots)
+        assert _native._delta_chunks_take(q, k, v, None, seq, D, Dv) == (T >= 18 * len(lens))
+        if T < 18 * len(lens):
+            return
+        args = (q, k, v, gate, pre, dt_bias, A_log, nw)
+        out = _native.head_delta_scan(*args, S, seq, H, G, D, Dv, 1e-5)
+        want = _native.head_delta_scan(*args, S2, seq, H, G, D, Dv, 1e-5, ranges=1)
+        for slot in slots:
+            near(S[slot], S2[slot].double(), 2e-5)
+        bar = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -9, torch.float32: 1e-4}[dtype]
+        assert ((out.double() - want.double()).abs() <= bar * want.double().abs() + 1e-3).all()
+    for slot in range(0, 2 * len(lens) + 1, 2):
+        assert torch.isnan(S[slot]).all()
