@@ -301,7 +301,7 @@ def instrument(clock: KernelClock, cfg):
              "embed_scale": embed, "norm_shift": io, "stream_add": io, "qkv_rotary_store": io, "pool_blocks": io,
              "window_attention": window, "small_linear_f32": small, "causal_conv_silu": io, "mamba2_scan": scan,
              "gated_group_norm": io, "mlstm_scan": mlstm, "moe_route_softmax": io,
-             "gated_add_norm": io, "relu_square": io, "scale_softcap": io, "delta_gates": io, "delta_recurrence": delta,
+             "gated_add_norm": io, "relu_square": io, "scale_softcap": io, "delta_gates": io, "delta_recurrence": delta, "delta_step": delta,
              "hgrn2_scan": hgrn, "linear_relu_square": gemm, "post_norm": join, "add_group_norm": io, "lowrank_gate": lowrank, "gated_delta_scan": gdelta,
              "latent_rotate_query": io, "head_linear": heads, "head_delta_scan": hdelta, "gelu_tanh_and_mul": io, "_skinny_glu": glu}
     for name, cost in costs.items():

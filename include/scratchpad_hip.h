@@ -650,6 +650,13 @@ SP_API int sp_delta_recurrence(void* out, int64_t out_stride, const void* r, int
                                const float* decay, const float* remove, const float* norm_w, float* state,
                                int64_t state_stride, int heads, int head_dim, float eps, SP_SEQ_PARAMS, int dtype,
                                void* stream);
+/* sp_delta_gates and sp_delta_recurrence of a decode step (one token per request) as one launch: head_dim 64 or 128, rank <= 512,
+ * else SP_ERR_UNSUPPORTED and nothing is launched. */
+SP_API int sp_delta_step(void* out, int64_t out_stride, const void* r, int64_t r_stride, const void* k, int64_t k_stride,
+                         const void* v, int64_t v_stride, const void* g, int64_t g_stride, const void* p, int64_t p_stride,
+                         const void* apre, int64_t a_stride, const float* w2t, const float* w0, const float* a_bias, int rank,
+                         float rate, const float* norm_w, float* state, int64_t state_stride, int heads, int head_dim,
+                         float eps, SP_SEQ_PARAMS, int dtype, void* stream);
 /* Per (request, head) over the request's rows in order, S [dim, vdim] fp32 from state[request slot] and back:
  *   q = silu(qpre);  f = lower + (1 - lower) sigmoid(fpre + f_bias);  S = diag(f) S + (1 - f) v^T;  o = S^T q
  *   out = o / rms_head(o) * norm_w   (norm_w [vdim], shared by the heads).  dim, vdim <= 256.                          */

@@ -153,6 +153,8 @@ SIGNATURES = {
     "sp_delta_gates": (_i32, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i32, _i32, _f32, _i32, _vp]),
     "sp_delta_recurrence": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i32, _i32,
                                    _f32, *_SEQ, _i32, _vp]),
+    "sp_delta_step": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i32, _f32,
+                             _vp, _vp, _i64, _i32, _i32, _f32, *_SEQ, _i32, _vp]),
     "sp_hgrn2_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _f32,
                              *_SEQ, _i32, _vp]),
     # ---- ABI 13
@@ -1702,6 +1704,30 @@ def delta_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch
                                       v.data_ptr(), v.stride(0), g.data_ptr(), g.stride(0), decay.data_ptr(), remove.data_ptr(),
                                       norm_w.data_ptr(), state.data_ptr(), state.stride(0), heads, dim, eps, *seq.args,
                                       _dt(r), _stream()), "sp_delta_recurrence")
+    return out
+
+
+def delta_step(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, p: torch.Tensor, apre: torch.Tensor,
+               w2t: torch.Tensor, w0: torch.Tensor, a_bias: torch.Tensor, rate: float, norm_w: torch.Tensor, state: torch.Tensor,
+               seq: SeqParams, heads: int, dim: int, eps: float) -> torch.Tensor:
+    """delta_gates, then delta_recurrence; one launch for a decode step with heads of 64 or 128 (the gates' and the heads' sums
+    then run in other orders)"""
+    T, n, rank = seq.num_tokens, heads * dim, p.shape[1]
+    if seq.extend_seq_lens is not None or dim not in (64, 128) or rank > 512:
+        decay, remove = delta_gates(p, w2t, w0, apre, a_bias, rate)
+        return delta_recurrence(r, k, v, g, decay, remove, norm_w, state, seq, heads, dim, eps)
+    for name, t, w in (("r", r, n), ("k", k, n), ("v", v, n), ("g", g, n), ("apre", apre, n), ("p", p, rank)):
+        if _mat(t, name).shape != (T, w) or t.dtype != r.dtype:
+            raise RuntimeError(f"delta_step: {name} must be [num_tokens, {w}] of one dtype")
+    for name, t in (("w2t", w2t), ("w0", w0), ("a_bias", a_bias), ("norm_w", norm_w), ("state", state)):
+        _f32(t, name)
+    if w2t.shape != (rank, n) or w0.numel() != n or a_bias.numel() != n or norm_w.numel() != n or state.shape[1:] != (heads, dim, dim):
+        raise RuntimeError("delta_step: w2t [rank, H*D], w0, a_bias, norm_w [H*D], state [slots, H, D, D]")
+    out = empty_rows(T, n, r.dtype, r.device)
+    _check(load().sp_delta_step(out.data_ptr(), out.stride(0), r.data_ptr(), r.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(),
+                                v.stride(0), g.data_ptr(), g.stride(0), p.data_ptr(), p.stride(0), apre.data_ptr(), apre.stride(0),
+                                w2t.data_ptr(), w0.data_ptr(), a_bias.data_ptr(), rank, rate, norm_w.data_ptr(), state.data_ptr(),
+                                state.stride(0), heads, dim, eps, *seq.args, _dt(r), _stream()), "sp_delta_step")
     return out
 
 

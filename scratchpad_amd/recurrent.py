@@ -166,11 +166,10 @@ class GeneralDeltaMixer(nn.Module):
         seq, states = forward_batch.attn_backend.seq, forward_batch.state_pool
         n = self.heads * self.dim
         a = _native.linear(h, self.in_proj)
-        decay, remove = _native.delta_gates(a[:, 5 * n:5 * n + self.rank], self.w2t.data, self.w0.data, a[:, 4 * n:5 * n],
-                                            self.a_bias.data, self.rate)
         S = states.state(self.layer_id if state_id is None else state_id, "S")
-        o = _native.delta_recurrence(a[:, :n], a[:, n:2 * n], a[:, 2 * n:3 * n], a[:, 3 * n:4 * n], decay, remove,
-                                     self.norm.data, S, seq, self.heads, self.dim, self.eps)
+        o = _native.delta_step(a[:, :n], a[:, n:2 * n], a[:, 2 * n:3 * n], a[:, 3 * n:4 * n], a[:, 5 * n:5 * n + self.rank],
+                               a[:, 4 * n:5 * n], self.w2t.data, self.w0.data, self.a_bias.data, self.rate, self.norm.data, S, seq,
+                               self.heads, self.dim, self.eps)
         y = _native.linear(o, self.o)
         return (y, a[:, 5 * n + self.rank:]) if self.extra_rows else y
 
