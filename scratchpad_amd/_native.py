@@ -1542,7 +1542,7 @@ def window_attention(q: torch.Tensor, kpool: torch.Tensor, vpool: torch.Tensor, 
     return out
 
 
-SMALL_LINEAR_OWN_ROWS = 64      # up to this many rows small_linear_f32 runs on the library's own kernel
+SMALL_LINEAR_OWN_ROWS = 64      # up to this many rows a workgroup per row; above, tiles where there are any for the type
 
 
 def small_linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -1550,8 +1550,10 @@ def small_linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     _mat(x, "x"), _f32(weight, "weight")
     if weight.dim() != 2 or weight.shape[1] != x.shape[1] or (bias is not None and _f32(bias, "bias").shape[0] != weight.shape[0]):
         raise RuntimeError("small_linear_f32: weight [n, k], bias [n]")
-    if x.shape[0] > SMALL_LINEAR_OWN_ROWS:
-        # many rows: the own kernel reads the weight rows again for every token; the library's fp32 product tiles them
+    if x.shape[0] > SMALL_LINEAR_OWN_ROWS and not (x.dtype == torch.bfloat16 and x.shape[1] % 32 == 0 and x.stride(0) % 8 == 0
+                                                   and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
+        # many rows of types or lengths without a tiled form (see sp_small_linear_f32): the kernel for few reads the weight rows
+        # again for every token, the library's fp32 product tiles them
         return torch.nn.functional.linear(x.to(torch.float32), weight, bias)
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=x.device)
     _check(load().sp_small_linear_f32(out.data_ptr(), x.data_ptr(), x.stride(0), weight.data_ptr(), _ptr(bias), x.shape[0],

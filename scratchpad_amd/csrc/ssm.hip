@@ -61,6 +61,91 @@ small_linear_f32_kernel(float* out, const void* x, int64_t x_stride, const float
   }
 }
 
+// The same for many rows of bf16 x, on the matrix cores with nothing rounded on the way: a weight is three bf16 parts whose sum is
+// exact (split3), x is bf16 already, the sums are fp32.  A workgroup takes 32 tokens x 16 NT outputs; its 8 waves share K (a
+// stretch each, two 32-deep steps of it in flight) and add up through LDS in wave order.  4096 tokens x 2048, us, with the library's
+// fp32 product behind a copy of x to fp32 -> now: 64 outputs 29.3 -> 14.9, 32 outputs 27.0 -> 10.2; 65 rows of 64 outputs
+// 24.8 -> 9.7.  (A weight or value that is not finite makes the sums it enters NaN, infinite ones too.)
+constexpr int kLinTokens = 32, kLinWaves = 8;
+template <int NT>
+__global__ void __launch_bounds__(kLinWaves * 64)
+linear_f32_mfma_kernel(float* out, const char* x, int64_t x_stride, const float* w, const float* bias, int64_t T, int K, int N) {
+  constexpr int MT = kLinTokens / 16, U = 2, ROW = 16 * NT + 4;
+  __shared__ __attribute__((aligned(16))) float part[kLinWaves / 2][kLinTokens][ROW];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, q = lane >> 4;
+  const int64_t t0 = (int64_t)blockIdx.x * kLinTokens;
+  const int n0 = blockIdx.y * 16 * NT;
+  const char* xp[MT];
+  const float* wp[NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xp[i] = x + ((t0 + 16 * i + r16 < T ? t0 + 16 * i + r16 : T - 1) * x_stride + 8 * q) * 2;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) wp[j] = w + (int64_t)min(n0 + 16 * j + r16, N - 1) * K + 8 * q;      // (rows past N: never stored)
+  f32x4_c acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_c{0.f, 0.f, 0.f, 0.f};
+  const int steps = K / 32, mine = (steps + kLinWaves - 1) / kLinWaves;
+  const int first = wave * mine, last = min(first + mine, steps);
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  for (int ks = first; ks < last; ks += U) {
+    u32x4 xf[U][MT], wf[U][NT][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = ks + u < last;
+      const int64_t k = (int64_t)(ks + u) * 32;
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) wf[u][j][h] = in ? ld16(wp[j] + k + 4 * h) : zero;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) xf[u][i] = in ? ld16(xp[i] + k * 2) : zero;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        u32x4 b[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          uint32_t hi, mid, lo;
+          split3(as_f32(wf[u][j][e / 2][2 * (e & 1)]), as_f32(wf[u][j][e / 2][2 * (e & 1) + 1]), hi, mid, lo);
+          b[0][e] = hi, b[1][e] = mid, b[2][e] = lo;
+        }
+#pragma unroll
+        for (int c = 2; c >= 0; --c)
+#pragma unroll
+          for (int i = 0; i < MT; ++i) acc[i][j] = mfma_c(xf[u][i], b[c], acc[i][j]);
+      }
+  }
+  // lane (r16, q): tokens 16 i + 4 q + r, output 16 j + r16; waves 4-7 first, then 0-3 add their own
+#pragma unroll
+  for (int half = 1; half >= 0; --half) {
+    if (wave / (kLinWaves / 2) == half) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float* to = &part[wave % (kLinWaves / 2)][16 * i + 4 * q + r][16 * j + r16];
+            *to = half ? acc[i][j][r] : acc[i][j][r] + *to;
+          }
+    }
+    __syncthreads();
+  }
+  for (int e = tid; e < kLinTokens * 16 * NT; e += kLinWaves * 64) {
+    const int t = e / (16 * NT), n = e % (16 * NT);
+    if (t0 + t >= T || n0 + n >= N) continue;
+    float v = 0.f;
+#pragma unroll
+    for (int u = 0; u < kLinWaves / 2; ++u) v += part[u][t][n];
+    out[(t0 + t) * N + n0 + n] = v + (bias ? bias[n0 + n] : 0.f);
+  }
+}
+
 // state [slot][taps - 1][C]: entry k = the input at position (tokens held) - (taps - 1) + k
 template <typename Tag>
 __global__ void __launch_bounds__(kBlock)
@@ -499,6 +584,21 @@ extern "C" int sp_small_linear_f32(float* out, const void* x, int64_t x_stride, 
   SP_CHECK_ARG(num_tokens >= 0 && k > 0 && n > 0);
   if (num_tokens == 0) return SP_OK;
   SP_CHECK_ARG(out && x && weight && x_stride >= k);
+  if (num_tokens > 64 && dtype == SP_BF16 && k % 32 == 0 && x_stride % 8 == 0 && (((uintptr_t)x | (uintptr_t)weight) & 15) == 0) {
+    // (up to 64 rows a workgroup per row has the shorter chain.)  16 outputs a workgroup while that leaves a CU one of them, 32
+    // beyond: the chain over K is half as long (4096 rows of 32 outputs: 10.2 against 14.3 us), x and the weights are read twice
+    // as often (16384 rows of 64: 59.7 against 46.7).
+    const int64_t rows = (num_tokens + kLinTokens - 1) / kLinTokens;
+    const int nt = rows * ((n + 15) / 16) <= 256 ? 1 : 2;
+    const dim3 tiles((unsigned)rows, (unsigned)((n + 16 * nt - 1) / (16 * nt)));
+#define SP_LIN(NT) \
+  linear_f32_mfma_kernel<NT><<<tiles, kLinWaves * 64, 0, (hipStream_t)stream>>>(out, (const char*)x, x_stride, weight, bias, num_tokens, k, n)
+    if (nt == 1) SP_LIN(1);
+    else SP_LIN(2);
+#undef SP_LIN
+    SP_LAUNCH_CHECK();
+    return SP_OK;
+  }
   const dim3 grid((unsigned)num_tokens, (unsigned)((n + 15) / 16));
   if (k % 4 == 0 && ((uintptr_t)weight & 15) == 0)
     SP_DISPATCH_DTYPE(dtype, (small_linear_f32_kernel<Tag, true><<<grid, 256, 0, (hipStream_t)stream>>>(

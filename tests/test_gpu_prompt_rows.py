@@ -88,3 +88,19 @@ def test_causal_conv_runs(lens, prefixes, C, taps, dtype):
     bar = 2.0 ** -8 if dtype == torch.bfloat16 else 1e-5
     # (a silu near its zero takes the absolute error of the sum before it)
     assert ((got.double() - want).abs() <= bar * want.abs() + 4e-6).all()
+
+
+@pytest.mark.parametrize("T", [65, 96, 257])
+@pytest.mark.parametrize("K,n,bias", [(32, 1, True), (288, 16, False), (2048, 31, True), (1024, 64, False), (544, 131, True)])
+def test_fp32_products_of_many_rows(T, K, n, bias):
+    """fp32 weights of all magnitudes against 64 bits: K fp32 additions and roundings of exact products"""
+    from scratchpad_amd import _native
+    g = torch.Generator(device=DEV).manual_seed(T + K + n)
+    wide = torch.randn(T, K + 8, generator=g, device=DEV).bfloat16()
+    x = wide[:, 8:]                                                       # a view, 16-byte aligned rows
+    w = torch.randn(n, K, generator=g, device=DEV) * torch.exp2(torch.randint(-30, 31, (n, 1), generator=g, device=DEV).float())
+    b = torch.randn(n, generator=g, device=DEV) if bias else None
+    out = _native.small_linear_f32(x, w, b)
+    want = x.double() @ w.double().T + (b.double() if bias else 0.0)
+    bound = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + (b.double().abs() if bias else 0.0))
+    assert out.shape == (T, n) and bool(((out.double() - want).abs() <= bound).all())
