@@ -16,15 +16,15 @@ namespace sp {
 
 static constexpr int kBlock = 256;
 
+// (once per kernel; the barrier leaves the residual's stores and the weights' loads under way)
 __device__ __forceinline__ float block_sum(float v, float* smem) {
   v = wave_sum(v);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0) smem[wave] = v;
-  __syncthreads();
+  lds_barrier();
   float t = 0.f;
 #pragma unroll
   for (int i = 0; i < kBlock / 64; ++i) t += smem[i];
-  __syncthreads();
   return t;
 }
 

@@ -224,18 +224,25 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // ---- wave reductions ------------------------------------------------------------------------
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-// sum over N neighbouring lanes (aligned groups of N = 1, 2, 4, 8 or 16) by data-parallel-primitive moves - register-to-register,
-// no trip through the LDS crossbar that __shfl_xor takes; every lane of a group ends with the same value
+// Sums over lanes by data-parallel-primitive moves and lane swaps - register to register, no trip through the LDS crossbar that
+// __shfl_xor takes (some 60 cycles of latency each against 8).
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
+// over the wave, whose lanes must all be active; every lane ends with the same value (the additions of an exchange with lane ^ 32,
+// then ^ 16, 8, 4, 2, 1)
+__device__ __forceinline__ float wave_sum(float v) {
+  const auto h = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);      // lanes 0-31 twice, lanes 32-63 twice
+  v = as_f32(h[0]) + as_f32(h[1]);
+  const auto r = __builtin_amdgcn_permlane16_swap(as_u32(v), as_u32(v), false, false);      // even rows of 16 twice, odd rows twice
+  v = as_f32(r[0]) + as_f32(r[1]);
+  v += dpp_f32<0x128>(v);                           // row_ror 8: lane ^ 8
+  v += dpp_f32<0x124>(v);                           // row_ror 4: the value of lane ^ 4, since lanes 8 apart hold the same by now
+  v += dpp_f32<0x4E>(v);                            // quad_perm [2,3,0,1]: lane ^ 2
+  return v + dpp_f32<0xB1>(v);                      // quad_perm [1,0,3,2]: lane ^ 1
+}
+// over N neighbouring lanes (aligned groups of N = 1, 2, 4, 8 or 16)
 template <int N>
 __device__ __forceinline__ float lanes_sum(float v) {
   static_assert(N == 1 || N == 2 || N == 4 || N == 8 || N == 16, "lanes per group");
