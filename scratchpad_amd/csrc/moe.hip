@@ -362,6 +362,29 @@ __device__ __forceinline__ bool grouped_tile(const int32_t* offsets, int E, int 
   return false;
 }
 
+// The same for a launch of `cols` column tiles per row tile, an expert's row tiles next to each other: the column tile as well.
+__device__ __forceinline__ bool grouped_tile_by_column(const int32_t* offsets, int E, int bm, int cols, int at, int lane, int& e_out,
+                                                       int& row0, int& rows_end, int& col) {
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane;
+    const int lo = e < E ? offsets[e] : 0, hi = e < E ? offsets[e + 1] : 0;
+    const int tiles = (hi - lo + bm - 1) / bm, incl = wave_inclusive(tiles * cols, lane);
+    const uint64_t hit = __ballot(at < incl);
+    if (hit) {
+      const int l = __ffsll((unsigned long long)hit) - 1;
+      e_out = e0 + l;
+      const int n = __builtin_amdgcn_readfirstlane(__shfl(tiles, l, 64));
+      const int in = __builtin_amdgcn_readfirstlane(at - __shfl(incl - tiles * cols, l, 64));
+      col = in / n;
+      row0 = __builtin_amdgcn_readfirstlane(__shfl(lo, l, 64)) + (in - col * n) * bm;
+      rows_end = __builtin_amdgcn_readfirstlane(__shfl(hi, l, 64));
+      return true;
+    }
+    at -= __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
+  }
+  return false;
+}
+
 // Steps with many rows per expert: BM rows x 128 weight rows per workgroup, k in steps of 64.  Both operands go to LDS by
 // direct loads (16 bytes per lane, no registers on the way), one step ahead of the MFMAs, in two buffers; a step costs one
 // barrier.  LDS rows are 128 bytes whose eight 16-byte chunks are permuted by the row's number (the SOURCE address is
@@ -487,6 +510,105 @@ __global__ void __launch_bounds__(256, 2) moe_grouped_tile_kernel(GroupedArgs p)
   }
 }
 
+// Steps with hundreds of rows per expert: 128 rows x 256 weight rows per workgroup, a wave 64 x 128 of them, k in steps of 32.
+// What the 128 x 128 tiles wait for is LDS (a wave reads 8 KB for 16 products of 16 cycles: 128 bytes per cycle for the four of
+// them, all there is) and the L2 (64 bytes per cycle and CU); here it is 96 and 48.  A step's operands are 24 KB, double-buffered,
+// so three workgroups share a CU and fill each other's waits.  The row tiles of one column tile follow each other: the weights
+// they share are in the L2 once.  LDS rows are 64 bytes; the chunk of a row is permuted by its number / 4, so that the 16 rows of a
+// fragment read lie in 64 banks.  Width 2048, 32 experts of ff 1024, up + down in us, 128 x 128 tiles -> these: 512 rows per
+// expert 336 -> 315 (three buffers and two workgroups: 323; column tiles of a row tile next to each other: 330), 256 rows
+// 215 -> 217, 96 rows 105 -> 123.  (Experts that start at k of their own, so that the XCDs ask for different pieces of their rows
+// at a time: 311, but a row's bits would then depend on its neighbours' number.)
+constexpr int kWideBM = 128, kWideBN = 256, kWideBK = 32;
+template <typename Tag, int ACT>
+__global__ void __launch_bounds__(256, 3) moe_grouped_wide_kernel(GroupedArgs p) {
+  constexpr bool GLU = ACT >= 2;
+  constexpr int CPW = kWideBN / 2, FM = 4, FN = CPW / 16, OUT_N = GLU ? kWideBN / 2 : kWideBN;
+  constexpr int LA = kWideBM / 64, LB = kWideBN / 64;            // direct loads per wave and step
+  constexpr int kBuf = (kWideBM + kWideBN) * kWideBK * 2;
+  extern __shared__ __attribute__((aligned(16))) char wide_lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+  const int ntiles = (p.N + OUT_N - 1) / OUT_N;
+  const int total = grouped_tiles(p.offsets, p.E, kWideBM, lane) * ntiles, share = (total + 7) / 8;
+  const int idx = (int)(blockIdx.x >> 3), at = (int)(blockIdx.x & 7) * share + idx;
+  if (idx >= share || at >= total) return;
+  int e = 0, row0 = 0, rows_end = 0, col = 0;
+  if (!grouped_tile_by_column(p.offsets, p.E, kWideBM, ntiles, at, lane, e, row0, rows_end, col)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  const int n0 = col * OUT_N;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int wrows = GLU ? 2 * p.N : p.N;
+  // sources of this wave's direct loads: lane -> row lane / 4 of the 16 rows of a load, chunk lane % 4 of LDS
+  const int chunk = (lane & 3) ^ (lane >> 4);
+  const char* src[LA + LB];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) {
+    const int pos = min(row0 + (wave * LA + i) * 16 + (lane >> 2), rows_end - 1);     // rows past the end: never stored
+    const int64_t arow = p.order ? p.order[pos] / p.row_div : pos;
+    src[i] = p.a + arow * p.a_stride * 2 + chunk * 16;
+  }
+  const char* wbase = p.w + (int64_t)e * wrows * p.K * 2 + chunk * 16;
+#pragma unroll
+  for (int i = 0; i < LB; ++i) {
+    const int br = (wave * LB + i) * 16 + (lane >> 2);
+    int row;
+    if constexpr (GLU) {
+      const int in = br % CPW, n = n0 + (br / CPW) * (CPW / 2) + in % (CPW / 2);
+      row = min(n, p.N - 1) + (in >= CPW / 2 ? p.N : 0);
+    } else {
+      row = min(n0 + br, p.N - 1);
+    }
+    src[LA + i] = wbase + (int64_t)row * p.K * 2;
+  }
+  const int steps = p.K / kWideBK;
+  const auto stage = [&](char* lds, int step) {
+#pragma unroll
+    for (int i = 0; i < LA + LB; ++i) {
+      char* dst = lds + (i < LA ? (wave * LA + i) : (kWideBM / 16 + wave * LB + i - LA)) * 1024;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + step * (kWideBK * 2)),
+                                       (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    }
+  };
+  f32x4_q acc[FM][FN];
+#pragma unroll
+  for (int f = 0; f < FM; ++f)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[f][j] = f32x4_q{0.f, 0.f, 0.f, 0.f};
+  const int c = (q ^ (r16 >> 2)) * 16;
+  const int arow0 = (wm * 64 + r16) * 64 + c, brow0 = (kWideBM + wn * CPW + r16) * 64 + c;
+  char *now = wide_lds, *next = wide_lds + kBuf;
+  stage(now, 0);
+  for (int s = 0; s < steps; ++s) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (s + 1 < steps) stage(next, s + 1);
+    u32x4 xf[FM], wf[FN];
+#pragma unroll
+    for (int f = 0; f < FM; ++f) xf[f] = ld16(now + arow0 + f * 1024);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) wf[j] = ld16(now + brow0 + j * 1024);
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int f = 0; f < FM; ++f) acc[f][j] = mfma_q<Tag>(wf[j], xf[f], acc[f][j]);
+    char* const t = now;
+    now = next, next = t;
+  }
+  constexpr int FO = GLU ? FN / 2 : FN;
+#pragma unroll
+  for (int f = 0; f < FM; ++f) {
+    const int pos = row0 + wm * 64 + 16 * f + r16;
+    if (pos >= rows_end) continue;
+#pragma unroll
+    for (int j = 0; j < FO; ++j) {
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = grouped_act<Tag, ACT>(acc[f][j][r], GLU ? acc[f][j + FN - FO][r] : 0.f, p);
+      store4<Tag>(p, pos, n0 + wn * (GLU ? CPW / 2 : CPW) + 16 * j + 4 * q, v);
+    }
+  }
+}
+
 // Steps with a few rows per expert (decode): a stream of the chosen experts' weights.  One wave per 16 rows x 32 weight rows
 // (GLU: 16 gate rows and their 16 up rows), operands straight from global memory, kRowsUnroll k-steps of loads in flight.
 // Single waves spread evenly over the 1024 SIMDs whatever the number of chosen experts; nothing is shared between them.
@@ -545,6 +667,7 @@ __global__ void __launch_bounds__(64) moe_grouped_rows_kernel(GroupedArgs p) {
 // 32 experts of ff 1024, top 4, up + down product in us (rows kernel | 64-row tiles | 128-row tiles):
 //   mean rows 1: 60 | 68 | 73     4: 85 | 92 | 94     8: 86 | 92 | 94     16: 104 | 93 | 96     32: 161 | 95 | 99
 //   64: 286 | 103 | 103     96: 410 | 138 | 107     128: 537 | 150 | 157     512: 2038 | 379 | 337
+// and from 320 rows on the 128 x 256 tiles (their comment has both sides)
 // (the kernel these replaced, one operand fragment per load and no LDS: 75 at mean 1, 1398 at mean 512)
 template <typename Tag, int ACT>
 int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
@@ -553,6 +676,21 @@ int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
     const int tiles = pairs / 16 + held, per = ACT >= 2 ? 16 : 32;
     if (tiles > 65535) return SP_ERR_UNSUPPORTED;                // (4096 experts, the most moe_align takes: 6656)
     moe_grouped_rows_kernel<Tag, ACT><<<dim3((unsigned)((p.N + per - 1) / per), (unsigned)tiles), 64, 0, st>>>(p);
+    SP_LAUNCH_CHECK();
+    return SP_OK;
+  }
+  if (pairs > 320 * (int64_t)p.E) {
+    constexpr int lds = 2 * (kWideBM + kWideBN) * kWideBK * 2;
+    static PerDevice<int> raised;
+    int ok = 0;
+    raised.get(ok, [&](int) {
+      return hipFuncSetAttribute((const void*)moe_grouped_wide_kernel<Tag, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) ==
+             hipSuccess ? 1 : 0;
+    });
+    if (!ok) return SP_ERR_LAUNCH;
+    const int wper = ACT >= 2 ? kWideBN / 2 : kWideBN;
+    const int64_t wtiles = (p.N + wper - 1) / wper;
+    moe_grouped_wide_kernel<Tag, ACT><<<dim3((unsigned)(((pairs / kWideBM + held) * wtiles + 7) / 8 * 8)), 256, lds, st>>>(p);
     SP_LAUNCH_CHECK();
     return SP_OK;
   }

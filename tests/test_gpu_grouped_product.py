@@ -1,4 +1,4 @@
-"""The grouped expert products on the matrix cores at the edges of their tiles (rows per expert around 16, 64 and 128, columns
+"""The grouped expert products on the matrix cores at the edges of their tiles (rows per expert around 16, 64, 128 and 320, columns
 and k that end inside a tile, experts without rows, more experts than lanes), against the product in fp32 by torch, and the
 gated form bit for bit against the product followed by its activation."""
 import pytest
@@ -21,12 +21,13 @@ def grouped_inputs(counts, N, K, dtype, top, seed=0):
     return a, w, offsets, order, expert, P
 
 
-COUNTS = [[1], [0, 3, 0, 17], [16, 0, 15, 33], [63, 64, 65, 1], [127, 128, 129, 257, 0], [300, 2, 140], [3] * 70, [90] * 67 + [0, 1]]
+COUNTS = [[1], [0, 3, 0, 17], [16, 0, 15, 33], [63, 64, 65, 1], [127, 128, 129, 257, 0], [300, 2, 140], [3] * 70, [90] * 67 + [0, 1],
+          [321], [0, 385, 700, 129], [1100] + [1] * 2]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("counts", COUNTS, ids=lambda c: "-".join(map(str, c[:5])))
-@pytest.mark.parametrize("N,K", [(64, 32), (130, 96), (200, 256)])
+@pytest.mark.parametrize("N,K", [(64, 32), (130, 96), (200, 256), (300, 160)])
 def test_grouped_products(counts, N, K, dtype):
     from scratchpad_amd import _native
     top = 3
@@ -52,7 +53,7 @@ def test_grouped_products(counts, N, K, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("counts", COUNTS, ids=lambda c: "-".join(map(str, c[:5])))
-@pytest.mark.parametrize("ff,K", [(32, 32), (67, 96), (136, 128)])
+@pytest.mark.parametrize("ff,K", [(32, 32), (67, 96), (136, 128), (260, 64)])
 def test_gated_form_is_the_two_steps(counts, ff, K, dtype):
     from scratchpad_amd import _native
     a, w, offsets, order, _, P = grouped_inputs(counts, 2 * ff, K, dtype, 2, seed=1)
