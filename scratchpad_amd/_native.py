@@ -755,14 +755,15 @@ _SKINNY_ON = os.environ.get("SP_SKINNY_GEMM", "1") != "0"
 
 
 def skinny_gemm_pays(M: int, N: int, K: int) -> bool:
-    """Where the weight-streaming kernel measured faster than hipBLASLt on MI355X
-    (tools/bench_gemv.py, Llama-3-8B shapes): every lane's x fragment is re-read from L2 per k-step,
-    so the win shrinks as rows fill the 16-wide tile and with long rows (down_proj)."""
+    """Where the weight-streaming kernels measured faster than hipBLASLt on MI355X (us, own / library, cold weights): 4096 x 4096
+    10 / 13 at 8 rows; at 4 rows 6144 x 4096 12.7 / 13.3, 28672 x 4096 44 / 58, 128256 x 2048 96 / 114, 128256 x 4096
+    183 / 189; at 8 rows 28672 x 4096 51 / 59, 65536 x 2048 59 / 66, 128256 x 2048 112 / 116 but 128256 x 4096 213 / 184.
+    Above 4 rows every workgroup reads as much x out of L2 as weights, so the win shrinks with rows and with K."""
     if M <= 16 and N * K <= 4096 * 4096:
-        return True                       # o_proj-sized: 11 vs 19 us at every M <= 16
-    if M <= 2 and K <= 8192:
-        return True                       # bs 1-2: qkv 13 vs 19, gate_up 44 vs 60, lm_head 166 vs 179 us
-    return M <= 8 and K <= 8192 and N <= 65536
+        return True
+    if M <= 4 and K <= 8192:
+        return True
+    return M <= 8 and K <= 8192 and (N <= 65536 or K <= 2048)
 
 
 # ---- the row count the library is handed -----------------------------------------------------------------------

@@ -227,6 +227,13 @@ def test_skinny_gemm_dispatch_rule_and_cpu_passthrough():
     assert torch.equal(_native.linear(x, w), torch.nn.functional.linear(x, w))           # host tensors: plain F.linear
 
 
+def test_skinny_gemm_takes_the_head_of_few_rows():
+    from scratchpad_amd import _native
+    pays = _native.skinny_gemm_pays
+    assert all(pays(m, 128256, k) for m in (1, 3, 4) for k in (2048, 4096)) and pays(8, 128256, 2048)
+    assert not pays(5, 128256, 4096) and not pays(9, 128256, 2048) and not pays(3, 4096, 14336)
+
+
 def test_vision_attention_plan_partition(monkeypatch):
     import torch
     from scratchpad_amd import vision
