@@ -512,7 +512,8 @@ window_attention_kernel(void* out, int64_t out_stride, const void* q, int64_t q_
 // the library's exponential and a rescaling of O per tile took 3500 per wave.  So masks are formed only where a tile is not wholly
 // visible, in the list's own 32-bit positions; a weight is one fma and one hardware exp2; O is rescaled when a maximum moved; and
 // a query's denominator stays spread over its lanes until the end.  4 requests of 4096 tokens together, 16 heads of 128 on 4, window
-// 512 and blocks of 64: 95 -> 62 us.
+// 512 and blocks of 64: 95 -> 62 us.  Keys (two buffers) and values go to LDS by direct loads: held in registers on the way, with
+// the next tile's on top, they left two workgroups per CU; three fit now, 62 -> 57.
 typedef float f32x4_w __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_w __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_w __attribute__((ext_vector_type(8)));
@@ -529,18 +530,26 @@ __device__ __forceinline__ f32x4_w mfma_w<f16_tag>(const u32x4& a, const u32x4& 
 
 typedef short s16x4_w __attribute__((ext_vector_type(4)));
 
+// by what a row's 16-byte chunks are turned in LDS: rows of 256 bytes begin in one bank, of 128 bytes in two, and a transposing
+// read takes pairs of chunks from four rows
+template <int RB>
+__device__ __forceinline__ int row_turn(int row) {
+  return RB == 256 ? 2 * (row & 7) : 2 * ((row >> 1) & 3);
+}
+
 template <typename Tag, int DS, int DT, bool SIG>      // DS = dim / 32, DT = vdim / 16
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 3)
 window_attention_mfma_kernel(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* kpool,
                              const void* vpool, const void* kpooled, const void* vpooled, int64_t kp_stride, int64_t vp_stride,
                              const int32_t* req_to_token, int64_t table_stride, SeqBatch s, int H, int G, int64_t size, int P,
                              int64_t lead, float scale, const float* sinks, float softcap, const float* head_bias, const void* gate,
                              int64_t gate_stride) {
   constexpr int D = 32 * DS, Dv = 16 * DT;
-  constexpr int KR = D + 8, VR = Dv + 8;                 // elements per LDS row: 16 bytes of padding spread the rows over the banks
-  constexpr int KP = D / 32, VP = Dv / 32;               // 16-byte pieces of a key (value) tile per thread
-  __shared__ __attribute__((aligned(16))) uint16_t skey[64 * KR], sval[64 * VR];
-  __shared__ int32_t sslot[64];                          // pool rows of the next tile's keys
+  constexpr int KB = 2 * D, VB = 2 * Dv;                 // bytes of an LDS row
+  constexpr int KL = KB / 64, VL = VB / 64;              // direct loads of 1 KB per wave for a tile of 64 keys
+  extern __shared__ __attribute__((aligned(16))) char wlds[];      // two tiles of keys, one of values
+  char *keys = wlds, *keys_next = wlds + 64 * KB, *const sval = wlds + 128 * KB;
+  __shared__ int32_t sslot[2][64];                       // pool rows of a tile's keys
   // which request and which of its 16-row tiles
   int tile = blockIdx.x, b = 0;
   for (; b < s.B; ++b) {
@@ -550,7 +559,7 @@ window_attention_mfma_kernel(void* out, int64_t out_stride, const void* q, int64
   }
   if (b >= s.B) return;
   const int g = blockIdx.y, R = H / G;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, qd = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, qd = lane >> 4;
   const int64_t start = s.extend_start_loc[b], len = s.extend_seq_lens[b], prefix = s.extend_prefix_lens[b];
   const int rows = (int)(len - 16 * tile < 16 ? len - 16 * tile : 16);
   const int64_t t0 = start + 16 * tile, pos0 = prefix + 16 * tile, pos_last = pos0 + rows - 1;
@@ -587,49 +596,58 @@ window_attention_mfma_kernel(void* out, int64_t out_stride, const void* q, int64
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) oacc[dt] = f32x4_w{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;
-    // the tiles go through registers, one ahead of the work; keys behind the last one repeat it, unseen by every query
+    // keys behind the last one repeat it, unseen by every query
     auto entry = [&](int64_t k0, int key) { return k0 + key < totalU ? k0 + key : totalU - 1; };
     auto slot_of = [&](int64_t k0) {                     // (threads 0 .. 63 use it)
       const int64_t kk = entry(k0, threadIdx.x & 63);
       return kk < nbU ? table[kk * P + P - 1] : table[w0U + (kk - nbU)];
     };
-    u32x4 kst[KP], vst[VP];
-    auto fetch = [&](int64_t k0) {
+    // a tile's rows straight into LDS, 1 KB per wave and load; a row's 16-byte chunks lie permuted by its number (the source address
+    // is: a direct load writes lane after lane), so that neither operand's reads meet a bank twice
+    // (its pool rows come out of LDS before any load is under way: a read of LDS behind one would wait for it)
+    auto rows_of = [&](auto row_bytes, int par, int32_t* slots) {
+      constexpr int RB = decltype(row_bytes)::value, CH = RB / 16, ROWS = 64 / CH;
 #pragma unroll
-      for (int u = 0; u < KP; ++u) {
-        const int c = threadIdx.x + 256 * u, key = c / (D / 8), col = c % (D / 8);
-        const void* src = entry(k0, key) < nbU ? kpooled : kpool;
-        kst[u] = ld16((const char*)src + ((int64_t)sslot[key] * kp_stride + (int64_t)g * D + 8 * col) * 2);
-      }
+      for (int u = 0; u < RB / 64; ++u) slots[u] = sslot[par][(wave * (RB / 64) + u) * ROWS + lane / CH];
+    };
+    auto fetch = [&](char* lds, const void* pool, const void* pooled_rows, int64_t stride, auto row_bytes, int64_t k0,
+                     const int32_t* slots) {
+      constexpr int RB = decltype(row_bytes)::value, CH = RB / 16, ROWS = 64 / CH;
 #pragma unroll
-      for (int u = 0; u < VP; ++u) {
-        const int c = threadIdx.x + 256 * u, key = c / (Dv / 8), col = c % (Dv / 8);
-        const void* src = entry(k0, key) < nbU ? vpooled : vpool;
-        vst[u] = ld16((const char*)src + ((int64_t)sslot[key] * vp_stride + (int64_t)g * Dv + 8 * col) * 2);
+      for (int u = 0; u < RB / 64; ++u) {
+        const int piece = wave * (RB / 64) + u, key = piece * ROWS + lane / CH;
+        const char* src = (const char*)(entry(k0, key) < nbU ? pooled_rows : pool) +
+                          ((int64_t)slots[u] * stride + (int64_t)g * (RB / 2)) * 2 + ((lane % CH) ^ row_turn<RB>(key)) * 16;
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)(lds + piece * 1024), 16, 0, 0);
       }
     };
-    int32_t slot = slot_of(0);
-    __syncthreads();                                     // (a further pass of heads: the last tile's readers are done)
-    if (threadIdx.x < 64) sslot[threadIdx.x] = slot;
-    __syncthreads();
-    fetch(0);
-    slot = slot_of(64);
+    const std::integral_constant<int, KB> key_bytes;
+    const std::integral_constant<int, VB> value_bytes;
+    lds_barrier();                                       // (a further pass of heads: the last tile's readers are done)
+    if (threadIdx.x < 64) {
+      sslot[0][threadIdx.x] = slot_of(0);
+      sslot[1][threadIdx.x] = slot_of(64);
+    }
+    lds_barrier();
+    int32_t kslots[KL], vslots[VL];
+    rows_of(key_bytes, 0, kslots);
+#pragma unroll
+    for (int st = 0; st < DS; ++st) asm volatile("" : "+v"(qf[st]));      // (the queries are here: no wait for them in the loop)
+    fetch(keys, kpool, kpooled, kp_stride, key_bytes, 0, kslots);
     for (int64_t k0 = 0; k0 < totalU; k0 += 64) {
-      __syncthreads();                                   // the previous tile's readers are done
-#pragma unroll
-      for (int u = 0; u < KP; ++u) {
-        const int c = threadIdx.x + 256 * u;
-        st16(skey + (c / (D / 8)) * KR + 8 * (c % (D / 8)), kst[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < VP; ++u) {
-        const int c = threadIdx.x + 256 * u;
-        st16(sval + (c / (Dv / 8)) * VR + 8 * (c % (Dv / 8)), vst[u]);
-      }
-      if (threadIdx.x < 64) sslot[threadIdx.x] = slot;
-      __syncthreads();
-      if (k0 + 64 < totalU) fetch(k0 + 64);
-      slot = slot_of(k0 + 128);
+      const int par = (int)(k0 >> 6) & 1;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();                                     // the tile's keys have landed; everyone is done with the values before
+      rows_of(value_bytes, par, vslots);
+      rows_of(key_bytes, par ^ 1, kslots);
+      fetch(sval, vpool, vpooled, vp_stride, value_bytes, k0, vslots);
+      __builtin_amdgcn_sched_barrier(0);                 // in this order: the wait below counts
+      const bool more = k0 + 64 < totalU;
+      if (more) fetch(keys_next, kpool, kpooled, kp_stride, key_bytes, k0 + 64, kslots);
+      __builtin_amdgcn_sched_barrier(0);
+      const int32_t slot = slot_of(k0 + 128);
+      u32x4 pb[2], pr[2];
       if (work) {
         f32x4_w sacc[4];
 #pragma unroll
@@ -637,7 +655,7 @@ window_attention_mfma_kernel(void* out, int64_t out_stride, const void* q, int64
           sacc[sb] = f32x4_w{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int st = 0; st < DS; ++st)
-            sacc[sb] = mfma_w<Tag>(ld16(skey + (16 * sb + r16) * KR + 32 * st + 8 * qd), qf[st], sacc[sb]);
+            sacc[sb] = mfma_w<Tag>(ld16(keys + (16 * sb + r16) * KB + ((4 * st + qd) ^ row_turn<KB>(r16)) * 16), qf[st], sacc[sb]);
         }
         if (!plain) {
 #pragma unroll
@@ -695,30 +713,44 @@ window_attention_mfma_kernel(void* out, int64_t out_stride, const void* q, int64
               pf[sb >> 1][4 * (sb & 1) + r] = p;
             }
         }
+        // the weights enter the product as a 16-bit value plus a 16-bit remainder: they are never rounded to 8 bits of
+        // mantissa (the second product costs an eighth of the step's matrix work again)
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
-          // the weights enter the product as a 16-bit value plus a 16-bit remainder: they are never rounded to 8 bits of
-          // mantissa (the second product costs an eighth of the step's matrix work again)
-          const u32x4 pb = pack16<Tag>(pf[hh]);
+          pb[hh] = pack16<Tag>(pf[hh]);
           float rest[8], back[8];
-          unpack16<Tag>(pb, back);
+          unpack16<Tag>(pb[hh], back);
 #pragma unroll
           for (int e = 0; e < 8; ++e) rest[e] = pf[hh][e] - back[e];
-          const u32x4 pr = pack16<Tag>(rest);
+          pr[hh] = pack16<Tag>(rest);
+        }
+      }
+      // the values were asked for before the next tile's keys: at most those (KL of them per wave) may still be under way
+      if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(KL) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();
+      if (work) {
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          // lane i of a 16-lane group addresses row 4 qd + (i >> 2), elements 4 (i & 3) .. + 3, and receives column i
+          const int row = 32 * hh + 4 * qd + (r16 >> 2), turn = row_turn<VB>(row);      // (16 rows on: the same turn)
+          const char* vr = sval + row * VB + 8 * (r16 & 1);
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) {
-            // lane i of a 16-lane group addresses row 4 qd + (i >> 2), elements 4 (i & 3) .. + 3, and receives column i
-            const uint16_t* vp = sval + (32 * hh + 4 * qd + (r16 >> 2)) * VR + 16 * dt + 4 * (r16 & 3);
+            const char* vp = vr + ((2 * dt + ((r16 & 3) >> 1)) ^ turn) * 16;
             const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                                                            (__attribute__((address_space(3))) s16x4_w*)vp));
             const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                                           (__attribute__((address_space(3))) s16x4_w*)(vp + 16 * VR)));
+                                                           (__attribute__((address_space(3))) s16x4_w*)(vp + 16 * VB)));
             const u32x4 a = {lo[0], lo[1], hi[0], hi[1]};
-            oacc[dt] = mfma_w<Tag>(a, pb, oacc[dt]);
-            oacc[dt] = mfma_w<Tag>(a, pr, oacc[dt]);
+            oacc[dt] = mfma_w<Tag>(a, pb[hh], oacc[dt]);
+            oacc[dt] = mfma_w<Tag>(a, pr[hh], oacc[dt]);
           }
         }
       }
+      if (threadIdx.x < 64) sslot[par][threadIdx.x] = slot;      // (waits for all loads: at the tile's end)
+      char* const t = keys;
+      keys = keys_next, keys_next = t;
     }
     if constexpr (!SIG) {                              // (outside the branch: every lane of a wave takes part)
       l += __shfl_xor(l, 16, 64);
@@ -846,7 +878,7 @@ extern "C" int sp_window_attention(void* out, int64_t out_stride, const void* q,
       (!gate || (((uintptr_t)gate & 7) == 0 && gate_stride % 4 == 0))) {
     const dim3 mgrid((unsigned)((num_tokens + 15) / 16 + batch_size), (unsigned)kv_heads);
 #define SP_WM2(T, DS, DT, SG)                                                                                            \
-  window_attention_mfma_kernel<T, DS, DT, SG><<<mgrid, 256, 0, (hipStream_t)stream>>>(                                     \
+  window_attention_mfma_kernel<T, DS, DT, SG><<<mgrid, 256, 64 * 2 * (2 * 32 * DS + 16 * DT), (hipStream_t)stream>>>(                                     \
       out, out_stride, q, q_stride, kpool, vpool, kpooled, vpooled, kp_stride, vp_stride, req_to_token, table_stride, s, heads, \
       kv_heads, window, block, lead, scale, sinks, softcap, head_bias, gate, gate_stride)
 #define SP_WM(T, DS, DT)                    \
