@@ -291,6 +291,9 @@ struct ChunkScan {
     for (int i = 0; i < DT; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) S[i][r] = held ? st[(int64_t)row_of(i, r) * Dv + column()] : 0.f;
+    // here before the loop over chunks: a wait for them inside it would be one for the next chunk's loads, every time
+#pragma unroll
+    for (int i = 0; i < DT; ++i) asm volatile("" : "+v"(S[i]));
   }
   __device__ __forceinline__ void store_state(float* st) const {
 #pragma unroll

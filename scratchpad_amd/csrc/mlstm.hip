@@ -202,7 +202,8 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
   const char* gb = (const char*)g + (start * g_stride + (int64_t)h * Dv) * 2;
   char* ob = (char*)out + (start * out_stride + (int64_t)h * Dv) * 2;
   const int col = c.column();
-  const float nw = norm_w[(int64_t)h * Dv + col];
+  float nw = norm_w[(int64_t)h * Dv + col];
+  asm volatile("" : "+v"(nw), "+v"(m));               // (as the state: waited for here)
   const auto load = [&](int64_t c0) {
     const int n = (int)(len - c0 < kCL ? len - c0 : kCL);
     c.load(q + c0 * q_stride * 2, q_stride * 2, k + c0 * k_stride * 2, k_stride * 2, v + c0 * v_stride * 2, v_stride * 2, n);

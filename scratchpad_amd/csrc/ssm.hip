@@ -461,8 +461,8 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
     c.stage();
     lds_barrier();
     if (c0 + kCL < len) {
+      load_steps(c0 + kCL);                           // (first: they are waited for first, and loads arrive in order)
       load(c0 + kCL);
-      load_steps(c0 + kCL);
     }
     c.scores();
     c.from_state(zero);
