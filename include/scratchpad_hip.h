@@ -611,6 +611,12 @@ SP_API int sp_mlstm_scan(void* out, int64_t out_stride, const void* q, int64_t q
                          const float* fpre, const float* norm_w, float* S_state, int64_t S_stride, float* n_state,
                          int64_t n_stride, float* m_state, int64_t m_stride, int heads, int dim, int vdim, float cap,
                          float eps, SP_SEQ_PARAMS, int dtype, void* stream);
+/* The same with gates whose rows lie gate_stride >= heads values apart (both halves of one product). */
+SP_API int sp_mlstm_scan_gates(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                               const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
+                               const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
+                               float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, int heads, int dim,
+                               int vdim, float cap, float eps, SP_SEQ_PARAMS, int dtype, void* stream);
 
 /* ================================================================================================================
  * ABI 12: sublayer results that are gated and normed before they join the fp32 stream, the generalized delta rule, a

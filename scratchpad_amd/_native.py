@@ -145,6 +145,8 @@ SIGNATURES = {
     "sp_gated_group_norm": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i32, _i32, _f32, _i32, _vp]),
     "sp_mlstm_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp,
                              _i64, _i32, _i32, _i32, _f32, _f32, *_SEQ, _i32, _vp]),
+    "sp_mlstm_scan_gates": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i64,
+                                   _vp, _i64, _i32, _i32, _i32, _f32, _f32, *_SEQ, _i32, _vp]),
     # ---- ABI 12
     "sp_gated_add_norm": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp,
                                  _i64, _i32, _f32, _i32, _vp]),
@@ -1608,20 +1610,26 @@ def mlstm_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tenso
                norm_w: torch.Tensor, S: torch.Tensor, n: torch.Tensor, m: torch.Tensor, seq: SeqParams, heads: int, dim: int,
                vdim: int, cap: float, eps: float) -> torch.Tensor:
     """q, k [T, heads * dim], v, g [T, heads * vdim] (views) -> [T, heads * vdim]; states S [slots, heads, dim, vdim],
-    n [slots, heads, dim], m [slots, heads] fp32"""
+    n [slots, heads, dim], m [slots, heads] fp32; ipre, fpre fp32 [T, heads], views with one row stride"""
     T = seq.num_tokens
     for name, t, w in (("q", q, heads * dim), ("k", k, heads * dim), ("v", v, heads * vdim), ("g", g, heads * vdim)):
         if _mat(t, name).shape != (T, w) or t.dtype != q.dtype:
             raise RuntimeError(f"mlstm_scan: {name} must be [num_tokens, {w}] of one dtype")
-    _f32(ipre, "ipre"), _f32(fpre, "fpre"), _f32(norm_w, "norm_w"), _f32(S, "S"), _f32(n, "n"), _f32(m, "m")
+    for name, t in (("ipre", ipre), ("fpre", fpre)):
+        if t.dtype != torch.float32 or not t.is_cuda or t.dim() != 2 or (t.stride(1) != 1 and t.shape[1] != 1):
+            raise RuntimeError(f"mlstm_scan: {name} must be fp32 device rows")
+    if ipre.stride(0) != fpre.stride(0):
+        ipre, fpre = ipre.contiguous(), fpre.contiguous()
+    _f32(norm_w, "norm_w"), _f32(S, "S"), _f32(n, "n"), _f32(m, "m")
     if ipre.shape != (T, heads) or fpre.shape != (T, heads) or norm_w.numel() != heads * vdim or \
             S.shape[1:] != (heads, dim, vdim) or n.shape[1:] != (heads, dim) or m.shape[1:] != (heads,):
         raise RuntimeError("mlstm_scan: gate or state shapes do not fit")
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
-    _check(load().sp_mlstm_scan(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
-                                v.data_ptr(), v.stride(0), g.data_ptr(), g.stride(0), ipre.data_ptr(), fpre.data_ptr(),
-                                norm_w.data_ptr(), S.data_ptr(), S.stride(0), n.data_ptr(), n.stride(0), m.data_ptr(),
-                                m.stride(0), heads, dim, vdim, cap, eps, *seq.args, _dt(q), _stream()), "sp_mlstm_scan")
+    _check(load().sp_mlstm_scan_gates(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
+                                      v.data_ptr(), v.stride(0), g.data_ptr(), g.stride(0), ipre.data_ptr(), fpre.data_ptr(),
+                                      max(ipre.stride(0), heads), norm_w.data_ptr(), S.data_ptr(), S.stride(0), n.data_ptr(),
+                                      n.stride(0), m.data_ptr(), m.stride(0), heads, dim, vdim, cap, eps, *seq.args, _dt(q),
+                                      _stream()), "sp_mlstm_scan_gates")
     return out
 
 

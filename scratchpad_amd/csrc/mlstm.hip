@@ -31,8 +31,8 @@ template <typename Tag, int DP>
 __global__ void __launch_bounds__(split_of(DP) == 1 ? 320 : (split_of(DP) == 2 ? 576 : 1024))
 mlstm_scan_kernel(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
                   const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre,
-                  const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride, float* m_state,
-                  int64_t m_stride, SeqBatch s, int H, int D, int Dv, float cap, float eps) {
+                  int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride,
+                  float* m_state, int64_t m_stride, SeqBatch s, int H, int D, int Dv, float cap, float eps) {
   typedef Elem<Tag> E;
   constexpr int kChunk = chunk_of(DP), SP = split_of(DP), DS = DP / SP, ROW = DP + 4 * SP;
   __shared__ float sq[kChunk][ROW], sk[kChunk][ROW], si[kChunk], sf[kChunk], sinv[kChunk], sden[kChunk], sm[kChunk];
@@ -78,8 +78,8 @@ mlstm_scan_kernel(void* out, int64_t out_stride, const void* q, int64_t q_stride
     }
     if (j < n) {
       const int64_t row = start + c0 + j;
-      si[j] = cap * tanhf(ipre[row * H + h] / cap);
-      sf[j] = logsigmoid_f(cap * tanhf(fpre[row * H + h] / cap));
+      si[j] = cap * tanhf(ipre[row * gate_stride + h] / cap);
+      sf[j] = logsigmoid_f(cap * tanhf(fpre[row * gate_stride + h] / cap));
     }
     __syncthreads();
     for (int tt = 0; tt < n; ++tt) {
@@ -168,9 +168,9 @@ struct MlstmLds {
 template <int D, int NW>
 __global__ void __launch_bounds__(NW * 64)
 mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_stride, const char* k, int64_t k_stride, const char* v,
-                   int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre, const float* norm_w,
-                   float* S_state, int64_t S_stride, float* n_state, int64_t n_stride, float* m_state, int64_t m_stride,
-                   SeqBatch s, int H, float cap, float eps) {
+                   int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre,
+                   int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride,
+                   float* m_state, int64_t m_stride, SeqBatch s, int H, float cap, float eps) {
   typedef Elem<bf16_tag> E;
   typedef ChunkScan<D, NW> C;
   typedef MlstmLds<D, NW> L;
@@ -214,7 +214,7 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
     const int64_t t = c0 + c.tid;
     double* to = sgate + c.wave * 3 * kCL + c.lane;
     const bool live = t < len;
-    const float gi = live ? ipre[(start + t) * H + h] : 0.f, gf = live ? fpre[(start + t) * H + h] : 0.f;
+    const float gi = live ? ipre[(start + t) * gate_stride + h] : 0.f, gf = live ? fpre[(start + t) * gate_stride + h] : 0.f;
     const double F = wave_scan_sum(live ? (double)logsigmoid_f(cap * tanhf(gf / cap)) : 0., c.lane);
     const double bs = live ? (double)(cap * tanhf(gi / cap)) - F : -INFINITY;
     to[0] = F;
@@ -329,14 +329,14 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
 template <int D, int NW>
 static int launch_mlstm_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
                                const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
-                               const float* fpre, const float* norm_w, float* S_state, int64_t S_stride, float* n_state,
-                               int64_t n_stride, float* m_state, int64_t m_stride, const SeqBatch& s, int H, float cap, float eps,
+                               const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
+                               float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, const SeqBatch& s, int H, float cap, float eps,
                                hipStream_t st) {
   constexpr int bytes = MlstmLds<D, NW>::kBytes;
   static PerDevice<int> raised;
   if (!chunk_lds_ready(raised, (const void*)mlstm_chunk_kernel<D, NW>, bytes)) return SP_ERR_LAUNCH;
   mlstm_chunk_kernel<D, NW><<<dim3((unsigned)s.B, (unsigned)H), NW * 64, bytes, st>>>(
-      out, out_stride, (const char*)q, q_stride, (const char*)k, k_stride, (const char*)v, v_stride, g, g_stride, ipre, fpre,
+      out, out_stride, (const char*)q, q_stride, (const char*)k, k_stride, (const char*)v, v_stride, g, g_stride, ipre, fpre, gate_stride,
       norm_w, S_state, S_stride, n_state, n_stride, m_state, m_stride, s, H, cap, eps);
   SP_LAUNCH_CHECK();
   return SP_OK;
@@ -345,7 +345,7 @@ static int launch_mlstm_chunks(void* out, int64_t out_stride, const void* q, int
 template <typename Tag>
 static int launch_mlstm(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
                         const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre,
-                        const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride,
+                        int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride,
                         float* m_state, int64_t m_stride, const SeqBatch& s, int H, int D, int Dv, float cap, float eps,
                         hipStream_t st) {
   // a step of one token per request stays with the per-token form (one sweep over the state is all there is to do), and so do
@@ -354,7 +354,7 @@ static int launch_mlstm(void* out, int64_t out_stride, const void* q, int64_t q_
       chunk_aligned(q, q_stride) && chunk_aligned(k, k_stride) && chunk_aligned(v, v_stride) &&
       g_stride < ((int64_t)1 << 24) && out_stride < ((int64_t)1 << 24)) {
 #define SP_MLSTM_CHUNKS(D_, NW_)                                                                                              \
-  return launch_mlstm_chunks<D_, NW_>(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, norm_w, \
+  return launch_mlstm_chunks<D_, NW_>(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, gate_stride, norm_w, \
                                       S_state, S_stride, n_state, n_stride, m_state, m_stride, s, H, cap, eps, st)
     if (D == 128 && Dv == 128) SP_MLSTM_CHUNKS(128, 8);
     if (D == 128) SP_MLSTM_CHUNKS(128, 4);
@@ -367,7 +367,7 @@ static int launch_mlstm(void* out, int64_t out_stride, const void* q, int64_t q_
 #define SP_MLSTM(DP)                                                                                                    \
   mlstm_scan_kernel<Tag, DP><<<grid, (unsigned)(((Dv + 1) * split_of(DP) + 63) / 64 * 64),                              \
                                (size_t)chunk_of(DP) * (2 * Dv + 1) * sizeof(float), st>>>(                              \
-      out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, norm_w, S_state, S_stride, n_state,  \
+      out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, gate_stride, norm_w, S_state, S_stride, n_state,  \
       n_stride, m_state, m_stride, s, H, D, Dv, cap, eps)
   if (D <= 16) SP_MLSTM(16);
   else if (D <= 32) SP_MLSTM(32);
@@ -385,20 +385,31 @@ static int launch_mlstm(void* out, int64_t out_stride, const void* q, int64_t q_
 
 using namespace sp;
 
-extern "C" int sp_mlstm_scan(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
-                             const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
-                             const float* fpre, const float* norm_w, float* S_state, int64_t S_stride, float* n_state,
-                             int64_t n_stride, float* m_state, int64_t m_stride, int heads, int dim, int vdim, float cap,
-                             float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
+// (gate_stride: values between the gates of a token and the next one's, so that both may be halves of one product's rows)
+extern "C" int sp_mlstm_scan_gates(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                   const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
+                                   const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
+                                   float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, int heads, int dim,
+                                   int vdim, float cap, float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
   SP_CHECK_ARG(batch_size >= 0 && heads > 0 && dim > 0 && vdim > 0 && vdim <= 256 && cap > 0.f);
   if (batch_size == 0) return SP_OK;
   SP_CHECK_ARG(out && q && k && v && g && ipre && fpre && norm_w && S_state && n_state && m_state && req_pool_indices && seq_lens);
   SP_CHECK_ARG(!extend_seq_lens || (extend_prefix_lens && extend_start_loc));
   const int64_t nk = (int64_t)heads * dim, nv = (int64_t)heads * vdim;
   SP_CHECK_ARG(q_stride >= nk && k_stride >= nk && v_stride >= nv && g_stride >= nv && out_stride >= nv);
-  SP_CHECK_ARG(S_stride >= nk * vdim && n_stride >= nk && m_stride >= heads);
+  SP_CHECK_ARG(S_stride >= nk * vdim && n_stride >= nk && m_stride >= heads && gate_stride >= heads);
   SEQ_BATCH(s);
   SP_DISPATCH_DTYPE(dtype, return (launch_mlstm<Tag>(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre,
-                                                     fpre, norm_w, S_state, S_stride, n_state, n_stride, m_state, m_stride, s,
+                                                     fpre, gate_stride, norm_w, S_state, S_stride, n_state, n_stride, m_state, m_stride, s,
                                                      heads, dim, vdim, cap, eps, (hipStream_t)stream)));
+}
+
+extern "C" int sp_mlstm_scan(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                             const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
+                             const float* fpre, const float* norm_w, float* S_state, int64_t S_stride, float* n_state,
+                             int64_t n_stride, float* m_state, int64_t m_stride, int heads, int dim, int vdim, float cap,
+                             float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
+  return sp_mlstm_scan_gates(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, heads, norm_w, S_state,
+                             S_stride, n_state, n_stride, m_state, m_stride, heads, dim, vdim, cap, eps, req_pool_indices, seq_lens,
+                             extend_seq_lens, extend_prefix_lens, extend_start_loc, token_req, idx64, batch_size, dtype, stream);
 }

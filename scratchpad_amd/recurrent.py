@@ -124,10 +124,9 @@ class MLSTMMixer(nn.Module):
         nk, nv, H = self.heads * self.dim, self.heads * self.vdim, self.heads
         a = _native.linear(h, self.qkvg)
         gates = _native.small_linear_f32(h, self.gates.data, self.gates_bias.data)
-        ipre, fpre = gates[:, :H].contiguous(), gates[:, H:].contiguous()
         L = self.layer_id
-        o = _native.mlstm_scan(a[:, :nk], a[:, nk:2 * nk], a[:, 2 * nk:2 * nk + nv], a[:, 2 * nk + nv:], ipre, fpre,
-                               self.norm.data, states.state(L, "S"), states.state(L, "n"), states.state(L, "m"), seq,
+        o = _native.mlstm_scan(a[:, :nk], a[:, nk:2 * nk], a[:, 2 * nk:2 * nk + nv], a[:, 2 * nk + nv:], gates[:, :H],
+                               gates[:, H:], self.norm.data, states.state(L, "S"), states.state(L, "n"), states.state(L, "m"), seq,
                                self.heads, self.dim, self.vdim, self.cap, self.eps)
         return _native.linear(o, self.o)
 

@@ -195,3 +195,24 @@ def test_head_delta_chunks_against_the_per_token_kernel(lens, H, G, D, Dv, dtype
         assert ((out.double() - want.double()).abs() <= bar * want.double().abs() + 1e-3).all()
     for slot in range(0, 2 * len(lens) + 1, 2):
         assert torch.isnan(S[slot]).all()
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.bfloat16, 32), (torch.float32, 64)])
+@pytest.mark.parametrize("lens", [[1, 1, 1], [70, 3]], ids=lambda l: "-".join(map(str, l)))
+def test_mlstm_gates_as_halves_of_one_product(dtype, D, lens):
+    """the bits of the scan on contiguous gates, in prompts and (one token each) in steps, for the chunk and the per-token kernels"""
+    from scratchpad_amd import _native
+    announce("mlstm gates", dtype, D, lens)
+    g = torch.Generator(device=DEV).manual_seed(9)
+    T, H, slots = sum(lens), 2, slots_of(lens)
+    q, k, v, gate = (torch.randn(T, H * D, generator=g, device=DEV).to(dtype) for _ in range(4))
+    gates, nw = torch.randn(T, 2 * H, generator=g, device=DEV), torch.rand(H * D, generator=g, device=DEV)
+    ip, fp = gates[:, :H], gates[:, H:]
+    got = []
+    for i, f in ((ip, fp), (ip.contiguous(), fp.contiguous()), (ip, fp.contiguous())):
+        S, n, m = (torch.zeros(2 * len(lens) + 1, H, *w, device=DEV) for w in ((D, D), (D,), ()))
+        seq = _native.SeqParams(torch.tensor(slots, device=DEV), torch.tensor([5] * len(lens), device=DEV)) if max(lens) == 1 \
+            else seq_extend(lens, [0] * len(lens), slots)
+        got.append((_native.mlstm_scan(q, k, v, gate, i, f, nw, S, n, m, seq, H, D, D, 15.0, 1e-5), S, n, m))
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
