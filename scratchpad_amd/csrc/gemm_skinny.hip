@@ -31,15 +31,14 @@
 // barrier come before the first product, and the loop's tail is longer than a launch of many small workgroups), 16 products in
 // flight, two weight rows a wave at one row.
 //
-// Epilogue fusion (round 4): with `epilogue` = 1 the weight is the merged gate|up matrix [2 I, K] of LlamaMLP
+// Epilogue fusion: with `epilogue` = 1 the weight is the merged gate|up matrix [2 I, K] of LlamaMLP
 // (nn/models/llama/llama.py:62-66) and the output is SiluAndMul (nn/layers/activation.py:21-31) of the projection,
-// [M, I]: a workgroup streams 8 gate rows and the 8 matching up rows (still 16 rows of W, still one workgroup per
-// 16 rows), and the lanes that finish the gate columns take the up sums of the same columns from the LDS reduction
-// and write round(silu(round(gate))) * round(up), rounded - bit for bit the plain projection followed by
-// sp_silu_and_mul, with the activation launch, its boundary and the [M, 2 I] round trip gone.  (The other way round -
-// the activation in the PROLOGUE of the down projection, every workgroup recomputing the M x K activations it
-// streams - was built first and measured 2 x SLOWER than the two launches: 76 vs 38 us at 1 row; the exponentials
-// of all 16 lane rows of every k-step are vector work the stream cannot hide.  profiles/NOTES.md, round 4.)
+// [M, I]: a workgroup streams gate rows and the up rows of the same columns, and whoever finishes a gate column takes
+// the up sum beside it and writes round(silu(round(gate))) * round(up), rounded - bit for bit the plain projection
+// followed by sp_silu_and_mul, with the activation launch, its boundary and the [M, 2 I] round trip gone.  (The other
+// way round - the activation in the PROLOGUE of the down projection, every workgroup recomputing the M x K activations
+// it streams - measured 2 x SLOWER than the two launches: 76 vs 38 us at 1 row; the exponentials of every k-step are
+// vector work the stream cannot hide.)
 // `epilogue` = 2: out = max(product, 0)^2 on the fp32 sum, rounded once (the up projection of a squared-ReLU feed-forward).
 // `epilogue` = 3: as 1 with the tanh form of GELU in SiLU's place, its product with the up sum rounded once (bit for bit the
 // plain projection followed by sp_gelu_tanh_and_mul).
