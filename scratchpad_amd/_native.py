@@ -1616,8 +1616,9 @@ def mlstm_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tenso
         if _mat(t, name).shape != (T, w) or t.dtype != q.dtype:
             raise RuntimeError(f"mlstm_scan: {name} must be [num_tokens, {w}] of one dtype")
     for name, t in (("ipre", ipre), ("fpre", fpre)):
-        if t.dtype != torch.float32 or not t.is_cuda or t.dim() != 2 or (t.stride(1) != 1 and t.shape[1] != 1):
-            raise RuntimeError(f"mlstm_scan: {name} must be fp32 device rows")
+        if t.dtype != torch.float32 or not t.is_cuda or t.dim() != 2 or (t.stride(1) != 1 and t.shape[1] != 1) or \
+                (t.shape[0] > 1 and t.stride(0) < heads):
+            raise RuntimeError(f"mlstm_scan: {name} must be fp32 device rows, at least {heads} values apart")
     if ipre.stride(0) != fpre.stride(0):
         ipre, fpre = ipre.contiguous(), fpre.contiguous()
     _f32(norm_w, "norm_w"), _f32(S, "S"), _f32(n, "n"), _f32(m, "m")
@@ -1627,7 +1628,7 @@ def mlstm_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tenso
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
     _check(load().sp_mlstm_scan_gates(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                                       v.data_ptr(), v.stride(0), g.data_ptr(), g.stride(0), ipre.data_ptr(), fpre.data_ptr(),
-                                      max(ipre.stride(0), heads), norm_w.data_ptr(), S.data_ptr(), S.stride(0), n.data_ptr(),
+                                      ipre.stride(0) if T > 1 else heads, norm_w.data_ptr(), S.data_ptr(), S.stride(0), n.data_ptr(),
                                       n.stride(0), m.data_ptr(), m.stride(0), heads, dim, vdim, cap, eps, *seq.args, _dt(q),
                                       _stream()), "sp_mlstm_scan_gates")
     return out

@@ -234,6 +234,38 @@ def test_skinny_gemm_takes_the_head_of_few_rows():
     assert not pays(5, 128256, 4096) and not pays(9, 128256, 2048) and not pays(3, 4096, 14336)
 
 
+def test_mlstm_scan_takes_no_gate_rows_that_overlap(monkeypatch):
+    """gates whose rows lie closer than their width (an expanded row, a sliding view) are refused before anything is launched: the
+    kernel reads [token, head] at rows at least `heads` apart.  Views of one product and strides that differ pass."""
+    import types
+
+    import torch
+    from scratchpad_amd import _native
+
+    class DeviceTensor(torch.Tensor):
+        is_cuda = True
+
+    calls = []
+    lib = types.SimpleNamespace(sp_mlstm_scan_gates=lambda *a: calls.append(a) or 0)
+    monkeypatch.setattr(_native, "load", lambda: lib)
+    monkeypatch.setattr(_native, "_stream", lambda: 0)
+    T, H, D = 6, 4, 16
+    dev = lambda *shape: torch.randn(*shape).as_subclass(DeviceTensor)  # noqa: E731
+    q, k, v, g = (dev(T, H * D) for _ in range(4))
+    nw, S, n, m = dev(H * D), dev(3, H, D, D), dev(3, H, D), dev(3, H)
+    seq = types.SimpleNamespace(num_tokens=T, batch_size=1, extend_seq_lens=object(), args=())
+    scan = lambda i, f: _native.mlstm_scan(q, k, v, g, i, f, nw, S, n, m, seq, H, D, D, 15.0, 1e-5)  # noqa: E731
+    both, row = dev(T, 2 * H), dev(1, H)
+    for i, f, stride in ((dev(T, H), dev(T, H), H), (both[:, :H], both[:, H:], 2 * H), (both[:, :H], dev(T, H), H)):
+        scan(i, f)
+        assert calls.pop()[12] == stride
+    near = dev(T + H).as_strided((T, H), (1, 1))
+    for i, f in ((row.expand(T, H), row.expand(T, H)), (row.expand(T, H), dev(T, H)), (near, near), (dev(T, H), near)):
+        with pytest.raises(RuntimeError):
+            scan(i, f)
+    assert not calls
+
+
 def test_vision_attention_plan_partition(monkeypatch):
     import torch
     from scratchpad_amd import vision
