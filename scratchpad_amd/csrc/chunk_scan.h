@@ -46,7 +46,8 @@ __device__ __forceinline__ void split3(float x, float y, uint32_t& hi, uint32_t&
 constexpr int kCL = 64;      // tokens per chunk
 
 // inclusive scans over a wave, in 64 bits: a chunk's log decays are summed and then subtracted from each other, and an exponent
-// that is wrong by the sum's fp32 rounding would be a weight wrong by as much
+// that is wrong by the sum's fp32 rounding would be a weight wrong by as much (6e-5 where the sums reach -1000).  For the same
+// reason the sums go to the weights as two fp32 parts, subtracted part by part: an exponent is then off by an ulp of itself.
 __device__ __forceinline__ double wave_scan_sum(double v, int lane) {
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -64,10 +65,17 @@ __device__ __forceinline__ double wave_scan_max(double v, int lane) {
   return v;
 }
 
-// what the products need of a chunk's tokens, in LDS: weight of s at t = exp(lt[t] - ls[s]) * cs[s] (s <= t), see above
+// what the products need of a chunk's tokens, in LDS: weight of s at t = exp(lt[t] - ls[s]) * cs[s] (s <= t), lt and ls each the
+// sum of two parts, see above
 struct ChunkScalars {
-  float lt[kCL], ls[kCL], cs[kCL], a0[kCL], w[kCL];
+  float lt[2][kCL], ls[2][kCL], cs[kCL], a0[kCL], w[kCL];
   float a_end, pad[3];
+
+  static __device__ __forceinline__ void put(float (*to)[kCL], int i, double v) {
+    const float hi = (float)v;
+    to[0][i] = hi;
+    to[1][i] = fabsf(hi) == INFINITY ? 0.f : (float)(v - (double)hi);
+  }
 };
 
 // rows that can be read 16 bytes at a time, a chunk's worth of them within 32-bit offsets
@@ -227,11 +235,11 @@ struct ChunkScan {
       int i, j;
       tile_of(id, i, j);
       const int t = 16 * i + r16, s0 = 16 * j + 4 * q;
-      const float lt = sc->lt[t];
-      const f32x4_c ls = *(const f32x4_c*)(sc->ls + s0), cs = *(const f32x4_c*)(sc->cs + s0);
+      const float lt = sc->lt[0][t], lt2 = sc->lt[1][t];
+      const f32x4_c ls = *(const f32x4_c*)(sc->ls[0] + s0), ls2 = *(const f32x4_c*)(sc->ls[1] + s0), cs = *(const f32x4_c*)(sc->cs + s0);
       float v[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = s0 + r <= t ? p[u][r] * (expf(lt - ls[r]) * cs[r]) : 0.f;
+      for (int r = 0; r < 4; ++r) v[r] = s0 + r <= t ? p[u][r] * (expf((lt - ls[r]) + (lt2 - ls2[r])) * cs[r]) : 0.f;
       if constexpr (SUMS) {
         float sum = (v[0] + v[1]) + (v[2] + v[3]);
         sum += __shfl_xor(sum, 16, 64);

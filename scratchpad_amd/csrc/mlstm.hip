@@ -227,8 +227,8 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
     const double F = from[0], bs = from[kCL], G = fmax((double)m, from[2 * kCL]);
     const double Gend = __shfl(G, 63, 64), Fend = __shfl(F, 63, 64);
     ChunkScalars& sc = *c.scalars(c0 / kCL);
-    sc.lt[c.lane] = (float)(Gend - G);                // (relative to the chunk's end: small where the weights are not)
-    sc.ls[c.lane] = (float)(Gend - bs);
+    ChunkScalars::put(sc.lt, c.lane, Gend - G);
+    ChunkScalars::put(sc.ls, c.lane, Gend - bs);
     sc.cs[c.lane] = qscale;
     sc.a0[c.lane] = expf((float)(m - G)) * qscale;
     sc.w[c.lane] = expf((float)(bs - Gend));

@@ -442,10 +442,13 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
   };
   const auto steps = [&](int64_t c0) {                // by the last wave: its share of the tiles is the smallest
     if (c.wave != NW - 1) return;
-    const float dt = c0 + c.lane < len ? softplus_f(raw + bias) : 0.f;
-    const double L = wave_scan_sum((double)(-a * dt), c.lane), Lend = __shfl(L, 63, 64);
+    const bool live = c0 + c.lane < len;
+    const float dt = live ? softplus_f(raw + bias) : 0.f, e = live ? -a * dt : 0.f;
+    // (e^-128 is zero in fp32: a stronger decay is the same one, and the sums stay where their differences are exact)
+    const double L = wave_scan_sum((double)(e < -128.f ? -128.f : e), c.lane), Lend = __shfl(L, 63, 64);
     ChunkScalars& sc = *c.scalars(c0 / kCL);
-    sc.lt[c.lane] = sc.ls[c.lane] = (float)L;
+    ChunkScalars::put(sc.lt, c.lane, L);
+    ChunkScalars::put(sc.ls, c.lane, L);
     sc.cs[c.lane] = dt;
     sc.a0[c.lane] = expf((float)L);
     sc.w[c.lane] = expf((float)(Lend - L)) * dt;

@@ -216,3 +216,84 @@ def test_mlstm_gates_as_halves_of_one_product(dtype, D, lens):
         got.append((_native.mlstm_scan(q, k, v, gate, i, f, nw, S, n, m, seq, H, D, D, 15.0, 1e-5), S, n, m))
     for other in got[1:]:
         assert all(torch.equal(a, b) for a, b in zip(got[0], other))
+
+
+def mamba2_in_64_bits(xbc, raw, bias, A, skip, lens, H, G, N, Dv):
+    """(outputs [T, H, Dv], the requests' states) from empty states"""
+    T = xbc.shape[0]
+    x = xbc[:, :H * Dv].double().view(T, H, Dv)
+    B, C = (xbc[:, H * Dv + i * G * N:H * Dv + (i + 1) * G * N].double().view(T, G, N).repeat_interleave(H // G, 1) for i in (0, 1))
+    dt = torch.nn.functional.softplus(raw.double() + bias.double())
+    dec = torch.exp(-torch.exp(A.double()) * dt)
+    want, at, states = torch.empty(T, H, Dv, dtype=torch.float64, device=DEV), 0, []
+    for length in lens:
+        S = torch.zeros(H, N, Dv, dtype=torch.float64, device=DEV)
+        for t in range(at, at + length):
+            S = dec[t][:, None, None] * S + (dt[t][:, None] * B[t])[:, :, None] * x[t][:, None]
+            want[t] = (S * C[t][:, :, None]).sum(1) + skip.double()[:, None] * x[t]
+        states.append(S)
+        at += length
+    return want, states
+
+
+@pytest.mark.parametrize("kind", ["rates to 16", "large steps before small ones", "forgotten at once"])
+def test_mamba2_chunks_of_strong_decays(kind):
+    """The weight of one token at another is the exponential of a difference of summed log decays, which reach -1000 and more in a
+    chunk: were the sums rounded to fp32 before they are subtracted, weights would be off by up to 6e-5.  What fp32 gives is an ulp of
+    the difference itself (below 10 where a weight matters), of the rate and of the sums: 4e-6 of a head's largest value."""
+    from scratchpad_amd import _native
+    announce("mamba2 strong decays", kind)
+    g = torch.Generator(device=DEV).manual_seed(14)
+    lens, H, G, N, Dv = [200, 65], 4, 1, 64, 64
+    T, slots = sum(lens), [1, 3]
+    A = torch.log(torch.tensor([1.0, 4.0, 16.0, 16.0], device=DEV))
+    raw, bias = torch.randn(T, H, generator=g, device=DEV), torch.zeros(H, device=DEV)
+    if kind.startswith("large"):
+        raw.fill_(-5.0)                                              # steps of 0.0067 ...
+        raw[::64], raw[20::64] = 50.0, 30.0                          # ... between steps of 50 and 30
+    if kind.startswith("forgotten"):
+        A[2] = 95.0                                                  # e^95 is past fp32: every decay is zero
+    xbc, skip = torch.randn(T, H * Dv + 2 * G * N, generator=g, device=DEV).bfloat16(), torch.zeros(H, device=DEV)
+    S = torch.full((5, H, N, Dv), float("nan"), device=DEV)
+    y = _native.mamba2_scan(xbc, raw, bias, A, skip, S, seq_extend(lens, [0, 0], slots), H, G, N, Dv).view(T, H, Dv)
+    want, states = mamba2_in_64_bits(xbc, raw, bias, A, skip, lens, H, G, N, Dv)
+    for h in range(H):
+        near(y[:, h], want[:, h], 4e-6)
+        for slot, ref in zip(slots, states):
+            near(S[slot, h], ref[h], 4e-6)
+
+
+def test_mlstm_chunks_of_closed_forget_gates():
+    """A chunk whose first 16 tokens forget nothing and whose others forget all but e^-15 each: the summed log gates reach -700, and a
+    weight taken from sums rounded to fp32 would be off by 3e-5.  Half of the values cancel in pairs (k is the same everywhere, v
+    alternates), so that what is left of them is 1e-3 of a weight; the other half is of that size and adds up.  Their ratio is what the
+    norm keeps: an error of 3e-5 would be percents of it, fp32's 1e-7 is below the result's 16-bit rounding."""
+    from scratchpad_amd import _native
+    announce("mlstm closed gates")
+    H, D, T = 2, 64, 64
+    g = torch.Generator(device=DEV).manual_seed(15)
+    one = torch.randn(1, H * D, generator=g, device=DEV).bfloat16()
+    k = q = one.expand(T, H * D).contiguous()
+    v = torch.ones(T, H * D, device=DEV)
+    v[1::2] = -1.0
+    v[:, 1::2] = 1e-4
+    v, gate = v.bfloat16(), torch.full((T, H * D), 3.0, device=DEV).bfloat16()
+    ip = torch.full((T, H), 0.25, device=DEV)
+    fp = torch.full((T, H), -40.0, device=DEV)
+    fp[:16] = 10.0
+    nw, cap, eps = torch.ones(H * D, device=DEV), 15.0, 1e-14
+    S, n, m = torch.zeros(2, H, D, D, device=DEV), torch.zeros(2, H, D, device=DEV), torch.zeros(2, H, device=DEV)
+    out = _native.mlstm_scan(q, k, v, gate, ip, fp, nw, S, n, m, seq_extend([T], [0], [1]), H, D, D, cap, eps)
+    ig, fg = cap * torch.tanh(ip.double() / cap), torch.nn.functional.logsigmoid(cap * torch.tanh(fp.double() / cap))
+    Sr, nr, mr = (torch.zeros(H, *w, dtype=torch.float64, device=DEV) for w in ((D, D), (D,), ()))
+    for t in range(16):
+        qt, kt, vt = q[t].double().view(H, D) * D ** -0.5, k[t].double().view(H, D), v[t].double().view(H, D)
+        top = torch.maximum(fg[t] + mr, ig[t])
+        keep, take = torch.exp(fg[t] + mr - top), torch.exp(ig[t] - top)
+        mr = top
+        Sr = keep[:, None, None] * Sr + take[:, None, None] * kt[:, :, None] * vt[:, None]
+        nr = keep[:, None] * nr + take[:, None] * kt
+        o = (Sr * qt[:, :, None]).sum(1) / (torch.maximum((nr * qt).sum(-1).abs(), torch.exp(-mr)) + 1e-6)[:, None]
+        want = o / torch.sqrt((o * o).mean(-1, keepdim=True) + eps) * torch.sigmoid(gate[t].double()).view(H, D)
+        if t % 2:                                                    # (the pairs are whole)
+            assert ((out[t].double().view(H, D) - want).abs() <= 2.0 ** -8 * want.abs() + 2e-3).all(), t
