@@ -593,7 +593,8 @@ SP_API int sp_causal_conv_silu(void* out, int64_t out_stride, const void* in, in
 /* Per (request, head) over the request's rows in order, S [state_size, vdim] fp32 from state[request slot] and back:
  *   dt = softplus(dt_raw[t, h] + dt_bias[h]); S = exp(-exp(A_log[h]) dt) S + dt B x^T; y = S^T C + D[h] x
  * xbc rows (in `dtype`): [x: heads * vdim | B: groups * state_size | C: groups * state_size]; y fp32 [T, heads * vdim].
- * state_size, vdim <= 256.                                                                                           */
+ * state_size, vdim <= 256.  Here and in the other recurrences a number that is not finite makes results of its own token and of
+ * later ones of its request NaN or infinite (which of the two is not specified), and touches no earlier token's.       */
 SP_API int sp_mamba2_scan(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
                           const float* dt_bias, const float* A_log, const float* Dskip, float* state, int64_t state_stride,
                           int heads, int groups, int state_size, int vdim, SP_SEQ_PARAMS, int dtype, void* stream);

@@ -18,7 +18,9 @@
 // 16 x 16 tiles of q k^T (and two of zeros) are dealt to the waves and exchanged through LDS.  Two products sum over tokens
 // and take their operands transposed: k and v are also staged as [channel][token], two tokens packed per 4-byte write.
 //
-// A value that is not finite reaches the other tokens of its chunk too (zero weights times it), not only the later ones.
+// Values that are not finite: a product with the tokens' values would carry one to the EARLIER tokens of its chunk (zero weights
+// times it), so such values are taken out of a chunk that has any (stage, clear), and in their column the outputs from their token on
+// and the state become NaN (spoil).  What is not finite in q, k, the weights or the state meets only its own tokens and later ones.
 #pragma once
 #include "seq_batch.h"
 
@@ -96,7 +98,9 @@ struct ChunkScan {
   static constexpr int kPBytes = 3 * kCL * TROW > kCL * QROW ? 3 * kCL * TROW : kCL * QROW;
   static constexpr int kSum = kP + kPBytes;                      // float [4][kCL]: sums of the weighted tiles over s
   static constexpr int kScalars = kSum + 4 * kCL * 4;
-  static constexpr int kBytes = kScalars + 2 * (int)sizeof(ChunkScalars);
+  static constexpr int kOdd = kScalars + 2 * (int)sizeof(ChunkScalars);      // int: the last chunk's number + 1 with such values
+  static constexpr int kFirst = kOdd + 16;                                   // int [Dv]: a column's first token of it
+  static constexpr int kBytes = kFirst + Dv * 4;
   static constexpr int QN = kCL * (D / 8), KN = kCL / 2 * (D / 8), VN = kCL / 2 * (Dv / 8);
   static constexpr int QU = (QN + NT - 1) / NT, KU = (KN + NT - 1) / NT, VU = (VN + NT - 1) / NT;
   static constexpr int TILES = 12 / NW + (12 % NW != 0), DT = D / 16;
@@ -117,6 +121,7 @@ struct ChunkScan {
   // the scalars of a chunk are formed while the one before it is worked on: two sets, the running chunk's in `sc`
   __device__ __forceinline__ ChunkScalars* scalars(int64_t chunk) const { return (ChunkScalars*)(lds + kScalars) + (chunk & 1); }
   __device__ __forceinline__ float* sums() const { return (float*)(lds + kSum); }
+  __device__ __forceinline__ int* odd() const { return (int*)(lds + kOdd); }
   // the d of register (i, r) and the column of this lane's part of the state
   __device__ __forceinline__ int row_of(int i, int r) const { return 32 * (i / 2) + 8 * q + 4 * (i & 1) + r; }
   __device__ __forceinline__ int column() const { return 16 * wave + r16; }
@@ -155,7 +160,7 @@ struct ChunkScan {
       *(uint32_t*)(dst + (2 * e + 1) * TROW) = __builtin_amdgcn_perm(b[e], a[e], 0x07060302u);    // the two high halves
     }
   }
-  __device__ __forceinline__ void stage() const {
+  __device__ __forceinline__ void stage(int chunk) const {
 #pragma unroll
     for (int u = 0; u < QU; ++u) {
       const int x = tid + u * NT;
@@ -173,7 +178,13 @@ struct ChunkScan {
 #pragma unroll
     for (int u = 0; u < VU; ++u) {
       const int x = tid + u * NT, t = x % (kCL / 2) * 2, c = x / (kCL / 2);
-      if (x < VN) put_transposed(lds + kVT + c * 8 * TROW + t * 2, rv[u][0], rv[u][1]);
+      if (x < VN) {
+        uint32_t ones = 0u;                            // (an exponent of ones carries into the sign)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ones |= (rv[u][e & 1][e / 2] & 0x7f807f80u) + 0x00800080u;
+        if (ones & 0x80008000u) *odd() = chunk + 1;
+        put_transposed(lds + kVT + c * 8 * TROW + t * 2, rv[u][0], rv[u][1]);
+      }
     }
   }
   static __device__ __forceinline__ void tile_of(int id, int& i, int& j) {      // ids 0 .. 9 lower tiles, 10 and 11 zeros
@@ -254,8 +265,35 @@ struct ChunkScan {
         *(u32x2*)(lds + kP + (x * kCL + t) * TROW + s0 * 2) = u32x2{part[x][0], part[x][1]};
     }
   }
+  // the values of this wave's columns without those that are not finite (lane (r16, q): 16 tokens of a column), and the first of them
+  __device__ __forceinline__ void clear() const {
+    uint16_t* v = (uint16_t*)(lds + kVT + column() * TROW) + 16 * q;
+    int first = kCL;
+    for (int t = 15; t >= 0; --t)
+      if ((v[t] & 0x7f80) == 0x7f80) {
+        v[t] = 0;
+        first = 16 * q + t;
+      }
+    first = min(first, __shfl_xor(first, 16, 64));
+    first = min(first, __shfl_xor(first, 32, 64));
+    ((int*)(lds + kFirst))[column()] = first;
+  }
+  __device__ __forceinline__ void spoil() {
+    const int first = ((const int*)(lds + kFirst))[column()];
+    const float nan = as_f32(0x7fc00000u);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[i][r] = 16 * i + 4 * q + r >= first ? nan : o[i][r];
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[i][r] = first < kCL ? nan : S[i][r];
+  }
   // o += (weighted tiles) v;  S = a_end S + k^T (w v)
-  __device__ __forceinline__ void absorb() {
+  __device__ __forceinline__ void absorb(int chunk) {
+    const bool any = __builtin_amdgcn_readfirstlane(*odd()) == chunk + 1;
+    if (any) clear();
     const float a_end = sc->a_end;
 #pragma unroll
     for (int i = 0; i < DT; ++i)
@@ -293,6 +331,7 @@ struct ChunkScan {
           for (int i = 0; i < 4; ++i) S[i0 + i] = mfma_c(a[i], b[x], S[i0 + i]);
       }
     }
+    if (any) spoil();
   }
   __device__ __forceinline__ void load_state(const float* st, bool held) {
 #pragma unroll
@@ -302,6 +341,8 @@ struct ChunkScan {
     // here before the loop over chunks: a wait for them inside it would be one for the next chunk's loads, every time
 #pragma unroll
     for (int i = 0; i < DT; ++i) asm volatile("" : "+v"(S[i]));
+    if (tid == 0) *odd() = 0;
+    lds_barrier();                                   // (before a first chunk's)
   }
   __device__ __forceinline__ void store_state(float* st) const {
 #pragma unroll

@@ -165,8 +165,9 @@ struct MlstmLds {
   static constexpr int kBytes = kGates + NW * 3 * kCL * 8;
 };
 
+// (heads of 64 x 64: registers for the two workgroups per CU that LDS has room for)
 template <int D, int NW>
-__global__ void __launch_bounds__(NW * 64)
+__global__ void __launch_bounds__(NW * 64, D == 64 ? 8 / NW : 1)
 mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_stride, const char* k, int64_t k_stride, const char* v,
                    int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre,
                    int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride,
@@ -246,7 +247,7 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
       lds_barrier();
       gates(c0);
     }
-    c.stage();
+    c.stage((int)(c0 / kCL));
     lds_barrier();
     if (c0 + kCL < len) load(c0 + kCL);
     c.scores();
@@ -293,7 +294,7 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
       if (part == 0) sn[d] = sc.a_end * sn[d] + x;
     }
     lds_barrier();
-    c.absorb();
+    c.absorb((int)(c0 / kCL));
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll

@@ -461,7 +461,7 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
   for (int64_t c0 = 0; c0 < len; c0 += kCL) {
     const int n = (int)(len - c0 < kCL ? len - c0 : kCL);
     c.sc = c.scalars(c0 / kCL);
-    c.stage();
+    c.stage((int)(c0 / kCL));
     lds_barrier();
     if (c0 + kCL < len) {
       load_steps(c0 + kCL);                           // (first: they are waited for first, and loads arrive in order)
@@ -474,7 +474,7 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
     c.template weigh<false>();
     if (c0 + kCL < len) steps(c0 + kCL);
     lds_barrier();
-    c.absorb();
+    c.absorb((int)(c0 / kCL));
     char* yc = (char*)(y + (start + c0) * y_stride + (int64_t)h * Dv);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

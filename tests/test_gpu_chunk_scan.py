@@ -297,3 +297,64 @@ def test_mlstm_chunks_of_closed_forget_gates():
         want = o / torch.sqrt((o * o).mean(-1, keepdim=True) + eps) * torch.sigmoid(gate[t].double()).view(H, D)
         if t % 2:                                                    # (the pairs are whole)
             assert ((out[t].double().view(H, D) - want).abs() <= 2.0 ** -8 * want.abs() + 2e-3).all(), t
+
+
+BAD = [float("nan"), float("inf"), float("-inf")]
+
+
+@pytest.mark.parametrize("bad", BAD, ids=str)
+@pytest.mark.parametrize("at", [0, 5, 40, 63, 70, 129])
+def test_mamba2_values_that_are_not_finite_reach_no_earlier_token(bad, at):
+    """... and no other column, head or request: all of that keeps the bits of a launch without them"""
+    from scratchpad_amd import _native
+    announce("mamba2 not finite", bad, at)
+    g = torch.Generator(device=DEV).manual_seed(16)
+    lens, H, G, N, Dv = [130, 20], 2, 1, 64, 64
+    T, slots = sum(lens), [1, 3]
+    A, bias, skip = (torch.randn(H, generator=g, device=DEV) * 0.5 - 1 for _ in range(3))
+    raw = torch.randn(T, H, generator=g, device=DEV)
+    clean = torch.randn(T, H * Dv + 2 * G * N, generator=g, device=DEV).bfloat16()
+    dirty = clean.clone()
+    dirty[at, Dv + 7] = bad                                          # head 1, column 7
+    got = []
+    for xbc in (clean, dirty):
+        S = torch.zeros(5, H, N, Dv, device=DEV)
+        got.append((_native.mamba2_scan(xbc, raw, bias, A, skip, S, seq_extend(lens, [0, 0], slots), H, G, N, Dv).view(T, H, Dv), S))
+    (y0, S0), (y1, S1) = got
+    hit = torch.zeros(T, H, Dv, dtype=torch.bool, device=DEV)
+    hit[at:130, 1, 7] = True
+    assert torch.equal(y1[~hit], y0[~hit]) and not torch.isfinite(y1[hit]).any()
+    hit = torch.zeros_like(S0, dtype=torch.bool)
+    hit[1, 1, :, 7] = True
+    assert torch.equal(S1[~hit], S0[~hit]) and not torch.isfinite(S1[hit]).any()
+
+
+@pytest.mark.parametrize("bad", BAD, ids=str)
+@pytest.mark.parametrize("where", ["q", "k", "v", "ipre", "fpre"])
+@pytest.mark.parametrize("at", [0, 40, 63, 70])
+def test_mlstm_values_that_are_not_finite_reach_no_earlier_token(at, where, bad):
+    from scratchpad_amd import _native
+    if where in ("ipre", "fpre") and bad == bad:
+        pytest.skip("an infinite gate is capped")
+    announce("mlstm not finite", where, bad, at)
+    g = torch.Generator(device=DEV).manual_seed(17)
+    lens, H, D = [100, 20], 2, 64
+    T, slots = sum(lens), [1, 3]
+    clean = {x: torch.randn(T, H * D, generator=g, device=DEV).bfloat16() for x in ("q", "k", "v", "gate")}
+    clean.update({x: torch.randn(T, H, generator=g, device=DEV) + 1 for x in ("ipre", "fpre")})
+    dirty = {x: t.clone() for x, t in clean.items()}
+    dirty[where][at, 1 if where[1:] == "pre" else D + 7] = bad       # head 1
+    nw, got = torch.rand(H * D, generator=g, device=DEV) + 0.5, []
+    for x in (clean, dirty):
+        S, n, m = torch.zeros(5, H, D, D, device=DEV), torch.zeros(5, H, D, device=DEV), torch.zeros(5, H, device=DEV)
+        got.append((_native.mlstm_scan(x["q"], x["k"], x["v"], x["gate"], x["ipre"], x["fpre"], nw, S, n, m,
+                                       seq_extend(lens, [0, 0], slots), H, D, D, 15.0, 1e-5).view(T, H, D), S, n))
+    (y0, S0, n0), (y1, S1, n1) = got
+    hit = torch.zeros(T, H, D, dtype=torch.bool, device=DEV)
+    hit[at:at + 1 if where == "q" else 100, 1] = True                # a query touches its own token only
+    assert torch.equal(y1[~hit], y0[~hit]) and not torch.isfinite(y1[hit]).any()
+    assert torch.equal(S1[:, 0], S0[:, 0]) and torch.equal(S1[3], S0[3]) and torch.equal(n1[3], n0[3])
+    if where == "v":
+        assert torch.equal(n1, n0) and not torch.isfinite(S1[1, 1, :, 7]).any()
+        hit = torch.arange(D, device=DEV) == 7
+        assert torch.equal(S1[1, 1][:, ~hit], S0[1, 1][:, ~hit])
