@@ -22,7 +22,8 @@
 // of 300 tokens 45 -> 33; below 8 tokens per request the per-token kernel is the faster one (1 token: 39 against 51 us).
 // With one decay per head: 8 requests 364 -> 179, one request 2101 -> 672, 16 requests of 300 tokens 41 -> 33.
 //
-// A value that is not finite reaches the other tokens of its chunk too (zero weights times it), not only the later ones.
+// A u that is not finite would reach the EARLIER tokens of its chunk too (zeros of (I + A)^{-1} and P times it): where a column has
+// one, its read-outs are formed again without the rows from the first such token on, which become NaN, as does the column's state.
 #pragma once
 #include "seq_batch.h"
 
@@ -219,7 +220,7 @@ __global__ void __launch_bounds__(D * 2) delta_chunk_prepare_kernel(DeltaChunks 
 #pragma unroll
     for (int j = 0; j < t; ++j) y -= sA[t][j] * x[j];
     x[t] = y;
-    if (lane < kDC) work[kDcT + t * kDC + s] = y * sbeta[s];
+    if (lane < kDC) work[kDcT + t * kDC + s] = t >= s ? y * sbeta[s] : 0.f;      // (a step size that is not finite: zeros stay)
   }
 }
 
@@ -423,17 +424,45 @@ __global__ void __launch_bounds__(768) delta_chunk_scan_kernel(DeltaChunks a, Se
     __builtin_amdgcn_sched_barrier(0);
     f32x4_d u = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) u = mfma_d(tr[r], v[r] - kd[r], u);
+    for (int r = 0; r < 4; ++r) {
+      v[r] -= kd[r];
+      u = mfma_d(tr[r], v[r], u);
+    }
 #pragma unroll
     for (int i = 0; i < DT; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) S[i][r] *= g[i][r];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r], S[i]);
-      o = mfma_d(pr[r], u[r], o);
+    int first = kDC;                                  // the column's first token whose u is not finite
+    const float probe = fmaf(u[0], 0.f, fmaf(u[1], 0.f, fmaf(u[2], 0.f, u[3] * 0.f)));
+    if (__ballot(probe != probe)) {
+      const auto finite = [](float x) { return fabsf(x) < INFINITY; };
+#pragma unroll
+      for (int r = 3; r >= 0; --r)
+        if (!finite(v[r])) {
+          v[r] = 0.f;
+          first = 4 * q + r;
+        }
+      u = f32x4_d{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u = mfma_d(tr[r], v[r], u);
+#pragma unroll
+      for (int r = 3; r >= 0; --r)
+        if (!finite(u[r])) first = min(first, 4 * q + r);
+      first = min(first, __shfl_xor(first, 16, 64));
+      first = min(first, __shfl_xor(first, 32, 64));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[r] = 4 * q + r < first ? u[r] : 0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o = mfma_d(pr[r], u[r], o);
+    if (__ballot(first < kDC)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = 4 * q + r < first ? o[r] : as_f32(0x7fc00000u);
     }
     if (live) {
 #pragma unroll

@@ -358,3 +358,44 @@ def test_mlstm_values_that_are_not_finite_reach_no_earlier_token(at, where, bad)
         assert torch.equal(n1, n0) and not torch.isfinite(S1[1, 1, :, 7]).any()
         hit = torch.arange(D, device=DEV) == 7
         assert torch.equal(S1[1, 1][:, ~hit], S0[1, 1][:, ~hit])
+
+
+@pytest.mark.parametrize("bad", BAD, ids=str)
+@pytest.mark.parametrize("where", ["q", "k", "v", "beta", "decay"])
+@pytest.mark.parametrize("at", [0, 9, 15, 16, 40])
+@pytest.mark.parametrize("channel", [True, False], ids=["gated", "head"])
+def test_delta_values_that_are_not_finite_reach_no_earlier_token(channel, at, where, bad):
+    from scratchpad_amd import _native
+    if bad == bad and where in ("beta", "decay"):
+        pytest.skip("an infinite step size or decay is a number")
+    announce("delta not finite", channel, where, bad, at)
+    g = torch.Generator(device=DEV).manual_seed(18)
+    lens, H, D, Dv = [61, 30], 2, 64, 64
+    T, slots = sum(lens), [1, 3]
+    rn = lambda n: torch.randn(T, n, generator=g, device=DEV)  # noqa: E731
+    clean = {"q": rn(H * D).bfloat16(), "k": rn(H * D).bfloat16(), "v": rn(H * Dv).bfloat16(), "gate": rn(H * Dv).bfloat16(),
+             "beta": rn(H).bfloat16(), "decay": torch.rand(T, H * D, generator=g, device=DEV), "pre": rn(2 * H)}
+    dirty = {x: t.clone() for x, t in clean.items()}
+    if not channel and where in ("beta", "decay"):
+        dirty["pre"][at, 1 + (H if where == "decay" else 0)] = bad
+    else:
+        dirty[where][at, 1 if where == "beta" else D + 7] = bad
+    nw, dt_bias, A_log = (torch.rand(n, generator=g, device=DEV) for n in (Dv, H, H))
+    seq, got = seq_extend(lens, [0, 0], slots), []
+    for x in (clean, dirty):
+        S = torch.zeros(5, H, D, Dv, device=DEV)
+        if channel:
+            assert _native._delta_chunks_take(x["q"], x["k"], x["v"], x["decay"], seq, D, Dv)
+            y = _native.gated_delta_scan(x["q"], x["k"], x["v"], x["beta"], x["decay"], x["gate"].float().abs(), nw, S, seq, H, H, D, Dv, 1e-5)
+        else:
+            assert _native._delta_chunks_take(x["q"], x["k"], x["v"], None, seq, D, Dv)
+            y = _native.head_delta_scan(x["q"], x["k"], x["v"], x["gate"], x["pre"], dt_bias, A_log, nw, S, seq, H, H, D, Dv, 1e-5)
+        got.append((y.view(T, H, Dv), S))
+    (y0, S0), (y1, S1) = got
+    hit = torch.zeros(T, H, Dv, dtype=torch.bool, device=DEV)
+    hit[at:at + 1 if where == "q" else 61, 1] = True
+    assert torch.equal(y1[~hit], y0[~hit]) and not torch.isfinite(y1[hit]).any()
+    assert torch.equal(S1[:, 0], S0[:, 0]) and torch.equal(S1[3], S0[3])
+    if where == "v":
+        hit = torch.arange(Dv, device=DEV) == 7
+        assert torch.equal(S1[1, 1][:, ~hit], S0[1, 1][:, ~hit]) and not torch.isfinite(S1[1, 1][:, hit]).any()
