@@ -399,3 +399,23 @@ def test_delta_values_that_are_not_finite_reach_no_earlier_token(channel, at, wh
     if where == "v":
         hit = torch.arange(Dv, device=DEV) == 7
         assert torch.equal(S1[1, 1][:, ~hit], S0[1, 1][:, ~hit]) and not torch.isfinite(S1[1, 1][:, hit]).any()
+
+
+@pytest.mark.parametrize("T", [40, 64, 129])
+def test_lowrank_decays_of_all_rates(T):
+    """exp(-rate softplus(z)) at the accuracy of fp32 functions - the product's, an ulp or two of softplus, rate and exponential -
+    whichever form a step takes: rates to 16, softplus from 2e-9 (a channel that hardly forgets) up"""
+    from scratchpad_amd import _native
+    announce("lowrank_gate of all rates", T)
+    rank, channels = 32, 1024
+    p, w2t = torch.zeros(T, rank, device=DEV).bfloat16(), torch.zeros(rank, channels, device=DEV)
+    bias = torch.linspace(-20, 15, channels // 8, device=DEV).repeat(8).contiguous()                     # z exactly
+    A = torch.log(torch.tensor([0.05, 0.4, 1.0, 2.0, 4.0, 8.0, 12.0, 16.0], device=DEV))
+    x = torch.exp(A.double()).repeat_interleave(channels // 8) * torch.nn.functional.softplus(bias.double())
+    want = torch.exp(-x)
+    got = _native.lowrank_gate(p, w2t, bias, "decay", A).double()
+    # half an ulp of the result and its exponential's ulp; three roundings of the exponent (rate, softplus, their product)
+    bar = want * (1.5 * 2.0 ** -23 + 6 * 2.0 ** -24 * x) + 1e-38
+    assert ((got - want).abs() <= bar).all(), float(((got - want).abs() / bar).max())
+    sig = torch.sigmoid(bias.double())
+    assert ((_native.lowrank_gate(p, w2t, bias, "sigmoid").double() - sig).abs() <= 4 * 2.0 ** -23 * sig).all()
