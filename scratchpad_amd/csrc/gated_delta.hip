@@ -137,6 +137,14 @@ lowrank_gate_mfma_kernel(float* out, const char* p, int64_t p_stride, const floa
     if (t0 + r16 < t1) {
       f32x4_c o;
 #pragma unroll
+      for (int r = 0; r < 4; ++r) {                    // an infinity's parts are not numbers: such a sum is formed again as it is
+        if (fabsf(z[r]) < INFINITY) continue;
+        const int c = c0 + 4 * q + r;
+        float sum = b[r];
+        for (int x = 0; x < RANK; ++x) sum += w2t[(int64_t)x * channels + c] * Elem<bf16_tag>::load(p, t * p_stride + x);
+        z[r] = sum;
+      }
+#pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = gate_value<ACT>(z[r], rate[r]);
       *(f32x4_c*)(out + t * channels + c0 + 4 * q) = o;
     }

@@ -65,7 +65,7 @@ small_linear_f32_kernel(float* out, const void* x, int64_t x_stride, const float
 // exact (split3), x is bf16 already, the sums are fp32.  A workgroup takes 32 tokens x 16 NT outputs; its 8 waves share K (a
 // stretch each, two 32-deep steps of it in flight) and add up through LDS in wave order.  4096 tokens x 2048, us, with the library's
 // fp32 product behind a copy of x to fp32 -> now: 64 outputs 29.3 -> 14.9, 32 outputs 27.0 -> 10.2; 65 rows of 64 outputs
-// 24.8 -> 9.7.  (A weight or value that is not finite makes the sums it enters NaN, infinite ones too.)
+// 24.8 -> 9.7.  An infinity has no parts that are numbers: a sum that is not finite is formed again, element by element.
 constexpr int kLinTokens = 32, kLinWaves = 8;
 template <int NT>
 __global__ void __launch_bounds__(kLinWaves * 64)
@@ -142,6 +142,10 @@ linear_f32_mfma_kernel(float* out, const char* x, int64_t x_stride, const float*
     float v = 0.f;
 #pragma unroll
     for (int u = 0; u < kLinWaves / 2; ++u) v += part[u][t][n];
+    if (!(fabsf(v) < INFINITY)) {
+      v = 0.f;
+      for (int k = 0; k < K; ++k) v += w[(int64_t)(n0 + n) * K + k] * Elem<bf16_tag>::load(x, (t0 + t) * x_stride + k);
+    }
     out[(t0 + t) * N + n0 + n] = v + (bias ? bias[n0 + n] : 0.f);
   }
 }

@@ -419,3 +419,19 @@ def test_lowrank_decays_of_all_rates(T):
     assert ((got - want).abs() <= bar).all(), float(((got - want).abs() / bar).max())
     sig = torch.sigmoid(bias.double())
     assert ((_native.lowrank_gate(p, w2t, bias, "sigmoid").double() - sig).abs() <= 4 * 2.0 ** -23 * sig).all()
+
+
+def test_lowrank_gate_of_infinite_inputs():
+    from scratchpad_amd import _native
+    T, rank, channels = 64, 64, 32
+    p, w2t = torch.ones(T, rank, device=DEV).bfloat16(), torch.full((rank, channels), 0.5, device=DEV)
+    p[3, 5], p[9, 60], p[17, 2] = float("inf"), float("-inf"), float("nan")
+    w2t[7, 31] = float("inf")
+    decay, sig = _native.lowrank_gate(p, w2t, None, "decay", torch.zeros(2, device=DEV)), _native.lowrank_gate(p, w2t, None, "sigmoid")
+    plain = p.float() @ w2t                                           # (no infinity meets a zero: the sums are infinite, not NaN)
+    assert torch.isnan(decay[17]).all() and torch.isnan(sig[17]).all()
+    keep = torch.arange(T, device=DEV) != 17
+    assert torch.isinf(plain[3]).all() and (plain[9, :31] == float("-inf")).all() and torch.isnan(plain[9, 31])
+    for got, ref in ((decay, torch.exp(-torch.nn.functional.softplus(plain))), (sig, torch.sigmoid(plain))):
+        assert torch.equal(torch.isnan(got[keep]), torch.isnan(ref[keep]))
+        assert torch.allclose(got[keep], ref[keep], rtol=1e-5, atol=1e-6, equal_nan=True)

@@ -104,3 +104,17 @@ def test_fp32_products_of_many_rows(T, K, n, bias):
     want = x.double() @ w.double().T + (b.double() if bias else 0.0)
     bound = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + (b.double().abs() if bias else 0.0))
     assert out.shape == (T, n) and bool(((out.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("T", [64, 65, 100])
+def test_fp32_products_of_infinite_inputs(T):
+    """an infinity is one in the sum it enters, in every form: not NaN"""
+    from scratchpad_amd import _native
+    K, n = 96, 20
+    x, w = torch.ones(T, K, device=DEV).bfloat16(), torch.full((n, K), 0.5, device=DEV)
+    x[3, 5], x[60, 95], x[9, 0] = float("inf"), float("-inf"), float("nan")
+    w[7, 31], w[8, 2] = float("inf"), 1.1                             # (1.1: a weight of three parts)
+    want = torch.nn.functional.linear(x.cpu().double(), w.cpu().double())
+    got = _native.small_linear_f32(x, w).cpu().double()
+    assert torch.isnan(want[9]).all() and torch.isinf(want[3]).all() and torch.isnan(want[60, 7])
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.allclose(got, want, rtol=1e-5, equal_nan=True)
