@@ -316,10 +316,9 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
       for (int r = 0; r < 4; ++r) {
         const int t = 16 * i + 4 * c.q + r;
         const float gate = bf16_bits_to_f32(gv[i][r]), f = __shfl(factor, t, 64);
-        // (the result is rounded to 16 bits: the hardware's exponential and reciprocal, 1 ulp each, are far below that)
         if (t < n)
           E::store(ob + c0 * out_stride * 2 + (uint32_t)(t * (uint32_t)out_stride + col) * 2u, 0,
-                   c.o[i][r] * f * nw * __builtin_amdgcn_rcpf(1.f + __expf(-gate)));
+                   c.o[i][r] * f * nw / (1.f + expf(-gate)));
       }
   }
   c.store_state(Sst);

@@ -143,7 +143,8 @@ __device__ __forceinline__ u32x4 pack16<f16_tag>(const float* f) {
 
 // SiLU as the reference's torch path evaluates it in fp32 (nn/layers/activation.py:22-24): a / (1 + exp(-a)), every
 // operation rounded on its own whatever the translation unit's contraction mode (shared by sp_silu_and_mul and the
-// fused prologue of sp_gemm_skinny, which must agree bit for bit)
+// fused epilogue of sp_gemm_skinny, which must agree bit for bit).  16-bit results take it too: the hardware's exponential alone is
+// off by |a| ulp, and its reciprocal of numbers past 2^126 is zero.
 __device__ __forceinline__ float silu_ref(float a) { return __fdiv_rn(a, __fadd_rn(1.0f, expf(-a))); }
 
 // the tanh form of GELU in fp32 (sp_gelu_tanh_and_mul and the fused epilogue of sp_gemm_skinny share it)
@@ -157,17 +158,6 @@ __device__ __forceinline__ float mul_f32(float a, float b) {
   float r = a * b;
   asm("" : "+v"(r));
   return r;
-}
-
-// z * sigmoid(z) for results that are rounded to 16 bits: the hardware's exponential and reciprocal (1 ulp of fp32 each) in place
-// of the library's exponential and the divide's refinement, a quarter of their instructions.  fp32 results keep the exact form.
-template <typename Tag>
-__device__ __forceinline__ float silu_for(float z) {
-  return z * __builtin_amdgcn_rcpf(1.f + __expf(-z));
-}
-template <>
-__device__ __forceinline__ float silu_for<f32_tag>(float z) {
-  return z / (1.f + expf(-z));
 }
 
 __device__ __forceinline__ u32x4 ld16(const void* p) { return *(const u32x4*)p; }

@@ -236,7 +236,7 @@ conv_silu_run_kernel(void* out, int64_t out_stride, const void* in, int64_t in_s
         float acc = bs[x];
 #pragma unroll
         for (int j = 0; j < TAPS; ++j) acc += wt[j][x] * past[j][x];
-        o[x] = silu_for<Tag>(acc);
+        o[x] = silu_ref(acc);
 #pragma unroll
         for (int j = 0; j < TAPS - 1; ++j) past[j][x] = past[j + 1][x];
       }
@@ -270,7 +270,7 @@ conv_silu_run_kernel(void* out, int64_t out_stride, const void* in, int64_t in_s
       float acc = bs[x];
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) acc += wt[j][x] * past[j][x];
-      o[x] = silu_for<Tag>(acc);
+      o[x] = silu_ref(acc);
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) past[j][x] = past[j + 1][x];
     }
@@ -539,7 +539,7 @@ gated_group_norm_vec_kernel(void* out, int64_t out_stride, const float* y, int64
     unpack16<Tag>(zr[u], zf);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      v[u][e] = as_f32(e < 4 ? ya[u][e] : yb[u][e - 4]) * silu_for<Tag>(zf[e]);
+      v[u][e] = as_f32(e < 4 ? ya[u][e] : yb[u][e - 4]) * silu_ref(zf[e]);
       ss += v[u][e] * v[u][e];
     }
   }

@@ -118,3 +118,21 @@ def test_fp32_products_of_infinite_inputs(T):
     got = _native.small_linear_f32(x, w).cpu().double()
     assert torch.isnan(want[9]).all() and torch.isinf(want[3]).all() and torch.isnan(want[60, 7])
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.allclose(got, want, rtol=1e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_silu_of_every_16_bit_value(dtype):
+    """the convolution's SiLU of every number of the type: its one rounding and little else"""
+    from scratchpad_amd import _native
+    C, T = 1024, 64
+    x = torch.arange(65536, dtype=torch.int32, device=DEV).to(torch.int16).view(dtype).view(T, C).clone()
+    x[~torch.isfinite(x)] = 0.0
+    w = torch.zeros(C, 4, device=DEV)
+    w[:, 3] = 1.0
+    got = _native.causal_conv_silu(x, w, None, torch.zeros(2, 3, C, device=DEV), seq_extend([T], [0], [1])).double()
+    want = x.double() * torch.sigmoid(x.double())
+    half = torch.exp2(torch.frexp(want)[1].double() - 1 - (8 if dtype == torch.bfloat16 else 11))          # half a step at the result
+    # what fp32 adds: four roundings.  Its exponential ends at e^88.72: below -88.72 the result is zero, 2.7e-37 off; subnormal halves
+    # keep 2^-25
+    floor = 3e-37 if dtype == torch.bfloat16 else 2.0 ** -25
+    assert ((got - want).abs() <= half + 2.0 ** -22 * want.abs() + floor).all()
