@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_scalar_kernel(void* out,  // m
 // ACT 1: gelu_tanh(a) * b, the product of two fp32 values rounded once.
 template <typename Tag, int ACT>
 __device__ __forceinline__ float glu_f32(float a, float b) {
-  if constexpr (ACT == 1) return mul_f32(gelu_tanh_f32(a), b);
+  if constexpr (ACT == 1) return mul_round<Tag>(gelu_tanh_f32(a), b);
   else return __fmul_rn(Elem<Tag>::round(silu_ref(a)), b);   // sp_common.h
 }
 

@@ -85,7 +85,7 @@ template <typename Tag, int EPI>
 __device__ __forceinline__ float glu_value(float gate, float up) {
   typedef Elem<Tag> E;
   const float act = EPI == 3 ? gelu_tanh_f32(E::round(gate)) : E::round(silu_ref(E::round(gate)));
-  return mul_f32(act, E::round(up));
+  return mul_round<Tag>(act, E::round(up));
 }
 
 // ---- 1 row

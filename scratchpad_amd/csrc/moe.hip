@@ -293,18 +293,19 @@ struct GroupedArgs {
 };
 
 // (shared by the separate launch and the fused epilogue, which agree bit for bit)
-__device__ __forceinline__ float moe_glu_f32(float g, float u, float limit, float alpha) {
+template <typename Tag>
+__device__ __forceinline__ float moe_glu_value(float g, float u, float limit, float alpha) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return mul_f32(g / (1.f + expf(-alpha * g)), u + 1.f);
+  return mul_round<Tag>(g / (1.f + expf(-alpha * g)), u + 1.f);
 }
 
 template <typename Tag, int ACT>
 __device__ __forceinline__ float grouped_act(float v, float up, const GroupedArgs& p) {
   typedef Elem<Tag> El;
   if constexpr (ACT == 1) return gemm_act(v, 1);
-  if constexpr (ACT == 2) return mul_f32(El::round(silu_ref(El::round(v))), El::round(up));
-  if constexpr (ACT == 3) return moe_glu_f32(El::round(v), El::round(up), p.limit, p.alpha);
+  if constexpr (ACT == 2) return mul_round<Tag>(El::round(silu_ref(El::round(v))), El::round(up));
+  if constexpr (ACT == 3) return moe_glu_value<Tag>(El::round(v), El::round(up), p.limit, p.alpha);
   return v;
 }
 
@@ -712,7 +713,7 @@ __global__ void moe_glu_kernel(void* out, const void* gu, int64_t P, int F, floa
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t p = i / F;
     const int f = (int)(i % F);
-    El::store(out, i, moe_glu_f32(El::load(gu, p * 2 * F + f), El::load(gu, p * 2 * F + F + f), limit, alpha));
+    El::store(out, i, moe_glu_value<Tag>(El::load(gu, p * 2 * F + f), El::load(gu, p * 2 * F + F + f), limit, alpha));
   }
 }
 

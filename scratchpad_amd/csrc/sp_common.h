@@ -152,12 +152,18 @@ __device__ __forceinline__ float gelu_tanh_f32(float a) {
   return 0.5f * a * (1.0f + tanhf(0.7978845608028654f * (a + 0.044715f * a * a * a)));
 }
 
-// a * b rounded to fp32 before anything else happens to it: a product that is then rounded to fp16 would otherwise become one
-// v_fma_mixlo_f16, which rounds once - in one kernel and perhaps not in the next
-__device__ __forceinline__ float mul_f32(float a, float b) {
-  float r = a * b;
-  asm("" : "+v"(r));
-  return r;
+// a * b of two fp32 factors rounded to Tag's type, as a float that the store's conversion leaves alone.  In fp16 that is ONE rounding
+// of the exact product, by the instruction that does it: the compiler picks it for a product that is stored in fp16 in some kernels
+// and two roundings in others, and forms of one operation have to agree bit for bit.
+template <typename Tag>
+__device__ __forceinline__ float mul_round(float a, float b) {
+  return __fmul_rn(a, b);
+}
+template <>
+__device__ __forceinline__ float mul_round<f16_tag>(float a, float b) {
+  uint32_t h;
+  asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(h) : "v"(a), "v"(b), "v"(-0.f));      // (- 0: the sign of a zero product stays)
+  return f16_bits_to_f32((uint16_t)h);
 }
 
 __device__ __forceinline__ u32x4 ld16(const void* p) { return *(const u32x4*)p; }
