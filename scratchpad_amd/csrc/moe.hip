@@ -673,10 +673,11 @@ __global__ void __launch_bounds__(64) moe_grouped_rows_kernel(GroupedArgs p) {
 template <typename Tag, int ACT>
 int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
   const int held = pairs < p.E ? pairs : p.E;                    // experts with a row, at most
-  if (pairs <= 10 * (int64_t)p.E) {
-    const int tiles = pairs / 16 + held, per = ACT >= 2 ? 16 : 32;
-    if (tiles > 65535) return SP_ERR_UNSUPPORTED;                // (4096 experts, the most moe_align takes: 6656)
-    moe_grouped_rows_kernel<Tag, ACT><<<dim3((unsigned)((p.N + per - 1) / per), (unsigned)tiles), 64, 0, st>>>(p);
+  const int row_tiles = pairs / 16 + held;
+  // (moe_align takes 4096 experts, 6656 tiles; more than a grid's second dimension holds go to the 64-row tiles)
+  if (pairs <= 10 * (int64_t)p.E && row_tiles <= 65535) {
+    const int per = ACT >= 2 ? 16 : 32;
+    moe_grouped_rows_kernel<Tag, ACT><<<dim3((unsigned)((p.N + per - 1) / per), (unsigned)row_tiles), 64, 0, st>>>(p);
     SP_LAUNCH_CHECK();
     return SP_OK;
   }

@@ -71,6 +71,18 @@ def test_gated_form_leaves_other_shapes_to_the_two_steps():
         assert _native.moe_grouped_glu(a, w, offsets, P, order, 2, "silu") is None
 
 
+def test_few_rows_of_very_many_experts():
+    """more row tiles than a launch's second dimension holds"""
+    from scratchpad_amd import _native
+    E, N, K = 70000, 32, 32
+    g = torch.Generator(device=DEV).manual_seed(3)
+    a, w = (torch.randn(E, *s, generator=g, device=DEV).bfloat16() for s in ((K,), (N, K)))
+    offsets = torch.arange(E + 1, dtype=torch.int32, device=DEV)
+    got = _native.moe_grouped_gemm(a, w, offsets, E)
+    want = (a.float()[:, None] * w.float()).sum(-1)
+    assert ((got.float() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -22 * (a.float().abs()[:, None] * w.float().abs()).sum(-1)).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T,width,top", [(1, 8, 1), (5, 264, 4), (3, 2056, 6), (9, 37, 5)])
 def test_combine(T, width, top, dtype):
