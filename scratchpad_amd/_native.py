@@ -1545,7 +1545,17 @@ def window_attention(q: torch.Tensor, kpool: torch.Tensor, vpool: torch.Tensor, 
     return out
 
 
-SMALL_LINEAR_OWN_ROWS = 64      # up to this many rows a workgroup per row; above, tiles where there are any for the type
+SMALL_LINEAR_OWN_ROWS = 64      # up to this many rows a workgroup per row; above, tiles where they pay
+
+
+def small_linear_tiles_pay(T: int, K: int, n: int) -> bool:
+    """Where the tiles for more than 64 bf16 rows measured faster than a copy of x to fp32 and the library's product (us, tiles /
+    library).  Their 8 waves share K in one workgroup, a chain that few rows of a long K do not hide (64 outputs of K 4096: 65 rows
+    17.6 / 14.2, 512 rows 17.9 / 18.8; of K 8192: 512 rows 32.5 / 28.7, 1024 rows 32.6 / 33.6).  They read x once per 32 outputs:
+    the library's larger tiles win with outputs and rows (K 2048: 4096 rows of 256 50.9 / 53.8, of 512 91 / 77, 8192 rows of 128
+    50.0 / 56.2, of 256 94.9 / 87.8; K 4096: 2048 rows of 256 49.0 / 49.7, 4096 of 256 93.7 / 87.8; few rows of many outputs: K 2048,
+    256 rows of 1024 17.5 / 18.8, of 2048 28.7 / 26.5)."""
+    return (K <= 2048 or 8 * T >= K) and (n <= 128 or (n <= 256 and T * K <= 1 << 23) or (K <= 2048 and T * n <= 1 << 18))
 
 
 def small_linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -1554,9 +1564,10 @@ def small_linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     if weight.dim() != 2 or weight.shape[1] != x.shape[1] or (bias is not None and _f32(bias, "bias").shape[0] != weight.shape[0]):
         raise RuntimeError("small_linear_f32: weight [n, k], bias [n]")
     if x.shape[0] > SMALL_LINEAR_OWN_ROWS and not (x.dtype == torch.bfloat16 and x.shape[1] % 32 == 0 and x.stride(0) % 8 == 0
-                                                   and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
-        # many rows of types or lengths without a tiled form (see sp_small_linear_f32): the kernel for few reads the weight rows
-        # again for every token, the library's fp32 product tiles them
+                                                   and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+                                                   and small_linear_tiles_pay(x.shape[0], x.shape[1], weight.shape[0])):
+        # many rows where sp_small_linear_f32's tiles do not pay, or of types or lengths without them: the kernel for few rows reads
+        # the weight rows again for every token, the library's fp32 product tiles them
         return torch.nn.functional.linear(x.to(torch.float32), weight, bias)
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=x.device)
     _check(load().sp_small_linear_f32(out.data_ptr(), x.data_ptr(), x.stride(0), weight.data_ptr(), _ptr(bias), x.shape[0],

@@ -234,6 +234,17 @@ def test_skinny_gemm_takes_the_head_of_few_rows():
     assert not pays(5, 128256, 4096) and not pays(9, 128256, 2048) and not pays(3, 4096, 14336)
 
 
+def test_fp32_product_dispatch_rule():
+    """the tiles for many bf16 rows where they measured faster than the library, the library elsewhere"""
+    from scratchpad_amd import _native
+    pays = _native.small_linear_tiles_pay
+    assert pays(65, 2048, 32) and pays(16384, 2048, 64) and pays(8192, 2048, 128) and pays(4096, 2048, 256) and pays(256, 2048, 1024)
+    assert pays(512, 4096, 64) and pays(2048, 4096, 256) and pays(1024, 8192, 64)
+    assert not pays(65, 4096, 64) and not pays(256, 4096, 16) and not pays(512, 8192, 64)             # a long chain, few rows
+    assert not pays(8192, 2048, 256) and not pays(4096, 2048, 512) and not pays(4096, 4096, 256)      # many outputs of many rows
+    assert not pays(256, 2048, 2048) and not pays(65, 4096, 2048)
+
+
 def test_mlstm_scan_takes_no_gate_rows_that_overlap(monkeypatch):
     """gates whose rows lie closer than their width (an expanded row, a sliding view) are refused before anything is launched: the
     kernel reads [token, head] at rows at least `heads` apart.  Views of one product and strides that differ pass."""
