@@ -221,15 +221,11 @@ __global__ __launch_bounds__(kQuadWaves * 64) void gemm_quad_kernel(SkinnyArgs a
 }
 
 // ---- 5-16 rows
-constexpr int kSkWaves = 8;
-
-// NT (sp_debug_set("skinny_nt", 1); OFF by default): non-temporal weight loads.  They lose: 1 row qkv 14.5 vs 13.6 us, gate_up
-// 46.5 vs 43.3, LM head 186 vs 166.
-__device__ __forceinline__ u32x4 ld16_nt(const void* p) { return __builtin_nontemporal_load((const u32x4*)p); }
+constexpr int kSkWaves = 8, kSkUnroll = 4;
 
 // EPI 1 and 3: a.N = I output columns; the 16 W rows of a workgroup are gate rows n0 .. n0+7 (tile rows 0-7) and up rows
 // I + n0 .. I + n0 + 7 (tile rows 8-15)
-template <typename Tag, int UNROLL, bool NT, int EPI>
+template <typename Tag, int EPI>
 __global__ __launch_bounds__(kSkWaves * 64) void gemm_skinny_kernel(SkinnyArgs a) {
   typedef Elem<Tag> E;
   constexpr bool GLU = EPI == 1 || EPI == 3;
@@ -245,19 +241,19 @@ __global__ __launch_bounds__(kSkWaves * 64) void gemm_skinny_kernel(SkinnyArgs a
   const int ksteps = a.K / 32;
   f32x4_g acc = {0.f, 0.f, 0.f, 0.f};
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  // this wave's k-steps: UNROLL in a row, then UNROLL more kSkWaves * UNROLL steps on, all loads of a group first
-  for (int ks = wave * UNROLL; ks < ksteps; ks += UNROLL * kSkWaves) {
-    u32x4 wf[UNROLL], xf[UNROLL];
+  // this wave's k-steps: kSkUnroll in a row, then kSkUnroll more kSkWaves * kSkUnroll steps on, all loads of a group first
+  for (int ks = wave * kSkUnroll; ks < ksteps; ks += kSkUnroll * kSkWaves) {
+    u32x4 wf[kSkUnroll], xf[kSkUnroll];
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
+    for (int u = 0; u < kSkUnroll; ++u) {
       const int64_t off = (int64_t)(ks + u) * 64;
       const bool in = ks + u < ksteps;
-      wf[u] = in ? (NT ? ld16_nt(wp + off) : ld16(wp + off)) : zero;
+      wf[u] = in ? ld16(wp + off) : zero;
       xf[u] = in && mrow ? ld16(xp + off) : zero;
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) acc = mfma_g<Tag>(wf[u], xf[u], acc);
+    for (int u = 0; u < kSkUnroll; ++u) acc = mfma_g<Tag>(wf[u], xf[u], acc);
   }
   // acc[r] = partial of out[m = r16][n0 + 4q + r]; sum the waves in wave order
 #pragma unroll
@@ -284,12 +280,6 @@ __global__ __launch_bounds__(kSkWaves * 64) void gemm_skinny_kernel(SkinnyArgs a
   }
 }
 
-static int g_skinny_nt = 0;     // sp_debug_set("skinny_nt", 0 / 1): A/B switch of the non-temporal weight loads
-void set_skinny_nt(int v) { g_skinny_nt = v; }
-// sp_debug_set("skinny_unroll16", 0 / 1): 16 k-steps of loads in flight per wave in place of 4
-static int g_skinny_u16 = 0;
-void set_skinny_unroll16(int v) { g_skinny_u16 = v; }
-
 // One group of 4 weight rows up to 2048 rows: 256 workgroups of two groups there (3 rows, K 4096, us: 1024 rows 4.6 one / 6.3 two,
 // 2048 rows 6.3 / 6.9, 2560 rows 7.8 / 8.9, 8192 rows 16.0 / 14.6).
 constexpr int kQuadOneGroup = 2048;
@@ -312,10 +302,7 @@ static void launch_skinny_as(const SkinnyArgs& a, hipStream_t st) {
     }
   } else {
     constexpr int cols = GLU ? 8 : 16;
-    const dim3 grid((a.N + cols - 1) / cols), block(kSkWaves * 64);
-    if (g_skinny_u16) gemm_skinny_kernel<Tag, 16, false, EPI><<<grid, block, 0, st>>>(a);
-    else if (g_skinny_nt) gemm_skinny_kernel<Tag, 4, true, EPI><<<grid, block, 0, st>>>(a);
-    else gemm_skinny_kernel<Tag, 4, false, EPI><<<grid, block, 0, st>>>(a);
+    gemm_skinny_kernel<Tag, EPI><<<dim3((a.N + cols - 1) / cols), dim3(kSkWaves * 64), 0, st>>>(a);
   }
 }
 
