@@ -598,6 +598,12 @@ SP_API int sp_causal_conv_silu(void* out, int64_t out_stride, const void* in, in
 SP_API int sp_mamba2_scan(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
                           const float* dt_bias, const float* A_log, const float* Dskip, float* state, int64_t state_stride,
                           int heads, int groups, int state_size, int vdim, SP_SEQ_PARAMS, int dtype, void* stream);
+/* The same with the step's number of rows (< 0: not known), by which short portions of many requests take the form that is faster
+ * for them. */
+SP_API int sp_mamba2_scan_tokens(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
+                                 const float* dt_bias, const float* A_log, const float* Dskip, float* state, int64_t state_stride,
+                                 int64_t num_tokens, int heads, int groups, int state_size, int vdim, SP_SEQ_PARAMS, int dtype,
+                                 void* stream);
 /* out = (y * silu(z)) / rms_part * weight: each row of n values normed in `parts` equal parts (y fp32; z, out in `dtype`) */
 SP_API int sp_gated_group_norm(void* out, int64_t out_stride, const float* y, int64_t y_stride, const void* z,
                                int64_t z_stride, const float* weight, int64_t num_tokens, int n, int parts, float eps,
@@ -612,7 +618,13 @@ SP_API int sp_mlstm_scan(void* out, int64_t out_stride, const void* q, int64_t q
                          const float* fpre, const float* norm_w, float* S_state, int64_t S_stride, float* n_state,
                          int64_t n_stride, float* m_state, int64_t m_stride, int heads, int dim, int vdim, float cap,
                          float eps, SP_SEQ_PARAMS, int dtype, void* stream);
-/* The same with gates whose rows lie gate_stride >= heads values apart (both halves of one product). */
+/* The same with gates whose rows lie gate_stride >= heads values apart (both halves of one product); and with the step's number of
+ * rows too, as sp_mamba2_scan_tokens. */
+SP_API int sp_mlstm_scan_tokens(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
+                                const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
+                                float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, int64_t num_tokens, int heads,
+                                int dim, int vdim, float cap, float eps, SP_SEQ_PARAMS, int dtype, void* stream);
 SP_API int sp_mlstm_scan_gates(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
                                const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
                                const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,

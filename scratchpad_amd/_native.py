@@ -142,11 +142,14 @@ SIGNATURES = {
     "sp_small_linear_f32": (_i32, [_vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _i32, _vp]),
     "sp_causal_conv_silu": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i32, _i32, *_SEQ, _i32, _vp]),
     "sp_mamba2_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, *_SEQ, _i32, _vp]),
+    "sp_mamba2_scan_tokens": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, *_SEQ, _i32, _vp]),
     "sp_gated_group_norm": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i32, _i32, _f32, _i32, _vp]),
     "sp_mlstm_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp,
                              _i64, _i32, _i32, _i32, _f32, _f32, *_SEQ, _i32, _vp]),
     "sp_mlstm_scan_gates": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i64,
                                    _vp, _i64, _i32, _i32, _i32, _f32, _f32, *_SEQ, _i32, _vp]),
+    "sp_mlstm_scan_tokens": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i64,
+                                    _vp, _i64, _i64, _i32, _i32, _i32, _f32, _f32, *_SEQ, _i32, _vp]),
     # ---- ABI 12
     "sp_gated_add_norm": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp,
                                  _i64, _i32, _f32, _i32, _vp]),
@@ -1599,9 +1602,10 @@ def mamba2_scan(xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, 
             state.shape[1:] != (heads, state_size, vdim) or dt_bias.numel() != heads or A_log.numel() != heads or D.numel() != heads:
         raise RuntimeError("mamba2_scan: shapes do not fit")
     y = torch.empty((xbc.shape[0], inner), dtype=torch.float32, device=xbc.device)
-    _check(load().sp_mamba2_scan(y.data_ptr(), y.stride(0), xbc.data_ptr(), xbc.stride(0), dt_raw.data_ptr(), dt_bias.data_ptr(),
-                                 A_log.data_ptr(), D.data_ptr(), state.data_ptr(), state.stride(0), heads, groups, state_size,
-                                 vdim, *seq.args, _dt(xbc), _stream()), "sp_mamba2_scan")
+    _check(load().sp_mamba2_scan_tokens(y.data_ptr(), y.stride(0), xbc.data_ptr(), xbc.stride(0), dt_raw.data_ptr(),
+                                        dt_bias.data_ptr(), A_log.data_ptr(), D.data_ptr(), state.data_ptr(), state.stride(0),
+                                        seq.num_tokens, heads, groups, state_size, vdim, *seq.args, _dt(xbc), _stream()),
+           "sp_mamba2_scan_tokens")
     return y
 
 
@@ -1637,11 +1641,11 @@ def mlstm_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tenso
             S.shape[1:] != (heads, dim, vdim) or n.shape[1:] != (heads, dim) or m.shape[1:] != (heads,):
         raise RuntimeError("mlstm_scan: gate or state shapes do not fit")
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
-    _check(load().sp_mlstm_scan_gates(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
+    _check(load().sp_mlstm_scan_tokens(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                                       v.data_ptr(), v.stride(0), g.data_ptr(), g.stride(0), ipre.data_ptr(), fpre.data_ptr(),
                                       ipre.stride(0) if T > 1 else heads, norm_w.data_ptr(), S.data_ptr(), S.stride(0), n.data_ptr(),
-                                      n.stride(0), m.data_ptr(), m.stride(0), heads, dim, vdim, cap, eps, *seq.args, _dt(q),
-                                      _stream()), "sp_mlstm_scan_gates")
+                                      n.stride(0), m.data_ptr(), m.stride(0), T, heads, dim, vdim, cap, eps, *seq.args, _dt(q),
+                                      _stream()), "sp_mlstm_scan_tokens")
     return out
 
 

@@ -342,17 +342,30 @@ static int launch_mlstm_chunks(void* out, int64_t out_stride, const void* q, int
   return SP_OK;
 }
 
+// Steps of short portions that the per-token form walks faster than a chunk of 64 mostly empty tokens costs: requests x heads of few
+// values that take the chunk form more than one round of workgroups, few tokens per request on average.  us, per token / in chunks, by
+// tokens per request (D x Dv, W = requests x heads):
+//   64 x 64     W 512: 1 18 / 15    W 640: 1 19 / 24, 6 24 / 25, 8 26 / 25    W 2048: 1 46 / 51, 2 49 / 51, 4 58 / 52
+//   128 x 64    W 256: 1 23 / 16    W 512: 1 27 / 30, 2 28 / 30, 4 30 / 30    W 640: 1 44 / 42
+//   64 x 128    W 320: 1 29 / 24    W 4096: 1 203 / 176      128 x 128   W 320: 1 46 / 31    W 4096: 1 487 / 239
+static bool short_portions(int64_t tokens, int64_t B, int H, int D, int Dv) {
+  const int64_t W = B * H;
+  if (tokens < 0 || Dv != 64) return false;
+  if (D == 64) return W > 512 && tokens <= (W <= 1024 ? 6 : 2) * B;
+  return W > 256 && W <= 512 && tokens <= 2 * B;
+}
+
 template <typename Tag>
 static int launch_mlstm(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
                         const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre,
                         int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride,
-                        float* m_state, int64_t m_stride, const SeqBatch& s, int H, int D, int Dv, float cap, float eps,
-                        hipStream_t st) {
+                        float* m_state, int64_t m_stride, const SeqBatch& s, int H, int D, int Dv, int64_t tokens, float cap,
+                        float eps, hipStream_t st) {
   // a step of one token per request stays with the per-token form (one sweep over the state is all there is to do), and so do
-  // the types and head sizes the matrix form is not built for
+  // the types and head sizes the matrix form is not built for, and short portions of many requests
   if (std::is_same<Tag, bf16_tag>::value && s.extend_seq_lens && (D == 64 || D == 128) && (Dv == 64 || Dv == 128) &&
       chunk_aligned(q, q_stride) && chunk_aligned(k, k_stride) && chunk_aligned(v, v_stride) &&
-      g_stride < ((int64_t)1 << 24) && out_stride < ((int64_t)1 << 24)) {
+      g_stride < ((int64_t)1 << 24) && out_stride < ((int64_t)1 << 24) && !short_portions(tokens, s.B, H, D, Dv)) {
 #define SP_MLSTM_CHUNKS(D_, NW_)                                                                                              \
   return launch_mlstm_chunks<D_, NW_>(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, gate_stride, norm_w, \
                                       S_state, S_stride, n_state, n_stride, m_state, m_stride, s, H, cap, eps, st)
@@ -385,12 +398,13 @@ static int launch_mlstm(void* out, int64_t out_stride, const void* q, int64_t q_
 
 using namespace sp;
 
-// (gate_stride: values between the gates of a token and the next one's, so that both may be halves of one product's rows)
-extern "C" int sp_mlstm_scan_gates(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
-                                   const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
-                                   const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
-                                   float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, int heads, int dim,
-                                   int vdim, float cap, float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
+// (gate_stride: values between the gates of a token and the next one's, so that both may be halves of one product's rows; num_tokens:
+// the step's rows, < 0 where the caller does not know; only the choice between the two forms depends on it)
+extern "C" int sp_mlstm_scan_tokens(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                    const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
+                                    const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
+                                    float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, int64_t num_tokens,
+                                    int heads, int dim, int vdim, float cap, float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
   SP_CHECK_ARG(batch_size >= 0 && heads > 0 && dim > 0 && vdim > 0 && vdim <= 256 && cap > 0.f);
   if (batch_size == 0) return SP_OK;
   SP_CHECK_ARG(out && q && k && v && g && ipre && fpre && norm_w && S_state && n_state && m_state && req_pool_indices && seq_lens);
@@ -401,7 +415,17 @@ extern "C" int sp_mlstm_scan_gates(void* out, int64_t out_stride, const void* q,
   SEQ_BATCH(s);
   SP_DISPATCH_DTYPE(dtype, return (launch_mlstm<Tag>(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre,
                                                      fpre, gate_stride, norm_w, S_state, S_stride, n_state, n_stride, m_state, m_stride, s,
-                                                     heads, dim, vdim, cap, eps, (hipStream_t)stream)));
+                                                     heads, dim, vdim, num_tokens, cap, eps, (hipStream_t)stream)));
+}
+
+extern "C" int sp_mlstm_scan_gates(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                   const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
+                                   const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
+                                   float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, int heads, int dim,
+                                   int vdim, float cap, float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
+  return sp_mlstm_scan_tokens(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, gate_stride, norm_w,
+                              S_state, S_stride, n_state, n_stride, m_state, m_stride, -1, heads, dim, vdim, cap, eps, req_pool_indices,
+                              seq_lens, extend_seq_lens, extend_prefix_lens, extend_start_loc, token_req, idx64, batch_size, dtype, stream);
 }
 
 extern "C" int sp_mlstm_scan(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,

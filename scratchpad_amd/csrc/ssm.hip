@@ -660,14 +660,28 @@ extern "C" int sp_causal_conv_silu(void* out, int64_t out_stride, const void* in
   return SP_OK;
 }
 
+// Steps of short portions that the per-token form walks faster than a chunk of 64 mostly empty tokens costs: requests x heads that take
+// the chunk form more than one round of workgroups (two per CU with Dv 64, one with 128), and few tokens per request on average.
+// us, per token / in chunks, by tokens per request (N x Dv, W = requests x heads):
+//   64 x 64     W 512: 1 14 / 12      W 640: 1 14 / 18, 8 18 / 19, 10 19 / 19     W 4096: 1 45 / 69, 10 66 / 71, 12 71 / 71
+//   64 x 128    W 256: 1 13 / 11      W 1024: 1 28 / 37, 8 39 / 41, 10 43 / 42    W 4096: 1 84 / 134, 12 137 / 142, 16 154 / 145
+//   128 x 64    W 512: 1 17 / 16      W 1024: 1 27 / 28, 4 30 / 28                W 4096: 1 91 / 97, 4 97 / 98    W 8192: 1 194 / 178
+//   128 x 128   W 256: 1 16 / 15      W 1024: 1 49 / 55, 4 54 / 55, 6 58 / 55     W 4096: 1 197 / 191
+static bool short_portions(int64_t tokens, int64_t B, int H, int N, int Dv) {
+  const int64_t W = B * H;
+  if (tokens < 0 || W <= (Dv == 64 ? 512 : 256)) return false;
+  if (N == 64) return tokens <= (Dv == 128 && W >= 1536 ? 12 : 10) * B;
+  return tokens <= 2 * B && W * Dv < (1 << 19);
+}
+
 template <typename Tag>
 static int launch_mamba2(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
                          const float* dt_bias, const float* A_log, const float* Dskip, float* state, int64_t state_stride,
-                         const SeqBatch& s, int H, int G, int N, int Dv, hipStream_t st) {
+                         const SeqBatch& s, int H, int G, int N, int Dv, int64_t tokens, hipStream_t st) {
   // a step of one token per request stays with the per-token form (one sweep over the state is all there is to do), and so do
-  // the types and head sizes the matrix form is not built for
+  // the types and head sizes the matrix form is not built for, and short portions of many requests
   if (std::is_same<Tag, bf16_tag>::value && s.extend_seq_lens && (N == 64 || N == 128) && (Dv == 64 || Dv == 128) &&
-      chunk_aligned(xbc, xbc_stride) && y_stride < ((int64_t)1 << 24)) {
+      chunk_aligned(xbc, xbc_stride) && y_stride < ((int64_t)1 << 24) && !short_portions(tokens, s.B, H, N, Dv)) {
 #define SP_CHUNKS(N_, NW_)                                                                                              \
   return launch_mamba2_chunks<N_, NW_>(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, state_stride, s, H, G, st)
     if (N == 128 && Dv == 128) SP_CHUNKS(128, 8);
@@ -691,10 +705,11 @@ static int launch_mamba2(float* y, int64_t y_stride, const void* xbc, int64_t xb
   return SP_OK;
 }
 
-extern "C" int sp_mamba2_scan(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
-                              const float* dt_bias, const float* A_log, const float* Dskip, float* state,
-                              int64_t state_stride, int heads, int groups, int state_size, int vdim, SP_SEQ_PARAMS,
-                              int dtype, void* stream) {
+// (num_tokens: the step's rows, < 0 where the caller does not know; only the choice between the two forms depends on it)
+extern "C" int sp_mamba2_scan_tokens(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
+                                     const float* dt_bias, const float* A_log, const float* Dskip, float* state,
+                                     int64_t state_stride, int64_t num_tokens, int heads, int groups, int state_size, int vdim,
+                                     SP_SEQ_PARAMS, int dtype, void* stream) {
   SP_CHECK_ARG(batch_size >= 0 && heads > 0 && groups > 0 && heads % groups == 0 && state_size > 0 && vdim > 0 && vdim <= 256);
   if (batch_size == 0) return SP_OK;
   SP_CHECK_ARG(y && xbc && dt_raw && dt_bias && A_log && Dskip && state && req_pool_indices && seq_lens);
@@ -704,7 +719,17 @@ extern "C" int sp_mamba2_scan(float* y, int64_t y_stride, const void* xbc, int64
   SP_CHECK_ARG(state_stride >= (int64_t)heads * state_size * vdim);
   SEQ_BATCH(s);
   SP_DISPATCH_DTYPE(dtype, return (launch_mamba2<Tag>(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state,
-                                                      state_stride, s, heads, groups, state_size, vdim, (hipStream_t)stream)));
+                                                      state_stride, s, heads, groups, state_size, vdim, num_tokens,
+                                                      (hipStream_t)stream)));
+}
+
+extern "C" int sp_mamba2_scan(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
+                              const float* dt_bias, const float* A_log, const float* Dskip, float* state,
+                              int64_t state_stride, int heads, int groups, int state_size, int vdim, SP_SEQ_PARAMS,
+                              int dtype, void* stream) {
+  return sp_mamba2_scan_tokens(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, state_stride, -1, heads, groups,
+                               state_size, vdim, req_pool_indices, seq_lens, extend_seq_lens, extend_prefix_lens, extend_start_loc,
+                               token_req, idx64, batch_size, dtype, stream);
 }
 
 extern "C" int sp_gated_group_norm(void* out, int64_t out_stride, const float* y, int64_t y_stride, const void* z,

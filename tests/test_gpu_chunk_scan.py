@@ -263,6 +263,57 @@ def test_mamba2_chunks_of_strong_decays(kind):
             near(S[slot, h], ref[h], 4e-6)
 
 
+@pytest.mark.parametrize("length", [1, 10, 11])
+def test_mamba2_short_portions_of_many_requests(length):
+    """on both sides of the line between the forms, and with the number of rows not given: the same numbers within fp32's sums"""
+    from scratchpad_amd import _native
+    announce("mamba2 short portions", length)
+    g = torch.Generator(device=DEV).manual_seed(19)
+    B, H, G, N, Dv = 64, 32, 1, 64, 64
+    T, slots = B * length, list(range(1, B + 1))
+    xbc, raw = torch.randn(T, H * Dv + 2 * G * N, generator=g, device=DEV).bfloat16(), torch.randn(T, H, generator=g, device=DEV)
+    A, bias, skip = (torch.randn(H, generator=g, device=DEV) * 0.5 - 1 for _ in range(3))
+    seq = seq_extend([length] * B, [0] * B, slots)
+    want, states = mamba2_in_64_bits(xbc, raw, bias, A, skip, [length] * B, H, G, N, Dv)
+    S = torch.zeros(2, B + 1, H, N, Dv, device=DEV)
+    y = [_native.mamba2_scan(xbc, raw, bias, A, skip, S[0], seq, H, G, N, Dv), torch.empty(T, H * Dv, device=DEV)]
+    _native._check(_native.load().sp_mamba2_scan(y[1].data_ptr(), H * Dv, xbc.data_ptr(), xbc.stride(0), raw.data_ptr(), bias.data_ptr(),
+                                                 A.data_ptr(), skip.data_ptr(), S[1].data_ptr(), S[1].stride(0), H, G, N, Dv, *seq.args,
+                                                 _native._dt(xbc), _native._stream()), "sp_mamba2_scan")
+    for i in (0, 1):
+        near(y[i].view(T, H, Dv), want, 2e-6)
+        near(S[i][1:], torch.stack(states), 2e-6)
+
+
+@pytest.mark.parametrize("length", [1, 6, 7])
+def test_mlstm_short_portions_of_many_requests(length):
+    """the same numbers within fp32's sums on both sides of the line between the forms (6 tokens), with the number of rows given and not"""
+    from scratchpad_amd import _native
+    announce("mlstm short portions", length)
+    g = torch.Generator(device=DEV).manual_seed(20)
+    B, H, D = 64, 16, 64
+    T, slots = B * length, list(range(1, B + 1))
+    q, k, v, gate = (torch.randn(T, H * D, generator=g, device=DEV).bfloat16() for _ in range(4))
+    ip, fp, nw = torch.randn(T, H, generator=g, device=DEV), torch.randn(T, H, generator=g, device=DEV) + 1, torch.ones(H * D, device=DEV)
+    seq, got = seq_extend([length] * B, [0] * B, slots), []
+    for known in (True, False):
+        S, n, m = torch.zeros(B + 1, H, D, D, device=DEV), torch.zeros(B + 1, H, D, device=DEV), torch.zeros(B + 1, H, device=DEV)
+        if known:
+            y = _native.mlstm_scan(q, k, v, gate, ip, fp, nw, S, n, m, seq, H, D, D, 15.0, 1e-5)
+        else:
+            y = torch.empty(T, H * D, dtype=torch.bfloat16, device=DEV)
+            _native._check(_native.load().sp_mlstm_scan(
+                y.data_ptr(), H * D, q.data_ptr(), H * D, k.data_ptr(), H * D, v.data_ptr(), H * D, gate.data_ptr(), H * D, ip.data_ptr(),
+                fp.data_ptr(), nw.data_ptr(), S.data_ptr(), S.stride(0), n.data_ptr(), n.stride(0), m.data_ptr(), m.stride(0), H, D, D,
+                15.0, 1e-5, *seq.args, _native._dt(q), _native._stream()), "sp_mlstm_scan")
+        got.append((y, S, n, m))
+    (y0, *a), (y1, *b) = got
+    for x, w in zip(a, b):
+        near(x, w.double(), 2e-6)
+    # two roundings of a result of 8 bits; a normaliser that nearly cancels scales fp32's sums up
+    assert ((y0.double() - y1.double()).abs() <= 2.0 ** -7 * y1.double().abs() + 2e-3).all()
+
+
 def test_mlstm_chunks_of_closed_forget_gates():
     """A chunk whose first 16 tokens forget nothing and whose others forget all but e^-15 each: the summed log gates reach -700, and a
     weight taken from sums rounded to fp32 would be off by 3e-5.  Half of the values cancel in pairs (k is the same everywhere, v

@@ -257,7 +257,7 @@ def test_mlstm_scan_takes_no_gate_rows_that_overlap(monkeypatch):
         is_cuda = True
 
     calls = []
-    lib = types.SimpleNamespace(sp_mlstm_scan_gates=lambda *a: calls.append(a) or 0)
+    lib = types.SimpleNamespace(sp_mlstm_scan_tokens=lambda *a: calls.append(a) or 0)
     monkeypatch.setattr(_native, "load", lambda: lib)
     monkeypatch.setattr(_native, "_stream", lambda: 0)
     T, H, D = 6, 4, 16
