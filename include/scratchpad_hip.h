@@ -711,7 +711,8 @@ SP_API int sp_gated_delta_scan(void* out, int64_t out_stride, const void* q, int
                                int64_t state_stride, int heads, int kv_heads, int dim, int vdim, float eps, SP_SEQ_PARAMS,
                                int dtype, void* stream);
 /* The same for steps of several tokens per request, 16 tokens at a time on the matrix cores (fp32 throughout): dim 64 or 128, vdim
- * a multiple of 16, q and k rows 16-byte aligned, decays in [0, 1]; else SP_ERR_UNSUPPORTED and nothing is launched.  work: fp32,
+ * a multiple of 16, q and k rows 16-byte aligned; else SP_ERR_UNSUPPORTED and nothing is launched.  Products of up to 16 decays are
+ * formed (never quotients): those in [0, 1], as the gates give them, cannot overflow.  work: fp32,
  * sp_delta_chunk_floats(num_tokens, batch_size, heads) values, 16-byte aligned; raw: fp32 [num_tokens, heads * vdim].            */
 SP_API int64_t sp_delta_chunk_floats(int64_t num_tokens, int batch_size, int heads);
 SP_API int sp_gated_delta_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,

@@ -12,8 +12,9 @@
 // lanes; the request's tokens of this step are walked in order from the state the previous step left in the pool (zeros
 // at a sequence's first token), staged through LDS in passes.  A token costs ONE sweep over the column: the update, the
 // numerator and - on the state just completed - the next token's u^T S, then two independent sums over the column's lanes
-// (register moves); no workgroup barrier.  Prompt portions and single decoded
-// tokens take the same path, and the order of every sum depends on the head only.
+// (register moves); no workgroup barrier.  The order of its sums depends on the head only.  Prompts take it; a decode step (one token
+// per request, heads of 64 or 128, rank up to 512) takes delta_step_kernel, which forms the gates too and adds a head's sums in
+// another order.
 #include "seq_batch.h"
 
 namespace sp {

@@ -12,8 +12,11 @@
 // lanes; the request's tokens of this step are walked in order from the state the previous step left in the pool (zeros at
 // a sequence's first token), staged through LDS in passes.  A token costs ONE sweep over the column: the update, the
 // read-out and - on the state just completed - the next token's (w * kn)^T S, then two independent sums over the column's
-// lanes (register moves); no workgroup barrier inside a pass.  Prompt portions and single decoded tokens take the same
-// path, and the order of every sum depends on the head's sizes only.
+// lanes (register moves); no workgroup barrier inside a pass.  The order of its sums depends on the head's sizes only.
+//
+// Decode steps and short portions take that path, steps of 8 and more tokens per request on average (of the sizes that chunk_delta.h
+// takes) the 16-token chunks of sp_gated_delta_chunks, whose sums associate by a token's place in its portion: a request's
+// roundings depend on how its prompt was cut and, through the mean, on the lengths of the others in the step.
 #include "chunk_delta.h"
 #include "chunk_scan.h"
 

@@ -18,8 +18,9 @@
 // Each form sums the partial results of its lanes and waves in a fixed order that M, K and the
 // number of weight rows alone decide.
 // us, cold weights under graph replay, N x K: 1 row / 4 rows / 8 rows; before (the third form for every M, the waves' k-steps
-// interleaved) -> now.  The line between the second and the third form is where their times cross (8 rows: 20.1 and 17.3 at
-// 16384 x 2048, 12.8 and 14.6 at 2048 x 8192), between the first and the second it is the one row itself.
+// interleaved) -> now.  The second form ends at the 4 rows that its instruction holds: a second group of x rows for 5 to 8 was
+// slower where there are many weight rows (8 rows: 20.1 against the third form's 17.3 at 16384 x 2048) and faster with few long ones (12.8
+// against 14.6 at 2048 x 8192), which is left on the table.  Below 5 rows few_and_short has the line to the third form.
 //   3072 x 2048     5.3 -> 4.6      5.7 -> 5.8      6.1 -> 6.1
 //   2048 x 2048     5.0 -> 3.8      5.3 -> 4.9      5.7 -> 5.8
 //   16384 x 2048   14.5 -> 12.3    15.9 -> 14.8    18.2 -> 17.3

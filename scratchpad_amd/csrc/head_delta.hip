@@ -13,8 +13,12 @@
 // update, the read-out and, on the state just completed, the next token's S^T kn (its decay is a factor of the whole sum),
 // then sums over the SP lanes by register moves; no workgroup barrier inside a pass of kChunk tokens.
 // With one range per head the norm and the gate are the pass's epilogue; where a step brings long portions of few requests,
-// several workgroups share a head and hand fp32 read-outs to head_norm_gate_kernel.  Prompt portions and single decoded
-// tokens take the same path, and the order of every sum depends on the head's sizes only.
+// several workgroups share a head and hand fp32 read-outs to head_norm_gate_kernel.  The order of its sums depends on the head's
+// sizes only.
+//
+// Decode steps and short portions take that path, steps of 18 and more tokens per request on average (of the sizes that chunk_delta.h
+// takes) the 16-token chunks of sp_head_delta_chunks, whose sums associate by a token's place in its portion: a request's
+// roundings depend on how its prompt was cut and, through the mean, on the lengths of the others in the step.
 #include "chunk_delta.h"
 
 namespace sp {

@@ -260,8 +260,9 @@ moe_grouped_gemm_kernel(void* out, const void* a, const void* w, const int32_t* 
 // ---- the same product on the matrix cores (16-bit types, K a multiple of 32, 16-byte aligned rows) -------------------
 // v_mfma_f32_16x16x32: lane (r16 = lane & 15, q = lane >> 4) holds 8 k-values of row r16 of each operand and receives
 // D[4 q + r][r16], r < 4 - with the weights as the first operand a lane ends up with 4 neighbouring output columns of ONE
-// row.  Both kernels below add the k-steps of 32 in ascending order into one accumulator, so an output element has the same
-// bits whichever of them - and whichever tile height - computes it: a token's result does not depend on the step's size.
+// row.  The three kernels below (tile, wide, rows) add the k-steps of 32 in ascending order into one accumulator, so an output
+// element has the same bits whichever of them - and whichever tile height - computes it: a token's result does not depend on the
+// step's size.
 //
 // ACT: 0 the product, 1 max(., 0)^2 of the fp32 sum; 2 and 3 take w [E, 2 N, K] (gate rows, then up rows), keep the two sums
 // of an output column in one lane and store the activation of the ROUNDED sums - bit for bit the plain product followed by
@@ -668,8 +669,11 @@ __global__ void __launch_bounds__(64) moe_grouped_rows_kernel(GroupedArgs p) {
 // 32 experts of ff 1024, top 4, up + down product in us (rows kernel | 64-row tiles | 128-row tiles):
 //   mean rows 1: 60 | 68 | 73     4: 85 | 92 | 94     8: 86 | 92 | 94     16: 104 | 93 | 96     32: 161 | 95 | 99
 //   64: 286 | 103 | 103     96: 410 | 138 | 107     128: 537 | 150 | 157     512: 2038 | 379 | 337
-// and from 320 rows on the 128 x 256 tiles (their comment has both sides)
-// (the kernel these replaced, one operand fragment per load and no LDS: 75 at mean 1, 1398 at mean 512)
+// and from 320 rows on the 128 x 256 tiles (their comment has both sides).  (The kernel these replaced, one operand fragment per load
+// and no LDS: 75 at mean 1, 1398 at mean 512.)  The mean says nothing of a skewed step: with every pair on 4 of 128 experts, mean 10, the
+// rows kernel reads an expert's weights 20 times (491 us at width 4096, ff 1536, where the 64-row tiles take 95 at mean 11 and the replaced
+// kernel took 683).  Widths 1024 to 4096, 8 to 128 experts, routing even, by 1 / rank and to 4 experts, means 1 to 321: 1.1 to 9.4 times
+// as fast as the replaced kernel throughout.
 template <typename Tag, int ACT>
 int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
   const int held = pairs < p.E ? pairs : p.E;                    // experts with a row, at most

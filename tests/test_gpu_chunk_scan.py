@@ -149,6 +149,32 @@ def test_gated_delta_chunks(lens, H, G, D, Dv, dtype):
         assert torch.isnan(S[slot]).all()
 
 
+def test_gated_delta_chunks_of_any_decays():
+    """products of up to 16 decays are formed and never quotients: zeros, negative ones and ones above 1 are numbers like others"""
+    from scratchpad_amd import _native
+    announce("gated delta chunks of any decays")
+    g = torch.Generator(device=DEV).manual_seed(7)
+    lens, slots, H, D, Dv = [48, 33], [1, 3], 2, 64, 64
+    T, seq = sum(lens), seq_extend([48, 33], [0, 0], [1, 3])
+    q, k, v, bp = (torch.randn(T, n, generator=g, device=DEV) for n in (H * D, H * D, H * Dv, H))
+    decay = torch.rand(T, H * D, generator=g, device=DEV) * 2.1 - 1.05
+    decay[::5] = 0.0
+    S, gate, nw = torch.zeros(4, H, D, Dv, device=DEV), torch.ones(T, H * Dv, device=DEV), torch.ones(Dv, device=DEV)
+    assert _native._delta_chunks_take(q, k, v, decay, seq, D, Dv)
+    _native.gated_delta_scan(q, k, v, bp, decay, gate, nw, S, seq, H, H, D, Dv, 1e-5)
+    kk = k.double().view(T, H, D)
+    kk, beta, w = kk / torch.sqrt((kk * kk).sum(-1, keepdim=True) + 1e-6), torch.sigmoid(bp.double()), decay.double().view(T, H, D)
+    at = 0
+    for length, slot in zip(lens, slots):
+        Sr = torch.zeros(H, D, Dv, dtype=torch.float64, device=DEV)
+        for t in range(at, at + length):
+            Sr = w[t][:, :, None] * Sr
+            u = beta[t][:, None] * (v[t].double().view(H, Dv) - (Sr * kk[t][:, :, None]).sum(1))
+            Sr = Sr + kk[t][:, :, None] * u[:, None]
+        at += length
+        near(S[slot], Sr, 2e-5)
+
+
 @pytest.mark.parametrize("T", [64, 129, 700])
 @pytest.mark.parametrize("rank,channels", [(32, 16), (64, 208), (96, 64), (128, 2048)])
 def test_lowrank_gate_of_many_tokens(T, rank, channels):
@@ -380,13 +406,11 @@ def test_mamba2_values_that_are_not_finite_reach_no_earlier_token(bad, at):
     assert torch.equal(S1[~hit], S0[~hit]) and not torch.isfinite(S1[hit]).any()
 
 
-@pytest.mark.parametrize("bad", BAD, ids=str)
-@pytest.mark.parametrize("where", ["q", "k", "v", "ipre", "fpre"])
+# (an infinite gate is capped)
+@pytest.mark.parametrize("where,bad", [(w, b) for w in "qkv" for b in BAD] + [("ipre", BAD[0]), ("fpre", BAD[0])])
 @pytest.mark.parametrize("at", [0, 40, 63, 70])
 def test_mlstm_values_that_are_not_finite_reach_no_earlier_token(at, where, bad):
     from scratchpad_amd import _native
-    if where in ("ipre", "fpre") and bad == bad:
-        pytest.skip("an infinite gate is capped")
     announce("mlstm not finite", where, bad, at)
     g = torch.Generator(device=DEV).manual_seed(17)
     lens, H, D = [100, 20], 2, 64
@@ -411,14 +435,12 @@ def test_mlstm_values_that_are_not_finite_reach_no_earlier_token(at, where, bad)
         assert torch.equal(S1[1, 1][:, ~hit], S0[1, 1][:, ~hit])
 
 
-@pytest.mark.parametrize("bad", BAD, ids=str)
-@pytest.mark.parametrize("where", ["q", "k", "v", "beta", "decay"])
+# (an infinite step size or decay is a number)
+@pytest.mark.parametrize("where,bad", [(w, b) for w in "qkv" for b in BAD] + [("beta", BAD[0]), ("decay", BAD[0])])
 @pytest.mark.parametrize("at", [0, 9, 15, 16, 40])
 @pytest.mark.parametrize("channel", [True, False], ids=["gated", "head"])
 def test_delta_values_that_are_not_finite_reach_no_earlier_token(channel, at, where, bad):
     from scratchpad_amd import _native
-    if bad == bad and where in ("beta", "decay"):
-        pytest.skip("an infinite step size or decay is a number")
     announce("delta not finite", channel, where, bad, at)
     g = torch.Generator(device=DEV).manual_seed(18)
     lens, H, D, Dv = [61, 30], 2, 64, 64
