@@ -13,20 +13,19 @@
 //               so a load covers 256 B of 4 rows and its two halves are two products; the 16 blocks are 16 partial sums over K.
 //               4 waves share K, 4 or 8 weight rows (columns of out) a workgroup
 //   to 16 rows  v_mfma_f32_16x16x32: 64 B of 16 weight rows a load, x read in the same form (as many bytes out of L2 as weights:
-//               what bounds it from 8 rows on).  A wave's loads in flight lie next to each other in K, so that both halves of a
-//               128-byte line are asked for by one wave
+//               what bounds it from 8 rows on), 8 waves share K
 // Each form sums the partial results of its lanes and waves in a fixed order that M, K and the
 // number of weight rows alone decide.
 // us, cold weights under graph replay, N x K: 1 row / 4 rows / 8 rows; before (the third form for every M, the waves' k-steps
 // interleaved) -> now.  The second form ends at the 4 rows that its instruction holds: a second group of x rows for 5 to 8 was
 // slower where there are many weight rows (8 rows: 20.1 against the third form's 17.3 at 16384 x 2048) and faster with few long ones (12.8
-// against 14.6 at 2048 x 8192), which is left on the table.  Below 5 rows few_and_short has the line to the third form.
-//   3072 x 2048     5.3 -> 4.6      5.7 -> 5.8      6.1 -> 6.1
-//   2048 x 2048     5.0 -> 3.8      5.3 -> 4.9      5.7 -> 5.8
-//   16384 x 2048   14.5 -> 12.3    15.9 -> 14.8    18.2 -> 17.3
-//   2048 x 8192    13.3 -> 8.2     14.7 -> 10.4    16.2 -> 14.6
-//   6144 x 4096    13.2 -> 9.9     14.4 -> 12.6    16.1 -> 15.6
-//   28672 x 4096   43.7 -> 40.7    47.4 -> 43.0    54.4 -> 50.4
+// against 14.6 at 2048 x 8192), which is left on the table.  Below 5 rows few_take_tiles has the line to the third form.
+//   3072 x 2048     5.3 -> 4.6      5.9 -> 5.8      6.3 -> 6.1
+//   2048 x 2048     5.0 -> 3.8      5.5 -> 5.3      5.7 -> 5.8
+//   16384 x 2048   14.5 -> 12.3    15.9 -> 15.8    18.3 -> 18.2
+//   2048 x 8192    13.3 -> 8.2     14.9 -> 12.0    16.4 -> 15.3
+//   6144 x 4096    13.2 -> 9.9     15.4 -> 13.2    16.9 -> 16.4
+//   28672 x 4096   43.7 -> 40.7    46.4 -> 42.9    52.7 -> 50.6
 //   128256 x 2048  89.0 -> 83.1    98.5 -> 90.1   118.0 -> 113.2
 // Tried and slower: x staged in LDS and a persistent loop over weight rows in any of 10 shapes (8 to 40 % slower: the copy and its
 // barrier come before the first product, and the loop's tail is longer than a launch of many small workgroups), 16 products in
@@ -222,13 +221,21 @@ __global__ __launch_bounds__(kQuadWaves * 64) void gemm_quad_kernel(SkinnyArgs a
 }
 
 // ---- 5-16 rows
-constexpr int kSkWaves = 8, kSkUnroll = 4;
+constexpr int kSkWaves = 8;
+
+// The waves' k-steps: NEAR, a wave's loads in flight lie next to each other in K (4 of them: both halves of a 128-byte line are asked for
+// by one wave), from K 2560 on; else they lie 8 steps apart and the workgroup's next to each other (8 of them), so that the waves
+// share lines of x in the L1.  us at 5 / 16 rows, apart | NEAR: 4096 x 2048 6.2 / 7.5 | 7.0 / 7.9; 4608 x 1536 7.0 / 8.5 | 7.4 / 9.4;
+// 1024 x 2560 5.8 / 7.0 | 5.5 / 6.9; 2048 x 3072 7.6 / 9.2 | 7.1 / 9.1; 16384 x 4096 29.2 / 39.6 | 28.7 / 38.7; 2048 x 8192 14.8 / 19.5 | 14.1 / 18.0.
+// (NEAR with 8 in flight, and pairs of neighbours 8 pairs apart, are slower than one of the two everywhere.)
+constexpr int kSkNearK = 2560;
 
 // EPI 1 and 3: a.N = I output columns; the 16 W rows of a workgroup are gate rows n0 .. n0+7 (tile rows 0-7) and up rows
 // I + n0 .. I + n0 + 7 (tile rows 8-15)
-template <typename Tag, int EPI>
+template <typename Tag, bool NEAR, int EPI>
 __global__ __launch_bounds__(kSkWaves * 64) void gemm_skinny_kernel(SkinnyArgs a) {
   typedef Elem<Tag> E;
+  constexpr int U = NEAR ? 4 : 8, STEP = NEAR ? 1 : kSkWaves;
   constexpr bool GLU = EPI == 1 || EPI == 3;
   __shared__ float red[kSkWaves][16 * 17];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -242,19 +249,19 @@ __global__ __launch_bounds__(kSkWaves * 64) void gemm_skinny_kernel(SkinnyArgs a
   const int ksteps = a.K / 32;
   f32x4_g acc = {0.f, 0.f, 0.f, 0.f};
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  // this wave's k-steps: kSkUnroll in a row, then kSkUnroll more kSkWaves * kSkUnroll steps on, all loads of a group first
-  for (int ks = wave * kSkUnroll; ks < ksteps; ks += kSkUnroll * kSkWaves) {
-    u32x4 wf[kSkUnroll], xf[kSkUnroll];
+  // this wave's k-steps, U at a time, all loads of a group first
+  for (int ks = wave * (NEAR ? U : 1); ks < ksteps; ks += U * kSkWaves) {
+    u32x4 wf[U], xf[U];
 #pragma unroll
-    for (int u = 0; u < kSkUnroll; ++u) {
-      const int64_t off = (int64_t)(ks + u) * 64;
-      const bool in = ks + u < ksteps;
+    for (int u = 0; u < U; ++u) {
+      const int64_t off = (int64_t)(ks + u * STEP) * 64;
+      const bool in = ks + u * STEP < ksteps;
       wf[u] = in ? ld16(wp + off) : zero;
       xf[u] = in && mrow ? ld16(xp + off) : zero;
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < kSkUnroll; ++u) acc = mfma_g<Tag>(wf[u], xf[u], acc);
+    for (int u = 0; u < U; ++u) acc = mfma_g<Tag>(wf[u], xf[u], acc);
   }
   // acc[r] = partial of out[m = r16][n0 + 4q + r]; sum the waves in wave order
 #pragma unroll
@@ -284,17 +291,21 @@ __global__ __launch_bounds__(kSkWaves * 64) void gemm_skinny_kernel(SkinnyArgs a
 // One group of 4 weight rows up to 2048 rows: 256 workgroups of two groups there (3 rows, K 4096, us: 1024 rows 4.6 one / 6.3 two,
 // 2048 rows 6.3 / 6.9, 2560 rows 7.8 / 8.9, 8192 rows 16.0 / 14.6).
 constexpr int kQuadOneGroup = 2048;
-// 2-4 rows go to the tiles of 16 weight rows where there are more than the one-group form's rows and K is too short for the
-// others' head start (us, 4 rows, tiles / two groups: K 1024, 3072 rows 3.9 / 4.8, 8192 rows 5.8 / 6.5; K 2048, 3072 rows
-// 5.8 / 6.4, 4096 rows 6.3 / 6.4, 6144 rows 9.0 / 7.9; K 4096, 3072 rows 8.7 / 9.6, 5120 rows 14.6 / 12.3).
-static bool few_and_short(int64_t rows, int K) { return rows > kQuadOneGroup && (K <= 1024 || (K <= 2048 && rows <= 4096)); }
+// Where 2-4 rows go to the tiles of 16 weight rows (us at 4 rows, groups of 4 / tiles): a short K, and more rows than one group takes while
+// they are too few for two groups to fill the card (512 x 512 2.8 / 2.7; K 1536: 2560 4.9 / 4.9, 4096 5.6 / 5.2, 8192 8.2 / 7.2, 28672 19.2 /
+// 19.5; K 2048: 3072 6.3 / 5.8, 4096 7.0 / 6.2, 4608 8.1 / 8.5, 16384 15.7 / 15.9; K 4096: 2048 7.4 / 8.3, 2560 9.7 / 8.8, 4096 10.3 / 10.1,
+// 4608 12.7 / 14.7; K 8192: 3072 16.1 / 15.2; 2 rows there 14.2 / 14.6).
+static bool few_take_tiles(int M, int64_t rows, int K) {
+  if (K <= 512) return true;
+  return rows > kQuadOneGroup && (K <= 1536 || (rows <= 4096 && (M > 2 || K <= 4096)));
+}
 
 template <typename Tag, int EPI>
 static void launch_skinny_as(const SkinnyArgs& a, hipStream_t st) {
   constexpr bool GLU = EPI == 1 || EPI == 3;
   if (a.M == 1) {
     gemm_row_kernel<Tag, EPI><<<dim3((a.N + kRowWaves - 1) / kRowWaves), dim3(kRowWaves * 64), 0, st>>>(a);
-  } else if (a.M <= kQuadRows && !few_and_short(GLU ? 2 * (int64_t)a.N : a.N, a.K)) {
+  } else if (a.M <= kQuadRows && !few_take_tiles(a.M, GLU ? 2 * (int64_t)a.N : a.N, a.K)) {
     if (!GLU && a.N <= kQuadOneGroup) {
       if constexpr (!GLU) gemm_quad_kernel<Tag, 1, EPI><<<dim3((a.N + 3) / 4), dim3(kQuadWaves * 64), 0, st>>>(a);
     } else {
@@ -303,7 +314,9 @@ static void launch_skinny_as(const SkinnyArgs& a, hipStream_t st) {
     }
   } else {
     constexpr int cols = GLU ? 8 : 16;
-    gemm_skinny_kernel<Tag, EPI><<<dim3((a.N + cols - 1) / cols), dim3(kSkWaves * 64), 0, st>>>(a);
+    const dim3 grid((a.N + cols - 1) / cols), block(kSkWaves * 64);
+    if (a.K >= kSkNearK) gemm_skinny_kernel<Tag, true, EPI><<<grid, block, 0, st>>>(a);
+    else gemm_skinny_kernel<Tag, false, EPI><<<grid, block, 0, st>>>(a);
   }
 }
 

@@ -40,6 +40,12 @@ def test_rows_columns_and_lengths(dtype, eps, M, N, K):
     assert bool((err <= eps * (ref.clamp(min=0) + slack).square() + 2 * (ref.abs() + slack) * slack + 2.0 ** -25).all())
 
 
+@pytest.mark.parametrize("M", [2, 3, 6])
+@pytest.mark.parametrize("N,K", [(130, 512), (130, 544), (2304, 1536), (2304, 4064), (2304, 4096), (2304, 4128), (4104, 1536), (4104, 1568)])
+def test_both_sides_of_the_lines_between_the_forms(M, N, K):
+    test_rows_columns_and_lengths(torch.bfloat16, 2.0 ** -8, M, N, K)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 2, 4, 5, 16])
 @pytest.mark.parametrize("I,K", [(1, 32), (6, 96), (13, 2080), (1024, 544), (1030, 1024), (2049, 2048)])
