@@ -96,15 +96,18 @@ lowrank_gate_kernel(float* out, const void* p, int64_t p_stride, const float* w2
 }
 
 // The same for steps of many tokens, bf16 rows and ranks that are multiples of 32, up to 128: the product on the matrix cores.  A
-// wave keeps 16 channels of w2t as three bf16 parts each (an exact split, chunk_scan.h) and walks kGateTokens tokens, 16 at a time:
+// wave keeps 16 channels of w2t as three bf16 parts each (an exact split, chunk_scan.h) and walks `run` tokens, 16 at a time:
 // p's rows are the other operand as they lie, a lane ends with 4 neighbouring channels of a token.  One channel per thread was bound
 // by its LDS reads (one per 4 multiply-adds): 51 us for 4096 tokens x 2048 channels of rank 64, 22 here (16 for a sigmoid).
-constexpr int kGateTokens = 128;
+// Where that leaves the chip idle a wave walks fewer: 128 tokens each were a chain of 8 products, exponentials and stores whatever the
+// step's size, longer than the form above in small ones (decays, rank 64: 128 tokens x 2048 channels 7.7 above, 10.3 with 128, 4.2 now; 512 x
+// 1024 8.0, 10.4, 4.8).
+constexpr int kGateTokens = 128, kGateGroups = 512;      // tokens per wave at the most; workgroups that fill the chip
 
 template <int RANK, int ACT>
 __global__ void __launch_bounds__(kBlock)
 lowrank_gate_mfma_kernel(float* out, const char* p, int64_t p_stride, const float* w2t, const float* bias, const float* A_log,
-                         int64_t T, int channels, int per_head) {
+                         int64_t T, int channels, int per_head, int run) {
   const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   const int c0 = (blockIdx.y * (kBlock / 64) + (threadIdx.x >> 6)) * 16;
   if (c0 >= channels) return;                          // (channels is a multiple of 16)
@@ -127,8 +130,8 @@ lowrank_gate_mfma_kernel(float* out, const char* p, int64_t p_stride, const floa
     b[r] = bias ? bias[c0 + 4 * q + r] : 0.f;
     rate[r] = ACT == 0 ? expf(A_log[(c0 + 4 * q + r) / per_head]) : 0.f;
   }
-  const int64_t t1 = (int64_t)(blockIdx.x + 1) * kGateTokens < T ? (int64_t)(blockIdx.x + 1) * kGateTokens : T;
-  for (int64_t t0 = (int64_t)blockIdx.x * kGateTokens; t0 < t1; t0 += 16) {
+  const int64_t t1 = (int64_t)(blockIdx.x + 1) * run < T ? (int64_t)(blockIdx.x + 1) * run : T;
+  for (int64_t t0 = (int64_t)blockIdx.x * run; t0 < t1; t0 += 16) {
     const int64_t t = t0 + r16 < t1 ? t0 + r16 : t1 - 1;
     f32x4_c z = {b[0], b[1], b[2], b[3]};
 #pragma unroll
@@ -360,10 +363,13 @@ extern "C" int sp_lowrank_gate(float* out, const void* p, int64_t p_stride, cons
   if (per_head <= 0) per_head = 1;
   if (dtype == SP_BF16 && num_tokens >= 64 && (rank == 32 || rank == 64 || rank == 96 || rank == 128) && channels % 16 == 0 &&
       p_stride % 8 == 0 && (((uintptr_t)p | (uintptr_t)out) & 15) == 0) {
-    const dim3 grid((unsigned)((num_tokens + kGateTokens - 1) / kGateTokens), (unsigned)((channels + kBlock / 4 - 1) / (kBlock / 4)));
+    const int64_t groups = (channels + kBlock / 4 - 1) / (kBlock / 4);
+    int run = kGateTokens;
+    while (run > 16 && (num_tokens + run - 1) / run * groups < kGateGroups) run /= 2;
+    const dim3 grid((unsigned)((num_tokens + run - 1) / run), (unsigned)groups);
 #define SP_LM(R, ACT)                                                                                                    \
   lowrank_gate_mfma_kernel<R, ACT><<<grid, kBlock, 0, (hipStream_t)stream>>>(out, (const char*)p, p_stride, w2t, bias, A_log, \
-                                                                              num_tokens, channels, per_head)
+                                                                              num_tokens, channels, per_head, run)
 #define SP_LM2(R)              \
   do {                         \
     if (act == 0) SP_LM(R, 0); \
