@@ -1825,12 +1825,42 @@ def lowrank_gate(p: torch.Tensor, w2t: torch.Tensor, bias: Optional[torch.Tensor
     return out
 
 
-# mean tokens per request from which a delta rule's step runs 16 tokens at a time
+# the least mean tokens per request at which a delta rule's step runs 16 tokens at a time, whatever its sizes (delta_chunk_tokens), and
+# with one decay per head, whose per-token kernel shares a head's columns out to more workgroups
 DELTA_CHUNK_MIN_TOKENS = 8
-# ... and with one decay per head, whose per-token kernel shares a head's columns out to more workgroups (16 heads of 128 x 128,
-# per-token against chunks, us): 8 requests of 4096 tokens together 364 / 179, one of 4096 2101 / 672, 16 of 300 41 / 33, one of
-# 65 tokens 42 / 27; 16 of 130 20 / 24, 4 of 64 20 / 26.
 HEAD_DELTA_CHUNK_MIN_TOKENS = 18
+
+
+def delta_chunk_tokens(channel: bool, W: int, dim: int, vdim: int) -> int:
+    """Mean tokens per request from which the 16-token chunks are the faster form (channel: a decay per key channel), by W = requests x
+    heads and the head's sizes.  What a chunk costs beside the columns - operand rows, the prepared matrices, 16 tokens even where 1 is
+    left - is shared by a workgroup's columns: 128, or 64 where there are no more or W is small.  us, per token / in chunks, by mean tokens:
+      channel  64 x 64    W 64: 24 16 / 18, 28 18 / 18     W 512: 33 31 / 35, 48 40 / 39     W 4096: 20 130 / 136, 24 150 / 142
+               128 x 64   W 64: 12 17 / 18, 16 19 / 18     W 512: 40 56 / 60, 48 65 / 62     W 4096: 33 359 / 394, 48 487 / 420
+               64 x 128   W 64: 12 14 / 16, 17 18 / 18     W 256: 24 23 / 25, 28 25 / 25     W 1024: 8 44 / 45, 12 53 / 47
+               128 x 128  W 64: 8 19 / 19, 12 23 / 19      W 256: 17 32 / 33, 24 37 / 35     W 1024: 4 60 / 64, 8 74 / 68
+      head     64 x 64    W 64: 24 17 / 18, 28 19 / 18     W 512: 40 35 / 36, 48 40 / 38     W 4096: 33 166 / 179, 48 220 / 201
+               128 x 64   W 64: 20 20 / 21, 24 22 / 21     W 512: 48 57 / 59, 56 64 / 67     W 4096: 33 294 / 343, 48 397 / 366
+               64 x 128   W 64: 24 18 / 19, 28 19 / 19     W 256: 24 24 / 26, 28 27 / 26     W 1024: 8 49 / 46
+               128 x 128  W 64: 20 21 / 22, 24 23 / 22     W 256: 20 32 / 33, 24 34 / 33     W 1024: 4 61 / 59
+               128 x 256  W 64: 20 24 / 23                 W 256: 4 43 / 38"""
+    if vdim < 64:
+        return 48
+    if vdim < 128:
+        if channel:
+            return (32 if W < 256 else 48 if W < 2048 else 24) if dim == 64 else (18 if W < 192 else 48)
+        return (32 if W < 512 else 48) if dim == 64 else (28 if W < 320 else 56)
+    if channel:
+        if 192 <= W < 320:
+            return 28 if dim == 64 else 22
+        return (17 if W < 192 else 12) if dim == 64 else 8
+    if W >= (192 if vdim >= 256 else 320):
+        return 12 if dim == 64 else 8
+    return 28 if dim == 64 else 24
+
+
+def delta_chunks_pay(channel: bool, seq: SeqParams, heads: int, dim: int, vdim: int) -> bool:
+    return seq.num_tokens >= delta_chunk_tokens(channel, seq.batch_size * heads, dim, vdim) * seq.batch_size
 
 
 def _delta_chunks_take(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay, seq: SeqParams, dim: int, vdim: int) -> bool:
@@ -1862,7 +1892,7 @@ def gated_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bpre: to
             state.shape[1:] != (heads, dim, vdim) or not decay.is_contiguous() or not gate.is_contiguous():
         raise RuntimeError("gated_delta_scan: decay [T, H*D], gate [T, H*Dv], norm_w [Dv], state [slots, H, D, Dv]")
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
-    if _delta_chunks_take(q, k, v, decay, seq, dim, vdim):
+    if _delta_chunks_take(q, k, v, decay, seq, dim, vdim) and delta_chunks_pay(True, seq, heads, dim, vdim):
         work, raw = _delta_chunk_buffers(seq, heads, vdim, q.device)
         _check(load().sp_gated_delta_chunks(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                                             v.data_ptr(), v.stride(0), bpre.data_ptr(), bpre.stride(0), decay.data_ptr(),
@@ -1895,7 +1925,7 @@ def head_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: tor
             A_log.numel() != heads or norm_w.numel() != vdim or state.shape[1:] != (heads, dim, vdim):
         raise RuntimeError("head_delta_scan: pre fp32 [T, 2 H], dt_bias / A_log [H], norm_w [Dv], state [slots, H, D, Dv]")
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
-    if ranges is None and _delta_chunks_take(q, k, v, None, seq, dim, vdim):
+    if ranges is None and _delta_chunks_take(q, k, v, None, seq, dim, vdim) and delta_chunks_pay(False, seq, heads, dim, vdim):
         work, raw = _delta_chunk_buffers(seq, heads, vdim, q.device)
         _check(load().sp_head_delta_chunks(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                                            v.data_ptr(), v.stride(0), gate.data_ptr(), gate.stride(0), pre.data_ptr(),

@@ -14,9 +14,9 @@
 // read-out and - on the state just completed - the next token's (w * kn)^T S, then two independent sums over the column's
 // lanes (register moves); no workgroup barrier inside a pass.  The order of its sums depends on the head's sizes only.
 //
-// Decode steps and short portions take that path, steps of 8 and more tokens per request on average (of the sizes that chunk_delta.h
-// takes) the 16-token chunks of sp_gated_delta_chunks, whose sums associate by a token's place in its portion: a request's
-// roundings depend on how its prompt was cut and, through the mean, on the lengths of the others in the step.
+// Decode steps and short portions take that path, longer ones (by the mean tokens per request, the head's sizes and their number; of
+// the sizes that chunk_delta.h takes) the 16-token chunks of sp_gated_delta_chunks, whose sums associate by a token's place in its
+// portion: a request's roundings depend on how its prompt was cut and, through the mean, on the lengths of the others in the step.
 #include "chunk_delta.h"
 #include "chunk_scan.h"
 

@@ -16,9 +16,9 @@
 // several workgroups share a head and hand fp32 read-outs to head_norm_gate_kernel.  The order of its sums depends on the head's
 // sizes only.
 //
-// Decode steps and short portions take that path, steps of 18 and more tokens per request on average (of the sizes that chunk_delta.h
-// takes) the 16-token chunks of sp_head_delta_chunks, whose sums associate by a token's place in its portion: a request's
-// roundings depend on how its prompt was cut and, through the mean, on the lengths of the others in the step.
+// Decode steps and short portions take that path, longer ones (by the mean tokens per request, the head's sizes and their number; of
+// the sizes that chunk_delta.h takes) the 16-token chunks of sp_head_delta_chunks, whose sums associate by a token's place in its
+// portion: a request's roundings depend on how its prompt was cut and, through the mean, on the lengths of the others in the step.
 #include "chunk_delta.h"
 
 namespace sp {

@@ -149,6 +149,15 @@ def test_gated_delta_chunks(lens, H, G, D, Dv, dtype):
         assert torch.isnan(S[slot]).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lens", DELTA_LENS, ids=lambda l: "-".join(map(str, l)))
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 1, 128, 128), (4, 4, 64, 64), (3, 3, 128, 48), (2, 2, 64, 208)])
+def test_gated_delta_chunks_where_the_other_form_pays(lens, H, G, D, Dv, dtype, monkeypatch):
+    from scratchpad_amd import _native
+    monkeypatch.setattr(_native, "delta_chunks_pay", lambda *a: True)
+    test_gated_delta_chunks(lens, H, G, D, Dv, dtype)
+
+
 def test_gated_delta_chunks_of_any_decays():
     """products of up to 16 decays are formed and never quotients: zeros, negative ones and ones above 1 are numbers like others"""
     from scratchpad_amd import _native
@@ -221,6 +230,15 @@ def test_head_delta_chunks_against_the_per_token_kernel(lens, H, G, D, Dv, dtype
         assert ((out.double() - want.double()).abs() <= bar * want.double().abs() + 1e-3).all()
     for slot in range(0, 2 * len(lens) + 1, 2):
         assert torch.isnan(S[slot]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lens", [[18], [15, 32, 17], [16, 200, 3]], ids=lambda l: "-".join(map(str, l)))
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 1, 128, 128), (4, 4, 64, 64), (3, 3, 128, 48), (2, 2, 64, 256)])
+def test_head_delta_chunks_where_the_other_form_pays(lens, H, G, D, Dv, dtype, monkeypatch):
+    from scratchpad_amd import _native
+    monkeypatch.setattr(_native, "delta_chunks_pay", lambda *a: True)
+    test_head_delta_chunks_against_the_per_token_kernel(lens, H, G, D, Dv, dtype)
 
 
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.bfloat16, 32), (torch.float32, 64)])

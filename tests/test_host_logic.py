@@ -234,6 +234,16 @@ def test_skinny_gemm_takes_the_head_of_few_rows():
     assert not pays(5, 128256, 4096) and not pays(9, 128256, 2048) and not pays(3, 4096, 14336)
 
 
+def test_delta_chunk_dispatch_rule():
+    """chunks where they measured faster than the walk token by token: not for portions of 8 (18) tokens whatever the head"""
+    from scratchpad_amd import _native
+    least = _native.delta_chunk_tokens
+    assert least(True, 128, 128, 128) == 8 and least(True, 1024, 128, 128) == 8 and least(False, 1024, 128, 128) == 8
+    assert least(True, 256, 128, 128) > 17 and least(True, 64, 64, 64) > 24 and least(True, 512, 128, 64) > 40
+    assert least(False, 64, 128, 128) > 20 and least(False, 512, 64, 64) > 40 and least(False, 4096, 128, 64) > 33
+    assert all(8 <= least(c, W, D, Dv) <= 56 for c in (True, False) for W in (1, 64, 256, 1024, 8192) for D in (64, 128) for Dv in (16, 64, 128, 256))
+
+
 def test_fp32_product_dispatch_rule():
     """the tiles for many bf16 rows where they measured faster than the library, the library elsewhere"""
     from scratchpad_amd import _native
