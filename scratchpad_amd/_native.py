@@ -761,14 +761,16 @@ _SKINNY_ON = os.environ.get("SP_SKINNY_GEMM", "1") != "0"
 
 def skinny_gemm_pays(M: int, N: int, K: int) -> bool:
     """Where the weight-streaming kernels measured faster than hipBLASLt on MI355X (us, own / library, cold weights): 4096 x 4096
-    10 / 13 at 8 rows; at 4 rows 6144 x 4096 12.7 / 13.3, 28672 x 4096 44 / 58, 128256 x 2048 96 / 114, 128256 x 4096
-    183 / 189; at 8 rows 28672 x 4096 51 / 59, 65536 x 2048 59 / 66, 128256 x 2048 112 / 116 but 128256 x 4096 213 / 184.
-    Above 4 rows every workgroup reads as much x out of L2 as weights, so the win shrinks with rows and with K."""
+    10 / 13 at 8 rows; at 4 rows 6144 x 4096 12.7 / 13.3, 28672 x 4096 44 / 58, 128256 x 2048 92 / 113, 128256 x 4096
+    177 / 184; at 8 rows 28672 x 4096 51 / 59, 65536 x 2048 60 / 66.  Above 4 rows every workgroup reads as much x out of L2 as
+    weights, so the win shrinks with rows and with K.  Heads of more than 65536 columns at 5 / 8 rows: K 512 25 / 28 against the
+    library's 30 / 31 and K 2048 100 / 117 against 114 / 115 at 128256, but K 1024 59 / 68 against 61 / 59 at 152064, K 1536 79 / 94
+    against 73 / 73, K 4096 186 / 211 against 183 / 186."""
     if M <= 16 and N * K <= 4096 * 4096:
         return True
     if M <= 4 and K <= 8192:
         return True
-    return M <= 8 and K <= 8192 and (N <= 65536 or K <= 2048)
+    return M <= 8 and K <= 8192 and (N <= 65536 or K <= 512 or 1792 < K <= 2048)
 
 
 # ---- the row count the library is handed -----------------------------------------------------------------------

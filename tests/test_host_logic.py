@@ -234,6 +234,13 @@ def test_skinny_gemm_takes_the_head_of_few_rows():
     assert not pays(5, 128256, 4096) and not pays(9, 128256, 2048) and not pays(3, 4096, 14336)
 
 
+def test_skinny_gemm_leaves_large_heads_of_short_rows_to_the_library():
+    from scratchpad_amd import _native
+    pays = _native.skinny_gemm_pays
+    assert not pays(8, 128256, 1024) and not pays(5, 128256, 1536) and not pays(8, 262144, 1024)
+    assert pays(4, 128256, 1024) and pays(8, 128256, 512) and pays(8, 65536, 1024)
+
+
 def test_delta_chunk_dispatch_rule():
     """chunks where they measured faster than the walk token by token: not for portions of 8 (18) tokens whatever the head"""
     from scratchpad_amd import _native
