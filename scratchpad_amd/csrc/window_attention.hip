@@ -258,22 +258,24 @@ qkv_norm_store_kernel(void* q, int64_t q_stride, const void* k, int64_t k_stride
 }
 
 // a token that completes a block (position + 1 divisible by P) writes the block's mean key and value at its own slot.
-// A workgroup looks at kPoolRows rows of the step (a lane each) and takes the completing ones in turn; a thread owns V
+// A workgroup looks at `rows` rows of the step (a lane each) and takes the completing ones in turn; a thread owns V
 // neighbouring channels (16 bytes of a row where rows and buffers allow it) and adds the block's rows in order, kPoolAhead of
 // them in flight.  One workgroup per row with a scalar channel per thread and a dependent table read per key took 86 us for
-// 4096 tokens in blocks of 64 x 1024 channels; this takes 9.
-constexpr int kPoolRows = 16, kPoolAhead = 16;
+// 4096 tokens in blocks of 64 x 1024 channels; this takes 9.  One row per workgroup up to kPoolSingles rows: a decode step's requests
+// may all complete a block at once, and 16 blocks in turn took longer than one scalar one (64 requests, blocks of 64 x 1024 channels: 35 us
+// scalar, 100 by sixteens, 8 one by one; 1000 rows of a prompt 8.2 by sixteens, 9.5 one by one).
+constexpr int kPoolRows = 16, kPoolSingles = 256, kPoolAhead = 16;
 
 template <typename Tag, int V>
 __global__ void __launch_bounds__(kBlock)
 pool_blocks_kernel(void* kpooled, void* vpooled, const void* kpool, const void* vpool, int64_t kp_stride, int64_t vp_stride,
-                   const int32_t* req_to_token, int64_t table_stride, SeqBatch s, int64_t T, int kw, int vw, int P) {
+                   const int32_t* req_to_token, int64_t table_stride, SeqBatch s, int64_t T, int rows, int kw, int vw, int P) {
   typedef Elem<Tag> E;
-  const int64_t t0 = (int64_t)blockIdx.x * kPoolRows;
+  const int64_t t0 = (int64_t)blockIdx.x * rows;
   const int lane = threadIdx.x & 63;
   int64_t pos = -1;
   int b = 0;
-  if (lane < kPoolRows && t0 + lane < T) {
+  if (lane < rows && t0 + lane < T) {
     int64_t start, prefix;
     seq_of_token(s, t0 + lane, b, start, prefix);
     pos = prefix + (t0 + lane - start);
@@ -330,15 +332,16 @@ static int launch_pool_blocks(void* kpooled, void* vpooled, const void* kpool, c
                               int64_t vp_stride, const int32_t* req_to_token, int64_t table_stride, const SeqBatch& s, int64_t T,
                               int kw, int vw, int P, hipStream_t st) {
   constexpr int V = Elem<Tag>::kVec;
-  const unsigned rows = (unsigned)((T + kPoolRows - 1) / kPoolRows);
+  const int rows = T <= kPoolSingles ? 1 : kPoolRows;
+  const unsigned groups = (unsigned)((T + rows - 1) / rows);
   const bool vec = kw % V == 0 && vw % V == 0 && kp_stride % V == 0 && vp_stride % V == 0 &&
                    (((uintptr_t)kpooled | (uintptr_t)vpooled | (uintptr_t)kpool | (uintptr_t)vpool) & 15) == 0;
   if (vec)
-    pool_blocks_kernel<Tag, V><<<dim3(rows, (unsigned)(((kw + vw) / V + kBlock - 1) / kBlock)), kBlock, 0, st>>>(
-        kpooled, vpooled, kpool, vpool, kp_stride, vp_stride, req_to_token, table_stride, s, T, kw, vw, P);
+    pool_blocks_kernel<Tag, V><<<dim3(groups, (unsigned)(((kw + vw) / V + kBlock - 1) / kBlock)), kBlock, 0, st>>>(
+        kpooled, vpooled, kpool, vpool, kp_stride, vp_stride, req_to_token, table_stride, s, T, rows, kw, vw, P);
   else
-    pool_blocks_kernel<Tag, 1><<<dim3(rows, (unsigned)((kw + vw + kBlock - 1) / kBlock)), kBlock, 0, st>>>(
-        kpooled, vpooled, kpool, vpool, kp_stride, vp_stride, req_to_token, table_stride, s, T, kw, vw, P);
+    pool_blocks_kernel<Tag, 1><<<dim3(groups, (unsigned)((kw + vw + kBlock - 1) / kBlock)), kBlock, 0, st>>>(
+        kpooled, vpooled, kpool, vpool, kp_stride, vp_stride, req_to_token, table_stride, s, T, rows, kw, vw, P);
   SP_LAUNCH_CHECK();
   return SP_OK;
 }

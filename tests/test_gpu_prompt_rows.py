@@ -47,6 +47,26 @@ def test_pool_blocks(P, kw, vw, dtype):
     assert torch.isnan(kp[~written]).all() and torch.isnan(vp[~written]).all()
 
 
+@pytest.mark.parametrize("B", [1, 17, 256, 257])
+def test_pool_blocks_of_requests_that_complete_together(B):
+    """decode steps whose requests all end a block, on both sides of the line between one row and sixteen per workgroup"""
+    from scratchpad_amd import _native
+    announce("pool_blocks together", B)
+    g = torch.Generator(device=DEV).manual_seed(21)
+    P, W = 16, 64
+    table = (torch.randperm(B * P, generator=g, device=DEV) + 1).to(torch.int32).view(B, P)
+    table = torch.cat([torch.zeros(1, P, dtype=torch.int32, device=DEV), table])
+    k, v = (torch.randn(B * P + 1, W, generator=g, device=DEV).bfloat16() for _ in range(2))
+    kp, vp = torch.full_like(k, float("nan")), torch.full_like(v, float("nan"))
+    seq = _native.SeqParams(torch.arange(1, B + 1, device=DEV), torch.full((B,), P, device=DEV))
+    _native.pool_blocks(kp, vp, k, v, table, seq, P)
+    rows = table[1:].long()
+    for got, src in ((kp, k), (vp, v)):
+        want = src[rows].double().mean(1)
+        assert ((got[rows[:, -1]].double() - want).abs() <= 2.0 ** -8 * src[rows].double().abs().mean(1)).all()
+        assert int(torch.isnan(got).all(1).sum()) == B * P + 1 - B
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("T,parts,per", [(1, 1, 8), (5, 3, 512), (3, 2, 520), (7, 1, 1024), (2, 3, 2048), (2, 1, 2056), (3, 4, 37)])
 def test_gated_group_norm(T, parts, per, dtype):
