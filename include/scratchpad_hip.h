@@ -31,6 +31,8 @@
 extern "C" {
 #endif
 
+/* Raised when an entry's arguments or meaning or a plan's layout change.  Entries that are only added may leave it: a library from
+ * before them lacks them by name, and the Python binding raises where one is called. */
 #define SP_ABI_VERSION 15
 #define SP_API __attribute__((visibility("default")))
 

@@ -185,7 +185,7 @@ SIGNATURES = {
 
 def _not_built(name: str):
     def missing(*_a, **_k):
-        raise RuntimeError(f"{name} is not in this build of {_LIB_PATH} (it was made of the sources of one model family): "
+        raise RuntimeError(f"{name} is not in this build of {_LIB_PATH} (it was made of the sources of one model family, or of older ones): "
                            "run `python -m scratchpad_amd.build` for the whole library")
     return missing
 
@@ -208,7 +208,7 @@ def load() -> ctypes.CDLL:
         try:
             fn = getattr(lib, name)
         except AttributeError:
-            # a library built from the sources of one model family (build.build_native(only=...)): the rest raises on use
+            # a library built from the sources of one model family (build.build_native(only=...)) or of older ones: the rest raises on use
             setattr(lib, name, _not_built(name))
             continue
         fn.restype = res
