@@ -509,7 +509,7 @@ int launch_mamba2_chunks(float* y, int64_t y_stride, const void* xbc, int64_t xb
 
 // The same with rows of 16-byte vectors: a wave per (token, part), the part's values in registers between the sum of squares and
 // the store (VPL vectors of 8 per lane, parts of up to 512 VPL values).  One workgroup per token and a workgroup sum per part
-// (two barriers each, eight parts) took 61 us for 4096 rows of 8 x 512; this takes 20.
+// (two barriers each, eight parts) took 61 us for 4096 rows of 8 x 512; this takes 25.
 template <typename Tag, int VPL>
 __global__ void __launch_bounds__(kBlock)
 gated_group_norm_vec_kernel(void* out, int64_t out_stride, const float* y, int64_t y_stride, const void* z, int64_t z_stride,

@@ -513,10 +513,11 @@ window_attention_kernel(void* out, int64_t out_stride, const void* q, int64_t q_
 // Scores, softmax and O are fp32; P enters the second product as a 16-bit value plus its 16-bit remainder (two products).
 // The vector unit bounds it: a tile's 48 products take 768 cycles, its LDS reads 1024 per workgroup, and masks in 64-bit positions,
 // the library's exponential and a rescaling of O per tile took 3500 per wave.  So masks are formed only where a tile is not wholly
-// visible, in the list's own 32-bit positions; a weight is one fma and one hardware exp2; O is rescaled when a maximum moved; and
-// a query's denominator stays spread over its lanes until the end.  4 requests of 4096 tokens together, 16 heads of 128 on 4, window
-// 512 and blocks of 64: 95 -> 62 us.  Keys (two buffers) and values go to LDS by direct loads: held in registers on the way, with
-// the next tile's on top, they left two workgroups per CU; three fit now, 62 -> 57.
+// visible, in the list's own 32-bit positions; a weight is one fma and one hardware exp2 (a score's product and difference are
+// rounded once; a layer's error against 64 bits is the one with the library's exponential, 4.72e-3); O is rescaled when a maximum
+// moved; and a query's denominator stays spread over its lanes until the end.  4 requests of 4096 tokens together, 16 heads of 128 on
+// 4, window 512 and blocks of 64: 95 -> 62 us.  Keys (two buffers) and values go to LDS by direct loads: held in registers on the way,
+// with the next tile's on top, they left two workgroups per CU; three fit now, 62 -> 57.
 typedef float f32x4_w __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_w __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_w __attribute__((ext_vector_type(8)));
