@@ -1017,8 +1017,9 @@ def linear_relu_square(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 def token_requests(extend_start_loc: torch.Tensor, num_tokens: int) -> torch.Tensor:
     """int32 [num_tokens]: the request that owns each token row of a step (extend_start_loc int32: the requests' first rows)"""
     _gpu(extend_start_loc)
-    if extend_start_loc.dtype != torch.int32 or extend_start_loc.dim() != 1 or not extend_start_loc.is_contiguous():
-        raise RuntimeError("extend_start_loc must be a contiguous int32 vector")
+    if extend_start_loc.dtype != torch.int32 or extend_start_loc.dim() != 1:
+        raise RuntimeError("extend_start_loc must be an int32 vector")
+    extend_start_loc = extend_start_loc.contiguous()
     out = torch.empty(num_tokens, dtype=torch.int32, device=extend_start_loc.device)
     _check(load().sp_token_requests(out.data_ptr(), extend_start_loc.data_ptr(), extend_start_loc.shape[0], num_tokens, _stream()),
            "sp_token_requests")

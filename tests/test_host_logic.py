@@ -580,3 +580,26 @@ def test_forward_batch_refuses_what_nothing_behind_it_reads():
         ForwardBatch.init_new(batch(input_embeds=torch.zeros(2, 8)), runner)
     with pytest.raises(NotImplementedError, match="DP attention"):
         ForwardBatch.init_new(batch(global_num_tokens=[2]), runner)
+
+
+def test_token_requests_takes_first_rows_with_a_stride(monkeypatch):
+    """the requests' first rows may be a column of a table of step lengths: the kernel, which reads them one after the other, is handed a
+    copy"""
+    import ctypes
+    import types
+
+    import torch
+    from scratchpad_amd import _native
+
+    class DeviceTensor(torch.Tensor):
+        is_cuda = True
+
+    seen = []
+    lib = types.SimpleNamespace(sp_token_requests=lambda out, start, batch, tokens, stream: seen.append(
+        list((ctypes.c_int32 * batch).from_address(start))) or 0)
+    monkeypatch.setattr(_native, "load", lambda: lib)
+    monkeypatch.setattr(_native, "_stream", lambda: 0)
+    table = torch.tensor([[0, 3], [3, 2], [5, 4]], dtype=torch.int32).as_subclass(DeviceTensor)
+    for start in (table[:, 0], table[:, 0].contiguous()):
+        assert _native.token_requests(start, 9).shape == (9,)
+    assert seen == [[0, 3, 5], [0, 3, 5]]
