@@ -5,8 +5,11 @@ There is no fallback: if the library is missing or a call fails, a ``RuntimeErro
 signalled, managers/tp_worker_client.py:110-116).  Tensors are passed as raw device pointers on
 ``torch.cuda.current_stream()``; nothing here synchronises.
 """
+import contextlib
 import ctypes
+import gc
 import os
+import threading
 import weakref
 from typing import Optional, Tuple
 
@@ -835,6 +838,32 @@ def library_rows_report() -> dict:
             "substituted": {f"N={n} K={k} M={m}": mp for (n, k, m), mp in sorted(_LIBROWS_USED.items())}}
 
 
+_collector_lock = threading.Lock()
+_collector_off = 0          # captures under way
+_collector_was_on = False
+
+
+@contextlib.contextmanager
+def capture_graph(graph, **kwargs):
+    """torch.cuda.graph with Python's cyclic collector off, in every thread, until the last capture under way has ended.  A graph that
+    is garbage - one of a model runner that was dropped: runner and graph runner hold each other - waits for the device when it is
+    destroyed; a collection inside a capture would do that there, where it is an error, and an error in a destructor ends the process."""
+    global _collector_off, _collector_was_on
+    with _collector_lock:
+        if _collector_off == 0:
+            _collector_was_on = gc.isenabled()
+            gc.disable()
+        _collector_off += 1
+    try:
+        with torch.cuda.graph(graph, **kwargs):
+            yield
+    finally:
+        with _collector_lock:
+            _collector_off -= 1
+            if _collector_off == 0 and _collector_was_on:
+                gc.enable()
+
+
 def _time_mm(x: torch.Tensor, weights, reps: int = 3) -> float:
     """device microseconds of x @ W.T, one call per weight captured into a HIP graph (the weights of different
     layers are cycled so that no call finds its weights in L2 / the Infinity Cache, as in the decode step)"""
@@ -845,7 +874,7 @@ def _time_mm(x: torch.Tensor, weights, reps: int = 3) -> float:
         for i, w in enumerate(weights):
             torch.mm(x, w.t(), out=outs[i % 2])
         st.synchronize()
-        with torch.cuda.graph(g, stream=st, capture_error_mode="thread_local"):
+        with capture_graph(g, stream=st, capture_error_mode="thread_local"):
             for i, w in enumerate(weights):
                 torch.mm(x, w.t(), out=outs[i % 2])
     torch.cuda.synchronize()

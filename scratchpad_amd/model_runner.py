@@ -404,7 +404,7 @@ class HipGraphRunner:
         # of another thread during a capture is an error ("operation not permitted when stream is
         # capturing") and takes the process group down - found by
         # tests/test_gpu_tensor_parallel.py::test_rccl_all_reduce_inside_a_hip_graph_single_rank
-        with torch.cuda.graph(graph, pool=self.pool, stream=self.stream, capture_error_mode="thread_local"):
+        with _native.capture_graph(graph, pool=self.pool, stream=self.stream, capture_error_mode="thread_local"):
             out = run_once()
         self.pool = graph.pool()
         return graph, out

@@ -603,3 +603,81 @@ def test_token_requests_takes_first_rows_with_a_stride(monkeypatch):
     for start in (table[:, 0], table[:, 0].contiguous()):
         assert _native.token_requests(start, 9).shape == (9,)
     assert seen == [[0, 3, 5], [0, 3, 5]]
+
+
+def test_no_garbage_is_collected_inside_a_graph_capture(monkeypatch):
+    """a dropped runner's graphs (runner and graph runner hold each other) are the collector's; destroying one waits for the device, which
+    is an error inside a capture and ends the process there"""
+    import gc
+    import types
+
+    import torch
+    from scratchpad_amd import _native
+    from scratchpad_amd.model_runner import HipGraphRunner
+
+    capturing, destroyed = [], []
+
+    class Graph:
+        def pool(self):
+            return None
+
+        def __del__(self):
+            destroyed.append(bool(capturing))
+
+    class Capture:
+        def __init__(self, graph, **kwargs):
+            pass
+
+        def __enter__(self):
+            capturing.append(1)
+
+        def __exit__(self, *args):
+            capturing.pop()
+
+    class Stream:
+        def wait_stream(self, other):
+            pass
+
+    class Entered:
+        def __init__(self, stream):
+            pass
+        __enter__ = __exit__ = lambda self, *args: None
+
+    for name, value in (("CUDAGraph", Graph), ("graph", Capture), ("Stream", Stream), ("current_stream", Stream), ("stream", Entered),
+                        ("synchronize", lambda: None)):
+        monkeypatch.setattr(torch.cuda, name, value)
+
+    def forward(ids, positions, fb):
+        if capturing:                       # as many containers as a collection of the youngest generation waits for, and more
+            [[i] for i in range(4 * gc.get_threshold()[0])]
+            assert not gc.isenabled()
+
+    runner = types.SimpleNamespace(
+        model=types.SimpleNamespace(forward=forward), req_to_token_pool=None, token_to_kv_pool=None,
+        attn_backend=types.SimpleNamespace(init_forward_metadata_capture_cuda_graph=lambda *a: None))
+    new = HipGraphRunner.__new__(HipGraphRunner)
+    new.model_runner, new.is_encoder_decoder, new.seq_len_fill_value, new.pool, new.stream = runner, False, 1, None, None
+    new.input_ids = new.req_pool_indices = new.seq_lens = new.out_cache_loc = new.positions = torch.zeros(2, dtype=torch.int64)
+    enabled = gc.isenabled()
+    gc.enable()
+    try:
+        gc.collect()
+        old = types.SimpleNamespace(graph=Graph())
+        old.itself = old
+        del old
+        new.capture_one_batch_size(2)
+        assert gc.isenabled() and True not in destroyed
+        with _native.capture_graph(None):
+            with _native.capture_graph(None):
+                pass
+            assert not gc.isenabled()
+        with pytest.raises(KeyError):
+            with _native.capture_graph(None):
+                raise KeyError
+        assert gc.isenabled()
+        gc.disable()
+        with _native.capture_graph(None):
+            pass
+        assert not gc.isenabled()
+    finally:
+        (gc.enable if enabled else gc.disable)()
