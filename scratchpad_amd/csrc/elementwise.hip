@@ -32,7 +32,8 @@ __device__ __forceinline__ float block_sum(float v, float* smem) {
 // nn/layers/layernorm.py:34-51.  y = round(xf * rsqrt(mean(xf^2)+eps)) * w  (second product
 // rounded again: torch multiplies two `dtype` tensors).  Fused: xf = x + residual in fp32,
 // residual <- round(xf), and the UNROUNDED xf is normalised.
-template <typename Tag, bool FUSED, int MAXIT>
+// EARLY: every load of the row, the weights' too, is on its way before the first is used - what a step of a few rows waits for.
+template <typename Tag, bool FUSED, int MAXIT, bool EARLY>
 __global__ __launch_bounds__(kBlock) void rmsnorm_vec_kernel(void* out,  // may alias x_io (fused)
                                                               void* x_io, void* residual,
                                                               const void* __restrict__ weight,
@@ -48,26 +49,29 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_vec_kernel(void* out,  // may 
   char* orow = (char*)out + row * o_stride * E::kBytes;
   const int nvec = hidden / V;
   float cache[MAXIT][V];
-  u32x4 xin[MAXIT], rin[MAXIT], win[MAXIT];
+  constexpr int AHEAD = EARLY ? MAXIT : 1;
+  u32x4 xin[AHEAD], rin[AHEAD], win[AHEAD];
   float ss = 0.f;
+  if constexpr (EARLY) {
 #pragma unroll
-  for (int it = 0; it < MAXIT; ++it) {
-    const int v = threadIdx.x + it * kBlock;
-    if (v < nvec) {
-      xin[it] = ld16(xrow + (int64_t)v * 16);
-      if (FUSED) rin[it] = ld16(rrow + (int64_t)v * 16);
-      win[it] = ld16((const char*)weight + (int64_t)v * 16);
+    for (int it = 0; it < MAXIT; ++it) {
+      const int v = threadIdx.x + it * kBlock;
+      if (v < nvec) {
+        xin[it] = ld16(xrow + (int64_t)v * 16);
+        if (FUSED) rin[it] = ld16(rrow + (int64_t)v * 16);
+        win[it] = ld16((const char*)weight + (int64_t)v * 16);
+      }
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int it = 0; it < MAXIT; ++it) {
     const int v = threadIdx.x + it * kBlock;
     if (v < nvec) {
-      unpack16<Tag>(xin[it], cache[it]);
+      unpack16<Tag>(EARLY ? xin[it % AHEAD] : ld16(xrow + (int64_t)v * 16), cache[it]);
       if (FUSED) {
         float r[V];
-        unpack16<Tag>(rin[it], r);
+        unpack16<Tag>(EARLY ? rin[it % AHEAD] : ld16(rrow + (int64_t)v * 16), r);
 #pragma unroll
         for (int e = 0; e < V; ++e) cache[it][e] = __fadd_rn(cache[it][e], r[e]);
         st16(rrow + (int64_t)v * 16, pack16<Tag>(cache[it]));
@@ -83,7 +87,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_vec_kernel(void* out,  // may 
     const int v = threadIdx.x + it * kBlock;
     if (v < nvec) {
       float w[V], y[V];
-      unpack16<Tag>(win[it], w);
+      unpack16<Tag>(EARLY ? win[it % AHEAD] : ld16((const char*)weight + (int64_t)v * 16), w);
 #pragma unroll
       for (int e = 0; e < V; ++e) y[e] = __fmul_rn(E::round(__fmul_rn(cache[it][e], rs)), w[e]);
       st16(orow + (int64_t)v * 16, pack16<Tag>(y));
@@ -520,8 +524,18 @@ static int launch_rmsnorm(void* out, void* x, void* residual, const void* weight
   const bool vec = hidden % V == 0 && xs % V == 0 && os % V == 0 && (!FUSED || rs % V == 0) &&
                    aligned16(out) && aligned16(x) && aligned16(weight) &&
                    (!FUSED || aligned16(residual)) && hidden / V <= kBlock * MAXIT;
-  if (vec)
-    rmsnorm_vec_kernel<Tag, FUSED, MAXIT><<<dim3((unsigned)T), kBlock, 0, st>>>(
+  // early (E) or late (L) loads, us, fused / plain, bf16.  A workgroup alone on its CU waits for its loads, so E where a thread has more than
+  // one of each: 1 x 4096 L 2.81 / 2.59 E 2.74 / 2.54, 64 x 8192 L 4.08 / 3.63 E 3.89 / 3.53, 256 x 6144 L 4.27 / 3.61 E 4.14 / 3.54; but 64 x
+  // 2048 L 2.66 / 2.49 E 2.79 / 2.59.  Above 256 rows other workgroups fill the waits and E's registers are room that they lack: 300 x 6144
+  // L 4.54 / 3.71 E 4.77 / 3.80, 777 x 8192 L 7.58 / 5.90 E 8.35 / 6.23; plain ones that run at the memory's rate gain again: 2048 x 4096
+  // L 6.84 E 7.03, 2048 x 6144 L 9.25 E 8.86, 4096 x 8192 L 21.7 E 20.7.  fp32 rows, twice the loads, are L only: E did not fit the
+  // registers (512 x 4096 L 6.1 / 4.5 E 61 / 9.2).
+  const bool early = E::kBytes == 2 && hidden > V * kBlock && (T <= 256 || (!FUSED && T * hidden >= 12 << 20));
+  if (vec && early)
+    rmsnorm_vec_kernel<Tag, FUSED, MAXIT, E::kBytes == 2><<<dim3((unsigned)T), kBlock, 0, st>>>(
+        out, x, residual, weight, hidden, xs, rs, os, eps);
+  else if (vec)
+    rmsnorm_vec_kernel<Tag, FUSED, MAXIT, false><<<dim3((unsigned)T), kBlock, 0, st>>>(
         out, x, residual, weight, hidden, xs, rs, os, eps);
   else
     rmsnorm_scalar_kernel<Tag, FUSED><<<dim3((unsigned)T), kBlock, 0, st>>>(

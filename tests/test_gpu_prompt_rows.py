@@ -156,3 +156,20 @@ def test_silu_of_every_16_bit_value(dtype):
     # keep 2^-25
     floor = 3e-37 if dtype == torch.bfloat16 else 2.0 ** -25
     assert ((got - want).abs() <= half + 2.0 ** -22 * want.abs() + floor).all()
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,hidden", [(300, 2048), (300, 2056), (300, 4096), (257, 8192), (2049, 6144)])
+def test_rmsnorm_of_many_rows_is_that_of_a_few(rows, hidden, dtype):
+    """where the loads are issued depends on type, rows and width, a row's bits do not: many rows at once against 128 at a time"""
+    from scratchpad_amd import _native
+    announce("rmsnorm", dtype, rows, hidden)
+    g = torch.Generator().manual_seed(rows + hidden)
+    x, res, w = (torch.randn(*s, generator=g).to(dtype).to(DEV) for s in ((rows, hidden), (rows, hidden), (hidden,)))
+    parts = [slice(i, min(i + 128, rows)) for i in range(0, rows, 128)]
+    many = _native.rmsnorm(x, w, 1e-5)
+    assert torch.equal(many, torch.cat([_native.rmsnorm(x[p], w, 1e-5) for p in parts]))
+    few_x, few_res = x.clone(), res.clone()
+    for p in parts:
+        _native.fused_add_rmsnorm(few_x[p], few_res[p], w, 1e-5)
+    _native.fused_add_rmsnorm(x, res, w, 1e-5)
+    assert torch.equal(x, few_x) and torch.equal(res, few_res)
