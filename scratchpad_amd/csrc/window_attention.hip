@@ -663,12 +663,14 @@ window_attention_mfma_kernel(void* out, int64_t out_stride, const void* q, int64
         }
         if (!plain) {
 #pragma unroll
-          for (int sb = 0; sb < 4; ++sb)
+          for (int sb = 0; sb < 4; ++sb) {
+            if (k0 + 16 * sb >= totalU) continue;         // (nobody sees these; 16 tanh a lane are 0.5 us of a short prompt's 8)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const float v = sacc[sb][r] * scale;
               sacc[sb][r] = softcap > 0.f ? softcap * tanhf(v / softcap) : v;
             }
+          }
         }
         if (k0 < open0 || k0 + 63 > open1) {              // (most tiles of a long window lie inside)
           const int e0 = (int)k0 + 4 * qd;
