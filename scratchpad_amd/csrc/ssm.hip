@@ -671,7 +671,7 @@ static bool short_portions(int64_t tokens, int64_t B, int H, int N, int Dv) {
   const int64_t W = B * H;
   if (tokens < 0 || W <= (Dv == 64 ? 512 : 256)) return false;
   if (N == 64) return tokens <= (Dv == 128 && W >= 1536 ? 12 : 10) * B;
-  return tokens <= 2 * B && W * Dv < (1 << 19);
+  return tokens <= (Dv == 128 ? 4 : 2) * B && W * Dv < (1 << 19);
 }
 
 template <typename Tag>
