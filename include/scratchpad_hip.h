@@ -606,6 +606,14 @@ SP_API int sp_mamba2_scan_tokens(float* y, int64_t y_stride, const void* xbc, in
                                  const float* dt_bias, const float* A_log, const float* Dskip, float* state, int64_t state_stride,
                                  int64_t num_tokens, int heads, int groups, int state_size, int vdim, SP_SEQ_PARAMS, int dtype,
                                  void* stream);
+/* The same (bf16 rows, state_size and vdim 64 or 128, several tokens per request; else SP_ERR_UNSUPPORTED and nothing is launched) with
+ * a request's tokens shared out in segments of segment_tokens (a multiple of 64) that run side by side.  work: fp32,
+ * sp_scan_segment_floats(num_tokens, batch_size, heads, state_size, vdim, segment_tokens) values, 16-byte aligned.             */
+SP_API int64_t sp_scan_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim, int segment_tokens);
+SP_API int sp_mamba2_scan_segments(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
+                                   const float* dt_bias, const float* A_log, const float* Dskip, float* state, int64_t state_stride,
+                                   float* work, int segment_tokens, int64_t num_tokens, int heads, int groups, int state_size, int vdim,
+                                   SP_SEQ_PARAMS, int dtype, void* stream);
 /* out = (y * silu(z)) / rms_part * weight: each row of n values normed in `parts` equal parts (y fp32; z, out in `dtype`) */
 SP_API int sp_gated_group_norm(void* out, int64_t out_stride, const float* y, int64_t y_stride, const void* z,
                                int64_t z_stride, const float* weight, int64_t num_tokens, int n, int parts, float eps,
@@ -627,6 +635,13 @@ SP_API int sp_mlstm_scan_tokens(void* out, int64_t out_stride, const void* q, in
                                 const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
                                 float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, int64_t num_tokens, int heads,
                                 int dim, int vdim, float cap, float eps, SP_SEQ_PARAMS, int dtype, void* stream);
+/* In segments, as sp_mamba2_scan_segments (dim and vdim 64 or 128). */
+SP_API int sp_mlstm_scan_segments(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                  const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
+                                  const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
+                                  float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, float* work, int segment_tokens,
+                                  int64_t num_tokens, int heads, int dim, int vdim, float cap, float eps, SP_SEQ_PARAMS, int dtype,
+                                  void* stream);
 SP_API int sp_mlstm_scan_gates(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
                                const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
                                const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,

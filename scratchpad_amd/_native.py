@@ -146,6 +146,11 @@ SIGNATURES = {
     "sp_causal_conv_silu": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i32, _i32, *_SEQ, _i32, _vp]),
     "sp_mamba2_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, *_SEQ, _i32, _vp]),
     "sp_mamba2_scan_tokens": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, *_SEQ, _i32, _vp]),
+    "sp_scan_segment_floats": (_i64, [_i64, _i32, _i32, _i32, _i32, _i32]),
+    "sp_mamba2_scan_segments": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i32, _i64, _i32, _i32, _i32, _i32, *_SEQ,
+                                       _i32, _vp]),
+    "sp_mlstm_scan_segments": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i64,
+                                      _vp, _i64, _vp, _i32, _i64, _i32, _i32, _i32, _f32, _f32, *_SEQ, _i32, _vp]),
     "sp_gated_group_norm": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i32, _i32, _f32, _i32, _vp]),
     "sp_mlstm_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp,
                              _i64, _i32, _i32, _i32, _f32, _f32, *_SEQ, _i32, _vp]),
@@ -1625,6 +1630,30 @@ def causal_conv_silu(u: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     return out
 
 
+SCAN_SEGMENT = None      # tests and measurements: the segments' length of every step that can be cut (0: none is)
+
+
+def _scan_segment(tokens: int, requests: int, heads: int, slots: int, least: int) -> int:
+    """Length of the segments that a step's requests are cut into (0: they are not): the shortest that keeps all segments (a last
+    partial one per request counts half) in one round of the ``slots`` workgroups that the chip holds at a time, where the longest
+    request - the lengths are on the device: taken for twice the mean - has at least ``least`` tokens and three and a half of them.
+    us per layer, whole / cut, width 2048 (requests x tokens together, segment):  mLSTM 1 x 4096, 320: 742 / 241   4 x 4096, 320: 328 / 243
+    5 x 3001, 256: 271 / 209   1 x 1000, 128: 211 / 109   2 x 500, 128: 121 / 106   1 x 300, 128: 98 / 106   8 x 4096, 384: 255 / 271
+    Mamba-2 1 x 4096, 576: 668 / 448   2 x 4096, 640: 529 / 457   1 x 1000, 192: 208 / 169   3 x 1000, 192: 169 / 175   4 x 4096, 704: 434 / 471"""
+    if SCAN_SEGMENT is not None:
+        return SCAN_SEGMENT
+    longest, room = min(tokens, 2 * tokens // requests), 2 * (slots // heads) - requests      # room: half segments
+    if longest < least or room <= 0:
+        return 0
+    length = max(128, -(-2 * tokens // (64 * room)) * 64)
+    return length if 7 * length <= 2 * longest else 0
+
+
+def _scan_segments_take(rows, dim: int, vdim: int, seq: SeqParams) -> bool:
+    return seq.extend_seq_lens is not None and dim in (64, 128) and vdim in (64, 128) and all(
+        t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(0) < 1 << 24 for t in rows)
+
+
 def mamba2_scan(xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor,
                 state: torch.Tensor, seq: SeqParams, heads: int, groups: int, state_size: int, vdim: int) -> torch.Tensor:
     """xbc [T, heads * vdim + 2 * groups * state_size] -> y fp32 [T, heads * vdim]; state [slots, heads, state_size, vdim]"""
@@ -1634,6 +1663,16 @@ def mamba2_scan(xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, 
             state.shape[1:] != (heads, state_size, vdim) or dt_bias.numel() != heads or A_log.numel() != heads or D.numel() != heads:
         raise RuntimeError("mamba2_scan: shapes do not fit")
     y = torch.empty((xbc.shape[0], inner), dtype=torch.float32, device=xbc.device)
+    segment = _scan_segment(seq.num_tokens, seq.batch_size, heads, 512 if vdim == 64 else 256, 800) if \
+        _scan_segments_take((xbc,), state_size, vdim, seq) and y.stride(0) < 1 << 24 else 0
+    if segment:
+        work = torch.empty(load().sp_scan_segment_floats(seq.num_tokens, seq.batch_size, heads, state_size, vdim, segment),
+                           dtype=torch.float32, device=xbc.device)
+        _check(load().sp_mamba2_scan_segments(y.data_ptr(), y.stride(0), xbc.data_ptr(), xbc.stride(0), dt_raw.data_ptr(),
+                                              dt_bias.data_ptr(), A_log.data_ptr(), D.data_ptr(), state.data_ptr(), state.stride(0),
+                                              work.data_ptr(), segment, seq.num_tokens, heads, groups, state_size, vdim, *seq.args,
+                                              _dt(xbc), _stream()), "sp_mamba2_scan_segments")
+        return y
     _check(load().sp_mamba2_scan_tokens(y.data_ptr(), y.stride(0), xbc.data_ptr(), xbc.stride(0), dt_raw.data_ptr(),
                                         dt_bias.data_ptr(), A_log.data_ptr(), D.data_ptr(), state.data_ptr(), state.stride(0),
                                         seq.num_tokens, heads, groups, state_size, vdim, *seq.args, _dt(xbc), _stream()),
@@ -1673,6 +1712,16 @@ def mlstm_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tenso
             S.shape[1:] != (heads, dim, vdim) or n.shape[1:] != (heads, dim) or m.shape[1:] != (heads,):
         raise RuntimeError("mlstm_scan: gate or state shapes do not fit")
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
+    segment = _scan_segment(T, seq.batch_size, heads, 512 if dim == 64 and vdim == 64 else 256, 448) if \
+        _scan_segments_take((q, k, v), dim, vdim, seq) and max(g.stride(0), out.stride(0)) < 1 << 24 else 0
+    if segment:
+        work = torch.empty(load().sp_scan_segment_floats(T, seq.batch_size, heads, dim, vdim, segment), dtype=torch.float32, device=q.device)
+        _check(load().sp_mlstm_scan_segments(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
+                                             v.data_ptr(), v.stride(0), g.data_ptr(), g.stride(0), ipre.data_ptr(), fpre.data_ptr(),
+                                             ipre.stride(0) if T > 1 else heads, norm_w.data_ptr(), S.data_ptr(), S.stride(0),
+                                             n.data_ptr(), n.stride(0), m.data_ptr(), m.stride(0), work.data_ptr(), segment, T, heads,
+                                             dim, vdim, cap, eps, *seq.args, _dt(q), _stream()), "sp_mlstm_scan_segments")
+        return out
     _check(load().sp_mlstm_scan_tokens(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                                       v.data_ptr(), v.stride(0), g.data_ptr(), g.stride(0), ipre.data_ptr(), fpre.data_ptr(),
                                       ipre.stride(0) if T > 1 else heads, norm_w.data_ptr(), S.data_ptr(), S.stride(0), n.data_ptr(),

@@ -90,14 +90,15 @@ __device__ __forceinline__ int64_t uniform64(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-template <int D, int NW>
+// (OUT false: the state's part only, for the sums of a request's segments - no q, no rows of k, no outputs)
+template <int D, int NW, bool OUT = true>
 struct ChunkScan {
   static constexpr int Dv = NW * 16, NT = NW * 64, QROW = D * 2 + 16, TROW = kCL * 2 + 16;
-  static constexpr int kQ = 0, kKT = kQ + kCL * QROW, kVT = kKT + D * TROW, kP = kVT + Dv * TROW;
+  static constexpr int kQ = 0, kKT = kQ + (OUT ? kCL * QROW : 0), kVT = kKT + D * TROW, kP = kVT + Dv * TROW;
   static constexpr int kK = kP;                                  // the rows of k are gone when the weighted tiles arrive
-  static constexpr int kPBytes = 3 * kCL * TROW > kCL * QROW ? 3 * kCL * TROW : kCL * QROW;
+  static constexpr int kPBytes = !OUT ? 0 : 3 * kCL * TROW > kCL * QROW ? 3 * kCL * TROW : kCL * QROW;
   static constexpr int kSum = kP + kPBytes;                      // float [4][kCL]: sums of the weighted tiles over s
-  static constexpr int kScalars = kSum + 4 * kCL * 4;
+  static constexpr int kScalars = kSum + (OUT ? 4 * kCL * 4 : 0);
   static constexpr int kOdd = kScalars + 2 * (int)sizeof(ChunkScalars);      // int: the last chunk's number + 1 with such values
   static constexpr int kFirst = kOdd + 16;                                   // int [Dv]: a column's first token of it
   static constexpr int kBytes = kFirst + Dv * 4;
@@ -134,7 +135,7 @@ struct ChunkScan {
 #pragma unroll
     for (int u = 0; u < QU; ++u) {
       const int x = tid + u * NT;
-      if (x < QN) rq[u] = row16(qb, qs, x / (D / 8), n, x % (D / 8) * 16);
+      if (OUT && x < QN) rq[u] = row16(qb, qs, x / (D / 8), n, x % (D / 8) * 16);
     }
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
@@ -164,14 +165,16 @@ struct ChunkScan {
 #pragma unroll
     for (int u = 0; u < QU; ++u) {
       const int x = tid + u * NT;
-      if (x < QN) st16(lds + kQ + x / (D / 8) * QROW + x % (D / 8) * 16, rq[u]);
+      if (OUT && x < QN) st16(lds + kQ + x / (D / 8) * QROW + x % (D / 8) * 16, rq[u]);
     }
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
       const int x = tid + u * NT, t = x % (kCL / 2) * 2, c = x / (kCL / 2);
       if (x < KN) {
-        st16(lds + kK + t * QROW + c * 16, rk[u][0]);
-        st16(lds + kK + (t + 1) * QROW + c * 16, rk[u][1]);
+        if constexpr (OUT) {
+          st16(lds + kK + t * QROW + c * 16, rk[u][0]);
+          st16(lds + kK + (t + 1) * QROW + c * 16, rk[u][1]);
+        }
         put_transposed(lds + kKT + c * 8 * TROW + t * 2, rk[u][0], rk[u][1]);
       }
     }
@@ -179,10 +182,12 @@ struct ChunkScan {
     for (int u = 0; u < VU; ++u) {
       const int x = tid + u * NT, t = x % (kCL / 2) * 2, c = x / (kCL / 2);
       if (x < VN) {
-        uint32_t ones = 0u;                            // (an exponent of ones carries into the sign)
+        if constexpr (OUT) {
+          uint32_t ones = 0u;                          // (an exponent of ones carries into the sign)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ones |= (rv[u][e & 1][e / 2] & 0x7f807f80u) + 0x00800080u;
-        if (ones & 0x80008000u) *odd() = chunk + 1;
+          for (int e = 0; e < 8; ++e) ones |= (rv[u][e & 1][e / 2] & 0x7f807f80u) + 0x00800080u;
+          if (ones & 0x80008000u) *odd() = chunk + 1;
+        }
         put_transposed(lds + kVT + c * 8 * TROW + t * 2, rv[u][0], rv[u][1]);
       }
     }
@@ -292,7 +297,8 @@ struct ChunkScan {
   }
   // o += (weighted tiles) v;  S = a_end S + k^T (w v)
   __device__ __forceinline__ void absorb(int chunk) {
-    const bool any = __builtin_amdgcn_readfirstlane(*odd()) == chunk + 1;
+    // (OUT false: a value that is not finite leaves its column of the state so by itself)
+    const bool any = OUT && __builtin_amdgcn_readfirstlane(*odd()) == chunk + 1;
     if (any) clear();
     const float a_end = sc->a_end;
 #pragma unroll
@@ -302,11 +308,12 @@ struct ChunkScan {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       const u32x4 v = ld16(lds + kVT + column() * TROW + ks * 64 + 16 * q);
+      if constexpr (OUT)
 #pragma unroll
-      for (int x = 2; x >= 0; --x)
+        for (int x = 2; x >= 0; --x)
 #pragma unroll
-        for (int i = 2 * ks; i < 4; ++i)
-          o[i] = mfma_c(ld16(lds + kP + (x * kCL + 16 * i + r16) * TROW + ks * 64 + 16 * q), v, o[i]);
+          for (int i = 2 * ks; i < 4; ++i)
+            o[i] = mfma_c(ld16(lds + kP + (x * kCL + 16 * i + r16) * TROW + ks * 64 + 16 * q), v, o[i]);
       float f[8];
       unpack16<bf16_tag>(v, f);
       const f32x4_c w0 = *(const f32x4_c*)(sc->w + ks * 32 + 8 * q), w1 = *(const f32x4_c*)(sc->w + ks * 32 + 8 * q + 4);
@@ -333,7 +340,7 @@ struct ChunkScan {
     }
     if (any) spoil();
   }
-  __device__ __forceinline__ void load_state(const float* st, bool held) {
+  __device__ __forceinline__ void load_state(const float* st, bool held) {      // (st is not read unless held)
 #pragma unroll
     for (int i = 0; i < DT; ++i)
 #pragma unroll
@@ -352,6 +359,113 @@ struct ChunkScan {
   }
 };
 
+// ---- segments: a request's chunks as several workgroups -----------------------------------------------------------------------
+// One workgroup per (request, head) walks the request's chunks in turn; few requests leave most of the chip idle and the longest one
+// sets the time.  The state is linear in the one a segment starts from, so segments of `tokens` tokens (a multiple of kCL) run side by
+// side in three launches: every segment but a request's last walks its own tokens from an empty state (kSegmentSums; no outputs, about
+// a third of the work), segment_states_kernel chains these sums into the state that each segment starts from, and every segment
+// walks its tokens once more from there (kSegmentOutputs); a request's last one leaves the new state in the pool.  3001
+// tokens of 5 requests, 16 heads of 128 x 128 (mLSTM), segments of 256: 146 us -> 19 (sums) + 8 (states) + 54 (outputs); the rule for the
+// segments' length (_native.py) has both sides' times of whole layers.
+enum { kWholeRequests = 0, kSegmentSums = 1, kSegmentOutputs = 2 };
+
+// of a segment and head, in the workspace: S [D * Dv], n [D] (mLSTM), then kSegScalars floats: the decay of what the segment started
+// from (mLSTM: as the sum of the log forget gates, a double, and the largest exponent of its own sums; the one that it starts from)
+constexpr int kSegScalars = 8, kSegDecay = 0, kSegMax = 2, kSegStart = 3;
+
+inline int64_t segment_floats(int D, int Dv, bool normaliser) { return (int64_t)D * Dv + (normaliser ? D : 0) + kSegScalars; }
+
+struct ScanSegments {
+  float* work;
+  int64_t stride;            // floats per segment and head
+  int tokens;
+};
+
+__device__ __forceinline__ int segments_of(int len, int tokens) { return (len + tokens - 1) / tokens; }
+// the request, first token (within it) and length of segment `id` of the step; false behind the last (all lanes of a wave ask)
+__device__ __forceinline__ bool segment_at(const SeqBatch& s, int id, int tokens, int lane, int& b, int& t0) {
+  for (int b0 = 0; b0 < s.B; b0 += 64) {
+    const int i = b0 + lane;
+    const int n = i < s.B ? segments_of(max(s.extend_seq_lens[i], 0), tokens) : 0;
+    int incl = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += o;
+    }
+    const uint64_t hit = __ballot(id < incl);
+    if (hit) {
+      const int l = __ffsll((unsigned long long)hit) - 1;
+      b = __builtin_amdgcn_readfirstlane(b0 + l);
+      t0 = __builtin_amdgcn_readfirstlane((id - __shfl(incl - n, l, 64)) * tokens);
+      return true;
+    }
+    id -= __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
+  }
+  return false;
+}
+
+// Workgroup (request, head, 1024 values of S): the sums of the request's segments become the states they start from.  Memory: a read
+// and a write of all segments' states.  MAXED (mLSTM): sums are relative to exp(their largest exponent), n is chained too.
+template <bool MAXED>
+__global__ void __launch_bounds__(256)
+segment_states_kernel(ScanSegments g, const float* S_state, int64_t S_stride, const float* n_state, int64_t n_stride, const float* m_state,
+                      int64_t m_stride, SeqBatch s, int H, int D, int Dv) {
+  const int b = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
+  const int segments = segments_of(s.extend_seq_lens[b], g.tokens);
+  if (segments <= 1) return;
+  int before = 0;
+  for (int i = lane; i < b; i += 64) before += segments_of(max(s.extend_seq_lens[i], 0), g.tokens);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
+  const bool held = s.extend_prefix_lens[b] > 0;
+  const int64_t slot = load_idx(s.req_pool_indices, b, s.idx64);
+  const int states = D * Dv, scalars = states + (MAXED ? D : 0), e = (blockIdx.z * 256 + threadIdx.x) * 4;
+  float* const first = g.work + ((int64_t)before * H + h) * g.stride;
+  const int64_t step = H * g.stride;
+  const bool live = e < scalars;                       // (n's values follow those of S)
+  f32x4_c S = {0.f, 0.f, 0.f, 0.f};
+  if (held && live) {
+    const float* from = e < states ? S_state + slot * S_stride + (int64_t)h * states + e : n_state + slot * n_stride + (int64_t)h * D + e - states;
+    S = f32x4_c{from[0], from[1], from[2], from[3]};
+  }
+  float m = MAXED && held ? m_state[slot * m_stride + h] : 0.f;
+  constexpr int AHEAD = 8;
+  for (int i0 = 0; i0 < segments; i0 += AHEAD) {
+    f32x4_c sum[AHEAD];
+    double F[AHEAD];
+    float top[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const float* at = first + min(i0 + u, segments - 2) * step;      // (the last segment has no sums)
+      sum[u] = live ? *(const f32x4_c*)(at + e) : f32x4_c{0.f, 0.f, 0.f, 0.f};
+      if constexpr (MAXED) {
+        F[u] = *(const double*)(at + scalars + kSegDecay);
+        top[u] = at[scalars + kSegMax];
+      } else {
+        top[u] = at[scalars + kSegDecay];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      if (i0 + u >= segments) break;
+      float* at = first + (i0 + u) * step;
+      if (live) *(f32x4_c*)(at + e) = S;
+      if (MAXED && e == 0) at[scalars + kSegStart] = m;
+      if constexpr (MAXED) {
+        const double old = F[u] + (double)m, now = fmax(old, (double)top[u]);
+        const float keep = expf((float)(old - now)), take = expf((float)((double)top[u] - now));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[r] = keep * S[r] + take * sum[u][r];
+        m = F[u] != F[u] ? (float)F[u] : (float)now;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[r] = top[u] * S[r] + sum[u][r];
+      }
+    }
+  }
+}
+
 // raise a kernel's dynamic-LDS limit to `bytes`, once per device of the process (`raised`: a static of the launching function)
 inline bool chunk_lds_ready(PerDevice<int>& raised, const void* kernel, int bytes) {
   int ok = 0;
@@ -360,3 +474,9 @@ inline bool chunk_lds_ready(PerDevice<int>& raised, const void* kernel, int byte
 }
 
 }  // namespace sp
+
+// (weak: both sources that include this define it, a library may hold either or both; with mLSTM's normaliser, for either)
+extern "C" __attribute__((weak)) int64_t sp_scan_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim,
+                                                                int segment_tokens) {
+  return (num_tokens / segment_tokens + batch_size) * heads * sp::segment_floats(dim, vdim, true);
+}

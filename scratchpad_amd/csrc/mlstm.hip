@@ -157,45 +157,56 @@ mlstm_scan_kernel(void* out, int64_t out_stride, const void* q, int64_t q_stride
 // lane exchanges (1.6 us per token: 1546 us at 3001 tokens of 5 requests, 16 heads of 128 x 128); this one takes 140 us there
 // and 568 us for one request of 4096 tokens, 8.9 us per chunk: about 1500 vector instructions per wave at two waves per SIMD
 // (the splits, the weights' exponentials, the epilogue) against 126 MFMAs and 0.5 MB of LDS reads.
-template <int D, int NW>
+template <int D, int NW, bool OUT = true>
 struct MlstmLds {
-  typedef ChunkScan<D, NW> C;
+  typedef ChunkScan<D, NW, OUT> C;
   static constexpr int kN = (C::kBytes + 15) / 16 * 16, kNq = kN + D * 4, kFloor = kNq + kCL * 4, kRed = kFloor + 2 * kCL * 4;
   static constexpr int kGates = (kRed + NW * kCL * 4 + 7) / 8 * 8;             // double [NW][3][kCL]: F, b and its running maximum of NW chunks
   static constexpr int kBytes = kGates + NW * 3 * kCL * 8;
 };
 
 // (heads of 64 x 64: registers for the two workgroups per CU that LDS has room for)
-template <int D, int NW>
-__global__ void __launch_bounds__(NW * 64, D == 64 ? 8 / NW : 1)
+// In segments (see chunk_scan.h): MODE.
+template <int D, int NW, int MODE>
+__global__ void __launch_bounds__(NW * 64, MODE == kSegmentSums ? 4 : D == 64 ? 8 / NW : 1)
 mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_stride, const char* k, int64_t k_stride, const char* v,
                    int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre,
                    int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride,
-                   float* m_state, int64_t m_stride, SeqBatch s, int H, float cap, float eps) {
+                   float* m_state, int64_t m_stride, ScanSegments seg, SeqBatch s, int H, float cap, float eps) {
+  constexpr bool OUT = MODE != kSegmentSums;
   typedef Elem<bf16_tag> E;
-  typedef ChunkScan<D, NW> C;
-  typedef MlstmLds<D, NW> L;
+  typedef ChunkScan<D, NW, OUT> C;
+  typedef MlstmLds<D, NW, OUT> L;
   constexpr int Dv = C::Dv, NT = C::NT;
   extern __shared__ __attribute__((aligned(16))) char chunk_lds[];
-  const int b = blockIdx.x, h = blockIdx.y;
+  C c(chunk_lds);
+  const int h = blockIdx.y;
+  int b = blockIdx.x, t0 = 0;
+  if constexpr (MODE != kWholeRequests)
+    if (!segment_at(s, (int)blockIdx.x, seg.tokens, c.lane, b, t0)) return;
   int64_t start, len, prefix;
   seq_span(s, b, start, len, prefix);
   if (len <= 0) return;
-  C c(chunk_lds);
+  const bool split = MODE != kWholeRequests && len > seg.tokens, final = t0 + seg.tokens >= len;
+  if (MODE == kSegmentSums && final) return;
   float* sn = (float*)(chunk_lds + L::kN);
   float* snq = (float*)(chunk_lds + L::kNq);
   float* sfloor = (float*)(chunk_lds + L::kFloor);
   float* red = (float*)(chunk_lds + L::kRed);
   double* sgate = (double*)(chunk_lds + L::kGates);
-  const bool held = prefix > 0;
-  start = uniform64(start), len = uniform64(len);
+  const bool held = OUT && (prefix > 0 || t0 > 0);
+  start = uniform64(start) + t0, len = uniform64(len) - t0;
+  if (MODE != kWholeRequests && len > seg.tokens) len = seg.tokens;
   const int64_t slot = uniform64(load_idx(s.req_pool_indices, b, s.idx64));
   float* Sst = S_state + slot * S_stride + (int64_t)h * D * Dv;
   float* nst = n_state + slot * n_stride + (int64_t)h * D;
   float* mst = m_state + slot * m_stride + h;
-  c.load_state(Sst, held);
-  if (c.tid < D) sn[c.tid] = held ? nst[c.tid] : 0.f;
-  float m = held ? mst[0] : 0.f;                      // (kept by the wave that forms the scalars)
+  float* const part = MODE == kWholeRequests ? nullptr : seg.work + ((int64_t)blockIdx.x * H + h) * seg.stride;
+  c.load_state(split ? part : Sst, held);
+  if (c.tid < D) sn[c.tid] = held ? (split ? part + D * Dv : nst)[c.tid] : 0.f;
+  // (kept by the wave that forms the scalars; a segment's sums know no earlier token)
+  float m = MODE == kSegmentSums ? -INFINITY : split ? part[D * Dv + D + kSegStart] : held ? mst[0] : 0.f;
+  double passed = 0.;                                 // kSegmentSums: the sum of the log forget gates
   const float qscale = 1.f / sqrtf((float)D);
   q += (start * q_stride + (int64_t)h * D) * 2;
   k += (start * k_stride + (int64_t)h * D) * 2;
@@ -228,12 +239,15 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
     const double F = from[0], bs = from[kCL], G = fmax((double)m, from[2 * kCL]);
     const double Gend = __shfl(G, 63, 64), Fend = __shfl(F, 63, 64);
     ChunkScalars& sc = *c.scalars(c0 / kCL);
-    ChunkScalars::put(sc.lt, c.lane, Gend - G);
-    ChunkScalars::put(sc.ls, c.lane, Gend - bs);
-    sc.cs[c.lane] = qscale;
-    sc.a0[c.lane] = expf((float)(m - G)) * qscale;
+    if constexpr (OUT) {
+      ChunkScalars::put(sc.lt, c.lane, Gend - G);
+      ChunkScalars::put(sc.ls, c.lane, Gend - bs);
+      sc.cs[c.lane] = qscale;
+      sc.a0[c.lane] = expf((float)(m - G)) * qscale;
+      sfloor[(c0 / kCL & 1) * kCL + c.lane] = expf((float)-(F + G));
+    }
     sc.w[c.lane] = expf((float)(bs - Gend));
-    sfloor[(c0 / kCL & 1) * kCL + c.lane] = expf((float)-(F + G));
+    passed += Fend;
     if (c.lane == 0) sc.a_end = expf((float)(m - Gend));
     m = (float)(Fend + Gend);
   };
@@ -250,33 +264,35 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
     c.stage((int)(c0 / kCL));
     lds_barrier();
     if (c0 + kCL < len) load(c0 + kCL);
-    c.scores();
-    c.from_state(zero);
-    zero = false;
-    {      // n_0 . q of a token: the lanes of a token share its D channels
-      constexpr int PER = NT / kCL, DP = D / PER;
-      const int t = c.tid / PER, part = c.tid % PER;
-      float d = 0.f;
-#pragma unroll
-      for (int i = 0; i < DP; i += 8) {
-        float f[8];
-        unpack16<bf16_tag>(ld16(chunk_lds + C::kQ + t * C::QROW + (part * DP + i) * 2), f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) d += sn[part * DP + i + e] * f[e];
-      }
-      d = lanes_sum<PER>(d);
-      if (part == 0) snq[t] = d;
-    }
     uint16_t gv[4][4];
+    if constexpr (OUT) {
+      c.scores();
+      c.from_state(zero);
+      zero = false;
+      {      // n_0 . q of a token: the lanes of a token share its D channels
+        constexpr int PER = NT / kCL, DP = D / PER;
+        const int t = c.tid / PER, part = c.tid % PER;
+        float d = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < DP; i += 8) {
+          float f[8];
+          unpack16<bf16_tag>(ld16(chunk_lds + C::kQ + t * C::QROW + (part * DP + i) * 2), f);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * i + 4 * c.q + r;
-        gv[i][r] = *(const uint16_t*)(gb + c0 * g_stride * 2 + (uint32_t)((t < n ? t : n - 1) * (uint32_t)g_stride + col) * 2u);
+          for (int e = 0; e < 8; ++e) d += sn[part * DP + i + e] * f[e];
+        }
+        d = lanes_sum<PER>(d);
+        if (part == 0) snq[t] = d;
       }
-    lds_barrier();
-    c.template weigh<true>();
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = 16 * i + 4 * c.q + r;
+          gv[i][r] = *(const uint16_t*)(gb + c0 * g_stride * 2 + (uint32_t)((t < n ? t : n - 1) * (uint32_t)g_stride + col) * 2u);
+        }
+      lds_barrier();
+      c.template weigh<true>();
+    }
     if (c0 + kCL < len && (c0 / kCL + 1) % NW != 0) gates(c0 + kCL);
     {      // the normaliser's update: the lanes of a channel share the chunk's tokens
       constexpr int PER = NT / D, TP = kCL / PER;
@@ -293,8 +309,12 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
       x = lanes_sum<PER>(x);
       if (part == 0) sn[d] = sc.a_end * sn[d] + x;
     }
-    lds_barrier();
+    if constexpr (OUT) lds_barrier();
     c.absorb((int)(c0 / kCL));
+    if constexpr (!OUT) {
+      lds_barrier();
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -321,25 +341,52 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
                    c.o[i][r] * f * nw / (1.f + expf(-gate)));
       }
   }
-  c.store_state(Sst);
-  if (c.tid < D) nst[c.tid] = sn[c.tid];
-  if (c.tid == (NW - 1) * 64) mst[0] = m;
+  if constexpr (MODE == kSegmentSums) {
+    c.store_state(part);
+    if (c.tid < D) part[D * Dv + c.tid] = sn[c.tid];
+    if (c.tid == (NW - 1) * 64) {
+      *(double*)(part + D * Dv + D + kSegDecay) = passed;
+      part[D * Dv + D + kSegMax] = m;
+    }
+  } else if (MODE == kWholeRequests || final) {
+    c.store_state(Sst);
+    if (c.tid < D) nst[c.tid] = sn[c.tid];
+    if (c.tid == (NW - 1) * 64) mst[0] = m;
+  }
 }
 
-template <int D, int NW>
-static int launch_mlstm_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
-                               const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
-                               const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
-                               float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, const SeqBatch& s, int H, float cap, float eps,
-                               hipStream_t st) {
-  constexpr int bytes = MlstmLds<D, NW>::kBytes;
+#define SP_MLSTM_SCAN_PARAMS                                                                                                             \
+  void *out, int64_t out_stride, const void *q, int64_t q_stride, const void *k, int64_t k_stride, const void *v, int64_t v_stride,       \
+      const void *g, int64_t g_stride, const float *ipre, const float *fpre, int64_t gate_stride, const float *norm_w, float *S_state,    \
+      int64_t S_stride, float *n_state, int64_t n_stride, float *m_state, int64_t m_stride, const ScanSegments &seg, const SeqBatch &s,   \
+      int H, float cap, float eps, hipStream_t st
+#define SP_MLSTM_SCAN_ARGS                                                                                                                \
+  out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, gate_stride, norm_w, S_state, S_stride, n_state,       \
+      n_stride, m_state, m_stride, seg, s, H, cap, eps, st
+
+template <int D, int NW, int MODE>
+static int launch_mlstm_mode(unsigned groups, SP_MLSTM_SCAN_PARAMS) {
+  constexpr int bytes = MlstmLds<D, NW, MODE != kSegmentSums>::kBytes;
   static PerDevice<int> raised;
-  if (!chunk_lds_ready(raised, (const void*)mlstm_chunk_kernel<D, NW>, bytes)) return SP_ERR_LAUNCH;
-  mlstm_chunk_kernel<D, NW><<<dim3((unsigned)s.B, (unsigned)H), NW * 64, bytes, st>>>(
+  if (!chunk_lds_ready(raised, (const void*)mlstm_chunk_kernel<D, NW, MODE>, bytes)) return SP_ERR_LAUNCH;
+  mlstm_chunk_kernel<D, NW, MODE><<<dim3(groups, (unsigned)H), NW * 64, bytes, st>>>(
       out, out_stride, (const char*)q, q_stride, (const char*)k, k_stride, (const char*)v, v_stride, g, g_stride, ipre, fpre, gate_stride,
-      norm_w, S_state, S_stride, n_state, n_stride, m_state, m_stride, s, H, cap, eps);
+      norm_w, S_state, S_stride, n_state, n_stride, m_state, m_stride, seg, s, H, cap, eps);
   SP_LAUNCH_CHECK();
   return SP_OK;
+}
+
+// (seg.tokens 0: a request's chunks by one workgroup per head)
+template <int D, int NW>
+static int launch_mlstm_chunks(int64_t tokens, SP_MLSTM_SCAN_PARAMS) {
+  if (seg.tokens == 0) return launch_mlstm_mode<D, NW, kWholeRequests>((unsigned)s.B, SP_MLSTM_SCAN_ARGS);
+  const unsigned groups = (unsigned)(tokens / seg.tokens + s.B);
+  const int rc = launch_mlstm_mode<D, NW, kSegmentSums>(groups, SP_MLSTM_SCAN_ARGS);
+  if (rc != SP_OK) return rc;
+  segment_states_kernel<true><<<dim3((unsigned)s.B, (unsigned)H, D * NW * 16 / 1024 + 1), 256, 0, st>>>(
+      seg, S_state, S_stride, n_state, n_stride, m_state, m_stride, s, H, D, NW * 16);
+  SP_LAUNCH_CHECK();
+  return launch_mlstm_mode<D, NW, kSegmentOutputs>(groups, SP_MLSTM_SCAN_ARGS);
 }
 
 // Steps of short portions that the per-token form walks faster than a chunk of 64 mostly empty tokens costs: requests x heads of few
@@ -356,25 +403,18 @@ static bool short_portions(int64_t tokens, int64_t B, int H, int D, int Dv) {
 }
 
 template <typename Tag>
-static int launch_mlstm(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
-                        const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre,
-                        int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride,
-                        float* m_state, int64_t m_stride, const SeqBatch& s, int H, int D, int Dv, int64_t tokens, float cap,
-                        float eps, hipStream_t st) {
+static int launch_mlstm(int D, int Dv, int64_t tokens, SP_MLSTM_SCAN_PARAMS) {
   // a step of one token per request stays with the per-token form (one sweep over the state is all there is to do), and so do
   // the types and head sizes the matrix form is not built for, and short portions of many requests
   if (std::is_same<Tag, bf16_tag>::value && s.extend_seq_lens && (D == 64 || D == 128) && (Dv == 64 || Dv == 128) &&
       chunk_aligned(q, q_stride) && chunk_aligned(k, k_stride) && chunk_aligned(v, v_stride) &&
-      g_stride < ((int64_t)1 << 24) && out_stride < ((int64_t)1 << 24) && !short_portions(tokens, s.B, H, D, Dv)) {
-#define SP_MLSTM_CHUNKS(D_, NW_)                                                                                              \
-  return launch_mlstm_chunks<D_, NW_>(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, gate_stride, norm_w, \
-                                      S_state, S_stride, n_state, n_stride, m_state, m_stride, s, H, cap, eps, st)
-    if (D == 128 && Dv == 128) SP_MLSTM_CHUNKS(128, 8);
-    if (D == 128) SP_MLSTM_CHUNKS(128, 4);
-    if (Dv == 128) SP_MLSTM_CHUNKS(64, 8);
-    SP_MLSTM_CHUNKS(64, 4);
-#undef SP_MLSTM_CHUNKS
+      g_stride < ((int64_t)1 << 24) && out_stride < ((int64_t)1 << 24) && (seg.tokens || !short_portions(tokens, s.B, H, D, Dv))) {
+    if (D == 128 && Dv == 128) return launch_mlstm_chunks<128, 8>(tokens, SP_MLSTM_SCAN_ARGS);
+    if (D == 128) return launch_mlstm_chunks<128, 4>(tokens, SP_MLSTM_SCAN_ARGS);
+    if (Dv == 128) return launch_mlstm_chunks<64, 8>(tokens, SP_MLSTM_SCAN_ARGS);
+    return launch_mlstm_chunks<64, 4>(tokens, SP_MLSTM_SCAN_ARGS);
   }
+  if (seg.tokens) return SP_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)s.B, (unsigned)H);
   if ((Dv + 1) * (D > 64 ? 4 : (D > 32 ? 2 : 1)) > 1024) return SP_ERR_UNSUPPORTED;      // vdim 256 with dim > 64
 #define SP_MLSTM(DP)                                                                                                    \
@@ -392,6 +432,8 @@ static int launch_mlstm(void* out, int64_t out_stride, const void* q, int64_t q_
   SP_LAUNCH_CHECK();
   return SP_OK;
 }
+#undef SP_MLSTM_SCAN_PARAMS
+#undef SP_MLSTM_SCAN_ARGS
 
 }  // namespace
 }  // namespace sp
@@ -400,11 +442,11 @@ using namespace sp;
 
 // (gate_stride: values between the gates of a token and the next one's, so that both may be halves of one product's rows; num_tokens:
 // the step's rows, < 0 where the caller does not know; only the choice between the two forms depends on it)
-extern "C" int sp_mlstm_scan_tokens(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
-                                    const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* ipre,
-                                    const float* fpre, int64_t gate_stride, const float* norm_w, float* S_state, int64_t S_stride,
-                                    float* n_state, int64_t n_stride, float* m_state, int64_t m_stride, int64_t num_tokens,
-                                    int heads, int dim, int vdim, float cap, float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
+static int mlstm_scan(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                      int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre, int64_t gate_stride,
+                      const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride, float* m_state,
+                      int64_t m_stride, const ScanSegments& seg, int64_t num_tokens, int heads, int dim, int vdim, float cap, float eps,
+                      SP_SEQ_PARAMS, int dtype, void* stream) {
   SP_CHECK_ARG(batch_size >= 0 && heads > 0 && dim > 0 && vdim > 0 && vdim <= 256 && cap > 0.f);
   if (batch_size == 0) return SP_OK;
   SP_CHECK_ARG(out && q && k && v && g && ipre && fpre && norm_w && S_state && n_state && m_state && req_pool_indices && seq_lens);
@@ -413,9 +455,32 @@ extern "C" int sp_mlstm_scan_tokens(void* out, int64_t out_stride, const void* q
   SP_CHECK_ARG(q_stride >= nk && k_stride >= nk && v_stride >= nv && g_stride >= nv && out_stride >= nv);
   SP_CHECK_ARG(S_stride >= nk * vdim && n_stride >= nk && m_stride >= heads && gate_stride >= heads);
   SEQ_BATCH(s);
-  SP_DISPATCH_DTYPE(dtype, return (launch_mlstm<Tag>(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre,
-                                                     fpre, gate_stride, norm_w, S_state, S_stride, n_state, n_stride, m_state, m_stride, s,
-                                                     heads, dim, vdim, num_tokens, cap, eps, (hipStream_t)stream)));
+  SP_DISPATCH_DTYPE(dtype, return (launch_mlstm<Tag>(dim, vdim, num_tokens, out, out_stride, q, q_stride, k, k_stride, v, v_stride, g,
+                                                     g_stride, ipre, fpre, gate_stride, norm_w, S_state, S_stride, n_state, n_stride,
+                                                     m_state, m_stride, seg, s, heads, cap, eps, (hipStream_t)stream)));
+}
+
+extern "C" int sp_mlstm_scan_tokens(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                                    int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre, int64_t gate_stride,
+                                    const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride, float* m_state,
+                                    int64_t m_stride, int64_t num_tokens, int heads, int dim, int vdim, float cap, float eps, SP_SEQ_PARAMS,
+                                    int dtype, void* stream) {
+  return mlstm_scan(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, gate_stride, norm_w, S_state, S_stride,
+                    n_state, n_stride, m_state, m_stride, ScanSegments{nullptr, 0, 0}, num_tokens, heads, dim, vdim, cap, eps,
+                    req_pool_indices, seq_lens, extend_seq_lens, extend_prefix_lens, extend_start_loc, token_req, idx64, batch_size, dtype,
+                    stream);
+}
+
+extern "C" int sp_mlstm_scan_segments(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                                      int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre, int64_t gate_stride,
+                                      const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride, float* m_state,
+                                      int64_t m_stride, float* work, int segment_tokens, int64_t num_tokens, int heads, int dim, int vdim,
+                                      float cap, float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
+  SP_CHECK_ARG(num_tokens >= 0 && segment_tokens > 0 && segment_tokens % kCL == 0 && work && ((uintptr_t)work & 15) == 0);
+  return mlstm_scan(out, out_stride, q, q_stride, k, k_stride, v, v_stride, g, g_stride, ipre, fpre, gate_stride, norm_w, S_state, S_stride,
+                    n_state, n_stride, m_state, m_stride, ScanSegments{work, segment_floats(dim, vdim, true), segment_tokens}, num_tokens,
+                    heads, dim, vdim, cap, eps, req_pool_indices, seq_lens, extend_seq_lens, extend_prefix_lens, extend_start_loc, token_req,
+                    idx64, batch_size, dtype, stream);
 }
 
 extern "C" int sp_mlstm_scan_gates(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,

@@ -415,22 +415,31 @@ mamba2_scan_kernel(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stri
 // old state exp(L_t).  One workgroup of Dv / 16 waves per (request, head); B and C are read once per head of their group.
 // The per-token form is a chain of LDS reads, sums and lane exchanges per token (1.2 us; 788 us at 8 requests of 4096 tokens
 // together, 64 heads of 128 x 64); this one takes 87 us there and 351 us for one request of 4096 tokens (5.5 us per chunk).
-template <int N, int NW>
-__global__ void __launch_bounds__(NW * 64, 8 / NW)
+// In segments (see chunk_scan.h): MODE.
+template <int N, int NW, int MODE>
+__global__ void __launch_bounds__(NW * 64, MODE == kSegmentSums ? 4 : 8 / NW)
 mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_stride, const float* dt_raw, const float* dt_bias,
-                    const float* A_log, const float* Dskip, float* state, int64_t state_stride, SeqBatch s, int H, int G) {
-  typedef ChunkScan<N, NW> C;
+                    const float* A_log, const float* Dskip, float* state, int64_t state_stride, ScanSegments seg, SeqBatch s, int H, int G) {
+  constexpr bool OUT = MODE != kSegmentSums;
+  typedef ChunkScan<N, NW, OUT> C;
   constexpr int Dv = C::Dv;
   extern __shared__ __attribute__((aligned(16))) char chunk_lds[];
-  const int b = blockIdx.x, h = blockIdx.y, g = h / (H / G);
+  C c(chunk_lds);
+  const int h = blockIdx.y, g = h / (H / G);
+  int b = blockIdx.x, t0 = 0;
+  if constexpr (MODE != kWholeRequests)
+    if (!segment_at(s, (int)blockIdx.x, seg.tokens, c.lane, b, t0)) return;
   int64_t start, len, prefix;
   seq_span(s, b, start, len, prefix);
   if (len <= 0) return;
-  C c(chunk_lds);
-  start = uniform64(start), len = uniform64(len);
-  const bool held = prefix > 0;
+  const bool split = MODE != kWholeRequests && len > seg.tokens, last = t0 + seg.tokens >= len;
+  if (MODE == kSegmentSums && last) return;
+  start = uniform64(start) + t0, len = uniform64(len) - t0;
+  if (MODE != kWholeRequests && len > seg.tokens) len = seg.tokens;
+  const bool held = OUT && (prefix > 0 || t0 > 0);
   float* st = state + uniform64(load_idx(s.req_pool_indices, b, s.idx64)) * state_stride + (int64_t)h * N * Dv;
-  c.load_state(st, held);
+  float* const part = MODE == kWholeRequests ? nullptr : seg.work + ((int64_t)blockIdx.x * H + h) * seg.stride;
+  c.load_state(split ? part : st, held);
   const int64_t inner = (int64_t)H * Dv, row = xbc_stride * 2;
   const char* x0 = xbc + start * row + (int64_t)h * Dv * 2;
   const char* b0 = xbc + start * row + (inner + (int64_t)g * N) * 2;
@@ -440,7 +449,7 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
     const int n = (int)(len - c0 < kCL ? len - c0 : kCL);
     c.load(c0p + c0 * row, row, b0 + c0 * row, row, x0 + c0 * row, row, n);
   };
-  float raw = 0.f;
+  float raw = 0.f, decay = 1.f;
   const auto load_steps = [&](int64_t c0) {
     if (c.wave == NW - 1 && c0 + c.lane < len) raw = dt_raw[(start + c0 + c.lane) * H + h];
   };
@@ -451,12 +460,16 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
     // (e^-128 is zero in fp32: a stronger decay is the same one, and the sums stay where their differences are exact)
     const double L = wave_scan_sum((double)(e < -128.f ? -128.f : e), c.lane), Lend = __shfl(L, 63, 64);
     ChunkScalars& sc = *c.scalars(c0 / kCL);
-    ChunkScalars::put(sc.lt, c.lane, L);
-    ChunkScalars::put(sc.ls, c.lane, L);
-    sc.cs[c.lane] = dt;
-    sc.a0[c.lane] = expf((float)L);
+    if constexpr (OUT) {
+      ChunkScalars::put(sc.lt, c.lane, L);
+      ChunkScalars::put(sc.ls, c.lane, L);
+      sc.cs[c.lane] = dt;
+      sc.a0[c.lane] = expf((float)L);
+    }
     sc.w[c.lane] = expf((float)(Lend - L)) * dt;
-    if (c.lane == 0) sc.a_end = expf((float)Lend);
+    const float a_end = expf((float)Lend);
+    if (c.lane == 0) sc.a_end = a_end;
+    decay *= a_end;
   };
   load(0);
   load_steps(0);
@@ -471,40 +484,67 @@ mamba2_chunk_kernel(float* y, int64_t y_stride, const char* xbc, int64_t xbc_str
       load_steps(c0 + kCL);                           // (first: they are waited for first, and loads arrive in order)
       load(c0 + kCL);
     }
-    c.scores();
-    c.from_state(zero);
-    zero = false;
-    lds_barrier();
-    c.template weigh<false>();
+    if constexpr (OUT) {
+      c.scores();
+      c.from_state(zero);
+      zero = false;
+      lds_barrier();
+      c.template weigh<false>();
+    }
     if (c0 + kCL < len) steps(c0 + kCL);
-    lds_barrier();
+    if constexpr (OUT) lds_barrier();
     c.absorb((int)(c0 / kCL));
-    char* yc = (char*)(y + (start + c0) * y_stride + (int64_t)h * Dv);
+    if constexpr (OUT) {
+      char* yc = (char*)(y + (start + c0) * y_stride + (int64_t)h * Dv);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t0 = 16 * i + 4 * c.q;
-      const u32x2 xv = *(const u32x2*)(chunk_lds + C::kVT + c.column() * C::TROW + t0 * 2);
-      const float x[4] = {as_f32(xv[0] << 16), as_f32(xv[0] & 0xffff0000u), as_f32(xv[1] << 16), as_f32(xv[1] & 0xffff0000u)};
+      for (int i = 0; i < 4; ++i) {
+        const int tt = 16 * i + 4 * c.q;
+        const u32x2 xv = *(const u32x2*)(chunk_lds + C::kVT + c.column() * C::TROW + tt * 2);
+        const float x[4] = {as_f32(xv[0] << 16), as_f32(xv[0] & 0xffff0000u), as_f32(xv[1] << 16), as_f32(xv[1] & 0xffff0000u)};
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (t0 + r < n) *(float*)(yc + (uint32_t)((t0 + r) * (uint32_t)y_stride + c.column()) * 4u) = c.o[i][r] + skip * x[r];
+        for (int r = 0; r < 4; ++r)
+          if (tt + r < n) *(float*)(yc + (uint32_t)((tt + r) * (uint32_t)y_stride + c.column()) * 4u) = c.o[i][r] + skip * x[r];
+      }
     }
     lds_barrier();
   }
-  c.store_state(st);
+  if constexpr (MODE == kSegmentSums) {
+    c.store_state(part);
+    if (c.tid == (NW - 1) * 64) part[N * Dv + kSegDecay] = decay;
+  } else if (MODE == kWholeRequests || last) {
+    c.store_state(st);
+  }
 }
 
-template <int N, int NW>
-int launch_mamba2_chunks(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw, const float* dt_bias,
-                         const float* A_log, const float* Dskip, float* state, int64_t state_stride, const SeqBatch& s, int H,
-                         int G, hipStream_t st) {
-  constexpr int bytes = ChunkScan<N, NW>::kBytes;
+template <int N, int NW, int MODE>
+int launch_mamba2_mode(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw, const float* dt_bias,
+                       const float* A_log, const float* Dskip, float* state, int64_t state_stride, const ScanSegments& seg, unsigned groups,
+                       const SeqBatch& s, int H, int G, hipStream_t st) {
+  constexpr int bytes = ChunkScan<N, NW, MODE != kSegmentSums>::kBytes;
   static PerDevice<int> raised;
-  if (!chunk_lds_ready(raised, (const void*)mamba2_chunk_kernel<N, NW>, bytes)) return SP_ERR_LAUNCH;
-  mamba2_chunk_kernel<N, NW><<<dim3((unsigned)s.B, (unsigned)H), NW * 64, bytes, st>>>(
-      y, y_stride, (const char*)xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, state_stride, s, H, G);
+  if (!chunk_lds_ready(raised, (const void*)mamba2_chunk_kernel<N, NW, MODE>, bytes)) return SP_ERR_LAUNCH;
+  mamba2_chunk_kernel<N, NW, MODE><<<dim3(groups, (unsigned)H), NW * 64, bytes, st>>>(
+      y, y_stride, (const char*)xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, state_stride, seg, s, H, G);
   SP_LAUNCH_CHECK();
   return SP_OK;
+}
+
+// (seg.tokens 0: a request's chunks by one workgroup per head)
+template <int N, int NW>
+int launch_mamba2_chunks(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw, const float* dt_bias,
+                         const float* A_log, const float* Dskip, float* state, int64_t state_stride, const ScanSegments& seg, int64_t tokens,
+                         const SeqBatch& s, int H, int G, hipStream_t st) {
+#define SP_MODE(MODE, GROUPS)                                                                                                            \
+  launch_mamba2_mode<N, NW, MODE>(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, state_stride, seg, GROUPS, s, H, G, st)
+  if (seg.tokens == 0) return SP_MODE(kWholeRequests, (unsigned)s.B);
+  const unsigned groups = (unsigned)(tokens / seg.tokens + s.B);
+  int rc = SP_MODE(kSegmentSums, groups);
+  if (rc != SP_OK) return rc;
+  segment_states_kernel<false><<<dim3((unsigned)s.B, (unsigned)H, N * NW * 16 / 1024), 256, 0, st>>>(
+      seg, state, state_stride, nullptr, 0, nullptr, 0, s, H, N, NW * 16);
+  SP_LAUNCH_CHECK();
+  return SP_MODE(kSegmentOutputs, groups);
+#undef SP_MODE
 }
 
 // The same with rows of 16-byte vectors: a wave per (token, part), the part's values in registers between the sum of squares and
@@ -677,19 +717,21 @@ static bool short_portions(int64_t tokens, int64_t B, int H, int N, int Dv) {
 template <typename Tag>
 static int launch_mamba2(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
                          const float* dt_bias, const float* A_log, const float* Dskip, float* state, int64_t state_stride,
-                         const SeqBatch& s, int H, int G, int N, int Dv, int64_t tokens, hipStream_t st) {
+                         const ScanSegments& seg, const SeqBatch& s, int H, int G, int N, int Dv, int64_t tokens,
+                         hipStream_t st) {
   // a step of one token per request stays with the per-token form (one sweep over the state is all there is to do), and so do
   // the types and head sizes the matrix form is not built for, and short portions of many requests
   if (std::is_same<Tag, bf16_tag>::value && s.extend_seq_lens && (N == 64 || N == 128) && (Dv == 64 || Dv == 128) &&
-      chunk_aligned(xbc, xbc_stride) && y_stride < ((int64_t)1 << 24) && !short_portions(tokens, s.B, H, N, Dv)) {
+      chunk_aligned(xbc, xbc_stride) && y_stride < ((int64_t)1 << 24) && (seg.tokens || !short_portions(tokens, s.B, H, N, Dv))) {
 #define SP_CHUNKS(N_, NW_)                                                                                              \
-  return launch_mamba2_chunks<N_, NW_>(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, state_stride, s, H, G, st)
+  return launch_mamba2_chunks<N_, NW_>(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, state_stride, seg, tokens, s, H, G, st)
     if (N == 128 && Dv == 128) SP_CHUNKS(128, 8);
     if (N == 128) SP_CHUNKS(128, 4);
     if (Dv == 128) SP_CHUNKS(64, 8);
     SP_CHUNKS(64, 4);
 #undef SP_CHUNKS
   }
+  if (seg.tokens) return SP_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)s.B, (unsigned)H);
 #define SP_SCAN(NP)                                                                                                    \
   mamba2_scan_kernel<Tag, NP><<<grid, (unsigned)((Dv * split_of(NP) + 63) / 64 * 64), (size_t)kChunk * Dv * sizeof(float), st>>>(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, \
@@ -706,10 +748,9 @@ static int launch_mamba2(float* y, int64_t y_stride, const void* xbc, int64_t xb
 }
 
 // (num_tokens: the step's rows, < 0 where the caller does not know; only the choice between the two forms depends on it)
-extern "C" int sp_mamba2_scan_tokens(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
-                                     const float* dt_bias, const float* A_log, const float* Dskip, float* state,
-                                     int64_t state_stride, int64_t num_tokens, int heads, int groups, int state_size, int vdim,
-                                     SP_SEQ_PARAMS, int dtype, void* stream) {
+static int mamba2_scan(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw, const float* dt_bias,
+                       const float* A_log, const float* Dskip, float* state, int64_t state_stride, const ScanSegments& seg,
+                       int64_t num_tokens, int heads, int groups, int state_size, int vdim, SP_SEQ_PARAMS, int dtype, void* stream) {
   SP_CHECK_ARG(batch_size >= 0 && heads > 0 && groups > 0 && heads % groups == 0 && state_size > 0 && vdim > 0 && vdim <= 256);
   if (batch_size == 0) return SP_OK;
   SP_CHECK_ARG(y && xbc && dt_raw && dt_bias && A_log && Dskip && state && req_pool_indices && seq_lens);
@@ -719,8 +760,28 @@ extern "C" int sp_mamba2_scan_tokens(float* y, int64_t y_stride, const void* xbc
   SP_CHECK_ARG(state_stride >= (int64_t)heads * state_size * vdim);
   SEQ_BATCH(s);
   SP_DISPATCH_DTYPE(dtype, return (launch_mamba2<Tag>(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state,
-                                                      state_stride, s, heads, groups, state_size, vdim, num_tokens,
+                                                      state_stride, seg, s, heads, groups, state_size, vdim, num_tokens,
                                                       (hipStream_t)stream)));
+}
+
+extern "C" int sp_mamba2_scan_tokens(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
+                                     const float* dt_bias, const float* A_log, const float* Dskip, float* state,
+                                     int64_t state_stride, int64_t num_tokens, int heads, int groups, int state_size, int vdim,
+                                     SP_SEQ_PARAMS, int dtype, void* stream) {
+  return mamba2_scan(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, state_stride, ScanSegments{nullptr, 0, 0},
+                     num_tokens, heads, groups, state_size, vdim, req_pool_indices, seq_lens, extend_seq_lens, extend_prefix_lens,
+                     extend_start_loc, token_req, idx64, batch_size, dtype, stream);
+}
+
+extern "C" int sp_mamba2_scan_segments(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
+                                       const float* dt_bias, const float* A_log, const float* Dskip, float* state, int64_t state_stride,
+                                       float* work, int segment_tokens, int64_t num_tokens, int heads, int groups, int state_size,
+                                       int vdim, SP_SEQ_PARAMS, int dtype, void* stream) {
+  SP_CHECK_ARG(num_tokens >= 0 && segment_tokens > 0 && segment_tokens % kCL == 0 && work && ((uintptr_t)work & 15) == 0);
+  return mamba2_scan(y, y_stride, xbc, xbc_stride, dt_raw, dt_bias, A_log, Dskip, state, state_stride,
+                     ScanSegments{work, segment_floats(state_size, vdim, false), segment_tokens}, num_tokens, heads, groups, state_size,
+                     vdim, req_pool_indices, seq_lens, extend_seq_lens, extend_prefix_lens, extend_start_loc, token_req, idx64, batch_size,
+                     dtype, stream);
 }
 
 extern "C" int sp_mamba2_scan(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,

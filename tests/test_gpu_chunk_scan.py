@@ -526,3 +526,50 @@ def test_lowrank_gate_of_infinite_inputs():
     for got, ref in ((decay, torch.exp(-torch.nn.functional.softplus(plain))), (sig, torch.sigmoid(plain))):
         assert torch.equal(torch.isnan(got[keep]), torch.isnan(ref[keep]))
         assert torch.allclose(got[keep], ref[keep], rtol=1e-5, atol=1e-6, equal_nan=True)
+
+
+SEGMENT_LENS = [[129], [64, 300, 1], [128, 127, 500, 2, 65], [257] + [3] * 66 + [192]]
+
+
+@pytest.mark.parametrize("lens", SEGMENT_LENS, ids=lambda l: "-".join(map(str, l[:5])))
+@pytest.mark.parametrize("H,D,Dv", [(3, 128, 128), (2, 128, 64), (2, 64, 128), (5, 64, 64)])
+def test_scans_in_segments(lens, H, D, Dv, monkeypatch):
+    """segments of 64 and 128 tokens around their edges, from an empty and from a held state, more requests than lanes: against the
+    64-bit recurrences, as the whole requests above"""
+    from scratchpad_amd import _native
+    for segment in (64, 128):
+        monkeypatch.setattr(_native, "SCAN_SEGMENT", segment)
+        test_mlstm_chunks(lens, H, D, Dv)
+        test_mamba2_chunks(lens, 2 * H, H, D, Dv)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_segments_keep_a_number_that_is_not_finite_from_earlier_tokens(bad, monkeypatch):
+    from scratchpad_amd import _native
+    monkeypatch.setattr(_native, "SCAN_SEGMENT", 64)
+    H, D, T, at = 2, 64, 320, 100
+    g = torch.Generator(device=DEV).manual_seed(5)
+    a = torch.randn(T, 4 * H * D, generator=g, device=DEV).bfloat16()
+    gates, ones = torch.randn(T, 2 * H, generator=g, device=DEV), torch.ones(H * D, device=DEV)
+    xbc, dt, zeros = torch.randn(T, 3 * H * D, generator=g, device=DEV).bfloat16(), torch.randn(T, H, generator=g, device=DEV), torch.zeros(H, device=DEV)
+
+    def run(where):
+        b, x, gt, d = a.clone(), xbc.clone(), gates.clone(), dt.clone()
+        if where == "value":
+            b[at, 2 * H * D + 3] = bad
+            x[at, 3] = bad
+        elif where == "gate":
+            gt[at] = d[at] = float("nan")
+        S, n, m = (torch.zeros(2, H, *s, device=DEV) for s in ((D, D), (D,), ()))
+        seq = seq_extend([T], [0], [1])
+        out = _native.mlstm_scan(*b.split([H * D] * 4, 1), gt[:, :H], gt[:, H:], ones, S, n, m, seq, H, D, D, 15.0, 1e-5)
+        S2 = torch.zeros(2, H, D, D, device=DEV)
+        y = _native.mamba2_scan(x, d, zeros, zeros, zeros, S2, seq, H, H, D, D)
+        return out, y, S[1], S2[1]
+    clean = run("nowhere")
+    for where in ("value", "gate"):
+        out, y, S, S2 = run(where)
+        assert torch.equal(out[:at], clean[0][:at]) and torch.equal(y[:at], clean[1][:at])
+        cols = [3] if where == "value" else list(range(D))
+        assert not torch.isfinite(S[0][:, cols]).any() and not torch.isfinite(S2[0][:, cols]).any()
+        assert not torch.isfinite(out[at:].view(-1, H, D)[:, 0, cols].float()).any() and not torch.isfinite(y[at:].view(-1, H, D)[:, 0, cols]).any()

@@ -262,6 +262,23 @@ def test_fp32_product_dispatch_rule():
     assert not pays(256, 2048, 2048) and not pays(65, 4096, 2048)
 
 
+def test_scan_segments_keep_to_one_round_and_to_long_requests():
+    """a step is cut only where its longest request is likely to be several segments, into multiples of 64 tokens whose workgroups the
+    chip holds at a time"""
+    from scratchpad_amd import _native
+    rule = _native._scan_segment
+    for tokens in (1, 64, 300, 448, 1000, 3001, 4096, 16384, 100000):
+        for requests in (1, 2, 5, 8, 16, 300):
+            for heads in (1, 8, 16, 64, 300):
+                for slots, least in ((256, 448), (512, 800)):
+                    n = rule(tokens, requests, heads, slots, least)
+                    if n:
+                        assert n % 64 == 0 and n >= 128 and tokens >= least and 7 * n <= 4 * tokens // requests
+                        assert (tokens / n + requests / 2) * heads <= slots
+    assert rule(4096, 1, 16, 256, 448) and rule(3001, 5, 16, 256, 448) and rule(4096, 1, 64, 512, 800)
+    assert not rule(4096, 8, 16, 256, 448) and not rule(300, 1, 16, 256, 448) and not rule(4096, 4, 64, 512, 800)
+
+
 def test_mlstm_scan_takes_no_gate_rows_that_overlap(monkeypatch):
     """gates whose rows lie closer than their width (an expanded row, a sliding view) are refused before anything is launched: the
     kernel reads [token, head] at rows at least `heads` apart.  Views of one product and strides that differ pass."""
