@@ -700,6 +700,16 @@ SP_API int sp_hgrn2_scan(void* out, int64_t out_stride, const void* qpre, int64_
                          int64_t f_stride, const void* v, int64_t v_stride, const float* f_bias, const float* lower,
                          const float* norm_w, float* state, int64_t state_stride, int heads, int dim, int vdim, float eps,
                          SP_SEQ_PARAMS, int dtype, void* stream);
+/* The same for steps of several tokens per request, 16 tokens at a time on the matrix cores (fp32 throughout): dim and vdim 64 or 128,
+ * rows of qpre and fpre 16-byte aligned; else SP_ERR_UNSUPPORTED and nothing is launched.  Products of up to 16 gates are formed (never
+ * quotients).  work: fp32, sp_hgrn2_chunk_floats values, 16-byte aligned.  segment_tokens > 0 (a multiple of 16): a request's tokens are
+ * shared out in segments that run side by side, segment_work (fp32, 16-byte aligned) holds sp_hgrn2_segment_floats values.          */
+SP_API int64_t sp_hgrn2_chunk_floats(int64_t num_tokens, int batch_size, int heads, int dim);
+SP_API int64_t sp_hgrn2_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim, int segment_tokens);
+SP_API int sp_hgrn2_chunks(void* out, int64_t out_stride, const void* qpre, int64_t q_stride, const void* fpre, int64_t f_stride,
+                           const void* v, int64_t v_stride, const float* f_bias, const float* lower, const float* norm_w, float* state,
+                           int64_t state_stride, float* work, float* segment_work, int segment_tokens, int64_t num_tokens, int heads,
+                           int dim, int vdim, float eps, SP_SEQ_PARAMS, int dtype, void* stream);
 
 
 /* ================================================================================================================

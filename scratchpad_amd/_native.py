@@ -168,6 +168,10 @@ SIGNATURES = {
                                    _f32, *_SEQ, _i32, _vp]),
     "sp_delta_step": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i32, _f32,
                              _vp, _vp, _i64, _i32, _i32, _f32, *_SEQ, _i32, _vp]),
+    "sp_hgrn2_chunk_floats": (_i64, [_i64, _i32, _i32, _i32]),
+    "sp_hgrn2_segment_floats": (_i64, [_i64, _i32, _i32, _i32, _i32, _i32]),
+    "sp_hgrn2_chunks": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _i32, _i64, _i32, _i32, _i32,
+                               _f32, *_SEQ, _i32, _vp]),
     "sp_hgrn2_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _f32,
                              *_SEQ, _i32, _vp]),
     # ---- ABI 13
@@ -1839,6 +1843,38 @@ def delta_step(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tenso
     return out
 
 
+HGRN2_CHUNKS = None      # tests and measurements: True / False takes / leaves the chunks of 16 wherever they are built for the form
+
+
+def hgrn2_chunks_pay(tokens: int, requests: int, heads: int) -> bool:
+    """Prompts whose longest request (the lengths are on the device: taken for twice the mean) is long enough to pay for two more
+    launches, or steps of so many requests x heads that the per-token form's walk is bound by its work.  us per layer of width 2048
+    (8 heads of 128 x 128; requests x tokens together), per token / in chunks:  1 x 65: 84 / 86   1 x 300: 215 / 90   16 x 512: 81 / 83
+    16 x 256: 81 / 86   4 x 1000: 245 / 91   1 x 4096: 2633 / 175   16 x 4096: 361 / 177   64 x 1024: 89 / 83   256 x 4096: 254 / 173"""
+    if HGRN2_CHUNKS is not None:
+        return HGRN2_CHUNKS
+    return min(tokens, 2 * tokens // requests) >= 72 or (tokens >= 16 * requests and requests * heads >= 512)
+
+
+def _hgrn2_chunks_take(rows, seq: SeqParams, dim: int, vdim: int) -> bool:
+    """the forms sp_hgrn2_chunks is built for"""
+    per = 4 if rows[0].dtype == torch.float32 else 8
+    return seq.extend_seq_lens is not None and dim in (64, 128) and vdim in (64, 128) and all(
+        t.stride(0) % per == 0 and t.data_ptr() % 16 == 0 for t in rows)
+
+
+def _hgrn2_segment(tokens: int, requests: int, heads: int) -> int:
+    """as _scan_segment, with two workgroups per CU; us at one request of 4096 tokens, width 2048, by the segment's length:  none 1053
+    64: 174   80: 175   128: 198   256: 204   512: 285;  16 requests together  none 209   64: 193   80: 177   256: 206"""
+    if SCAN_SEGMENT is not None:
+        return SCAN_SEGMENT
+    room = 2 * (512 // heads) - requests
+    if room <= 0:
+        return 0
+    length = max(64, -(-2 * tokens // (16 * room)) * 16)
+    return length if 7 * length <= 2 * min(tokens, 2 * tokens // requests) else 0
+
+
 def hgrn2_scan(qpre: torch.Tensor, fpre: torch.Tensor, v: torch.Tensor, f_bias: torch.Tensor, lower: torch.Tensor,
                norm_w: torch.Tensor, state: torch.Tensor, seq: SeqParams, heads: int, dim: int, vdim: int, eps: float) -> torch.Tensor:
     """qpre, fpre [T, heads * dim], v [T, heads * vdim] (views) -> [T, heads * vdim]; state [slots, heads, dim, vdim] fp32"""
@@ -1851,6 +1887,16 @@ def hgrn2_scan(qpre: torch.Tensor, fpre: torch.Tensor, v: torch.Tensor, f_bias: 
             state.shape[1:] != (heads, dim, vdim):
         raise RuntimeError("hgrn2_scan: f_bias, lower [H*D], norm_w [vdim], state [slots, H, D, vdim]")
     out = empty_rows(T, heads * vdim, qpre.dtype, qpre.device)
+    if _hgrn2_chunks_take((qpre, fpre), seq, dim, vdim) and hgrn2_chunks_pay(T, seq.batch_size, heads):
+        lib, segment = load(), _hgrn2_segment(T, seq.batch_size, heads)
+        work = torch.empty(lib.sp_hgrn2_chunk_floats(T, seq.batch_size, heads, dim), dtype=torch.float32, device=qpre.device)
+        sums = torch.empty(lib.sp_hgrn2_segment_floats(T, seq.batch_size, heads, dim, vdim, segment), dtype=torch.float32,
+                           device=qpre.device) if segment else None
+        _check(lib.sp_hgrn2_chunks(out.data_ptr(), out.stride(0), qpre.data_ptr(), qpre.stride(0), fpre.data_ptr(), fpre.stride(0),
+                                   v.data_ptr(), v.stride(0), f_bias.data_ptr(), lower.data_ptr(), norm_w.data_ptr(), state.data_ptr(),
+                                   state.stride(0), work.data_ptr(), _ptr(sums), segment, T, heads, dim, vdim, eps, *seq.args,
+                                   _dt(qpre), _stream()), "sp_hgrn2_chunks")
+        return out
     _check(load().sp_hgrn2_scan(out.data_ptr(), out.stride(0), qpre.data_ptr(), qpre.stride(0), fpre.data_ptr(), fpre.stride(0),
                                 v.data_ptr(), v.stride(0), f_bias.data_ptr(), lower.data_ptr(), norm_w.data_ptr(),
                                 state.data_ptr(), state.stride(0), heads, dim, vdim, eps, *seq.args, _dt(qpre), _stream()),

@@ -1,0 +1,458 @@
+// Linear recurrences with a decay per key channel, 16 tokens at a time, fp32 on the matrix cores, their operands formed beforehand.
+//
+//   FORGET:  S_t = diag(w_t) S_{t-1} + k_t v_t^T                                            o_t = S_t^T r_t        (S [D, Dv])
+//   DELTA:   S_t = diag(w_t) S_{t-1} - b_t (u_t^T S_{t-1}) + k_t v_t^T                       o_t = S_t^T r_t        (b = a * u)
+//
+// Over a chunk that starts from S_0, with w_{i..j} the product of the decays of tokens i .. j per channel:
+//   Rd_t = r_t w_{1..t},   Ke_s = k_s w_{s+1..16},   P_ts = r_t . (k_s w_{s+1..t})  (s <= t),   G = w_{1..16}
+//   FORGET:  O = Rd S_0 + P V,            S_16 = diag(G) S_0 + Ke^T V
+//   DELTA:   Ud_t = u_t w_{1..t-1},  Be_s = b_s w_{s+1..16},  L_ts = u_t . (b_s w_{s+1..t-1}),  M_ts = u_t . (k_s w_{s+1..t-1})  (s < t),
+//            Q_ts = r_t . (b_s w_{s+1..t})  (s <= t):   Y = (I + L)^{-1} (Ud S_0 + M V)     (y_t = u_t^T S_{t-1})
+//            O = Rd S_0 + P V - Q Y,       S_16 = diag(G) S_0 + Ke^T V - Be^T Y
+// Every factor is a product of decays, never a quotient: with decays in [0, 1] nothing overflows however strong they are.
+//
+// chunk16_prepare_kernel forms all of this but the products with S_0, V and Y for all chunks at once (one workgroup per chunk and
+// head) and lays it out as the walk reads it from LDS.  chunk16_walk_kernel walks a request's chunks: a wave owns 16 columns of S in the
+// accumulator layout of v_mfma_f32_16x16x4_f32 (lane (r16, q): column r16, rows 16 i + 4 q + r), in which register (i, r) IS the second
+// operand of Rd S for the channels 16 i + 4 q + r, and the registers of v and Y are the second operands of the products over tokens.
+// Operands come into LDS by direct loads, one chunk ahead; one barrier per chunk.  The head's norm of a chunk follows behind the next
+// barrier (the waves' sums of squares have met there).
+//
+// A FORGET request's tokens may be cut into segments that run side by side (chunk_scan.h: the state is linear in the one a segment
+// starts from, here with a decay per row).
+//
+// A value that is not finite would reach the EARLIER tokens of its chunk (zeros of P and M times it): where a column has one, it is
+// taken out, the column's read-outs from that token on become NaN, and so does the column of the state.
+#pragma once
+#include "chunk_scan.h"
+
+namespace sp {
+
+constexpr int kC16 = 16;
+
+// floats of a chunk and head: KeT [D][16], G [D], Rd [16][D], P [16][16]; DELTA: BeT (negative) [D][16], Ud [16][D], T = (I + L)^{-1},
+// M and Q (negative), [16][16] each.  Pieces of 4 floats are permuted so that the 16 lanes of an LDS read phase meet no bank twice: in
+// rows of 16 by place16, in rows of D by XOR with the row's number.
+template <int D, bool DELTA>
+struct Chunk16 {
+  static constexpr int kKe = 0, kG = 16 * D, kSums = kG + D;               // what a segment's sums need comes first
+  static constexpr int kRd = kSums, kP = kRd + 16 * D, kBe = kP + 256, kUd = kBe + 16 * D, kT = kUd + 16 * D, kM = kT + 256, kQ = kM + 256;
+  static constexpr int kUsed = DELTA ? kQ + 256 : kBe;
+  static constexpr int kFloats = (kUsed + 255) / 256 * 256;                // whole direct loads of 1 KiB
+};
+// where piece q of row `row` lies, in rows of four pieces
+__device__ __forceinline__ int place16(int row, int q) { return ((q & 1) * 2 + (q >> 1)) ^ ((row >> 3) & 1); }
+
+__device__ __forceinline__ f32x4_c mfma_4(float a, float b, const f32x4_c& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// the sum over the lanes whose numbers differ in bits 3, 4 and 5
+__device__ __forceinline__ float sum_over_8s(float v) {
+  v += dpp_f32<0x128>(v);                             // row_ror 8
+  const auto r = __builtin_amdgcn_permlane16_swap(as_u32(v), as_u32(v), false, false);
+  v = as_f32(r[0]) + as_f32(r[1]);
+  const auto h = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);
+  return as_f32(h[0]) + as_f32(h[1]);
+}
+
+// Workgroup (chunk, head).  `fill` puts the chunk's rows of r, k, w (DELTA: u and b too) into LDS in fp32, rows past the request's end
+// as zeros with decay 1.  Vector work bounds it: a lane sums two columns s of the 16 x 16 matrices over D / 32 channels, the decays
+// between s and t building up as t walks on.
+template <int D, bool DELTA, typename Fill>
+__device__ __forceinline__ void chunk16_prepare(float* work, const Fill& fill) {
+  typedef Chunk16<D, DELTA> C;
+  constexpr int ROW = D + 4, CH = D / 32, NM = DELTA ? 4 : 1;             // matrices: P; L, M, Q
+  __shared__ __attribute__((aligned(16))) float sr[kC16][ROW], sk[kC16][ROW], sw[kC16][ROW];
+  __shared__ __attribute__((aligned(16))) float su[DELTA ? kC16 : 1][ROW], sb[DELTA ? kC16 : 1][ROW];
+  __shared__ float part[4][NM][kC16][kC16 + 1];
+  __shared__ float sL[DELTA ? kC16 : 1][kC16 + 1];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  fill(sr, sk, sw, su, sb);
+  __syncthreads();
+  const int s0 = lane & 7, c0 = wave * (D / 4) + (lane >> 3) * CH;
+  typedef float vec __attribute__((ext_vector_type(CH)));
+  vec rk[2], rb[2];
+#pragma unroll
+  for (int z = 0; z < 2; ++z) {
+    rk[z] = *(const vec*)&sk[s0 + 8 * z][c0];
+    if constexpr (DELTA) rb[z] = *(const vec*)&sb[s0 + 8 * z][c0];
+  }
+#pragma unroll
+  for (int t = 0; t < kC16; ++t) {
+    const vec rt = *(const vec*)&sr[t][c0], wt = *(const vec*)&sw[t][c0];
+    vec ut;
+    if constexpr (DELTA) ut = *(const vec*)&su[t][c0];
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+      const int s = s0 + 8 * z;
+      if (t < 8 * z) continue;                        // (t < s for every lane)
+      float sum[NM] = {};
+      if constexpr (DELTA) {
+#pragma unroll
+        for (int x = 0; x < CH; ++x) {
+          sum[1] += ut[x] * rb[z][x];
+          sum[2] += ut[x] * rk[z][x];
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < CH; ++x) {
+        rk[z][x] *= t > s ? wt[x] : 1.f;
+        sum[0] += rt[x] * rk[z][x];
+        if constexpr (DELTA) {
+          rb[z][x] *= t > s ? wt[x] : 1.f;
+          sum[3] += rt[x] * rb[z][x];
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        const float v = sum_over_8s(sum[m]);
+        if (lane < 8) part[wave][m][t][s] = v;
+      }
+    }
+  }
+  // Rd, Ud, G by one half of the threads, Ke and Be by the other: a channel's tokens forward or backward
+  for (int e = tid; e < 2 * D; e += 256) {
+    const int d = e < D ? e : e - D;
+    float g = 1.f;
+    if (e < D) {
+#pragma unroll
+      for (int t = 0; t < kC16; ++t) {
+        const int at = t * D + (((d >> 2) ^ t) << 2) + (d & 3);
+        if constexpr (DELTA) work[C::kUd + at] = su[t][d] * g;
+        g *= sw[t][d];
+        work[C::kRd + at] = sr[t][d] * g;
+      }
+      work[C::kG + d] = g;
+    } else {
+#pragma unroll
+      for (int p4 = 3; p4 >= 0; --p4) {
+        f32x4_c ke, be;
+#pragma unroll
+        for (int x = 3; x >= 0; --x) {
+          const int t = 4 * p4 + x;
+          ke[x] = sk[t][d] * g;
+          if constexpr (DELTA) be[x] = -(sb[t][d] * g);
+          g *= sw[t][d];
+        }
+        *(f32x4_c*)(work + C::kKe + d * 16 + place16(d, p4) * 4) = ke;
+        if constexpr (DELTA) *(f32x4_c*)(work + C::kBe + d * 16 + place16(d, p4) * 4) = be;
+      }
+    }
+  }
+  __syncthreads();
+  const int t = tid >> 4, s = tid & 15, at = t * 16 + place16(t, s >> 2) * 4 + (s & 3);
+  float sum[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) sum[m] = (part[0][m][t][s] + part[1][m][t][s]) + (part[2][m][t][s] + part[3][m][t][s]);
+  work[C::kP + at] = t >= s ? sum[0] : 0.f;
+  if constexpr (DELTA) {
+    work[C::kM + at] = t > s ? sum[2] : 0.f;
+    work[C::kQ + at] = t >= s ? -sum[3] : 0.f;
+    sL[t][s] = t > s ? sum[1] : 0.f;
+    __syncthreads();
+    if (tid < kC16) {                                 // column tid of (I + L)^{-1}: forward substitution
+      float x[kC16];
+#pragma unroll
+      for (int i = 0; i < kC16; ++i) {
+        float y = i == tid ? 1.f : 0.f;
+#pragma unroll
+        for (int j = 0; j < i; ++j) y -= sL[i][j] * x[j];
+        x[i] = i >= tid ? y : 0.f;
+        work[C::kT + i * 16 + place16(i, tid >> 2) * 4 + (tid & 3)] = x[i];
+      }
+    }
+  }
+}
+
+// 16 bytes per lane from `from` to lds + 16 lane.  (The builtin of the same makes every later read of LDS wait for it; the walk waits
+// once a chunk.)
+__device__ __forceinline__ void load_to_lds(const float* from, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds) : "memory");
+}
+
+// chunks of the requests before `b`, by all lanes of a wave
+__device__ __forceinline__ int chunks16_before(const SeqBatch& s, int b, int lane) {
+  int n = 0;
+  for (int i = lane; i < b; i += 64) n += segments_of(max(s.extend_seq_lens[i], 0), kC16);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+  return __builtin_amdgcn_readfirstlane(n);
+}
+
+struct Walk16 {
+  void* out;
+  const void *v, *gate;                               // gate: DELTA
+  const float *norm_w, *work;                         // norm_w [Dv] (DELTA: [H * Dv])
+  float* state;
+  int64_t out_stride, v_stride, gate_stride, state_stride;
+  ScanSegments seg;
+  int H;
+  float eps;
+};
+
+// Workgroup (request or segment, head) of NW waves.  Per chunk and wave, in matrix instructions of 32 cycles: FORGET 2 D / 4 + 4,
+// DELTA 4 D / 4 + 16.
+template <typename Tag, int D, int NW, bool DELTA, int MODE>
+__global__ void __launch_bounds__(NW * 64) chunk16_walk_kernel(Walk16 a, SeqBatch sb) {
+  typedef Elem<Tag> E;
+  typedef Chunk16<D, DELTA> C;
+  constexpr bool OUT = MODE != kSegmentSums;
+  constexpr int Dv = NW * 16, DT = D / 16, kUse = OUT ? C::kFloats : (C::kSums + 255) / 256 * 256, LOADS = kUse / 256;
+  __shared__ __attribute__((aligned(16))) float lds[2][kUse];
+  __shared__ float red[2][NW][kC16];
+  const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, q = lane >> 4, h = blockIdx.y;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int b = blockIdx.x, t0 = 0;
+  if constexpr (MODE != kWholeRequests)
+    if (!segment_at(sb, (int)blockIdx.x, a.seg.tokens, lane, b, t0)) return;
+  int len = __builtin_amdgcn_readfirstlane(sb.extend_seq_lens[b]);
+  if (len <= 0) return;
+  const bool split = MODE != kWholeRequests && len > a.seg.tokens, last = MODE == kWholeRequests || t0 + a.seg.tokens >= len;
+  if (MODE == kSegmentSums && last) return;
+  const bool held = OUT && (sb.extend_prefix_lens[b] > 0 || t0 > 0);
+  const float* work = a.work + (int64_t)(chunks16_before(sb, b, lane) + t0 / kC16) * a.H * C::kFloats + (int64_t)h * C::kFloats;
+  const int64_t start = __builtin_amdgcn_readfirstlane(sb.extend_start_loc[b]) + t0;
+  len -= t0;
+  if (MODE != kWholeRequests && len > a.seg.tokens) len = a.seg.tokens;
+  const int chunks = (len + kC16 - 1) / kC16, col = 16 * wave + r16;
+  float* st = a.state + load_idx(sb.req_pool_indices, b, sb.idx64) * a.state_stride + (int64_t)h * D * Dv;
+  float* const part = MODE == kWholeRequests ? nullptr : a.seg.work + ((int64_t)blockIdx.x * a.H + h) * a.seg.stride;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)&lds[0][0];
+  const auto fetch = [&](int c) {
+    const float* from = work + (int64_t)c * a.H * C::kFloats + lane * 4;
+    for (int u = wave; u < LOADS; u += NW) load_to_lds(from + u * 256, lds0 + (c & 1) * (kUse * 4) + u * 1024);
+  };
+  const int64_t vc = (int64_t)h * Dv + col;
+  typename E::storage vn[4], gn[4];                   // the next chunk's values as they lie in memory
+  const auto fetch_v = [&](int c) {
+    const int end = len - c * kC16 - 1;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t row = start + c * kC16 + min(4 * q + r, end);
+      vn[r] = ((const typename E::storage*)a.v)[row * a.v_stride + vc];
+      if constexpr (DELTA) gn[r] = ((const typename E::storage*)a.gate)[row * a.gate_stride + vc];
+    }
+  };
+  fetch(0);
+  fetch_v(0);
+  const float* from = split ? part : st;
+  f32x4_c S[DT], decay[MODE == kSegmentSums ? DT : 1];
+#pragma unroll
+  for (int i = 0; i < DT; ++i) {
+    if constexpr (MODE == kSegmentSums) decay[i] = f32x4_c{1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[i][r] = held ? from[(int64_t)(16 * i + 4 * q + r) * Dv + col] : 0.f;
+  }
+  const float nw = a.norm_w[DELTA ? (int64_t)h * Dv + col : col];
+  f32x4_c o = {0.f, 0.f, 0.f, 0.f};
+  float gate[4] = {1.f, 1.f, 1.f, 1.f};
+  // outputs of chunk c: `red` holds its waves' sums of squares
+  const auto finish = [&](int c) {
+    const int n = len - c * kC16;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float ss = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) ss += red[c & 1][w][4 * q + r];
+      const float y = o[r] * (1.f / sqrtf(ss / (float)Dv + a.eps)) * nw;
+      if (4 * q + r < n) E::store(a.out, (start + c * kC16 + 4 * q + r) * a.out_stride + vc, DELTA ? y / (1.f + expf(-gate[r])) : y);
+    }
+  };
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_barrier();
+  for (int c = 0; c < chunks; ++c) {
+    const int n = len - c * kC16;
+    const float* m = lds[c & 1];
+    float v[4], now[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      v[r] = 4 * q + r < n ? E::load(&vn[r], 0) : 0.f;
+      if constexpr (DELTA) now[r] = E::load(&gn[r], 0);
+    }
+    if (c + 1 < chunks) {
+      fetch(c + 1);
+      fetch_v(c + 1);
+    }
+    if (OUT && c > 0) finish(c - 1);
+    if constexpr (DELTA) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gate[r] = now[r];
+    }
+    const auto row16 = [&](int at) { return *(const f32x4_c*)(m + at + r16 * 16 + place16(r16, q) * 4); };
+    const auto row_d = [&](int at, int i) { return *(const f32x4_c*)(m + at + r16 * D + (((4 * i + q) ^ r16) << 2)); };
+    int first = kC16;                                 // the column's first token that is not finite
+    bool any = false;
+    f32x4_c y = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (OUT) {
+      const auto finite = [](float x) { return fabsf(x) < INFINITY; };
+      const auto rows_from = [&] {                    // `first` of the column, over the lanes that share it
+        first = min(first, __shfl_xor(first, 16, 64));
+        first = min(first, __shfl_xor(first, 32, 64));
+      };
+      const float probe = fmaf(v[0], 0.f, fmaf(v[1], 0.f, fmaf(v[2], 0.f, v[3] * 0.f)));
+      if (__ballot(probe != probe)) {
+        any = true;
+#pragma unroll
+        for (int r = 3; r >= 0; --r)
+          if (!finite(v[r])) v[r] = 0.f, first = 4 * q + r;
+        rows_from();
+      }
+      o = f32x4_c{0.f, 0.f, 0.f, 0.f};
+      f32x4_c x = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (DELTA) {
+        const f32x4_c mr = row16(C::kM);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x = mfma_4(mr[r], v[r], x);
+      }
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        const f32x4_c rd = row_d(C::kRd, i);
+        f32x4_c ud;
+        if constexpr (DELTA) ud = row_d(C::kUd, i);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if constexpr (DELTA) x = mfma_4(ud[r], S[i][r], x);
+          o = mfma_4(rd[r], S[i][r], o);
+        }
+      }
+      const f32x4_c pr = row16(C::kP);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o = mfma_4(pr[r], v[r], o);
+      if constexpr (DELTA) {
+        const f32x4_c tr = row16(C::kT), qr = row16(C::kQ);
+        const float odd = fmaf(x[0], 0.f, fmaf(x[1], 0.f, fmaf(x[2], 0.f, x[3] * 0.f)));
+        if (__ballot(odd != odd)) {
+          any = true;
+#pragma unroll
+          for (int r = 3; r >= 0; --r)
+            if (!finite(x[r])) x[r] = 0.f, first = min(first, 4 * q + r);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y = mfma_4(tr[r], x[r], y);
+        const float odd2 = fmaf(y[0], 0.f, fmaf(y[1], 0.f, fmaf(y[2], 0.f, y[3] * 0.f)));
+        if (any || __ballot(odd2 != odd2)) {
+          any = true;
+#pragma unroll
+          for (int r = 3; r >= 0; --r)
+            if (!finite(y[r])) first = min(first, 4 * q + r);
+          rows_from();
+#pragma unroll
+          for (int r = 0; r < 4; ++r) y[r] = 4 * q + r < first ? y[r] : 0.f;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o = mfma_4(qr[r], y[r], o);
+      }
+      if (any) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = 4 * q + r < first ? o[r] : as_f32(0x7fc00000u);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float ss = lanes_sum<16>(o[r] * o[r]);
+        if (r16 == 0) red[c & 1][wave][4 * q + r] = ss;
+      }
+    }
+    if (MODE != kSegmentOutputs || c + 1 < chunks || last) {
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        const f32x4_c g = *(const f32x4_c*)(m + C::kG + 16 * i + 4 * q);
+        const f32x4_c ke = *(const f32x4_c*)(m + C::kKe + (16 * i + r16) * 16 + place16(r16, q) * 4);
+        f32x4_c be;
+        if constexpr (DELTA) be = *(const f32x4_c*)(m + C::kBe + (16 * i + r16) * 16 + place16(r16, q) * 4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          S[i][r] *= g[r];
+          if constexpr (MODE == kSegmentSums) decay[i][r] *= g[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          S[i] = mfma_4(ke[r], v[r], S[i]);
+          if constexpr (DELTA) S[i] = mfma_4(be[r], y[r], S[i]);
+        }
+        if (OUT && any) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[i][r] = first < kC16 ? as_f32(0x7fc00000u) : S[i][r];
+        }
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+  }
+  if constexpr (OUT) finish(chunks - 1);
+  float* to = MODE == kSegmentSums ? part : st;
+  if (MODE == kSegmentSums || last) {
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) to[(int64_t)(16 * i + 4 * q + r) * Dv + col] = S[i][r];
+  }
+  if constexpr (MODE == kSegmentSums) {
+    if (wave == 0 && r16 == 0) {
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[D * Dv + 16 * i + 4 * q + r] = decay[i][r];
+    }
+  }
+}
+
+// Workgroup (request, head, 1024 values of S): segment_states_kernel with a decay per row
+template <int D, int Dv>
+__global__ void __launch_bounds__(256) segment_rows_kernel(ScanSegments g, const float* state, int64_t state_stride, SeqBatch s, int H) {
+  const int b = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
+  const int segments = segments_of(s.extend_seq_lens[b], g.tokens);
+  if (segments <= 1) return;
+  int before = 0;
+  for (int i = lane; i < b; i += 64) before += segments_of(max(s.extend_seq_lens[i], 0), g.tokens);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
+  const int e = (blockIdx.z * 256 + threadIdx.x) * 4;
+  float* const first = g.work + ((int64_t)before * H + h) * g.stride;
+  const int64_t step = H * g.stride;
+  f32x4_c S = {0.f, 0.f, 0.f, 0.f};
+  if (s.extend_prefix_lens[b] > 0) {
+    const float* from = state + load_idx(s.req_pool_indices, b, s.idx64) * state_stride + (int64_t)h * D * Dv + e;
+    S = f32x4_c{from[0], from[1], from[2], from[3]};
+  }
+  constexpr int AHEAD = 8;
+  for (int i0 = 0; i0 < segments; i0 += AHEAD) {
+    f32x4_c sum[AHEAD];
+    float decay[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const float* at = first + min(i0 + u, segments - 2) * step;      // (the last segment has no sums)
+      sum[u] = *(const f32x4_c*)(at + e);
+      decay[u] = at[D * Dv + e / Dv];
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      if (i0 + u >= segments) break;
+      *(f32x4_c*)(first + (i0 + u) * step + e) = S;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[r] = decay[u] * S[r] + sum[u][r];
+    }
+  }
+}
+
+template <typename Tag, int D, int NW, bool DELTA>
+int launch_walk16(const Walk16& a, int64_t tokens, const SeqBatch& s, hipStream_t st) {
+  if (a.seg.tokens == 0) {
+    chunk16_walk_kernel<Tag, D, NW, DELTA, kWholeRequests><<<dim3((unsigned)s.B, (unsigned)a.H), NW * 64, 0, st>>>(a, s);
+    SP_LAUNCH_CHECK();
+    return SP_OK;
+  }
+  if constexpr (!DELTA) {
+    const dim3 grid((unsigned)(tokens / a.seg.tokens + s.B), (unsigned)a.H);
+    chunk16_walk_kernel<Tag, D, NW, DELTA, kSegmentSums><<<grid, NW * 64, 0, st>>>(a, s);
+    SP_LAUNCH_CHECK();
+    segment_rows_kernel<D, NW * 16><<<dim3((unsigned)s.B, (unsigned)a.H, D * NW * 16 / 1024), 256, 0, st>>>(a.seg, a.state, a.state_stride, s, a.H);
+    SP_LAUNCH_CHECK();
+    chunk16_walk_kernel<Tag, D, NW, DELTA, kSegmentOutputs><<<grid, NW * 64, 0, st>>>(a, s);
+    SP_LAUNCH_CHECK();
+    return SP_OK;
+  }
+  return SP_ERR_UNSUPPORTED;
+}
+
+inline int64_t chunk16_units(int64_t tokens, int B) { return tokens / kC16 + B; }      // at most: a request's last chunk may be partial
+
+}  // namespace sp

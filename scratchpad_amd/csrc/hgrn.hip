@@ -8,7 +8,7 @@
 // One workgroup per (request, head): a column of S (one value channel) lives in the registers of 1 to 8 neighbouring
 // lanes; the request's tokens of this step are walked in order from the state the previous step left in the pool (zeros at
 // a sequence's first token), staged through LDS in passes of 16 tokens, the head norm as the pass's epilogue.
-#include "seq_batch.h"
+#include "chunk16.h"
 
 namespace sp {
 namespace {
@@ -185,6 +185,50 @@ static int launch_hgrn2(void* out, int64_t out_stride, const void* qpre, int64_t
   return SP_OK;
 }
 
+// ---- steps of several tokens per request, 16 tokens at a time on the matrix cores (chunk16.h: w = f, k = 1 - f, r = q) ---------------
+// The per-token form above is a chain of one token's LDS reads and sums with as many workgroups as requests x heads.  Width 2048 (8 heads of
+// 128 x 128), us per layer: one request
+// of 4096 tokens 2633 -> 175 (prepare 32, segments' sums 22, states 12, outputs 42, library products 68), 16 requests of 4096 tokens together
+// 361 -> 177.  The rule for taking it and both sides' times are in _native.py (hgrn2_chunks_pay).
+template <typename Tag, int D>
+__global__ void __launch_bounds__(256)
+hgrn2_prepare_kernel(float* work, const char* qpre, int64_t q_stride, const char* fpre, int64_t f_stride, const float* f_bias,
+                     const float* lower, SeqBatch s, int H) {
+  typedef Elem<Tag> E;
+  constexpr int V = E::kVec, QP = D / V;
+  const int h = blockIdx.y;
+  int b, t0;
+  if (!segment_at(s, (int)blockIdx.x, kC16, threadIdx.x & 63, b, t0)) return;
+  const int64_t row0 = (int64_t)s.extend_start_loc[b] + t0;
+  const int n = s.extend_seq_lens[b] - t0;
+  chunk16_prepare<D, false>(work + ((int64_t)blockIdx.x * H + h) * Chunk16<D, false>::kFloats,
+                            [&](auto& sr, auto& sk, auto& sw, auto&, auto&) {
+    for (int e = threadIdx.x; e < kC16 * QP; e += 256) {
+      const int t = e / QP, i = e % QP * V, c = h * D + i;
+      float q[V], f[V];
+      const u32x4 zero = {0u, 0u, 0u, 0u};
+      unpack16<Tag>(t < n ? ld16(qpre + ((row0 + t) * q_stride + c) * E::kBytes) : zero, q);
+      unpack16<Tag>(t < n ? ld16(fpre + ((row0 + t) * f_stride + c) * E::kBytes) : zero, f);
+#pragma unroll
+      for (int x = 0; x < V; ++x) {
+        const float lo = lower[c + x], w = t < n ? lo + (1.f - lo) / (1.f + expf(-(f[x] + f_bias[c + x]))) : 1.f;
+        sr[t][i + x] = q[x] / (1.f + expf(-q[x]));
+        sw[t][i + x] = w;
+        sk[t][i + x] = 1.f - w;
+      }
+    }
+  });
+}
+
+template <typename Tag, int D, int NW>
+static int launch_hgrn2_chunks(const Walk16& w, float* work, const void* qpre, int64_t q_stride, const void* fpre, int64_t f_stride,
+                               const float* f_bias, const float* lower, int64_t tokens, const SeqBatch& s, hipStream_t st) {
+  hgrn2_prepare_kernel<Tag, D><<<dim3((unsigned)chunk16_units(tokens, s.B), (unsigned)w.H), 256, 0, st>>>(
+      work, (const char*)qpre, q_stride, (const char*)fpre, f_stride, f_bias, lower, s, w.H);
+  SP_LAUNCH_CHECK();
+  return launch_walk16<Tag, D, NW, false>(w, tokens, s, st);
+}
+
 }  // namespace
 }  // namespace sp
 
@@ -204,4 +248,40 @@ extern "C" int sp_hgrn2_scan(void* out, int64_t out_stride, const void* qpre, in
   SP_DISPATCH_DTYPE(dtype, return (launch_hgrn2<Tag>(out, out_stride, qpre, q_stride, fpre, f_stride, v, v_stride, f_bias, lower,
                                                      norm_w, state, state_stride, s, heads, dim, vdim, eps,
                                                      (hipStream_t)stream)));
+}
+
+extern "C" int64_t sp_hgrn2_chunk_floats(int64_t num_tokens, int batch_size, int heads, int dim) {
+  return chunk16_units(num_tokens, batch_size) * heads * (dim == 64 ? Chunk16<64, false>::kFloats : Chunk16<128, false>::kFloats);
+}
+
+extern "C" int64_t sp_hgrn2_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim, int segment_tokens) {
+  return (num_tokens / segment_tokens + batch_size) * heads * ((int64_t)dim * vdim + dim);
+}
+
+extern "C" int sp_hgrn2_chunks(void* out, int64_t out_stride, const void* qpre, int64_t q_stride, const void* fpre, int64_t f_stride,
+                               const void* v, int64_t v_stride, const float* f_bias, const float* lower, const float* norm_w, float* state,
+                               int64_t state_stride, float* work, float* segment_work, int segment_tokens, int64_t num_tokens, int heads,
+                               int dim, int vdim, float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
+  SP_CHECK_ARG(batch_size >= 0 && num_tokens >= 0 && heads > 0 && dim > 0 && vdim > 0);
+  if (batch_size == 0 || num_tokens == 0) return SP_OK;
+  SP_CHECK_ARG(out && qpre && fpre && v && f_bias && lower && norm_w && state && work && req_pool_indices && seq_lens);
+  SP_CHECK_ARG(!extend_seq_lens || (extend_prefix_lens && extend_start_loc));
+  SP_CHECK_ARG(segment_tokens >= 0 && segment_tokens % kC16 == 0 && (segment_tokens == 0 || segment_work));
+  const int64_t nk = (int64_t)heads * dim, nv = (int64_t)heads * vdim;
+  SP_CHECK_ARG(q_stride >= nk && f_stride >= nk && v_stride >= nv && out_stride >= nv && state_stride >= nk * vdim);
+  SEQ_BATCH(s);
+  const int per = dtype == SP_F32 ? 4 : 8;
+  if (!extend_seq_lens || (dim != 64 && dim != 128) || (vdim != 64 && vdim != 128) || q_stride % per || f_stride % per || heads > 65535 ||
+      (((uintptr_t)qpre | (uintptr_t)fpre | (uintptr_t)work | (uintptr_t)segment_work) & 15) || chunk16_units(num_tokens, batch_size) >> 31)
+    return SP_ERR_UNSUPPORTED;
+  const Walk16 w{out, v, nullptr, norm_w, work, state, out_stride, v_stride, 0, state_stride,
+                 ScanSegments{segment_work, (int64_t)dim * vdim + dim, segment_tokens}, heads, eps};
+#define SP_HGRN_CHUNKS(D, NW)                                                                                                     \
+  SP_DISPATCH_DTYPE(dtype, return (launch_hgrn2_chunks<Tag, D, NW>(w, work, qpre, q_stride, fpre, f_stride, f_bias, lower, num_tokens, s, \
+                                                                   (hipStream_t)stream)))
+  if (dim == 128 && vdim == 128) SP_HGRN_CHUNKS(128, 8);
+  if (dim == 128) SP_HGRN_CHUNKS(128, 4);
+  if (vdim == 128) SP_HGRN_CHUNKS(64, 8);
+  SP_HGRN_CHUNKS(64, 4);
+#undef SP_HGRN_CHUNKS
 }

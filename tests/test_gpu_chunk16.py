@@ -1,0 +1,91 @@
+"""The recurrences that run 16 tokens at a time with their operands formed beforehand: requests whose lengths lie around the chunk's and the
+segment's edges, from an empty and from a held state, against the token-by-token recurrence in 64 bits.  Everything is fp32 in both: the
+states differ by accumulated fp32 roundings - the sums over 16 tokens and D channels and a product of decays per chunk - 2e-5 of the largest
+value being ten times that; outputs by that and one rounding of their type, amplified by the head's norm where a row nearly cancels."""
+import pytest
+import torch
+
+from tests.test_gpu_toredra_kernels import DEV, announce, seq_extend
+
+pytestmark = pytest.mark.gpu
+LENS = [[1], [15, 16, 17], [48, 1, 33, 2], [16, 200, 3], [40] + [2] * 66 + [20]]
+HALF = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}
+
+
+def near(got, want, bar=2e-5):
+    assert torch.isfinite(got).all()
+    err = (got.double() - want).abs().max() / want.abs().max()
+    assert err <= bar, f"{err:.2e} > {bar:.0e}"
+
+
+def rms(x, eps=1e-5):
+    return x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps)
+
+
+def hgrn2_reference(q, f, v, fb, lower, S, H):
+    T, D, Dv = q.shape[0], q.shape[1] // H, v.shape[1] // H
+    q, f, v, lo = q.double(), f.double(), v.double().view(T, H, Dv), lower.double()
+    q, w = (q * torch.sigmoid(q)).view(T, H, D), (lo + (1 - lo) * torch.sigmoid(f + fb.double())).view(T, H, D)
+    o = torch.empty(T, H, Dv, dtype=torch.float64, device=DEV)
+    for t in range(T):
+        S = w[t][:, :, None] * S + (1 - w[t])[:, :, None] * v[t][:, None]
+        o[t] = (S * q[t][:, :, None]).sum(1)
+    return rms(o), S
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("segment", [0, 16, 64])
+@pytest.mark.parametrize("lens", LENS, ids=lambda l: "-".join(map(str, l[:5])))
+@pytest.mark.parametrize("H,D,Dv", [(2, 128, 128), (3, 64, 64), (1, 128, 64), (2, 64, 128)])
+def test_hgrn2_chunks(lens, H, D, Dv, segment, dtype, monkeypatch):
+    from scratchpad_amd import _native
+    announce("hgrn2 chunks", dtype, lens, H, D, Dv, segment)
+    monkeypatch.setattr(_native, "SCAN_SEGMENT", segment)
+    monkeypatch.setattr(_native, "HGRN2_CHUNKS", True)
+    g = torch.Generator(device=DEV).manual_seed(7)
+    T, slots = sum(lens), [2 * i + 1 for i in range(len(lens))]
+    S = torch.full((2 * len(lens) + 1, H, D, Dv), float("nan"), device=DEV)
+    fb, lower, nw = torch.randn(H * D, generator=g, device=DEV), torch.rand(H * D, generator=g, device=DEV) * 0.5, torch.rand(Dv, generator=g, device=DEV) + 0.5
+    ref = [torch.zeros(H, D, Dv, dtype=torch.float64, device=DEV) for _ in lens]
+    for prefixes in ([0] * len(lens), lens):                     # the second launch goes on from what the first one left
+        a = (torch.randn(T, 2 * H * D + H * Dv, generator=g, device=DEV) * 2).to(dtype)
+        q, f, v = a.split([H * D, H * D, H * Dv], 1)
+        out = _native.hgrn2_scan(q, f, v, fb, lower, nw, S, seq_extend(lens, prefixes, slots), H, D, Dv, 1e-5).view(T, H, Dv)
+        at = 0
+        for i, n in enumerate(lens):
+            want, ref[i] = hgrn2_reference(q[at:at + n], f[at:at + n], v[at:at + n], fb, lower, ref[i], H)
+            near(S[slots[i]], ref[i])
+            want = want * nw.double()
+            assert ((out[at:at + n].double() - want).abs() <= HALF[dtype] * want.abs() + 1e-3).all()
+            at += n
+    assert torch.isnan(S[::2]).all()                             # no other slot was touched
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["query", "forget", "value"])
+@pytest.mark.parametrize("at", [0, 5, 15, 16, 50])
+def test_hgrn2_numbers_that_are_not_finite_reach_no_earlier_token(at, where, bad, monkeypatch):
+    from scratchpad_amd import _native
+    monkeypatch.setattr(_native, "SCAN_SEGMENT", 32)
+    monkeypatch.setattr(_native, "HGRN2_CHUNKS", True)
+    H, D, T = 2, 64, 70
+    g = torch.Generator(device=DEV).manual_seed(8)
+    a = torch.randn(T, 3 * H * D, generator=g, device=DEV).bfloat16()
+    zero, one = torch.zeros(H * D, device=DEV), torch.ones(D, device=DEV)
+
+    def run(a):
+        S = torch.zeros(2, H, D, D, device=DEV)
+        out = _native.hgrn2_scan(*a.split(H * D, 1), zero, zero, one, S, seq_extend([T], [0], [1]), H, D, D, 1e-5)
+        return out.view(T, H, D), S[1]
+    clean = run(a)
+    b = a.clone()
+    b[at, {"query": 0, "forget": H * D, "value": 2 * H * D}[where] + 3] = bad
+    out, S = run(b)
+    assert torch.equal(out[:at], clean[0][:at]) and torch.equal(out[:, 1], clean[0][:, 1]) and torch.equal(S[1], clean[1][1])
+    if where == "query":
+        assert not torch.isfinite(out[at, 0].float()).any() or bad == float("inf")
+        assert torch.equal(S, clean[1]) and torch.equal(out[at + 1:], clean[0][at + 1:])
+    elif where == "value":
+        assert not torch.isfinite(out[at:, 0, 3].float()).any() and not torch.isfinite(S[0, :, 3]).any()
+    elif bad != float("inf"):                                    # (an infinite pre-activation is an open gate)
+        assert not torch.isfinite(out[at:, 0].float()).any() and not torch.isfinite(S[0, 3]).any()
