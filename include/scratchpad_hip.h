@@ -686,6 +686,14 @@ SP_API int sp_delta_recurrence(void* out, int64_t out_stride, const void* r, int
                                const float* decay, const float* remove, const float* norm_w, float* state,
                                int64_t state_stride, int heads, int head_dim, float eps, SP_SEQ_PARAMS, int dtype,
                                void* stream);
+/* The same for steps of several tokens per request, 16 tokens at a time on the matrix cores (fp32 throughout): head_dim 64, rows of r, k,
+ * v and g 16-byte aligned; else SP_ERR_UNSUPPORTED and nothing is launched.  Products of up to 16 decays are formed (never quotients):
+ * those in [0, 1] cannot overflow.  work: fp32, sp_delta_recurrence_chunk_floats values, 16-byte aligned.                      */
+SP_API int64_t sp_delta_recurrence_chunk_floats(int64_t num_tokens, int batch_size, int heads, int head_dim);
+SP_API int sp_delta_recurrence_chunks(void* out, int64_t out_stride, const void* r, int64_t r_stride, const void* k, int64_t k_stride,
+                                      const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* decay,
+                                      const float* remove, const float* norm_w, float* state, int64_t state_stride, float* work,
+                                      int64_t num_tokens, int heads, int head_dim, float eps, SP_SEQ_PARAMS, int dtype, void* stream);
 /* sp_delta_gates and sp_delta_recurrence of a decode step (one token per request) as one launch: head_dim 64 or 128, rank <= 512,
  * else SP_ERR_UNSUPPORTED and nothing is launched. */
 SP_API int sp_delta_step(void* out, int64_t out_stride, const void* r, int64_t r_stride, const void* k, int64_t k_stride,
@@ -701,7 +709,7 @@ SP_API int sp_hgrn2_scan(void* out, int64_t out_stride, const void* qpre, int64_
                          const float* norm_w, float* state, int64_t state_stride, int heads, int dim, int vdim, float eps,
                          SP_SEQ_PARAMS, int dtype, void* stream);
 /* The same for steps of several tokens per request, 16 tokens at a time on the matrix cores (fp32 throughout): dim and vdim 64 or 128,
- * rows of qpre and fpre 16-byte aligned; else SP_ERR_UNSUPPORTED and nothing is launched.  Products of up to 16 gates are formed (never
+ * rows of qpre, fpre and v 16-byte aligned; else SP_ERR_UNSUPPORTED and nothing is launched.  Products of up to 16 gates are formed (never
  * quotients).  work: fp32, sp_hgrn2_chunk_floats values, 16-byte aligned.  segment_tokens > 0 (a multiple of 16): a request's tokens are
  * shared out in segments that run side by side, segment_work (fp32, 16-byte aligned) holds sp_hgrn2_segment_floats values.          */
 SP_API int64_t sp_hgrn2_chunk_floats(int64_t num_tokens, int batch_size, int heads, int dim);

@@ -166,6 +166,9 @@ SIGNATURES = {
     "sp_delta_gates": (_i32, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i32, _i32, _f32, _i32, _vp]),
     "sp_delta_recurrence": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i32, _i32,
                                    _f32, *_SEQ, _i32, _vp]),
+    "sp_delta_recurrence_chunk_floats": (_i64, [_i64, _i32, _i32, _i32]),
+    "sp_delta_recurrence_chunks": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i32,
+                                          _i32, _f32, *_SEQ, _i32, _vp]),
     "sp_delta_step": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i32, _f32,
                              _vp, _vp, _i64, _i32, _i32, _f32, *_SEQ, _i32, _vp]),
     "sp_hgrn2_chunk_floats": (_i64, [_i64, _i32, _i32, _i32]),
@@ -1800,6 +1803,18 @@ def delta_gates(p: torch.Tensor, w2t: torch.Tensor, w0: torch.Tensor, apre: torc
     return decay, remove
 
 
+DELTA_RECURRENCE_CHUNKS = None      # tests and measurements, as HGRN2_CHUNKS
+
+
+def delta_recurrence_chunks_pay(tokens: int, requests: int, heads: int) -> bool:
+    """As hgrn2_chunks_pay.  us per layer of width 2048 (32 heads of 64; requests x tokens together), per token / in chunks:  1 x 65: 96 / 101
+    1 x 300: 191 / 108   2 x 500: 272 / 142   16 x 512: 104 / 100   1 x 4096: 2309 / 1010   4 x 4096: 835 / 531   16 x 4096: 558 / 497
+    64 x 1024: 168 / 167   64 x 512: 101 / 113   256 x 4096: 542 / 624"""
+    if DELTA_RECURRENCE_CHUNKS is not None:
+        return DELTA_RECURRENCE_CHUNKS
+    return min(tokens, 2 * tokens // requests) >= 72
+
+
 def delta_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, decay: torch.Tensor,
                      remove: torch.Tensor, norm_w: torch.Tensor, state: torch.Tensor, seq: SeqParams, heads: int, dim: int,
                      eps: float) -> torch.Tensor:
@@ -1812,6 +1827,16 @@ def delta_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch
     if decay.shape != (T, n) or remove.shape != (T, n) or norm_w.numel() != n or state.shape[1:] != (heads, dim, dim):
         raise RuntimeError("delta_recurrence: decay, remove [T, H*D], norm_w [H*D], state [slots, H, D, D]")
     out = empty_rows(T, n, r.dtype, r.device)
+    per = 4 if r.dtype == torch.float32 else 8
+    if seq.extend_seq_lens is not None and dim == 64 and delta_recurrence_chunks_pay(T, seq.batch_size, heads) and \
+            all(t.stride(0) % per == 0 and t.data_ptr() % 16 == 0 for t in (r, k, v, g)) and decay.data_ptr() % 16 == 0 and remove.data_ptr() % 16 == 0:
+        work = torch.empty(load().sp_delta_recurrence_chunk_floats(T, seq.batch_size, heads, dim), dtype=torch.float32, device=r.device)
+        _check(load().sp_delta_recurrence_chunks(out.data_ptr(), out.stride(0), r.data_ptr(), r.stride(0), k.data_ptr(), k.stride(0),
+                                                 v.data_ptr(), v.stride(0), g.data_ptr(), g.stride(0), decay.data_ptr(),
+                                                 remove.data_ptr(), norm_w.data_ptr(), state.data_ptr(), state.stride(0),
+                                                 work.data_ptr(), T, heads, dim, eps, *seq.args, _dt(r), _stream()),
+               "sp_delta_recurrence_chunks")
+        return out
     _check(load().sp_delta_recurrence(out.data_ptr(), out.stride(0), r.data_ptr(), r.stride(0), k.data_ptr(), k.stride(0),
                                       v.data_ptr(), v.stride(0), g.data_ptr(), g.stride(0), decay.data_ptr(), remove.data_ptr(),
                                       norm_w.data_ptr(), state.data_ptr(), state.stride(0), heads, dim, eps, *seq.args,
@@ -1887,7 +1912,7 @@ def hgrn2_scan(qpre: torch.Tensor, fpre: torch.Tensor, v: torch.Tensor, f_bias: 
             state.shape[1:] != (heads, dim, vdim):
         raise RuntimeError("hgrn2_scan: f_bias, lower [H*D], norm_w [vdim], state [slots, H, D, vdim]")
     out = empty_rows(T, heads * vdim, qpre.dtype, qpre.device)
-    if _hgrn2_chunks_take((qpre, fpre), seq, dim, vdim) and hgrn2_chunks_pay(T, seq.batch_size, heads):
+    if _hgrn2_chunks_take((qpre, fpre, v), seq, dim, vdim) and hgrn2_chunks_pay(T, seq.batch_size, heads):
         lib, segment = load(), _hgrn2_segment(T, seq.batch_size, heads)
         work = torch.empty(lib.sp_hgrn2_chunk_floats(T, seq.batch_size, heads, dim), dtype=torch.float32, device=qpre.device)
         sums = torch.empty(lib.sp_hgrn2_segment_floats(T, seq.batch_size, heads, dim, vdim, segment), dtype=torch.float32,

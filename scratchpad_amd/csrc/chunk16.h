@@ -15,8 +15,8 @@
 // head) and lays it out as the walk reads it from LDS.  chunk16_walk_kernel walks a request's chunks: a wave owns 16 columns of S in the
 // accumulator layout of v_mfma_f32_16x16x4_f32 (lane (r16, q): column r16, rows 16 i + 4 q + r), in which register (i, r) IS the second
 // operand of Rd S for the channels 16 i + 4 q + r, and the registers of v and Y are the second operands of the products over tokens.
-// Operands come into LDS by direct loads, one chunk ahead; one barrier per chunk.  The head's norm of a chunk follows behind the next
-// barrier (the waves' sums of squares have met there).
+// Operands and rows come into LDS by direct loads, two chunks ahead; one barrier per chunk.  Read-outs go
+// through LDS to the waves that norm, gate and store them, a chunk behind.
 //
 // A FORGET request's tokens may be cut into segments that run side by side (chunk_scan.h: the state is linear in the one a segment
 // starts from, here with a decay per row).
@@ -40,19 +40,18 @@ struct Chunk16 {
   static constexpr int kUsed = DELTA ? kQ + 256 : kBe;
   static constexpr int kFloats = (kUsed + 255) / 256 * 256;                // whole direct loads of 1 KiB
 };
+// the walk's LDS: three chunks' operands, rows of v (and of the gate), then two chunks' read-outs in fp32 (rows of Dv + 4: the four rows that
+// a wave writes at a time lie in different banks)
+template <typename Tag, int D, int NW, bool DELTA, int MODE>
+struct Walk16Lds {
+  static constexpr int kOps = (MODE != kSegmentSums ? Chunk16<D, DELTA>::kFloats : (Chunk16<D, DELTA>::kSums + 255) / 256 * 256) * 4;
+  static constexpr int kRows = kC16 * NW * 16 * Elem<Tag>::kBytes, kBuf = kOps + (DELTA ? 2 : 1) * kRows, kRow = NW * 16 + 4;
+  static constexpr int kOut = 3 * kBuf, kBytes = kOut + (MODE != kSegmentSums ? 2 * kC16 * kRow * 4 : 0);
+};
 // where piece q of row `row` lies, in rows of four pieces
 __device__ __forceinline__ int place16(int row, int q) { return ((q & 1) * 2 + (q >> 1)) ^ ((row >> 3) & 1); }
 
 __device__ __forceinline__ f32x4_c mfma_4(float a, float b, const f32x4_c& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
-// the sum over the lanes whose numbers differ in bits 3, 4 and 5
-__device__ __forceinline__ float sum_over_8s(float v) {
-  v += dpp_f32<0x128>(v);                             // row_ror 8
-  const auto r = __builtin_amdgcn_permlane16_swap(as_u32(v), as_u32(v), false, false);
-  v = as_f32(r[0]) + as_f32(r[1]);
-  const auto h = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);
-  return as_f32(h[0]) + as_f32(h[1]);
-}
 
 // Workgroup (chunk, head).  `fill` puts the chunk's rows of r, k, w (DELTA: u and b too) into LDS in fp32, rows past the request's end
 // as zeros with decay 1.  Vector work bounds it: a lane sums two columns s of the 16 x 16 matrices over D / 32 channels, the decays
@@ -77,37 +76,41 @@ __device__ __forceinline__ void chunk16_prepare(float* work, const Fill& fill) {
     if constexpr (DELTA) rb[z] = *(const vec*)&sb[s0 + 8 * z][c0];
   }
 #pragma unroll
-  for (int t = 0; t < kC16; ++t) {
-    const vec rt = *(const vec*)&sr[t][c0], wt = *(const vec*)&sw[t][c0];
-    vec ut;
-    if constexpr (DELTA) ut = *(const vec*)&su[t][c0];
+  for (int half = 0; half < 2; ++half) {
+    float sums[NM][2][8];                             // of tokens t = 8 half + u and columns s0 + 8 z
 #pragma unroll
-    for (int z = 0; z < 2; ++z) {
-      const int s = s0 + 8 * z;
-      if (t < 8 * z) continue;                        // (t < s for every lane)
-      float sum[NM] = {};
-      if constexpr (DELTA) {
+    for (int u = 0; u < 8; ++u) {
+      const int t = 8 * half + u;
+      const vec rt = *(const vec*)&sr[t][c0], wt = *(const vec*)&sw[t][c0];
+      vec ut;
+      if constexpr (DELTA) ut = *(const vec*)&su[t][c0];
+#pragma unroll
+      for (int z = 0; z <= half; ++z) {               // (tokens below 8 are before every second column)
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (DELTA) {
+#pragma unroll
+          for (int x = 0; x < CH; ++x) {
+            sum[1] += ut[x] * rb[z][x];
+            sum[2] += ut[x] * rk[z][x];
+          }
+        }
 #pragma unroll
         for (int x = 0; x < CH; ++x) {
-          sum[1] += ut[x] * rb[z][x];
-          sum[2] += ut[x] * rk[z][x];
+          rk[z][x] *= t > s0 + 8 * z ? wt[x] : 1.f;
+          sum[0] += rt[x] * rk[z][x];
+          if constexpr (DELTA) {
+            rb[z][x] *= t > s0 + 8 * z ? wt[x] : 1.f;
+            sum[3] += rt[x] * rb[z][x];
+          }
         }
-      }
 #pragma unroll
-      for (int x = 0; x < CH; ++x) {
-        rk[z][x] *= t > s ? wt[x] : 1.f;
-        sum[0] += rt[x] * rk[z][x];
-        if constexpr (DELTA) {
-          rb[z][x] *= t > s ? wt[x] : 1.f;
-          sum[3] += rt[x] * rb[z][x];
-        }
-      }
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        const float v = sum_over_8s(sum[m]);
-        if (lane < 8) part[wave][m][t][s] = v;
+        for (int m = 0; m < NM; ++m) sums[m][z][u] = sum[m];
       }
     }
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+      for (int z = 0; z <= half; ++z) part[wave][m][8 * half + (lane >> 3)][s0 + 8 * z] = eight_sums(sums[m][z], lane);
   }
   // Rd, Ud, G by one half of the threads, Ke and Be by the other: a channel's tokens forward or backward
   for (int e = tid; e < 2 * D; e += 256) {
@@ -165,7 +168,7 @@ __device__ __forceinline__ void chunk16_prepare(float* work, const Fill& fill) {
 
 // 16 bytes per lane from `from` to lds + 16 lane.  (The builtin of the same makes every later read of LDS wait for it; the walk waits
 // once a chunk.)
-__device__ __forceinline__ void load_to_lds(const float* from, uint32_t lds) {
+__device__ __forceinline__ void load_to_lds(const void* from, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds) : "memory");
 }
 
@@ -187,18 +190,21 @@ struct Walk16 {
   ScanSegments seg;
   int H;
   float eps;
+  int vec_out;                                        // rows of `out` take 16-byte stores (fp32: two of them per 8 values)
 };
 
-// Workgroup (request or segment, head) of NW waves.  Per chunk and wave, in matrix instructions of 32 cycles: FORGET 2 D / 4 + 4,
-// DELTA 4 D / 4 + 16.
+// Workgroup (request or segment, head): NW waves own 16 columns each, NW / 2 more fetch the operands of the chunk after the next and finish
+// the one before - the head's norm, the gate, the stores.  What bounds it is the chain of a wave's matrix instructions of 32 cycles, 2 D / 4 + 4
+// per chunk (DELTA: 4 D / 4 + 16): with waves that also finished their own columns a chunk
+// of a single request (DELTA, heads of 64) took 3.2 us, now 2.4.
 template <typename Tag, int D, int NW, bool DELTA, int MODE>
-__global__ void __launch_bounds__(NW * 64) chunk16_walk_kernel(Walk16 a, SeqBatch sb) {
+__global__ void __launch_bounds__(NW * 96) chunk16_walk_kernel(Walk16 a, SeqBatch sb) {
   typedef Elem<Tag> E;
   typedef Chunk16<D, DELTA> C;
+  typedef Walk16Lds<Tag, D, NW, DELTA, MODE> L;
   constexpr bool OUT = MODE != kSegmentSums;
-  constexpr int Dv = NW * 16, DT = D / 16, kUse = OUT ? C::kFloats : (C::kSums + 255) / 256 * 256, LOADS = kUse / 256;
-  __shared__ __attribute__((aligned(16))) float lds[2][kUse];
-  __shared__ float red[2][NW][kC16];
+  constexpr int Dv = NW * 16, DT = D / 16, NH = NW / 2, OPS = L::kOps / 1024, ROWS = L::kRows / 1024;
+  extern __shared__ __attribute__((aligned(16))) char walk_lds[];
   const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, q = lane >> 4, h = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int b = blockIdx.x, t0 = 0;
@@ -209,31 +215,93 @@ __global__ void __launch_bounds__(NW * 64) chunk16_walk_kernel(Walk16 a, SeqBatc
   const bool split = MODE != kWholeRequests && len > a.seg.tokens, last = MODE == kWholeRequests || t0 + a.seg.tokens >= len;
   if (MODE == kSegmentSums && last) return;
   const bool held = OUT && (sb.extend_prefix_lens[b] > 0 || t0 > 0);
-  const float* work = a.work + (int64_t)(chunks16_before(sb, b, lane) + t0 / kC16) * a.H * C::kFloats + (int64_t)h * C::kFloats;
   const int64_t start = __builtin_amdgcn_readfirstlane(sb.extend_start_loc[b]) + t0;
+  const int whole = len;
   len -= t0;
-  if (MODE != kWholeRequests && len > a.seg.tokens) len = a.seg.tokens;
-  const int chunks = (len + kC16 - 1) / kC16, col = 16 * wave + r16;
+  if (MODE != kWholeRequests && whole > a.seg.tokens && len > a.seg.tokens) len = a.seg.tokens;
+  const int chunks = (len + kC16 - 1) / kC16;
+  float* const outs = (float*)(walk_lds + L::kOut);
+  if (wave >= NW) {
+    const int hw = wave - NW;
+    const float* work = a.work + (int64_t)(chunks16_before(sb, b, lane) + t0 / kC16) * a.H * C::kFloats + (int64_t)h * C::kFloats;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)walk_lds;
+    // a chunk's operands and rows (past the request's end: its last one again), 1 KiB per load, shared out over the helpers; the gates of a
+    // helper's tokens are its own loads (it reads them when the others may be on to the next chunk)
+    constexpr int LEAST = (OPS + ROWS) / NH + (DELTA ? ROWS / NH : 0);      // loads of a chunk by any helper, at the least
+    const auto row_piece = [&](const void* rows, int64_t stride, int c, int piece) {
+      const int at = piece * 1024 + lane * 16, t = at / (Dv * E::kBytes);
+      const int64_t row = start + c * kC16 + min(t, len - c * kC16 - 1);
+      return (const char*)rows + (row * stride + (int64_t)h * Dv) * E::kBytes + at % (Dv * E::kBytes);
+    };
+    const auto fetch = [&](int c) {
+      const uint32_t to = lds0 + c % 3 * L::kBuf;
+      for (int u = hw; u < OPS + ROWS; u += NH) {
+        const char* from = (const char*)(work + (int64_t)c * a.H * C::kFloats) + u * 1024 + lane * 16;
+        if (u >= OPS) from = row_piece(a.v, a.v_stride, c, u - OPS);
+        load_to_lds(from, to + u * 1024);
+      }
+      if constexpr (DELTA) {
+#pragma unroll
+        for (int u = 0; u < ROWS / NH; ++u) {
+          const int piece = hw * (ROWS / NH) + u;
+          load_to_lds(row_piece(a.gate, a.gate_stride, c, piece), to + (OPS + ROWS + piece) * 1024);
+        }
+      }
+    };
+    // lane: 8 values of a token
+    constexpr int PER = Dv / 8;
+    const int t = hw * (kC16 / NH) + lane / PER, at = lane % PER * 8;
+    float nw[8];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) nw[x] = OUT ? a.norm_w[(DELTA ? (int64_t)h * Dv : 0) + at + x] : 0.f;
+    const auto finish = [&](int c) {
+      const float* o = outs + ((c & 1) * kC16 + t) * L::kRow + at;
+      const f32x4_c o0 = *(const f32x4_c*)o, o1 = *(const f32x4_c*)(o + 4);
+      float f[8] = {o0[0], o0[1], o0[2], o0[3], o1[0], o1[1], o1[2], o1[3]}, ss = 0.f;
+#pragma unroll
+      for (int x = 0; x < 8; ++x) ss += f[x] * f[x];
+      const float inv = 1.f / sqrtf(lanes_sum<PER>(ss) / (float)Dv + a.eps);
+#pragma unroll
+      for (int x = 0; x < 8; ++x) f[x] = f[x] * inv * nw[x];
+      if constexpr (DELTA) {
+        float g[8];
+        const char* rows = walk_lds + c % 3 * L::kBuf + L::kOps + L::kRows + (t * Dv + at) * E::kBytes;
+#pragma unroll
+        for (int x = 0; x < 8; x += E::kVec) unpack16<Tag>(ld16(rows + x * E::kBytes), g + x);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) f[x] /= 1.f + expf(-g[x]);
+      }
+      if (t >= len - c * kC16) return;
+      char* to = (char*)a.out + ((start + c * kC16 + t) * a.out_stride + (int64_t)h * Dv + at) * E::kBytes;
+      if (a.vec_out) {
+#pragma unroll
+        for (int x = 0; x < 8; x += E::kVec) st16(to + x * E::kBytes, pack16<Tag>(f + x));
+      } else {
+#pragma unroll
+        for (int x = 0; x < 8; ++x) E::store(to, x, f[x]);
+      }
+    };
+    fetch(0);
+    if (chunks > 1) fetch(1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    for (int c = 0; c < chunks; ++c) {
+      if (OUT && c > 0) finish(c - 1);                 // (the gates of chunk c - 1 lie where chunk c + 2 goes)
+      if (c + 2 < chunks) {
+        if constexpr (DELTA) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        fetch(c + 2);
+      }
+      // waiting for all but the last LEAST loads is waiting for the chunk before
+      if (c + 2 < chunks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEAST) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();
+    }
+    if constexpr (OUT) finish(chunks - 1);
+    return;
+  }
+  const int col = 16 * wave + r16;
   float* st = a.state + load_idx(sb.req_pool_indices, b, sb.idx64) * a.state_stride + (int64_t)h * D * Dv;
   float* const part = MODE == kWholeRequests ? nullptr : a.seg.work + ((int64_t)blockIdx.x * a.H + h) * a.seg.stride;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)&lds[0][0];
-  const auto fetch = [&](int c) {
-    const float* from = work + (int64_t)c * a.H * C::kFloats + lane * 4;
-    for (int u = wave; u < LOADS; u += NW) load_to_lds(from + u * 256, lds0 + (c & 1) * (kUse * 4) + u * 1024);
-  };
-  const int64_t vc = (int64_t)h * Dv + col;
-  typename E::storage vn[4], gn[4];                   // the next chunk's values as they lie in memory
-  const auto fetch_v = [&](int c) {
-    const int end = len - c * kC16 - 1;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t row = start + c * kC16 + min(4 * q + r, end);
-      vn[r] = ((const typename E::storage*)a.v)[row * a.v_stride + vc];
-      if constexpr (DELTA) gn[r] = ((const typename E::storage*)a.gate)[row * a.gate_stride + vc];
-    }
-  };
-  fetch(0);
-  fetch_v(0);
   const float* from = split ? part : st;
   f32x4_c S[DT], decay[MODE == kSegmentSums ? DT : 1];
 #pragma unroll
@@ -242,142 +310,147 @@ __global__ void __launch_bounds__(NW * 64) chunk16_walk_kernel(Walk16 a, SeqBatc
 #pragma unroll
     for (int r = 0; r < 4; ++r) S[i][r] = held ? from[(int64_t)(16 * i + 4 * q + r) * Dv + col] : 0.f;
   }
-  const float nw = a.norm_w[DELTA ? (int64_t)h * Dv + col : col];
-  f32x4_c o = {0.f, 0.f, 0.f, 0.f};
-  float gate[4] = {1.f, 1.f, 1.f, 1.f};
-  // outputs of chunk c: `red` holds its waves' sums of squares
-  const auto finish = [&](int c) {
-    const int n = len - c * kC16;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float ss = 0.f;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) ss += red[c & 1][w][4 * q + r];
-      const float y = o[r] * (1.f / sqrtf(ss / (float)Dv + a.eps)) * nw;
-      if (4 * q + r < n) E::store(a.out, (start + c * kC16 + 4 * q + r) * a.out_stride + vc, DELTA ? y / (1.f + expf(-gate[r])) : y);
-    }
-  };
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   lds_barrier();
   for (int c = 0; c < chunks; ++c) {
     const int n = len - c * kC16;
-    const float* m = lds[c & 1];
-    float v[4], now[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      v[r] = 4 * q + r < n ? E::load(&vn[r], 0) : 0.f;
-      if constexpr (DELTA) now[r] = E::load(&gn[r], 0);
-    }
-    if (c + 1 < chunks) {
-      fetch(c + 1);
-      fetch_v(c + 1);
-    }
-    if (OUT && c > 0) finish(c - 1);
-    if constexpr (DELTA) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) gate[r] = now[r];
-    }
+    const float* m = (const float*)(walk_lds + c % 3 * L::kBuf);
     const auto row16 = [&](int at) { return *(const f32x4_c*)(m + at + r16 * 16 + place16(r16, q) * 4); };
     const auto row_d = [&](int at, int i) { return *(const f32x4_c*)(m + at + r16 * D + (((4 * i + q) ^ r16) << 2)); };
+    f32x4_c rd[OUT ? DT : 1], ud[DELTA ? DT : 1], g[DT], ke[DT], be[DELTA ? DT : 1], mr, pr, tr, qr;
+    float v[4];
+    // the operands of the next products are read while the matrix cores are on the ones before (left to itself the compiler keeps
+    // registers free and waits for each read)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = E::load((const char*)m + L::kOps, (4 * q + r) * Dv + col);
+    if constexpr (DELTA) mr = row16(C::kM);
+    if constexpr (OUT) {
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        rd[i] = row_d(C::kRd, i);
+        if constexpr (DELTA) ud[i] = row_d(C::kUd, i);
+      }
+    }
+    const auto read_update = [&] {
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        g[i] = *(const f32x4_c*)(m + C::kG + 16 * i + 4 * q);
+        ke[i] = *(const f32x4_c*)(m + C::kKe + (16 * i + r16) * 16 + place16(r16, q) * 4);
+        if constexpr (DELTA) be[i] = *(const f32x4_c*)(m + C::kBe + (16 * i + r16) * 16 + place16(r16, q) * 4);
+      }
+    };
+    if constexpr (!OUT) read_update();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = 4 * q + r < n ? v[r] : 0.f;
     int first = kC16;                                 // the column's first token that is not finite
     bool any = false;
     f32x4_c y = {0.f, 0.f, 0.f, 0.f};
     if constexpr (OUT) {
       const auto finite = [](float x) { return fabsf(x) < INFINITY; };
-      const auto rows_from = [&] {                    // `first` of the column, over the lanes that share it
+      const auto odd = [](const auto& x) {            // (in any lane)
+        const float probe = fmaf(x[0], 0.f, fmaf(x[1], 0.f, fmaf(x[2], 0.f, x[3] * 0.f)));
+        return __ballot(probe != probe) != 0;
+      };
+      const auto share_first = [&] {                  // over the lanes of the column
         first = min(first, __shfl_xor(first, 16, 64));
         first = min(first, __shfl_xor(first, 32, 64));
       };
-      const float probe = fmaf(v[0], 0.f, fmaf(v[1], 0.f, fmaf(v[2], 0.f, v[3] * 0.f)));
-      if (__ballot(probe != probe)) {
+      if (odd(v)) {
         any = true;
 #pragma unroll
         for (int r = 3; r >= 0; --r)
           if (!finite(v[r])) v[r] = 0.f, first = 4 * q + r;
-        rows_from();
+        share_first();
       }
-      o = f32x4_c{0.f, 0.f, 0.f, 0.f};
-      f32x4_c x = {0.f, 0.f, 0.f, 0.f};
+      f32x4_c o = {0.f, 0.f, 0.f, 0.f}, x = {0.f, 0.f, 0.f, 0.f};
       if constexpr (DELTA) {
-        const f32x4_c mr = row16(C::kM);
 #pragma unroll
         for (int r = 0; r < 4; ++r) x = mfma_4(mr[r], v[r], x);
       }
+      const auto read_state = [&](int i0, int i1) {
 #pragma unroll
-      for (int i = 0; i < DT; ++i) {
-        const f32x4_c rd = row_d(C::kRd, i);
-        f32x4_c ud;
-        if constexpr (DELTA) ud = row_d(C::kUd, i);
+        for (int i = i0; i < i1; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if constexpr (DELTA) x = mfma_4(ud[r], S[i][r], x);
-          o = mfma_4(rd[r], S[i][r], o);
-        }
-      }
-      const f32x4_c pr = row16(C::kP);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o = mfma_4(pr[r], v[r], o);
+          for (int r = 0; r < 4; ++r) {
+            if constexpr (DELTA) x = mfma_4(ud[i][r], S[i][r], x);
+            o = mfma_4(rd[i][r], S[i][r], o);
+          }
+      };
+      read_state(0, DT / 2);
+      __builtin_amdgcn_sched_barrier(0);
+      pr = row16(C::kP);
+      if constexpr (DELTA) tr = row16(C::kT), qr = row16(C::kQ);
+      read_update();
+      __builtin_amdgcn_sched_barrier(0);
+      read_state(DT / 2, DT);
       if constexpr (DELTA) {
-        const f32x4_c tr = row16(C::kT), qr = row16(C::kQ);
-        const float odd = fmaf(x[0], 0.f, fmaf(x[1], 0.f, fmaf(x[2], 0.f, x[3] * 0.f)));
-        if (__ballot(odd != odd)) {
+        if (odd(x)) {
           any = true;
 #pragma unroll
           for (int r = 3; r >= 0; --r)
             if (!finite(x[r])) x[r] = 0.f, first = min(first, 4 * q + r);
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) y = mfma_4(tr[r], x[r], y);
-        const float odd2 = fmaf(y[0], 0.f, fmaf(y[1], 0.f, fmaf(y[2], 0.f, y[3] * 0.f)));
-        if (any || __ballot(odd2 != odd2)) {
+        for (int r = 0; r < 4; ++r) {
+          y = mfma_4(tr[r], x[r], y);
+          o = mfma_4(pr[r], v[r], o);
+        }
+        if (any || odd(y)) {
           any = true;
 #pragma unroll
           for (int r = 3; r >= 0; --r)
             if (!finite(y[r])) first = min(first, 4 * q + r);
-          rows_from();
+          share_first();
 #pragma unroll
           for (int r = 0; r < 4; ++r) y[r] = 4 * q + r < first ? y[r] : 0.f;
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) o = mfma_4(qr[r], y[r], o);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o = mfma_4(pr[r], v[r], o);
       }
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[i][r] *= g[i][r];
       if (any) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] = 4 * q + r < first ? o[r] : as_f32(0x7fc00000u);
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float ss = lanes_sum<16>(o[r] * o[r]);
-        if (r16 == 0) red[c & 1][wave][4 * q + r] = ss;
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < DT; ++i) S[i] = mfma_4(ke[i][r], v[r], S[i]);
+      if constexpr (DELTA) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int i = 0; i < DT; ++i) S[i] = mfma_4(be[i][r], y[r], S[i]);
       }
-    }
-    if (MODE != kSegmentOutputs || c + 1 < chunks || last) {
 #pragma unroll
-      for (int i = 0; i < DT; ++i) {
-        const f32x4_c g = *(const f32x4_c*)(m + C::kG + 16 * i + 4 * q);
-        const f32x4_c ke = *(const f32x4_c*)(m + C::kKe + (16 * i + r16) * 16 + place16(r16, q) * 4);
-        f32x4_c be;
-        if constexpr (DELTA) be = *(const f32x4_c*)(m + C::kBe + (16 * i + r16) * 16 + place16(r16, q) * 4);
+      for (int r = 0; r < 4; ++r) outs[((c & 1) * kC16 + 4 * q + r) * L::kRow + col] = o[r];
+      if (any) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          S[i][r] *= g[r];
-          if constexpr (MODE == kSegmentSums) decay[i][r] *= g[r];
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          S[i] = mfma_4(ke[r], v[r], S[i]);
-          if constexpr (DELTA) S[i] = mfma_4(be[r], y[r], S[i]);
-        }
-        if (OUT && any) {
+        for (int i = 0; i < DT; ++i)
 #pragma unroll
           for (int r = 0; r < 4; ++r) S[i][r] = first < kC16 ? as_f32(0x7fc00000u) : S[i][r];
-        }
       }
+    } else {
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          S[i][r] *= g[i][r];
+          decay[i][r] *= g[i][r];
+        }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < DT; ++i) S[i] = mfma_4(ke[i][r], v[r], S[i]);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
   }
-  if constexpr (OUT) finish(chunks - 1);
   float* to = MODE == kSegmentSums ? part : st;
   if (MODE == kSegmentSums || last) {
 #pragma unroll
@@ -433,24 +506,32 @@ __global__ void __launch_bounds__(256) segment_rows_kernel(ScanSegments g, const
   }
 }
 
+template <typename Tag, int D, int NW, bool DELTA, int MODE>
+int launch_walk16_mode(const Walk16& a, unsigned groups, const SeqBatch& s, hipStream_t st) {
+  constexpr int bytes = Walk16Lds<Tag, D, NW, DELTA, MODE>::kBytes;
+  static PerDevice<int> raised;
+  if (!chunk_lds_ready(raised, (const void*)chunk16_walk_kernel<Tag, D, NW, DELTA, MODE>, bytes)) return SP_ERR_LAUNCH;
+  chunk16_walk_kernel<Tag, D, NW, DELTA, MODE><<<dim3(groups, (unsigned)a.H), NW * 96, bytes, st>>>(a, s);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
 template <typename Tag, int D, int NW, bool DELTA>
 int launch_walk16(const Walk16& a, int64_t tokens, const SeqBatch& s, hipStream_t st) {
-  if (a.seg.tokens == 0) {
-    chunk16_walk_kernel<Tag, D, NW, DELTA, kWholeRequests><<<dim3((unsigned)s.B, (unsigned)a.H), NW * 64, 0, st>>>(a, s);
-    SP_LAUNCH_CHECK();
-    return SP_OK;
-  }
+  if (a.seg.tokens == 0) return launch_walk16_mode<Tag, D, NW, DELTA, kWholeRequests>(a, (unsigned)s.B, s, st);
   if constexpr (!DELTA) {
-    const dim3 grid((unsigned)(tokens / a.seg.tokens + s.B), (unsigned)a.H);
-    chunk16_walk_kernel<Tag, D, NW, DELTA, kSegmentSums><<<grid, NW * 64, 0, st>>>(a, s);
-    SP_LAUNCH_CHECK();
+    const unsigned groups = (unsigned)(tokens / a.seg.tokens + s.B);
+    const int rc = launch_walk16_mode<Tag, D, NW, DELTA, kSegmentSums>(a, groups, s, st);
+    if (rc != SP_OK) return rc;
     segment_rows_kernel<D, NW * 16><<<dim3((unsigned)s.B, (unsigned)a.H, D * NW * 16 / 1024), 256, 0, st>>>(a.seg, a.state, a.state_stride, s, a.H);
     SP_LAUNCH_CHECK();
-    chunk16_walk_kernel<Tag, D, NW, DELTA, kSegmentOutputs><<<grid, NW * 64, 0, st>>>(a, s);
-    SP_LAUNCH_CHECK();
-    return SP_OK;
+    return launch_walk16_mode<Tag, D, NW, DELTA, kSegmentOutputs>(a, groups, s, st);
   }
   return SP_ERR_UNSUPPORTED;
+}
+
+// 16-byte loads of rows of `type` at `p`
+inline bool rows_aligned(const void* p, int64_t stride, int dtype) {
+  return ((uintptr_t)p & 15) == 0 && stride % (dtype == SP_F32 ? 4 : 8) == 0;
 }
 
 inline int64_t chunk16_units(int64_t tokens, int B) { return tokens / kC16 + B; }      // at most: a request's last chunk may be partial

@@ -15,7 +15,7 @@
 // (register moves); no workgroup barrier.  The order of its sums depends on the head only.  Prompts take it; a decode step (one token
 // per request, heads of 64 or 128, rank up to 512) takes delta_step_kernel, which forms the gates too and adds a head's sums in
 // another order.
-#include "seq_batch.h"
+#include "chunk16.h"
 
 namespace sp {
 namespace {
@@ -341,6 +341,62 @@ static int launch_delta(void* out, int64_t out_stride, const void* r, int64_t r_
   return SP_OK;
 }
 
+// ---- steps of several tokens per request, 16 tokens at a time on the matrix cores (chunk16.h: u the unit key, b = remove * u) ----------
+// The per-token form above is a chain of a sweep over the column and two sums over its lanes per token.  32 heads of 64 (width 2048), us per
+// layer: one request of 4096 tokens 2309 -> 1010 (the walk 625: 2.4 per chunk; prepare 80, gates 57), 4 requests of 4096 tokens together
+// 835 -> 531, 16 of them 558 -> 497.  Heads of 128 stay with the per-token form (their operands and state crowd the registers).
+template <typename Tag, int D>
+__global__ void __launch_bounds__(256)
+delta_prepare_kernel(float* work, const char* r, int64_t r_stride, const char* k, int64_t k_stride, const float* decay, const float* remove,
+                     SeqBatch s, int H) {
+  typedef Elem<Tag> E;
+  constexpr int V = E::kVec, QP = D / V;
+  const int h = blockIdx.y;
+  int b, t0;
+  if (!segment_at(s, (int)blockIdx.x, kC16, threadIdx.x & 63, b, t0)) return;
+  const int64_t row0 = (int64_t)s.extend_start_loc[b] + t0;
+  const int n = s.extend_seq_lens[b] - t0;
+  chunk16_prepare<D, true>(work + ((int64_t)blockIdx.x * H + h) * Chunk16<D, true>::kFloats,
+                           [&](auto& sr, auto& sk, auto& sw, auto& su, auto& sb) {
+    for (int e = threadIdx.x; e < kC16 * QP; e += 256) {               // (whole groups of QP lanes)
+      const int t = e / QP, i = e % QP * V, c = h * D + i;
+      float rf[V], kf[V], k2 = 0.f;
+      const u32x4 zero = {0u, 0u, 0u, 0u};
+      unpack16<Tag>(t < n ? ld16(r + ((row0 + t) * r_stride + c) * E::kBytes) : zero, rf);
+      unpack16<Tag>(t < n ? ld16(k + ((row0 + t) * k_stride + c) * E::kBytes) : zero, kf);
+#pragma unroll
+      for (int x = 0; x < V; ++x) k2 += kf[x] * kf[x];
+      k2 = lanes_sum<(QP < 16 ? QP : 16)>(k2);
+      if constexpr (QP == 32) k2 += __shfl_xor(k2, 16, 64);
+      const float inv = 1.f / sqrtf(k2 + 1e-6f);
+#pragma unroll
+      for (int x = 0; x < V; x += 4) {
+        const int64_t at = (row0 + t) * H * D + c + x;
+        const f32x4_c w = t < n ? *(const f32x4_c*)(decay + at) : f32x4_c{1.f, 1.f, 1.f, 1.f};
+        const f32x4_c a = t < n ? *(const f32x4_c*)(remove + at) : f32x4_c{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int z = 0; z < 4; ++z) {
+          const float u = kf[x + z] * inv;
+          sr[t][i + x + z] = rf[x + z];
+          sk[t][i + x + z] = kf[x + z];
+          sw[t][i + x + z] = w[z];
+          su[t][i + x + z] = u;
+          sb[t][i + x + z] = a[z] * u;
+        }
+      }
+    }
+  });
+}
+
+template <typename Tag>
+static int launch_delta_chunks16(Tag, const Walk16& w, float* work, const void* r, int64_t r_stride, const void* k, int64_t k_stride,
+                                 const float* decay, const float* remove, int64_t tokens, const SeqBatch& s, hipStream_t st) {
+  delta_prepare_kernel<Tag, 64><<<dim3((unsigned)chunk16_units(tokens, s.B), (unsigned)w.H), 256, 0, st>>>(
+      work, (const char*)r, r_stride, (const char*)k, k_stride, decay, remove, s, w.H);
+  SP_LAUNCH_CHECK();
+  return launch_walk16<Tag, 64, 4, true>(w, tokens, s, st);
+}
+
 }  // namespace
 }  // namespace sp
 
@@ -382,6 +438,33 @@ extern "C" int sp_delta_recurrence(void* out, int64_t out_stride, const void* r,
   SP_DISPATCH_DTYPE(dtype, return (launch_delta<Tag>(out, out_stride, r, r_stride, k, k_stride, v, v_stride, g, g_stride, decay,
                                                      remove, norm_w, state, state_stride, s, heads, head_dim, eps,
                                                      (hipStream_t)stream)));
+}
+
+extern "C" int64_t sp_delta_recurrence_chunk_floats(int64_t num_tokens, int batch_size, int heads, int head_dim) {
+  return head_dim == 64 ? chunk16_units(num_tokens, batch_size) * heads * Chunk16<64, true>::kFloats : 0;
+}
+
+extern "C" int sp_delta_recurrence_chunks(void* out, int64_t out_stride, const void* r, int64_t r_stride, const void* k, int64_t k_stride,
+                                          const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* decay,
+                                          const float* remove, const float* norm_w, float* state, int64_t state_stride, float* work,
+                                          int64_t num_tokens, int heads, int head_dim, float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
+  SP_CHECK_ARG(batch_size >= 0 && num_tokens >= 0 && heads > 0 && head_dim > 0);
+  if (batch_size == 0 || num_tokens == 0) return SP_OK;
+  SP_CHECK_ARG(out && r && k && v && g && decay && remove && norm_w && state && work && req_pool_indices && seq_lens);
+  SP_CHECK_ARG(!extend_seq_lens || (extend_prefix_lens && extend_start_loc));
+  SP_CHECK_ARG(state_stride >= (int64_t)heads * head_dim * head_dim);
+  const int64_t n = (int64_t)heads * head_dim;
+  SP_CHECK_ARG(r_stride >= n && k_stride >= n && v_stride >= n && g_stride >= n && out_stride >= n);
+  SEQ_BATCH(s);
+  if (!extend_seq_lens || head_dim != 64 || heads > 65535 || !rows_aligned(r, r_stride, dtype) ||
+      !rows_aligned(k, k_stride, dtype) || !rows_aligned(v, v_stride, dtype) || !rows_aligned(g, g_stride, dtype) ||
+      (((uintptr_t)decay | (uintptr_t)remove | (uintptr_t)work) & 15) ||
+      chunk16_units(num_tokens, batch_size) >> 31)
+    return SP_ERR_UNSUPPORTED;
+  const Walk16 w{out, v, g, norm_w, work, state, out_stride, v_stride, g_stride, state_stride, ScanSegments{nullptr, 0, 0}, heads, eps,
+                 rows_aligned(out, out_stride, dtype)};
+  SP_DISPATCH_DTYPE(dtype, return (launch_delta_chunks16(Tag(), w, work, r, r_stride, k, k_stride, decay, remove, num_tokens, s,
+                                                         (hipStream_t)stream)));
 }
 
 extern "C" int sp_delta_step(void* out, int64_t out_stride, const void* r, int64_t r_stride, const void* k, int64_t k_stride,

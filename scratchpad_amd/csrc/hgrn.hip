@@ -270,12 +270,13 @@ extern "C" int sp_hgrn2_chunks(void* out, int64_t out_stride, const void* qpre, 
   const int64_t nk = (int64_t)heads * dim, nv = (int64_t)heads * vdim;
   SP_CHECK_ARG(q_stride >= nk && f_stride >= nk && v_stride >= nv && out_stride >= nv && state_stride >= nk * vdim);
   SEQ_BATCH(s);
-  const int per = dtype == SP_F32 ? 4 : 8;
-  if (!extend_seq_lens || (dim != 64 && dim != 128) || (vdim != 64 && vdim != 128) || q_stride % per || f_stride % per || heads > 65535 ||
-      (((uintptr_t)qpre | (uintptr_t)fpre | (uintptr_t)work | (uintptr_t)segment_work) & 15) || chunk16_units(num_tokens, batch_size) >> 31)
+  if (!extend_seq_lens || (dim != 64 && dim != 128) || (vdim != 64 && vdim != 128) || heads > 65535 ||
+      !rows_aligned(qpre, q_stride, dtype) || !rows_aligned(fpre, f_stride, dtype) || !rows_aligned(v, v_stride, dtype) ||
+      (((uintptr_t)work | (uintptr_t)segment_work) & 15) || chunk16_units(num_tokens, batch_size) >> 31)
     return SP_ERR_UNSUPPORTED;
   const Walk16 w{out, v, nullptr, norm_w, work, state, out_stride, v_stride, 0, state_stride,
-                 ScanSegments{segment_work, (int64_t)dim * vdim + dim, segment_tokens}, heads, eps};
+                 ScanSegments{segment_work, (int64_t)dim * vdim + dim, segment_tokens}, heads, eps,
+                 rows_aligned(out, out_stride, dtype)};
 #define SP_HGRN_CHUNKS(D, NW)                                                                                                     \
   SP_DISPATCH_DTYPE(dtype, return (launch_hgrn2_chunks<Tag, D, NW>(w, work, qpre, q_stride, fpre, f_stride, f_bias, lower, num_tokens, s, \
                                                                    (hipStream_t)stream)))

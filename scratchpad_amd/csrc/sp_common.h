@@ -238,6 +238,24 @@ __device__ __forceinline__ float wave_sum(float v) {
   v += dpp_f32<0x4E>(v);                            // quad_perm [2,3,0,1]: lane ^ 2
   return v + dpp_f32<0xB1>(v);                      // quad_perm [1,0,3,2]: lane ^ 1
 }
+// Eight sums at a time over the lanes whose numbers differ in bits 3, 4 and 5 (all lanes active): lane l ends with the sum of v[l >> 3].
+// Every step halves the values that a lane carries - 15 instructions where eight sums one after the other take 56.
+__device__ __forceinline__ float eight_sums(const float* v, int lane) {
+  float a[4], b[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const auto h = __builtin_amdgcn_permlane32_swap(as_u32(v[i]), as_u32(v[i + 4]), false, false);
+    a[i] = as_f32(h[0]) + as_f32(h[1]);             // lanes 0-31: of v[i], lanes 32-63: of v[i + 4]
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto h = __builtin_amdgcn_permlane16_swap(as_u32(a[i]), as_u32(a[i + 2]), false, false);
+    b[i] = as_f32(h[0]) + as_f32(h[1]);             // even rows of 16: of a[i], odd rows: of a[i + 2]
+  }
+  const bool up = lane & 8;
+  const float keep = up ? b[1] : b[0], give = up ? b[0] : b[1];
+  return keep + dpp_f32<0x128>(give);               // row_ror 8: lane ^ 8
+}
 // over N neighbouring lanes (aligned groups of N = 1, 2, 4, 8 or 16)
 template <int N>
 __device__ __forceinline__ float lanes_sum(float v) {

@@ -89,3 +89,71 @@ def test_hgrn2_numbers_that_are_not_finite_reach_no_earlier_token(at, where, bad
         assert not torch.isfinite(out[at:, 0, 3].float()).any() and not torch.isfinite(S[0, :, 3]).any()
     elif bad != float("inf"):                                    # (an infinite pre-activation is an open gate)
         assert not torch.isfinite(out[at:, 0].float()).any() and not torch.isfinite(S[0, 3]).any()
+
+
+def delta_reference(r, k, v, g, w, a, S, H):
+    T, D = r.shape[0], r.shape[1] // H
+    r, k, v, g, w, a = (x.double().view(T, H, D) for x in (r, k, v, g, w, a))
+    o = torch.empty(T, H, D, dtype=torch.float64, device=DEV)
+    for t in range(T):
+        u = k[t] / torch.sqrt((k[t] * k[t]).sum(-1, keepdim=True) + 1e-6)
+        y = (S * u[:, :, None]).sum(1)
+        S = w[t][:, :, None] * S - (a[t] * u)[:, :, None] * y[:, None] + k[t][:, :, None] * v[t][:, None]
+        o[t] = (S * r[t][:, :, None]).sum(1)
+    return rms(o) * torch.sigmoid(g), S
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lens", LENS, ids=lambda l: "-".join(map(str, l[:5])))
+@pytest.mark.parametrize("H,D", [(3, 64), (1, 64)])
+def test_delta_recurrence_chunks(lens, H, D, dtype, monkeypatch):
+    from scratchpad_amd import _native
+    announce("delta recurrence chunks", dtype, lens, H, D)
+    monkeypatch.setattr(_native, "DELTA_RECURRENCE_CHUNKS", True)
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    T, slots = sum(lens), [2 * i + 1 for i in range(len(lens))]
+    S = torch.full((2 * len(lens) + 1, H, D, D), float("nan"), device=DEV)
+    nw = torch.rand(H * D, generator=gen, device=DEV) + 0.5
+    ref = [torch.zeros(H, D, D, dtype=torch.float64, device=DEV) for _ in lens]
+    for prefixes in ([0] * len(lens), lens):
+        r, k, v, g = torch.randn(T, 4 * H * D, generator=gen, device=DEV).to(dtype).split(H * D, 1)
+        w = torch.exp(-0.6 * torch.rand(T, H * D, generator=gen, device=DEV))
+        a = torch.rand(T, H * D, generator=gen, device=DEV)
+        out = _native.delta_recurrence(r, k, v, g, w, a, nw, S, seq_extend(lens, prefixes, slots), H, D, 1e-5).view(T, H, D)
+        at = 0
+        for i, n in enumerate(lens):
+            rows = slice(at, at + n)
+            want, ref[i] = delta_reference(r[rows], k[rows], v[rows], g[rows], w[rows], a[rows], ref[i], H)
+            near(S[slots[i]], ref[i])
+            want = want * nw.double().view(H, D)
+            assert ((out[rows].double() - want).abs() <= HALF[dtype] * want.abs() + 1e-3).all()
+            at += n
+    assert torch.isnan(S[::2]).all()
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["read", "key", "value", "decay", "remove"])
+@pytest.mark.parametrize("at", [0, 5, 15, 16, 50])
+def test_delta_numbers_that_are_not_finite_reach_no_earlier_token(at, where, bad, monkeypatch):
+    from scratchpad_amd import _native
+    monkeypatch.setattr(_native, "DELTA_RECURRENCE_CHUNKS", True)
+    H, D, T = 2, 64, 70
+    gen = torch.Generator(device=DEV).manual_seed(10)
+    x = [torch.randn(T, H * D, generator=gen, device=DEV).bfloat16() for _ in range(4)]
+    x += [torch.exp(-0.6 * torch.rand(T, H * D, generator=gen, device=DEV)), torch.rand(T, H * D, generator=gen, device=DEV)]
+
+    def run(x):
+        S = torch.zeros(2, H, D, D, device=DEV)
+        out = _native.delta_recurrence(*x, torch.ones(H * D, device=DEV), S, seq_extend([T], [0], [1]), H, D, 1e-5)
+        return out.view(T, H, D), S[1]
+    clean = run(x)
+    y = [t.clone() for t in x]
+    y[{"read": 0, "key": 1, "value": 2, "decay": 4, "remove": 5}[where]][at, 3] = bad
+    out, S = run(y)
+    assert torch.equal(out[:at], clean[0][:at]) and torch.equal(out[:, 1], clean[0][:, 1]) and torch.equal(S[1], clean[1][1])
+    if where == "read":
+        assert torch.equal(S, clean[1]) and torch.equal(out[at + 1:], clean[0][at + 1:])
+    elif where == "value":
+        assert not torch.isfinite(out[at:, 0, 3].float()).any() and not torch.isfinite(S[0, :, 3]).any()
+    else:
+        assert not torch.isfinite(out[at + 1:, 0].float()).any() and not torch.isfinite(S[0, 3]).any()
