@@ -155,42 +155,43 @@ __global__ void __launch_bounds__(D * 2) delta_chunk_prepare_kernel(DeltaChunks 
   // lane (s0, part): columns s0 and s0 + 8 over 4 channels; only rows t >= 8 matter to the second
   const int s0 = lane & 7, part = lane >> 3, i = wave * 32 + part * 4;
   f32x4_d rat = *(const f32x4_d*)&sk[s0][i], rat8 = *(const f32x4_d*)&sk[s0 + 8][i];
-  const auto all_parts = [](float v) {
-    v += dpp_f32<0x128>(v);                           // row_ror 8: the other half of the 16 lanes
-    v += __shfl_xor(v, 16, 64);
-    return v + __shfl_xor(v, 32, 64);
-  };
-  float kks[kDC], qks[kDC], kk8s[kDC / 2], qk8s[kDC / 2];
+  float kks[2][2], qks[2][2];                         // [half][column]: of token 8 half + part
 #pragma unroll
-  for (int t = 0; t < kDC; ++t) {
-    const f32x4_d kt = *(const f32x4_d*)&sk[t][i], qt = *(const f32x4_d*)&sq[t][i];
-    if constexpr (CHANNEL) {
-      const f32x4_d wt = *(const f32x4_d*)&sw[t][i];
+  for (int half = 0; half < 2; ++half) {
+    float kk[2][8], qk[2][8];
 #pragma unroll
-      for (int x = 0; x < 4; ++x) rat[x] *= t >= 8 || t > s0 ? wt[x] : 1.f;
-      if (t > 8) {
+    for (int u = 0; u < 8; ++u) {
+      const int t = 8 * half + u;
+      const f32x4_d kt = *(const f32x4_d*)&sk[t][i], qt = *(const f32x4_d*)&sq[t][i];
+      if constexpr (CHANNEL) {
+        const f32x4_d wt = *(const f32x4_d*)&sw[t][i];
 #pragma unroll
-        for (int x = 0; x < 4; ++x) rat8[x] *= t > s0 + 8 ? wt[x] : 1.f;
+        for (int x = 0; x < 4; ++x) rat[x] *= t >= 8 || t > s0 ? wt[x] : 1.f;
+        if (t > 8) {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) rat8[x] *= t > s0 + 8 ? wt[x] : 1.f;
+        }
       }
+      // (t < s: a number that nobody reads)
+      kk[0][u] = (kt[0] * rat[0] + kt[1] * rat[1]) + (kt[2] * rat[2] + kt[3] * rat[3]);
+      qk[0][u] = (qt[0] * rat[0] + qt[1] * rat[1]) + (qt[2] * rat[2] + qt[3] * rat[3]);
+      kk[1][u] = (kt[0] * rat8[0] + kt[1] * rat8[1]) + (kt[2] * rat8[2] + kt[3] * rat8[3]);
+      qk[1][u] = (qt[0] * rat8[0] + qt[1] * rat8[1]) + (qt[2] * rat8[2] + qt[3] * rat8[3]);
     }
-    // (t < s: a number that nobody reads)
-    kks[t] = all_parts((kt[0] * rat[0] + kt[1] * rat[1]) + (kt[2] * rat[2] + kt[3] * rat[3]));
-    qks[t] = all_parts((qt[0] * rat[0] + qt[1] * rat[1]) + (qt[2] * rat[2] + qt[3] * rat[3]));
-    if (t >= 8) {
-      kk8s[t & 7] = all_parts((kt[0] * rat8[0] + kt[1] * rat8[1]) + (kt[2] * rat8[2] + kt[3] * rat8[3]));
-      qk8s[t & 7] = all_parts((qt[0] * rat8[0] + qt[1] * rat8[1]) + (qt[2] * rat8[2] + qt[3] * rat8[3]));
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+      kks[half][z] = z <= half ? eight_sums(kk[z], lane) : 0.f;
+      qks[half][z] = z <= half ? eight_sums(qk[z], lane) : 0.f;
     }
   }
   __syncthreads();                                    // every wave is done with the rows
-  if (part == 0) {
 #pragma unroll
-    for (int t = 0; t < kDC; ++t) {
-      skk[wave][t][s0] = kks[t];
-      sqk[wave][t][s0] = qks[t];
-      skk[wave][t][s0 + 8] = t >= 8 ? kk8s[t & 7] : 0.f;
-      sqk[wave][t][s0 + 8] = t >= 8 ? qk8s[t & 7] : 0.f;
+  for (int half = 0; half < 2; ++half)
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+      skk[wave][8 * half + part][s0 + 8 * z] = kks[half][z];
+      sqk[wave][8 * half + part][s0 + 8 * z] = qks[half][z];
     }
-  }
   __syncthreads();
   for (int e = tid; e < kDC * kDC; e += NT) {
     const int t = e / kDC, s = e % kDC;
