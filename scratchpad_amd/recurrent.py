@@ -90,11 +90,11 @@ class Mamba2Mixer(nn.Module):
         inner = self.heads * self.vdim
         zxbc = _native.linear(h, self.in_proj)
         dt = _native.small_linear_f32(h, self.dt_proj.data)
-        xbc = _native.causal_conv_silu(zxbc[:, inner:], self.conv.data, self.conv_bias.data,
-                                       states.state(self.layer_id, "conv"), seq)
+        z, xbc = zxbc.split_with_sizes([inner, zxbc.shape[1] - inner], 1)
+        xbc = _native.causal_conv_silu(xbc, self.conv.data, self.conv_bias.data, states.state(self.layer_id, "conv"), seq)
         y = _native.mamba2_scan(xbc, dt, self.dt_bias.data, self.A_log.data, self.D.data, states.state(self.layer_id, "ssm"),
                                 seq, self.heads, self.groups, self.state, self.vdim)
-        return _native.linear(_native.gated_group_norm(y, zxbc[:, :inner], self.norm.data, self.norm_groups, self.eps), self.o)
+        return _native.linear(_native.gated_group_norm(y, z, self.norm.data, self.norm_groups, self.eps), self.o)
 
 
 class MLSTMMixer(nn.Module):
@@ -125,8 +125,7 @@ class MLSTMMixer(nn.Module):
         a = _native.linear(h, self.qkvg)
         gates = _native.small_linear_f32(h, self.gates.data, self.gates_bias.data)
         L = self.layer_id
-        o = _native.mlstm_scan(a[:, :nk], a[:, nk:2 * nk], a[:, 2 * nk:2 * nk + nv], a[:, 2 * nk + nv:], gates[:, :H],
-                               gates[:, H:], self.norm.data, states.state(L, "S"), states.state(L, "n"), states.state(L, "m"), seq,
+        o = _native.mlstm_scan(*a.split_with_sizes([nk, nk, nv, nv], 1), *gates.split_with_sizes([H, H], 1), self.norm.data, states.state(L, "S"), states.state(L, "n"), states.state(L, "m"), seq,
                                self.heads, self.dim, self.vdim, self.cap, self.eps)
         return _native.linear(o, self.o)
 
@@ -166,11 +165,12 @@ class GeneralDeltaMixer(nn.Module):
         n = self.heads * self.dim
         a = _native.linear(h, self.in_proj)
         S = states.state(self.layer_id if state_id is None else state_id, "S")
-        o = _native.delta_step(a[:, :n], a[:, n:2 * n], a[:, 2 * n:3 * n], a[:, 3 * n:4 * n], a[:, 5 * n:5 * n + self.rank],
-                               a[:, 4 * n:5 * n], self.w2t.data, self.w0.data, self.a_bias.data, self.rate, self.norm.data, S, seq,
+        # (one call for all views: a slice each is a sixth of an eager decode step's host time)
+        r, k, v, g, remove, p, extra = a.split_with_sizes([n, n, n, n, n, self.rank, self.extra_rows], 1)
+        o = _native.delta_step(r, k, v, g, p, remove, self.w2t.data, self.w0.data, self.a_bias.data, self.rate, self.norm.data, S, seq,
                                self.heads, self.dim, self.eps)
         y = _native.linear(o, self.o)
-        return (y, a[:, 5 * n + self.rank:]) if self.extra_rows else y
+        return (y, extra) if self.extra_rows else y
 
 
 class HGRN2Mixer(nn.Module):
@@ -201,7 +201,8 @@ class HGRN2Mixer(nn.Module):
         seq, states = forward_batch.attn_backend.seq, forward_batch.state_pool
         nk = self.heads * self.dim
         S = states.state(self.layer_id if state_id is None else state_id, "S")
-        o = _native.hgrn2_scan(a[:, :nk], a[:, nk:2 * nk], a[:, 2 * nk:self.in_rows], self.f_bias.data, self.lower.data,
+        q, f, v, _ = a.split_with_sizes([nk, nk, self.in_rows - 2 * nk, a.shape[1] - self.in_rows], 1)
+        o = _native.hgrn2_scan(q, f, v, self.f_bias.data, self.lower.data,
                                self.norm.data, S, seq, self.heads, self.dim, self.vdim, self.eps)
         return _native.linear(o, self.o)
 
@@ -248,11 +249,11 @@ class GatedDeltaMixer(nn.Module):
         seq, states = forward_batch.attn_backend.seq, forward_batch.state_pool
         sid = self.layer_id if state_id is None else state_id
         nk, H, c = self.kv_heads * self.dim, self.heads, self.conv_rows
-        qkv = _native.causal_conv_silu(a[:, :c], self.conv.data, None, states.state(sid, "conv"), seq)
-        decay = _native.lowrank_gate(a[:, c + H:c + H + self.decay_rank], self.a2t.data, self.dt_bias.data, "decay",
-                                     self.A_log.data)
-        gate = _native.lowrank_gate(a[:, c + H + self.decay_rank:self.in_rows], self.g2t.data, None, "sigmoid")
-        o = _native.gated_delta_scan(qkv[:, :nk], qkv[:, nk:2 * nk], qkv[:, 2 * nk:], a[:, c:c + H], decay, gate,
+        rows, b, a1, g1, _ = a.split_with_sizes([c, H, self.decay_rank, self.gate_rank, a.shape[1] - self.in_rows], 1)
+        qkv = _native.causal_conv_silu(rows, self.conv.data, None, states.state(sid, "conv"), seq)
+        decay = _native.lowrank_gate(a1, self.a2t.data, self.dt_bias.data, "decay", self.A_log.data)
+        gate = _native.lowrank_gate(g1, self.g2t.data, None, "sigmoid")
+        o = _native.gated_delta_scan(*qkv.split_with_sizes([nk, nk, c - 2 * nk], 1), b, decay, gate,
                                      self.norm.data, states.state(sid, "S"), seq, H, self.kv_heads, self.dim, self.vdim,
                                      self.eps)
         return _native.linear(o, self.o)
@@ -301,8 +302,9 @@ class HeadDeltaMixer(nn.Module):
         sid = self.layer_id if state_id is None else state_id
         nk, c = self.kv_heads * self.dim, self.conv_rows
         pre = _native.small_linear_f32(x, self.gates.data)
-        qkv = _native.causal_conv_silu(a[:, :c], self.conv.data, None, states.state(sid, "conv"), seq)
-        o = _native.head_delta_scan(qkv[:, :nk], qkv[:, nk:2 * nk], qkv[:, 2 * nk:], a[:, c:self.in_rows], pre, self.dt_bias.data,
+        rows, gate, _ = a.split_with_sizes([c, self.in_rows - c, a.shape[1] - self.in_rows], 1)
+        qkv = _native.causal_conv_silu(rows, self.conv.data, None, states.state(sid, "conv"), seq)
+        o = _native.head_delta_scan(*qkv.split_with_sizes([nk, nk, c - 2 * nk], 1), gate, pre, self.dt_bias.data,
                                     self.A_log.data, self.norm.data, states.state(sid, "S"), seq, self.heads, self.kv_heads,
                                     self.dim, self.vdim, self.eps)
         return _native.linear(o, self.o)
