@@ -755,6 +755,13 @@ SP_API int sp_gated_delta_chunks(void* out, int64_t out_stride, const void* q, i
                                  const float* gate, const float* norm_w, float* state, int64_t state_stride, float* work,
                                  float* raw, int64_t num_tokens, int heads, int kv_heads, int dim, int vdim, float eps,
                                  SP_SEQ_PARAMS, int dtype, void* stream);
+/* The same with gate = sigmoid(p w2t) formed where it is used (p [num_tokens, rank] in `dtype`, w2t fp32 [rank, heads * vdim]): bf16, rank 32
+ * or 64, vdim 64 or 128, rows of p 16-byte and of out 8-byte aligned; else SP_ERR_UNSUPPORTED and nothing is launched.        */
+SP_API int sp_gated_delta_chunks_lowrank(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                         const void* v, int64_t v_stride, const void* bpre, int64_t b_stride, const float* decay,
+                                         const void* p, int64_t p_stride, const float* w2t, int rank, const float* norm_w, float* state,
+                                         int64_t state_stride, float* work, float* raw, int64_t num_tokens, int heads, int kv_heads,
+                                         int dim, int vdim, float eps, SP_SEQ_PARAMS, int dtype, void* stream);
 
 /* ================================================================================================================
  * ABI 14: post-norm layers (the stream itself is normed after every sum) whose experts may hand their input on.

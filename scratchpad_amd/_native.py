@@ -186,6 +186,8 @@ SIGNATURES = {
     "sp_gated_delta_chunks": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64,
                                      _i32, _i32, _i32, _i32, _f32, *_SEQ, _i32, _vp]),
     # ---- ABI 14
+    "sp_gated_delta_chunks_lowrank": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _i32, _vp, _vp, _i64,
+                                             _vp, _vp, _i64, _i32, _i32, _i32, _i32, _f32, *_SEQ, _i32, _vp]),
     "sp_post_norm": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _f32, _vp, _vp, _i64, _i64, _i32,
                             _f32, _i32, _vp]),
     # ---- ABI 15
@@ -2031,21 +2033,40 @@ def _delta_chunk_buffers(seq: SeqParams, heads: int, vdim: int, device):
 
 
 def gated_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bpre: torch.Tensor, decay: torch.Tensor,
-                     gate: torch.Tensor, norm_w: torch.Tensor, state: torch.Tensor, seq: SeqParams, heads: int, kv_heads: int,
+                     gate, norm_w: torch.Tensor, state: torch.Tensor, seq: SeqParams, heads: int, kv_heads: int,
                      dim: int, vdim: int, eps: float) -> torch.Tensor:
     """q, k [T, kv_heads * dim], v [T, heads * vdim], bpre [T, heads] (views) -> [T, heads * vdim]; decay fp32
-    [T, heads * dim], gate fp32 [T, heads * vdim]; state [slots, heads, dim, vdim] fp32 is read and moved on"""
+    [T, heads * dim], gate fp32 [T, heads * vdim], or (p [T, rank] a view, w2t fp32 [rank, heads * vdim]) for sigmoid(p w2t);
+    state [slots, heads, dim, vdim] fp32 is read and moved on"""
     T = seq.num_tokens
     for name, t, w in (("q", q, kv_heads * dim), ("k", k, kv_heads * dim), ("v", v, heads * vdim), ("bpre", bpre, heads)):
         if _mat(t, name).shape != (T, w) or t.dtype != q.dtype:
             raise RuntimeError(f"gated_delta_scan: {name} must be [num_tokens, {w}] of one dtype")
-    _f32(decay, "decay"), _f32(gate, "gate"), _f32(norm_w, "norm_w"), _f32(state, "state")
-    if decay.shape != (T, heads * dim) or gate.shape != (T, heads * vdim) or norm_w.numel() != vdim or \
-            state.shape[1:] != (heads, dim, vdim) or not decay.is_contiguous() or not gate.is_contiguous():
-        raise RuntimeError("gated_delta_scan: decay [T, H*D], gate [T, H*Dv], norm_w [Dv], state [slots, H, D, Dv]")
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
-    if _delta_chunks_take(q, k, v, decay, seq, dim, vdim) and delta_chunks_pay(True, seq, heads, dim, vdim):
+    chunks = _delta_chunks_take(q, k, v, decay, seq, dim, vdim) and delta_chunks_pay(True, seq, heads, dim, vdim)
+    lowrank = None
+    if isinstance(gate, tuple):
+        p, w2t = gate
+        if chunks and q.dtype == p.dtype == torch.bfloat16 and _mat(p, "p").shape == (T, w2t.shape[0]) and w2t.shape[0] in (32, 64) and \
+                vdim in (64, 128) and _f32(w2t, "w2t").shape[1] == heads * vdim and p.stride(0) % 8 == 0 and (p.data_ptr() | norm_w.data_ptr()) % 16 == 0:
+            lowrank = gate
+        else:
+            gate = lowrank_gate(p, w2t, None, "sigmoid")
+    _f32(decay, "decay"), _f32(norm_w, "norm_w"), _f32(state, "state")
+    if lowrank is None and (_f32(gate, "gate").shape != (T, heads * vdim) or not gate.is_contiguous()):
+        raise RuntimeError("gated_delta_scan: gate [T, H*Dv]")
+    if decay.shape != (T, heads * dim) or norm_w.numel() != vdim or state.shape[1:] != (heads, dim, vdim) or \
+            not decay.is_contiguous():
+        raise RuntimeError("gated_delta_scan: decay [T, H*D], norm_w [Dv], state [slots, H, D, Dv]")
+    if chunks:
         work, raw = _delta_chunk_buffers(seq, heads, vdim, q.device)
+        if lowrank is not None:
+            _check(load().sp_gated_delta_chunks_lowrank(
+                out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
+                bpre.data_ptr(), bpre.stride(0), decay.data_ptr(), p.data_ptr(), p.stride(0), w2t.data_ptr(), w2t.shape[0],
+                norm_w.data_ptr(), state.data_ptr(), state.stride(0), work.data_ptr(), raw.data_ptr(), T, heads, kv_heads, dim, vdim, eps,
+                *seq.args, _dt(q), _stream()), "sp_gated_delta_chunks_lowrank")
+            return out
         _check(load().sp_gated_delta_chunks(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                                             v.data_ptr(), v.stride(0), bpre.data_ptr(), bpre.stride(0), decay.data_ptr(),
                                             gate.data_ptr(), norm_w.data_ptr(), state.data_ptr(), state.stride(0),

@@ -324,6 +324,73 @@ gated_norm_kernel(void* out, int64_t out_stride, const float* raw, const float* 
   }
 }
 
+// The same with the gate sigmoid(p w2t) formed on the spot (bf16 rows, RANK 32 or 64, heads of 16 TILES values): a workgroup keeps its head's
+// columns of w2t in LDS as three bf16 parts each, in the order the matrix instructions take them, and a wave takes 16 tokens - a lane ends with 4
+// neighbouring channels of every tile of its token, the head's sum of squares is over the four lanes of a token.  Memory bounds it: read-outs
+// in, results out.  The gates as a launch of their own are written and read once more in fp32: 4096 tokens of 16 heads of 128, rank 64, 16.2 us
+// for the gates and 19.5 for the norm; together 20.6.
+constexpr int kGateNormWaves = 8;
+template <int RANK, int TILES>
+__global__ void __launch_bounds__(kGateNormWaves * 64)
+gated_norm_lowrank_kernel(char* out, int64_t out_stride, const float* raw, const char* p, int64_t p_stride, const float* w2t,
+                          const float* norm_w, int64_t T, int H, float eps) {
+  constexpr int Dv = TILES * 16, KS = RANK / 32, FRAGS = KS * TILES * 64;
+  __shared__ u32x4 parts[3][FRAGS];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, q = lane >> 4, h = blockIdx.y;
+  const int64_t channels = (int64_t)H * Dv, t = ((int64_t)blockIdx.x * kGateNormWaves + wave) * 16 + r16, tt = t < T ? t : T - 1;
+  // this wave's rows are on their way while the weights are split
+  f32x4_c o[TILES];
+  u32x4 x[KS];
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk) x[kk] = ld16(p + (tt * p_stride + 32 * kk + 8 * q) * 2);
+#pragma unroll
+  for (int i = 0; i < TILES; ++i) o[i] = *(const f32x4_c*)(raw + (tt * H + h) * Dv + 16 * i + 4 * q);
+  for (int f = tid; f < FRAGS; f += kGateNormWaves * 64) {
+    const int l = f & 63, i = (f >> 6) % TILES, kk = (f >> 6) / TILES;
+    const float* from = w2t + (int64_t)(32 * kk + 8 * (l >> 4)) * channels + h * Dv + 16 * i + (l & 15);
+    float w[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = from[e * channels];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t hi, mid, lo;
+      split3(w[2 * e], w[2 * e + 1], hi, mid, lo);
+      parts[0][f][e] = hi, parts[1][f][e] = mid, parts[2][f][e] = lo;
+    }
+  }
+  __syncthreads();
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < TILES; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ss += o[i][r] * o[i][r];
+  ss += __shfl_xor(ss, 16, 64);
+  ss += __shfl_xor(ss, 32, 64);
+  const float inv = 1.f / sqrtf(ss / (float)Dv + eps);
+#pragma unroll
+  for (int i = 0; i < TILES; ++i) {
+    f32x4_c z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+      for (int part = 2; part >= 0; --part) z = mfma_c(parts[part][(kk * TILES + i) * 64 + lane], x[kk], z);
+    const f32x4_c nw = *(const f32x4_c*)(norm_w + 16 * i + 4 * q);
+    float y[8] = {};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (!(fabsf(z[r]) < INFINITY)) {                 // an infinity's parts are not numbers: such a sum is formed again as it is
+        float sum = 0.f;
+        for (int k = 0; k < RANK; ++k)
+          sum += w2t[k * channels + h * Dv + 16 * i + 4 * q + r] * Elem<bf16_tag>::load(p, tt * p_stride + k);
+        z[r] = sum;
+      }
+      y[r] = o[i][r] * inv * nw[r] * gate_value<1>(z[r], 0.f);
+    }
+    const u32x4 two = pack16<bf16_tag>(y);
+    if (t < T) *(u32x2*)(out + (t * out_stride + h * Dv + 16 * i + 4 * q) * 2) = u32x2{two[0], two[1]};
+  }
+}
+
 template <typename Tag>
 static int launch_gated_delta(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
                               const void* v, int64_t v_stride, const void* bpre, int64_t b_stride, const float* decay,
@@ -419,14 +486,16 @@ extern "C" int sp_gated_delta_scan(void* out, int64_t out_stride, const void* q,
                                                            vdim, eps, (hipStream_t)stream)));
 }
 
-extern "C" int sp_gated_delta_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k,
-                                     int64_t k_stride, const void* v, int64_t v_stride, const void* bpre, int64_t b_stride,
-                                     const float* decay, const float* gate, const float* norm_w, float* state,
-                                     int64_t state_stride, float* work, float* raw, int64_t num_tokens, int heads, int kv_heads,
-                                     int dim, int vdim, float eps, SP_SEQ_PARAMS, int dtype, void* stream) {
+// (gate: the gates themselves; else p [T, rank] and w2t [rank, heads * vdim])
+static int gated_delta_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                              int64_t v_stride, const void* bpre, int64_t b_stride, const float* decay, const float* gate, const void* p,
+                              int64_t p_stride, const float* w2t, int rank, const float* norm_w, float* state, int64_t state_stride,
+                              float* work, float* raw, int64_t num_tokens, int heads, int kv_heads, int dim, int vdim, float eps,
+                              SP_SEQ_PARAMS, int dtype, void* stream) {
   SP_CHECK_ARG(batch_size >= 0 && num_tokens >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && dim > 0 && vdim > 0);
   if (batch_size == 0 || num_tokens == 0) return SP_OK;
-  SP_CHECK_ARG(out && q && k && v && bpre && decay && gate && norm_w && state && work && raw && req_pool_indices && seq_lens);
+  SP_CHECK_ARG(out && q && k && v && bpre && decay && (gate || (p && w2t && p_stride >= rank)) && norm_w && state && work && raw &&
+               req_pool_indices && seq_lens);
   SP_CHECK_ARG(!extend_seq_lens || (extend_prefix_lens && extend_start_loc));
   SP_CHECK_ARG(state_stride >= (int64_t)heads * dim * vdim);
   SP_CHECK_ARG(q_stride >= (int64_t)kv_heads * dim && k_stride >= (int64_t)kv_heads * dim && b_stride >= heads);
@@ -436,13 +505,52 @@ extern "C" int sp_gated_delta_chunks(void* out, int64_t out_stride, const void* 
   const DeltaChunks a{q, k, v, bpre, decay, nullptr, nullptr, nullptr, state, work, raw, q_stride, k_stride, v_stride, b_stride, 0,
                       state_stride, num_tokens, heads, kv_heads, vdim, vdim};
   if (!delta_chunks_take(a, dim, dtype, s)) return SP_ERR_UNSUPPORTED;
+  if (!gate && (dtype != SP_BF16 || (rank != 32 && rank != 64) || (vdim != 64 && vdim != 128) || p_stride % 8 != 0 || out_stride % 4 != 0 ||
+                ((((uintptr_t)p | (uintptr_t)raw | (uintptr_t)norm_w) & 15) | ((uintptr_t)out & 7)) || heads > 65535))
+    return SP_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
   int rc = SP_OK;
   SP_DISPATCH_DTYPE(dtype, rc = (dim == 64 ? launch_delta_chunks<Tag, 64, true>(a, s, st) : launch_delta_chunks<Tag, 128, true>(a, s, st)));
   if (rc != SP_OK) return rc;
+  if (!gate) {
+    const dim3 grid((unsigned)((num_tokens + 16 * kGateNormWaves - 1) / (16 * kGateNormWaves)), (unsigned)heads);
+#define SP_GN(R, TILES)                                                                                                         \
+  gated_norm_lowrank_kernel<R, TILES><<<grid, kGateNormWaves * 64, 0, st>>>((char*)out, out_stride, raw, (const char*)p, p_stride, \
+                                                                            w2t, norm_w, num_tokens, heads, eps)
+    if (rank == 64 && vdim == 128) SP_GN(64, 8);
+    else if (rank == 64) SP_GN(64, 4);
+    else if (vdim == 128) SP_GN(32, 8);
+    else SP_GN(32, 4);
+#undef SP_GN
+    SP_LAUNCH_CHECK();
+    return SP_OK;
+  }
   const int64_t jobs = num_tokens * heads;
   SP_DISPATCH_DTYPE(dtype, (gated_norm_kernel<Tag><<<dim3((unsigned)((jobs + kBlock / 64 - 1) / (kBlock / 64))), kBlock, 0, st>>>(
                                out, out_stride, raw, gate, norm_w, heads, vdim, eps, jobs)));
   SP_LAUNCH_CHECK();
   return SP_OK;
+}
+
+extern "C" int sp_gated_delta_chunks(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k,
+                                     int64_t k_stride, const void* v, int64_t v_stride, const void* bpre, int64_t b_stride,
+                                     const float* decay, const float* gate, const float* norm_w, float* state, int64_t state_stride, float* work, float* raw,
+                                     int64_t num_tokens, int heads, int kv_heads, int dim, int vdim, float eps, SP_SEQ_PARAMS, int dtype,
+                                     void* stream) {
+  SP_CHECK_ARG(gate || batch_size == 0 || num_tokens == 0);
+  return gated_delta_chunks(out, out_stride, q, q_stride, k, k_stride, v, v_stride, bpre, b_stride, decay, gate, nullptr, 0, nullptr, 0, norm_w, state,
+                            state_stride, work, raw, num_tokens, heads, kv_heads, dim, vdim, eps, req_pool_indices, seq_lens,
+                            extend_seq_lens, extend_prefix_lens, extend_start_loc, token_req, idx64, batch_size, dtype, stream);
+}
+
+extern "C" int sp_gated_delta_chunks_lowrank(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k,
+                                             int64_t k_stride, const void* v, int64_t v_stride, const void* bpre, int64_t b_stride,
+                                             const float* decay, const void* p, int64_t p_stride, const float* w2t, int rank,
+                                             const float* norm_w, float* state, int64_t state_stride, float* work, float* raw,
+                                             int64_t num_tokens, int heads, int kv_heads, int dim, int vdim, float eps, SP_SEQ_PARAMS, int dtype,
+                                             void* stream) {
+  SP_CHECK_ARG(rank > 0);
+  return gated_delta_chunks(out, out_stride, q, q_stride, k, k_stride, v, v_stride, bpre, b_stride, decay, nullptr, p, p_stride, w2t, rank, norm_w, state,
+                            state_stride, work, raw, num_tokens, heads, kv_heads, dim, vdim, eps, req_pool_indices, seq_lens,
+                            extend_seq_lens, extend_prefix_lens, extend_start_loc, token_req, idx64, batch_size, dtype, stream);
 }

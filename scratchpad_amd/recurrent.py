@@ -252,8 +252,7 @@ class GatedDeltaMixer(nn.Module):
         rows, b, a1, g1, _ = a.split_with_sizes([c, H, self.decay_rank, self.gate_rank, a.shape[1] - self.in_rows], 1)
         qkv = _native.causal_conv_silu(rows, self.conv.data, None, states.state(sid, "conv"), seq)
         decay = _native.lowrank_gate(a1, self.a2t.data, self.dt_bias.data, "decay", self.A_log.data)
-        gate = _native.lowrank_gate(g1, self.g2t.data, None, "sigmoid")
-        o = _native.gated_delta_scan(*qkv.split_with_sizes([nk, nk, c - 2 * nk], 1), b, decay, gate,
+        o = _native.gated_delta_scan(*qkv.split_with_sizes([nk, nk, c - 2 * nk], 1), b, decay, (g1, self.g2t.data),
                                      self.norm.data, states.state(sid, "S"), seq, H, self.kv_heads, self.dim, self.vdim,
                                      self.eps)
         return _native.linear(o, self.o)

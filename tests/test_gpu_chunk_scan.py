@@ -573,3 +573,31 @@ def test_segments_keep_a_number_that_is_not_finite_from_earlier_tokens(bad, monk
         cols = [3] if where == "value" else list(range(D))
         assert not torch.isfinite(S[0][:, cols]).any() and not torch.isfinite(S2[0][:, cols]).any()
         assert not torch.isfinite(out[at:].view(-1, H, D)[:, 0, cols].float()).any() and not torch.isfinite(y[at:].view(-1, H, D)[:, 0, cols]).any()
+
+
+@pytest.mark.parametrize("lens", [[20], [9, 130, 300], [128], [17] * 3], ids=lambda l: "-".join(map(str, l)))
+@pytest.mark.parametrize("H,D,Dv,rank", [(3, 128, 128, 64), (2, 64, 64, 64), (2, 128, 128, 32), (5, 64, 64, 32)])
+@pytest.mark.parametrize("spoiled", [False, True])
+def test_gated_delta_norm_forms_its_gates(lens, H, D, Dv, rank, spoiled, monkeypatch):
+    """the gate formed behind the norm against the gate as a step of its own: the same three-part product in another order, the same fp32
+    norm - one bf16 ulp where a rounding falls the other way; an infinite or undefined projection spoils its own token and head only"""
+    from scratchpad_amd import _native
+    announce("gated delta lowrank norm", lens, H, D, Dv, rank, spoiled)
+    monkeypatch.setattr(_native, "delta_chunks_pay", lambda *a: True)
+    g = torch.Generator(device=DEV).manual_seed(21)
+    T, slots = sum(lens), slots_of(lens)
+    q, k, v, bp, p = torch.randn(T, 2 * H * D + H * Dv + 8 * H + rank, generator=g, device=DEV).bfloat16().split([H * D, H * D, H * Dv, 8 * H, rank], 1)
+    bp, p = bp[:, :H], p.clone()
+    w2t = torch.randn(rank, H * Dv, generator=g, device=DEV) * rank ** -0.5 * 2
+    if spoiled:
+        p[3, 1], p[7, 0] = float("inf"), float("nan")
+        w2t[2, 5] = float("inf")
+    decay, nw = torch.rand(T, H * D, generator=g, device=DEV), torch.rand(Dv, generator=g, device=DEV) + 0.5
+    outs = []
+    for gate in ((p, w2t), _native.lowrank_gate(p, w2t, None, "sigmoid")):
+        S = torch.zeros(2 * len(lens) + 1, H, D, Dv, device=DEV)
+        outs.append(_native.gated_delta_scan(q, k, v, bp, decay, gate, nw, S, seq_extend(lens, [0] * len(lens), slots), H, H, D, Dv, 1e-5).float())
+    got, want = outs
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.isfinite(want).any()
+    ok = torch.isfinite(want)
+    assert ((got - want).abs()[ok] <= 2.0 ** -7 * want.abs()[ok] + 1e-6).all() and (got != want)[ok].float().mean() < 0.01
