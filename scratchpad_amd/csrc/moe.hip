@@ -260,7 +260,7 @@ moe_grouped_gemm_kernel(void* out, const void* a, const void* w, const int32_t* 
 // ---- the same product on the matrix cores (16-bit types, K a multiple of 32, 16-byte aligned rows) -------------------
 // v_mfma_f32_16x16x32: lane (r16 = lane & 15, q = lane >> 4) holds 8 k-values of row r16 of each operand and receives
 // D[4 q + r][r16], r < 4 - with the weights as the first operand a lane ends up with 4 neighbouring output columns of ONE
-// row.  The three kernels below (tile, wide, rows) add the k-steps of 32 in ascending order into one accumulator, so an output
+// row.  The kernels below (tile, wide, rows, narrow rows) add the k-steps of 32 in ascending order into one accumulator, so an output
 // element has the same bits whichever of them - and whichever tile height - computes it: a token's result does not depend on the
 // step's size.
 //
@@ -665,6 +665,52 @@ __global__ void __launch_bounds__(64) moe_grouped_rows_kernel(GroupedArgs p) {
   }
 }
 
+// The same with half the weight rows per wave (16; GLU: 8 gate rows and their 8 up rows) and twice the k-steps on their way, while
+// the kernel above would have at most two waves per SIMD (256 CUs of four; were every pair another expert's): the SIMDs that got
+// one wave more then set its time.  8 tokens, top 4 of 32 experts of 2048 x 1024: 33.8 + 18.2 us -> 32.4 + 16.3, the layer
+// 70.1 -> 66.5; 1024 x 512: 10.6 + 7.1 -> 10.3 + 6.7.  With two rows per expert the second reading of x's rows costs more than it
+// gives: 16 tokens 82.3 -> 90.7 (1024 x 512: 13.7 + 8.2 -> 14.6 + 7.9), 64 tokens 109 -> 113.
+constexpr long kNarrowWaves = 2 * 4 * 256;
+constexpr int kNarrowUnroll = 16;
+
+template <typename Tag, int ACT>
+__global__ void __launch_bounds__(64) moe_grouped_narrow_rows_kernel(GroupedArgs p) {
+  constexpr bool GLU = ACT >= 2;
+  const int lane = threadIdx.x, r16 = lane & 15, q = lane >> 4;
+  int e = 0, row0 = 0, rows_end = 0;
+  if (!grouped_tile(p.offsets, p.E, 16, (int)blockIdx.y, lane, e, row0, rows_end)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  const int n0 = blockIdx.x * (GLU ? 8 : 16);
+  const int pos = min(row0 + r16, rows_end - 1);                 // rows past the end: never stored
+  const int64_t arow = p.order ? p.order[pos] / p.row_div : pos;
+  const char* xp = p.a + (arow * p.a_stride + 8 * q) * 2;
+  const char* wp = p.w + ((int64_t)e * (GLU ? 2 * p.N : p.N) * p.K + 8 * q) * 2 +
+                   (int64_t)(GLU ? (r16 >> 3) * p.N + min(n0 + (r16 & 7), p.N - 1) : min(n0 + r16, p.N - 1)) * p.K * 2;
+  f32x4_q acc = {0.f, 0.f, 0.f, 0.f};
+  const int ksteps = p.K / 32;
+  int ks = 0;
+  for (; ks + kNarrowUnroll <= ksteps; ks += kNarrowUnroll) {
+    u32x4 wf[kNarrowUnroll], xf[kNarrowUnroll];
+#pragma unroll
+    for (int u = 0; u < kNarrowUnroll; ++u) {
+      wf[u] = ld16(wp + (ks + u) * 64);
+      xf[u] = ld16(xp + (ks + u) * 64);
+    }
+    __builtin_amdgcn_sched_barrier(0);      // all loads of the round first: the scheduler would trade them for registers
+#pragma unroll
+    for (int u = 0; u < kNarrowUnroll; ++u) acc = mfma_q<Tag>(wf[u], xf[u], acc);
+  }
+  for (; ks < ksteps; ++ks) acc = mfma_q<Tag>(ld16(wp + ks * 64), ld16(xp + ks * 64), acc);
+  float v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float up = GLU ? __shfl_xor(acc[r], 32, 64) : 0.f;     // (gates in the lanes below 32, their up sums 32 above)
+    v[r] = grouped_act<Tag, ACT>(acc[r], up, p);
+  }
+  if (row0 + r16 >= rows_end || (GLU && lane >= 32)) return;
+  store4<Tag>(p, row0 + r16, n0 + 4 * q, v);
+}
+
 // Which kernel: by the mean rows per expert, pairs / experts (the counts themselves are on the device).  Measured at width 2048,
 // 32 experts of ff 1024, top 4, up + down product in us (rows kernel | 64-row tiles | 128-row tiles):
 //   mean rows 1: 60 | 68 | 73     4: 85 | 92 | 94     8: 86 | 92 | 94     16: 104 | 93 | 96     32: 161 | 95 | 99
@@ -680,8 +726,12 @@ int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
   const int row_tiles = pairs / 16 + held;
   // (moe_align takes 4096 experts, 6656 tiles; more than a grid's second dimension holds go to the 64-row tiles)
   if (pairs <= 10 * (int64_t)p.E && row_tiles <= 65535) {
-    const int per = ACT >= 2 ? 16 : 32;
-    moe_grouped_rows_kernel<Tag, ACT><<<dim3((unsigned)((p.N + per - 1) / per), (unsigned)row_tiles), 64, 0, st>>>(p);
+    const int wide_per = ACT >= 2 ? 16 : 32;
+    const bool narrow = pairs <= p.E && (long)pairs * ((p.N + wide_per - 1) / wide_per) <= kNarrowWaves;
+    const int per = narrow ? wide_per / 2 : wide_per;
+    const dim3 grid((unsigned)((p.N + per - 1) / per), (unsigned)row_tiles);
+    if (narrow) moe_grouped_narrow_rows_kernel<Tag, ACT><<<grid, 64, 0, st>>>(p);
+    else moe_grouped_rows_kernel<Tag, ACT><<<grid, 64, 0, st>>>(p);
     SP_LAUNCH_CHECK();
     return SP_OK;
   }

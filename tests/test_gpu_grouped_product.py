@@ -22,7 +22,8 @@ def grouped_inputs(counts, N, K, dtype, top, seed=0):
 
 
 COUNTS = [[1], [0, 3, 0, 17], [16, 0, 15, 33], [63, 64, 65, 1], [127, 128, 129, 257, 0], [300, 2, 140], [3] * 70, [90] * 67 + [0, 1],
-          [321], [0, 385, 700, 129], [1100] + [1] * 2]
+          [321], [0, 385, 700, 129], [1100] + [1] * 2,
+          [2, 0, 1, 0, 1], [0] * 66 + [17, 1, 0, 40]]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
