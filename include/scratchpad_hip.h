@@ -61,7 +61,9 @@ SP_API const char* sp_status_string(int status);
  * 0 = never; without it mode 1 of "extend_w64" means mean extend length >= 768 or a cached prefix >= 1024
  * tokens; the two forms agree bit for bit), "decode_ranges" (0 = decode launches never take the range geometry of
  * their plan: the (request, split) items everywhere; -1 = the default, wherever the range kernel applies),
- * "decode_nt_min_mb" (see sp_decode_attention), "ar_fused_blocks".  Nothing on the call path reads the environment.  Returns
+ * "extend_small" (16-bit extend launches that leave compute units idle: 0 = the form by their size, the default; 1 = as all others;
+ * 2 = four waves per half row block where that form exists; n > 2 = every row block's keys shared by n - 1 workgroups where the
+ * workspace allows it), "decode_nt_min_mb" (see sp_decode_attention), "ar_fused_blocks".  Nothing on the call path reads the environment.  Returns
  * SP_ERR_INVALID_ARG for an unknown key.                                                          */
 SP_API int sp_debug_set(const char* key, int value);
 /* Read-only counterpart (ABI 6): "w64_descriptor_patched" (1 = extend_w64.hip was built in stages with its kernels'
@@ -260,7 +262,9 @@ SP_API int sp_decode_attention(void* out, const void* q, const void* k_buffer, c
  * q,o: [T, Hq, D]; extend_* are int32 [bs].  Hq / Hkv: any width for fp16/bf16, 1/2/4/8 for fp32.
  * num_tokens = sum(extend_seq_lens) (host-known: ForwardBatch.extend_num_tokens) and
  * max_extend_len >= max(extend_seq_lens), max_seq_len >= max(seq_lens) fix the launch geometry.
- * workspace: sp_extend_attention_workspace_bytes().                                              */
+ * workspace: sp_extend_attention_workspace_bytes(); one launch at a time (two streams: one each).  16-bit launches with
+ * fewer row blocks than half the compute units, and not a case of the 4-wave x 64-row kernel, share a block's keys over workgroups, whose 32-bit partial sums go there (the
+ * other sums' order differs in the last bits); 12 bytes per token + 64 are accepted too: nothing is shared then. */
 SP_API size_t sp_extend_attention_workspace_bytes(int64_t num_tokens, int batch_size, int num_q_heads,
                                            int head_dim, int dtype);
 /* `plan` (optional, may be NULL): the step's (request, row block) work items, heaviest first, built once

@@ -23,7 +23,10 @@ int run_extend_mfma(void* out, const void* q, const void* k_buffer, const void* 
                     int batch_size, int num_q_heads, int num_kv_heads, int head_dim, int64_t q_stride,
                     int64_t out_stride, int64_t kv_buffer_stride, float sm_scale, float logit_cap,
                     float out_scale, int causal, int window_left, int max_extend_len, int64_t max_seq_len,
-                    const int32_t* plan, int plan_items, int num_tokens, int dtype, int kv8, hipStream_t st);
+                    const int32_t* plan, int plan_items, int num_tokens, int dtype, int kv8, void* workspace, size_t workspace_bytes,
+                    hipStream_t st);
+// bytes of workspace with which a launch of this size can share its row blocks' keys over workgroups; 0: it never would
+size_t extend_split_bytes(int64_t num_tokens, int num_q_heads, int head_dim);
 
 // extend_w64.hip: the 4-wave x 64-row form of the same kernel (16-bit, D = 128, plain attention, query-head group a
 // multiple of 4); returns 1 (one workgroup per item) or 2 (persistent workgroups) when it took the launch, 0 otherwise.
@@ -40,6 +43,9 @@ int w64_descriptor_patched();
 
 // test / tuning hooks behind sp_debug_set
 void set_extend_defer_x10(int tenths);
+// launches that leave compute units idle: 0 by their size (default), 1 as all others, 2 four waves per half row block where that form
+// exists, n > 2 every row block's keys shared by n - 1 workgroups where the workspace allows it
+void set_extend_small(int v);
 void set_extend_dma(int v);   // 0: register-staged K/V tiles for every shape (the LDS-DMA ring is the default where it applies)
 
 }  // namespace sp

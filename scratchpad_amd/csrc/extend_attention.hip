@@ -162,6 +162,7 @@ extern "C" int sp_debug_set(const char* key, int value) {
   if (!strcmp(key, "decode_nt_min_mb")) { set_decode_nt_min_mb(value); return SP_OK; }
   if (!strcmp(key, "decode_ranges")) { set_decode_ranges(value); return SP_OK; }
   if (!strcmp(key, "extend_defer_x10")) { set_extend_defer_x10(value); return SP_OK; }
+  if (!strcmp(key, "extend_small")) { set_extend_small(value); return SP_OK; }
   if (!strcmp(key, "extend_dma")) { set_extend_dma(value); return SP_OK; }
   if (!strcmp(key, "extend_w64")) { set_extend_w64(value); return SP_OK; }
   if (!strcmp(key, "extend_w64_persist")) { set_extend_w64_persist(value); return SP_OK; }
@@ -190,9 +191,10 @@ extern "C" SP_API int sp_debug_extend_stamp_buffer(void* device_u64x8) {
 
 extern "C" size_t sp_extend_attention_workspace_bytes(int64_t num_tokens, int batch_size,
                                                       int num_q_heads, int head_dim, int dtype) {
-  (void)batch_size; (void)num_q_heads; (void)head_dim; (void)dtype;
+  (void)batch_size;
   if (num_tokens <= 0) return 16;
-  return (size_t)num_tokens * 3 * sizeof(int32_t) + 64;
+  const size_t rows = (size_t)num_tokens * 3 * sizeof(int32_t) + 64;
+  return dtype == SP_F32 ? rows : std::max(rows, extend_split_bytes(num_tokens, num_q_heads, head_dim));
 }
 
 extern "C" int sp_extend_attention(void* out, const void* q, const void* k_buffer,
@@ -228,8 +230,7 @@ extern "C" int sp_extend_attention(void* out, const void* q, const void* k_buffe
   const int vec = dtype == SP_F32 ? 4 : 8;
   SP_CHECK_ARG(q_stride % vec == 0 && kv_buffer_stride % vec == 0);
   if (num_tokens > 0x7fffffffLL / 64) return SP_ERR_INVALID_ARG;
-  const size_t need =
-      sp_extend_attention_workspace_bytes(num_tokens, batch_size, num_q_heads, head_dim, dtype);
+  const size_t need = (size_t)num_tokens * 3 * sizeof(int32_t) + 64;   // (less than asked for: no keys shared over workgroups)
   if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15)) return SP_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   // a plan must be large enough for every grid row this launch reads an item for (its CONTENT is checked by
@@ -247,7 +248,7 @@ extern "C" int sp_extend_attention(void* out, const void* q, const void* k_buffe
                                    causal, window_left, max_extend_len, max_seq_len, plan,
                                    (int)std::min<int64_t>(extend_plan_items(num_tokens, batch_size,
                                        extend_block_rows(num_q_heads, num_kv_heads)), 0x7fffffff),
-                                   (int)num_tokens, dtype, kv8 ? 1 : 0, st);
+                                   (int)num_tokens, dtype, kv8 ? 1 : 0, workspace, workspace_bytes, st);
     if (rc != SP_ERR_UNSUPPORTED || kv8) return rc;   // an fp8 pool has no row-stream path
   }
 

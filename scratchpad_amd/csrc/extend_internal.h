@@ -41,7 +41,38 @@ struct ExtendArgs {
   const int32_t* plan;
   int plan_items;       // grid rows when a plan is given (an upper bound of its count)
   int num_tokens;       // sum of the extend lengths (host-known)
+  // keys of a row block shared by `splits` workgroups (1: none): each leaves its unnormalised O^T tile and the rows' maximum and sum
+  // in 32 bits, tile ((item * gridDim.x + kv-head group) * waves + wave) * splits + split, for extend_merge_kernel
+  int splits;
+  int half_blocks;      // 1: a workgroup of four waves takes half a row block (heads of 64)
+  float* part_o;        // per tile: [D / 4][32 rows][4]
+  float* part_ml;       // per tile: 32 maxima (log2 domain), 32 sums
 };
+
+// the (request, first row) of item `y` of a step without a list of this launch's own: the requests' row blocks, last rows first
+__device__ __forceinline__ bool extend_walk_item(const ExtendArgs& a, int block_rows, int y, int& b, int& row0) {
+  int rem = y, nblk = 0;
+  for (b = 0; b < a.bs; ++b) {
+    const int e = a.ext_lens[b];
+    nblk = e > 0 ? (e + block_rows - 1) / block_rows : 0;
+    if (rem < nblk) break;
+    rem -= nblk;
+  }
+  if (b >= a.bs) return false;
+  row0 = (nblk - 1 - rem) * block_rows;
+  return true;
+}
+
+// item `y` out of the plan where it was built for this launch's shape, else by the walk (same results, no ordering)
+__device__ __forceinline__ bool extend_item(const ExtendArgs& a, int block_rows, int y, int& b, int& row0) {
+  const bool mine = a.plan && a.plan[1] == block_rows && a.plan[2] == a.Hq && a.plan[3] == a.Hkv && a.plan[4] == a.num_tokens &&
+                    a.plan[5] == a.bs;
+  if (!mine) return extend_walk_item(a, block_rows, y, b, row0);
+  if (y >= a.plan[0]) return false;
+  b = a.plan[kExtPlanHeader + 2 * y];
+  row0 = a.plan[kExtPlanHeader + 1 + 2 * y] * block_rows;
+  return true;
+}
 
 static constexpr float kLog2eX = 1.4426950408889634f;
 static constexpr float kNegBigX = -1.0e30f;

@@ -65,10 +65,19 @@ __device__ unsigned long long* g_stamp_buf = nullptr;
 #define SP_STAMP_ACC(slot, from, to) do { } while (0)
 #endif
 
+typedef float f32x4_x __attribute__((ext_vector_type(4)));
+
+// this wave's tile of the shares (ExtendArgs::splits)
+__device__ __forceinline__ int64_t split_tile(const ExtendArgs& a, int wave) {
+  return (((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 8 + wave) * a.splits + blockIdx.z;
+}
+
 // PLAIN: no logit cap and no sliding window (both compiled out of the tile loop)
-template <typename Tag, int D, int GK, int NW, bool KV8, bool PLAIN, bool DMA>
+// SPLIT: the row block's tiles are shared by a.splits workgroups (blockIdx.z), see ExtendArgs::splits
+template <typename Tag, int D, int GK, int NW, bool KV8, bool PLAIN, bool DMA, bool SPLIT = false>
 __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
-  static_assert(!DMA || ((D == 128 || D == 64) && !KV8 && NW == 8), "the LDS-DMA images are laid out for 256- / 128-byte rows and 8 waves");
+  static_assert(!DMA || ((D == 128 || D == 64) && !KV8), "the LDS-DMA images are laid out for 256- / 128-byte rows");
+  static_assert(NW == 8 || (NW == 4 && D == 64 && !SPLIT), "a row block of 8 waves, or one half of it");
   constexpr int NT = NW * 64;
   constexpr int NB = 2;                // LDS tile buffers: tile t lives in buffer t & 1
   typedef ExtCfg<D, NT> C;
@@ -84,30 +93,16 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
 #endif
 
   int b, row0;
-  if (a.plan) {                                    // planned: items are sorted heaviest first
-    const bool mine = a.plan[1] == BM && a.plan[2] == a.Hq && a.plan[3] == a.Hkv && a.plan[4] == a.num_tokens &&
-                      a.plan[5] == a.bs;
-    if (mine) {
-      if ((int)blockIdx.y >= a.plan[0]) return;
-      b = a.plan[kExtPlanHeader + 2 * blockIdx.y];
-      row0 = a.plan[kExtPlanHeader + 1 + 2 * blockIdx.y] * BM;
-    } else {
-      // a plan built for another block size, other head counts or another step: walk the requests for
-      // grid row blockIdx.y (the grid has a row for every item of THIS step); same results, no ordering
-      int rem = blockIdx.y, nblk = 0;
-      for (b = 0; b < a.bs; ++b) {
-        const int e = a.ext_lens[b];
-        nblk = e > 0 ? (e + BM - 1) / BM : 0;
-        if (rem < nblk) break;
-        rem -= nblk;
-      }
-      if (b >= a.bs) return;
-      row0 = (nblk - 1 - rem) * BM;
-    }
+  // four waves: blockIdx.z names the half of the 8-wave row block
+  constexpr int HALVES = 8 / NW;
+  const int half = HALVES == 1 ? 0 : (int)blockIdx.z % HALVES;
+  if (SPLIT || a.plan) {                           // planned: items are sorted heaviest first
+    if (!extend_item(a, BM * HALVES, (int)blockIdx.y, b, row0)) return;
   } else {
-    b = blockIdx.z;
-    row0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * BM;    // heaviest row blocks first
+    b = blockIdx.z / HALVES;
+    row0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * (BM * HALVES);    // heaviest row blocks first
   }
+  row0 += half * BM;
   const int E = a.ext_lens[b];
   if (row0 >= E) return;
   const int G = a.Hq / a.Hkv;
@@ -122,10 +117,15 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
   const int64_t t0 = a.ext_start[b];
   // keys this workgroup can see: the prefix and new tokens up to its last row (causal), else all
   const int kv_len = a.causal ? min(L, P + min(row0 + BM, E)) : L;
-  const int ntiles = (kv_len + BN - 1) / BN;
+  int ntiles = (kv_len + BN - 1) / BN;
   // sliding window (causal only): the first row of the block reaches furthest back
   const bool windowed = !PLAIN && a.causal && a.window >= 0;
-  const int tbeg = windowed ? max(0, P + row0 - a.window) / BN : 0;
+  int tbeg = windowed ? max(0, P + row0 - a.window) / BN : 0;
+  if constexpr (SPLIT) {                           // this workgroup's share: equal parts of the row block's own tiles
+    const int n = max(ntiles - tbeg, 0), part = blockIdx.z;
+    ntiles = tbeg + (int)((int64_t)n * (part + 1) / a.splits);
+    tbeg += (int)((int64_t)n * part / a.splits);
+  }
   SP_WGSTAMP(wg1);
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -138,7 +138,13 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
   if (ntiles <= tbeg) {
     // no key at all (a request without encoder tokens): zeros, and no look at req_to_token, whose row
     // need not hold a valid slot then.  Workgroup-uniform: taken before the first barrier.
-    if (my_row < E && wave_live) {
+    if constexpr (SPLIT) {
+      if (wave_live && h == 0) {
+        float* ml = a.part_ml + split_tile(a, wave) * 64;
+        ml[c] = kNegBigX;
+        ml[32 + c] = 0.f;
+      }
+    } else if (my_row < E && wave_live) {
       char* op = (char*)a.out + ((t0 + my_row) * a.o_stride + (int64_t)head * D) * 2;
       for (int d = 4 * h; d < D; d += 8) *(u32x2*)(op + d * 2) = u32x2{0u, 0u};
     }
@@ -243,7 +249,8 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
   constexpr int kDmaBufs = 4;   // tile t is consumed from buffer t % 4 while t+1, t+2 and t+3 are in flight
   constexpr int kCPR = kRowB / 16;                   // 16-byte chunks per row (16 / 8)
   constexpr int kRPP = 64 / kCPR;                    // rows per DMA piece (4 / 8)
-  constexpr int kPPW = 8 / kRPP;                     // pieces per wave and tile, each for K and for V (2 / 1)
+  constexpr int kRPW = 64 / NW;                      // rows a wave fetches of every tile
+  constexpr int kPPW = kRPW / kRPP;                  // its pieces, each for K and for V (8 waves: 2 / 1, 4 waves: 2 at D = 64)
   const int k_swz = D == 128 ? ((c & 15) ^ h) : (((c >> 1) & 7) ^ h);
   // pipeline: the gathers of tiles t+1 and t+2 fly during compute(t); tile t+1 is written to the other
   // LDS buffer right after compute(t), and one barrier per tile both publishes tile t+1 and retires
@@ -452,20 +459,20 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
     auto load_slots = [&](Slots& r, int tile) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < kPPW; ++j) {
-        const int key = tile * BN + wave * 8 + kRPP * j + dR;
+        const int key = tile * BN + wave * kRPW + kRPP * j + dR;
         r.s[j] = idx_row[max(min(key, kv_len - 1), 0)];   // see fetch_slots
       }
     };
     auto dma = [&](const Slots& r, int buf) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < kPPW; ++j) {
-        const int R = wave * 8 + kRPP * j + dR;
+        const int R = wave * kRPW + kRPP * j + dR;
         const int64_t off = (int64_t)r.s[j] * tok_bytes + row_off;
         const int fk = D == 128 ? (R & 15) : ((R >> 1) & 7);
         const int fv = D == 128 ? ((R & 3) << 2) : (((R >> 1) & 1) << 2);
         const char* ks = a.kbuf + off + ((dp ^ fk) << 4);
         const char* vs = a.vbuf + off + ((dp ^ fv) << 4);
-        char* kd = lds + buf * kDmaTile + (wave * 8 + kRPP * j) * kRowB;
+        char* kd = lds + buf * kDmaTile + (wave * kRPW + kRPP * j) * kRowB;
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)ks,
                                          (__attribute__((address_space(3))) void*)kd, 16, 0, 0);
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)vs,
@@ -605,6 +612,26 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
   // tile ring is free by now: barrier first, every wave has left it and drained its DMA) and leaves as
   // whole rows, 16 bytes per lane, 4 rows of 256 B per store instruction.
   const float l_run = l_part + xchg32(l_part);
+  if constexpr (SPLIT) {
+    // (the accumulators as they lie: every store writes two runs of 512 bytes; rows past the request's end are never read back)
+    if (wave_live) {
+      const int64_t tile = split_tile(a, wave);
+      f32x4_x* po = (f32x4_x*)(a.part_o + tile * (32 * D)) + h * 32 + c;
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+        for (int quad = 0; quad < 4; ++quad) {
+          const f32x4_x v = {oacc[db][4 * quad], oacc[db][4 * quad + 1], oacc[db][4 * quad + 2], oacc[db][4 * quad + 3]};
+          po[(db * 8 + quad * 2) * 32] = v;
+        }
+      if (h == 0) {
+        float* ml = a.part_ml + tile * 64;
+        ml[c] = m_run;
+        ml[32 + c] = l_run;
+      }
+    }
+    return;
+  }
   __syncthreads();
   {
     constexpr int EPS = C::ROW_B + 8;                   // padded row: the 8-byte writes of 16 lanes hit 32 different banks
@@ -648,6 +675,60 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
 #endif
 }
 
+// The shares of a row block (ExtendArgs::splits) become its output: a workgroup takes one wave's 32 rows of one query head, weighs the
+// shares' sums by the distance of their maxima and writes whole rows (through LDS).  Reads 32 bits per value and share; two shares of
+// 777 tokens x 32 heads of 64 (15.7 MB) in 5.8 us; what it reads was written a moment ago and lies in the caches.
+template <typename Tag, int D, int GK>
+__global__ __launch_bounds__(256) void extend_merge_kernel(ExtendArgs a) {
+  constexpr int NW = 8, BM = 32 * (NW / GK), QPT = 32 * D / 4 / 256, PITCH = 2 * D + 8;
+  __shared__ __attribute__((aligned(16))) char rows[32 * PITCH];
+  int b, row0;
+  if (!extend_item(a, BM, (int)blockIdx.y, b, row0)) return;
+  const int E = a.ext_lens[b], wave = blockIdx.z, tid = threadIdx.x;
+  const int r0 = row0 + wave / GK * 32;
+  if (r0 >= E) return;
+  const int G = a.Hq / a.Hkv, halves = G / GK;
+  const int head = (int)blockIdx.x / halves * G + (int)blockIdx.x % halves * GK + wave % GK;
+  const int64_t tile = (((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * NW + wave) * a.splits;
+  const float* ml = a.part_ml + tile * 64;
+  const int c = tid & 31;
+  // a share without a visible key for the row counts for nothing, and what it left in part_o is not looked at
+  float top = kNegBigX;
+  for (int s = 0; s < a.splits; ++s)
+    if (as_u32(ml[s * 64 + 32 + c]) != 0u) top = fmaxf(top, ml[s * 64 + c]);
+  f32x4_x acc[QPT];
+#pragma unroll
+  for (int i = 0; i < QPT; ++i) acc[i] = f32x4_x{0.f, 0.f, 0.f, 0.f};
+  float sum = 0.f;
+  const f32x4_x* po = (const f32x4_x*)(a.part_o + tile * (32 * D)) + tid;
+  for (int s = 0; s < a.splits; ++s) {
+    const float l = ml[s * 64 + 32 + c];
+    if (as_u32(l) == 0u) continue;
+    const float w = __builtin_amdgcn_exp2f(ml[s * 64 + c] - top);
+    sum = __builtin_fmaf(l, w, sum);
+#pragma unroll
+    for (int i = 0; i < QPT; ++i) acc[i] += po[s * (8 * D) + i * 256] * w;
+  }
+  const float inv = as_u32(sum) != 0u ? a.out_scale / sum : 0.f;   // no visible key (empty encoder): zeros
+#pragma unroll
+  for (int i = 0; i < QPT; ++i) {
+    u32x2 v;
+    v[0] = pack2<Tag>(acc[i][0] * inv, acc[i][1] * inv);
+    v[1] = pack2<Tag>(acc[i][2] * inv, acc[i][3] * inv);
+    *(u32x2*)(rows + c * PITCH + ((tid >> 5) + 8 * i) * 8) = v;
+  }
+  __syncthreads();
+  constexpr int LPR = D / 8;                            // lanes per output row
+  const int64_t t0 = a.ext_start[b];
+#pragma unroll
+  for (int i = 0; i < 32 * LPR / 256; ++i) {
+    const int rr = (tid + i * 256) / LPR, ch = tid % LPR;
+    if (r0 + rr >= E) continue;
+    const u32x2 lo = *(const u32x2*)(rows + rr * PITCH + ch * 16), hi = *(const u32x2*)(rows + rr * PITCH + ch * 16 + 8);
+    st16((char*)a.out + ((t0 + r0 + rr) * a.o_stride + (int64_t)head * D) * 2 + ch * 16, u32x4{lo[0], lo[1], hi[0], hi[1]});
+  }
+}
+
 // test hook (set through sp_debug_set, never read from the environment on the call path): how far the
 // running maximum may trail (log2 units); < 0 restores the shipped value.  tests compare 0 (rescale at
 // every growth of a row maximum) with the shipped threshold.
@@ -665,6 +746,10 @@ void set_extend_dma(int v) { g_extend_dma = v; }
 int g_extend_last_kernel = 0;
 
 constexpr int kExtendWaves = 8;
+constexpr int kSplitGroups = 256, kMaxSplits = 16;
+
+static int g_extend_small = 0;
+void set_extend_small(int v) { g_extend_small = v; }
 
 // row blocks per workgroup tile for a query-head group of width G (any G: Gk = the largest of 4, 2, 1
 // that divides it; the remaining G / Gk head blocks become extra workgroups)
@@ -673,12 +758,103 @@ int extend_block_rows(int num_q_heads, int num_kv_heads) {
   return 32 * (kExtendWaves / extend_gk(num_q_heads / num_kv_heads));
 }
 
+// one tile (a wave's 32 rows) of one share
+static size_t split_tile_bytes(int head_dim) { return (size_t)(32 * head_dim + 64) * sizeof(float); }
+
+size_t extend_split_bytes(int64_t num_tokens, int num_q_heads, int head_dim) {
+  if (num_q_heads <= 0 || (head_dim != 64 && head_dim != 128)) return 0;
+  const int64_t groups = num_tokens * num_q_heads / (32 * kExtendWaves);   // at least; every grouping of heads has as many
+  if (2 * groups > kSplitGroups) return 0;
+  return (size_t)kSplitGroups * kExtendWaves * split_tile_bytes(head_dim);
+}
+
+// The form of a launch whose row blocks leave compute units idle (at most half as many workgroups as there are; plain attention).
+// A row block costs its workgroup about a + t * tiles, t = 1.05 us per 64-key tile at heads of 64 (vector work of two waves per SIMD), 1.15 - 1.35
+// at 128.  Two ways to use the idle units:
+//   * half_blocks (heads of 64): four waves take half a row block, one wave per SIMD, 0.8 us per tile, same bits, twice the workgroups;
+//   * splits: workgroups share the block's keys, t * tiles / splits, and pay for the partial sums (5 us for the merge, and their traffic).
+// Taken is the one that this model puts ahead, in ns (us at one form for all | half blocks | two | four | eight shares; 16-bit pool):
+//   heads of 64, 32 on 8:   3 requests, 777 tokens behind 1500: 37.3 | 29.0 | 29.0        1, 64 behind 2000:  38.9 | 31.5 | 25.5 | 18.1 | 16.1
+//                           1, 1024 behind 2000: 55.3 | 49.5 | 40.7                       2, 200 behind 500:  15.8 | 13.6 | 14.6 | 14.3 | 14.7
+//                           1, 512: 13.6 | 11.6 | 13.9                                    1, 1024: 22.5 | 18.6 | 21.7
+//   heads of 128, byte pool:  1, 17 behind 2000: 41.6 | - | 28.0 | 19.9 | 17.7            3, 777 behind 1500: 54.6 | - | 44.2
+//                           1, 1024 behind 2000: 86.5 | - | 64.7                          1, 1024: 34.3 | - | 33.2 (not taken)
+// What the 4 x 64-row kernel applies to stays whole: its forms and this file's agree to the bit, whichever of them a size selects.
+// With more than half of the units busy the same forms lose: 4 requests, 2048 tokens behind 1500, heads of 64: 45 | 46; 4096 tokens: 90 | 102.
+static void extend_small_form(ExtendArgs& a, int head_dim, int64_t max_seq_len, void* workspace, size_t workspace_bytes) {
+  a.splits = 1;
+  a.half_blocks = 0;
+  const int G = a.Hq / a.Hkv, gk = extend_gk(G), gx = a.Hkv * (G / gk), rows = 32 * (kExtendWaves / gk);
+  // (every request's last block may be short: no plan has more items)
+  const int64_t items = ((int64_t)a.num_tokens + (int64_t)a.bs * (rows - 1)) / rows, groups = items * gx;
+  if (a.window >= 0 || a.logit_cap > 0.f || g_extend_small == 1) return;
+  if (head_dim == 128 && !a.kv8 && G % 4 == 0) return;
+  if (groups <= 0 || items > 65535 || (2 * groups > kSplitGroups && g_extend_small <= 1)) return;
+  const int64_t fit = (int64_t)(workspace_bytes / (split_tile_bytes(head_dim) * kExtendWaves)) / groups;
+  int64_t s = std::min<int64_t>(std::min<int64_t>(kSplitGroups / groups, max_seq_len / 256), kMaxSplits);
+  if (g_extend_small > 1) s = g_extend_small - 1;
+  s = std::min(s, fit);
+  const int64_t tiles = max_seq_len / 64, alone = head_dim == 64 ? 800 : 1350, shared = head_dim == 64 ? 1050 : 1150;
+  if (tiles < 2 && !g_extend_small) return;
+  if (s > 1 && (g_extend_small > 2 || tiles * (alone - shared / s) > 5000 + (head_dim == 64 ? 20 : 40) * groups * s)) {
+    a.splits = (int)s;
+    a.plan_items = (int)items;
+    a.part_o = (float*)workspace;
+    a.part_ml = a.part_o + groups * kExtendWaves * s * 32 * head_dim;
+  }
+  else if (head_dim == 64 && (a.kv8 || g_extend_dma) && a.bs < 32768) a.half_blocks = 1;
+}
+
+#define SP_EXT_SET_LDS(KERNEL, BYTES)                                                                              \
+  do {                                                                                                           \
+    static bool attr_set = false; /* benign race: idempotent */                                                  \
+    if (!attr_set && (BYTES) > 64 * 1024) {                                                                      \
+      (void)hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);         \
+      attr_set = true;                                                                                           \
+    }                                                                                                            \
+  } while (0)
+
+template <typename Tag, int D, int GK>
+static int launch_splits(const ExtendArgs& a, int halves, hipStream_t st) {
+  constexpr int NW = kExtendWaves, kDma = 8 * 64 * 2 * D, kStaged = 2 * ExtCfg<D, NW * 64>::kTileBytes;
+  const dim3 grid(a.Hkv * halves, a.plan_items, a.splits);
+#define SP_EXT_SPLITS(KV8_, DMA_, BYTES)                                                                           \
+  do {                                                                                                           \
+    constexpr auto kernel = extend_mfma_kernel<Tag, D, GK, NW, KV8_, true, DMA_, true>;                          \
+    SP_EXT_SET_LDS(kernel, BYTES);                                                                               \
+    kernel<<<grid, NW * 64, BYTES, st>>>(a);                                                                     \
+  } while (0)
+  if (a.kv8) SP_EXT_SPLITS(true, false, kStaged);
+  else if (g_extend_dma) SP_EXT_SPLITS(false, true, kDma);
+  else SP_EXT_SPLITS(false, false, kStaged);
+#undef SP_EXT_SPLITS
+  SP_LAUNCH_CHECK();
+  extend_merge_kernel<Tag, D, GK><<<dim3(grid.x, grid.y, NW), 256, 0, st>>>(a);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
+
+template <typename Tag, int GK>
+static int launch_half_blocks(const ExtendArgs& a, int max_extend_len, int halves, hipStream_t st) {
+  constexpr int D = 64, NW = 4, rows = 32 * (kExtendWaves / GK), kDma = 8 * 64 * 2 * D, kStaged = 2 * ExtCfg<D, NW * 64>::kTileBytes;
+  const dim3 grid(a.Hkv * halves, a.plan ? a.plan_items : (max_extend_len + rows - 1) / rows, 2 * (a.plan ? 1 : a.bs));
+  if (a.kv8) extend_mfma_kernel<Tag, D, GK, NW, true, true, false><<<grid, NW * 64, kStaged, st>>>(a);
+  else extend_mfma_kernel<Tag, D, GK, NW, false, true, true><<<grid, NW * 64, kDma, st>>>(a);
+  static_assert(kDma <= 64 * 1024 && kStaged <= 64 * 1024, "LDS without an attribute");
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
+
 template <typename Tag, int D, int GK>
 static int launch_extend(const ExtendArgs& a, int max_extend_len, int halves, hipStream_t st) {
   constexpr int NW = kExtendWaves;
   typedef ExtCfg<D, NW * 64> C;
   constexpr int BM = 32 * (NW / GK);
   constexpr int kLds = 2 * C::kTileBytes;
+  if (a.splits > 1) return launch_splits<Tag, D, GK>(a, halves, st);
+  if constexpr (D == 64) {
+    if (a.half_blocks) return launch_half_blocks<Tag, GK>(a, max_extend_len, halves, st);
+  }
   // with a plan: one grid row per (request, row block) item, heaviest first; without: every
   // request x every possible row block (workgroups past a request's end exit at once)
   const dim3 grid(a.Hkv * halves, a.plan ? a.plan_items : (max_extend_len + BM - 1) / BM, a.plan ? 1 : a.bs);
@@ -723,7 +899,8 @@ int run_extend_mfma(void* out, const void* q, const void* k_buffer, const void* 
                     int batch_size, int num_q_heads, int num_kv_heads, int head_dim, int64_t q_stride,
                     int64_t out_stride, int64_t kv_buffer_stride, float sm_scale, float logit_cap,
                     float out_scale, int causal, int window_left, int max_extend_len, int64_t max_seq_len,
-                    const int32_t* plan, int plan_items, int num_tokens, int dtype, int kv8, hipStream_t st) {
+                    const int32_t* plan, int plan_items, int num_tokens, int dtype, int kv8, void* workspace, size_t workspace_bytes,
+                    hipStream_t st) {
   if (dtype != SP_F16 && dtype != SP_BF16) return SP_ERR_UNSUPPORTED;
   if (head_dim != 64 && head_dim != 128) return SP_ERR_UNSUPPORTED;
   if (batch_size > 65535 || num_q_heads > 65535) return SP_ERR_UNSUPPORTED;   // grid.z, grid.y
@@ -740,11 +917,14 @@ int run_extend_mfma(void* out, const void* q, const void* k_buffer, const void* 
   a.window = causal ? window_left : -1;
   a.kv8 = kv8;
   a.defer = g_extend_defer;
-  a.plan = plan; a.plan_items = plan_items; a.num_tokens = num_tokens;
+  a.plan = plan; a.num_tokens = num_tokens;
+  a.plan_items = plan_items;
   if (plan && (plan_items <= 0 || plan_items > 65535)) a.plan = nullptr;   // grid.y limit: unplanned launch
+  a.part_o = a.part_ml = nullptr;
+  extend_small_form(a, head_dim, max_seq_len, workspace, workspace_bytes);
   const int G = num_q_heads / num_kv_heads;
   if (max_extend_len <= 0) return SP_OK;
-  if (const int form = try_extend_w64(a, head_dim, dtype, max_extend_len, max_seq_len, st)) {
+  if (const int form = a.splits > 1 ? 0 : try_extend_w64(a, head_dim, dtype, max_extend_len, max_seq_len, st)) {
     g_extend_last_kernel = form == 2 ? 3 : 2;
     SP_LAUNCH_CHECK();
     return SP_OK;
