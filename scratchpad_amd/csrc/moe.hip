@@ -10,6 +10,18 @@
 namespace sp {
 namespace {
 
+// the lowest of the lanes' indexes that hold the largest value; 0x7fffffff where no lane has one.  A butterfly of value and index through
+// LDS took 12 exchanges in a row; the lanes that hold the largest value are usually one.  Top 4 of 32 experts: 4096 tokens 7.6 -> 5.5 us,
+// 8 tokens 6.2 -> 4.4.
+__device__ __forceinline__ int first_of_largest(float best, int at) {
+  const unsigned long long ties = __ballot(best == wave_max(best));
+  if (__popcll(ties) == 1) return __builtin_amdgcn_readlane(at, __ffsll(ties) - 1);
+  at = ties >> (threadIdx.x & 63) & 1 ? at : 0x7fffffff;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) at = min(at, __shfl_xor(at, off, 64));
+  return at;
+}
+
 // ---- router: one wave per token ----------------------------------------------------------------------------------
 // z = W x (fp32), s = sigmoid(z), choice = s + correction; groups: score = sum of the two largest choices of the group,
 // the best `keep` groups stay, the others' choices count as -inf; the `top` largest choices win; weights = their s.
@@ -66,12 +78,7 @@ __global__ void moe_route_kernel(int32_t* ids, float* weights, const void* x, in
       const float c = choice[e];
       if (c > best || (c == best && e < at && c > -INFINITY)) { best = c; at = e; }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ob = __shfl_xor(best, off, 64);
-      const int oa = __shfl_xor(at, off, 64);
-      if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
-    }
+    at = first_of_largest(best, at);
     if (at >= E) at = 0;                                  // fewer finite choices than `top`: cannot happen for top <= kept experts
     if (lane == 0) {
       ids[t * top + k] = at;
@@ -135,12 +142,7 @@ __global__ void moe_softmax_topk_kernel(int32_t* ids, float* weights, float* gat
       const float c = choice[e];
       if (c > best) { best = c; at = e; }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ob = __shfl_xor(best, off, 64);
-      const int oa = __shfl_xor(at, off, 64);
-      if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
-    }
+    at = first_of_largest(best, at);
     if (at >= E) at = 0;
     if (lane == 0) {
       ids[t * top + k] = at;
@@ -156,27 +158,74 @@ __global__ void moe_softmax_topk_kernel(int32_t* ids, float* weights, float* gat
 }
 
 // ---- pairs ordered by expert: offsets[E + 1], order[pos] = pair, place[pair] = pos.  One workgroup. ---------------
-__global__ void moe_align_kernel(int32_t* offsets, int32_t* order, int32_t* place, const int32_t* ids, int P, int E) {
-  extern __shared__ int32_t cnt[];          // counts[E], then cursors[E]
-  int32_t* cur = cnt + E;
-  for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
-  __syncthreads();
-  for (int p = threadIdx.x; p < P; p += blockDim.x) atomicAdd(&cnt[ids[p]], 1);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t run = 0;
-    for (int e = 0; e < E; ++e) {
-      offsets[e] = run;
-      cur[e] = run;
-      run += cnt[e];
+// Bound by its chain of latencies.  A pair's place inside its expert is what the count gave back, so the counters are gone through once;
+// a thread's ids are on their way together (up to 16384 pairs they stay in registers), the sums over experts go 64 at a time, and the order
+// is written in rows out of LDS.  16384 pairs of 32 experts: 14.6 -> 8.8 us (scattered stores of the order: 10.5); 32 pairs: 2.9 -> 2.3.
+constexpr int kAlignThreads = 1024, kAlignHeld = 16, kAlignPairs = kAlignThreads * kAlignHeld;
+
+__global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(int32_t* offsets, int32_t* order, int32_t* place, const int32_t* ids, int P,
+                                                                  int E) {
+  extern __shared__ int32_t cnt[];          // counts[E], first positions[E], then the held pairs in their order
+  int32_t* first = cnt + E;
+  uint16_t* sorted = (uint16_t*)(first + E);
+  const int tid = threadIdx.x;
+  const bool held = P <= kAlignPairs;
+  int32_t id[kAlignHeld], rank[kAlignHeld];
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < kAlignHeld; ++i) {
+      if (i * kAlignThreads >= P) break;
+      id[i] = ids[min(i * kAlignThreads + tid, P - 1)];
     }
-    offsets[E] = run;
+  }
+  for (int e = tid; e < E; e += kAlignThreads) cnt[e] = 0;
+  __syncthreads();
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < kAlignHeld; ++i) {
+      if (i * kAlignThreads >= P) break;
+      if (i * kAlignThreads + tid < P) rank[i] = atomicAdd(&cnt[id[i]], 1);
+    }
+  } else {
+    for (int p = tid; p < P; p += kAlignThreads) place[p] = atomicAdd(&cnt[ids[p]], 1);
   }
   __syncthreads();
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
-    const int pos = atomicAdd(&cur[ids[p]], 1);
-    order[pos] = p;
-    place[p] = pos;
+  if (tid < 64) {
+    int32_t run = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + tid;
+      const int32_t n = e < E ? cnt[e] : 0;
+      int32_t sum = n;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int32_t below = __shfl_up(sum, off, 64);
+        if (tid >= off) sum += below;
+      }
+      if (e < E) offsets[e] = first[e] = run + sum - n;
+      run += __shfl(sum, 63, 64);
+    }
+    if (tid == 0) offsets[E] = run;
+  }
+  __syncthreads();
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < kAlignHeld; ++i) {
+      if (i * kAlignThreads >= P) break;
+      const int p = i * kAlignThreads + tid;
+      if (p < P) {
+        const int pos = first[id[i]] + rank[i];
+        sorted[pos] = (uint16_t)p;
+        place[p] = pos;
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < P; i += kAlignThreads) order[i] = sorted[i];
+  } else {
+    for (int p = tid; p < P; p += kAlignThreads) {
+      const int pos = first[ids[p]] + place[p];
+      order[pos] = p;
+      place[p] = pos;
+    }
   }
 }
 
@@ -865,8 +914,9 @@ extern "C" int sp_moe_align(int32_t* offsets, int32_t* order, int32_t* place, co
                             void* stream) {
   SP_CHECK_ARG(pairs >= 0 && experts > 0 && experts <= 4096);
   SP_CHECK_ARG(offsets && (pairs == 0 || (order && place && ids)));
-  moe_align_kernel<<<1, 1024, 2 * (size_t)experts * sizeof(int32_t), (hipStream_t)stream>>>(offsets, order, place, ids,
-                                                                                            pairs, experts);
+  // (at most 32 + 32 KB)
+  const size_t lds = 2 * (size_t)experts * sizeof(int32_t) + (pairs <= kAlignPairs ? (size_t)pairs * sizeof(uint16_t) : 0);
+  moe_align_kernel<<<1, kAlignThreads, lds, (hipStream_t)stream>>>(offsets, order, place, ids, pairs, experts);
   SP_LAUNCH_CHECK();
   return SP_OK;
 }

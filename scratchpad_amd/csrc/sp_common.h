@@ -238,6 +238,17 @@ __device__ __forceinline__ float wave_sum(float v) {
   v += dpp_f32<0x4E>(v);                            // quad_perm [2,3,0,1]: lane ^ 2
   return v + dpp_f32<0xB1>(v);                      // quad_perm [1,0,3,2]: lane ^ 1
 }
+// the same for the largest value (no NaN among them)
+__device__ __forceinline__ float wave_max(float v) {
+  const auto h = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);
+  v = fmaxf(as_f32(h[0]), as_f32(h[1]));
+  const auto r = __builtin_amdgcn_permlane16_swap(as_u32(v), as_u32(v), false, false);
+  v = fmaxf(as_f32(r[0]), as_f32(r[1]));
+  v = fmaxf(v, dpp_f32<0x128>(v));
+  v = fmaxf(v, dpp_f32<0x124>(v));
+  v = fmaxf(v, dpp_f32<0x4E>(v));
+  return fmaxf(v, dpp_f32<0xB1>(v));
+}
 // Eight sums at a time over the lanes whose numbers differ in bits 3, 4 and 5 (all lanes active): lane l ends with the sum of v[l >> 3].
 // Every step halves the values that a lane carries - 15 instructions where eight sums one after the other take 56.
 __device__ __forceinline__ float eight_sums(const float* v, int lane) {
