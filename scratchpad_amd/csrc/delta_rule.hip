@@ -12,7 +12,8 @@
 // lanes; the request's tokens of this step are walked in order from the state the previous step left in the pool (zeros
 // at a sequence's first token), staged through LDS in passes.  A token costs ONE sweep over the column: the update, the
 // numerator and - on the state just completed - the next token's u^T S, then two independent sums over the column's lanes
-// (register moves); no workgroup barrier.  The order of its sums depends on the head only.  Prompts take it; a decode step (one token
+// (register moves); no workgroup barrier.  The order of its sums depends on the head only.  Prompts
+// take it, but for longer portions with heads of 64, which go 16 tokens at a time (delta_prepare_kernel and the walk of chunk16.h); a decode step (one token
 // per request, heads of 64 or 128, rank up to 512) takes delta_step_kernel, which forms the gates too and adds a head's sums in
 // another order.
 #include "chunk16.h"

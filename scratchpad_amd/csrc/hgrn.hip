@@ -5,7 +5,8 @@
 //   out = o / rms_head(o) * norm_w         (norm_w [Dv], the same for every head)
 // There is no key: the row of S that belongs to query channel i takes in (1 - f_i) of the value.
 //
-// One workgroup per (request, head): a column of S (one value channel) lives in the registers of 1 to 8 neighbouring
+// Longer portions with aligned rows go 16 tokens at a time on the matrix cores (hgrn2_prepare_kernel and the walk of chunk16.h).  The others,
+// one workgroup per (request, head): a column of S (one value channel) lives in the registers of 1 to 8 neighbouring
 // lanes; the request's tokens of this step are walked in order from the state the previous step left in the pool (zeros at
 // a sequence's first token), staged through LDS in passes of 16 tokens, the head norm as the pass's epilogue.
 #include "chunk16.h"
