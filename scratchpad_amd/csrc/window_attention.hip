@@ -330,18 +330,26 @@ qkv_norm_store_kernel(void* q, int64_t q_stride, const void* k, int64_t k_stride
 // scalar, 100 by sixteens, 8 one by one; 1000 rows of a prompt 8.2 by sixteens, 9.5 one by one).
 constexpr int kPoolRows = 16, kPoolSingles = 256, kPoolAhead = 16;
 
-// Where the channels are few enough that several groups of whole waves have them all (GROUPS: 1, 2 or 4 of kBlock / GROUPS threads), each
-// takes its share of the block's rows and the shares are added in order; the block's rows of the table come in one load, a lane each.  4096
-// tokens in blocks of 64 x 1024 channels: 10.7 us with one group and a dependent table read per row, now 6.9.
-template <typename Tag, int V, int GROUPS>
+// Where 16-byte pieces would leave threads of the workgroup without channels, a thread takes half or a quarter of one and keeps as many
+// bytes on their way (AHEAD rows of V channels); the block's rows of the table come in one load, a lane each.  The rows are added in their
+// order whatever the piece: a block's bits depend on its rows alone.  4096 tokens in blocks of 64 x 1024 channels: 10.4 us with
+// 16-byte pieces and a dependent table read per row, in half pieces 7.7; x 512 channels 7.8, in quarters 5.4.  (Shares of the rows
+// side by side, added up at the end, take 6.6 and 4.2, but give other bits.)
+template <typename Tag, int V>
+__device__ __forceinline__ u32x4 load_piece(const char* row, int at) {
+  const char* p = row + (uint32_t)(at * Elem<Tag>::kBytes);
+  if constexpr (V * Elem<Tag>::kBytes == 16) return ld16(p);
+  else if constexpr (V * Elem<Tag>::kBytes == 8) { const u32x2 h = *(const u32x2*)p; return u32x4{h[0], h[1], 0u, 0u}; }
+  else if constexpr (V * Elem<Tag>::kBytes == 4) return u32x4{*(const uint32_t*)p, 0u, 0u, 0u};
+  else return u32x4{*(const uint16_t*)p, 0u, 0u, 0u};
+}
+template <typename Tag, int V, int AHEAD>
 __global__ void __launch_bounds__(kBlock)
 pool_blocks_kernel(void* kpooled, void* vpooled, const void* kpool, const void* vpool, int64_t kp_stride, int64_t vp_stride,
                    const int32_t* req_to_token, int64_t table_stride, SeqBatch s, int64_t T, int rows, int kw, int vw, int P) {
   typedef Elem<Tag> E;
-  constexpr int PER = kBlock / GROUPS;
-  __shared__ float share[GROUPS > 1 ? GROUPS - 1 : 1][V][GROUPS > 1 ? PER : 1];
   const int64_t t0 = (int64_t)blockIdx.x * rows;
-  const int lane = threadIdx.x & 63, group = __builtin_amdgcn_readfirstlane(threadIdx.x / PER), at = threadIdx.x % PER;
+  const int lane = threadIdx.x & 63;
   int64_t pos = -1;
   int b = 0;
   if (lane < rows && t0 + lane < T) {
@@ -351,66 +359,54 @@ pool_blocks_kernel(void* kpooled, void* vpooled, const void* kpool, const void* 
   }
   uint64_t hits = __ballot(pos >= 0 && (pos + 1) % P == 0);          // (the same in every wave of the workgroup)
   const float inv = 1.f / (float)P;
-  const int part = (P + GROUPS - 1) / GROUPS, j_first = group * part, j_end = min(j_first + part, P);
   for (; hits; hits &= hits - 1) {
     const int l = __ffsll((unsigned long long)hits) - 1;
     const int64_t p = __shfl(pos, l, 64);
     const int32_t* table = req_to_token + load_idx(s.req_pool_indices, __shfl(b, l, 64), s.idx64) * table_stride;
     const int64_t first = p - P + 1, dst = table[p];
-    for (int c0 = blockIdx.y * PER * V; c0 < kw + vw; c0 += gridDim.y * PER * V) {
-      const int c = c0 + at * V;
-      const bool live = c < kw + vw, isk = c < kw;                    // (V divides kw: a thread's channels are of one buffer)
-      const void* src = isk ? kpool : vpool;
+    // a wave's pieces are of one buffer (the keys' share is filled up to whole waves): the rows' addresses are scalar
+    const int keys = (kw / V + 63) / 64 * 64, pieces = keys + (vw / V + 63) / 64 * 64;
+    for (int e0 = blockIdx.y * kBlock + (threadIdx.x & ~63); e0 < pieces; e0 += gridDim.y * kBlock) {
+      const bool isk = __builtin_amdgcn_readfirstlane(e0) < keys;
       const int64_t stride = isk ? kp_stride : vp_stride;
-      const int col = !live ? 0 : isk ? c : c - kw;
-      float acc[V];
+      const int c = (e0 - (isk ? 0 : keys) + lane) * V;
+      const bool live = c < (isk ? kw : vw);
+      const int col = live ? c : 0;
+      const char* src = (const char*)(isk ? kpool : vpool);
+      float acc[8];
 #pragma unroll
-      for (int x = 0; x < V; ++x) acc[x] = 0.f;
-      for (int j64 = j_first; j64 < j_end; j64 += 64) {
-        const int slots = table[first + min(j64 + lane, j_end - 1)];
-        for (int j0 = j64; j0 < min(j64 + 64, j_end); j0 += kPoolAhead) {
-          const int n = min(kPoolAhead, j_end - j0);
-          u32x4 raw[V > 1 ? kPoolAhead : 1];
-          float one[V > 1 ? 1 : kPoolAhead];
+      for (int x = 0; x < 8; ++x) acc[x] = 0.f;
+      for (int j64 = 0; j64 < P; j64 += 64) {
+        const int64_t row = table[first + min(j64 + lane, P - 1)] * stride * E::kBytes;
+        const int row_lo = (int)row, row_hi = (int)(row >> 32);
+        for (int j0 = j64; j0 < min(j64 + 64, P); j0 += AHEAD) {
+          const int n = min(AHEAD, P - j0);
+          u32x4 raw[AHEAD];
 #pragma unroll
-          for (int j = 0; j < kPoolAhead; ++j) {
-            const int64_t row = (int64_t)__builtin_amdgcn_readlane(slots, j0 - j64 + min(j, n - 1)) * stride + col;
-            if constexpr (V > 1) raw[j] = ld16((const char*)src + row * E::kBytes);
-            else one[j] = E::load(src, row);
+          for (int j = 0; j < AHEAD; ++j) {
+            const int at = j0 - j64 + j;               // (past the block: its last row again)
+            const int64_t off = ((int64_t)__builtin_amdgcn_readlane(row_hi, at) << 32) | (uint32_t)__builtin_amdgcn_readlane(row_lo, at);
+            raw[j] = load_piece<Tag, V>(src + off, col);
           }
 #pragma unroll
-          for (int j = 0; j < kPoolAhead; ++j)
+          for (int j = 0; j < AHEAD; ++j)
             if (j < n) {
-              if constexpr (V > 1) {
-                float f[V];
-                unpack16<Tag>(raw[j], f);
+              float f[8];
+              unpack16<Tag>(raw[j], f);
 #pragma unroll
-                for (int x = 0; x < V; ++x) acc[x] += f[x];
-              } else {
-                acc[0] += one[j];
-              }
+              for (int x = 0; x < V; ++x) acc[x] += f[x];
             }
         }
-      }
-      if constexpr (GROUPS > 1) {
-        __syncthreads();                                              // (the shares of a block before)
-        if (group > 0) {
-#pragma unroll
-          for (int x = 0; x < V; ++x) share[group - 1][x][at] = acc[x];
-        }
-        __syncthreads();
-        if (group > 0) continue;
-#pragma unroll
-        for (int g = 0; g < GROUPS - 1; ++g)
-#pragma unroll
-          for (int x = 0; x < V; ++x) acc[x] += share[g][x][at];
       }
       if (!live) continue;
 #pragma unroll
       for (int x = 0; x < V; ++x) acc[x] *= inv;
-      void* out = isk ? kpooled : vpooled;
-      if constexpr (V > 1) st16((char*)out + (dst * stride + col) * E::kBytes, pack16<Tag>(acc));
-      else E::store(out, dst * stride + col, acc[0]);
+      char* out = (char*)(isk ? kpooled : vpooled) + (dst * stride + col) * E::kBytes;
+      const u32x4 w = pack16<Tag>(acc);
+      if constexpr (V * E::kBytes == 16) st16(out, w);
+      else if constexpr (V * E::kBytes == 8) *(u32x2*)out = u32x2{w[0], w[1]};
+      else if constexpr (V * E::kBytes == 4) *(uint32_t*)out = w[0];
+      else *(uint16_t*)out = (uint16_t)w[0];
     }
   }
 }
@@ -424,15 +420,15 @@ static int launch_pool_blocks(void* kpooled, void* vpooled, const void* kpool, c
   const unsigned groups = (unsigned)((T + rows - 1) / rows);
   const bool vec = kw % V == 0 && vw % V == 0 && kp_stride % V == 0 && vp_stride % V == 0 &&
                    (((uintptr_t)kpooled | (uintptr_t)vpooled | (uintptr_t)kpool | (uintptr_t)vpool) & 15) == 0;
-#define SP_POOL(VEC, GROUPS)                                                                                                            \
-  pool_blocks_kernel<Tag, VEC, GROUPS><<<dim3(groups, (unsigned)(((kw + vw) / VEC + kBlock / GROUPS - 1) / (kBlock / GROUPS))), kBlock, 0, \
-                                         st>>>(kpooled, vpooled, kpool, vpool, kp_stride, vp_stride, req_to_token, table_stride, s, T,   \
-                                               rows, kw, vw, P)
-  // (blocks of fewer rows than a group has on their way at a time are one round either way)
-  if (vec && P >= 2 * kPoolAhead && (kw + vw) / V <= kBlock / 4) SP_POOL(V, 4);
-  else if (vec && P >= 2 * kPoolAhead && (kw + vw) / V <= kBlock / 2) SP_POOL(V, 2);
-  else if (vec) SP_POOL(V, 1);
-  else SP_POOL(1, 1);
+  const auto pieces = [&](int per) { return (kw / per + 63) / 64 * 64 + (vw / per + 63) / 64 * 64; };
+#define SP_POOL(VEC, AHEAD)                                                                                                             \
+  pool_blocks_kernel<Tag, VEC, AHEAD><<<dim3(groups, (unsigned)((pieces(VEC) + kBlock - 1) / kBlock)), kBlock, 0, st>>>(                \
+      kpooled, vpooled, kpool, vpool, kp_stride, vp_stride, req_to_token, table_stride, s, T, rows, kw, vw, P)
+  // (rows past the block are loaded for nothing: as many on their way as it has)
+  if (vec && P >= 4 * kPoolAhead && pieces(V / 4) <= kBlock) SP_POOL(V / 4, 4 * kPoolAhead);
+  else if (vec && P >= 2 * kPoolAhead && pieces(V / 2) <= kBlock) SP_POOL(V / 2, 2 * kPoolAhead);
+  else if (vec) SP_POOL(V, kPoolAhead);
+  else SP_POOL(1, kPoolAhead);
 #undef SP_POOL
   SP_LAUNCH_CHECK();
   return SP_OK;

@@ -47,6 +47,41 @@ def test_pool_blocks(P, kw, vw, dtype):
     assert torch.isnan(kp[~written]).all() and torch.isnan(vp[~written]).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("P", [16, 31, 33, 50, 64, 65, 130, 257])
+@pytest.mark.parametrize("kw,vw", [(64, 128), (256, 256), (256, 264), (512, 512), (520, 504), (512, 520), (7, 9)])
+def test_pool_blocks_add_their_rows_in_order(P, kw, vw, dtype):
+    """whole, half and quarter pieces per thread, partial rounds and more rows than lanes: the bits of the rows added one after the
+    other in fp32, whatever the width - a block's mean does not depend on what else the kernel is launched for"""
+    from scratchpad_amd import _native
+    announce("pool_blocks in order", dtype, P, kw, vw)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    lens, prefixes, slots = [1, P + 3, 2 * P, 1], [P - 1, 5, 0, 3 * P - 1], [1, 2, 3, 5]
+    total = sum(lens) + sum(prefixes)
+    table = torch.zeros(6, 4 * P + 8, dtype=torch.int32, device=DEV)
+    perm, at = torch.randperm(total, generator=g, device=DEV) + 1, 0
+    for n, p, s in zip(lens, prefixes, slots):
+        table[s, :n + p] = perm[at:at + n + p].to(torch.int32)
+        at += n + p
+    k, v = (torch.randn(total + 1, w, generator=g, device=DEV).to(dtype) for w in (kw, vw))
+    kp, vp = torch.full_like(k, float("nan")), torch.full_like(v, float("nan"))
+    _native.pool_blocks(kp, vp, k, v, table, seq_extend(lens, prefixes, slots), P)
+    ends = [(table[s, pos - P + 1:pos + 1].long(), int(table[s, pos])) for n, p, s in zip(lens, prefixes, slots)
+            for pos in range(p, p + n) if (pos + 1) % P == 0]
+    rows, dst = torch.stack([r for r, _ in ends]), torch.tensor([d for _, d in ends], device=DEV)
+    for got, src in ((kp, k), (vp, v)):
+        acc = torch.zeros(len(ends), src.shape[1], device=DEV)
+        for j in range(P):
+            acc += src[rows[:, j]].float()
+        inv = (torch.tensor(1.0) / P).to(DEV)
+        same = got[dst] == (acc * inv).to(dtype)
+        if dtype == torch.float16:      # (an instruction multiplies in 32 bits and rounds once, to 16; numpy's cast does so from 64)
+            once = (acc.double() * inv.double()).cpu().numpy().astype("float16")
+            same |= got[dst] == torch.from_numpy(once).to(DEV)
+        assert same.all()
+        assert int(torch.isnan(got).any(1).sum()) == total + 1 - len(ends)
+
+
 @pytest.mark.parametrize("B", [1, 17, 256, 257])
 def test_pool_blocks_of_requests_that_complete_together(B):
     """decode steps whose requests all end a block, on both sides of the line between one row and sixteen per workgroup"""
