@@ -166,6 +166,18 @@ __device__ __forceinline__ float mul_round<f16_tag>(float a, float b) {
   return f16_bits_to_f32((uint16_t)h);
 }
 
+// the same for a * b + c
+template <typename Tag>
+__device__ __forceinline__ float fma_round(float a, float b, float c) {
+  return fmaf(a, b, c);
+}
+template <>
+__device__ __forceinline__ float fma_round<f16_tag>(float a, float b, float c) {
+  uint32_t h;
+  asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(h) : "v"(a), "v"(b), "v"(c));
+  return f16_bits_to_f32((uint16_t)h);
+}
+
 __device__ __forceinline__ u32x4 ld16(const void* p) { return *(const u32x4*)p; }
 __device__ __forceinline__ void st16(void* p, const u32x4& v) { *(u32x4*)p = v; }
 

@@ -28,6 +28,15 @@
 namespace sp {
 namespace {
 
+// a pair (u, w) turned by an angle, rounded to Tag's type.  The fused operations are written out: the compiler fuses one product or the
+// other, and rounds to 16 bits inside or behind the sum, as a loop's unrolling suggests to it - a token's row must not depend on the
+// kernel that stores it.
+template <typename Tag>
+__device__ __forceinline__ void turn_pair(float u, float w, float cosine, float sine, float& first, float& second) {
+  first = fma_round<Tag>(u, cosine, -(w * sine));
+  second = fma_round<Tag>(u, sine, w * cosine);
+}
+
 // q rotated in place; k rotated and v (normed per head unless norm_v is 0) into the pool rows loc[t]
 template <typename Tag>
 __global__ void __launch_bounds__(kBlock)
@@ -48,8 +57,10 @@ qkv_rotary_store_kernel(void* q, int64_t q_stride, const void* k, int64_t k_stri
     const int col = h * D + i * step;
     const int64_t at = t * q_stride + col;
     const float u = E::load(q, at) + (qb ? qb[col] : 0.f), w = E::load(q, at + second) + (qb ? qb[col + second] : 0.f);
-    E::store(q, at, u * c - w * sn);
-    E::store(q, at + second, w * c + u * sn);
+    float x, y;
+    turn_pair<Tag>(u, w, c, sn, x, y);
+    E::store(q, at, x);
+    E::store(q, at + second, y);
   }
   for (int e = threadIdx.x; e < G * half; e += blockDim.x) {
     const int g = e / half, i = e % half;
@@ -58,8 +69,10 @@ qkv_rotary_store_kernel(void* q, int64_t q_stride, const void* k, int64_t k_stri
     const int col = g * D + i * step;
     const int64_t at = t * k_stride + col, to = slot * kp_stride + col;
     const float u = E::load(k, at) + (kb ? kb[col] : 0.f), w = E::load(k, at + second) + (kb ? kb[col + second] : 0.f);
-    E::store(kpool, to, u * c - w * sn);
-    E::store(kpool, to + second, w * c + u * sn);
+    float x, y;
+    turn_pair<Tag>(u, w, c, sn, x, y);
+    E::store(kpool, to, x);
+    E::store(kpool, to + second, y);
   }
   const int rest = D - dims;
   if (qb)
@@ -87,15 +100,15 @@ qkv_rotary_store_kernel(void* q, int64_t q_stride, const void* k, int64_t k_stri
     }
     ss = wave_sum(ss);
     const float inv = 1.f / sqrtf(ss / (float)Dv + eps);
-    for (int i = lane; i < Dv; i += 64) E::store(vpool, to + i, (E::load(v, at + i) + (vb ? vb[g * Dv + i] : 0.f)) * inv);
+    for (int i = lane; i < Dv; i += 64) E::store(vpool, to + i, mul_round<Tag>(E::load(v, at + i) + (vb ? vb[g * Dv + i] : 0.f), inv));
   }
 }
 
-// The same for prompt steps in 16-byte pieces, a wave per token: its angles' cosines and sines are formed once, a lane each, and wait in
-// LDS; a lane then takes V neighbouring pairs of a head, or V of its values (halves, no biases, values normed; VL lanes share a value
-// head).  With the two functions pair by pair of every head, and a value per lane
-// and load, 4096 tokens of 16 + 4 heads of 128 with 64 rotated took 17.7 us; this takes 7.9 (a workgroup per
-// token with these pieces: 13.4).
+// The same for steps of more than 64 tokens (prompts, and decode steps of so many requests) in 16-byte pieces, a wave per token: its
+// angles' cosines and sines are formed once, a lane each, and wait in LDS; a lane then takes V neighbouring pairs of a head, or V of its
+// values (halves, no biases, values normed; VL lanes share a value head).  The kernel above forms the two functions pair by pair of every
+// head and takes a value per lane and load.  16 + 4 heads of 128 with 64 rotated, it / this one in us: 65 tokens 4.4 / 4.1, 256: 4.5 / 4.1,
+// 1024: 6.0 / 4.5, 4096: 15.0 / 7.6 (a workgroup per token with these pieces: 13.4).  The same bits.
 template <typename Tag, int VL>
 __global__ void __launch_bounds__(kBlock)
 qkv_rotary_wave_kernel(char* q, int64_t q_stride, const char* k, int64_t k_stride, const char* v, int64_t v_stride, char* kpool,
@@ -130,10 +143,7 @@ qkv_rotary_wave_kernel(char* q, int64_t q_stride, const char* k, int64_t k_strid
     unpack16<Tag>(ld16(from), u);
     unpack16<Tag>(ld16(from + half * E::kBytes), w);
 #pragma unroll
-    for (int x = 0; x < V; ++x) {
-      a[x] = u[x] * cosine[i + x] - w[x] * sine[i + x];
-      b[x] = w[x] * cosine[i + x] + u[x] * sine[i + x];
-    }
+    for (int x = 0; x < V; ++x) turn_pair<Tag>(u[x], w[x], cosine[i + x], sine[i + x], a[x], b[x]);
     st16(to, pack16<Tag>(a));
     st16(to + half * E::kBytes, pack16<Tag>(b));
   }
@@ -144,13 +154,30 @@ qkv_rotary_wave_kernel(char* q, int64_t q_stride, const char* k, int64_t k_strid
   }
   for (int e = lane; e < (G * VL + 63) / 64 * 64; e += 64) {          // (whole waves: the sum is over lanes)
     const bool in = e < G * VL;
-    float x[V], ss = 0.f;
+    float x[V], sq[V];
     unpack16<Tag>(ld16(v + (t * v_stride + (in ? e : 0) * V) * E::kBytes), x);
+    // the squares in the order of the kernel above (a value per lane, wave_sum): values 64 apart, then 32, 16 ... 1 - here over the
+    // lanes of a head first, then over a lane's own values - so that a row's bits do not depend on how many tokens a step has
 #pragma unroll
-    for (int c = 0; c < V; ++c) ss += x[c] * x[c];
-    const float inv = 1.f / sqrtf(lanes_sum<VL>(ss) / (float)Dv + eps);
+    for (int c = 0; c < V; ++c) {
+      sq[c] = x[c] * x[c];
+      asm("" : "+v"(sq[c]));                          // (rounded here, not inside a fused multiply-add)
+      if constexpr (VL == 16) {
+        sq[c] += dpp_f32<0x128>(sq[c]);               // row_ror 8: lane ^ 8
+        sq[c] += dpp_f32<0x124>(sq[c]);               // row_ror 4: lane ^ 4, since lanes 8 apart hold the same by now
+      } else {
+        sq[c] += __shfl_xor(sq[c], 4, 64);
+      }
+      sq[c] += dpp_f32<0x4E>(sq[c]);                  // lane ^ 2
+      sq[c] += dpp_f32<0xB1>(sq[c]);                  // lane ^ 1
+    }
 #pragma unroll
-    for (int c = 0; c < V; ++c) x[c] *= inv;
+    for (int off = V / 2; off > 0; off /= 2)
+#pragma unroll
+      for (int c = 0; c < off; ++c) sq[c] += sq[c + off];
+    const float inv = 1.f / sqrtf(sq[0] / (float)Dv + eps);
+#pragma unroll
+    for (int c = 0; c < V; ++c) x[c] = mul_round<Tag>(x[c], inv);
     if (in) st16(vpool + (slot * vp_stride + e * V) * E::kBytes, pack16<Tag>(x));
   }
 }
@@ -911,7 +938,7 @@ extern "C" int sp_qkv_rotary_store(void* q, int64_t q_stride, const void* k, int
     SP_LAUNCH_CHECK();
     return SP_OK;
   }
-  // (a decode step's few tokens keep to a workgroup per token: more threads to a token's chain of loads)
+  // (the line of 64 tokens is not a crossing: at 1 - 64 tokens of 16 + 4 heads of 128 the wave takes 3.4 - 4.1 us, the workgroup 4.0 - 4.3)
   const int per = dtype == SP_F32 ? 4 : 8, half = rot_dims / 2;
   if (num_tokens > 64 && !adjacent && !q_bias && !k_bias && !v_bias && norm_values && v && half <= 64 && half % per == 0 && dim % per == 0 &&
       (vdim == 8 * per || vdim == 16 * per) && q_stride % per == 0 && k_stride % per == 0 && v_stride % per == 0 && kp_stride % per == 0 &&

@@ -49,3 +49,26 @@ def test_qkv_rotary_store(T, H, G, D, dims, adjacent, bias, pad, dtype):
     want = (vv / torch.sqrt((vv * vv).mean(-1, keepdim=True) + 1e-5)).view(T, -1)
     assert ((vp[loc].double() - want).abs() <= half * want.abs() + 1e-5 * want.abs().max()).all()
     assert torch.isnan(kp[:2]).all() and torch.isnan(vp[:2]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,G,D,dims", [(65, 4, 1, 128, 64), (300, 3, 5, 64, 64), (70, 2, 9, 64, 32), (200, 3, 5, 32, 16), (130, 2, 1, 128, 0),
+                                         (1500, 4, 4, 128, 64)])
+def test_a_tokens_rows_do_not_depend_on_the_steps_size(T, H, G, D, dims, dtype):
+    """the bits of a step of T tokens are those of the same tokens in steps of at most 64"""
+    from scratchpad_amd import _native
+    print("qkv rotary store, step sizes", T, H, G, D, dims, dtype, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(12)
+    rows = torch.randn(T, (H + 2 * G) * D, generator=g, device=DEV).to(dtype)
+    pos, loc = torch.randint(0, 5000, (T,), generator=g, device=DEV), torch.randperm(T, generator=g, device=DEV)
+    freq = 10000.0 ** (-torch.arange(dims // 2, device=DEV) / (dims // 2)) if dims else None
+    results = []
+    for step in (T, 64):
+        a, kp, vp = rows.clone(), *(torch.full((T, G * D), float("nan"), device=DEV, dtype=dtype) for _ in range(2))
+        q, k, v = a.split([H * D, G * D, G * D], 1)
+        for t0 in range(0, T, step):
+            at = slice(t0, t0 + step)
+            _native.qkv_rotary_store(q[at], k[at], v[at], kp, vp, pos[at], loc[at], freq, 1.0, H, G, D, D, 1e-5)
+        results.append((q, kp, vp))
+    for whole, parts in zip(*results):
+        assert torch.isfinite(whole).all() and torch.equal(whole, parts)
