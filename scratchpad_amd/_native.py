@@ -1643,16 +1643,21 @@ def causal_conv_silu(u: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
 SCAN_SEGMENT = None      # tests and measurements: the segments' length of every step that can be cut (0: none is)
 
 
+def _longest_request(tokens: int, requests: int) -> int:
+    """what a step's longest request is taken for (the lengths are on the device): twice the mean, all tokens at the most; no request: 0"""
+    return min(tokens, 2 * tokens // requests) if requests else 0
+
+
 def _scan_segment(tokens: int, requests: int, heads: int, slots: int, least: int) -> int:
     """Length of the segments that a step's requests are cut into (0: they are not): the shortest that keeps all segments (a last
     partial one per request counts half) in one round of the ``slots`` workgroups that the chip holds at a time, where the longest
-    request - the lengths are on the device: taken for twice the mean - has at least ``least`` tokens and three and a half of them.
+    request has at least ``least`` tokens and three and a half of them.
     us per layer, whole / cut, width 2048 (requests x tokens together, segment):  mLSTM 1 x 4096, 320: 742 / 241   4 x 4096, 320: 328 / 243
     5 x 3001, 256: 271 / 209   1 x 1000, 128: 211 / 109   2 x 500, 128: 121 / 106   1 x 300, 128: 98 / 106   8 x 4096, 384: 255 / 271
     Mamba-2 1 x 4096, 576: 668 / 448   2 x 4096, 640: 529 / 457   1 x 1000, 192: 208 / 169   3 x 1000, 192: 169 / 175   4 x 4096, 704: 434 / 471"""
     if SCAN_SEGMENT is not None:
         return SCAN_SEGMENT
-    longest, room = min(tokens, 2 * tokens // requests), 2 * (slots // heads) - requests      # room: half segments
+    longest, room = _longest_request(tokens, requests), 2 * (slots // heads) - requests      # room: half segments
     if longest < least or room <= 0:
         return 0
     length = max(128, -(-2 * tokens // (64 * room)) * 64)
@@ -1815,7 +1820,7 @@ def delta_recurrence_chunks_pay(tokens: int, requests: int, heads: int) -> bool:
     64 x 1024: 168 / 167   64 x 512: 101 / 113   256 x 4096: 542 / 624"""
     if DELTA_RECURRENCE_CHUNKS is not None:
         return DELTA_RECURRENCE_CHUNKS
-    return min(tokens, 2 * tokens // requests) >= 72
+    return _longest_request(tokens, requests) >= 72
 
 
 def delta_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, decay: torch.Tensor,
@@ -1875,13 +1880,12 @@ HGRN2_CHUNKS = None      # tests and measurements: True / False takes / leaves t
 
 
 def hgrn2_chunks_pay(tokens: int, requests: int, heads: int) -> bool:
-    """Prompts whose longest request (the lengths are on the device: taken for twice the mean) is long enough to pay for two more
-    launches, or steps of so many requests x heads that the per-token form's walk is bound by its work.  us per layer of width 2048
+    """Prompts whose longest request is long enough to pay for two more launches, or steps of so many requests x heads that the per-token form's walk is bound by its work.  us per layer of width 2048
     (8 heads of 128 x 128; requests x tokens together), per token / in chunks:  1 x 65: 84 / 86   1 x 300: 215 / 90   16 x 512: 81 / 83
     16 x 256: 81 / 86   4 x 1000: 245 / 91   1 x 4096: 2633 / 175   16 x 4096: 361 / 177   64 x 1024: 89 / 83   256 x 4096: 254 / 173"""
     if HGRN2_CHUNKS is not None:
         return HGRN2_CHUNKS
-    return min(tokens, 2 * tokens // requests) >= 72 or (tokens >= 16 * requests and requests * heads >= 512)
+    return _longest_request(tokens, requests) >= 72 or (tokens >= 16 * requests > 0 and requests * heads >= 512)
 
 
 def _hgrn2_chunks_take(rows, seq: SeqParams, dim: int, vdim: int) -> bool:
@@ -1900,7 +1904,7 @@ def _hgrn2_segment(tokens: int, requests: int, heads: int) -> int:
     if room <= 0:
         return 0
     length = max(64, -(-2 * tokens // (16 * room)) * 16)
-    return length if 7 * length <= 2 * min(tokens, 2 * tokens // requests) else 0
+    return length if 7 * length <= 2 * _longest_request(tokens, requests) else 0
 
 
 def hgrn2_scan(qpre: torch.Tensor, fpre: torch.Tensor, v: torch.Tensor, f_bias: torch.Tensor, lower: torch.Tensor,

@@ -601,3 +601,25 @@ def test_gated_delta_norm_forms_its_gates(lens, H, D, Dv, rank, spoiled, monkeyp
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.isfinite(want).any()
     ok = torch.isfinite(want)
     assert ((got - want).abs()[ok] <= 2.0 ** -7 * want.abs()[ok] + 1e-6).all() and (got != want)[ok].float().mean() < 0.01
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_steps_without_requests(dtype):
+    """every recurrence takes a multi-token step of no request: no rows, no state moved"""
+    from scratchpad_amd import _native as nat
+    H, D = 2, 64
+    n = H * D
+    ints = lambda dt: torch.zeros(0, dtype=dt, device=DEV)  # noqa: E731
+    seq = nat.SeqParams(ints(torch.int64), ints(torch.int64), ints(torch.int32), ints(torch.int32), ints(torch.int32),
+                        torch.zeros(0, dtype=torch.int32, device=DEV))
+    x = lambda w=n, dt=dtype: torch.zeros(0, w, dtype=dt, device=DEV)  # noqa: E731
+    f32 = lambda *s: torch.ones(*s, device=DEV)  # noqa: E731
+    S, m = f32(1, H, D, D), f32(1, H)
+    outs = [nat.mamba2_scan(x(3 * n), x(H, torch.float32), f32(H), f32(H), f32(H), S, seq, H, H, D, D),
+            nat.mlstm_scan(x(), x(), x(), x(), x(H, torch.float32), x(H, torch.float32), f32(n), S, f32(1, H, D), m, seq, H, D, D, 15.0, 1e-5),
+            nat.delta_recurrence(x(), x(), x(), x(), x(n, torch.float32), x(n, torch.float32), f32(n), S, seq, H, D, 1e-5),
+            nat.hgrn2_scan(x(), x(), x(), f32(n), f32(n), f32(D), S, seq, H, D, D, 1e-5),
+            nat.gated_delta_scan(x(), x(), x(), x(H), x(n, torch.float32), (x(32), f32(32, n)), f32(D), S, seq, H, H, D, D, 1e-5),
+            nat.gated_delta_scan(x(), x(), x(), x(H), x(n, torch.float32), x(n, torch.float32), f32(D), S, seq, H, H, D, D, 1e-5)]
+    torch.cuda.synchronize()
+    assert all(o.shape == (0, n) for o in outs) and bool((S == 1).all()) and bool((m == 1).all())

@@ -279,6 +279,14 @@ def test_scan_segments_keep_to_one_round_and_to_long_requests():
     assert not rule(4096, 8, 16, 256, 448) and not rule(300, 1, 16, 256, 448) and not rule(4096, 4, 64, 512, 800)
 
 
+def test_rules_of_the_recurrences_take_steps_without_requests():
+    """an empty step (a batch that was filtered away) asks the same rules"""
+    from scratchpad_amd import _native
+    assert _native._scan_segment(0, 0, 16, 256, 448) == 0 and _native._hgrn2_segment(0, 0, 8) == 0
+    assert not _native.hgrn2_chunks_pay(0, 0, 8) and not _native.delta_recurrence_chunks_pay(0, 0, 32)
+    assert not _native.hgrn2_chunks_pay(0, 3, 8) and _native._scan_segment(0, 3, 16, 256, 448) == 0      # requests of no tokens
+
+
 def test_mlstm_scan_takes_no_gate_rows_that_overlap(monkeypatch):
     """gates whose rows lie closer than their width (an expanded row, a sliding view) are refused before anything is launched: the
     kernel reads [token, head] at rows at least `heads` apart.  Views of one product and strides that differ pass."""
