@@ -375,6 +375,11 @@ constexpr int kSegScalars = 8, kSegDecay = 0, kSegMax = 2, kSegStart = 3;
 
 inline int64_t segment_floats(int D, int Dv, bool normaliser) { return (int64_t)D * Dv + (normaliser ? D : 0) + kSegScalars; }
 
+// floats of a step's segments (with mLSTM's normaliser, for either recurrence); no segments: none
+inline int64_t scan_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim, int segment_tokens) {
+  return segment_tokens > 0 ? (num_tokens / segment_tokens + batch_size) * heads * segment_floats(dim, vdim, true) : 0;
+}
+
 struct ScanSegments {
   float* work;
   int64_t stride;            // floats per segment and head
@@ -474,9 +479,3 @@ inline bool chunk_lds_ready(PerDevice<int>& raised, const void* kernel, int byte
 }
 
 }  // namespace sp
-
-// (weak: both sources that include this define it, a library may hold either or both; with mLSTM's normaliser, for either)
-extern "C" __attribute__((weak)) int64_t sp_scan_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim,
-                                                                int segment_tokens) {
-  return (num_tokens / segment_tokens + batch_size) * heads * sp::segment_floats(dim, vdim, true);
-}

@@ -256,7 +256,7 @@ extern "C" int64_t sp_hgrn2_chunk_floats(int64_t num_tokens, int batch_size, int
 }
 
 extern "C" int64_t sp_hgrn2_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim, int segment_tokens) {
-  return (num_tokens / segment_tokens + batch_size) * heads * ((int64_t)dim * vdim + dim);
+  return segment_tokens > 0 ? (num_tokens / segment_tokens + batch_size) * heads * ((int64_t)dim * vdim + dim) : 0;
 }
 
 extern "C" int sp_hgrn2_chunks(void* out, int64_t out_stride, const void* qpre, int64_t q_stride, const void* fpre, int64_t f_stride,

@@ -471,6 +471,12 @@ extern "C" int sp_mlstm_scan_tokens(void* out, int64_t out_stride, const void* q
                     stream);
 }
 
+// (weak: mlstm.hip and ssm.hip define it, a library may hold either or both)
+extern "C" __attribute__((weak)) int64_t sp_scan_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim,
+                                                                int segment_tokens) {
+  return scan_segment_floats(num_tokens, batch_size, heads, dim, vdim, segment_tokens);
+}
+
 extern "C" int sp_mlstm_scan_segments(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
                                       int64_t v_stride, const void* g, int64_t g_stride, const float* ipre, const float* fpre, int64_t gate_stride,
                                       const float* norm_w, float* S_state, int64_t S_stride, float* n_state, int64_t n_stride, float* m_state,

@@ -773,6 +773,12 @@ extern "C" int sp_mamba2_scan_tokens(float* y, int64_t y_stride, const void* xbc
                      extend_start_loc, token_req, idx64, batch_size, dtype, stream);
 }
 
+// (weak: mlstm.hip and ssm.hip define it, a library may hold either or both)
+extern "C" __attribute__((weak)) int64_t sp_scan_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim,
+                                                                int segment_tokens) {
+  return scan_segment_floats(num_tokens, batch_size, heads, dim, vdim, segment_tokens);
+}
+
 extern "C" int sp_mamba2_scan_segments(float* y, int64_t y_stride, const void* xbc, int64_t xbc_stride, const float* dt_raw,
                                        const float* dt_bias, const float* A_log, const float* Dskip, float* state, int64_t state_stride,
                                        float* work, int segment_tokens, int64_t num_tokens, int heads, int groups, int state_size,

@@ -128,3 +128,12 @@ def test_kv_pool_views_are_checked_before_a_launch():
         _native._kv_layout(torch.zeros(11, 2, 128)[:, :, :64], k, "test")
     with pytest.raises(RuntimeError, match="disagree"):
         _native._kv_layout(k, torch.zeros(12, 2, 64), "test")
+
+
+def test_workspace_sizes_of_segments_take_no_segments(lib):
+    """segment_tokens 0 is "no segments" to the launches that take these workspaces: the size is none, not a division by it"""
+    for name, per in (("sp_scan_segment_floats", 64 * 128 + 64 + 8), ("sp_hgrn2_segment_floats", 64 * 128 + 64)):
+        size = getattr(lib, name)
+        size.restype, size.argtypes = ctypes.c_int64, [ctypes.c_int64] + [ctypes.c_int] * 5
+        assert size(1000, 3, 5, 64, 128, 128) == (1000 // 128 + 3) * 5 * per
+        assert size(1000, 3, 5, 64, 128, 0) == 0 and size(1000, 3, 5, 64, 128, -64) == 0
