@@ -167,10 +167,13 @@ __device__ __forceinline__ void chunk16_prepare(float* work, const Fill& fill) {
 }
 
 // 16 bytes per lane from `from` to lds + 16 lane.  (The builtin of the same makes every later read of LDS wait for it; the walk waits
-// once a chunk.)
+// once a chunk.  m0 is named, so that no value another instruction needs in it is carried past; the compiler calls that reserved.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_to_lds(const void* from, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 // chunks of the requests before `b`, by all lanes of a wave
 __device__ __forceinline__ int chunks16_before(const SeqBatch& s, int b, int lane) {

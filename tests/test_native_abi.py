@@ -137,3 +137,15 @@ def test_workspace_sizes_of_segments_take_no_segments(lib):
         size.restype, size.argtypes = ctypes.c_int64, [ctypes.c_int64] + [ctypes.c_int] * 5
         assert size(1000, 3, 5, 64, 128, 128) == (1000 // 128 + 3) * 5 * per
         assert size(1000, 3, 5, 64, 128, 0) == 0 and size(1000, 3, 5, 64, 128, -64) == 0
+
+
+def test_assembly_that_writes_m0_names_it():
+    """m0 holds an operand of several intrinsics (direct loads, indexed moves): assembly that writes it says so to the compiler"""
+    import glob
+    seen = 0
+    for path in sorted(glob.glob(os.path.join(ROOT, "scratchpad_amd", "csrc", "*"))):
+        for stmt in re.findall(r"\basm\b[^;]*?\(.*?\);", open(path).read(), flags=re.S):
+            if re.search(r"s_mov_b32 m0|s_add_u32 m0", stmt):
+                seen += 1
+                assert re.search(r':[^:"]*"memory"[^:]*"m0"|:[^:]*"m0"[^:]*\)\s*;$', stmt), f"{os.path.basename(path)}: {stmt}"
+    assert seen
