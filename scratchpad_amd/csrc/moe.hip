@@ -715,11 +715,13 @@ __global__ void __launch_bounds__(64) moe_grouped_rows_kernel(GroupedArgs p) {
 }
 
 // The same with half the weight rows per wave (16; GLU: 8 gate rows and their 8 up rows) and twice the k-steps on their way, while
-// the kernel above would have at most two waves per SIMD (256 CUs of four; were every pair another expert's): the SIMDs that got
-// one wave more then set its time.  8 tokens, top 4 of 32 experts of 2048 x 1024: 33.8 + 18.2 us -> 32.4 + 16.3, the layer
-// 70.1 -> 66.5; 1024 x 512: 10.6 + 7.1 -> 10.3 + 6.7.  With two rows per expert the second reading of x's rows costs more than it
-// gives: 16 tokens 82.3 -> 90.7 (1024 x 512: 13.7 + 8.2 -> 14.6 + 7.9), 64 tokens 109 -> 113.
-constexpr long kNarrowWaves = 2 * 4 * 256;
+// the kernel above would have at most one wave per compute unit (were every pair another expert's) and leave units idle.  us of the up
+// and down product, kernel above -> this, top 4 of 32 experts: 1 token of 2048 x 1024 (256 waves each) 10.7 + 6.8 -> 10.0 + 6.2, of
+// 1024 x 512 (128 waves) 6.7 + 4.1 -> 5.4 + 3.5, 2 tokens of 1024 x 512 (256) 6.9 + 4.1 -> 6.8 + 4.0.  Past that the second reading of
+// x's rows costs as much as the evener shares give, or more: 2 tokens of 2048 x 1024 (512 waves) 13.3 + 7.8 -> 15.4 + 8.2, 4 tokens
+// 21.2 + 11.9 -> 21.9 + 11.8, 8 tokens 29.8 + 17.4 -> 31.0 + 16.6, 16 tokens 39.2 + 21.3 -> 44.1 + 23.0; top 8 of 64, 4 tokens
+// 40.3 + 20.9 -> 45.9 + 22.2.
+constexpr long kNarrowWaves = 256;
 constexpr int kNarrowUnroll = 16;
 
 template <typename Tag, int ACT>

@@ -65,6 +65,38 @@ def test_gated_form_is_the_two_steps(counts, ff, K, dtype):
     assert torch.equal(_native.moe_grouped_glu(a, w, offsets, P, order, 2, "clamped", 2.0, 1.702), _native.moe_glu(gu, 2.0, 1.702))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K", [480, 512, 544, 1024, 1056])
+@pytest.mark.parametrize("E,pairs,N", [(8, 4, 512), (8, 4, 1024), (8, 4, 1028), (8, 8, 513), (16, 2, 2048), (8, 9, 256)])
+def test_few_pairs_have_the_bits_of_many(E, pairs, N, K, dtype):
+    """few pairs over whole and partial rounds of k-steps, at both sides of the line of one wave per compute unit: the bits of the same
+    rows beside so many others that another kernel takes them, in the product and in its gated form"""
+    from scratchpad_amd import _native
+    print("few pairs", E, pairs, N, K, dtype, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(6)
+    a = torch.randn(pairs, K, generator=g, device=DEV).to(dtype)
+    many = torch.randn(24 * E, K, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(E, 2 * N, K, generator=g, device=DEV) * K ** -0.5).to(dtype)
+    expert = torch.sort(torch.randint(0, E, (pairs,), generator=g, device=DEV)).values
+    counts = torch.bincount(expert, minlength=E)
+    offsets = torch.cat([counts.new_zeros(1), counts.cumsum(0)]).int()
+    # the same rows at the head of their experts' groups of a step of 24 more rows per expert
+    big = torch.cat([torch.cat([a[expert == e], many[24 * e:24 * (e + 1)]]) for e in range(E)])
+    big_offsets = (offsets + 24 * torch.arange(E + 1, device=DEV)).int()
+    at = torch.arange(pairs, device=DEV) + 24 * expert
+    for width in (N, 2 * N):
+        ww = w[:, :width].contiguous()
+        got = _native.moe_grouped_gemm(a, ww, offsets, pairs)
+        want = (a.float()[:, None] * ww[expert].float()).sum(-1)
+        size = (a.float()[:, None] * ww[expert].float()).abs().sum(-1)
+        bar = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11          # half an ulp, and K fp32 additions in either order
+        assert ((got.float() - want).abs() <= bar * want.abs() + 2 * K * 2.0 ** -24 * size).all()
+        assert torch.equal(got, _native.moe_grouped_gemm(big, ww, big_offsets, big.shape[0])[at])
+    for act, more in (("silu", ()), ("clamped", (2.0, 1.702))):
+        got = _native.moe_grouped_glu(a, w, offsets, pairs, None, 1, act, *more)
+        assert torch.equal(got, _native.moe_grouped_glu(big, w, big_offsets, big.shape[0], None, 1, act, *more)[at])
+
+
 def test_gated_form_leaves_other_shapes_to_the_two_steps():
     from scratchpad_amd import _native
     for dtype, K in ((torch.float32, 64), (torch.bfloat16, 40)):
