@@ -771,7 +771,8 @@ size_t extend_split_bytes(int64_t num_tokens, int num_q_heads, int head_dim) {
 // The form of a launch whose row blocks leave compute units idle (at most half as many workgroups as there are; plain attention).
 // A row block costs its workgroup about a + t * tiles, t = 1.05 us per 64-key tile at heads of 64 (vector work of two waves per SIMD), 1.15 - 1.35
 // at 128.  Two ways to use the idle units:
-//   * half_blocks (heads of 64): four waves take half a row block, one wave per SIMD, 0.8 us per tile, same bits, twice the workgroups;
+//   * half_blocks (heads of 64): four waves take half a row block, one wave per SIMD, 0.8 us per tile, same bits, twice the workgroups -
+//     where the other half has rows: 4 requests of 17 behind 1000, heads of 64, 16 on 16: 15.4 | 16.5, of 64 behind 1000: 17.8 | 18.8;
 //   * splits: workgroups share the block's keys, t * tiles / splits, and pay for the partial sums (5 us for the merge, and their traffic).
 // Taken is the one that this model puts ahead, in ns (us at one form for all | half blocks | two | four | eight shares; 16-bit pool):
 //   heads of 64, 32 on 8:   3 requests, 777 tokens behind 1500: 37.3 | 29.0 | 29.0        1, 64 behind 2000:  38.9 | 31.5 | 25.5 | 18.1 | 16.1
@@ -781,7 +782,8 @@ size_t extend_split_bytes(int64_t num_tokens, int num_q_heads, int head_dim) {
 //                           1, 1024 behind 2000: 86.5 | - | 64.7                          1, 1024: 34.3 | - | 33.2 (not taken)
 // What the 4 x 64-row kernel applies to stays whole: its forms and this file's agree to the bit, whichever of them a size selects.
 // With more than half of the units busy the same forms lose: 4 requests, 2048 tokens behind 1500, heads of 64: 45 | 46; 4096 tokens: 90 | 102.
-static void extend_small_form(ExtendArgs& a, int head_dim, int64_t max_seq_len, void* workspace, size_t workspace_bytes) {
+static void extend_small_form(ExtendArgs& a, int head_dim, int max_extend_len, int64_t max_seq_len, void* workspace,
+                              size_t workspace_bytes) {
   a.splits = 1;
   a.half_blocks = 0;
   const int G = a.Hq / a.Hkv, gk = extend_gk(G), gx = a.Hkv * (G / gk), rows = 32 * (kExtendWaves / gk);
@@ -802,7 +804,8 @@ static void extend_small_form(ExtendArgs& a, int head_dim, int64_t max_seq_len, 
     a.part_o = (float*)workspace;
     a.part_ml = a.part_o + groups * kExtendWaves * s * 32 * head_dim;
   }
-  else if (head_dim == 64 && (a.kv8 || g_extend_dma) && a.bs < 32768) a.half_blocks = 1;
+  // (portions of one half only would leave four waves to load what eight do)
+  else if (head_dim == 64 && (a.kv8 || g_extend_dma) && a.bs < 32768 && (max_extend_len > rows / 2 || g_extend_small == 2)) a.half_blocks = 1;
 }
 
 #define SP_EXT_SET_LDS(KERNEL, BYTES)                                                                              \
@@ -921,7 +924,7 @@ int run_extend_mfma(void* out, const void* q, const void* k_buffer, const void* 
   a.plan_items = plan_items;
   if (plan && (plan_items <= 0 || plan_items > 65535)) a.plan = nullptr;   // grid.y limit: unplanned launch
   a.part_o = a.part_ml = nullptr;
-  extend_small_form(a, head_dim, max_seq_len, workspace, workspace_bytes);
+  extend_small_form(a, head_dim, max_extend_len, max_seq_len, workspace, workspace_bytes);
   const int G = num_q_heads / num_kv_heads;
   if (max_extend_len <= 0) return SP_OK;
   if (const int form = a.splits > 1 ? 0 : try_extend_w64(a, head_dim, dtype, max_extend_len, max_seq_len, st)) {
