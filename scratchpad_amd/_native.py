@@ -1072,10 +1072,11 @@ def token_requests(extend_start_loc: torch.Tensor, num_tokens: int) -> torch.Ten
 
 class SeqParams:
     """The header's SP_SEQ_PARAMS of one step, built once per forward (``from_forward_batch``) and handed to every kernel
-    that reads or writes per-request state.  Holds the tensors, so the pointers stay valid while it lives."""
+    that reads or writes per-request state.  Holds the tensors, so the pointers stay valid while it lives.  ``longest``: the
+    step's longest extend length where the host knows it (only the choice between a recurrence's forms depends on it)."""
 
     def __init__(self, req_pool_indices: torch.Tensor, seq_lens: torch.Tensor, extend_seq_lens=None,
-                 extend_prefix_lens=None, extend_start_loc=None, token_req=None):
+                 extend_prefix_lens=None, extend_start_loc=None, token_req=None, longest: Optional[int] = None):
         _gpu(req_pool_indices, seq_lens, extend_seq_lens, extend_prefix_lens, extend_start_loc, token_req)
         if req_pool_indices.dtype not in (torch.int32, torch.int64):
             raise RuntimeError("req_pool_indices must be int32 or int64")
@@ -1089,6 +1090,7 @@ class SeqParams:
                                    "token_req, all int32")
             ext = tuple(t.contiguous() for t in ext)
         self.extend_seq_lens, self.extend_prefix_lens, self.extend_start_loc, self.token_req = ext
+        self.longest = longest
         self.batch_size = int(self.req_pool_indices.shape[0])
         self.num_tokens = self.batch_size if token_req is None else int(self.token_req.shape[0])
         self.args = [self.req_pool_indices.data_ptr(), self.seq_lens.data_ptr(), _ptr(self.extend_seq_lens),
@@ -1100,8 +1102,9 @@ class SeqParams:
         if fb.forward_mode.is_decode():
             return cls(fb.req_pool_indices, fb.seq_lens)
         token_req = token_requests(fb.extend_start_loc, fb.extend_num_tokens)
+        lens = fb.extend_seq_lens_cpu
         return cls(fb.req_pool_indices, fb.seq_lens, fb.extend_seq_lens, fb.extend_prefix_lens, fb.extend_start_loc,
-                   token_req)
+                   token_req, int(max(lens)) if lens is not None and len(lens) else None)
 
 
 def _f32(t: torch.Tensor, what: str) -> torch.Tensor:
@@ -1644,24 +1647,31 @@ SCAN_SEGMENT = None      # tests and measurements: the segments' length of every
 
 
 def _longest_request(tokens: int, requests: int) -> int:
-    """what a step's longest request is taken for (the lengths are on the device): twice the mean, all tokens at the most; no request: 0"""
+    """what a step's longest request is taken for where the host does not know the lengths: twice the mean; no request: 0"""
     return min(tokens, 2 * tokens // requests) if requests else 0
 
 
-def _scan_segment(tokens: int, requests: int, heads: int, slots: int, least: int) -> int:
+def _scan_segment(tokens: int, requests: int, heads: int, slots: int, least: int, longest: Optional[int] = None,
+                  parts: float = 3.5) -> int:
     """Length of the segments that a step's requests are cut into (0: they are not): the shortest that keeps all segments (a last
     partial one per request counts half) in one round of the ``slots`` workgroups that the chip holds at a time, where the longest
-    request has at least ``least`` tokens and three and a half of them.
+    request has at least ``least`` tokens and ``parts`` of them (3.5 of the guess where its length is not known).
     us per layer, whole / cut, width 2048 (requests x tokens together, segment):  mLSTM 1 x 4096, 320: 742 / 241   4 x 4096, 320: 328 / 243
     5 x 3001, 256: 271 / 209   1 x 1000, 128: 211 / 109   2 x 500, 128: 121 / 106   1 x 300, 128: 98 / 106   8 x 4096, 384: 255 / 271
-    Mamba-2 1 x 4096, 576: 668 / 448   2 x 4096, 640: 529 / 457   1 x 1000, 192: 208 / 169   3 x 1000, 192: 169 / 175   4 x 4096, 704: 434 / 471"""
+    Mamba-2 1 x 4096, 576: 668 / 448   2 x 4096, 640: 529 / 457   1 x 1000, 192: 208 / 169   3 x 1000, 192: 169 / 175   4 x 4096, 704: 434 / 471
+    Cut / whole by the longest request's segments, mean (largest) over 1 - 16 requests, equal and unequal, of 150 - 3000 tokens, widths 1024 and
+    2048:  mLSTM 2 - 2.5: 1.01 (1.22)   2.5 - 3: 0.95 (1.11)   3 - 3.5: 0.87 (1.04)   3.5 - 4: 0.81 (1.07)   4 - 5: 0.72 (0.96)
+    Mamba-2 2 - 2.5: 1.04 (1.11)   2.5 - 3: 1.00 (1.06)   3 - 3.5: 0.96 (1.05)   3.5 - 4: 0.87 (1.05)   4 - 5: 0.84 (1.00); the largest
+    with few tokens, where the host's issue of two more launches is what counts"""
     if SCAN_SEGMENT is not None:
         return SCAN_SEGMENT
-    longest, room = _longest_request(tokens, requests), 2 * (slots // heads) - requests      # room: half segments
+    if longest is None:
+        longest, parts = _longest_request(tokens, requests), 3.5
+    room = 2 * (slots // heads) - requests                           # half segments
     if longest < least or room <= 0:
         return 0
     length = max(128, -(-2 * tokens // (64 * room)) * 64)
-    return length if 7 * length <= 2 * longest else 0
+    return length if parts * length <= longest else 0
 
 
 def _scan_segments_take(rows, dim: int, vdim: int, seq: SeqParams) -> bool:
@@ -1678,7 +1688,8 @@ def mamba2_scan(xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, 
             state.shape[1:] != (heads, state_size, vdim) or dt_bias.numel() != heads or A_log.numel() != heads or D.numel() != heads:
         raise RuntimeError("mamba2_scan: shapes do not fit")
     y = torch.empty((xbc.shape[0], inner), dtype=torch.float32, device=xbc.device)
-    segment = _scan_segment(seq.num_tokens, seq.batch_size, heads, 512 if vdim == 64 else 256, 800) if \
+    segment = _scan_segment(seq.num_tokens, seq.batch_size, heads, 512 if vdim == 64 else 256, 800 if seq.longest is None else 576,
+                            seq.longest, 2.75) if \
         _scan_segments_take((xbc,), state_size, vdim, seq) and y.stride(0) < 1 << 24 else 0
     if segment:
         work = torch.empty(load().sp_scan_segment_floats(seq.num_tokens, seq.batch_size, heads, state_size, vdim, segment),
@@ -1727,7 +1738,9 @@ def mlstm_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tenso
             S.shape[1:] != (heads, dim, vdim) or n.shape[1:] != (heads, dim) or m.shape[1:] != (heads,):
         raise RuntimeError("mlstm_scan: gate or state shapes do not fit")
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
-    segment = _scan_segment(T, seq.batch_size, heads, 512 if dim == 64 and vdim == 64 else 256, 448) if \
+    # (400 - 447 tokens pay for two more launches where there are heads enough: 1 x 420 of 8 heads 98 / 105 us, 2 x 420 of 16 126 / 106)
+    least = 448 if seq.longest is None or T * heads < 6144 else 400
+    segment = _scan_segment(T, seq.batch_size, heads, 512 if dim == 64 and vdim == 64 else 256, least, seq.longest, 2.5) if \
         _scan_segments_take((q, k, v), dim, vdim, seq) and max(g.stride(0), out.stride(0)) < 1 << 24 else 0
     if segment:
         work = torch.empty(load().sp_scan_segment_floats(T, seq.batch_size, heads, dim, vdim, segment), dtype=torch.float32, device=q.device)
@@ -1814,13 +1827,17 @@ def delta_gates(p: torch.Tensor, w2t: torch.Tensor, w0: torch.Tensor, apre: torc
 DELTA_RECURRENCE_CHUNKS = None      # tests and measurements, as HGRN2_CHUNKS
 
 
-def delta_recurrence_chunks_pay(tokens: int, requests: int, heads: int) -> bool:
-    """As hgrn2_chunks_pay.  us per layer of width 2048 (32 heads of 64; requests x tokens together), per token / in chunks:  1 x 65: 96 / 101
+def delta_recurrence_chunks_pay(tokens: int, requests: int, heads: int, longest: Optional[int] = None) -> bool:
+    """As hgrn2_chunks_pay; but where requests x heads of like lengths fill the chip either form is bound by its work, and the chunks' is
+    the larger.  us per layer of width 2048 (32 heads of 64; requests x tokens together), per token / in chunks:  1 x 65: 96 / 101
     1 x 300: 191 / 108   2 x 500: 272 / 142   16 x 512: 104 / 100   1 x 4096: 2309 / 1010   4 x 4096: 835 / 531   16 x 4096: 558 / 497
-    64 x 1024: 168 / 167   64 x 512: 101 / 113   256 x 4096: 542 / 624"""
+    64 x 1024: 168 / 167   64 x 512: 101 / 113   256 x 4096: 542 / 624;  equal lengths, requests x tokens each:  8 x 300: 325 / 273
+    16 x 100: 203 / 204   16 x 300: 546 / 532   32 x 100: 368 / 392   32 x 300: 1010 / 1000   64 x 100: 651 / 668   32 x 40: 173 / 179"""
     if DELTA_RECURRENCE_CHUNKS is not None:
         return DELTA_RECURRENCE_CHUNKS
-    return _longest_request(tokens, requests) >= 72
+    if longest is None:
+        longest = _longest_request(tokens, requests)
+    return longest >= 72 and tokens * heads < 768 * longest
 
 
 def delta_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, decay: torch.Tensor,
@@ -1836,7 +1853,7 @@ def delta_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch
         raise RuntimeError("delta_recurrence: decay, remove [T, H*D], norm_w [H*D], state [slots, H, D, D]")
     out = empty_rows(T, n, r.dtype, r.device)
     per = 4 if r.dtype == torch.float32 else 8
-    if seq.extend_seq_lens is not None and dim == 64 and delta_recurrence_chunks_pay(T, seq.batch_size, heads) and \
+    if seq.extend_seq_lens is not None and dim == 64 and delta_recurrence_chunks_pay(T, seq.batch_size, heads, seq.longest) and \
             all(t.stride(0) % per == 0 and t.data_ptr() % 16 == 0 for t in (r, k, v, g)) and decay.data_ptr() % 16 == 0 and remove.data_ptr() % 16 == 0:
         work = torch.empty(load().sp_delta_recurrence_chunk_floats(T, seq.batch_size, heads, dim), dtype=torch.float32, device=r.device)
         _check(load().sp_delta_recurrence_chunks(out.data_ptr(), out.stride(0), r.data_ptr(), r.stride(0), k.data_ptr(), k.stride(0),
@@ -1879,13 +1896,17 @@ def delta_step(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tenso
 HGRN2_CHUNKS = None      # tests and measurements: True / False takes / leaves the chunks of 16 wherever they are built for the form
 
 
-def hgrn2_chunks_pay(tokens: int, requests: int, heads: int) -> bool:
-    """Prompts whose longest request is long enough to pay for two more launches, or steps of so many requests x heads that the per-token form's walk is bound by its work.  us per layer of width 2048
-    (8 heads of 128 x 128; requests x tokens together), per token / in chunks:  1 x 65: 84 / 86   1 x 300: 215 / 90   16 x 512: 81 / 83
-    16 x 256: 81 / 86   4 x 1000: 245 / 91   1 x 4096: 2633 / 175   16 x 4096: 361 / 177   64 x 1024: 89 / 83   256 x 4096: 254 / 173"""
+def hgrn2_chunks_pay(tokens: int, requests: int, heads: int, longest: Optional[int] = None) -> bool:
+    """Prompts whose longest request is long enough to pay for two more launches, or steps of so many tokens x heads that the per-token
+    form's walk is bound by its work.  us per layer of width 2048 (8 heads of 128 x 128; requests x tokens together), per token / in chunks:  1 x 65: 84 / 86   1 x 300: 215 / 90   16 x 512: 81 / 83
+    16 x 256: 81 / 86   4 x 1000: 245 / 91   1 x 4096: 2633 / 175   16 x 4096: 361 / 177   64 x 1024: 89 / 83   256 x 4096: 254 / 173
+    Requests of equal lengths, each:  64 x 16: 76 / 83   100 x 17: 123 / 107   32 x 60: 92 / 84   64 x 64: 177 / 134   8 x 40: 76 / 81
+    32 x 40: 76 / 80   4 x 60: 80 / 84   2 x 100: 92 / 83   8 x 100: 103 / 83"""
     if HGRN2_CHUNKS is not None:
         return HGRN2_CHUNKS
-    return _longest_request(tokens, requests) >= 72 or (tokens >= 16 * requests > 0 and requests * heads >= 512)
+    if longest is None:
+        longest = _longest_request(tokens, requests)
+    return longest >= 72 or (tokens >= 16 * requests > 0 and tokens * heads >= 12288)
 
 
 def _hgrn2_chunks_take(rows, seq: SeqParams, dim: int, vdim: int) -> bool:
@@ -1895,16 +1916,21 @@ def _hgrn2_chunks_take(rows, seq: SeqParams, dim: int, vdim: int) -> bool:
         t.stride(0) % per == 0 and t.data_ptr() % 16 == 0 for t in rows)
 
 
-def _hgrn2_segment(tokens: int, requests: int, heads: int) -> int:
-    """as _scan_segment, with two workgroups per CU; us at one request of 4096 tokens, width 2048, by the segment's length:  none 1053
-    64: 174   80: 175   128: 198   256: 204   512: 285;  16 requests together  none 209   64: 193   80: 177   256: 206"""
+def _hgrn2_segment(tokens: int, requests: int, heads: int, longest: Optional[int] = None) -> int:
+    """as _scan_segment, with two workgroups per CU and four and a half segments to a longest request that is known; us at one request of
+    4096 tokens, width 2048, by the segment's length:  none 1053   64: 174   80: 175   128: 198   256: 204   512: 285;  16 requests together
+    none 209   64: 193   80: 177   256: 206.  Cut / whole by the longest request's segments, as there:  3 - 3.5: 1.10 (1.15)
+    3.5 - 4: 1.03 (1.10)   4 - 4.5: 1.00 (1.07)   4.5 - 5: 0.96 (1.06)   5 - 6: 0.89 (0.98)   6 - 8: 0.79 (0.94)"""
     if SCAN_SEGMENT is not None:
         return SCAN_SEGMENT
+    parts = 4.5
+    if longest is None:
+        longest, parts = _longest_request(tokens, requests), 3.5
     room = 2 * (512 // heads) - requests
     if room <= 0:
         return 0
     length = max(64, -(-2 * tokens // (16 * room)) * 16)
-    return length if 7 * length <= 2 * _longest_request(tokens, requests) else 0
+    return length if parts * length <= longest else 0
 
 
 def hgrn2_scan(qpre: torch.Tensor, fpre: torch.Tensor, v: torch.Tensor, f_bias: torch.Tensor, lower: torch.Tensor,
@@ -1919,8 +1945,8 @@ def hgrn2_scan(qpre: torch.Tensor, fpre: torch.Tensor, v: torch.Tensor, f_bias: 
             state.shape[1:] != (heads, dim, vdim):
         raise RuntimeError("hgrn2_scan: f_bias, lower [H*D], norm_w [vdim], state [slots, H, D, vdim]")
     out = empty_rows(T, heads * vdim, qpre.dtype, qpre.device)
-    if _hgrn2_chunks_take((qpre, fpre, v), seq, dim, vdim) and hgrn2_chunks_pay(T, seq.batch_size, heads):
-        lib, segment = load(), _hgrn2_segment(T, seq.batch_size, heads)
+    if _hgrn2_chunks_take((qpre, fpre, v), seq, dim, vdim) and hgrn2_chunks_pay(T, seq.batch_size, heads, seq.longest):
+        lib, segment = load(), _hgrn2_segment(T, seq.batch_size, heads, seq.longest)
         work = torch.empty(lib.sp_hgrn2_chunk_floats(T, seq.batch_size, heads, dim), dtype=torch.float32, device=qpre.device)
         sums = torch.empty(lib.sp_hgrn2_segment_floats(T, seq.batch_size, heads, dim, vdim, segment), dtype=torch.float32,
                            device=qpre.device) if segment else None

@@ -287,6 +287,40 @@ def test_rules_of_the_recurrences_take_steps_without_requests():
     assert not _native.hgrn2_chunks_pay(0, 3, 8) and _native._scan_segment(0, 3, 16, 256, 448) == 0      # requests of no tokens
 
 
+def test_rules_of_the_recurrences_know_the_longest_request(monkeypatch):
+    """a forward batch's lengths are on the host: the forms for long requests are taken where one is long and not where twice the mean
+    would be, and where the lengths are not known the guess stays"""
+    from scratchpad_amd import _native
+    from scratchpad_amd.forward_info import ForwardBatch, ForwardMode
+    monkeypatch.setattr(_native, "_gpu", lambda *a: None)
+    monkeypatch.setattr(_native, "token_requests", lambda starts, n: torch.zeros(n, dtype=torch.int32))
+    ints = lambda v, dt=torch.int32: torch.tensor(v, dtype=dt)  # noqa: E731
+
+    def params(lens, known=True):
+        n = len(lens)
+        fb = ForwardBatch(forward_mode=ForwardMode.EXTEND, batch_size=n, input_ids=ints([0] * sum(lens), torch.int64),
+                          req_pool_indices=ints(list(range(n)), torch.int64), seq_lens=ints(lens, torch.int64),
+                          out_cache_loc=ints([0] * sum(lens), torch.int64), seq_lens_sum=sum(lens))
+        fb.extend_num_tokens, fb.extend_seq_lens, fb.extend_prefix_lens = sum(lens), ints(lens), ints([0] * n)
+        fb.extend_start_loc = ints([sum(lens[:i]) for i in range(n)])
+        fb.extend_seq_lens_cpu = list(lens) if known else None
+        return _native.SeqParams.from_forward_batch(fb)
+    assert params([3, 70, 5]).longest == 70 and params([3, 70, 5], False).longest is None
+    rule = lambda r, lens, *more: r(sum(lens), len(lens), *more, longest=params(lens).longest)  # noqa: E731
+    mlstm, mamba2 = (256, 448), (512, 576)
+    cut = lambda parts: lambda *a, **k: _native._scan_segment(*a, **k, parts=parts)  # noqa: E731
+    for lens in ([230] * 2, [300] * 4, [300] * 8):
+        assert not rule(cut(2.5), lens, 8, *mlstm)
+    for lens in ([500] * 3, [1000] * 3, [4000] * 3):
+        assert not rule(cut(2.75), lens, 64, *mamba2)
+    for lens in ([40] * 8, [60] * 4, [40] * 32, [16] * 64):
+        assert not rule(_native.hgrn2_chunks_pay, lens, 8)
+    assert not rule(_native.delta_recurrence_chunks_pay, [40] * 16, 32) and not rule(_native.delta_recurrence_chunks_pay, [100] * 32, 32)
+    uneven = [2000] + [3] * 60                     # one prompt among the portions of a running batch
+    assert rule(_native.hgrn2_chunks_pay, uneven, 8) and rule(_native._hgrn2_segment, uneven, 8)
+    assert rule(_native.delta_recurrence_chunks_pay, uneven, 32) and rule(cut(2.5), [4000] + [10] * 7, 16, *mlstm)
+
+
 def test_mlstm_scan_takes_no_gate_rows_that_overlap(monkeypatch):
     """gates whose rows lie closer than their width (an expanded row, a sliding view) are refused before anything is launched: the
     kernel reads [token, head] at rows at least `heads` apart.  Views of one product and strides that differ pass."""
