@@ -1739,8 +1739,8 @@ def mlstm_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tenso
         raise RuntimeError("mlstm_scan: gate or state shapes do not fit")
     out = empty_rows(T, heads * vdim, q.dtype, q.device)
     # (400 - 447 tokens pay for two more launches where there are heads enough: 1 x 420 of 8 heads 98 / 105 us, 2 x 420 of 16 126 / 106)
-    least = 448 if seq.longest is None or T * heads < 6144 else 400
-    segment = _scan_segment(T, seq.batch_size, heads, 512 if dim == 64 and vdim == 64 else 256, least, seq.longest, 2.5) if \
+    segment = _scan_segment(T, seq.batch_size, heads, 512 if dim == 64 and vdim == 64 else 256,
+                            448 if seq.longest is None or T * heads < 6144 else 400, seq.longest, 2.5) if \
         _scan_segments_take((q, k, v), dim, vdim, seq) and max(g.stride(0), out.stride(0)) < 1 << 24 else 0
     if segment:
         work = torch.empty(load().sp_scan_segment_floats(T, seq.batch_size, heads, dim, vdim, segment), dtype=torch.float32, device=q.device)
