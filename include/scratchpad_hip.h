@@ -692,7 +692,9 @@ SP_API int sp_delta_recurrence(void* out, int64_t out_stride, const void* r, int
                                void* stream);
 /* The same for steps of several tokens per request, 16 tokens at a time on the matrix cores (fp32 throughout): head_dim 64, rows of r, k,
  * v and g 16-byte aligned; else SP_ERR_UNSUPPORTED and nothing is launched.  Products of up to 16 decays are formed (never quotients):
- * those in [0, 1] cannot overflow.  work: fp32, sp_delta_recurrence_chunk_floats values, 16-byte aligned.                      */
+ * those in [0, 1] cannot overflow.  work: fp32, sp_delta_recurrence_chunk_floats values, 16-byte aligned: 21.5 KB per 16 tokens and head
+ * (43 KB per token of 32 heads), 192 MiB at the most and 12 bytes per request and further pass - a larger step goes through it in passes,
+ * the states through the pool.                                                                                                  */
 SP_API int64_t sp_delta_recurrence_chunk_floats(int64_t num_tokens, int batch_size, int heads, int head_dim);
 SP_API int sp_delta_recurrence_chunks(void* out, int64_t out_stride, const void* r, int64_t r_stride, const void* k, int64_t k_stride,
                                       const void* v, int64_t v_stride, const void* g, int64_t g_stride, const float* decay,
@@ -714,9 +716,11 @@ SP_API int sp_hgrn2_scan(void* out, int64_t out_stride, const void* qpre, int64_
                          SP_SEQ_PARAMS, int dtype, void* stream);
 /* The same for steps of several tokens per request, 16 tokens at a time on the matrix cores (fp32 throughout): dim and vdim 64 or 128,
  * rows of qpre, fpre and v 16-byte aligned; else SP_ERR_UNSUPPORTED and nothing is launched.  Products of up to 16 gates are formed (never
- * quotients).  work: fp32, sp_hgrn2_chunk_floats values, 16-byte aligned.  segment_tokens > 0 (a multiple of 16): a request's tokens are
- * shared out in segments that run side by side, segment_work (fp32, 16-byte aligned) holds sp_hgrn2_segment_floats values.          */
+ * quotients).  work: fp32, sp_hgrn2_chunk_floats values, 16-byte aligned: 18 KB (dim 64: 10) per 16 tokens and head, 192 MiB at the most,
+ * as above; sp_hgrn2_window_tokens: what a pass takes.  segment_tokens > 0 (a multiple of 16): a request's tokens (of a pass) are shared out
+ * in segments that run side by side, segment_work (fp32, 16-byte aligned) holds sp_hgrn2_segment_floats values.                     */
 SP_API int64_t sp_hgrn2_chunk_floats(int64_t num_tokens, int batch_size, int heads, int dim);
+SP_API int64_t sp_hgrn2_window_tokens(int heads, int dim);
 SP_API int64_t sp_hgrn2_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim, int segment_tokens);
 SP_API int sp_hgrn2_chunks(void* out, int64_t out_stride, const void* qpre, int64_t q_stride, const void* fpre, int64_t f_stride,
                            const void* v, int64_t v_stride, const float* f_bias, const float* lower, const float* norm_w, float* state,

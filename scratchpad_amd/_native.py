@@ -172,6 +172,7 @@ SIGNATURES = {
     "sp_delta_step": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i32, _f32,
                              _vp, _vp, _i64, _i32, _i32, _f32, *_SEQ, _i32, _vp]),
     "sp_hgrn2_chunk_floats": (_i64, [_i64, _i32, _i32, _i32]),
+    "sp_hgrn2_window_tokens": (_i64, [_i32, _i32]),
     "sp_hgrn2_segment_floats": (_i64, [_i64, _i32, _i32, _i32, _i32, _i32]),
     "sp_hgrn2_chunks": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _i32, _i64, _i32, _i32, _i32,
                                _f32, *_SEQ, _i32, _vp]),
@@ -1946,7 +1947,9 @@ def hgrn2_scan(qpre: torch.Tensor, fpre: torch.Tensor, v: torch.Tensor, f_bias: 
         raise RuntimeError("hgrn2_scan: f_bias, lower [H*D], norm_w [vdim], state [slots, H, D, vdim]")
     out = empty_rows(T, heads * vdim, qpre.dtype, qpre.device)
     if _hgrn2_chunks_take((qpre, fpre, v), seq, dim, vdim) and hgrn2_chunks_pay(T, seq.batch_size, heads, seq.longest):
-        lib, segment = load(), _hgrn2_segment(T, seq.batch_size, heads, seq.longest)
+        lib = load()
+        window = lib.sp_hgrn2_window_tokens(heads, dim)              # (a larger step goes through the kernels in passes of so many tokens)
+        segment = _hgrn2_segment(min(T, window), seq.batch_size, heads, seq.longest and min(seq.longest, window))
         work = torch.empty(lib.sp_hgrn2_chunk_floats(T, seq.batch_size, heads, dim), dtype=torch.float32, device=qpre.device)
         sums = torch.empty(lib.sp_hgrn2_segment_floats(T, seq.batch_size, heads, dim, vdim, segment), dtype=torch.float32,
                            device=qpre.device) if segment else None

@@ -26,6 +26,8 @@
 #pragma once
 #include "chunk_scan.h"
 
+#include <algorithm>
+
 namespace sp {
 
 constexpr int kC16 = 16;
@@ -538,5 +540,99 @@ inline bool rows_aligned(const void* p, int64_t stride, int dtype) {
 }
 
 inline int64_t chunk16_units(int64_t tokens, int B) { return tokens / kC16 + B; }      // at most: a request's last chunk may be partial
+
+// ---- windows: a step's chunks in passes over one bounded workspace ----------------------------------------------------------------
+// A chunk's prepared operands take 18 - 21 KB per head, so a step takes the chunks that 192 MiB hold at a time (general delta rule, 32 heads
+// of 64: 4672 tokens; HGRN2, 8 heads of 128: 21840), and a request's state goes from pass to pass through the pool.  A window
+// is a range of the chunks in the order (chunk within its request, request): all requests advance side by side in every pass.  To the
+// kernels it is a step of its own - lengths, prefixes and first rows of the requests' pieces (each 16 tokens a chunk but a request's last,
+// so the chunks and their bits are the same).  us, whole step at once -> in passes (scratch in MB): general delta rule 1 x 16384 2851 -> 2875 (736
+// -> 256 with the rows out), 16 x 1024 663 -> 738, 16 x 2048 1289 -> 1459 (1482 -> 319), 1 x 65536 11419 -> 11423 (2944 -> 447); HGRN2 1 x 65536
+// 973 -> 1062, 16 x 2048 524 -> 568.
+constexpr int64_t kChunk16Work = (int64_t)192 << 20;
+
+inline int64_t chunk16_window(int H, int floats) { return std::max<int64_t>(1, kChunk16Work / ((int64_t)H * floats * (int64_t)sizeof(float))); }
+inline int64_t chunk16_work_floats(int64_t tokens, int B, int H, int floats) {
+  const int64_t units = chunk16_units(tokens, B), per = chunk16_window(H, floats);
+  return std::min(units, per) * H * floats + (units > per ? (units + per - 1) / per * 3 * B : 0);
+}
+
+__device__ __forceinline__ int block_count(int v, int* red) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return (red[0] + red[1]) + (red[2] + red[3]);
+}
+// the rounds (a chunk of every request that has one) among the first `rank` chunks, and how many chunks of the round after: by a block of 256
+__device__ __forceinline__ void rounds_of(const SeqBatch& s, int rank, int longest, int* red, int& rounds, int& rest) {
+  const auto chunks = [&](int c) {
+    int n = 0;
+    for (int b = threadIdx.x; b < s.B; b += 256) n += min(segments_of(max(s.extend_seq_lens[b], 0), kC16), c);
+    return block_count(n, red);
+  };
+  int lo = 0, hi = longest;                            // the most rounds with at most `rank` chunks
+  while (lo < hi) {
+    const int mid = lo + (hi - lo + 1) / 2;
+    if (chunks(mid) <= rank) lo = mid;
+    else hi = mid - 1;
+  }
+  rounds = lo;
+  rest = rank - chunks(lo);
+}
+// Workgroup: window blockIdx.x.  tables: [window][length, prefix, first row][request]
+static __global__ void __launch_bounds__(256) chunk16_windows_kernel(int32_t* tables, SeqBatch s, int per) {
+  __shared__ int red[4];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  int longest = 0;
+  for (int b = threadIdx.x; b < s.B; b += 256) longest = max(longest, segments_of(max(s.extend_seq_lens[b], 0), kC16));
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off, 64));
+  if (lane == 0) red[wave] = longest;
+  __syncthreads();
+  longest = max(max(red[0], red[1]), max(red[2], red[3]));
+  int rounds[2], rest[2];
+  for (int i = 0; i < 2; ++i) rounds_of(s, (int)(blockIdx.x + i) * per, longest, red, rounds[i], rest[i]);
+  int before[2] = {0, 0};                              // requests below this tile of 256 with a chunk in the round that a bound cuts
+  int32_t* table = tables + (int64_t)blockIdx.x * 3 * s.B;
+  for (int b0 = 0; b0 < s.B; b0 += 256) {
+    const int b = b0 + threadIdx.x, len = b < s.B ? max(s.extend_seq_lens[b], 0) : 0, n = segments_of(len, kC16);
+    int at[2];
+    for (int i = 0; i < 2; ++i) {
+      const uint64_t has = __ballot(n > rounds[i]);
+      __syncthreads();
+      if (lane == 0) red[wave] = __popcll(has);
+      __syncthreads();
+      int below = before[i] + __popcll(has & ((1ull << lane) - 1));
+      for (int w = 0; w < wave; ++w) below += red[w];
+      at[i] = min(n, rounds[i]) + (n > rounds[i] && below < rest[i] ? 1 : 0);
+      before[i] += (red[0] + red[1]) + (red[2] + red[3]);
+    }
+    if (b < s.B) {
+      table[b] = min(len, at[1] * kC16) - min(len, at[0] * kC16);
+      table[s.B + b] = s.extend_prefix_lens[b] + at[0] * kC16;
+      table[2 * s.B + b] = s.extend_start_loc[b] + at[0] * kC16;
+    }
+  }
+}
+
+// launch(the step or a window of it, its chunks and tokens at the most) for every window of the step
+template <typename Launch>
+int each_window16(float* work, int64_t tokens, int H, int floats, const SeqBatch& s, hipStream_t st, const Launch& launch) {
+  const int64_t units = chunk16_units(tokens, s.B), per = chunk16_window(H, floats);
+  if (units <= per) return launch(s, units, tokens);
+  const int windows = (int)((units + per - 1) / per);
+  int32_t* table = (int32_t*)(work + per * H * floats);
+  chunk16_windows_kernel<<<dim3((unsigned)windows), 256, 0, st>>>(table, s, (int)per);
+  SP_LAUNCH_CHECK();
+  for (int w = 0; w < windows; ++w, table += 3 * s.B) {
+    SeqBatch piece = s;
+    piece.extend_seq_lens = table, piece.extend_prefix_lens = table + s.B, piece.extend_start_loc = table + 2 * s.B;
+    const int rc = launch(piece, per, per * kC16);
+    if (rc != SP_OK) return rc;
+  }
+  return SP_OK;
+}
 
 }  // namespace sp

@@ -391,11 +391,13 @@ delta_prepare_kernel(float* work, const char* r, int64_t r_stride, const char* k
 
 template <typename Tag>
 static int launch_delta_chunks16(Tag, const Walk16& w, float* work, const void* r, int64_t r_stride, const void* k, int64_t k_stride,
-                                 const float* decay, const float* remove, int64_t tokens, const SeqBatch& s, hipStream_t st) {
-  delta_prepare_kernel<Tag, 64><<<dim3((unsigned)chunk16_units(tokens, s.B), (unsigned)w.H), 256, 0, st>>>(
-      work, (const char*)r, r_stride, (const char*)k, k_stride, decay, remove, s, w.H);
-  SP_LAUNCH_CHECK();
-  return launch_walk16<Tag, 64, 4, true>(w, tokens, s, st);
+                                 const float* decay, const float* remove, int64_t num_tokens, const SeqBatch& step, hipStream_t st) {
+  return each_window16(work, num_tokens, w.H, Chunk16<64, true>::kFloats, step, st, [&](const SeqBatch& s, int64_t units, int64_t tokens) -> int {
+    delta_prepare_kernel<Tag, 64><<<dim3((unsigned)units, (unsigned)w.H), 256, 0, st>>>(
+        work, (const char*)r, r_stride, (const char*)k, k_stride, decay, remove, s, w.H);
+    SP_LAUNCH_CHECK();
+    return launch_walk16<Tag, 64, 4, true>(w, tokens, s, st);
+  });
 }
 
 }  // namespace
@@ -442,7 +444,7 @@ extern "C" int sp_delta_recurrence(void* out, int64_t out_stride, const void* r,
 }
 
 extern "C" int64_t sp_delta_recurrence_chunk_floats(int64_t num_tokens, int batch_size, int heads, int head_dim) {
-  return head_dim == 64 ? chunk16_units(num_tokens, batch_size) * heads * Chunk16<64, true>::kFloats : 0;
+  return head_dim == 64 && heads > 0 ? chunk16_work_floats(num_tokens, batch_size, heads, Chunk16<64, true>::kFloats) : 0;
 }
 
 extern "C" int sp_delta_recurrence_chunks(void* out, int64_t out_stride, const void* r, int64_t r_stride, const void* k, int64_t k_stride,

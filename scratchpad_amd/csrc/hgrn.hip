@@ -223,11 +223,13 @@ hgrn2_prepare_kernel(float* work, const char* qpre, int64_t q_stride, const char
 
 template <typename Tag, int D, int NW>
 static int launch_hgrn2_chunks(const Walk16& w, float* work, const void* qpre, int64_t q_stride, const void* fpre, int64_t f_stride,
-                               const float* f_bias, const float* lower, int64_t tokens, const SeqBatch& s, hipStream_t st) {
-  hgrn2_prepare_kernel<Tag, D><<<dim3((unsigned)chunk16_units(tokens, s.B), (unsigned)w.H), 256, 0, st>>>(
-      work, (const char*)qpre, q_stride, (const char*)fpre, f_stride, f_bias, lower, s, w.H);
-  SP_LAUNCH_CHECK();
-  return launch_walk16<Tag, D, NW, false>(w, tokens, s, st);
+                               const float* f_bias, const float* lower, int64_t num_tokens, const SeqBatch& step, hipStream_t st) {
+  return each_window16(work, num_tokens, w.H, Chunk16<D, false>::kFloats, step, st, [&](const SeqBatch& s, int64_t units, int64_t tokens) -> int {
+    hgrn2_prepare_kernel<Tag, D><<<dim3((unsigned)units, (unsigned)w.H), 256, 0, st>>>(
+        work, (const char*)qpre, q_stride, (const char*)fpre, f_stride, f_bias, lower, s, w.H);
+    SP_LAUNCH_CHECK();
+    return launch_walk16<Tag, D, NW, false>(w, tokens, s, st);
+  });
 }
 
 }  // namespace
@@ -251,12 +253,19 @@ extern "C" int sp_hgrn2_scan(void* out, int64_t out_stride, const void* qpre, in
                                                      (hipStream_t)stream)));
 }
 
+static int hgrn2_unit_floats(int dim) { return dim == 64 ? Chunk16<64, false>::kFloats : Chunk16<128, false>::kFloats; }
+
 extern "C" int64_t sp_hgrn2_chunk_floats(int64_t num_tokens, int batch_size, int heads, int dim) {
-  return chunk16_units(num_tokens, batch_size) * heads * (dim == 64 ? Chunk16<64, false>::kFloats : Chunk16<128, false>::kFloats);
+  return heads > 0 ? chunk16_work_floats(num_tokens, batch_size, heads, hgrn2_unit_floats(dim)) : 0;
+}
+
+extern "C" int64_t sp_hgrn2_window_tokens(int heads, int dim) {
+  return heads > 0 ? chunk16_window(heads, hgrn2_unit_floats(dim)) * kC16 : 0;
 }
 
 extern "C" int64_t sp_hgrn2_segment_floats(int64_t num_tokens, int batch_size, int heads, int dim, int vdim, int segment_tokens) {
-  return segment_tokens > 0 ? (num_tokens / segment_tokens + batch_size) * heads * ((int64_t)dim * vdim + dim) : 0;
+  const int64_t tokens = std::min(num_tokens, sp_hgrn2_window_tokens(heads, dim));
+  return segment_tokens > 0 ? (tokens / segment_tokens + batch_size) * heads * ((int64_t)dim * vdim + dim) : 0;
 }
 
 extern "C" int sp_hgrn2_chunks(void* out, int64_t out_stride, const void* qpre, int64_t q_stride, const void* fpre, int64_t f_stride,

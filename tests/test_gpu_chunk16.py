@@ -157,3 +157,66 @@ def test_delta_numbers_that_are_not_finite_reach_no_earlier_token(at, where, bad
         assert not torch.isfinite(out[at:, 0, 3].float()).any() and not torch.isfinite(S[0, :, 3]).any()
     else:
         assert not torch.isfinite(out[at + 1:, 0].float()).any() and not torch.isfinite(S[0, 3]).any()
+
+
+WINDOW_LENS = [[400], [130, 0, 16, 1, 250], [5] * 40 + [200, 33], [17] * 300]
+
+
+def window_problem(H, cols, lens, seed):
+    """heads so many that a step of these lengths takes several passes over the workspace; half of the requests hold a state"""
+    from scratchpad_amd import _native
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    T, prefixes, slots = sum(lens), [(3 * i) % 2 * 7 for i in range(len(lens))], list(range(1, len(lens) + 1))
+    return g, T, seq_extend(lens, prefixes, slots), len(lens) + 1, _native
+
+
+@pytest.mark.parametrize("lens", WINDOW_LENS, ids=lambda l: "-".join(map(str, l[:5])))
+def test_delta_recurrence_in_passes_over_a_bounded_workspace(lens, monkeypatch):
+    """1024 heads: 9 chunks a pass; the heads' bits are those of the same heads in a step of one pass"""
+    H, D, sub = (128 if len(lens) > 100 else 1024), 64, 2
+    g, T, seq, slots, nat = window_problem(H, D, lens, 31)
+    announce("delta recurrence in passes", lens[:5], H)
+    monkeypatch.setattr(nat, "DELTA_RECURRENCE_CHUNKS", True)
+    floats = nat.load().sp_delta_recurrence_chunk_floats
+    assert 4 * floats(T, len(lens), H, D) <= (192 << 20) + 12 * len(lens) * 200 < 4 * 5376 * H * (T // 16 + len(lens))
+    rows = torch.randn(T, 4 * H * D, generator=g, device=DEV).bfloat16()
+    w = torch.exp(-0.6 * torch.rand(T, H * D, generator=g, device=DEV))
+    a, nw = torch.rand(T, H * D, generator=g, device=DEV), torch.rand(H * D, generator=g, device=DEV) + 0.5
+    S = torch.randn(slots, H, D, D, generator=g, device=DEV)
+    start = S.clone()
+    out = nat.delta_recurrence(*rows.split(H * D, 1), w, a, nw, S, seq, H, D, 1e-5)
+    assert torch.equal(S[0], start[0])
+    for h in (0, H // 2 - 1, H - sub):
+        cut = slice(h * D, (h + sub) * D)
+        part = start[:, h:h + sub].contiguous()
+        few = nat.delta_recurrence(*(x[:, cut] for x in rows.split(H * D, 1)), w[:, cut].contiguous(), a[:, cut].contiguous(), nw[cut].contiguous(),
+                                   part, seq, sub, D, 1e-5)
+        assert torch.isfinite(few.float()).all() and torch.equal(out[:, cut], few) and torch.equal(S[:, h:h + sub], part)
+
+
+@pytest.mark.parametrize("lens", WINDOW_LENS, ids=lambda l: "-".join(map(str, l[:5])))
+@pytest.mark.parametrize("segment", [0, 64])
+def test_hgrn2_in_passes_over_a_bounded_workspace(lens, segment, monkeypatch):
+    """512 heads of 128: 21 chunks a pass; bit for bit without segments, with them within their own roundings"""
+    H, D, sub = (64 if len(lens) > 100 else 512), 128, 2
+    g, T, seq, slots, nat = window_problem(H, D, lens, 32)
+    announce("hgrn2 in passes", lens[:5], H, segment)
+    monkeypatch.setattr(nat, "HGRN2_CHUNKS", True)
+    assert 4 * nat.load().sp_hgrn2_chunk_floats(T, len(lens), H, D) <= (192 << 20) + 12 * len(lens) * 200 < 4 * 4608 * H * (T // 16 + len(lens))
+    rows = torch.randn(T, 3 * H * D, generator=g, device=DEV).bfloat16()
+    fb, lower = torch.randn(H * D, generator=g, device=DEV), torch.rand(H * D, generator=g, device=DEV) * 0.5
+    nw, S = torch.rand(D, generator=g, device=DEV) + 0.5, torch.randn(slots, H, D, D, generator=g, device=DEV)
+    start = S.clone()
+    monkeypatch.setattr(nat, "SCAN_SEGMENT", segment)
+    out = nat.hgrn2_scan(*rows.split(H * D, 1), fb, lower, nw, S, seq, H, D, D, 1e-5)
+    assert torch.equal(S[0], start[0])
+    monkeypatch.setattr(nat, "SCAN_SEGMENT", 0)
+    for h in (0, H // 2 - 1, H - sub):
+        cut = slice(h * D, (h + sub) * D)
+        part = start[:, h:h + sub].contiguous()
+        few = nat.hgrn2_scan(*(x[:, cut] for x in rows.split(H * D, 1)), fb[cut].contiguous(), lower[cut].contiguous(), nw, part, seq, sub, D, D, 1e-5)
+        if segment == 0:
+            assert torch.isfinite(few.float()).all() and torch.equal(out[:, cut], few) and torch.equal(S[:, h:h + sub], part)
+        else:
+            near(S[:, h:h + sub], part.double())
+            assert ((out[:, cut].double() - few.double()).abs() <= 2 * HALF[torch.bfloat16] * few.double().abs() + 1e-3).all()
