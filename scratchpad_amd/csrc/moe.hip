@@ -158,9 +158,10 @@ __global__ void moe_softmax_topk_kernel(int32_t* ids, float* weights, float* gat
 }
 
 // ---- pairs ordered by expert: offsets[E + 1], order[pos] = pair, place[pair] = pos.  One workgroup. ---------------
-// Bound by its chain of latencies.  A pair's place inside its expert is what the count gave back, so the counters are gone through once;
-// a thread's ids are on their way together (up to 16384 pairs they stay in registers), the sums over experts go 64 at a time, and the order
-// is written in rows out of LDS.  16384 pairs of 32 experts: 14.6 -> 8.8 us (scattered stores of the order: 10.5); 32 pairs: 2.9 -> 2.3.
+// Bound by its chain of latencies.  Up to 16384 pairs a thread's ids are on their way together and stay in registers, and a pair's place
+// inside its expert is what the count gave back, so the counters are gone through once; the order is written in rows out of LDS.  More
+// pairs go through the counters a second time (the count's answer kept in `place` meanwhile: 65536 pairs of 32 experts 41 us, so 34).  The
+// sums over experts go 64 at a time.  16384 pairs of 32 experts: 14.6 -> 8.8 us (scattered stores of the order: 10.5); 32 pairs: 2.9 -> 2.3.
 constexpr int kAlignThreads = 1024, kAlignHeld = 16, kAlignPairs = kAlignThreads * kAlignHeld;
 
 __global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(int32_t* offsets, int32_t* order, int32_t* place, const int32_t* ids, int P,
@@ -187,7 +188,7 @@ __global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(int32_t* offse
       if (i * kAlignThreads + tid < P) rank[i] = atomicAdd(&cnt[id[i]], 1);
     }
   } else {
-    for (int p = tid; p < P; p += kAlignThreads) place[p] = atomicAdd(&cnt[ids[p]], 1);
+    for (int p = tid; p < P; p += kAlignThreads) atomicAdd(&cnt[ids[p]], 1);
   }
   __syncthreads();
   if (tid < 64) {
@@ -222,7 +223,7 @@ __global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(int32_t* offse
     for (int i = tid; i < P; i += kAlignThreads) order[i] = sorted[i];
   } else {
     for (int p = tid; p < P; p += kAlignThreads) {
-      const int pos = first[ids[p]] + place[p];
+      const int pos = atomicAdd(&first[ids[p]], 1);
       order[pos] = p;
       place[p] = pos;
     }
