@@ -5,6 +5,7 @@
 // a fixed order, so a token's result does not depend on which other tokens share the step.
 #include "seq_batch.h"
 
+#include <cmath>
 #include <type_traits>
 
 namespace sp {
@@ -715,14 +716,8 @@ __global__ void __launch_bounds__(64) moe_grouped_rows_kernel(GroupedArgs p) {
   }
 }
 
-// The same with half the weight rows per wave (16; GLU: 8 gate rows and their 8 up rows) and twice the k-steps on their way, while
-// the kernel above would have at most one wave per compute unit (were every pair another expert's) and leave units idle.  us of the up
-// and down product, kernel above -> this, top 4 of 32 experts: 1 token of 2048 x 1024 (256 waves each) 10.7 + 6.8 -> 10.0 + 6.2, of
-// 1024 x 512 (128 waves) 6.7 + 4.1 -> 5.4 + 3.5, 2 tokens of 1024 x 512 (256) 6.9 + 4.1 -> 6.8 + 4.0.  Past that the second reading of
-// x's rows costs as much as the evener shares give, or more: 2 tokens of 2048 x 1024 (512 waves) 13.3 + 7.8 -> 15.4 + 8.2, 4 tokens
-// 21.2 + 11.9 -> 21.9 + 11.8, 8 tokens 29.8 + 17.4 -> 31.0 + 16.6, 16 tokens 39.2 + 21.3 -> 44.1 + 23.0; top 8 of 64, 4 tokens
-// 40.3 + 20.9 -> 45.9 + 22.2.
-constexpr long kNarrowWaves = 256;
+// The same with half the weight rows per wave (16; GLU: 8 gate rows and their 8 up rows) and twice the k-steps on their way, where
+// narrow_pays below.
 constexpr int kNarrowUnroll = 16;
 
 template <typename Tag, int ACT>
@@ -763,6 +758,20 @@ __global__ void __launch_bounds__(64) moe_grouped_narrow_rows_kernel(GroupedArgs
   store4<Tag>(p, row0 + r16, n0 + 4 * q, v);
 }
 
+// Half the weight rows per wave, of a product with `blocks` column blocks of the wider kernel:
+//   * at most one wave per compute unit, were every pair another expert's: units are idle.  us of the up and down product, wider -> narrow,
+//     top 4 of 32 experts: 1 token of 2048 x 1024 (256 waves each) 10.7 + 6.8 -> 10.0 + 6.2, of 1024 x 512 (128 waves) 6.7 + 4.1 -> 5.4 + 3.5;
+//   * one to one and a half waves per SIMD (four to a unit) of the experts that so many pairs are expected to choose: the SIMDs with a second
+//     wave set the time, and half a wave more does less to them.  Layers, mean of 8 routings (single ones 0.91 - 1.07): 32 experts of
+//     2048 x 1024, 6 - 8 tokens 59.9 -> 58.9, 64 experts, top 4, 6 tokens 61.5 -> 60.8, of 1024 x 512, top 8, 8 tokens 43.8 -> 43.2.
+// Elsewhere the second reading of x's rows costs as much as the evener shares give, or more: 2 tokens of 2048 x 1024 (512 waves) 13.3 + 7.8
+// -> 15.4 + 8.2; 64 experts, top 8, 4 tokens (1660) 80.3 -> 85.5; 16 tokens of 32 experts 39.2 + 21.3 -> 44.1 + 23.0.
+static bool narrow_pays(int pairs, int experts, int blocks) {
+  if (pairs > experts) return false;
+  const double chosen = experts * (1. - pow(1. - 1. / experts, pairs)) * blocks;
+  return (long)pairs * blocks <= 256 || (chosen > 1024. && chosen <= 1536.);
+}
+
 // Which kernel: by the mean rows per expert, pairs / experts (the counts themselves are on the device).  Measured at width 2048,
 // 32 experts of ff 1024, top 4, up + down product in us (rows kernel | 64-row tiles | 128-row tiles):
 //   mean rows 1: 60 | 68 | 73     4: 85 | 92 | 94     8: 86 | 92 | 94     16: 104 | 93 | 96     32: 161 | 95 | 99
@@ -779,7 +788,7 @@ int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
   // (moe_align takes 4096 experts, 6656 tiles; more than a grid's second dimension holds go to the 64-row tiles)
   if (pairs <= 10 * (int64_t)p.E && row_tiles <= 65535) {
     const int wide_per = ACT >= 2 ? 16 : 32;
-    const bool narrow = pairs <= p.E && (long)pairs * ((p.N + wide_per - 1) / wide_per) <= kNarrowWaves;
+    const bool narrow = narrow_pays(pairs, p.E, (p.N + wide_per - 1) / wide_per);
     const int per = narrow ? wide_per / 2 : wide_per;
     const dim3 grid((unsigned)((p.N + per - 1) / per), (unsigned)row_tiles);
     if (narrow) moe_grouped_narrow_rows_kernel<Tag, ACT><<<grid, 64, 0, st>>>(p);

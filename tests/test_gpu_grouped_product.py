@@ -67,10 +67,10 @@ def test_gated_form_is_the_two_steps(counts, ff, K, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("K", [480, 512, 544, 1024, 1056])
-@pytest.mark.parametrize("E,pairs,N", [(8, 4, 512), (8, 4, 1024), (8, 4, 1028), (8, 8, 513), (16, 2, 2048), (8, 9, 256)])
+@pytest.mark.parametrize("E,pairs,N", [(8, 4, 512), (8, 4, 1024), (8, 4, 1028), (8, 8, 513), (16, 2, 2048), (8, 9, 256), (32, 24, 1024)])
 def test_few_pairs_have_the_bits_of_many(E, pairs, N, K, dtype):
-    """few pairs over whole and partial rounds of k-steps, at both sides of the line of one wave per compute unit: the bits of the same
-    rows beside so many others that another kernel takes them, in the product and in its gated form"""
+    """few pairs over whole and partial rounds of k-steps, at both sides of the line of one wave per compute unit and at one to one and a
+    half per SIMD: the bits of the same rows beside so many others that another kernel takes them, in the product and in its gated form"""
     from scratchpad_amd import _native
     print("few pairs", E, pairs, N, K, dtype, flush=True)
     g = torch.Generator(device=DEV).manual_seed(6)
