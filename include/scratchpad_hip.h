@@ -352,6 +352,16 @@ SP_API int sp_top_k_top_p_min_p_renorm(const float* probs, int64_t row_stride, c
 SP_API int sp_gemm_skinny(void* out, const void* x, const void* w, int M, int N, int K, int64_t x_stride,
                    int64_t w_stride, int64_t out_stride, int epilogue, int dtype, void* stream);
 
+/* ---- The same product for more rows (decode steps of a full batch, short prompts): x [M, K], w [N, K], K % 64 == 0, fp16/bf16, fp32
+ *      accumulation, one rounding; M * x_stride and the weight rows * w_stride below 2^31 elements.  sp_gemm_dense_plan: how it is
+ *      cut - tile + 256 * shares of K - by sizes alone (host code; -1: no tile takes it).  `sums`: shares * M * N floats (16-byte
+ *      aligned) where a plan has more than one share, else unused.  epilogue 1: w is [2 N, K], gate rows then up rows, and out
+ *      the rounded silu(gate) * up of the rounded sums, bit for bit the plain call followed by sp_silu_and_mul; its plans have one
+ *      share, and there are none where the plain product's has more. */
+SP_API int sp_gemm_dense_plan(int M, int N, int K, int epilogue);
+SP_API int sp_gemm_dense(void* out, const void* x, const void* w, float* sums, int64_t sums_floats, int M, int N, int K,
+                         int64_t x_stride, int64_t w_stride, int64_t out_stride, int epilogue, int plan, int dtype, void* stream);
+
 /* ---- Direct all-reduce through IPC-mapped peer regions: fills GroupCoordinator.ca_comm
  *      (distributed/parallel_state.py:266-267, 326-347; the reference never constructs one and always
  *      calls NCCL, linear.py:1148-1149).  Each rank sp_ar_alloc()s one fine-grained region of

@@ -106,6 +106,8 @@ SIGNATURES = {
     "sp_fused_allreduce_add_rmsnorm": (_i32, [_vp, _vp, _vp, _i64, _i32, _i64, _i64, _f32, _i32, _vp, _i32, _i32,
                                               _sz, _i64, _vp, _vp]),
     "sp_gemm_skinny": (_i32, [_vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i64, _i32, _i32, _vp]),
+    "sp_gemm_dense_plan": (_i32, [_i32, _i32, _i32, _i32]),
+    "sp_gemm_dense": (_i32, [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i64, _i64, _i64, _i32, _i32, _i32, _vp]),
     # ---- ABI 10 (_SEQ: the header's SP_SEQ_PARAMS)
     "sp_bigram_rows": (_i32, [_vp, _vp, _vp, _i64, *_SEQ, _i64, _i64, _i64, _vp]),
     "sp_save_last_token": (_i32, [_vp, _vp, *_SEQ, _vp]),
@@ -854,6 +856,74 @@ def library_rows_report() -> dict:
             "substituted": {f"N={n} K={k} M={m}": mp for (n, k, m), mp in sorted(_LIBROWS_USED.items())}}
 
 
+# --------------------------------------------------------------------------- products of 17 rows and more
+DENSE_MAX_ROWS = 256          # and to 640 of long rows: dense_gemm_pays
+_DENSE_ON = os.environ.get("SP_DENSE_GEMM", "1") != "0"
+_DENSE_PLANS = {}             # (M, N, K, epilogue) -> sp_gemm_dense_plan: sizes alone, at most 640 row counts per projection
+
+
+def dense_gemm_pays(M: int, N: int, K: int) -> bool:
+    """Where sp_gemm_dense measured faster than hipBLASLt on MI355X (us under graph replay, cold weights, library / own): 17 - 256
+    rows of most shapes (the table in gemm_dense.hip; mean 0.83 of the library's time over 21 shapes).  Past that the library's large
+    tiles win (320 rows: 28672 x 4096 79 / 98, 3072 x 2048 11.1 / 14.6) but where K is three times N it still runs few of them:
+    2048 x 8192 33 / 26 at 320 and 44 / 36 at 640 rows, 4096 x 14336 75 / 55 and 109 / 94, both even at 777 (1024 x 8192 22.6 / 24.2 at 512).
+    Left to the library below that: up to 512 weight rows, where it depends on K and rows (512 x 2048 5.5 / 6.7, 512 x 4096 11.7 / 7.1 at 64
+    rows); up to 2048 of them at K 2560 - 4096 past 64 rows (2048 x 4096 11.1 / 10.3 at 64 rows, 10.6 / 11.2 at 128, 1024 x 4096 12.2 / 8.0
+    and 9.4 / 9.6, 1536 x 4096 9.4 / 10.2 at 96); heads past 65536 columns with K <= 2048 from 96 rows on (128256 x 2048: 96 rows
+    131 / 130, 128 134 / 142, 192 142 / 155)."""
+    if K % 64 or M <= SKINNY_MAX_ROWS or N <= 512 or M > (640 if K >= 3 * N and N >= 2048 else DENSE_MAX_ROWS):
+        return False
+    if N <= 2048 and 2048 < K <= 4096:
+        return M <= 64
+    return N <= 65536 or K > 2048 or M < 96
+
+
+def _dense_plan(M: int, N: int, K: int, epilogue: int) -> int:
+    key = (M, N, K, epilogue)
+    plan = _DENSE_PLANS.get(key)
+    if plan is None:
+        plan = _DENSE_PLANS[key] = load().sp_gemm_dense_plan(M, N, K, epilogue)
+    return plan
+
+
+def _dense_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """a 16-bit product of rows on the GPU that sp_gemm_dense runs, and runs faster than the library; autograd, function transforms and
+    dispatch modes keep the library call they can see"""
+    if not _DENSE_ON or x.dim() != 2 or weight.dim() != 2 or not x.is_cuda or x.shape[1] != weight.shape[1]:
+        return False
+    dtype = x.dtype
+    if (dtype is not torch.bfloat16 and dtype is not torch.float16) or weight.dtype is not dtype or weight.device != x.device \
+            or not dense_gemm_pays(x.shape[0], weight.shape[0], weight.shape[1]):
+        return False
+    sx, sw = x.stride(), weight.stride()
+    if sx[1] != 1 or sw[1] != 1 or sx[0] % 8 or sw[0] % 8 or sx[0] < x.shape[1] or sw[0] < x.shape[1] \
+            or x.shape[0] * sx[0] >= 1 << 31 or weight.shape[0] * sw[0] >= 1 << 31:
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
+        return False
+    if torch._C._len_torch_dispatch_stack() or torch._C._functorch.peek_interpreter_stack() is not None \
+            or torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing() \
+            or type(x) not in _PLAIN or type(weight) not in _PLAIN:
+        return False
+    # a table that was calibrated on this box says how the library runs these projections
+    if (weight.shape[0], weight.shape[1]) in getattr(_LIBRARY_ROWS, "calibrated", ()):
+        return False
+    return x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _dense(x: torch.Tensor, weight: torch.Tensor, cols: int, epilogue: int, plan: int) -> torch.Tensor:
+    M, K = x.shape
+    out = empty_rows(M, cols, x.dtype, x.device)
+    splits = plan >> 8
+    sums = torch.empty(splits * M * cols, dtype=torch.float32, device=x.device) if splits > 1 else None
+    _check(load().sp_gemm_dense(out.data_ptr(), x.data_ptr(), weight.data_ptr(), _ptr(sums), 0 if sums is None else sums.numel(), M, cols, K,
+                                x.stride(0), weight.stride(0), out.stride(0), epilogue, plan, _dt(x), _stream()), "sp_gemm_dense")
+    return out
+
+
 _collector_lock = threading.Lock()
 _collector_off = 0          # captures under way
 _collector_was_on = False
@@ -904,13 +974,17 @@ def _time_mm(x: torch.Tensor, weights, reps: int = 3) -> float:
     return e0.elapsed_time(e1) / (reps * len(weights)) * 1e3
 
 
+class _CalibratedRows(dict):
+    calibrated = frozenset()          # the shapes that were timed, whether or not a row count replaced another
+
+
 def calibrate_library_rows(weights_by_shape, rows, min_gain: float = 0.05, step: int = 8) -> dict:
     """SP_LIBRARY_ROWS=auto.  weights_by_shape: {(N, K): [weight tensors of that shape]} (the model's own
     projections); rows: the batch-size buckets of the decode graphs.  Every (shape, M) is timed against
     M' = M + step .. M + ROW_SLACK; a substitute is kept only where it is at least `min_gain` faster than M
     itself ON THIS BOX.  Replaces the active table and returns it."""
     global _LIBRARY_ROWS
-    found = {}
+    found = _CalibratedRows()
     for (N, K), ws in weights_by_shape.items():
         ws = list(ws)[:8]
         if not ws or ws[0].dtype not in (torch.float16, torch.bfloat16) or not ws[0].is_cuda:
@@ -934,6 +1008,7 @@ def calibrate_library_rows(weights_by_shape, rows, min_gain: float = 0.05, step:
                     best_t, best_m = t, Mp
             if best_m != M and best_t <= base * (1.0 - min_gain):
                 found.setdefault((N, K), {})[M] = best_m
+    found.calibrated = frozenset(weights_by_shape)
     _LIBRARY_ROWS = found
     return found
 
@@ -969,6 +1044,16 @@ def linear_silu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor, any_rows: boo
     result [M, I].  Bit for bit the skinny projection followed by silu_and_mul.  None when the shape is not taken (the
     caller runs the two steps)."""
     return _skinny_glu(x, gate_up_weight, any_rows, 1, "sp_gemm_skinny(silu)")
+
+
+def dense_silu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """the same for the rows that sp_gemm_dense takes: bit for bit ``linear`` followed by silu_and_mul.  None when the projection is not one
+    of its own, or is one whose K is shared out."""
+    if not _SILU_LINEAR_ON or gate_up_weight.shape[0] % 2 or not _dense_takes(x, gate_up_weight):
+        return None
+    inter = gate_up_weight.shape[0] // 2
+    plan = _dense_plan(x.shape[0], inter, x.shape[1], 1)
+    return None if plan < 0 else _dense(x, gate_up_weight, inter, 1, plan)
 
 
 def linear_gelu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.Tensor:
@@ -1012,7 +1097,7 @@ def _skinny_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x @ weight.T.  Small-batch 16-bit products go to the weight-streaming kernel
-    (sp_gemm_skinny) where it pays; everything else is the library GEMM - exactly F.linear, except
+    (sp_gemm_skinny) where it pays, those of 17 rows and more to sp_gemm_dense where that does; everything else is the library GEMM - exactly F.linear, except
     that a product of at most SLACK_MAX_ROWS rows whose (shape, rows) is in the active library_rows
     table is computed over more rows than asked for (first M rows returned; rows are independent)."""
     if _skinny_takes(x, weight):
@@ -1022,6 +1107,11 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         _check(load().sp_gemm_skinny(out.data_ptr(), x.data_ptr(), weight.data_ptr(), M, N, K, x.stride(0),
                                      weight.stride(0), out.stride(0), 0, _dt(x), _stream()), "sp_gemm_skinny")
         return out
+    if _dense_takes(x, weight):
+        M, K = x.shape
+        plan = _dense_plan(M, weight.shape[0], K, 0)
+        if plan >= 0:
+            return _dense(x, weight, weight.shape[0], 0, plan)
     if (_LIBRARY_ROWS and x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= SLACK_MAX_ROWS and weight.dim() == 2
             and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and x.stride(1) == 1):
         M, K = x.shape

@@ -26,7 +26,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hi
 # allreduce.hip: its fused all-reduce + add + RMSNorm kernel reproduces elementwise.hip's norm bit for bit
 PER_FILE_FLAGS = {"elementwise.hip": ["-ffp-contract=off"], "allreduce.hip": ["-ffp-contract=off"],
                   # its epilogues repeat the roundings of elementwise.hip's activations
-                  "gemm_skinny.hip": ["-ffp-contract=off"],
+                  "gemm_skinny.hip": ["-ffp-contract=off"], "gemm_dense.hip": ["-ffp-contract=off"],
                   "extend_mfma.hip": ["-fno-honor-nans"],
                   # extend_w64.hip: every filler of its hand-placed MFMA gaps is a single instruction: no SLP packing
                   # of adjacent f32 adds / multiplies into v_pk_* (MI355X_MICROARCH.md: an anti-lever beside MFMAs).  Its
@@ -35,7 +35,7 @@ PER_FILE_FLAGS = {"elementwise.hip": ["-ffp-contract=off"], "allreduce.hip": ["-
                   "extend_w64.hip": ["-fno-honor-nans", "-fno-slp-vectorize", "-std=c++20", "-mllvm", "-amdgpu-atomic-optimizer-strategy=None"]}
 # Sources a model family needs beyond these: a model class names them (NATIVE_SOURCES) and build_native(only=...) makes
 # a library of just those, so the first start of a small model does not compile the attention kernels of another.
-CORE_SOURCES = ["elementwise.hip", "gemm_skinny.hip", "sampling.hip"]
+CORE_SOURCES = ["elementwise.hip", "gemm_skinny.hip", "gemm_dense.hip", "sampling.hip"]
 
 
 def _newer(target, deps):

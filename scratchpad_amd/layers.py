@@ -361,6 +361,10 @@ class GluFF(nn.Module):
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         if self.act == "gelu_tanh":
             return _native.linear(_native.linear_gelu_mul(h, self.gate_up), self.down)
+        if self.act == "silu":
+            y = _native.dense_silu_mul(h, self.gate_up)
+            if y is not None:
+                return _native.linear(y, self.down)
         gu = _native.linear(h, self.gate_up)
         y = _native.silu_and_mul(gu) if self.act == "silu" else _native.moe_glu(gu.contiguous(), self.limit, self.alpha)
         return _native.linear(y, self.down)

@@ -368,8 +368,10 @@ class LlamaMLP(nn.Module):
 
     def forward(self, x, reduce_output: bool = True):
         # small decode steps (<= _native.SILU_FUSED_MAX_ROWS tokens): projection and activation in one weight-streaming launch, the bits of
-        # the skinny projection followed by act_fn
+        # the skinny projection followed by act_fn; steps of 17 rows and more likewise where the tiled kernel takes the projection
         act = _native.linear_silu_mul(x, self.gate_up_proj.weight)
+        if act is None:
+            act = _native.dense_silu_mul(x, self.gate_up_proj.weight)
         if act is None:
             gate_up, _ = self.gate_up_proj(x)
             act = self.act_fn(gate_up)
