@@ -856,10 +856,10 @@ def library_rows_report() -> dict:
             "substituted": {f"N={n} K={k} M={m}": mp for (n, k, m), mp in sorted(_LIBROWS_USED.items())}}
 
 
-# --------------------------------------------------------------------------- products of 17 rows and more
+# --------------------------------------------------------------------------- products of more rows
 DENSE_MAX_ROWS = 256          # and to 640 of long rows: dense_gemm_pays
 _DENSE_ON = os.environ.get("SP_DENSE_GEMM", "1") != "0"
-_DENSE_PLANS = {}             # (M, N, K, epilogue) -> sp_gemm_dense_plan: sizes alone, at most 640 row counts per projection
+_DENSE_PLANS = {}             # (M, weight rows, K, epilogue) -> _dense_plan: sizes alone, at most 640 row counts per projection
 
 
 def dense_gemm_pays(M: int, N: int, K: int) -> bool:
@@ -870,8 +870,14 @@ def dense_gemm_pays(M: int, N: int, K: int) -> bool:
     Left to the library below that: up to 512 weight rows, where it depends on K and rows (512 x 2048 5.5 / 6.7, 512 x 4096 11.7 / 7.1 at 64
     rows); up to 2048 of them at K 2560 - 4096 past 64 rows (2048 x 4096 11.1 / 10.3 at 64 rows, 10.6 / 11.2 at 128, 1024 x 4096 12.2 / 8.0
     and 9.4 / 9.6, 1536 x 4096 9.4 / 10.2 at 96); heads past 65536 columns with K <= 2048 from 96 rows on (128256 x 2048: 96 rows
-    131 / 130, 128 134 / 142, 192 142 / 155)."""
-    if K % 64 or M <= SKINNY_MAX_ROWS or N <= 512 or M > (640 if K >= 3 * N and N >= 2048 else DENSE_MAX_ROWS):
+    131 / 130, 128 134 / 142, 192 142 / 155).
+    5 - 16 rows: matrices of more than 2^23 elements, where 16 rows of x beside every 16 weight rows are what sp_gemm_skinny waits for (that or
+    the library, whichever is faster / own, at 5 / 8 / 16 rows: 28672 x 4096 49 / 42, 54 / 43, 61 / 44; 2048 x 8192 13.1 / 11.6, 12.8 / 11.7, 13.3 / 11.9;
+    128256 x 4096 190 / 161, 193 / 162, 193 / 164; 4096 x 4096 10.2 / 9.9, 10.2 / 9.9, 11.5 / 10.1; 6144 x 2048 9.1 / 8.5, 9.4 / 8.5, 10.9 / 8.6); below that a
+    launch of small workgroups is over sooner (2048 x 4096 7.9 / 8.4, 3072 x 2048 5.7 / 6.8, 2048 x 2048 5.6 / 6.3)."""
+    if M <= SKINNY_MAX_ROWS:
+        return M > 4 and K % 64 == 0 and N * K > 1 << 23
+    if K % 64 or N <= 512 or M > (640 if K >= 3 * N and N >= 2048 else DENSE_MAX_ROWS):
         return False
     if N <= 2048 and 2048 < K <= 4096:
         return M <= 64
@@ -879,48 +885,54 @@ def dense_gemm_pays(M: int, N: int, K: int) -> bool:
 
 
 def _dense_plan(M: int, N: int, K: int, epilogue: int) -> int:
+    """sp_gemm_dense_plan of a product with N weight rows that dense_gemm_pays for, else -1"""
+    if M > 640:
+        return -1
     key = (M, N, K, epilogue)
     plan = _DENSE_PLANS.get(key)
     if plan is None:
-        plan = _DENSE_PLANS[key] = load().sp_gemm_dense_plan(M, N, K, epilogue)
+        plan = load().sp_gemm_dense_plan(M, N >> epilogue, K, epilogue) if dense_gemm_pays(M, N, K) and N % (epilogue + 1) == 0 else -1
+        _DENSE_PLANS[key] = plan
     return plan
 
 
-def _dense_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """a 16-bit product of rows on the GPU that sp_gemm_dense runs, and runs faster than the library; autograd, function transforms and
-    dispatch modes keep the library call they can see"""
-    if not _DENSE_ON or x.dim() != 2 or weight.dim() != 2 or not x.is_cuda or x.shape[1] != weight.shape[1]:
-        return False
-    dtype = x.dtype
-    if (dtype is not torch.bfloat16 and dtype is not torch.float16) or weight.dtype is not dtype or weight.device != x.device \
-            or not dense_gemm_pays(x.shape[0], weight.shape[0], weight.shape[1]):
-        return False
-    sx, sw = x.stride(), weight.stride()
-    if sx[1] != 1 or sw[1] != 1 or sx[0] % 8 or sw[0] % 8 or sx[0] < x.shape[1] or sw[0] < x.shape[1] \
-            or x.shape[0] * sx[0] >= 1 << 31 or weight.shape[0] * sw[0] >= 1 << 31:
-        return False
-    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
-        return False
-    if torch._C._len_torch_dispatch_stack() or torch._C._functorch.peek_interpreter_stack() is not None \
-            or torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing() \
-            or type(x) not in _PLAIN or type(weight) not in _PLAIN:
-        return False
-    # a table that was calibrated on this box says how the library runs these projections
-    if (weight.shape[0], weight.shape[1]) in getattr(_LIBRARY_ROWS, "calibrated", ()):
-        return False
-    return x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
-
-
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+_forward_ad = torch.autograd.forward_ad
+_transforms = torch._C._functorch.peek_interpreter_stack
+_dispatch_modes = torch._C._len_torch_dispatch_stack
 
 
-def _dense(x: torch.Tensor, weight: torch.Tensor, cols: int, epilogue: int, plan: int) -> torch.Tensor:
-    M, K = x.shape
-    out = empty_rows(M, cols, x.dtype, x.device)
-    splits = plan >> 8
-    sums = torch.empty(splits * M * cols, dtype=torch.float32, device=x.device) if splits > 1 else None
-    _check(load().sp_gemm_dense(out.data_ptr(), x.data_ptr(), weight.data_ptr(), _ptr(sums), 0 if sums is None else sums.numel(), M, cols, K,
-                                x.stride(0), weight.stride(0), out.stride(0), epilogue, plan, _dt(x), _stream()), "sp_gemm_dense")
+def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Optional[torch.Tensor]:
+    """x @ weight.T (epilogue 1: silu of its first half of columns times its second) by sp_gemm_dense, or None: a product it does not run,
+    or not faster than what else would.  Autograd, function transforms, tracing and dispatch modes keep the library call they can see."""
+    shape, wshape = x.shape, weight.shape
+    if not _DENSE_ON or len(shape) != 2 or len(wshape) != 2:
+        return None
+    M, K = shape
+    N = wshape[0]
+    plan = _dense_plan(M, N, K, epilogue)
+    dtype = x.dtype
+    if plan < 0 or wshape[1] != K or (dtype is not torch.bfloat16 and dtype is not torch.float16) or weight.dtype is not dtype \
+            or not x.is_cuda or x.get_device() != weight.get_device() or type(x) not in _PLAIN or type(weight) not in _PLAIN:
+        return None
+    (xs, x1), (ws, w1) = x.stride(), weight.stride()
+    if x1 != 1 or w1 != 1 or xs % 8 or ws % 8 or xs < K or ws < K or M * xs >= 1 << 31 or N * ws >= 1 << 31:
+        return None
+    if (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)) or _dispatch_modes() or _transforms() is not None \
+            or _forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None:
+        return None
+    # a table that was calibrated on this box says how the library runs these projections
+    if (N, K) in getattr(_LIBRARY_ROWS, "calibrated", ()):
+        return None
+    xp, wp = x.data_ptr(), weight.data_ptr()
+    if xp % 16 or wp % 16:
+        return None
+    cols, splits = N >> epilogue, plan >> 8
+    out = _rows_like(x, M, cols)
+    floats = splits * M * cols if splits > 1 else 0
+    sums = torch.empty(floats, dtype=torch.float32, device=x.device) if floats else None
+    _check(load().sp_gemm_dense(out.data_ptr(), xp, wp, _ptr(sums), floats, M, cols, K, xs, ws, cols, epilogue, plan, _dt(x), _stream()),
+           "sp_gemm_dense")
     return out
 
 
@@ -1019,6 +1031,11 @@ def empty_rows(rows: int, cols: int, dtype, device, zero: bool = False) -> torch
     return full[:rows]
 
 
+def _rows_like(x: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
+    """empty_rows of x's type on x's device (3 instead of 4.6 us of the host)"""
+    return x.new_empty((rows + ROW_SLACK, cols)).as_strided((rows, cols), (cols, 1))
+
+
 def extend_rows(x: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
     """x re-viewed over `rows` >= x.shape[0] rows of its own storage, or None if the storage ends before"""
     if rows <= x.shape[0]:
@@ -1041,19 +1058,19 @@ SILU_FUSED_MAX_ROWS = 8
 def linear_silu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor, any_rows: bool = False) -> Optional[torch.Tensor]:
     """SiluAndMul(x @ gate_up_weight.T) as ONE launch (sp_gemm_skinny, epilogue 1) for a step of at most
     SILU_FUSED_MAX_ROWS tokens (any_rows: up to the kernel's 16): x [M, K], gate_up_weight [2 I, K] (gate rows first),
-    result [M, I].  Bit for bit the skinny projection followed by silu_and_mul.  None when the shape is not taken (the
-    caller runs the two steps)."""
+    result [M, I].  Bit for bit ``linear`` followed by silu_and_mul; with any_rows the skinny projection whatever its size, else
+    sp_gemm_dense where linear would take it.  None when the shape is not taken (the caller runs the two steps)."""
+    if not any_rows and x.dim() == 2 and 4 < x.shape[0] <= SILU_FUSED_MAX_ROWS and gate_up_weight.numel() > 1 << 23:
+        out = dense_silu_mul(x, gate_up_weight)
+        if out is not None:
+            return out
     return _skinny_glu(x, gate_up_weight, any_rows, 1, "sp_gemm_skinny(silu)")
 
 
 def dense_silu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> Optional[torch.Tensor]:
     """the same for the rows that sp_gemm_dense takes: bit for bit ``linear`` followed by silu_and_mul.  None when the projection is not one
     of its own, or is one whose K is shared out."""
-    if not _SILU_LINEAR_ON or gate_up_weight.shape[0] % 2 or not _dense_takes(x, gate_up_weight):
-        return None
-    inter = gate_up_weight.shape[0] // 2
-    plan = _dense_plan(x.shape[0], inter, x.shape[1], 1)
-    return None if plan < 0 else _dense(x, gate_up_weight, inter, 1, plan)
+    return _dense_product(x, gate_up_weight, 1) if _SILU_LINEAR_ON else None
 
 
 def linear_gelu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.Tensor:
@@ -1097,21 +1114,21 @@ def _skinny_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x @ weight.T.  Small-batch 16-bit products go to the weight-streaming kernel
-    (sp_gemm_skinny) where it pays, those of 17 rows and more to sp_gemm_dense where that does; everything else is the library GEMM - exactly F.linear, except
+    (sp_gemm_skinny) where it pays, those of more rows to sp_gemm_dense where that does; everything else is the library GEMM - exactly F.linear, except
     that a product of at most SLACK_MAX_ROWS rows whose (shape, rows) is in the active library_rows
     table is computed over more rows than asked for (first M rows returned; rows are independent)."""
-    if _skinny_takes(x, weight):
-        M, K = x.shape
+    shape = x.shape
+    rows = shape[0] if len(shape) == 2 else 0
+    if rows > SKINNY_MAX_ROWS or (rows > 4 and weight.numel() > 1 << 23):
+        out = _dense_product(x, weight, 0)
+        if out is not None:
+            return out
+    if 0 < rows <= SKINNY_MAX_ROWS and _skinny_takes(x, weight):
         N = weight.shape[0]
-        out = empty_rows(M, N, x.dtype, x.device)
-        _check(load().sp_gemm_skinny(out.data_ptr(), x.data_ptr(), weight.data_ptr(), M, N, K, x.stride(0),
-                                     weight.stride(0), out.stride(0), 0, _dt(x), _stream()), "sp_gemm_skinny")
+        out = _rows_like(x, rows, N)
+        _check(load().sp_gemm_skinny(out.data_ptr(), x.data_ptr(), weight.data_ptr(), rows, N, shape[1], x.stride(0),
+                                     weight.stride(0), N, 0, _dt(x), _stream()), "sp_gemm_skinny")
         return out
-    if _dense_takes(x, weight):
-        M, K = x.shape
-        plan = _dense_plan(M, weight.shape[0], K, 0)
-        if plan >= 0:
-            return _dense(x, weight, weight.shape[0], 0, plan)
     if (_LIBRARY_ROWS and x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= SLACK_MAX_ROWS and weight.dim() == 2
             and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and x.stride(1) == 1):
         M, K = x.shape

@@ -1,5 +1,5 @@
-// out[M, N] = x[M, K] . w[N, K]^T for steps of 17 - 256 rows (a server's decode batch, a short prompt; to 640 rows where K is three times N),
-// 16-bit types.
+// out[M, N] = x[M, K] . w[N, K]^T for steps of 17 - 256 rows (a server's decode batch, a short prompt; to 640 rows where K is three times N)
+// and of 5 - 16 rows over large weights, 16-bit types.
 //
 // Call sites: the projections of every layer and the LM head (QKVParallelLinear / RowParallelLinear / MergedColumnParallelLinear.forward,
 // nn/layers/linear.py:696-760, 423-470, 1033-1155 -> F.linear; LogitsProcessor._get_logits, nn/layers/logits_processor.py:340-376).
@@ -7,7 +7,7 @@
 // What bounds it: at 64 rows a product is still a stream of its weights, at 256 rows the matrix cores need half the stream's time.
 // The library's kernels for these sizes are tiles of 128 - 256 rows without a split of K: too few workgroups to pull the weights
 // in (4096 x 14336 at 128 rows: 32 tiles), or rows computed for nothing.  Here
-//   * the tile follows the rows (32 - 256) and is narrow (16 - 128 weight rows), so that about one workgroup per compute unit streams;
+//   * the tile follows the rows (16 - 256) and is narrow (16 - 128 weight rows), so that about one workgroup per compute unit streams;
 //     where K is long, its shares go to workgroups of their own and a second launch adds them (2 us + the sums' traffic);
 //   * both operands go to LDS by direct loads, into rings of steps: the first waves load x, the others w, each with its own count of
 //     steps in flight (loads retire in order: in one wave, x out of the L2 would wait behind weights out of HBM);
@@ -23,7 +23,8 @@
 //   4096 x 4096                                            14.2 -> 11.9  15.3 -> 12.6   24.6 -> 15.7   22.7 -> 21.4
 //   28672 x 4096                                           55.4 -> 48.5  54.7 -> 48.6   58.7 -> 55.6   71.9 -> 68.7
 //   4096 x 14336                                           30.0 -> 23.8  38.9 -> 28.6   75.9 -> 34.0   62.1 -> 48.2
-// At 256 rows x 28672 the x tile takes two thirds of what a unit can have in flight (160 KB of LDS); from 512 rows on the library's
+// 5 / 8 / 16 rows (the library or sp_gemm_skinny, whichever was faster): 28672 x 4096 49 -> 42, 54 -> 43, 61 -> 44; 128256 x 4096 190 -> 161,
+// 193 -> 162, 193 -> 164.  At 256 rows x 28672 the x tile takes two thirds of what a unit can have in flight (160 KB of LDS); from 512 rows on the library's
 // 256 x 256 tiles are up to 30 % faster where N is large.
 #include "sp_common.h"
 
@@ -89,7 +90,6 @@ struct Tile {
   static constexpr int kWaves = WK * WM * WN, kX = BM * BK * 2, kW = BN * BK * 2;
   static constexpr int kRing = SX * kX + SW * kW, kSums = WK > 1 ? BM * BN * 4 : 0;
   static constexpr int kLds = kRing > kSums ? kRing : kSums;
-  static constexpr int kGlu = BN / WN % 32 == 0;                              // a wave holds gate columns and their up columns
   static constexpr int kOcc = kLds <= 80 * 1024 && kWaves <= 4 ? 2 : kWaves / 4;      // waves per SIMD
 };
 
@@ -103,7 +103,6 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
   constexpr int LX = (GX + T::WX - 1) / T::WX, LW = (GW + WW - 1) / WW, LM = LX > LW ? LX : LW;
   static_assert(T::BM % RPL == 0 && T::BN % RPL == 0 && TM % 16 == 0 && TN % 16 == 0 && T::BK % (32 * T::WK) == 0 && T::WK <= 2, "tile");
   static_assert(LX * (T::SX - 1) <= 63 && LW * (T::SW - 1) <= 63 && T::SX >= 2 && T::SW >= 2 && T::kLds <= 160 * 1024, "ring");
-  static_assert(!EPI || FN % 2 == 0, "gate and up columns of one wave");
   extern __shared__ __attribute__((aligned(1024))) char dense_lds[];
   char* const lds = dense_lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
@@ -125,8 +124,8 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
     if (loads_x) {
       row = min(m0 + r, p.M - 1);
     } else if constexpr (EPI) {
-      const int in = r % TN;
-      row = min(n0 + r / TN * (TN / 2) + in % (TN / 2), p.N - 1) + (in >= TN / 2 ? p.N : 0);
+      const int in = r % 16;                             // 8 gate rows, then the up rows of the same 8 columns
+      row = min(n0 + r / 16 * 8 + in % 8, p.N - 1) + (in >= 8 ? p.N : 0);
     } else {
       row = min(n0 + r, p.N - 1);
     }
@@ -222,19 +221,19 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
 #pragma unroll
       for (int n = 0; n < FN; ++n) acc[f][n] += sums[(f * FN + n) * 64];
   }
-  // acc[f][j][r] = out[row 16 f + r16][column 16 j + 4 q + r] of the wave's tile
-  constexpr int FO = EPI ? FN / 2 : FN;
+  // acc[f][j][r] = out[row 16 f + r16][column 16 j + 4 q + r] of the wave's tile (EPI: the lanes below 32 the gate sums of column
+  // 8 j + 4 q + r, the lanes 32 above them its up sums)
 #pragma unroll
   for (int f = 0; f < FM; ++f) {
     const int m = m0 + wm * TM + 16 * f + r16;
-    if (m >= p.M) continue;
 #pragma unroll
-    for (int j = 0; j < FO; ++j) {
-      const int n = n0 + wn * (EPI ? TN / 2 : TN) + 16 * j + 4 * q;
+    for (int j = 0; j < FN; ++j) {
+      const int n = EPI ? n0 + wn * (TN / 2) + 8 * j + 4 * q : n0 + wn * TN + 16 * j + 4 * q;
+      const bool mine = m < p.M && n < p.N && !(EPI && q >= 2);
       if constexpr (SPLIT) {
         float* const to = p.part + ((int64_t)split * p.M + m) * p.N + n;
-        if (p.vec && n < p.N) *(f32x4_d*)to = acc[f][j];
-        else
+        if (mine && p.vec) *(f32x4_d*)to = acc[f][j];
+        else if (mine)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             if (n + r < p.N) to[r] = acc[f][j][r];
@@ -243,13 +242,16 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float v = acc[f][j][r];
-          if constexpr (EPI) v = mul_round<Tag>(E::round(silu_ref(E::round(v))), E::round(acc[f][j + FN - FO][r]));
+          if constexpr (EPI) {
+            const auto both = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);      // lanes 0-31 twice, 32-63 twice
+            v = mul_round<Tag>(E::round(silu_ref(E::round(v))), E::round(as_f32(both[1])));
+          }
           if constexpr (std::is_same<Tag, bf16_tag>::value) h[r] = f32_to_bf16_bits(v);
           else h[r] = f32_to_f16_bits(v);
         }
         char* const to = p.out + ((int64_t)m * p.out_stride + n) * 2;
-        if (p.vec && n < p.N) *(u32x2*)to = u32x2{h[0] | h[1] << 16, h[2] | h[3] << 16};
-        else
+        if (mine && p.vec) *(u32x2*)to = u32x2{h[0] | h[1] << 16, h[2] | h[3] << 16};
+        else if (mine)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             if (n + r < p.N) ((uint16_t*)to)[r] = (uint16_t)h[r];
@@ -312,10 +314,7 @@ int launch_dense_tile(DenseArgs p, int epilogue, hipStream_t st) {
   const int per = epilogue ? T::BN / 2 : T::BN;
   p.mblocks = (p.M + T::BM - 1) / T::BM;
   p.nblocks = (p.N + per - 1) / per;
-  if (epilogue) {
-    if constexpr (T::kGlu) return p.splits == 1 ? launch_dense_kernel<Tag, T, 1, false>(p, st) : SP_ERR_UNSUPPORTED;
-    return SP_ERR_UNSUPPORTED;
-  }
+  if (epilogue) return p.splits == 1 ? launch_dense_kernel<Tag, T, 1, false>(p, st) : SP_ERR_UNSUPPORTED;
   if (p.splits == 1) return launch_dense_kernel<Tag, T, 0, false>(p, st);
   const int rc = launch_dense_kernel<Tag, T, 0, true>(p, st);
   if (rc != SP_OK) return rc;
@@ -329,35 +328,38 @@ int launch_dense_tile(DenseArgs p, int epilogue, hipStream_t st) {
 
 // ---- which tile, how many shares of K
 // Every tile's cost: us of one step of one workgroup and of a workgroup's beginning and end, both fitted (with the constants below) to
-// 7600 timings over 23 shapes of 1 - 1050 MB at 17 - 640 rows.  A product takes the chain of its busiest unit, the traffic into
-// that unit's LDS or the weights' stream, whichever is longest; the choice is within 1.1 % of the fastest tile and split on average.
-#define SP_DENSE_TILES(F)                                   \
-  F(0, 0.417f, 1.98f, 32, 32, 256, 2, 2, 2, 4, 3, 6)        \
-  F(1, 0.307f, 2.25f, 32, 16, 256, 2, 2, 1, 2, 4, 8)        \
-  F(2, 0.950f, 1.58f, 32, 64, 256, 2, 1, 4, 2, 2, 4)        \
-  F(3, 0.634f, 2.51f, 32, 128, 128, 1, 1, 8, 2, 3, 4)       \
-  F(4, 0.465f, 2.84f, 48, 32, 256, 2, 1, 2, 2, 3, 5)        \
-  F(5, 0.239f, 3.08f, 64, 16, 256, 2, 4, 1, 4, 3, 7)        \
-  F(6, 0.252f, 2.61f, 64, 32, 128, 2, 2, 2, 4, 4, 6)        \
-  F(7, 0.224f, 2.51f, 64, 64, 64, 1, 2, 2, 2, 4, 6)         \
-  F(8, 0.552f, 3.55f, 64, 64, 256, 2, 2, 2, 4, 2, 3)        \
-  F(9, 0.636f, 3.53f, 64, 128, 128, 1, 2, 4, 4, 2, 4)       \
-  F(10, 0.556f, 2.63f, 96, 64, 128, 1, 2, 4, 4, 3, 4)       \
-  F(11, 0.389f, 3.14f, 96, 128, 64, 1, 2, 4, 4, 4, 6)       \
-  F(12, 0.392f, 3.01f, 128, 96, 64, 1, 4, 2, 4, 4, 6)       \
-  F(13, 0.468f, 3.41f, 128, 128, 64, 1, 2, 4, 4, 4, 6)      \
-  F(14, 0.529f, 5.47f, 192, 128, 64, 2, 2, 2, 4, 3, 5)      \
-  F(15, 0.654f, 6.56f, 256, 128, 64, 2, 2, 2, 4, 2, 6)
-constexpr int kDenseTiles = 16;
-constexpr float kLaunch = 1.78f, kStream = 5.05e6f, kFill = 67.45e3f, kSumLaunch = 2.03f, kSumRate = 3.88e6f;     // us, bytes per us
+// 7600 timings over 23 shapes of 1 - 1050 MB at 5 - 640 rows.  A product takes the chain of its busiest unit, the traffic into
+// that unit's LDS or the weights' stream, whichever is longest; the choice is within 1.2 % of the fastest tile and split on average.
+#define SP_DENSE_TILES(F)                              \
+  F(0, 0.655f, 2.26f, 16, 64, 256, 2, 1, 4, 2, 3, 4)   \
+  F(1, 0.588f, 2.04f, 16, 128, 128, 1, 1, 8, 1, 4, 4)  \
+  F(2, 0.293f, 2.39f, 32, 16, 256, 2, 2, 1, 2, 4, 8)   \
+  F(3, 0.418f, 2.60f, 32, 32, 256, 1, 2, 2, 2, 4, 5)   \
+  F(4, 0.404f, 2.17f, 32, 32, 256, 2, 2, 2, 4, 3, 6)   \
+  F(5, 0.933f, 1.78f, 32, 64, 256, 2, 1, 4, 2, 2, 4)   \
+  F(6, 0.627f, 2.62f, 32, 128, 128, 1, 1, 8, 2, 3, 4)  \
+  F(7, 0.474f, 2.86f, 48, 32, 256, 2, 1, 2, 2, 3, 5)   \
+  F(8, 0.248f, 3.08f, 64, 16, 256, 2, 4, 1, 4, 3, 7)   \
+  F(9, 0.258f, 2.62f, 64, 32, 128, 2, 2, 2, 4, 4, 6)   \
+  F(10, 0.228f, 2.55f, 64, 64, 64, 1, 2, 2, 2, 4, 6)   \
+  F(11, 0.578f, 3.53f, 64, 64, 256, 2, 2, 2, 4, 2, 3)  \
+  F(12, 0.648f, 3.52f, 64, 128, 128, 1, 2, 4, 4, 2, 4) \
+  F(13, 0.565f, 2.63f, 96, 64, 128, 1, 2, 4, 4, 3, 4)  \
+  F(14, 0.395f, 3.12f, 96, 128, 64, 1, 2, 4, 4, 4, 6)  \
+  F(15, 0.398f, 2.98f, 128, 96, 64, 1, 4, 2, 4, 4, 6)  \
+  F(16, 0.474f, 3.37f, 128, 128, 64, 1, 2, 4, 4, 4, 6) \
+  F(17, 0.536f, 5.39f, 192, 128, 64, 2, 2, 2, 4, 3, 5) \
+  F(18, 0.661f, 6.46f, 256, 128, 64, 2, 2, 2, 4, 2, 6)
+constexpr int kDenseTiles = 19;
+constexpr float kLaunch = 1.72f, kStream = 5.43e6f, kFill = 67.72e3f, kSumLaunch = 2.f, kSumRate = 3.76e6f;     // us, bytes per us
 constexpr int kUnits = 256;
 
 struct TileCost {
-  int bm, bn, bk, wk, lds, glu;
+  int bm, bn, bk, wk, lds;
   float step, fixed;
 };
 #define SP_DENSE_COST(I, STEP, FIXED, ...) \
-  {Tile<__VA_ARGS__>::BM, Tile<__VA_ARGS__>::BN, Tile<__VA_ARGS__>::BK, Tile<__VA_ARGS__>::WK, Tile<__VA_ARGS__>::kLds, Tile<__VA_ARGS__>::kGlu, STEP, FIXED},
+  {Tile<__VA_ARGS__>::BM, Tile<__VA_ARGS__>::BN, Tile<__VA_ARGS__>::BK, Tile<__VA_ARGS__>::WK, Tile<__VA_ARGS__>::kLds, STEP, FIXED},
 constexpr TileCost kCosts[kDenseTiles] = {SP_DENSE_TILES(SP_DENSE_COST)};
 
 float dense_us(const TileCost& c, int M, int64_t rows, int K, int splits) {
@@ -395,7 +397,7 @@ extern "C" int sp_gemm_dense_plan(int M, int N, int K, int epilogue) {
   float least = 0.f;
   for (int i = 0; i < sp::kDenseTiles; ++i) {
     const sp::TileCost& c = sp::kCosts[i];
-    if (K % c.bk || (epilogue && (!c.glu || c.wk != sp::kCosts[plain & 255].wk))) continue;
+    if (K % c.bk || (epilogue && c.wk != sp::kCosts[plain & 255].wk)) continue;
     for (int splits = 1; splits <= (epilogue ? 1 : 8); splits *= 2) {
       // shares of at least three steps, for launches that would leave units idle, with sums that stay in the caches
       if (splits > 1 && (K / c.bk / splits < 3 || (M + c.bm - 1) / c.bm * (int64_t)((rows + c.bn - 1) / c.bn) * splits > 600 ||
