@@ -17,7 +17,7 @@
 // Each form sums the partial results of its lanes and waves in a fixed order that M, K and the
 // number of weight rows alone decide.
 // us, cold weights under graph replay, N x K: 1 row / 4 rows / 8 rows; before (the third form for every M, the waves' k-steps
-// interleaved) -> now.  The second form ends at the 4 rows that its instruction holds: a second group of x rows for 5 to 8 was
+// interleaved) -> now (1 row of large weights: kRowOnce has the later figures; 5 - 16 rows of them go to sp_gemm_dense).  The second form ends at the 4 rows that its instruction holds: a second group of x rows for 5 to 8 was
 // slower where there are many weight rows (8 rows: 20.1 against the third form's 17.3 at 16384 x 2048) and faster with few long ones (12.8
 // against 14.6 at 2048 x 8192), which is left on the table.  Below 5 rows few_take_tiles has the line to the third form.
 //   3072 x 2048     5.3 -> 4.6      5.9 -> 5.8      6.3 -> 6.1
@@ -91,7 +91,8 @@ __device__ __forceinline__ float glu_value(float gate, float up) {
 // ---- 1 row
 constexpr int kRowWaves = 2, kRowLoads = 4;
 
-template <typename Tag, int EPI>
+// ONCE: weights past the L2 (launch_skinny_as has the line)
+template <typename Tag, int EPI, bool ONCE>
 __global__ __launch_bounds__(kRowWaves * 64) void gemm_row_kernel(SkinnyArgs a) {
   typedef Elem<Tag> E;
   constexpr bool GLU = EPI == 1 || EPI == 3;
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(kRowWaves * 64) void gemm_row_kernel(SkinnyArgs a) 
       const int k = k0 + u * 512 + lane * 8;           // K is a multiple of 8: a lane's 16 bytes are in the row or past it
       const bool in = k < a.K;
 #pragma unroll
-      for (int r = 0; r < R; ++r) wf[u][r] = in ? ld16(wp[r] + (int64_t)k * 2) : zero;
+      for (int r = 0; r < R; ++r) wf[u][r] = !in ? zero : ONCE ? ld16_once(wp[r] + (int64_t)k * 2) : ld16(wp[r] + (int64_t)k * 2);
       xf[u] = in ? ld16(a.x + (int64_t)k * 2) : zero;
     }
     __builtin_amdgcn_sched_barrier(0);                 // all of them on their way before the first is waited for
@@ -157,7 +158,7 @@ constexpr int kQuadWaves = 4, kQuadLoads = 4, kQuadRows = 4;
 
 // G groups of 4 weight rows: two where there are enough of them to fill the card (x is read half as often) and for gate and up,
 // else one and twice the length of K in flight.  The order of the sums is the same.
-template <typename Tag, int G, int EPI>
+template <typename Tag, int G, int EPI, bool ONCE>
 __global__ __launch_bounds__(kQuadWaves * 64) void gemm_quad_kernel(SkinnyArgs a) {
   typedef Elem<Tag> E;
   constexpr bool GLU = EPI == 1 || EPI == 3;
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(kQuadWaves * 64) void gemm_quad_kernel(SkinnyArgs a
       const int k = k0 + (u / kQuadLoads) * kQuadWaves * kSpan + (u % kQuadLoads) * 128;
       const bool in = k + 8 * b < a.K;
 #pragma unroll
-      for (int g = 0; g < G; ++g) wf[u][g] = in ? ld16(wp[g] + (int64_t)k * 2) : zero;
+      for (int g = 0; g < G; ++g) wf[u][g] = !in ? zero : ONCE ? ld16_once(wp[g] + (int64_t)k * 2) : ld16(wp[g] + (int64_t)k * 2);
       xf[u] = in && mrow ? ld16(xp + (int64_t)k * 2) : zero;
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -300,17 +301,30 @@ static bool few_take_tiles(int M, int64_t rows, int K) {
   return rows > kQuadOneGroup && (K <= 1536 || (rows <= 4096 && (M > 2 || K <= 4096)));
 }
 
+// Weights past the L2, in elements: at 1 row from what the eight L2s hold together on (32 MB), at 2 - 4 rows, which read less of a row at
+// a time, from half the last-level cache on.  us, kept / past it, 1 row, of weights out of HBM: 4096 x 4096 8.2 / 7.6, 2048 x 8192
+// 8.3 / 7.7, 16384 x 2048 with the activation 13.6 / 12.3, 28672 x 4096 38.7 / 35.9, 128256 x 2048 86 / 78; out of the last-level cache (2
+// weights in turn) 4096 x 4096 7.1 / 7.0, 16384 x 2048 11.2 / 11.1; below the line 3072 x 2048 4.2 / 4.2 and, out of the L2, 2.9 / 3.5.  2 rows:
+// 28672 x 4096 41.1 / 38.6, 128256 x 2048 88 / 80; 16384 x 2048 14.3 / 14.0, but 12.5 / 13.6 out of the last-level cache.  (The tiles of 5 -
+// 16 rows read half a line at a time: 28672 x 4096 47 / 54.)
+constexpr int64_t kRowOnce = 1 << 24, kQuadOnce = 1 << 26;
+
 template <typename Tag, int EPI>
 static void launch_skinny_as(const SkinnyArgs& a, hipStream_t st) {
   constexpr bool GLU = EPI == 1 || EPI == 3;
+  const int64_t elements = (GLU ? 2 : 1) * (int64_t)a.N * a.K;
   if (a.M == 1) {
-    gemm_row_kernel<Tag, EPI><<<dim3((a.N + kRowWaves - 1) / kRowWaves), dim3(kRowWaves * 64), 0, st>>>(a);
+    const dim3 grid((a.N + kRowWaves - 1) / kRowWaves), block(kRowWaves * 64);
+    if (elements >= kRowOnce) gemm_row_kernel<Tag, EPI, true><<<grid, block, 0, st>>>(a);
+    else gemm_row_kernel<Tag, EPI, false><<<grid, block, 0, st>>>(a);
   } else if (a.M <= kQuadRows && !few_take_tiles(a.M, GLU ? 2 * (int64_t)a.N : a.N, a.K)) {
     if (!GLU && a.N <= kQuadOneGroup) {
-      if constexpr (!GLU) gemm_quad_kernel<Tag, 1, EPI><<<dim3((a.N + 3) / 4), dim3(kQuadWaves * 64), 0, st>>>(a);
+      if constexpr (!GLU) gemm_quad_kernel<Tag, 1, EPI, false><<<dim3((a.N + 3) / 4), dim3(kQuadWaves * 64), 0, st>>>(a);
     } else {
       constexpr int cols = GLU ? 4 : 8;
-      gemm_quad_kernel<Tag, 2, EPI><<<dim3((a.N + cols - 1) / cols), dim3(kQuadWaves * 64), 0, st>>>(a);
+      const dim3 grid((a.N + cols - 1) / cols), block(kQuadWaves * 64);
+      if (elements >= kQuadOnce) gemm_quad_kernel<Tag, 2, EPI, true><<<grid, block, 0, st>>>(a);
+      else gemm_quad_kernel<Tag, 2, EPI, false><<<grid, block, 0, st>>>(a);
     }
   } else {
     constexpr int cols = GLU ? 8 : 16;

@@ -179,6 +179,9 @@ __device__ __forceinline__ float fma_round<f16_tag>(float a, float b, float c) {
 }
 
 __device__ __forceinline__ u32x4 ld16(const void* p) { return *(const u32x4*)p; }
+// the same for data that is read once: past the L2's other lines (both halves of a 128-byte line have to be in one wave's load - the line
+// does not wait there for the next one)
+__device__ __forceinline__ u32x4 ld16_once(const void* p) { return __builtin_nontemporal_load((const u32x4*)p); }
 __device__ __forceinline__ void st16(void* p, const u32x4& v) { *(u32x4*)p = v; }
 
 // ---- fp8 e5m2 (1-5-2 = the top byte of an IEEE half) ---------------------------------------------
