@@ -874,9 +874,10 @@ def dense_gemm_pays(M: int, N: int, K: int) -> bool:
     5 - 16 rows: matrices of more than 2^23 elements, where 16 rows of x beside every 16 weight rows are what sp_gemm_skinny waits for (that or
     the library, whichever is faster / own, at 5 / 8 / 16 rows: 28672 x 4096 49 / 42, 54 / 43, 61 / 44; 2048 x 8192 13.1 / 11.6, 12.8 / 11.7, 13.3 / 11.9;
     128256 x 4096 190 / 161, 193 / 162, 193 / 164; 4096 x 4096 10.2 / 9.9, 10.2 / 9.9, 11.5 / 10.1; 6144 x 2048 9.1 / 8.5, 9.4 / 8.5, 10.9 / 8.6); below that a
-    launch of small workgroups is over sooner (2048 x 4096 7.9 / 8.4, 3072 x 2048 5.7 / 6.8, 2048 x 2048 5.6 / 6.3)."""
+    launch of small workgroups is over sooner (2048 x 4096 7.9 / 8.4, 3072 x 2048 5.7 / 6.8, 2048 x 2048 5.6 / 6.3).  Up to 4096 x 4096
+    both are even up to 8 rows (sp_gemm_skinny)."""
     if M <= SKINNY_MAX_ROWS:
-        return M > 4 and K % 64 == 0 and N * K > 1 << 23
+        return M > 4 and K % 64 == 0 and N * K > 1 << 23 and (M > 8 or N > 4096 or K > 4096)
     if K % 64 or N <= 512 or M > (640 if K >= 3 * N and N >= 2048 else DENSE_MAX_ROWS):
         return False
     if N <= 2048 and 2048 < K <= 4096:

@@ -26,7 +26,7 @@
 // 5 / 8 / 16 rows (the library or sp_gemm_skinny, whichever was faster): 28672 x 4096 49 -> 42, 54 -> 43, 61 -> 44; 128256 x 4096 190 -> 161,
 // 193 -> 162, 193 -> 164.  At 256 rows x 28672 the x tile takes two thirds of what a unit can have in flight (160 KB of LDS); from 512 rows on the library's
 // 256 x 256 tiles are up to 30 % faster where N is large.
-#include "sp_common.h"
+#include "lds_ring.h"
 
 #include <type_traits>
 
@@ -54,33 +54,6 @@ struct DenseArgs {
   int64_t x_stride, w_stride, out_stride;  // elements
   int vec;                            // 4 neighbouring output columns are one aligned store
 };
-
-// 16 bytes per lane from base + off to lds + 16 lane, without a register on the way.  (m0 is named, so that no value another
-// instruction needs in it is carried past; the compiler calls that reserved.)
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void load_to_lds(uint32_t off, const char* base, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void stream_to_lds(uint32_t off, const char* base, uint32_t lds) {      // read once: not kept in the L2
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-// Waits until at most min(later, MOST) steps of L loads each are on their way (and for this wave's reads of LDS)
-template <int L, int MOST>
-__device__ __forceinline__ void wait_steps(int later) {
-  if constexpr (MOST == 0) {
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-  } else {
-    if (later >= MOST) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(L* MOST) : "memory");
-    else wait_steps<L, MOST - 1>(later);
-  }
-}
-__device__ __forceinline__ void barrier() {
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // BM x BN outputs per workgroup, BK of k a step, WK x WM x WN waves, the first WX of which load x and the others w; SX and SW steps of
 // x and w in LDS
@@ -132,15 +105,15 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
     off[i] = (uint32_t)row * (uint32_t)((loads_x ? p.x_stride : p.w_stride) * 2) + chunk * 16;
   }
   const char* const src = (loads_x ? p.x : p.w) + (int64_t)first * RB;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const uint32_t lds0 = lds_address(lds);
   const auto stage_x = [&](int s, int buf) {
 #pragma unroll
-    for (int i = 0; i < LX; ++i) load_to_lds(off[i], src + (int64_t)s * RB, lds0 + buf + min(wave * LX + i, GX - 1) * 1024);
+    for (int i = 0; i < LX; ++i) ring_load<false>(off[i], src + (int64_t)s * RB, lds0 + buf + min(wave * LX + i, GX - 1) * 1024);
   };
   const auto stage_w = [&](int s, int buf) {
 #pragma unroll
     for (int i = 0; i < LW; ++i)
-      stream_to_lds(off[i], src + (int64_t)s * RB, lds0 + T::SX * T::kX + buf + min((wave - T::WX) * LW + i, GW - 1) * 1024);
+      ring_load<true>(off[i], src + (int64_t)s * RB, lds0 + T::SX * T::kX + buf + min((wave - T::WX) * LW + i, GW - 1) * 1024);
   };
   f32x4_d acc[FM][FN];
 #pragma unroll
@@ -158,12 +131,12 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
   };
   if (loads_x) {
     for (int s = 0; s < T::SX && s < steps; ++s) stage_x(s, s * T::kX);
-    wait_steps<LX, T::SX - 1>(steps - 1);
+    ring_wait<LX, T::SX - 1>(steps - 1);
   } else {
     for (int s = 0; s < T::SW && s < steps; ++s) stage_w(s, s * T::kW);
-    wait_steps<LW, T::SW - 1>(steps - 1);
+    ring_wait<LW, T::SW - 1>(steps - 1);
   }
-  barrier();
+  ring_barrier();
   read(0, 0, wk, 0);
   int cx = 0, cw = 0;
   // One step: its products, behind the reads of the next one's first operands.  PAR: which of the two operand sets is the step's first
@@ -177,9 +150,9 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
         read(cx, cw, (j + 1) * T::WK + wk, at ^ 1);
       } else if (s + 1 < steps) {
         // the step's last operands are in registers: when every wave is here its buffers are free, and the next step's are full
-        if (loads_x) wait_steps<LX, T::SX - 2>(steps - 2 - s);
-        else wait_steps<LW, T::SW - 2>(steps - 2 - s);
-        barrier();
+        if (loads_x) ring_wait<LX, T::SX - 2>(steps - 2 - s);
+        else ring_wait<LW, T::SW - 2>(steps - 2 - s);
+        ring_barrier();
         if (loads_x) {
           if (s + T::SX < steps) stage_x(s + T::SX, cx);
         } else if (s + T::SW < steps) {
@@ -205,7 +178,7 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
   }
   if constexpr (T::WK > 1) {                              // the two halves of every 64 of k meet in LDS, the first wave's plus the second's
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    barrier();
+    ring_barrier();
     f32x4_d* const sums = (f32x4_d*)lds + wmn * FM * FN * 64 + lane;
     if (wk) {
 #pragma unroll
@@ -214,7 +187,7 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
         for (int n = 0; n < FN; ++n) sums[(f * FN + n) * 64] = acc[f][n];
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    barrier();
+    ring_barrier();
     if (wk) return;
 #pragma unroll
     for (int f = 0; f < FM; ++f)
@@ -275,7 +248,9 @@ __global__ void __launch_bounds__(256) dense_sum_kernel(DenseArgs p) {
 #pragma unroll
     for (int s = 0; s < S; ++s) v[s] = *(const f32x4_d*)(from + s * step);
 #pragma unroll
-    for (int s = 1; s < S; ++s) v[0] += v[s];
+    for (int by = 1; by < S; by *= 2)                          // in pairs: each share is rounded log2 S times
+#pragma unroll
+      for (int s = 0; s < S; s += 2 * by) v[s] += v[s + by];
     u32x2 o;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -286,9 +261,14 @@ __global__ void __launch_bounds__(256) dense_sum_kernel(DenseArgs p) {
     *(u32x2*)(p.out + ((int64_t)m * p.out_stride + n) * 2) = o;
   } else {
     for (int r = 0; r < 4 && n + r < p.N; ++r) {
-      float v = from[r];
-      for (int s = 1; s < S; ++s) v += from[s * step + r];
-      E::store(p.out, (int64_t)m * p.out_stride + n + r, v);
+      float v[S];
+#pragma unroll
+      for (int s = 0; s < S; ++s) v[s] = from[s * step + r];
+#pragma unroll
+      for (int by = 1; by < S; by *= 2)
+#pragma unroll
+        for (int s = 0; s < S; s += 2 * by) v[s] += v[s + by];
+      E::store(p.out, (int64_t)m * p.out_stride + n + r, v[0]);
     }
   }
 }
