@@ -3,8 +3,10 @@
 // pairs of a step ordered by expert on the device; a grouped matrix product over that order (every expert's weights are
 // read once per row tile, fp32 accumulation); the clamped gated activation; and the weighted sum of a token's experts in
 // a fixed order, so a token's result does not depend on which other tokens share the step.
+#include "lds_ring.h"
 #include "seq_batch.h"
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -311,7 +313,7 @@ moe_grouped_gemm_kernel(void* out, const void* a, const void* w, const int32_t* 
 // ---- the same product on the matrix cores (16-bit types, K a multiple of 32, 16-byte aligned rows) -------------------
 // v_mfma_f32_16x16x32: lane (r16 = lane & 15, q = lane >> 4) holds 8 k-values of row r16 of each operand and receives
 // D[4 q + r][r16], r < 4 - with the weights as the first operand a lane ends up with 4 neighbouring output columns of ONE
-// row.  The kernels below (tile, wide, rows, narrow rows) add the k-steps of 32 in ascending order into one accumulator, so an output
+// row.  The kernels below (tile, ring, rows, narrow rows) add the k-steps of 32 in ascending order into one accumulator, so an output
 // element has the same bits whichever of them - and whichever tile height - computes it: a token's result does not depend on the
 // step's size.
 //
@@ -417,7 +419,7 @@ __device__ __forceinline__ bool grouped_tile(const int32_t* offsets, int E, int 
 
 // The same for a launch of `cols` column tiles per row tile, an expert's row tiles next to each other: the column tile as well.
 __device__ __forceinline__ bool grouped_tile_by_column(const int32_t* offsets, int E, int bm, int cols, int at, int lane, int& e_out,
-                                                       int& row0, int& rows_end, int& col) {
+                                                       int& row0, int& rows_end, int& col, int& rows_tiles) {
   for (int e0 = 0; e0 < E; e0 += 64) {
     const int e = e0 + lane;
     const int lo = e < E ? offsets[e] : 0, hi = e < E ? offsets[e + 1] : 0;
@@ -429,6 +431,7 @@ __device__ __forceinline__ bool grouped_tile_by_column(const int32_t* offsets, i
       const int n = __builtin_amdgcn_readfirstlane(__shfl(tiles, l, 64));
       const int in = __builtin_amdgcn_readfirstlane(at - __shfl(incl - tiles * cols, l, 64));
       col = in / n;
+      rows_tiles = n;
       row0 = __builtin_amdgcn_readfirstlane(__shfl(lo, l, 64)) + (in - col * n) * bm;
       rows_end = __builtin_amdgcn_readfirstlane(__shfl(hi, l, 64));
       return true;
@@ -438,7 +441,7 @@ __device__ __forceinline__ bool grouped_tile_by_column(const int32_t* offsets, i
   return false;
 }
 
-// Steps with many rows per expert: BM rows x 128 weight rows per workgroup, k in steps of 64.  Both operands go to LDS by
+// Steps with more than a few rows per expert, any K that is a multiple of 8: BM rows x 128 weight rows per workgroup, k in steps of 64.  Both operands go to LDS by
 // direct loads (16 bytes per lane, no registers on the way), one step ahead of the MFMAs, in two buffers; a step costs one
 // barrier.  LDS rows are 128 bytes whose eight 16-byte chunks are permuted by the row's number (the SOURCE address is
 // permuted: a direct load writes lane after lane), so the 16 rows of a fragment read meet no bank twice in a phase.
@@ -563,103 +566,216 @@ __global__ void __launch_bounds__(256, 2) moe_grouped_tile_kernel(GroupedArgs p)
   }
 }
 
-// Steps with hundreds of rows per expert: 128 rows x 256 weight rows per workgroup, a wave 64 x 128 of them, k in steps of 32.
-// What the 128 x 128 tiles wait for is LDS (a wave reads 8 KB for 16 products of 16 cycles: 128 bytes per cycle for the four of
-// them, all there is) and the L2 (64 bytes per cycle and CU); here it is 96 and 48.  A step's operands are 24 KB, double-buffered,
-// so three workgroups share a CU and fill each other's waits.  The row tiles of one column tile follow each other: the weights
-// they share are in the L2 once.  LDS rows are 64 bytes; the chunk of a row is permuted by its number / 4, so that the 16 rows of a
-// fragment read lie in 64 banks.  Width 2048, 32 experts of ff 1024, up + down in us, 128 x 128 tiles -> these: 512 rows per
-// expert 336 -> 315 (three buffers and two workgroups: 323; column tiles of a row tile next to each other: 330), 256 rows
-// 215 -> 217, 96 rows 105 -> 123.  (Experts that start at k of their own, so that the XCDs ask for different pieces of their rows
-// at a time: 311, but a row's bits would then depend on its neighbours' number.)
-constexpr int kWideBM = 128, kWideBN = 256, kWideBK = 32;
-template <typename Tag, int ACT>
-__global__ void __launch_bounds__(256, 3) moe_grouped_wide_kernel(GroupedArgs p) {
+// The same for K a multiple of 64: BM rows x BN weight rows per workgroup, k in steps of BK, ST steps in a ring of LDS buffers.
+// One barrier a step, in front of its last products: behind it the next step's first operands are read, and the loads into the buffer
+// that has become free are spread between those products - in one piece they hold a wave's products up (an instruction a wave can't
+// issue stops the ones behind it): a 256 x 256 tile's loop, operands in the L2, 1245 -> 1480 TFLOP/s with the loads spread and the waves
+// in their products ahead of the others.  Two workgroups share a CU (of all tiles but the largest) and fill each other's beginnings and ends.  GLU: 8 gate rows and the up
+// rows of the same 8 columns in one operand, their sums 32 lanes apart.  ONCE: an expert with one row tile reads its weights past the L2.
+// The row tiles of one column tile follow each other: the weights they share are in the L2.
+// Width 2048, 32 experts of ff 1024, up + down in us, the kernels before (64 x 128, 128 x 128 and 128 x 256 tiles, one wave per 16 rows) -> these: mean rows
+// 3: 63 + 27 -> 55 + 24, 16: 67 + 28 -> 55 + 23, 32: 68 + 29 -> 59 + 25, 50: 69 + 30 -> 60 + 30, 88: 72 + 32 -> 74 + 32, 125: 97 + 51 -> 82 + 34, 188: 98 + 52 ->
+// 102 + 53, 250: 134 + 70 -> 111 + 58, 512: 180 + 107 -> 171 + 92; width 4096, 128 experts of 1536, 4: 560 + 270 -> 481 + 239, 256: 1344 + 735 -> 1110 + 617;
+// 16 experts of 1408, 50: 50 + 26 -> 52 + 21, 750: 172 + 107 -> 173 + 85; 8 of 1536, 40: 38 + 20 -> 31 + 12, 1024: 142 + 86 -> 131 + 58.
+// (the second launch bound: waves of a SIMD, with as many workgroups in a unit as its LDS holds, at most two)
+constexpr int ring_waves(int bm, int bn, int bk, int waves, int st) { return (st * (bm + bn) * bk * 2 <= 80 * 1024 ? 2 : 1) * waves / 4; }
+
+template <typename Tag, int BM, int BN, int BK, int WM, int WN, int ST, bool ONCE, int ACT>
+__global__ void __launch_bounds__(WM * WN * 64, ring_waves(BM, BN, BK, WM * WN, ST)) moe_grouped_ring_kernel(GroupedArgs p) {
   constexpr bool GLU = ACT >= 2;
-  constexpr int CPW = kWideBN / 2, FM = 4, FN = CPW / 16, OUT_N = GLU ? kWideBN / 2 : kWideBN;
-  constexpr int LA = kWideBM / 64, LB = kWideBN / 64;            // direct loads per wave and step
-  constexpr int kBuf = (kWideBM + kWideBN) * kWideBK * 2;
-  extern __shared__ __attribute__((aligned(16))) char wide_lds[];
+  constexpr int W = WM * WN, RB = BK * 2, RPL = 1024 / RB, CH = BK / 8;                 // a row's bytes, rows and 16-byte chunks a load
+  constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16, KK = BK / 32, OUT_N = GLU ? BN / 2 : BN;
+  constexpr int G = (BM + BN) / RPL, L = (G + W - 1) / W, kStage = (BM + BN) * RB, PER = FM * FN / L;
+  static_assert(BM % RPL == 0 && TM % 16 == 0 && TN % 16 == 0 && KK % 2 == 0 && ST * kStage <= 160 * 1024 && L * (ST - 1) <= 63, "tile");
+  extern __shared__ __attribute__((aligned(1024))) char ring_lds[];
+  char* const lds = ring_lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   const int ntiles = (p.N + OUT_N - 1) / OUT_N;
-  const int total = grouped_tiles(p.offsets, p.E, kWideBM, lane) * ntiles, share = (total + 7) / 8;
+  const int total = grouped_tiles(p.offsets, p.E, BM, lane) * ntiles, share = (total + 7) / 8;
   const int idx = (int)(blockIdx.x >> 3), at = (int)(blockIdx.x & 7) * share + idx;
   if (idx >= share || at >= total) return;
-  int e = 0, row0 = 0, rows_end = 0, col = 0;
-  if (!grouped_tile_by_column(p.offsets, p.E, kWideBM, ntiles, at, lane, e, row0, rows_end, col)) return;
+  int e = 0, row0 = 0, rows_end = 0, col = 0, row_tiles = 0;
+  if (!grouped_tile_by_column(p.offsets, p.E, BM, ntiles, at, lane, e, row0, rows_end, col, row_tiles)) return;
   e = __builtin_amdgcn_readfirstlane(e);
-  const int n0 = col * OUT_N;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int wrows = GLU ? 2 * p.N : p.N;
-  // sources of this wave's direct loads: lane -> row lane / 4 of the 16 rows of a load, chunk lane % 4 of LDS
-  const int chunk = (lane & 3) ^ (lane >> 4);
-  const char* src[LA + LB];
+  const int n0 = col * OUT_N, wrows = GLU ? 2 * p.N : p.N, steps = p.K / BK;
+  const int wm = wave / WN, wn = wave % WN;
+  // this wave's direct loads: load i is the (i W + wave)-th of the tile's rows, x's first; lane -> row lane / CH of a load, chunk lane % CH
+  uint32_t off[L];
+  const char* base[L];
+  const char* const we = p.w + (int64_t)e * wrows * p.K * 2;
 #pragma unroll
-  for (int i = 0; i < LA; ++i) {
-    const int pos = min(row0 + (wave * LA + i) * 16 + (lane >> 2), rows_end - 1);     // rows past the end: never stored
-    const int64_t arow = p.order ? p.order[pos] / p.row_div : pos;
-    src[i] = p.a + arow * p.a_stride * 2 + chunk * 16;
-  }
-  const char* wbase = p.w + (int64_t)e * wrows * p.K * 2 + chunk * 16;
-#pragma unroll
-  for (int i = 0; i < LB; ++i) {
-    const int br = (wave * LB + i) * 16 + (lane >> 2);
-    int row;
-    if constexpr (GLU) {
-      const int in = br % CPW, n = n0 + (br / CPW) * (CPW / 2) + in % (CPW / 2);
-      row = min(n, p.N - 1) + (in >= CPW / 2 ? p.N : 0);
+  for (int i = 0; i < L; ++i) {
+    const int g = min(i * W + wave, G - 1), r = g * RPL + lane / CH, chunk = (lane % CH) ^ (r & 7);
+    const bool is_x = g * RPL < BM;
+    int64_t row;                                         // rows and columns past the end: the last one again, never stored
+    if (is_x) {
+      const int pos = min(row0 + r, rows_end - 1);
+      row = p.order ? p.order[pos] / p.row_div : pos;
+    } else if constexpr (GLU) {
+      const int in = (r - BM) % 16;
+      row = min(n0 + (r - BM) / 16 * 8 + in % 8, p.N - 1) + (in >= 8 ? p.N : 0);
     } else {
-      row = min(n0 + br, p.N - 1);
+      row = min(n0 + r - BM, p.N - 1);
     }
-    src[LA + i] = wbase + (int64_t)row * p.K * 2;
+    off[i] = (uint32_t)(row * (is_x ? p.a_stride : p.K) * 2) + chunk * 16;
+    base[i] = is_x ? p.a : we;
   }
-  const int steps = p.K / kWideBK;
-  const auto stage = [&](char* lds, int step) {
-#pragma unroll
-    for (int i = 0; i < LA + LB; ++i) {
-      char* dst = lds + (i < LA ? (wave * LA + i) : (kWideBM / 16 + wave * LB + i - LA)) * 1024;
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + step * (kWideBK * 2)),
-                                       (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-    }
-  };
+  const uint32_t lds0 = lds_address(lds);
   f32x4_q acc[FM][FN];
 #pragma unroll
   for (int f = 0; f < FM; ++f)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[f][j] = f32x4_q{0.f, 0.f, 0.f, 0.f};
-  const int c = (q ^ (r16 >> 2)) * 16;
-  const int arow0 = (wm * 64 + r16) * 64 + c, brow0 = (kWideBM + wn * CPW + r16) * 64 + c;
-  char *now = wide_lds, *next = wide_lds + kBuf;
-  stage(now, 0);
-  for (int s = 0; s < steps; ++s) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_barrier();
-    if (s + 1 < steps) stage(next, s + 1);
-    u32x4 xf[FM], wf[FN];
+  const int arow = (wm * TM + r16) * RB, brow = (BM + wn * TN + r16) * RB;
+  u32x4 xf[2][FM], wf[2][FN];
+  const auto read = [&](int buf, int kk) {
+    const int c = ((kk * 4 + q) ^ (r16 & 7)) * 16;
 #pragma unroll
-    for (int f = 0; f < FM; ++f) xf[f] = ld16(now + arow0 + f * 1024);
+    for (int j = 0; j < FN; ++j) wf[kk & 1][j] = ld16(lds + buf + brow + j * 16 * RB + c);
 #pragma unroll
-    for (int j = 0; j < FN; ++j) wf[j] = ld16(now + brow0 + j * 1024);
+    for (int f = 0; f < FM; ++f) xf[kk & 1][f] = ld16(lds + buf + arow + f * 16 * RB + c);
+  };
+  const auto product = [&](auto past) {                    // past: the weights past the L2
+    const auto load = [&](int i, int s, int buf) {
+      ring_load<decltype(past)::value>(off[i], base[i] + (int64_t)s * RB, lds0 + buf + min(i * W + wave, G - 1) * 1024);
+    };
+    for (int s = 0; s < ST && s < steps; ++s)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+      for (int i = 0; i < L; ++i) load(i, s, s * kStage);
+    ring_wait<L, ST - 1>(steps - 1);
+    ring_barrier();
+    read(0, 0);
+    int cur = 0;
+    const auto step = [&](int s, auto more) {               // more: there is a step ST ahead to load
+      constexpr bool MORE = decltype(more)::value;
+      const int next = cur == (ST - 1) * kStage ? 0 : cur + kStage;
 #pragma unroll
-      for (int f = 0; f < FM; ++f) acc[f][j] = mfma_q<Tag>(wf[j], xf[f], acc[f][j]);
-    char* const t = now;
-    now = next, next = t;
-  }
-  constexpr int FO = GLU ? FN / 2 : FN;
+      for (int kk = 0; kk < KK; ++kk) {
+        if (kk < KK - 1) {
+          read(cur, kk + 1);
+        } else if (MORE || s + 1 < steps) {
+          ring_wait<L, ST - 2>(MORE ? ST : steps - 2 - s);
+          ring_barrier();
+          if constexpr (MORE && PER < 2) {
+#pragma unroll
+            for (int i = 0; i < L; ++i) load(i, s + ST, cur);
+          }
+          read(next, 0);
+        }
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int n = 0; n < FN; ++n)
+#pragma unroll
+          for (int f = 0; f < FM; ++f) {
+            if constexpr (MORE && PER >= 2) {
+              if (kk == KK - 1 && (n * FM + f) % PER == 0 && (n * FM + f) / PER < L) {
+                __builtin_amdgcn_sched_barrier(0);
+                load((n * FM + f) / PER, s + ST, cur);
+                __builtin_amdgcn_sched_barrier(0);
+              }
+            }
+            acc[f][n] = mfma_q<Tag>(wf[kk & 1][n], xf[kk & 1][f], acc[f][n]);
+          }
+        __builtin_amdgcn_s_setprio(0);
+      }
+      cur = next;
+    };
+    int s = 0;
+    for (; s + ST < steps; ++s) step(s, std::true_type());
+    for (; s < steps; ++s) step(s, std::false_type());
+  };
+  if (ONCE && row_tiles == 1) product(std::integral_constant<bool, ONCE>());
+  else product(std::false_type());
 #pragma unroll
   for (int f = 0; f < FM; ++f) {
-    const int pos = row0 + wm * 64 + 16 * f + r16;
-    if (pos >= rows_end) continue;
+    const int pos = row0 + wm * TM + 16 * f + r16;
 #pragma unroll
-    for (int j = 0; j < FO; ++j) {
+    for (int j = 0; j < FN; ++j) {
       float v[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = grouped_act<Tag, ACT>(acc[f][j][r], GLU ? acc[f][j + FN - FO][r] : 0.f, p);
-      store4<Tag>(p, pos, n0 + wn * (GLU ? CPW / 2 : CPW) + 16 * j + 4 * q, v);
+      for (int r = 0; r < 4; ++r) {
+        const auto both = __builtin_amdgcn_permlane32_swap(as_u32(acc[f][j][r]), as_u32(acc[f][j][r]), false, false);      // [1]: lanes 32-63 twice
+        v[r] = grouped_act<Tag, ACT>(acc[f][j][r], GLU ? as_f32(both[1]) : 0.f, p);
+      }
+      if (pos < rows_end && !(GLU && q >= 2)) store4<Tag>(p, pos, GLU ? n0 + wn * (TN / 2) + 8 * j + 4 * q : n0 + wn * TN + 16 * j + 4 * q, v);
     }
   }
+}
+
+template <typename Tag, int BM, int BN, int BK, int WM, int WN, int ST, bool ONCE, int ACT>
+int launch_grouped_ring(const GroupedArgs& p, int pairs, int held, hipStream_t st) {
+  constexpr int lds = ST * (BM + BN) * BK * 2, per = ACT >= 2 ? BN / 2 : BN;
+  static PerDevice<int> raised;
+  int ok = 0;
+  raised.get(ok, [&](int) {
+    return hipFuncSetAttribute((const void*)moe_grouped_ring_kernel<Tag, BM, BN, BK, WM, WN, ST, ONCE, ACT>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess ? 1 : 0;
+  });
+  if (!ok) return SP_ERR_LAUNCH;
+  const int64_t ntiles = (p.N + per - 1) / per;
+  const unsigned blocks = (unsigned)(((pairs / BM + held) * ntiles + 7) / 8 * 8);
+  moe_grouped_ring_kernel<Tag, BM, BN, BK, WM, WN, ST, ONCE, ACT><<<dim3(blocks), dim3(WM * WN * 64), lds, st>>>(p);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
+
+// The tiles, and what one costs: us per step of BK where two workgroups share a unit and where one has it alone, and us besides.
+#define SP_RING_TILES(F)                                        \
+  F(0, 0.856f, 0.454f, 1.53f, 32, 128, 64, 1, 4, 4, true)       \
+  F(1, 0.787f, 0.389f, 2.88f, 32, 64, 128, 1, 4, 3, true)       \
+  F(2, 1.127f, 0.490f, 2.10f, 64, 128, 64, 2, 2, 3, true)       \
+  F(3, 0.636f, 0.129f, 4.05f, 64, 128, 64, 1, 4, 3, false)      \
+  F(4, 0.753f, 0.295f, 4.33f, 80, 128, 64, 1, 4, 3, false)      \
+  F(5, 0.423f, 0.118f, 3.98f, 96, 64, 64, 2, 2, 4, false)       \
+  F(6, 1.102f, 0.533f, 4.92f, 128, 128, 64, 2, 4, 2, false)     \
+  F(7, 1.269f, 0.664f, 5.16f, 160, 128, 64, 2, 2, 2, false)     \
+  F(8, 1.432f, 0.658f, 5.84f, 192, 128, 64, 4, 2, 2, false)     \
+  F(9, 3.326f, 1.018f, 5.36f, 192, 192, 64, 2, 4, 3, false)
+
+struct RingTile {
+  float two, one, fixed;
+  int bm, bn, bk, lds;
+  bool once;
+};
+#define SP_RING_ROW(I, TWO, ONE, FIXED, BM, BN, BK, WM, WN, ST, ONCE) {TWO, ONE, FIXED, BM, BN, BK, ST * (BM + BN) * BK * 2, ONCE},
+constexpr RingTile kRingTiles[] = {SP_RING_TILES(SP_RING_ROW)};
+
+// Expected row tiles of one expert of `experts`, each pair choosing each of them alike
+inline double ring_row_tiles(int pairs, int experts, int bm) {
+  const double mean = (double)pairs / experts, sd = sqrt(mean * (1. - 1. / experts));
+  double tiles = 1. - exp(-mean);
+  for (double edge = bm; edge < mean + 4. * sd; edge += bm) tiles += edge < mean - 4. * sd ? 1. : .5 * erfc((edge + .5 - mean) / (1.41421356 * sd));
+  return tiles;
+}
+
+// The time of a product with tile `t`: the longest of the chains of tiles that a unit works through, of what it loads into its LDS and of the
+// weights' way from memory, the two lesser ones added softly.  The last, not full round of tiles counts by the chance that it is there and that
+// some unit holds two of it.  Measured: 20 tiles, 58 products (widths 1024 and 2048, 8 to 128 experts, 8 to 4096 rows): 11 % rms from this, and the tile
+// chosen by it 3 % behind the best of the 20 on average.
+inline double ring_us(const RingTile& t, int pairs, int experts, int64_t wrows, int K) {
+  const double cols = (double)((wrows + t.bn - 1) / t.bn), tiles = experts * ring_row_tiles(pairs, experts, t.bm) * cols, steps = K / t.bk;
+  const bool pair = t.lds <= 80 * 1024;
+  const double slots = pair ? 512. : 256., one = t.fixed + steps * t.one, two = t.fixed + steps * t.two;
+  const double full = floor(tiles / slots), rest = tiles - full * slots, round = pair ? two : one;
+  double last = one;
+  if (pair && rest > 256.) last += (two - one) * (1. - exp((256. - rest) / cols)) * (.8 + .2 * std::min(1., std::max(0., rest / 256. - 1.)));
+  last *= 1. - exp(-rest / cols);
+  const double chain = full * round + (full > 0. ? .88 * last + .12 * std::min(last, rest / slots * round) : last);
+  const double fill = std::max(1., tiles / 256.) * steps * (t.bm + t.bn) * t.bk * 2. / 76.8e3;              // bytes per us of a unit
+  const double stream = experts * (1. - exp(-(double)pairs / experts)) * (double)wrows * K * 2. / (t.once ? 6.11e6 : 5.15e6);
+  const double c2 = chain * chain, f2 = fill * fill, s2 = stream * stream;
+  return c2 * c2 + f2 * f2 + s2 * s2;                                                                         // (its fourth power)
+}
+
+inline int ring_tile(int pairs, int experts, int64_t wrows, int K) {
+  int best = -1;
+  double least = 0.;
+  for (int i = 0; i < (int)(sizeof(kRingTiles) / sizeof(kRingTiles[0])); ++i) {
+    if (K % kRingTiles[i].bk) continue;
+    const double us = ring_us(kRingTiles[i], pairs, experts, wrows, K);
+    if (best < 0 || us < least) best = i, least = us;
+  }
+  return best;
 }
 
 // Steps with a few rows per expert (decode): a stream of the chosen experts' weights.  One wave per 16 rows x 32 weight rows
@@ -772,23 +888,27 @@ static bool narrow_pays(int pairs, int experts, int blocks) {
   return (long)pairs * blocks <= 256 || (chosen > 1024. && chosen <= 1536.);
 }
 
-// Which kernel: by the mean rows per expert, pairs / experts (the counts themselves are on the device).  Measured at width 2048,
-// 32 experts of ff 1024, top 4, up + down product in us (rows kernel | 64-row tiles | 128-row tiles):
-//   mean rows 1: 60 | 68 | 73     4: 85 | 92 | 94     8: 86 | 92 | 94     16: 104 | 93 | 96     32: 161 | 95 | 99
-//   64: 286 | 103 | 103     96: 410 | 138 | 107     128: 537 | 150 | 157     512: 2038 | 379 | 337
-// and from 320 rows on the 128 x 256 tiles (their comment has both sides).  (The kernel these replaced, one operand fragment per load
-// and no LDS: 75 at mean 1, 1398 at mean 512.)  The mean says nothing of a skewed step: with every pair on 4 of 128 experts, mean 10, the
-// rows kernel reads an expert's weights 20 times (491 us at width 4096, ff 1536, where the 64-row tiles take 95 at mean 11 and the replaced
-// kernel took 683).  Widths 1024 to 4096, 8 to 128 experts, routing even, by 1 / rank and to 4 experts, means 1 to 321: 1.1 to 9.4 times
-// as fast as the replaced kernel throughout.
+// Which kernel: by the mean rows per expert, pairs / experts (the counts themselves are on the device).  The rows kernel up to a mean of
+//   * 1.5.  Width 2048, 16 experts of ff 1408, up + down in us, rows kernel | ring tiles: mean 2: 44 + 18 | 40 + 18, 4: 43 + 19 | 39 + 18, 10: 43 + 19 |
+//     38 + 18; 32 experts of ff 1024, 3: 63 + 27 | 55 + 24, 16: 67 + 28 (64-row tiles) | 55 + 23; 128 of 512, width 1024, 4: 50 + 28 | 45 + 26;
+//   * 10 where it is at most one wave per SIMD: width 1024, 16 experts of ff 512, mean 2: 9.2 + 6.7 | 10.5 + 7.3, 10: 10.0 + 7.0 | 10.5 + 7.7; 32 experts,
+//     2 - 8: 14.5 + 9.2 | 15.0 + 9.6; 8 of 1536, width 2048, 2: 24.6 + 11.5 | 26.4 + 12.7, 10: 22.9 + 12.3 | 23.7 + 12.1 - and 12: 35 + 20 | 24 + 12;
+//   * 10 where the ring does not take the product (K no multiple of 64, 2^31 bytes of offsets), the 64-row tiles from there.
+// Else the ring tiles, the tile by ring_tile.  The mean says nothing of a skewed step.  Every pair on top_k experts, both products together, the
+// kernels and rules before -> these: 32 experts of ff 1024, 24 tokens 25.4 -> 29.2, 48: 33.3 -> 22.5, 200: 42.2 -> 31.8, 1000: 66.6 -> 72.3; 128 of 1536,
+// width 4096, 200: 114 -> 143, 800: 405 -> 316 (a tile chosen for fewer rows than there are reads an expert's weights more often).
 template <typename Tag, int ACT>
 int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
   const int held = pairs < p.E ? pairs : p.E;                    // experts with a row, at most
   const int row_tiles = pairs / 16 + held;
   // (moe_align takes 4096 experts, 6656 tiles; more than a grid's second dimension holds go to the 64-row tiles)
-  if (pairs <= 10 * (int64_t)p.E && row_tiles <= 65535) {
-    const int wide_per = ACT >= 2 ? 16 : 32;
-    const bool narrow = narrow_pays(pairs, p.E, (p.N + wide_per - 1) / wide_per);
+  // (a ring's loads have 32-bit offsets from the operand's first byte)
+  const int64_t last_row = p.order ? (int64_t)pairs / p.row_div + 1 : pairs;
+  const bool ring = p.K % 64 == 0 && last_row * p.a_stride < (int64_t)1 << 31 && (ACT >= 2 ? 2 : 1) * (int64_t)p.N * p.K < (int64_t)1 << 31;
+  const int wide_per = ACT >= 2 ? 16 : 32, blocks_of_rows = (p.N + wide_per - 1) / wide_per;
+  const int most = ring && (int64_t)p.E * blocks_of_rows > 1024 ? 3 : 20;                         // half rows per expert
+  if (2 * (int64_t)pairs <= most * (int64_t)p.E && row_tiles <= 65535) {
+    const bool narrow = narrow_pays(pairs, p.E, blocks_of_rows);
     const int per = narrow ? wide_per / 2 : wide_per;
     const dim3 grid((unsigned)((p.N + per - 1) / per), (unsigned)row_tiles);
     if (narrow) moe_grouped_narrow_rows_kernel<Tag, ACT><<<grid, 64, 0, st>>>(p);
@@ -796,20 +916,10 @@ int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
     SP_LAUNCH_CHECK();
     return SP_OK;
   }
-  if (pairs > 320 * (int64_t)p.E) {
-    constexpr int lds = 2 * (kWideBM + kWideBN) * kWideBK * 2;
-    static PerDevice<int> raised;
-    int ok = 0;
-    raised.get(ok, [&](int) {
-      return hipFuncSetAttribute((const void*)moe_grouped_wide_kernel<Tag, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) ==
-             hipSuccess ? 1 : 0;
-    });
-    if (!ok) return SP_ERR_LAUNCH;
-    const int wper = ACT >= 2 ? kWideBN / 2 : kWideBN;
-    const int64_t wtiles = (p.N + wper - 1) / wper;
-    moe_grouped_wide_kernel<Tag, ACT><<<dim3((unsigned)(((pairs / kWideBM + held) * wtiles + 7) / 8 * 8)), 256, lds, st>>>(p);
-    SP_LAUNCH_CHECK();
-    return SP_OK;
+  if (ring) {
+#define SP_RING_CASE(I, TWO, ONE, FIXED, ...) case I: return launch_grouped_ring<Tag, __VA_ARGS__, ACT>(p, pairs, held, st);
+    switch (ring_tile(pairs, p.E, (ACT >= 2 ? 2 : 1) * (int64_t)p.N, p.K)) { SP_RING_TILES(SP_RING_CASE) }
+    return SP_ERR_INVALID_ARG;
   }
   const int per = ACT >= 2 ? kGroupedBN / 2 : kGroupedBN;
   const int64_t ntiles = (p.N + per - 1) / per;

@@ -127,3 +127,50 @@ def test_combine(T, width, top, dtype):
     want = (z.float()[place.long()] * wt[..., None]).sum(1)
     bar = 2.0 ** -8 if dtype == torch.bfloat16 else top * 2.0 ** -23
     assert ((_native.moe_combine(z, place.view(-1), wt).float() - want).abs() <= bar * want.abs() + 1e-5).all()
+
+
+# (experts, mean rows, weight rows, K): the sizes at which each of the ring kernel's ten tiles is the one taken, K of fewer steps than a ring holds and more
+RING = [(2, 16, 128, 64), (8, 30, 200, 192), (2, 8, 128, 512), (2, 100, 128, 512), (32, 300, 200, 64), (32, 200, 384, 320), (16, 800, 200, 320),
+        (16, 800, 384, 64), (16, 150, 1024, 192), (32, 300, 200, 256), (32, 800, 200, 64), (8, 800, 1024, 64), (32, 500, 512, 64), (8, 500, 2048, 64),
+        (32, 800, 384, 64), (32, 150, 2048, 64), (16, 800, 512, 1024), (4, 800, 2048, 512)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("E,mean,N,K", RING)
+def test_ring_tiles_have_the_bits_of_the_rows_kernel(E, mean, N, K, dtype):
+    """the same rows among so many experts without any that the rows kernel takes them; uneven experts, one without rows and one with one"""
+    from scratchpad_amd import _native
+    print("ring", E, mean, N, K, dtype, flush=True)
+    counts = [mean] * E
+    counts[0], counts[1] = 2 * mean - 1, 1
+    if E > 2:
+        counts[2], counts[3] = 0, 2 * mean
+    a, w, offsets, order, expert, P = grouped_inputs(counts, N, K, dtype, 2, seed=7)
+    many = torch.empty(E + P, N, K, dtype=dtype, device=DEV)                   # (experts without rows are not read)
+    many[:E] = w
+    more = torch.cat([offsets, offsets[-1:].expand(P)]).contiguous()
+    got = _native.moe_grouped_gemm(a, w, offsets, P, order, 2)
+    assert torch.equal(got, _native.moe_grouped_gemm(a, many, more, P, order, 2))
+    rows = a[(order // 2).long()].float()
+    want = torch.cat([rows[expert == e] @ w[e].float().t() for e in range(E)])
+    scale = rows.abs().max() * w.float().abs().sum(-1).max()
+    bar = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11                  # as in test_grouped_products
+    assert ((got.float() - want).abs() <= 2 * bar * want.abs() + K * 2.0 ** -22 * scale).all()
+    assert torch.equal(_native.moe_grouped_gemm(a, w, offsets, P, order, 2, act="relu2"), _native.moe_grouped_gemm(a, many, more, P, order, 2, act="relu2"))
+    for act in (("silu",), ("clamped", 2.0, 1.702)):
+        assert torch.equal(_native.moe_grouped_glu(a, w, offsets, P, order, 2, *act), _native.moe_grouped_glu(a, many, more, P, order, 2, *act))
+
+
+def test_rows_far_from_the_first():
+    """rows of `a` that 32-bit offsets do not reach, named by an order of fewer pairs"""
+    from scratchpad_amd import _native
+    K, N, E, P = 4096, 64, 2, 100
+    a = torch.zeros(2 ** 31 // K + P, K, dtype=torch.bfloat16, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(9)
+    a[-P:] = torch.randn(P, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(E, N, K, generator=g, device=DEV) * K ** -0.5).bfloat16()
+    offsets = torch.tensor([0, 40, P], dtype=torch.int32, device=DEV)
+    order = torch.arange(a.shape[0] - P, a.shape[0], dtype=torch.int32, device=DEV)
+    near = a[-P:].clone()
+    assert torch.equal(_native.moe_grouped_gemm(a, w, offsets, P, order), _native.moe_grouped_gemm(near, w, offsets, P))
+    assert torch.equal(_native.moe_grouped_glu(a, w, offsets, P, order, 1, "silu"), _native.moe_grouped_glu(near, w, offsets, P, None, 1, "silu"))
