@@ -857,37 +857,43 @@ def library_rows_report() -> dict:
 
 
 # --------------------------------------------------------------------------- products of more rows
-DENSE_MAX_ROWS = 256          # and to 640 of long rows: dense_gemm_pays
+DENSE_MAX_ROWS = 256          # and to 1024 of long rows: dense_gemm_pays
 _DENSE_ON = os.environ.get("SP_DENSE_GEMM", "1") != "0"
-_DENSE_PLANS = {}             # (M, weight rows, K, epilogue) -> _dense_plan: sizes alone, at most 640 row counts per projection
+_DENSE_PLANS = {}             # (M, weight rows, K, epilogue) -> _dense_plan: sizes alone, at most 1024 row counts per projection
 
 
 def dense_gemm_pays(M: int, N: int, K: int) -> bool:
     """Where sp_gemm_dense measured faster than hipBLASLt on MI355X (us under graph replay, cold weights, library / own): 17 - 256
-    rows of most shapes (the table in gemm_dense.hip; mean 0.83 of the library's time over 21 shapes).  Past that the library's large
-    tiles win (320 rows: 28672 x 4096 79 / 98, 3072 x 2048 11.1 / 14.6) but where K is three times N it still runs few of them:
-    2048 x 8192 33 / 26 at 320 and 44 / 36 at 640 rows, 4096 x 14336 75 / 55 and 109 / 94, both even at 777 (1024 x 8192 22.6 / 24.2 at 512).
-    Left to the library below that: up to 512 weight rows, where it depends on K and rows (512 x 2048 5.5 / 6.7, 512 x 4096 11.7 / 7.1 at 64
+    rows of most shapes (the table in gemm_dense.hip).  Past that the library's large tiles win (320 rows: 28672 x 4096 81 / 84, 3072 x 2048
+    11.2 / 13.8; 1024: 28672 x 4096 169 / 208, 4096 x 4096 39 / 38) but where K is long and twice N, where it runs few of them:
+    2048 x 8192 33 / 26 at 320 rows, 45 / 36 at 640 and 50 / 45 at 1024, 4096 x 14336 76 / 52, 111 / 78 and 134 / 118, 4096 x 8192 47 / 38, 64 / 54 and
+    74 / 75, 8192 x 28672 226 / 164 and 262 / 267 (2048 x 4608 24.3 / 24.8 at 640; 1024 x 8192 22.6 / 24.2 at 512).
+    Left to the library below 257: up to 512 weight rows, where it depends on K and rows (512 x 2048 5.5 / 6.7, 512 x 4096 11.7 / 7.1 at 64
     rows); up to 2048 of them at K 2560 - 4096 past 64 rows (2048 x 4096 11.1 / 10.3 at 64 rows, 10.6 / 11.2 at 128, 1024 x 4096 12.2 / 8.0
-    and 9.4 / 9.6, 1536 x 4096 9.4 / 10.2 at 96); heads past 65536 columns with K <= 2048 from 96 rows on (128256 x 2048: 96 rows
-    131 / 130, 128 134 / 142, 192 142 / 155).
+    and 9.4 / 9.6, 1536 x 4096 9.4 / 10.2 at 96); 2049 to 4096 at K 1536 - 3072 and 10 M elements, where its tiles fit the rows (3072 x 2048 at 144:
+    9.6 / 11.5, 192: 16.1 / 12.1, 256: 11.0 / 12.2, 2560 x 2560 11.0 / 10.8, 11.0 / 11.6 and 12.4 / 14.3); heads past 65536 columns with K <= 2048 from 96
+    rows on (128256 x 2048: 96 rows 131 / 130, 128 134 / 142, 192 142 / 155).
     5 - 16 rows: matrices of more than 2^23 elements, where 16 rows of x beside every 16 weight rows are what sp_gemm_skinny waits for (that or
     the library, whichever is faster / own, at 5 / 8 / 16 rows: 28672 x 4096 49 / 42, 54 / 43, 61 / 44; 2048 x 8192 13.1 / 11.6, 12.8 / 11.7, 13.3 / 11.9;
     128256 x 4096 190 / 161, 193 / 162, 193 / 164; 4096 x 4096 10.2 / 9.9, 10.2 / 9.9, 11.5 / 10.1; 6144 x 2048 9.1 / 8.5, 9.4 / 8.5, 10.9 / 8.6); below that a
     launch of small workgroups is over sooner (2048 x 4096 7.9 / 8.4, 3072 x 2048 5.7 / 6.8, 2048 x 2048 5.6 / 6.3).  Up to 4096 x 4096
     both are even up to 8 rows (sp_gemm_skinny)."""
-    if M <= SKINNY_MAX_ROWS:
-        return M > 4 and K % 64 == 0 and N * K > 1 << 23 and (M > 8 or N > 4096 or K > 4096)
-    if K % 64 or N <= 512 or M > (640 if K >= 3 * N and N >= 2048 else DENSE_MAX_ROWS):
+    if K % 64:
         return False
-    if N <= 2048 and 2048 < K <= 4096:
-        return M <= 64
+    if M <= SKINNY_MAX_ROWS:
+        return M > 4 and N * K > 1 << 23 and (M > 8 or N > 4096 or K > 4096)
+    if M > DENSE_MAX_ROWS:
+        return N >= 2048 and K >= 2 * N and K > 5120 and M <= (1024 if N <= 6144 else 512)
+    if N <= 2048 and (N <= 512 or (2048 < K <= 4096 and M > 64)):
+        return False
+    if 2048 < N <= 4096 and 1536 <= K <= 3072 and N * K <= 10 << 20 and (128 < M <= 160 or M > 208):
+        return False
     return N <= 65536 or K > 2048 or M < 96
 
 
 def _dense_plan(M: int, N: int, K: int, epilogue: int) -> int:
     """sp_gemm_dense_plan of a product with N weight rows that dense_gemm_pays for, else -1"""
-    if M > 640:
+    if M > 1024:
         return -1
     key = (M, N, K, epilogue)
     plan = _DENSE_PLANS.get(key)

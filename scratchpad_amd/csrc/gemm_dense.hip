@@ -1,4 +1,4 @@
-// out[M, N] = x[M, K] . w[N, K]^T for steps of 17 - 256 rows (a server's decode batch, a short prompt; to 640 rows where K is three times N)
+// out[M, N] = x[M, K] . w[N, K]^T for steps of 17 - 256 rows (a server's decode batch, a short prompt; to 1024 rows where K is long and twice N)
 // and of 5 - 16 rows over large weights, 16-bit types.
 //
 // Call sites: the projections of every layer and the LM head (QKVParallelLinear / RowParallelLinear / MergedColumnParallelLinear.forward,
@@ -9,41 +9,29 @@
 // in (4096 x 14336 at 128 rows: 32 tiles), or rows computed for nothing.  Here
 //   * the tile follows the rows (16 - 256) and is narrow (16 - 128 weight rows), so that about one workgroup per compute unit streams;
 //     where K is long, its shares go to workgroups of their own and a second launch adds them (2 us + the sums' traffic);
-//   * both operands go to LDS by direct loads, into rings of steps: the first waves load x, the others w, each with its own count of
+//   * both operands go to LDS by direct loads, into rings of steps; up to about 128 rows the first waves load x, the others w, each with its own count of
 //     steps in flight (loads retire in order: in one wave, x out of the L2 would wait behind weights out of HBM);
 //   * weights are loaded past the L2 (nt): a stream of 235 MB takes 37 us with it and 42 without;
 //   * a step is one barrier, in front of its last products: the next step's first operands are read behind it, under them;
 //   * small tiles split every 64 of k over two groups of waves (WK): twice the waves to hide LDS behind, one exchange at the end.
+// From about 128 rows on the matrix cores and the stream take as long as each other, and a wave's direct loads hold its products up: there
+// dense_wide_kernel, whose waves all load both operands and spread the loads between their products (28672 x 4096 at 256 rows 74.7 us by waves of
+// either kind, 66.2 so; 4096 x 14336 48.2 and 44.2, at 640 rows 94 and 76; 2048 x 8192 24.2 and 21.4).
 // us under graph replay, cold weights, library -> this:         rows 17           64           128          256
-//   3072 x 2048 (qkv, hidden 2048)                          8.9 ->  7.6   9.5 ->  7.8   12.1 ->  9.7   10.9 -> 12.7
-//   2048 x 2048                                             8.6 ->  7.4   9.2 ->  7.5    8.8 ->  7.7   10.0 ->  9.8
-//   16384 x 2048 (gate and up)                             18.6 -> 16.2  18.3 -> 17.0   20.9 -> 21.1   30.7 -> 26.5
-//   2048 x 8192 (down)                                     14.2 -> 12.2  22.5 -> 13.9   21.3 -> 18.1   27.1 -> 22.6
-//   6144 x 4096 (qkv, hidden 4096)                         16.3 -> 13.4  18.3 -> 17.0   25.5 -> 21.9   40.2 -> 29.7
-//   4096 x 4096                                            14.2 -> 11.9  15.3 -> 12.6   24.6 -> 15.7   22.7 -> 21.4
-//   28672 x 4096                                           55.4 -> 48.5  54.7 -> 48.6   58.7 -> 55.6   71.9 -> 68.7
-//   4096 x 14336                                           30.0 -> 23.8  38.9 -> 28.6   75.9 -> 34.0   62.1 -> 48.2
+//   3072 x 2048 (qkv, hidden 2048)                          8.9 ->  7.6   9.5 ->  7.8   12.1 ->  9.6   11.0 -> 12.2
+//   2048 x 2048                                             8.6 ->  7.4   9.2 ->  7.5    8.8 ->  7.5    9.8 ->  9.6
+//   16384 x 2048 (gate and up)                             18.6 -> 16.2  18.3 -> 17.0   22.4 -> 20.7   30.6 -> 26.1
+//   2048 x 8192 (down)                                     14.2 -> 12.2  22.5 -> 13.9   21.4 -> 17.3   26.9 -> 21.4
+//   6144 x 4096 (qkv, hidden 4096)                         16.3 -> 13.4  18.3 -> 17.0   25.4 -> 21.3   41.0 -> 28.3
+//   4096 x 4096                                            14.2 -> 11.9  15.3 -> 12.6   24.7 -> 16.2   22.9 -> 20.4
+//   28672 x 4096                                           55.4 -> 48.5  54.7 -> 48.6   60.3 -> 53.1   74.2 -> 66.2
+//   4096 x 14336                                           30.0 -> 23.8  38.9 -> 28.6   76.2 -> 34.2   61.2 -> 47.5
 // 5 / 8 / 16 rows (the library or sp_gemm_skinny, whichever was faster): 28672 x 4096 49 -> 42, 54 -> 43, 61 -> 44; 128256 x 4096 190 -> 161,
-// 193 -> 162, 193 -> 164.  At 256 rows x 28672 the x tile takes two thirds of what a unit can have in flight (160 KB of LDS); from 512 rows on the library's
-// 256 x 256 tiles are up to 30 % faster where N is large.
+// 193 -> 162, 193 -> 164.  From 512 rows on the library's 256 x 256 tiles are 10 - 30 % faster where N is large.
 #include "lds_ring.h"
-
-#include <type_traits>
 
 namespace sp {
 namespace {
-
-typedef float f32x4_d __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8_d __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_d __attribute__((ext_vector_type(8)));
-
-template <typename Tag>
-__device__ __forceinline__ f32x4_d mfma_d(const u32x4& a, const u32x4& b, const f32x4_d& c) {
-  if constexpr (std::is_same<Tag, bf16_tag>::value)
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_d, a), __builtin_bit_cast(bf16x8_d, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_d, a), __builtin_bit_cast(f16x8_d, b), c, 0, 0, 0);
-}
 
 struct DenseArgs {
   char* out;
@@ -66,10 +54,52 @@ struct Tile {
   static constexpr int kOcc = kLds <= 80 * 1024 && kWaves <= 4 ? 2 : kWaves / 4;      // waves per SIMD
 };
 
+// acc[f][j][r] = out[row 16 f + lane % 16][column 16 j + 4 (lane / 16) + r] of a wave's FM x FN tiles at m0, n0 (EPI: the lanes below 32 the gate
+// sums of column 8 j + 4 q + r, the lanes 32 above them its up sums)
+template <typename Tag, int FM, int FN, int EPI, bool SPLIT>
+__device__ __forceinline__ void dense_store(const DenseArgs& p, const ring_f32x4 (&acc)[FM][FN], int m0, int n0, int split, int lane) {
+  typedef Elem<Tag> E;
+  const int r16 = lane & 15, q = lane >> 4;
+#pragma unroll
+  for (int f = 0; f < FM; ++f) {
+    const int m = m0 + 16 * f + r16;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int n = n0 + (EPI ? 8 : 16) * j + 4 * q;
+      const bool mine = m < p.M && n < p.N && !(EPI && q >= 2);
+      if constexpr (SPLIT) {
+        float* const to = p.part + ((int64_t)split * p.M + m) * p.N + n;
+        if (mine && p.vec) *(ring_f32x4*)to = acc[f][j];
+        else if (mine)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < p.N) to[r] = acc[f][j][r];
+      } else {
+        uint32_t h[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float v = acc[f][j][r];
+          if constexpr (EPI) {
+            const auto both = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);      // lanes 0-31 twice, 32-63 twice
+            v = mul_round<Tag>(E::round(silu_ref(E::round(v))), E::round(as_f32(both[1])));
+          }
+          if constexpr (std::is_same<Tag, bf16_tag>::value) h[r] = f32_to_bf16_bits(v);
+          else h[r] = f32_to_f16_bits(v);
+        }
+        char* const to = p.out + ((int64_t)m * p.out_stride + n) * 2;
+        if (mine && p.vec) *(u32x2*)to = u32x2{h[0] | h[1] << 16, h[2] | h[3] << 16};
+        else if (mine)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < p.N) ((uint16_t*)to)[r] = (uint16_t)h[r];
+      }
+    }
+  }
+}
+
 // EPI: 0 the product; 1 w is [2 N, K], gate rows then up rows, and the output silu(gate) * up of the rounded sums
 template <typename Tag, typename T, int EPI, bool SPLIT>
 __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArgs p) {
-  typedef Elem<Tag> E;
   constexpr int RB = T::BK * 2, RPL = 1024 / RB, CH = T::BK / 8;          // bytes of a row, rows and chunks of 16 bytes a load
   constexpr int TM = T::BM / T::WM, TN = T::BN / T::WN, FM = TM / 16, FN = TN / 16, KS = T::BK / 32 / T::WK;
   constexpr int GX = T::BM / RPL, GW = T::BN / RPL, WW = T::kWaves - T::WX;
@@ -115,11 +145,11 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
     for (int i = 0; i < LW; ++i)
       ring_load<true>(off[i], src + (int64_t)s * RB, lds0 + T::SX * T::kX + buf + min((wave - T::WX) * LW + i, GW - 1) * 1024);
   };
-  f32x4_d acc[FM][FN];
+  ring_f32x4 acc[FM][FN];
 #pragma unroll
   for (int f = 0; f < FM; ++f)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[f][j] = f32x4_d{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < FN; ++j) acc[f][j] = ring_f32x4{0.f, 0.f, 0.f, 0.f};
   const int arow = (wm * TM + r16) * RB, brow = T::SX * T::kX + (wn * TN + r16) * RB;
   u32x4 xf[2][FM], wf[2][FN];
   const auto read = [&](int bx, int bw, int kk, int to) {
@@ -163,7 +193,7 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
 #pragma unroll
       for (int n = 0; n < FN; ++n)
 #pragma unroll
-        for (int f = 0; f < FM; ++f) acc[f][n] = mfma_d<Tag>(wf[at][n], xf[at][f], acc[f][n]);
+        for (int f = 0; f < FM; ++f) acc[f][n] = mfma32<Tag>(wf[at][n], xf[at][f], acc[f][n]);
     }
     cx = nx, cw = nw;
   };
@@ -179,7 +209,7 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
   if constexpr (T::WK > 1) {                              // the two halves of every 64 of k meet in LDS, the first wave's plus the second's
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     ring_barrier();
-    f32x4_d* const sums = (f32x4_d*)lds + wmn * FM * FN * 64 + lane;
+    ring_f32x4* const sums = (ring_f32x4*)lds + wmn * FM * FN * 64 + lane;
     if (wk) {
 #pragma unroll
       for (int f = 0; f < FM; ++f)
@@ -194,43 +224,51 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
 #pragma unroll
       for (int n = 0; n < FN; ++n) acc[f][n] += sums[(f * FN + n) * 64];
   }
-  // acc[f][j][r] = out[row 16 f + r16][column 16 j + 4 q + r] of the wave's tile (EPI: the lanes below 32 the gate sums of column
-  // 8 j + 4 q + r, the lanes 32 above them its up sums)
+  dense_store<Tag, FM, FN, EPI, SPLIT>(p, acc, m0 + wm * TM, n0 + wn * (EPI ? TN / 2 : TN), split, lane);
+}
+
+// The same by ring_product's loop, for more rows: every wave loads both operands, its loads spread between its products.  Past the L2 only the weights of
+// an unsplit product with one row block: at 256 rows 28672 x 4096 66 us with it and 72 without, 4096 x 14336 in 8 shares 44 and 45, at 192 41 and 39.
+// Four row blocks share the columns they pass: their rows of x and a few columns stay in an XCD's L2.
+constexpr int kRowGroup = 4;
+
+template <typename Tag, typename T, int EPI, bool SPLIT>
+__global__ void __launch_bounds__(T::W * 64, T::kWaves) dense_wide_kernel(DenseArgs p) {
+  extern __shared__ __attribute__((aligned(1024))) char dense_lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int total = p.mblocks * p.nblocks * p.splits, share = (total + 7) / 8;
+  const int idx = (int)(blockIdx.x >> 3), at = (int)(blockIdx.x & 7) * share + idx;
+  if (idx >= share || at >= total) return;
+  const int blocks = p.mblocks * p.nblocks, split = at / blocks, t = at % blocks;
+  const int group = t / (kRowGroup * p.nblocks), high = min(kRowGroup, p.mblocks - group * kRowGroup), in = t - group * kRowGroup * p.nblocks;
+  const int m0 = (group * kRowGroup + in % high) * T::BM, n0 = in / high * (EPI ? T::BN / 2 : T::BN);
+  const int ksteps = p.K / T::BK, first = ksteps * split / p.splits, steps = ksteps * (split + 1) / p.splits - first;
+  uint32_t off[T::L];
+  const char* base[T::L];
 #pragma unroll
-  for (int f = 0; f < FM; ++f) {
-    const int m = m0 + wm * TM + 16 * f + r16;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int n = EPI ? n0 + wn * (TN / 2) + 8 * j + 4 * q : n0 + wn * TN + 16 * j + 4 * q;
-      const bool mine = m < p.M && n < p.N && !(EPI && q >= 2);
-      if constexpr (SPLIT) {
-        float* const to = p.part + ((int64_t)split * p.M + m) * p.N + n;
-        if (mine && p.vec) *(f32x4_d*)to = acc[f][j];
-        else if (mine)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (n + r < p.N) to[r] = acc[f][j][r];
-      } else {
-        uint32_t h[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float v = acc[f][j][r];
-          if constexpr (EPI) {
-            const auto both = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);      // lanes 0-31 twice, 32-63 twice
-            v = mul_round<Tag>(E::round(silu_ref(E::round(v))), E::round(as_f32(both[1])));
-          }
-          if constexpr (std::is_same<Tag, bf16_tag>::value) h[r] = f32_to_bf16_bits(v);
-          else h[r] = f32_to_f16_bits(v);
-        }
-        char* const to = p.out + ((int64_t)m * p.out_stride + n) * 2;
-        if (mine && p.vec) *(u32x2*)to = u32x2{h[0] | h[1] << 16, h[2] | h[3] << 16};
-        else if (mine)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (n + r < p.N) ((uint16_t*)to)[r] = (uint16_t)h[r];
-      }
+  for (int i = 0; i < T::L; ++i) {
+    const int g = min(i * T::W + wave, T::G - 1), r = g * T::RPL + lane / T::CH, chunk = (lane % T::CH) ^ (r & 7);
+    const bool is_x = g * T::RPL < T::BM;
+    int row;                                               // rows and columns past the end: the last one again, never stored
+    if (is_x) {
+      row = min(m0 + r, p.M - 1);
+    } else if constexpr (EPI) {
+      const int pos = (r - T::BM) % 16;                    // 8 gate rows, then the up rows of the same 8 columns
+      row = min(n0 + (r - T::BM) / 16 * 8 + pos % 8, p.N - 1) + (pos >= 8 ? p.N : 0);
+    } else {
+      row = min(n0 + r - T::BM, p.N - 1);
     }
+    off[i] = (uint32_t)row * (uint32_t)((is_x ? p.x_stride : p.w_stride) * 2) + chunk * 16;
+    base[i] = (is_x ? p.x : p.w) + (int64_t)first * T::RB;
   }
+  ring_f32x4 acc[T::FM][T::FN];
+#pragma unroll
+  for (int f = 0; f < T::FM; ++f)
+#pragma unroll
+    for (int j = 0; j < T::FN; ++j) acc[f][j] = ring_f32x4{0.f, 0.f, 0.f, 0.f};
+  if (!SPLIT && p.mblocks == 1) ring_product<Tag, T, 2, 1>(acc, off, base, dense_lds, steps, wave, lane);
+  else ring_product<Tag, T, 0, 1>(acc, off, base, dense_lds, steps, wave, lane);
+  dense_store<Tag, T::FM, T::FN, EPI, SPLIT>(p, acc, m0 + wave / T::WN * T::TM, n0 + wave % T::WN * (EPI ? T::TN / 2 : T::TN), split, lane);
 }
 
 // the shares of K summed in their order, 4 columns of a row a thread
@@ -244,13 +282,13 @@ __global__ void __launch_bounds__(256) dense_sum_kernel(DenseArgs p) {
   const float* from = p.part + (int64_t)m * p.N + n;
   const int64_t step = (int64_t)p.M * p.N;
   if (p.vec) {
-    f32x4_d v[S];
+    ring_f32x4 v[S];
 #pragma unroll
-    for (int s = 0; s < S; ++s) v[s] = *(const f32x4_d*)(from + s * step);
+    for (int s = 0; s < S; ++s) v[s] = *(const ring_f32x4*)(from + s * step);
 #pragma unroll
     for (int by = 1; by < S; by *= 2)                          // in pairs: each share is rounded log2 S times
 #pragma unroll
-      for (int s = 0; s < S; s += 2 * by) v[s] += v[s + by];
+      for (int s = 0; s + by < S; s += 2 * by) v[s] += v[s + by];
     u32x2 o;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -267,23 +305,31 @@ __global__ void __launch_bounds__(256) dense_sum_kernel(DenseArgs p) {
 #pragma unroll
       for (int by = 1; by < S; by *= 2)
 #pragma unroll
-        for (int s = 0; s < S; s += 2 * by) v[s] += v[s + by];
+        for (int s = 0; s + by < S; s += 2 * by) v[s] += v[s + by];
       E::store(p.out, (int64_t)m * p.out_stride + n + r, v[0]);
     }
   }
 }
 
+template <typename T, typename = void>
+struct IsRing : std::false_type {};
+template <typename T>
+struct IsRing<T, std::enable_if_t<(T::ST > 0)>> : std::true_type {};
+
 template <typename Tag, typename T, int EPI, bool SPLIT>
 int launch_dense_kernel(const DenseArgs& p, hipStream_t st) {
+  void (*kernel)(DenseArgs);
+  int threads;
+  if constexpr (IsRing<T>::value) kernel = dense_wide_kernel<Tag, T, EPI, SPLIT>, threads = T::W * 64;
+  else kernel = dense_kernel<Tag, T, EPI, SPLIT>, threads = T::kWaves * 64;
   static PerDevice<int> raised;
   int ok = 0;
   raised.get(ok, [&](int) {
-    return hipFuncSetAttribute((const void*)dense_kernel<Tag, T, EPI, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, T::kLds) ==
-                   hipSuccess ? 1 : 0;
+    return hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, T::kLds) == hipSuccess ? 1 : 0;
   });
   if (!ok) return SP_ERR_LAUNCH;
   const int total = p.mblocks * p.nblocks * p.splits;
-  dense_kernel<Tag, T, EPI, SPLIT><<<dim3((total + 7) / 8 * 8), dim3(T::kWaves * 64), T::kLds, st>>>(p);
+  kernel<<<dim3((total + 7) / 8 * 8), dim3(threads), T::kLds, st>>>(p);
   SP_LAUNCH_CHECK();
   return SP_OK;
 }
@@ -299,9 +345,13 @@ int launch_dense_tile(DenseArgs p, int epilogue, hipStream_t st) {
   const int rc = launch_dense_kernel<Tag, T, 0, true>(p, st);
   if (rc != SP_OK) return rc;
   const dim3 grid((unsigned)(((int64_t)p.M * ((p.N + 3) / 4) + 255) / 256));
-  if (p.splits == 2) dense_sum_kernel<Tag, 2><<<grid, 256, 0, st>>>(p);
-  else if (p.splits == 4) dense_sum_kernel<Tag, 4><<<grid, 256, 0, st>>>(p);
-  else dense_sum_kernel<Tag, 8><<<grid, 256, 0, st>>>(p);
+  switch (p.splits) {
+    case 2: dense_sum_kernel<Tag, 2><<<grid, 256, 0, st>>>(p); break;
+    case 3: dense_sum_kernel<Tag, 3><<<grid, 256, 0, st>>>(p); break;
+    case 4: dense_sum_kernel<Tag, 4><<<grid, 256, 0, st>>>(p); break;
+    case 6: dense_sum_kernel<Tag, 6><<<grid, 256, 0, st>>>(p); break;
+    default: dense_sum_kernel<Tag, 8><<<grid, 256, 0, st>>>(p);
+  }
   SP_LAUNCH_CHECK();
   return SP_OK;
 }
@@ -310,37 +360,43 @@ int launch_dense_tile(DenseArgs p, int epilogue, hipStream_t st) {
 // Every tile's cost: us of one step of one workgroup and of a workgroup's beginning and end, both fitted (with the constants below) to
 // 7600 timings over 23 shapes of 1 - 1050 MB at 5 - 640 rows.  A product takes the chain of its busiest unit, the traffic into
 // that unit's LDS or the weights' stream, whichever is longest; the choice is within 1.2 % of the fastest tile and split on average.
-#define SP_DENSE_TILES(F)                              \
-  F(0, 0.655f, 2.26f, 16, 64, 256, 2, 1, 4, 2, 3, 4)   \
-  F(1, 0.588f, 2.04f, 16, 128, 128, 1, 1, 8, 1, 4, 4)  \
-  F(2, 0.293f, 2.39f, 32, 16, 256, 2, 2, 1, 2, 4, 8)   \
-  F(3, 0.418f, 2.60f, 32, 32, 256, 1, 2, 2, 2, 4, 5)   \
-  F(4, 0.404f, 2.17f, 32, 32, 256, 2, 2, 2, 4, 3, 6)   \
-  F(5, 0.933f, 1.78f, 32, 64, 256, 2, 1, 4, 2, 2, 4)   \
-  F(6, 0.627f, 2.62f, 32, 128, 128, 1, 1, 8, 2, 3, 4)  \
-  F(7, 0.474f, 2.86f, 48, 32, 256, 2, 1, 2, 2, 3, 5)   \
-  F(8, 0.248f, 3.08f, 64, 16, 256, 2, 4, 1, 4, 3, 7)   \
-  F(9, 0.258f, 2.62f, 64, 32, 128, 2, 2, 2, 4, 4, 6)   \
-  F(10, 0.228f, 2.55f, 64, 64, 64, 1, 2, 2, 2, 4, 6)   \
-  F(11, 0.578f, 3.53f, 64, 64, 256, 2, 2, 2, 4, 2, 3)  \
-  F(12, 0.648f, 3.52f, 64, 128, 128, 1, 2, 4, 4, 2, 4) \
-  F(13, 0.565f, 2.63f, 96, 64, 128, 1, 2, 4, 4, 3, 4)  \
-  F(14, 0.395f, 3.12f, 96, 128, 64, 1, 2, 4, 4, 4, 6)  \
-  F(15, 0.398f, 2.98f, 128, 96, 64, 1, 4, 2, 4, 4, 6)  \
-  F(16, 0.474f, 3.37f, 128, 128, 64, 1, 2, 4, 4, 4, 6) \
-  F(17, 0.536f, 5.39f, 192, 128, 64, 2, 2, 2, 4, 3, 5) \
-  F(18, 0.661f, 6.46f, 256, 128, 64, 2, 2, 2, 4, 2, 6)
-constexpr int kDenseTiles = 19;
-constexpr float kLaunch = 1.72f, kStream = 5.43e6f, kFill = 67.72e3f, kSumLaunch = 2.f, kSumRate = 3.76e6f;     // us, bytes per us
+#define SP_DENSE_TILES(F)                                \
+  F(0, 0.655f, 2.26f, 16, 64, 256, 2, 1, 4, 2, 3, 4)     \
+  F(1, 0.588f, 2.04f, 16, 128, 128, 1, 1, 8, 1, 4, 4)    \
+  F(2, 0.293f, 2.39f, 32, 16, 256, 2, 2, 1, 2, 4, 8)     \
+  F(3, 0.404f, 2.17f, 32, 32, 256, 2, 2, 2, 4, 3, 6)     \
+  F(4, 0.933f, 1.78f, 32, 64, 256, 2, 1, 4, 2, 2, 4)     \
+  F(5, 0.627f, 2.62f, 32, 128, 128, 1, 1, 8, 2, 3, 4)    \
+  F(6, 0.474f, 2.86f, 48, 32, 256, 2, 1, 2, 2, 3, 5)     \
+  F(7, 0.258f, 2.62f, 64, 32, 128, 2, 2, 2, 4, 4, 6)     \
+  F(8, 0.228f, 2.55f, 64, 64, 64, 1, 2, 2, 2, 4, 6)      \
+  F(9, 0.578f, 3.53f, 64, 64, 256, 2, 2, 2, 4, 2, 3)     \
+  F(10, 0.648f, 3.52f, 64, 128, 128, 1, 2, 4, 4, 2, 4)   \
+  F(11, 0.565f, 2.63f, 96, 64, 128, 1, 2, 4, 4, 3, 4)    \
+  F(12, 0.395f, 3.12f, 96, 128, 64, 1, 2, 4, 4, 4, 6)    \
+  F(13, 0.398f, 2.98f, 128, 96, 64, 1, 4, 2, 4, 4, 6)
+// and of dense_wide_kernel, from 2300 timings over 10 shapes at 96 - 1024 rows; the choice among all tiles is within 0.9 % of the fastest there
+#define SP_WIDE_TILES(F)                        \
+  F(14, 0.315f, 1.07f, 128, 64, 64, 2, 2, 3)    \
+  F(15, 0.372f, 2.90f, 128, 128, 64, 2, 4, 4)   \
+  F(16, 0.428f, 4.44f, 192, 128, 64, 4, 2, 4)   \
+  F(17, 0.511f, 4.85f, 256, 128, 64, 4, 2, 3)   \
+  F(18, 0.426f, 3.97f, 256, 96, 64, 4, 2, 3)    \
+  F(19, 0.768f, 4.95f, 160, 256, 64, 2, 4, 3)   \
+  F(20, 0.548f, 5.27f, 192, 192, 64, 2, 4, 3)
+constexpr int kDenseTiles = 21, kFirstWide = 14;
+constexpr float kLaunch = 1.72f, kStream = 5.43e6f, kFill = 67.72e3f;     // us, bytes per us
 constexpr int kUnits = 256;
 
 struct TileCost {
   int bm, bn, bk, wk, lds;
-  float step, fixed;
+  float step, fixed, sum, rate;       // the launch that adds the shares: us, and bytes per us
 };
 #define SP_DENSE_COST(I, STEP, FIXED, ...) \
-  {Tile<__VA_ARGS__>::BM, Tile<__VA_ARGS__>::BN, Tile<__VA_ARGS__>::BK, Tile<__VA_ARGS__>::WK, Tile<__VA_ARGS__>::kLds, STEP, FIXED},
-constexpr TileCost kCosts[kDenseTiles] = {SP_DENSE_TILES(SP_DENSE_COST)};
+  {Tile<__VA_ARGS__>::BM, Tile<__VA_ARGS__>::BN, Tile<__VA_ARGS__>::BK, Tile<__VA_ARGS__>::WK, Tile<__VA_ARGS__>::kLds, STEP, FIXED, 2.f, 3.76e6f},
+#define SP_WIDE_COST(I, STEP, FIXED, ...) \
+  {RingTile<__VA_ARGS__>::BM, RingTile<__VA_ARGS__>::BN, RingTile<__VA_ARGS__>::BK, 1, RingTile<__VA_ARGS__>::kLds, STEP, FIXED, 4.03f, 5.9e6f},
+constexpr TileCost kCosts[kDenseTiles] = {SP_DENSE_TILES(SP_DENSE_COST) SP_WIDE_TILES(SP_WIDE_COST)};
 
 float dense_us(const TileCost& c, int M, int64_t rows, int K, int splits) {
   const int64_t wgs = (M + c.bm - 1) / c.bm * ((rows + c.bn - 1) / c.bn) * splits;
@@ -351,7 +407,7 @@ float dense_us(const TileCost& c, int M, int64_t rows, int K, int splits) {
   const float stream = 2.f * (float)rows * (float)K / kStream;
   const float c2 = chain * chain, f2 = fill * fill, s2 = stream * stream;
   float us = kLaunch + sqrtf(sqrtf(c2 * c2 + f2 * f2 + s2 * s2));
-  if (splits > 1) us += kSumLaunch + 8.f * (float)splits * (float)M * (float)rows / kSumRate;
+  if (splits > 1) us += c.sum + 8.f * (float)splits * (float)M * (float)rows / c.rate;
   return us;
 }
 
@@ -359,7 +415,9 @@ template <typename Tag>
 int launch_dense(const DenseArgs& p, int tile, int epilogue, hipStream_t st) {
 #define SP_DENSE_CASE(I, STEP, FIXED, ...) \
   case I: return launch_dense_tile<Tag, Tile<__VA_ARGS__>>(p, epilogue, st);
-  switch (tile) { SP_DENSE_TILES(SP_DENSE_CASE) }
+#define SP_WIDE_CASE(I, STEP, FIXED, ...) \
+  case I: return launch_dense_tile<Tag, RingTile<__VA_ARGS__>>(p, epilogue, st);
+  switch (tile) { SP_DENSE_TILES(SP_DENSE_CASE) SP_WIDE_TILES(SP_WIDE_CASE) }
   return SP_ERR_INVALID_ARG;
 }
 
@@ -377,8 +435,11 @@ extern "C" int sp_gemm_dense_plan(int M, int N, int K, int epilogue) {
   float least = 0.f;
   for (int i = 0; i < sp::kDenseTiles; ++i) {
     const sp::TileCost& c = sp::kCosts[i];
-    if (K % c.bk || (epilogue && c.wk != sp::kCosts[plain & 255].wk)) continue;
-    for (int splits = 1; splits <= (epilogue ? 1 : 8); splits *= 2) {
+    // (the first tiles' costs hold up to 256 rows: 3072 x 3072 at 777 they promise less than the 29 us that they take, dense_wide_kernel 25 - 30)
+    if (K % c.bk || (M > 256 && i < sp::kFirstWide) || (epilogue && c.wk != sp::kCosts[plain & 255].wk)) continue;
+    for (int splits : {1, 2, 3, 4, 6, 8}) {
+      if (splits > 1 && epilogue) break;
+      if (i < sp::kFirstWide && splits % 3 == 0) continue;
       // shares of at least three steps, for launches that would leave units idle, with sums that stay in the caches
       if (splits > 1 && (K / c.bk / splits < 3 || (M + c.bm - 1) / c.bm * (int64_t)((rows + c.bn - 1) / c.bn) * splits > 600 ||
                          4 * (int64_t)splits * M * N > (int64_t)128 << 20))
@@ -396,7 +457,7 @@ extern "C" int sp_gemm_dense(void* out, const void* x, const void* w, float* sum
   if (M == 0 || N == 0) return SP_OK;
   SP_CHECK_ARG(out && x && w && plan >= 0);
   const int tile = plan & 255, splits = plan >> 8;
-  SP_CHECK_ARG(tile < sp::kDenseTiles && (splits == 1 || splits == 2 || splits == 4 || splits == 8));
+  SP_CHECK_ARG(tile < sp::kDenseTiles && (splits <= 4 || splits == 6 || splits == 8) && splits >= 1);
   SP_CHECK_ARG(splits == 1 || (sums && ((uintptr_t)sums & 15) == 0 && sums_floats >= (int64_t)splits * M * N));
   const int64_t rows = epilogue ? 2 * (int64_t)N : N;
   SP_CHECK_ARG(x_stride % 8 == 0 && w_stride % 8 == 0 && x_stride >= K && w_stride >= K && out_stride >= N);

@@ -566,27 +566,17 @@ __global__ void __launch_bounds__(256, 2) moe_grouped_tile_kernel(GroupedArgs p)
   }
 }
 
-// The same for K a multiple of 64: BM rows x BN weight rows per workgroup, k in steps of BK, ST steps in a ring of LDS buffers.
-// One barrier a step, in front of its last products: behind it the next step's first operands are read, and the loads into the buffer
-// that has become free are spread between those products - in one piece they hold a wave's products up (an instruction a wave can't
-// issue stops the ones behind it): a 256 x 256 tile's loop, operands in the L2, 1245 -> 1480 TFLOP/s with the loads spread and the waves
-// in their products ahead of the others.  Two workgroups share a CU (of all tiles but the largest) and fill each other's beginnings and ends.  GLU: 8 gate rows and the up
-// rows of the same 8 columns in one operand, their sums 32 lanes apart.  ONCE: an expert with one row tile reads its weights past the L2.
-// The row tiles of one column tile follow each other: the weights they share are in the L2.
+// The same for K a multiple of 64, by ring_product's loop.  Two workgroups share a CU (of all tiles but the largest) and fill each other's beginnings
+// and ends.  GLU: 8 gate rows and the up rows of the same 8 columns in one operand, their sums 32 lanes apart.  ONCE: an expert with one row tile reads
+// its weights past the L2.  The row tiles of one column tile follow each other: the weights they share are in the L2.
 // Width 2048, 32 experts of ff 1024, up + down in us, the kernels before (64 x 128, 128 x 128 and 128 x 256 tiles, one wave per 16 rows) -> these: mean rows
 // 3: 63 + 27 -> 55 + 24, 16: 67 + 28 -> 55 + 23, 32: 68 + 29 -> 59 + 25, 50: 69 + 30 -> 60 + 30, 88: 72 + 32 -> 74 + 32, 125: 97 + 51 -> 82 + 34, 188: 98 + 52 ->
 // 102 + 53, 250: 134 + 70 -> 111 + 58, 512: 180 + 107 -> 171 + 92; width 4096, 128 experts of 1536, 4: 560 + 270 -> 481 + 239, 256: 1344 + 735 -> 1110 + 617;
 // 16 experts of 1408, 50: 50 + 26 -> 52 + 21, 750: 172 + 107 -> 173 + 85; 8 of 1536, 40: 38 + 20 -> 31 + 12, 1024: 142 + 86 -> 131 + 58.
-// (the second launch bound: waves of a SIMD, with as many workgroups in a unit as its LDS holds, at most two)
-constexpr int ring_waves(int bm, int bn, int bk, int waves, int st) { return (st * (bm + bn) * bk * 2 <= 80 * 1024 ? 2 : 1) * waves / 4; }
-
-template <typename Tag, int BM, int BN, int BK, int WM, int WN, int ST, bool ONCE, int ACT>
-__global__ void __launch_bounds__(WM * WN * 64, ring_waves(BM, BN, BK, WM * WN, ST)) moe_grouped_ring_kernel(GroupedArgs p) {
+template <typename Tag, typename T, bool ONCE, int ACT>
+__global__ void __launch_bounds__(T::W * 64, T::kWaves) moe_grouped_ring_kernel(GroupedArgs p) {
   constexpr bool GLU = ACT >= 2;
-  constexpr int W = WM * WN, RB = BK * 2, RPL = 1024 / RB, CH = BK / 8;                 // a row's bytes, rows and 16-byte chunks a load
-  constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16, KK = BK / 32, OUT_N = GLU ? BN / 2 : BN;
-  constexpr int G = (BM + BN) / RPL, L = (G + W - 1) / W, kStage = (BM + BN) * RB, PER = FM * FN / L;
-  static_assert(BM % RPL == 0 && TM % 16 == 0 && TN % 16 == 0 && KK % 2 == 0 && ST * kStage <= 160 * 1024 && L * (ST - 1) <= 63, "tile");
+  constexpr int BM = T::BM, RB = T::RB, RPL = T::RPL, CH = T::CH, L = T::L, FM = T::FM, FN = T::FN, OUT_N = GLU ? T::BN / 2 : T::BN;
   extern __shared__ __attribute__((aligned(1024))) char ring_lds[];
   char* const lds = ring_lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
@@ -597,15 +587,15 @@ __global__ void __launch_bounds__(WM * WN * 64, ring_waves(BM, BN, BK, WM * WN, 
   int e = 0, row0 = 0, rows_end = 0, col = 0, row_tiles = 0;
   if (!grouped_tile_by_column(p.offsets, p.E, BM, ntiles, at, lane, e, row0, rows_end, col, row_tiles)) return;
   e = __builtin_amdgcn_readfirstlane(e);
-  const int n0 = col * OUT_N, wrows = GLU ? 2 * p.N : p.N, steps = p.K / BK;
-  const int wm = wave / WN, wn = wave % WN;
-  // this wave's direct loads: load i is the (i W + wave)-th of the tile's rows, x's first; lane -> row lane / CH of a load, chunk lane % CH
+  const int n0 = col * OUT_N, wrows = GLU ? 2 * p.N : p.N, steps = p.K / T::BK;
+  const int wm = wave / T::WN, wn = wave % T::WN;
+  // this wave's direct loads: lane -> row lane / CH of a load, chunk lane % CH
   uint32_t off[L];
   const char* base[L];
   const char* const we = p.w + (int64_t)e * wrows * p.K * 2;
 #pragma unroll
   for (int i = 0; i < L; ++i) {
-    const int g = min(i * W + wave, G - 1), r = g * RPL + lane / CH, chunk = (lane % CH) ^ (r & 7);
+    const int g = min(i * T::W + wave, T::G - 1), r = g * RPL + lane / CH, chunk = (lane % CH) ^ (r & 7);
     const bool is_x = g * RPL < BM;
     int64_t row;                                         // rows and columns past the end: the last one again, never stored
     if (is_x) {
@@ -620,75 +610,16 @@ __global__ void __launch_bounds__(WM * WN * 64, ring_waves(BM, BN, BK, WM * WN, 
     off[i] = (uint32_t)(row * (is_x ? p.a_stride : p.K) * 2) + chunk * 16;
     base[i] = is_x ? p.a : we;
   }
-  const uint32_t lds0 = lds_address(lds);
   f32x4_q acc[FM][FN];
 #pragma unroll
   for (int f = 0; f < FM; ++f)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[f][j] = f32x4_q{0.f, 0.f, 0.f, 0.f};
-  const int arow = (wm * TM + r16) * RB, brow = (BM + wn * TN + r16) * RB;
-  u32x4 xf[2][FM], wf[2][FN];
-  const auto read = [&](int buf, int kk) {
-    const int c = ((kk * 4 + q) ^ (r16 & 7)) * 16;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) wf[kk & 1][j] = ld16(lds + buf + brow + j * 16 * RB + c);
-#pragma unroll
-    for (int f = 0; f < FM; ++f) xf[kk & 1][f] = ld16(lds + buf + arow + f * 16 * RB + c);
-  };
-  const auto product = [&](auto past) {                    // past: the weights past the L2
-    const auto load = [&](int i, int s, int buf) {
-      ring_load<decltype(past)::value>(off[i], base[i] + (int64_t)s * RB, lds0 + buf + min(i * W + wave, G - 1) * 1024);
-    };
-    for (int s = 0; s < ST && s < steps; ++s)
-#pragma unroll
-      for (int i = 0; i < L; ++i) load(i, s, s * kStage);
-    ring_wait<L, ST - 1>(steps - 1);
-    ring_barrier();
-    read(0, 0);
-    int cur = 0;
-    const auto step = [&](int s, auto more) {               // more: there is a step ST ahead to load
-      constexpr bool MORE = decltype(more)::value;
-      const int next = cur == (ST - 1) * kStage ? 0 : cur + kStage;
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk) {
-        if (kk < KK - 1) {
-          read(cur, kk + 1);
-        } else if (MORE || s + 1 < steps) {
-          ring_wait<L, ST - 2>(MORE ? ST : steps - 2 - s);
-          ring_barrier();
-          if constexpr (MORE && PER < 2) {
-#pragma unroll
-            for (int i = 0; i < L; ++i) load(i, s + ST, cur);
-          }
-          read(next, 0);
-        }
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int n = 0; n < FN; ++n)
-#pragma unroll
-          for (int f = 0; f < FM; ++f) {
-            if constexpr (MORE && PER >= 2) {
-              if (kk == KK - 1 && (n * FM + f) % PER == 0 && (n * FM + f) / PER < L) {
-                __builtin_amdgcn_sched_barrier(0);
-                load((n * FM + f) / PER, s + ST, cur);
-                __builtin_amdgcn_sched_barrier(0);
-              }
-            }
-            acc[f][n] = mfma_q<Tag>(wf[kk & 1][n], xf[kk & 1][f], acc[f][n]);
-          }
-        __builtin_amdgcn_s_setprio(0);
-      }
-      cur = next;
-    };
-    int s = 0;
-    for (; s + ST < steps; ++s) step(s, std::true_type());
-    for (; s < steps; ++s) step(s, std::false_type());
-  };
-  if (ONCE && row_tiles == 1) product(std::integral_constant<bool, ONCE>());
-  else product(std::false_type());
+  if (ONCE && row_tiles == 1) ring_product<Tag, T, ONCE, 2>(acc, off, base, lds, steps, wave, lane);
+  else ring_product<Tag, T, 0, 2>(acc, off, base, lds, steps, wave, lane);
 #pragma unroll
   for (int f = 0; f < FM; ++f) {
-    const int pos = row0 + wm * TM + 16 * f + r16;
+    const int pos = row0 + wm * T::TM + 16 * f + r16;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
       float v[4];
@@ -697,48 +628,49 @@ __global__ void __launch_bounds__(WM * WN * 64, ring_waves(BM, BN, BK, WM * WN, 
         const auto both = __builtin_amdgcn_permlane32_swap(as_u32(acc[f][j][r]), as_u32(acc[f][j][r]), false, false);      // [1]: lanes 32-63 twice
         v[r] = grouped_act<Tag, ACT>(acc[f][j][r], GLU ? as_f32(both[1]) : 0.f, p);
       }
-      if (pos < rows_end && !(GLU && q >= 2)) store4<Tag>(p, pos, GLU ? n0 + wn * (TN / 2) + 8 * j + 4 * q : n0 + wn * TN + 16 * j + 4 * q, v);
+      if (pos < rows_end && !(GLU && q >= 2)) store4<Tag>(p, pos, GLU ? n0 + wn * (T::TN / 2) + 8 * j + 4 * q : n0 + wn * T::TN + 16 * j + 4 * q, v);
     }
   }
 }
 
-template <typename Tag, int BM, int BN, int BK, int WM, int WN, int ST, bool ONCE, int ACT>
+template <typename Tag, typename T, bool ONCE, int ACT>
 int launch_grouped_ring(const GroupedArgs& p, int pairs, int held, hipStream_t st) {
-  constexpr int lds = ST * (BM + BN) * BK * 2, per = ACT >= 2 ? BN / 2 : BN;
+  constexpr int per = ACT >= 2 ? T::BN / 2 : T::BN;
   static PerDevice<int> raised;
   int ok = 0;
   raised.get(ok, [&](int) {
-    return hipFuncSetAttribute((const void*)moe_grouped_ring_kernel<Tag, BM, BN, BK, WM, WN, ST, ONCE, ACT>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess ? 1 : 0;
+    return hipFuncSetAttribute((const void*)moe_grouped_ring_kernel<Tag, T, ONCE, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize, T::kLds) ==
+                   hipSuccess ? 1 : 0;
   });
   if (!ok) return SP_ERR_LAUNCH;
   const int64_t ntiles = (p.N + per - 1) / per;
-  const unsigned blocks = (unsigned)(((pairs / BM + held) * ntiles + 7) / 8 * 8);
-  moe_grouped_ring_kernel<Tag, BM, BN, BK, WM, WN, ST, ONCE, ACT><<<dim3(blocks), dim3(WM * WN * 64), lds, st>>>(p);
+  const unsigned blocks = (unsigned)(((pairs / T::BM + held) * ntiles + 7) / 8 * 8);
+  moe_grouped_ring_kernel<Tag, T, ONCE, ACT><<<dim3(blocks), dim3(T::W * 64), T::kLds, st>>>(p);
   SP_LAUNCH_CHECK();
   return SP_OK;
 }
 
 // The tiles, and what one costs: us per step of BK where two workgroups share a unit and where one has it alone, and us besides.
 #define SP_RING_TILES(F)                                        \
-  F(0, 0.856f, 0.454f, 1.53f, 32, 128, 64, 1, 4, 4, true)       \
-  F(1, 0.787f, 0.389f, 2.88f, 32, 64, 128, 1, 4, 3, true)       \
-  F(2, 1.127f, 0.490f, 2.10f, 64, 128, 64, 2, 2, 3, true)       \
-  F(3, 0.636f, 0.129f, 4.05f, 64, 128, 64, 1, 4, 3, false)      \
-  F(4, 0.753f, 0.295f, 4.33f, 80, 128, 64, 1, 4, 3, false)      \
-  F(5, 0.423f, 0.118f, 3.98f, 96, 64, 64, 2, 2, 4, false)       \
-  F(6, 1.102f, 0.533f, 4.92f, 128, 128, 64, 2, 4, 2, false)     \
-  F(7, 1.269f, 0.664f, 5.16f, 160, 128, 64, 2, 2, 2, false)     \
-  F(8, 1.432f, 0.658f, 5.84f, 192, 128, 64, 4, 2, 2, false)     \
-  F(9, 3.326f, 1.018f, 5.36f, 192, 192, 64, 2, 4, 3, false)
+  F(0, 0.856f, 0.454f, 1.53f, true, 32, 128, 64, 1, 4, 4)       \
+  F(1, 0.787f, 0.389f, 2.88f, true, 32, 64, 128, 1, 4, 3)       \
+  F(2, 1.127f, 0.490f, 2.10f, true, 64, 128, 64, 2, 2, 3)       \
+  F(3, 0.636f, 0.129f, 4.05f, false, 64, 128, 64, 1, 4, 3)      \
+  F(4, 0.753f, 0.295f, 4.33f, false, 80, 128, 64, 1, 4, 3)      \
+  F(5, 0.423f, 0.118f, 3.98f, false, 96, 64, 64, 2, 2, 4)       \
+  F(6, 1.102f, 0.533f, 4.92f, false, 128, 128, 64, 2, 4, 2)     \
+  F(7, 1.269f, 0.664f, 5.16f, false, 160, 128, 64, 2, 2, 2)     \
+  F(8, 1.432f, 0.658f, 5.84f, false, 192, 128, 64, 4, 2, 2)     \
+  F(9, 3.326f, 1.018f, 5.36f, false, 192, 192, 64, 2, 4, 3)
 
-struct RingTile {
+struct RingCost {
   float two, one, fixed;
   int bm, bn, bk, lds;
   bool once;
 };
-#define SP_RING_ROW(I, TWO, ONE, FIXED, BM, BN, BK, WM, WN, ST, ONCE) {TWO, ONE, FIXED, BM, BN, BK, ST * (BM + BN) * BK * 2, ONCE},
-constexpr RingTile kRingTiles[] = {SP_RING_TILES(SP_RING_ROW)};
+#define SP_RING_ROW(I, TWO, ONE, FIXED, ONCE, ...) \
+  {TWO, ONE, FIXED, RingTile<__VA_ARGS__>::BM, RingTile<__VA_ARGS__>::BN, RingTile<__VA_ARGS__>::BK, RingTile<__VA_ARGS__>::kLds, ONCE},
+constexpr RingCost kRingTiles[] = {SP_RING_TILES(SP_RING_ROW)};
 
 // Expected row tiles of one expert of `experts`, each pair choosing each of them alike
 inline double ring_row_tiles(int pairs, int experts, int bm) {
@@ -752,7 +684,7 @@ inline double ring_row_tiles(int pairs, int experts, int bm) {
 // weights' way from memory, the two lesser ones added softly.  The last, not full round of tiles counts by the chance that it is there and that
 // some unit holds two of it.  Measured: 20 tiles, 58 products (widths 1024 and 2048, 8 to 128 experts, 8 to 4096 rows): 11 % rms from this, and the tile
 // chosen by it 3 % behind the best of the 20 on average.
-inline double ring_us(const RingTile& t, int pairs, int experts, int64_t wrows, int K) {
+inline double ring_us(const RingCost& t, int pairs, int experts, int64_t wrows, int K) {
   const double cols = (double)((wrows + t.bn - 1) / t.bn), tiles = experts * ring_row_tiles(pairs, experts, t.bm) * cols, steps = K / t.bk;
   const bool pair = t.lds <= 80 * 1024;
   const double slots = pair ? 512. : 256., one = t.fixed + steps * t.one, two = t.fixed + steps * t.two;
@@ -917,7 +849,8 @@ int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
     return SP_OK;
   }
   if (ring) {
-#define SP_RING_CASE(I, TWO, ONE, FIXED, ...) case I: return launch_grouped_ring<Tag, __VA_ARGS__, ACT>(p, pairs, held, st);
+#define SP_RING_CASE(I, TWO, ONE, FIXED, ONCE, ...) \
+  case I: return launch_grouped_ring<Tag, RingTile<__VA_ARGS__>, ONCE, ACT>(p, pairs, held, st);
     switch (ring_tile(pairs, p.E, (ACT >= 2 ? 2 : 1) * (int64_t)p.N, p.K)) { SP_RING_TILES(SP_RING_CASE) }
     return SP_ERR_INVALID_ARG;
   }

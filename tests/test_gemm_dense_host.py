@@ -5,8 +5,8 @@ import pytest
 def test_plans_fit_their_products():
     from scratchpad_amd import _native
     lib = _native.load()
-    steps = [256, 128, 256, 256, 256, 256, 128, 256, 256, 128, 64, 256, 128, 128, 64, 64, 64, 64, 64]
-    for M in (5, 16, 17, 31, 32, 33, 64, 65, 100, 128, 192, 255, 256, 640):
+    steps = [256, 128, 256, 256, 256, 128, 256, 128, 64, 256, 128, 128, 64, 64] + [64] * 7
+    for M in (5, 16, 17, 31, 32, 33, 64, 65, 100, 128, 192, 255, 256, 640, 1024):
         for N in (1024, 1032, 1536, 3072, 8448, 16384, 128256):
             for K in (64, 192, 512, 1024, 2048, 3584, 8192, 14336):
                 for epilogue in (0, 1):
@@ -14,7 +14,7 @@ def test_plans_fit_their_products():
                     tile, splits = plan & 255, plan >> 8
                     if epilogue and plan < 0:          # the plain product has shares, or no tile with its order of sums takes pairs
                         continue
-                    assert plan >= 0 and tile < len(steps) and splits in (1, 2, 4, 8)
+                    assert plan >= 0 and tile < len(steps) and splits in (1, 2, 3, 4, 6, 8)
                     assert K % steps[tile] == 0 and K // steps[tile] >= (3 * splits if splits > 1 else 1)
                     assert splits == 1 or epilogue == 0
     for bad in ((0, 1024, 1024, 0), (64, 1024, 1000, 0), (64, 1024, 1024, 2), (64, -1, 64, 0)):
@@ -22,7 +22,7 @@ def test_plans_fit_their_products():
 
 
 @pytest.mark.parametrize("M, N, K, takes", [(4, 28672, 4096, False), (5, 28672, 4096, True), (16, 2048, 4096, False), (16, 4096, 4096, True), (17, 4096, 4096, True), (256, 4096, 4096, True), (257, 4096, 4096, False),
-                                            (640, 4096, 14336, True), (641, 4096, 14336, False), (64, 512, 4096, False), (64, 1024, 1000, False),
+                                            (640, 4096, 14336, True), (1024, 4096, 14336, True), (1025, 4096, 14336, False), (512, 7168, 14336, True), (513, 7168, 14336, False), (640, 2048, 4608, False), (144, 3072, 2048, False), (192, 3072, 2048, True), (209, 3072, 2048, False), (256, 4096, 3072, True), (64, 512, 4096, False), (64, 1024, 1000, False),
                                             (64, 2048, 4096, True), (65, 2048, 4096, False), (17, 520, 2048, True), (300, 1024, 8192, False), (95, 128256, 2048, True), (96, 128256, 2048, False),
                                             (256, 128256, 4096, True)])
 def test_where_it_pays(M, N, K, takes):

@@ -6,9 +6,9 @@ import torch
 
 pytestmark = pytest.mark.gpu
 # rows, columns and k-step of a tile, in the order of its number
-TILES = [(16, 64, 256), (16, 128, 128), (32, 16, 256), (32, 32, 256), (32, 32, 256), (32, 64, 256), (32, 128, 128), (48, 32, 256), (64, 16, 256),
-         (64, 32, 128), (64, 64, 64), (64, 64, 256), (64, 128, 128), (96, 64, 128), (96, 128, 64), (128, 96, 64), (128, 128, 64),
-         (192, 128, 64), (256, 128, 64)]
+TILES = [(16, 64, 256), (16, 128, 128), (32, 16, 256), (32, 32, 256), (32, 64, 256), (32, 128, 128), (48, 32, 256), (64, 32, 128),
+         (64, 64, 64), (64, 64, 256), (64, 128, 128), (96, 64, 128), (96, 128, 64), (128, 96, 64),
+         (128, 64, 64), (128, 128, 64), (192, 128, 64), (256, 128, 64), (256, 96, 64), (160, 256, 64), (192, 192, 64)]
 
 
 def check(got, x, w, dtype):
@@ -36,7 +36,7 @@ def test_tiles_at_their_edges(tile, dtype):
     bm, bn, bk = TILES[tile]
     g = torch.Generator().manual_seed(tile)
     for M, N, steps, splits in [(1, 1, 1, 1), (bm - 1, bn + 1, 2, 2), (bm, bn, 3, 1), (bm + 1, 2 * bn - 2, 5, 4), (2 * bm + 17, 3 * bn - 4, 17, 8),
-                                (17, 4 * bn, 24, 1)]:
+                                (17, 4 * bn, 24, 1), (5 * bm + 3, 2 * bn + 4, 7, 3), (4 * bm, bn - 1, 20, 6)]:
         K = bk * steps
         x = torch.randn(M, K, generator=g).to(dtype).cuda()
         w = (torch.randn(N, K, generator=g) * 0.05).to(dtype).cuda()
@@ -70,7 +70,7 @@ def test_silu_epilogue_is_the_product_then_the_activation(dtype):
 def test_linear_takes_it_and_leaves_the_rest():
     from scratchpad_amd import _native
     g = torch.Generator().manual_seed(5)
-    for M, N, K in [(5, 6144, 2048), (16, 4096, 2560), (17, 1024, 1024), (61, 3072, 2048), (100, 2048, 8192), (256, 4096, 1024), (500, 2048, 6144)]:
+    for M, N, K in [(5, 6144, 2048), (16, 4096, 2560), (17, 1024, 1024), (61, 3072, 2048), (100, 2048, 8192), (256, 4096, 1024), (500, 2048, 6144), (777, 2048, 8192)]:
         assert _native.dense_gemm_pays(M, N, K)
         x = torch.randn(M, K, generator=g).bfloat16().cuda()
         w = (torch.randn(N, K, generator=g) * 0.05).bfloat16().cuda()
@@ -89,7 +89,7 @@ def test_linear_takes_it_and_leaves_the_rest():
     x = torch.randn(3, 61, 1024, generator=g).bfloat16().cuda()
     assert torch.func.vmap(lambda t: _native.linear(t, w))(x).shape == (3, 61, 1024)
     assert _native.linear(x, w).shape == (3, 61, 1024)
-    rc, _ = dense(x[0], w, 0 + 256 * 3)
+    rc, _ = dense(x[0], w, 0 + 256 * 5)
     assert rc == -1
     rc, _ = dense(x[0][:, :192], w[:, :192], 0 + 256)                                         # K is no multiple of the tile's step
     assert rc == -2
