@@ -865,9 +865,13 @@ _DENSE_PLANS = {}             # (M, weight rows, K, epilogue) -> _dense_plan: si
 def dense_gemm_pays(M: int, N: int, K: int) -> bool:
     """Where sp_gemm_dense measured faster than hipBLASLt on MI355X (us under graph replay, cold weights, library / own): 17 - 256
     rows of most shapes (the table in gemm_dense.hip).  Past that the library's large tiles win (320 rows: 28672 x 4096 81 / 84, 3072 x 2048
-    11.2 / 13.8; 1024: 28672 x 4096 169 / 208, 4096 x 4096 39 / 38) but where K is long and twice N, where it runs few of them:
+    11.2 / 13.8; 1024: 28672 x 4096 169 / 208) but
+    where K is long and twice N, where it runs few of them:
     2048 x 8192 33 / 26 at 320 rows, 45 / 36 at 640 and 50 / 45 at 1024, 4096 x 14336 76 / 52, 111 / 78 and 134 / 118, 4096 x 8192 47 / 38, 64 / 54 and
-    74 / 75, 8192 x 28672 226 / 164 and 262 / 267 (2048 x 4608 24.3 / 24.8 at 640; 1024 x 8192 22.6 / 24.2 at 512).
+    74 / 75, 8192 x 28672 226 / 164 and 262 / 267 (2048 x 4608 24.3 / 24.8 at 640; 1024 x 8192 22.6 / 24.2 at 512); and where 128-row tiles
+    nearly fill the units once, K to 4096 (between two other kernels, 777 / 900 / 1024 rows: 2048 x 2048 18.0 / 16.2, 18.0 / 16.7, 19.0 / 17.5, 3072 x 2048
+    21.6 / 20.8, 21.5 / 21.4, 23.0 / 22.2, 4096 x 4096 41.7 / 38.6, 43.4 / 41.1, 46.1 / 42.2, 3072 x 3072 30.5 / 27.0, 26.9 / 28.4, 29.3 / 28.8; with fewer
+    tiles 2560 x 2560 23.2 / 24.0, 24.0 / 23.5, 23.8 / 24.3; 700 rows 4096 x 4096 37.3 / 38.6).
     Left to the library below 257: up to 512 weight rows, where it depends on K and rows (512 x 2048 5.5 / 6.7, 512 x 4096 11.7 / 7.1 at 64
     rows); up to 2048 of them at K 2560 - 4096 past 64 rows (2048 x 4096 11.1 / 10.3 at 64 rows, 10.6 / 11.2 at 128, 1024 x 4096 12.2 / 8.0
     and 9.4 / 9.6, 1536 x 4096 9.4 / 10.2 at 96); 2049 to 4096 at K 1536 - 3072 and 10 M elements, where its tiles fit the rows (3072 x 2048 at 144:
@@ -883,6 +887,8 @@ def dense_gemm_pays(M: int, N: int, K: int) -> bool:
     if M <= SKINNY_MAX_ROWS:
         return M > 4 and N * K > 1 << 23 and (M > 8 or N > 4096 or K > 4096)
     if M > DENSE_MAX_ROWS:
+        if 768 < M <= 1024 and 1024 <= K <= 4096 and N <= 4096:
+            return 160 < -(-M // 128) * -(-N // (64 if N <= 2048 else 128)) <= 256
         return N >= 2048 and K >= 2 * N and K > 5120 and M <= (1024 if N <= 6144 else 512)
     if N <= 2048 and (N <= 512 or (2048 < K <= 4096 and M > 64)):
         return False

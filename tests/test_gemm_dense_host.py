@@ -22,7 +22,7 @@ def test_plans_fit_their_products():
 
 
 @pytest.mark.parametrize("M, N, K, takes", [(4, 28672, 4096, False), (5, 28672, 4096, True), (16, 2048, 4096, False), (16, 4096, 4096, True), (17, 4096, 4096, True), (256, 4096, 4096, True), (257, 4096, 4096, False),
-                                            (640, 4096, 14336, True), (1024, 4096, 14336, True), (1025, 4096, 14336, False), (512, 7168, 14336, True), (513, 7168, 14336, False), (640, 2048, 4608, False), (144, 3072, 2048, False), (192, 3072, 2048, True), (209, 3072, 2048, False), (256, 4096, 3072, True), (64, 512, 4096, False), (64, 1024, 1000, False),
+                                            (640, 4096, 14336, True), (1024, 4096, 14336, True), (1025, 4096, 14336, False), (512, 7168, 14336, True), (513, 7168, 14336, False), (640, 2048, 4608, False), (144, 3072, 2048, False), (192, 3072, 2048, True), (209, 3072, 2048, False), (256, 4096, 3072, True), (768, 2048, 2048, False), (769, 2048, 2048, True), (1024, 4096, 4096, True), (1025, 2048, 2048, False), (777, 2560, 2560, False), (777, 1024, 2048, False), (777, 2048, 4160, False), (64, 512, 4096, False), (64, 1024, 1000, False),
                                             (64, 2048, 4096, True), (65, 2048, 4096, False), (17, 520, 2048, True), (300, 1024, 8192, False), (95, 128256, 2048, True), (96, 128256, 2048, False),
                                             (256, 128256, 4096, True)])
 def test_where_it_pays(M, N, K, takes):

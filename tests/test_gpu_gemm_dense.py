@@ -70,7 +70,7 @@ def test_silu_epilogue_is_the_product_then_the_activation(dtype):
 def test_linear_takes_it_and_leaves_the_rest():
     from scratchpad_amd import _native
     g = torch.Generator().manual_seed(5)
-    for M, N, K in [(5, 6144, 2048), (16, 4096, 2560), (17, 1024, 1024), (61, 3072, 2048), (100, 2048, 8192), (256, 4096, 1024), (500, 2048, 6144), (777, 2048, 8192)]:
+    for M, N, K in [(5, 6144, 2048), (16, 4096, 2560), (17, 1024, 1024), (61, 3072, 2048), (100, 2048, 8192), (256, 4096, 1024), (500, 2048, 6144), (777, 2048, 8192), (1001, 2048, 1024)]:
         assert _native.dense_gemm_pays(M, N, K)
         x = torch.randn(M, K, generator=g).bfloat16().cuda()
         w = (torch.randn(N, K, generator=g) * 0.05).bfloat16().cuda()
