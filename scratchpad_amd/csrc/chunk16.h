@@ -274,7 +274,7 @@ __global__ void __launch_bounds__(NW * 96) chunk16_walk_kernel(Walk16 a, SeqBatc
 #pragma unroll
         for (int x = 0; x < 8; x += E::kVec) unpack16<Tag>(ld16(rows + x * E::kBytes), g + x);
 #pragma unroll
-        for (int x = 0; x < 8; ++x) f[x] /= 1.f + expf(-g[x]);
+        for (int x = 0; x < 8; ++x) f[x] = over_one_plus_exp(f[x], g[x]);
       }
       if (t >= len - c * kC16) return;
       char* to = (char*)a.out + ((start + c * kC16 + t) * a.out_stride + (int64_t)h * Dv + at) * E::kBytes;

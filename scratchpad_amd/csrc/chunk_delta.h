@@ -140,10 +140,10 @@ __global__ void __launch_bounds__(D * 2) delta_chunk_prepare_kernel(DeltaChunks 
     float beta = 0.f, dec = 1.f;
     if (tid < n) {
       if constexpr (CHANNEL) {
-        beta = 1.f / (1.f + expf(-E::load(a.bpre, (row0 + tid) * a.b_stride + h)));
+        beta = over_one_plus_exp(1.f, E::load(a.bpre, (row0 + tid) * a.b_stride + h));
       } else {
         const float* pre = a.pre + (row0 + tid) * a.pre_stride;
-        beta = 1.f / (1.f + expf(-pre[h]));
+        beta = over_one_plus_exp(1.f, pre[h]);
         dec = expf(-expf(a.A_log[h]) * softplus_dc(pre[a.H + h] + a.dt_bias[h]));
       }
     }

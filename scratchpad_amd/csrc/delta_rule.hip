@@ -64,8 +64,8 @@ delta_gates_kernel(float* decay, float* remove, const void* p, int64_t p_stride,
   for (int tt = 0; tt < TPB; ++tt) {
     const int64_t t = t0 + tt;
     if (t < T) {
-      decay[t * channels + c] = expf(-rate / (1.f + expf(-(acc[tt] + bias))));
-      remove[t * channels + c] = 1.f / (1.f + expf(-(E::load(apre, t * a_stride + c) + ab)));
+      decay[t * channels + c] = expf(-over_one_plus_exp(rate, acc[tt] + bias));
+      remove[t * channels + c] = over_one_plus_exp(1.f, E::load(apre, t * a_stride + c) + ab);
     }
   }
 }
@@ -238,7 +238,7 @@ delta_recurrence_kernel(void* out, int64_t out_stride, const void* r, int64_t r_
       for (int u = 0; u < PERG; ++u) {
         const int tt = part + u * SP;
         if (tt < n)
-          E::store(out, (start + c0 + tt) * out_stride + hc + col, so[tt][col] * sinv[tt] * nw / (1.f + expf(-gate[u])));
+          E::store(out, (start + c0 + tt) * out_stride + hc + col, over_one_plus_exp(so[tt][col] * sinv[tt] * nw, gate[u]));
       }
     }
   }
@@ -292,9 +292,9 @@ delta_step_kernel(void* out, int64_t out_stride, const void* r, int64_t r_stride
   };
   if (part == 0) {
     const float u = kf / sqrtf(k2 + 1e-6f);
-    sw[col] = expf(-rate / (1.f + expf(-(over_parts() + bias))));
+    sw[col] = expf(-over_one_plus_exp(rate, over_parts() + bias));
     su[col] = u;
-    sau[col] = u / (1.f + expf(-af));
+    sau[col] = over_one_plus_exp(u, af);
     sk[col] = kf;
     sr[col] = rf;
   }
@@ -318,7 +318,7 @@ delta_step_kernel(void* out, int64_t out_stride, const void* r, int64_t r_stride
   __syncthreads();
   const float o = over_parts();
   const float ss = block_sum(part == 0 ? o * o : 0.f, red);
-  if (part == 0) E::store(out, b * out_stride + hc + col, o / sqrtf(ss / (float)K + eps) * nw / (1.f + expf(-gf)));
+  if (part == 0) E::store(out, b * out_stride + hc + col, over_one_plus_exp(o / sqrtf(ss / (float)K + eps) * nw, gf));
 }
 
 template <typename Tag>

@@ -48,7 +48,7 @@ __device__ __forceinline__ float softplus_gd(float z) { return fmaxf(z, 0.f) + l
 // place of log1p has lost e^z's low bits there, all of them from z = -17 down)
 template <int ACT>
 __device__ __forceinline__ float gate_value(float z, float rate) {
-  return ACT == 0 ? expf(-rate * softplus_gd(z)) : 1.f / (1.f + expf(-z));
+  return ACT == 0 ? expf(-rate * softplus_gd(z)) : over_one_plus_exp(1.f, z);
 }
 
 template <typename Tag, int TPB, int ACT>
@@ -210,7 +210,7 @@ gated_delta_scan_kernel(void* out, int64_t out_stride, const void* q, int64_t q_
       const int tt = e / Dv, i = e % Dv;
       sv[tt][i] = E::load(v, (start + c0 + tt) * v_stride + vc + i);
     }
-    if (j < n) sbeta[j] = 1.f / (1.f + expf(-E::load(bpre, (start + c0 + j) * b_stride + h)));
+    if (j < n) sbeta[j] = over_one_plus_exp(1.f, E::load(bpre, (start + c0 + j) * b_stride + h));
     __syncthreads();
     // unit query and key of every token of the pass, and the decayed key: a wave per token
     for (int tt = wave; tt < n; tt += waves) {

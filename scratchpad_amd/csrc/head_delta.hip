@@ -152,7 +152,7 @@ head_delta_kernel(HeadDelta a, SeqBatch s) {
     for (int x = 0; x < V; x += 4) st16(sv + e * V + x, pack16<f32_tag>(v_ + x));
   };
   auto put_gates = [&](float b_, float a_) {
-    sbeta[j] = 1.f / (1.f + expf(-b_));
+    sbeta[j] = over_one_plus_exp(1.f, b_);
     sg[j] = expf(-rate * softplus_hd(a_ + bias));
   };
   auto fetch = [&](int64_t t0) {
@@ -321,7 +321,7 @@ head_delta_kernel(HeadDelta a, SeqBatch s) {
       const int tt = e / Dv, i = e % Dv;
       const int64_t row = start + t0 + tt;
       const float z = E::load(a.gate, row * a.gate_stride + vc + i);
-      E::store(a.out, row * a.out_stride + vc + i, so[tt * cols + i] * sinv[tt] * a.norm_w[i] * (z / (1.f + expf(-z))));
+      E::store(a.out, row * a.out_stride + vc + i, so[tt * cols + i] * sinv[tt] * a.norm_w[i] * over_one_plus_exp(z, z));
     }
   }
 #pragma unroll
@@ -359,7 +359,7 @@ __global__ void __launch_bounds__(kBlock) head_norm_gate_kernel(HeadDelta a, int
     const int i = lane + 64 * u;
     if (i < Dv) {
       const float z = E::load(a.gate, t * a.gate_stride + h * Dv + i);
-      E::store(a.out, t * a.out_stride + h * Dv + i, f[u] * inv * a.norm_w[i] * (z / (1.f + expf(-z))));
+      E::store(a.out, t * a.out_stride + h * Dv + i, f[u] * inv * a.norm_w[i] * over_one_plus_exp(z, z));
     }
   }
 }

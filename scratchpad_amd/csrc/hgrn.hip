@@ -92,8 +92,8 @@ hgrn2_scan_kernel(void* out, int64_t out_stride, const void* qpre, int64_t q_str
       if (e < kChunk * DP) {
         const int at = i + 4 * (i / DS);
         const bool ok = i < D;                           // register rows past D: f = 0 and q = 0, never stored
-        sq[tt][at] = ok ? fq[u] / (1.f + expf(-fq[u])) : 0.f;
-        sf[tt][at] = ok ? flo[u] + (1.f - flo[u]) / (1.f + expf(-(ff[u] + fbi[u]))) : 0.f;
+        sq[tt][at] = ok ? over_one_plus_exp(fq[u], fq[u]) : 0.f;
+        sf[tt][at] = ok ? flo[u] + over_one_plus_exp(1.f - flo[u], ff[u] + fbi[u]) : 0.f;
       }
     }
     if (live) {
@@ -212,8 +212,8 @@ hgrn2_prepare_kernel(float* work, const char* qpre, int64_t q_stride, const char
       unpack16<Tag>(t < n ? ld16(fpre + ((row0 + t) * f_stride + c) * E::kBytes) : zero, f);
 #pragma unroll
       for (int x = 0; x < V; ++x) {
-        const float lo = lower[c + x], w = t < n ? lo + (1.f - lo) / (1.f + expf(-(f[x] + f_bias[c + x]))) : 1.f;
-        sr[t][i + x] = q[x] / (1.f + expf(-q[x]));
+        const float lo = lower[c + x], w = t < n ? lo + over_one_plus_exp(1.f - lo, f[x] + f_bias[c + x]) : 1.f;
+        sr[t][i + x] = over_one_plus_exp(q[x], q[x]);
         sw[t][i + x] = w;
         sk[t][i + x] = 1.f - w;
       }

@@ -611,7 +611,7 @@ __device__ __forceinline__ void head_linear_store(const f32x4_l (&acc)[NT], void
         const u32x2 g2 = *(const u32x2*)((const char*)gate + (t * gate_stride + h * N + n) * 2);
         unpack16<Tag>(u32x4{g2[0], g2[1], 0u, 0u}, g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f[e] /= 1.f + expf(-g[e]);
+        for (int e = 0; e < 4; ++e) f[e] = over_one_plus_exp(f[e], g[e]);
       }
       const u32x4 pk = pack16<Tag>(f);
       char* to = (char*)out + (t * out_stride + h * out_head + n) * 2;
@@ -741,7 +741,7 @@ head_linear_kernel(void* out, int64_t out_stride, int64_t out_head, const void* 
     const int64_t row = (h * N + n) * (int64_t)K;
     float acc = 0.f;
     for (int k = 0; k < K; ++k) acc += smem[k] * E::load(w, row + k);
-    if (gate) acc /= 1.f + expf(-E::load(gate, t * gate_stride + h * N + n));
+    if (gate) acc = over_one_plus_exp(acc, E::load(gate, t * gate_stride + h * N + n));
     E::store(out, t * out_stride + h * out_head + n, acc);
   }
 }

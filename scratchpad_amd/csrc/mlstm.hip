@@ -132,7 +132,7 @@ mlstm_scan_kernel(void* out, int64_t out_stride, const void* q, int64_t q_stride
         const int tt = part + u * SP;
         if (tt < n)
           E::store(out, (start + c0 + tt) * out_stride + colv + col,
-                   so[tt * (Dv + 1) + col] * sden[tt] * sinv[tt] * nw / (1.f + expf(-gv[u])));
+                   over_one_plus_exp(so[tt * (Dv + 1) + col] * sden[tt] * sinv[tt] * nw, gv[u]));
       }
     }
   }
@@ -338,7 +338,7 @@ mlstm_chunk_kernel(void* out, int64_t out_stride, const char* q, int64_t q_strid
         const float gate = bf16_bits_to_f32(gv[i][r]), f = __shfl(factor, t, 64);
         if (t < n)
           E::store(ob + c0 * out_stride * 2 + (uint32_t)(t * (uint32_t)out_stride + col) * 2u, 0,
-                   c.o[i][r] * f * nw / (1.f + expf(-gate)));
+                   over_one_plus_exp(c.o[i][r] * f * nw, gate));
       }
   }
   if constexpr (MODE == kSegmentSums) {

@@ -351,7 +351,7 @@ template <typename Tag>
 __device__ __forceinline__ float moe_glu_value(float g, float u, float limit, float alpha) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return mul_round<Tag>(g / (1.f + expf(-alpha * g)), u + 1.f);
+  return mul_round<Tag>(over_one_plus_exp(g, alpha * g), u + 1.f);
 }
 
 template <typename Tag, int ACT>

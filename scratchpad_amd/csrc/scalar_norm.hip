@@ -125,7 +125,7 @@ __global__ void gate_heads_kernel(void* out, const void* o, const void* g, int64
     const int d = (int)(i % D);
     const int h = (int)((i / D) % H);
     const int64_t t = i / ((int64_t)D * H);
-    const float gate = 1.f / (1.f + expf(-E::load(g, t * g_stride + h)));
+    const float gate = over_one_plus_exp(1.f, E::load(g, t * g_stride + h));
     E::store(out, i, E::load(o, ((int64_t)h * T + t) * D + d) * gate);
   }
 }

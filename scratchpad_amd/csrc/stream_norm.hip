@@ -142,7 +142,7 @@ gated_add_norm_kernel(float* x, int64_t x_stride, const void* a, int64_t a_strid
   for (int i = threadIdx.x; i < width; i += blockDim.x) {
     float y = E::load(a, t * a_stride + i);
     if (b) y = 0.5f * (y * ia * wa[i] + E::load(b, t * b_stride + i) * ib * wb[i]);
-    if (gate) y /= 1.f + expf(-(E::load(gate, t * gate_stride + i) + (gate_bias ? gate_bias[i] : 0.f)));
+    if (gate) y = over_one_plus_exp(y, E::load(gate, t * gate_stride + i) + (gate_bias ? gate_bias[i] : 0.f));
     rowbuf[i] = y;
     ss += y * y;
   }
@@ -255,7 +255,7 @@ gated_add_norm_vec_kernel(float* x, int64_t x_stride, const void* a, int64_t a_s
         float gb[4] = {0.f, 0.f, 0.f, 0.f};
         if (gate_bias) row4(gate_bias, (int64_t)vi * V + 4 * q, gb);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ya[u][4 * q + e] /= 1.f + expf(-(yg[u][4 * q + e] + gb[e]));
+        for (int e = 0; e < 4; ++e) ya[u][4 * q + e] = over_one_plus_exp(ya[u][4 * q + e], yg[u][4 * q + e] + gb[e]);
       }
     }
 #pragma unroll

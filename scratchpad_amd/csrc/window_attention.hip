@@ -534,7 +534,7 @@ window_attention_kernel(void* out, int64_t out_stride, const void* q, int64_t q_
       if (softcap > 0.f) sc = softcap * tanhf(sc / softcap);
     }
     if constexpr (SIG) {                                // every visible key on its own: no maximum, no denominator
-      sw[lane] = lane < n ? 1.f / (1.f + expf(-(sc + hbias))) : 0.f;
+      sw[lane] = lane < n ? over_one_plus_exp(1.f, sc + hbias) : 0.f;
       __builtin_amdgcn_wave_barrier();
     } else {
       float tm = sc;
@@ -591,7 +591,7 @@ window_attention_kernel(void* out, int64_t out_stride, const void* q, int64_t q_
     for (int c = threadIdx.x; c < Dv; c += blockDim.x) {
       float num = 0.f;
       for (int w = 0; w < NW; ++w) num += sacc[w * Dv + c];
-      if (gate) num /= 1.f + expf(-E::load(gate, t * gate_stride + (int64_t)h * Dv + c));
+      if (gate) num = over_one_plus_exp(num, E::load(gate, t * gate_stride + (int64_t)h * Dv + c));
       E::store(out, t * out_stride + (int64_t)h * Dv + c, num);
     }
     return;
@@ -609,7 +609,7 @@ window_attention_kernel(void* out, int64_t out_stride, const void* q, int64_t q_
     float num = 0.f;
     for (int w = 0; w < NW; ++w) num += sacc[w * Dv + c] * expf(sml[w] - M);
     num *= inv;
-    if (gate) num /= 1.f + expf(-E::load(gate, t * gate_stride + (int64_t)h * Dv + c));
+    if (gate) num = over_one_plus_exp(num, E::load(gate, t * gate_stride + (int64_t)h * Dv + c));
     E::store(out, t * out_stride + (int64_t)h * Dv + c, num);
   }
 }
@@ -804,7 +804,7 @@ window_attention_mfma_kernel(void* out, int64_t out_stride, const void* q, int64
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const float v = plain ? sacc[sb][r] * scale : sacc[sb][r];
-              pf[sb >> 1][4 * (sb & 1) + r] = v == -INFINITY ? 0.f : 1.f / (1.f + expf(-(v + hbias)));
+              pf[sb >> 1][4 * (sb & 1) + r] = v == -INFINITY ? 0.f : over_one_plus_exp(1.f, v + hbias);
             }
         } else {
           float mx = fmaxf(fmaxf(sacc[0][0], sacc[0][1]), fmaxf(sacc[0][2], sacc[0][3]));
@@ -894,7 +894,7 @@ window_attention_mfma_kernel(void* out, int64_t out_stride, const void* q, int64
           const u32x2 g2 = *(const u32x2*)((const char*)gate + ((t0 + r16) * gate_stride + (int64_t)hq * Dv + 16 * dt + 4 * qd) * 2);
           unpack16<Tag>(u32x4{g2[0], g2[1], 0u, 0u}, gf);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) f[e] /= 1.f + expf(-gf[e]);
+          for (int e = 0; e < 4; ++e) f[e] = over_one_plus_exp(f[e], gf[e]);
         }
         const u32x4 pk = pack16<Tag>(f);
         *(u32x2*)((char*)out + ((t0 + r16) * out_stride + (int64_t)hq * Dv + 16 * dt + 4 * qd) * 2) = u32x2{pk[0], pk[1]};

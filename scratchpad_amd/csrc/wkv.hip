@@ -103,7 +103,7 @@ wkv_recurrence_kernel(void* out, const void* r, const void* k, const void* v, co
       const int64_t row = start + c0 + tt;
       for (int i = lane; i < K; i += 64) {
         const float gv = E::load(g, row * gs + col + i);
-        const float gate = gv / (1.f + expf(-gv));
+        const float gate = over_one_plus_exp(gv, gv);
         E::store(out, row * os + col + i, so[tt][i] * inv * norm_w[col + i] * gate);
       }
     }
