@@ -175,25 +175,43 @@ conv_silu_kernel(void* out, int64_t out_stride, const void* in, int64_t in_strid
     }
     acc += w[(int64_t)c * taps + j] * val;
   }
-  E::store(out, t * out_stride + c, acc / (1.f + expf(-acc)));
+  E::store(out, t * out_stride + c, over_one_plus_exp(acc, acc));
 }
 
 constexpr int kMaxTaps = 16;
 
-// The same on 16-byte pieces of rows, at most 4 taps: a thread keeps one piece's latest inputs in registers while it walks RUN
-// consecutive tokens of the step (a request's start inside the run re-reads them), so a row is read once, not once per tap.  A run
-// inside one request - all but a few - has every row on its way before the first is used.
-constexpr int kConvRun = 8;
-template <typename Tag, int TAPS>
+// The same on 16-byte pieces of rows, at most 4 taps: a thread keeps one piece's latest inputs in registers while it walks RUN consecutive
+// tokens of the step, so a row is read once, not once per tap, and a piece's taps once per run.  Bound by vector work (30 instructions of a
+// channel and token, 18 of them the exponential and the quotient) and by bytes about equally: the next kConvAhead rows are on their way under the
+// work on the ones before, which a load under a condition would wait for - runs inside one request, all but a few, have none.
+// With the carried inputs' kernel, us, before (every row of 8 tokens loaded first) -> now: 4096 tokens x 6144 channels 44.9 -> 36.1, of 819 requests
+// 89 -> 62, 16384 x 8192 179 -> 152, 500 x 2048 16.1 -> 11.6.
+constexpr int kConvAhead = 4;
+template <typename Tag, int TAPS, int RUN>
 __global__ void __launch_bounds__(kBlock)
 conv_silu_run_kernel(void* out, int64_t out_stride, const void* in, int64_t in_stride, const float* w, const float* bias,
                      const float* state, int64_t state_stride, SeqBatch s, int64_t T, int C) {
   typedef Elem<Tag> E;
-  constexpr int V = E::kVec;
-  const int c = (blockIdx.y * kBlock + threadIdx.x) * V;
-  if (c >= C) return;
-  const int64_t t0 = (int64_t)blockIdx.x * kConvRun, t1 = t0 + kConvRun < T ? t0 + kConvRun : T;
-  float wt[TAPS][V], bs[V], past[TAPS][V];           // past[j]: the input TAPS - 1 - j rows back (the last one: this row's)
+  constexpr int V = E::kVec, A = kConvAhead, P = TAPS > 1 ? TAPS - 1 : 1;
+  static_assert(RUN % A == 0, "run");
+  const int piece = (blockIdx.y * kBlock + threadIdx.x) * V, c = min(piece, C - V);      // (past the end: the last piece again, not stored)
+  const int64_t t0 = (int64_t)blockIdx.x * RUN;
+  const int run = (int)(T - t0 < RUN ? T - t0 : RUN);
+  const char* const from = (const char*)in + (int64_t)c * E::kBytes;
+  u32x4 row[A], halo[P];
+  int req[A];
+#pragma unroll
+  for (int u = 0; u < A; ++u) {
+    const int64_t t = t0 + min(u, run - 1);
+    row[u] = ld16(from + t * in_stride * E::kBytes);
+    req[u] = s.token_req[t];
+  }
+#pragma unroll
+  for (int j = 0; j < TAPS - 1; ++j) {
+    const int64_t t = t0 - (TAPS - 1) + j;
+    halo[j] = ld16(from + (t > 0 ? t : 0) * in_stride * E::kBytes);
+  }
+  float wt[TAPS][V], bs[V];
   const bool quads = TAPS == 4 && ((uintptr_t)w & 15) == 0;          // a channel's taps are one load
 #pragma unroll
   for (int x = 0; x < V; ++x) {
@@ -207,75 +225,68 @@ conv_silu_run_kernel(void* out, int64_t out_stride, const void* in, int64_t in_s
       for (int j = 0; j < TAPS; ++j) wt[j][x] = w[(int64_t)(c + x) * TAPS + j];
     }
   }
-  int b = -1;
-  int64_t start = 0, prefix = 0;
-  if (t1 - t0 == kConvRun && s.extend_seq_lens && s.token_req[t0] == s.token_req[t1 - 1]) {
-    seq_of_token(s, t0, b, start, prefix);
-    const float* st = state + load_idx(s.req_pool_indices, b, s.idx64) * state_stride;
-    u32x4 row[TAPS - 1 + kConvRun];
+  float past[P][V];                                                   // past[j]: the input TAPS - 1 - j rows back
 #pragma unroll
-    for (int j = 0; j < TAPS - 1 + kConvRun; ++j) {
-      const int64_t r = t0 - (TAPS - 1) + j;
-      row[j] = ld16((const char*)in + ((j < TAPS - 1 && r < start ? t0 : r) * in_stride + c) * E::kBytes);
-    }
+  for (int j = 0; j < TAPS - 1; ++j) unpack16<Tag>(halo[j], past[j]);
+  int b = __builtin_amdgcn_readfirstlane(req[0]);
+  const bool same = b == s.token_req[t0 + run - 1];                    // all of the run one request's
+  // request b's inputs before its token t: rows of the step stay, those before it are carried ones, or none
+  const auto carry = [&](int64_t t) {
+    const int64_t start = s.extend_start_loc[b], prefix = s.extend_prefix_lens[b];
+    if (t - (TAPS - 1) >= start) return;
+    const float* st = state + load_idx(s.req_pool_indices, b, s.idx64) * state_stride;
 #pragma unroll
     for (int j = 0; j < TAPS - 1; ++j) {
-      unpack16<Tag>(row[j], past[j]);
-      const int64_t back = start - (t0 - (TAPS - 1) + j);            // > 0: so many rows before the step
+      const int64_t back = start - (t - (TAPS - 1) + j);              // > 0: so many rows before the step
       if (back > 0) {
 #pragma unroll
         for (int x = 0; x < V; ++x) past[j][x] = prefix - back >= 0 ? st[(TAPS - 1 - back) * C + c + x] : 0.f;
       }
     }
+  };
+  if (TAPS > 1) carry(t0);
+  const auto walk = [&](auto several) {                                // several: requests may end inside the run
+#pragma unroll 1
+    for (int g = 0; g < run; g += A) {
+      u32x4 next[A];
+      int next_req[A];
 #pragma unroll
-    for (int u = 0; u < kConvRun; ++u) {
-      unpack16<Tag>(row[TAPS - 1 + u], past[TAPS - 1]);
-      float o[V];
-#pragma unroll
-      for (int x = 0; x < V; ++x) {
-        float acc = bs[x];
-#pragma unroll
-        for (int j = 0; j < TAPS; ++j) acc += wt[j][x] * past[j][x];
-        o[x] = silu_ref(acc);
-#pragma unroll
-        for (int j = 0; j < TAPS - 1; ++j) past[j][x] = past[j + 1][x];
+      for (int u = 0; u < A; ++u) {
+        const int64_t t = t0 + min(g + A + u, run - 1);
+        next[u] = ld16(from + t * in_stride * E::kBytes);
+        if constexpr (decltype(several)::value) next_req[u] = s.token_req[t];
       }
-      st16((char*)out + ((t0 + u) * out_stride + c) * E::kBytes, pack16<Tag>(o));
-    }
-    return;
-  }
-  for (int64_t t = t0; t < t1; ++t) {
-    int nb;
-    int64_t nstart, nprefix;
-    seq_of_token(s, t, nb, nstart, nprefix);
-    if (nb != b) {                                   // (also the run's first token)
-      b = nb, start = nstart, prefix = nprefix;
-      const float* st = state + load_idx(s.req_pool_indices, b, s.idx64) * state_stride;
 #pragma unroll
-      for (int j = 0; j < TAPS - 1; ++j) {
-        const int64_t r = t - (TAPS - 1) + j;
-        if (r >= start) {
-          unpack16<Tag>(ld16((const char*)in + (r * in_stride + c) * E::kBytes), past[j]);
-        } else {
-          const int64_t back = start - r;            // 1 .. TAPS - 1 rows before the step
-#pragma unroll
-          for (int x = 0; x < V; ++x) past[j][x] = prefix - back >= 0 ? st[(TAPS - 1 - back) * C + c + x] : 0.f;
+      for (int u = 0; u < A; ++u) {
+        const int64_t t = t0 + g + u;
+        if constexpr (TAPS > 1 && decltype(several)::value) {
+          const int nb = __builtin_amdgcn_readfirstlane(req[u]);
+          if (nb != b) b = nb, carry(t);
         }
+        float here[V], o[V];
+        unpack16<Tag>(row[u], here);
+#pragma unroll
+        for (int x = 0; x < V; ++x) {
+          float acc = bs[x];
+#pragma unroll
+          for (int j = 0; j < TAPS - 1; ++j) acc += wt[j][x] * past[j][x];
+          acc += wt[TAPS - 1][x] * here[x];
+          o[x] = silu_ref(acc);
+#pragma unroll
+          for (int j = 0; j < TAPS - 2; ++j) past[j][x] = past[j + 1][x];
+          past[P - 1][x] = here[x];
+        }
+        if (g + u < run && piece < C) st16((char*)out + (t * out_stride + c) * E::kBytes, pack16<Tag>(o));
+      }
+#pragma unroll
+      for (int u = 0; u < A; ++u) {
+        row[u] = next[u];
+        if constexpr (decltype(several)::value) req[u] = next_req[u];
       }
     }
-    unpack16<Tag>(ld16((const char*)in + (t * in_stride + c) * E::kBytes), past[TAPS - 1]);
-    float o[V];
-#pragma unroll
-    for (int x = 0; x < V; ++x) {
-      float acc = bs[x];
-#pragma unroll
-      for (int j = 0; j < TAPS; ++j) acc += wt[j][x] * past[j][x];
-      o[x] = silu_ref(acc);
-#pragma unroll
-      for (int j = 0; j < TAPS - 1; ++j) past[j][x] = past[j + 1][x];
-    }
-    st16((char*)out + (t * out_stride + c) * E::kBytes, pack16<Tag>(o));
-  }
+  };
+  if (same) walk(std::false_type());                                   // (its loads stay on their way: no load is conditional)
+  else walk(std::true_type());
 }
 
 template <typename Tag>
@@ -323,7 +334,7 @@ conv_silu_step_kernel(void* out, int64_t out_stride, const void* in, int64_t in_
   const float cur = E::load(in, (int64_t)b * in_stride + c);
   acc += w[(int64_t)c * taps + keep] * cur;
   if (keep > 0) st[(int64_t)(keep - 1) * C + c] = cur;
-  E::store(out, (int64_t)b * out_stride + c, acc / (1.f + expf(-acc)));
+  E::store(out, (int64_t)b * out_stride + c, over_one_plus_exp(acc, acc));
 }
 
 constexpr int kChunk = 16;      // tokens staged in LDS per pass
@@ -608,7 +619,7 @@ gated_group_norm_kernel(void* out, int64_t out_stride, const float* y, int64_t y
     float ss = 0.f;
     for (int i = threadIdx.x; i < per; i += blockDim.x) {
       const float zv = E::load(z, t * z_stride + p * per + i);
-      const float v = y[t * y_stride + p * per + i] * (zv / (1.f + expf(-zv)));
+      const float v = y[t * y_stride + p * per + i] * over_one_plus_exp(zv, zv);
       ss += v * v;
     }
     ss = block_sum(ss, red);
@@ -616,7 +627,7 @@ gated_group_norm_kernel(void* out, int64_t out_stride, const float* y, int64_t y
     for (int i = threadIdx.x; i < per; i += blockDim.x) {
       const int c = p * per + i;
       const float zv = E::load(z, t * z_stride + c);
-      E::store(out, t * out_stride + c, y[t * y_stride + c] * (zv / (1.f + expf(-zv))) * inv * w[c]);
+      E::store(out, t * out_stride + c, y[t * y_stride + c] * over_one_plus_exp(zv, zv) * inv * w[c]);
     }
   }
 }
@@ -678,9 +689,13 @@ extern "C" int sp_causal_conv_silu(void* out, int64_t out_stride, const void* in
   const int vecn = dtype == SP_F32 ? 4 : 8;
   if (taps <= 4 && num_tokens > 64 && channels % vecn == 0 && in_stride % vecn == 0 && out_stride % vecn == 0 &&
       (((uintptr_t)in | (uintptr_t)out) & 15) == 0) {
-    const dim3 grid((unsigned)((num_tokens + kConvRun - 1) / kConvRun), (unsigned)((channels / vecn + kBlock - 1) / kBlock));
+    // runs of 16 tokens where they leave two waves for every SIMD, else of 8 (500 tokens x 2048 channels: 63 workgroups)
+    const unsigned pieces = (unsigned)((channels / vecn + kBlock - 1) / kBlock);
+    const bool longer = (num_tokens + 15) / 16 * pieces * (kBlock / 64) >= 2048;
+    const dim3 grid((unsigned)(longer ? (num_tokens + 15) / 16 : (num_tokens + 7) / 8), pieces);
 #define SP_CONV(TAPS)                                                                                                  \
-  SP_DISPATCH_DTYPE(dtype, (conv_silu_run_kernel<Tag, TAPS><<<grid, kBlock, 0, (hipStream_t)stream>>>(                  \
+  SP_DISPATCH_DTYPE(dtype, ((longer ? conv_silu_run_kernel<Tag, TAPS, 16> : conv_silu_run_kernel<Tag, TAPS, 8>)<<<      \
+                               grid, kBlock, 0, (hipStream_t)stream>>>(                                                \
                                out, out_stride, in, in_stride, weight, bias, state, state_stride, s, num_tokens, channels)))
     if (taps == 1) SP_CONV(1);
     else if (taps == 2) SP_CONV(2);

@@ -145,6 +145,31 @@ def test_causal_conv_runs(lens, prefixes, C, taps, dtype):
     assert ((got.double() - want).abs() <= bar * want.abs() + 4e-6).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lens", [[65], [3, 1, 1, 60, 16, 17, 2], [1] * 70, [5000, 9, 3190]], ids=lambda l: str(sum(l)))
+@pytest.mark.parametrize("C,taps", [(8, 4), (264, 3), (1032, 2), (16, 1)])
+def test_causal_conv_of_long_steps(lens, C, taps, dtype):
+    """runs of 8 and of 16 tokens in which requests end, the last one short; fewer pieces of a row than lanes"""
+    from scratchpad_amd import _native
+    announce("conv", dtype, lens[:8], len(lens), C, taps)
+    g = torch.Generator(device=DEV).manual_seed(4)
+    prefixes, slots = [(0, 2, 7)[i % 3] for i in range(len(lens))], list(range(1, len(lens) + 1))
+    x = torch.randn(sum(lens), C + 8, generator=g, device=DEV).to(dtype)[:, 8:]
+    w, bias = torch.randn(C, taps, generator=g, device=DEV), torch.randn(C, generator=g, device=DEV)
+    state = torch.randn(len(lens) + 1, taps - 1, C, generator=g, device=DEV)
+    before, at, want = state.clone(), 0, []
+    for n, p, s in zip(lens, prefixes, slots):
+        past = before[s].double().clone()
+        past[:max(0, taps - 1 - p)] = 0
+        pad = torch.cat([past, x[at:at + n].double()])
+        want.append(torch.nn.functional.silu(sum(pad[j:j + n] * w[:, j].double() for j in range(taps)) + bias.double()))
+        at += n
+    got = _native.causal_conv_silu(x, w, bias, state, seq_extend(lens, prefixes, slots))
+    want = torch.cat(want)
+    bar = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 1e-5}[dtype]          # as in test_causal_conv_runs
+    assert ((got.double() - want).abs() <= bar * want.abs() + 4e-6).all()
+
+
 @pytest.mark.parametrize("T", [65, 96, 257])
 @pytest.mark.parametrize("K,n,bias", [(32, 1, True), (288, 16, False), (2048, 31, True), (1024, 64, False), (544, 131, True)])
 def test_fp32_products_of_many_rows(T, K, n, bias):
