@@ -821,6 +821,9 @@ static bool narrow_pays(int pairs, int experts, int blocks) {
 }
 
 // Which kernel: by the mean rows per expert, pairs / experts (the counts themselves are on the device).  The rows kernel up to a mean of
+//   * 0 - it reads half a line at a time, the ring's loads whole ones past the L2 - where the chosen experts' weights are a stream out of HBM (160 MB and
+//     700 tiles of 64 weight rows): width 4096, 128 experts of ff 1536, 2 / 4 / 16 tokens, top 8: 70 + 33 | 63 + 33, 134 + 62 | 114 + 58, 366 + 173 | 309 + 151;
+//     8 of 14336, 2 / 6 tokens, top 2, up 137 | 117, 303 | 265; with fewer tiles 1 token of the former, up 37.5 | 39.7, of the latter, down 45 | 64;
 //   * 1.5.  Width 2048, 16 experts of ff 1408, up + down in us, rows kernel | ring tiles: mean 2: 44 + 18 | 40 + 18, 4: 43 + 19 | 39 + 18, 10: 43 + 19 |
 //     38 + 18; 32 experts of ff 1024, 3: 63 + 27 | 55 + 24, 16: 67 + 28 (64-row tiles) | 55 + 23; 128 of 512, width 1024, 4: 50 + 28 | 45 + 26;
 //   * 10 where it is at most one wave per SIMD: width 1024, 16 experts of ff 512, mean 2: 9.2 + 6.7 | 10.5 + 7.3, 10: 10.0 + 7.0 | 10.5 + 7.7; 32 experts,
@@ -838,7 +841,9 @@ int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
   const int64_t last_row = p.order ? (int64_t)pairs / p.row_div + 1 : pairs;
   const bool ring = p.K % 64 == 0 && last_row * p.a_stride < (int64_t)1 << 31 && (ACT >= 2 ? 2 : 1) * (int64_t)p.N * p.K < (int64_t)1 << 31;
   const int wide_per = ACT >= 2 ? 16 : 32, blocks_of_rows = (p.N + wide_per - 1) / wide_per;
-  const int most = ring && (int64_t)p.E * blocks_of_rows > 1024 ? 3 : 20;                         // half rows per expert
+  const double wrows = p.E * (1. - exp(-(double)pairs / p.E)) * (ACT >= 2 ? 2. : 1.) * p.N;                  // of the experts expected to be chosen
+  const bool streams = wrows * p.K >= 80e6 && wrows >= 700. * 64.;
+  const int most = !ring ? 20 : streams ? 0 : (int64_t)p.E * blocks_of_rows > 1024 ? 3 : 20;              // half rows per expert
   if (2 * (int64_t)pairs <= most * (int64_t)p.E && row_tiles <= 65535) {
     const bool narrow = narrow_pays(pairs, p.E, blocks_of_rows);
     const int per = narrow ? wide_per / 2 : wide_per;
