@@ -857,7 +857,8 @@ def library_rows_report() -> dict:
 
 
 # --------------------------------------------------------------------------- products of more rows
-DENSE_MAX_ROWS = 256          # and to 1024 of long rows: dense_gemm_pays
+DENSE_MAX_ROWS = 256
+DENSE_LONG_ROWS = 1024        # of long rows and of some small products: dense_gemm_pays
 _DENSE_ON = os.environ.get("SP_DENSE_GEMM", "1") != "0"
 _DENSE_PLANS = {}             # (M, weight rows, K, epilogue) -> _dense_plan: sizes alone, at most 1024 row counts per projection
 
@@ -887,9 +888,9 @@ def dense_gemm_pays(M: int, N: int, K: int) -> bool:
     if M <= SKINNY_MAX_ROWS:
         return M > 4 and N * K > 1 << 23 and (M > 8 or N > 4096 or K > 4096)
     if M > DENSE_MAX_ROWS:
-        if 768 < M <= 1024 and 1024 <= K <= 4096 and N <= 4096:
+        if 768 < M <= DENSE_LONG_ROWS and 1024 <= K <= 4096 and N <= 4096:
             return 160 < -(-M // 128) * -(-N // (64 if N <= 2048 else 128)) <= 256
-        return N >= 2048 and K >= 2 * N and K > 5120 and M <= (1024 if N <= 6144 else 512)
+        return N >= 2048 and K >= 2 * N and K > 5120 and M <= (DENSE_LONG_ROWS if N <= 6144 else 512)
     if N <= 2048 and (N <= 512 or (2048 < K <= 4096 and M > 64)):
         return False
     if 2048 < N <= 4096 and 1536 <= K <= 3072 and N * K <= 10 << 20 and (128 < M <= 160 or M > 208):
@@ -899,7 +900,7 @@ def dense_gemm_pays(M: int, N: int, K: int) -> bool:
 
 def _dense_plan(M: int, N: int, K: int, epilogue: int) -> int:
     """sp_gemm_dense_plan of a product with N weight rows that dense_gemm_pays for, else -1"""
-    if M > 1024:
+    if M > DENSE_LONG_ROWS:
         return -1
     key = (M, N, K, epilogue)
     plan = _DENSE_PLANS.get(key)
@@ -1132,7 +1133,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     table is computed over more rows than asked for (first M rows returned; rows are independent)."""
     shape = x.shape
     rows = shape[0] if len(shape) == 2 else 0
-    if rows > SKINNY_MAX_ROWS or (rows > 4 and weight.numel() > 1 << 23):
+    # (past DENSE_MAX_ROWS what dense_gemm_pays asks first: a product that is the library's pays no call)
+    if (SKINNY_MAX_ROWS < rows <= DENSE_MAX_ROWS or (DENSE_MAX_ROWS < rows <= DENSE_LONG_ROWS and (rows > 768 or shape[1] > 5120))
+            or (4 < rows <= SKINNY_MAX_ROWS and weight.numel() > 1 << 23)):
         out = _dense_product(x, weight, 0)
         if out is not None:
             return out

@@ -699,7 +699,15 @@ inline double ring_us(const RingCost& t, int pairs, int experts, int64_t wrows, 
   return c2 * c2 + f2 * f2 + s2 * s2;                                                                         // (its fourth power)
 }
 
+// (2 us of the host: the layers of a model ask for the same sizes one after the other, so a thread's last answers are kept)
 inline int ring_tile(int pairs, int experts, int64_t wrows, int K) {
+  struct Answer {
+    int64_t wrows;
+    int pairs, experts, K, tile;
+  };
+  thread_local Answer kept[16] = {};
+  Answer& a = kept[((unsigned)pairs * 5u + (unsigned)experts * 3u + (unsigned)(wrows >> 4) + (unsigned)(K >> 6)) % 16];
+  if (a.pairs == pairs && a.experts == experts && a.wrows == wrows && a.K == K) return a.tile;
   int best = -1;
   double least = 0.;
   for (int i = 0; i < (int)(sizeof(kRingTiles) / sizeof(kRingTiles[0])); ++i) {
@@ -707,6 +715,7 @@ inline int ring_tile(int pairs, int experts, int64_t wrows, int K) {
     const double us = ring_us(kRingTiles[i], pairs, experts, wrows, K);
     if (best < 0 || us < least) best = i, least = us;
   }
+  a = Answer{wrows, pairs, experts, K, best};
   return best;
 }
 
@@ -821,7 +830,7 @@ static bool narrow_pays(int pairs, int experts, int blocks) {
 }
 
 // Which kernel: by the mean rows per expert, pairs / experts (the counts themselves are on the device).  The rows kernel up to a mean of
-//   * 0 - it reads half a line at a time, the ring's loads whole ones past the L2 - where the chosen experts' weights are a stream out of HBM (160 MB and
+//   * 0 - it reads half a line at a time, the ring's loads whole ones past the L2 - where the chosen experts' weights are a stream out of HBM (220 MB and
 //     700 tiles of 64 weight rows): width 4096, 128 experts of ff 1536, 2 / 4 / 16 tokens, top 8: 70 + 33 | 63 + 33, 134 + 62 | 114 + 58, 366 + 173 | 309 + 151;
 //     8 of 14336, 2 / 6 tokens, top 2, up 137 | 117, 303 | 265; with fewer tiles 1 token of the former, up 37.5 | 39.7, of the latter, down 45 | 64;
 //   * 1.5.  Width 2048, 16 experts of ff 1408, up + down in us, rows kernel | ring tiles: mean 2: 44 + 18 | 40 + 18, 4: 43 + 19 | 39 + 18, 10: 43 + 19 |
@@ -842,7 +851,7 @@ int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
   const bool ring = p.K % 64 == 0 && last_row * p.a_stride < (int64_t)1 << 31 && (ACT >= 2 ? 2 : 1) * (int64_t)p.N * p.K < (int64_t)1 << 31;
   const int wide_per = ACT >= 2 ? 16 : 32, blocks_of_rows = (p.N + wide_per - 1) / wide_per;
   const double wrows = p.E * (1. - exp(-(double)pairs / p.E)) * (ACT >= 2 ? 2. : 1.) * p.N;                  // of the experts expected to be chosen
-  const bool streams = wrows * p.K >= 80e6 && wrows >= 700. * 64.;
+  const bool streams = wrows * p.K >= 110e6 && wrows >= 700. * 64.;
   const int most = !ring ? 20 : streams ? 0 : (int64_t)p.E * blocks_of_rows > 1024 ? 3 : 20;              // half rows per expert
   if (2 * (int64_t)pairs <= most * (int64_t)p.E && row_tiles <= 65535) {
     const bool narrow = narrow_pays(pairs, p.E, blocks_of_rows);
