@@ -809,6 +809,7 @@ def skinny_gemm_pays(M: int, N: int, K: int) -> bool:
 #                       only where it measured faster (calibrate_library_rows); on this build that reproduces the
 #                       table, on another library it falls back to M wherever the table's entry does not pay;
 #   "0"               - off: every product is run with the row count it was asked for.
+# It holds for products that are the library's: most of 17 - 256 rows are sp_gemm_dense's, unless the shape was calibrated.
 ROW_SLACK = 64
 _LIBRARY_ROWS_MEASURED_ON = {"torch": "2.10", "hip": "7.0"}      # version prefixes of the build the table is for
 _LIBRARY_ROWS_TABLE = {

@@ -3,7 +3,7 @@
 // Call sites it serves: the four per-layer projections and the LM head at decode time -
 // QKVParallelLinear / RowParallelLinear / MergedColumnParallelLinear.forward (nn/layers/linear.py:
 // 696-760, 423-470, 1033-1155 -> F.linear) and LogitsProcessor._get_logits
-// (nn/layers/logits_processor.py:340-376).  Above 16 rows the library GEMM (hipBLASLt) stays.
+// (nn/layers/logits_processor.py:340-376).  More rows, and 5 - 16 over large weights: gemm_dense.hip, then the library.
 //
 // At M <= 16 the product is a pure stream of the weight matrix (2 flop per weight byte per row): HBM-bound.  What decides the
 // rate is how many bytes of each weight row one load covers and how many workgroups share the stream, so there are three forms:
