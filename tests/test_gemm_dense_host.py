@@ -28,3 +28,13 @@ def test_plans_fit_their_products():
 def test_where_it_pays(M, N, K, takes):
     from scratchpad_amd import _native
     assert _native.dense_gemm_pays(M, N, K) is takes
+
+
+def test_linear_asks_for_every_product_that_pays():
+    """what linear looks at before the call, for steps past DENSE_MAX_ROWS: more than 768 rows, or K past 5120"""
+    from scratchpad_amd import _native
+    for M in (257, 400, 768, 769, 900, 1024, 1025):
+        for N in (1024, 2048, 3072, 4096, 6144, 8192, 28672):
+            for K in (1024, 2048, 4096, 5120, 5184, 8192, 14336, 28672):
+                if _native.dense_gemm_pays(M, N, K):
+                    assert M <= _native.DENSE_LONG_ROWS and (M > 768 or K > 5120)
