@@ -289,7 +289,9 @@ conv_silu_run_kernel(void* out, int64_t out_stride, const void* in, int64_t in_s
   else walk(std::true_type());
 }
 
-template <typename Tag>
+// KEEP: taps - 1, or 0 for any number of them (whose values wait in memory, loaded one after the other: with the convolution, 400 requests of a
+// token 30.4 us so, 27.0 with three in registers)
+template <typename Tag, int KEEP>
 __global__ void __launch_bounds__(kBlock)
 conv_state_kernel(float* state, int64_t state_stride, const void* in, int64_t in_stride, SeqBatch s, int C, int taps) {
   typedef Elem<Tag> E;
@@ -300,8 +302,9 @@ conv_state_kernel(float* state, int64_t state_stride, const void* in, int64_t in
   seq_span(s, b, start, len, prefix);
   if (len <= 0) return;
   float* st = state + load_idx(s.req_pool_indices, b, s.idx64) * state_stride;
-  const int keep = taps - 1;
-  float fresh[kMaxTaps];
+  const int keep = KEEP ? KEEP : taps - 1;
+  float fresh[KEEP ? KEEP : kMaxTaps];
+#pragma unroll
   for (int k = 0; k < keep; ++k) {
     const int64_t p = prefix + len - keep + k;       // position of the new entry k
     float val = 0.f;
@@ -309,6 +312,7 @@ conv_state_kernel(float* state, int64_t state_stride, const void* in, int64_t in
     else if (p >= 0) val = st[(p - prefix + keep) * C + c];
     fresh[k] = val;
   }
+#pragma unroll
   for (int k = 0; k < keep; ++k) st[(int64_t)k * C + c] = fresh[k];
 }
 
@@ -708,7 +712,8 @@ extern "C" int sp_causal_conv_silu(void* out, int64_t out_stride, const void* in
   }
   SP_LAUNCH_CHECK();
   if (taps > 1) {      // after every reader of the old state (stream order)
-    SP_DISPATCH_DTYPE(dtype, (conv_state_kernel<Tag><<<dim3((unsigned)batch_size, cb), kBlock, 0, (hipStream_t)stream>>>(
+    SP_DISPATCH_DTYPE(dtype, ((taps == 4 ? conv_state_kernel<Tag, 3> : conv_state_kernel<Tag, 0>)<<<dim3((unsigned)batch_size, cb), kBlock, 0,
+                                                                                                 (hipStream_t)stream>>>(
                                  state, state_stride, in, in_stride, s, channels, taps)));
     SP_LAUNCH_CHECK();
   }
