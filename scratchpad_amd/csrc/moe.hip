@@ -652,12 +652,12 @@ int launch_grouped_ring(const GroupedArgs& p, int pairs, int held, hipStream_t s
 
 // The tiles, and what one costs: us per step of BK where two workgroups share a unit and where one has it alone, and us besides.
 #define SP_RING_TILES(F)                                        \
-  F(0, 0.856f, 0.454f, 1.53f, true, 32, 128, 64, 1, 4, 4)       \
-  F(1, 0.787f, 0.389f, 2.88f, true, 32, 64, 128, 1, 4, 3)       \
-  F(2, 1.127f, 0.490f, 2.10f, true, 64, 128, 64, 2, 2, 3)       \
-  F(3, 0.636f, 0.129f, 4.05f, false, 64, 128, 64, 1, 4, 3)      \
-  F(4, 0.753f, 0.295f, 4.33f, false, 80, 128, 64, 1, 4, 3)      \
-  F(5, 0.423f, 0.118f, 3.98f, false, 96, 64, 64, 2, 2, 4)       \
+  F(0, 0.979f, 0.454f, 1.63f, true, 32, 128, 64, 1, 4, 4)       \
+  F(1, 0.801f, 0.389f, 2.88f, true, 32, 64, 128, 1, 4, 3)       \
+  F(2, 0.967f, 0.519f, 2.19f, true, 64, 128, 64, 2, 2, 3)       \
+  F(3, 0.529f, 0.129f, 4.16f, false, 64, 128, 64, 1, 4, 3)      \
+  F(4, 0.680f, 0.290f, 4.94f, false, 80, 128, 64, 1, 4, 3)      \
+  F(5, 0.455f, 0.118f, 3.98f, false, 96, 64, 64, 2, 2, 4)       \
   F(6, 1.102f, 0.533f, 4.92f, false, 128, 128, 64, 2, 4, 2)     \
   F(7, 1.269f, 0.664f, 5.16f, false, 160, 128, 64, 2, 2, 2)     \
   F(8, 1.432f, 0.658f, 5.84f, false, 192, 128, 64, 4, 2, 2)     \
@@ -682,8 +682,9 @@ inline double ring_row_tiles(int pairs, int experts, int bm) {
 
 // The time of a product with tile `t`: the longest of the chains of tiles that a unit works through, of what it loads into its LDS and of the
 // weights' way from memory, the two lesser ones added softly.  The last, not full round of tiles counts by the chance that it is there and that
-// some unit holds two of it.  Measured: 20 tiles, 58 products (widths 1024 and 2048, 8 to 128 experts, 8 to 4096 rows): 11 % rms from this, and the tile
-// chosen by it 3 % behind the best of the 20 on average.
+// some unit holds two of it.  Costs by least squares
+// from 20 tiles' timings of 58 products (widths 1024 and 2048, 8 to 128 experts, 8 to 4096 rows: 11 % rms), those of the smaller tiles then moved to what picks the
+// fastest tile: 2 - 3 % behind the best of the 20 on average (70 other row counts: 1 % faster than by the plain fit, 0.96 - 1.10).
 inline double ring_us(const RingCost& t, int pairs, int experts, int64_t wrows, int K) {
   const double cols = (double)((wrows + t.bn - 1) / t.bn), tiles = experts * ring_row_tiles(pairs, experts, t.bm) * cols, steps = K / t.bk;
   const bool pair = t.lds <= 80 * 1024;
