@@ -928,8 +928,9 @@ def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Opti
     plan = _dense_plan(M, N, K, epilogue)
     dtype = x.dtype
     if plan < 0 or wshape[1] != K or (dtype is not torch.bfloat16 and dtype is not torch.float16) or weight.dtype is not dtype \
-            or not x.is_cuda or x.get_device() != weight.get_device() or type(x) not in _PLAIN or type(weight) not in _PLAIN:
-        return None
+            or not x.is_cuda or not x.get_device() == weight.get_device() == torch._C._cuda_getDevice() \
+            or type(x) not in _PLAIN or type(weight) not in _PLAIN:
+        return None          # (another device's tensors: the launch would be on the current one's stream)
     (xs, x1), (ws, w1) = x.stride(), weight.stride()
     if x1 != 1 or w1 != 1 or xs % 8 or ws % 8 or xs < K or ws < K or M * xs >= 1 << 31 or N * ws >= 1 << 31:
         return None

@@ -1,5 +1,6 @@
 """sp_gemm_dense_plan over the sizes that linear hands it: a tile that divides K, shares that it can serve (host code, no GPU)."""
 import pytest
+import torch
 
 
 def test_plans_fit_their_products():
@@ -38,3 +39,42 @@ def test_linear_asks_for_every_product_that_pays():
             for K in (1024, 2048, 4096, 5120, 5184, 8192, 14336, 28672):
                 if _native.dense_gemm_pays(M, N, K):
                     assert M <= _native.DENSE_LONG_ROWS and (M > 768 or K > 5120)
+
+
+class _OnDevice(torch.Tensor):
+    """a tensor that says it is on GPU `device`, for what looks at that and launches nothing"""
+    device_index = 0
+    is_cuda = True
+
+    def get_device(self):
+        return self.device_index
+
+
+def _own_product(monkeypatch, device=0, current=0, dtype=torch.bfloat16):
+    """whether _dense_product hands x @ w.T of 64 rows to the native product"""
+    from scratchpad_amd import _native
+    calls = []
+
+    class Library:
+        sp_gemm_dense_plan = staticmethod(lambda *a: 256)
+        sp_gemm_dense = staticmethod(lambda *a: calls.append(a) or 0)
+
+    with monkeypatch.context() as m:
+        m.setattr(_native, "load", lambda: Library)
+        m.setattr(_native, "_PLAIN", (_OnDevice,))
+        m.setattr(_native, "_DENSE_PLANS", {})
+        m.setattr(_native, "_DENSE_ON", True)
+        m.setattr(_native, "_stream", lambda: 0)
+        m.setattr(torch._C, "_cuda_getDevice", lambda: current, raising=False)
+        x, w = (torch.zeros(rows, 1024, dtype=dtype).as_subclass(_OnDevice) for rows in (64, 1024))
+        x.device_index = w.device_index = device
+        out = _native._dense_product(x, w, 0)
+    assert (out is None) == (not calls)
+    return bool(calls)
+
+
+def test_only_tensors_of_the_current_device(monkeypatch):
+    """the launch is on the current device's stream: a product on another one is the library's, which sets the device itself"""
+    assert _own_product(monkeypatch)
+    assert _own_product(monkeypatch, device=1, current=1)
+    assert not _own_product(monkeypatch, device=1, current=0)
