@@ -505,8 +505,7 @@ SP_API int sp_moe_align(int32_t* offsets, int32_t* order, int32_t* place, const 
                         void* stream);
 /* out[pos, :] = w[expert(pos)] a[row(pos)], w [experts, n, k]; row(pos) = order[pos] / row_div, or pos when order is null.
  * act (ABI 14): 0 none, 1 max(out, 0)^2 on the fp32 sum.  `experts` may be less than sp_moe_align's: the pairs of the ids
- * behind them (outputs that have no weight) get no row written.  An order names rows of a below pairs / row_div + 1, as
- * sp_moe_align's does, or of less than 2^31 elements from a's first.                                                     */
+ * behind them (outputs that have no weight) get no row written.                                                        */
 SP_API int sp_moe_grouped_gemm(void* out, const void* a, const void* w, const int32_t* offsets, const int32_t* order,
                                int row_div, int pairs, int n, int k, int experts, int64_t a_stride, int64_t out_stride,
                                int act, int dtype, void* stream);

@@ -1494,14 +1494,6 @@ def moe_align(ids: torch.Tensor, experts: int):
     return offsets, order, place
 
 
-def _near_rows(a: torch.Tensor, pairs: int, order: torch.Tensor, row_div: int):
-    """Rows that lie further into ``a`` than its pairs say (the kernels tell from these whether 32-bit offsets reach a row): a copy
-    of those that are wanted"""
-    if a.shape[0] <= pairs // row_div + 1:
-        return a, order, row_div
-    return a[torch.div(order[:pairs], row_div, rounding_mode="floor").long()], None, 1
-
-
 def moe_grouped_gemm(a: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, pairs: int, order: Optional[torch.Tensor] = None,
                      row_div: int = 1, act: str = "none") -> torch.Tensor:
     """out [pairs, N]: row pos = w[expert of pos] @ a[order[pos] // row_div] (a[pos] without order); w [E, N, K]; act
@@ -1510,8 +1502,6 @@ def moe_grouped_gemm(a: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, pa
     if w.dim() != 3 or not w.is_contiguous() or w.dtype != a.dtype or w.shape[2] != a.shape[1]:
         raise RuntimeError("moe_grouped_gemm: w [E, N, K] contiguous of a's dtype")
     E, N, K = w.shape
-    if order is not None and a.shape[0] * a.stride(0) >= 1 << 31:
-        a, order, row_div = _near_rows(a, pairs, order, row_div)
     out = torch.empty((pairs, N), dtype=a.dtype, device=a.device)
     _check(load().sp_moe_grouped_gemm(out.data_ptr(), a.data_ptr(), w.data_ptr(), offsets.data_ptr(), _ptr(order), row_div,
                                       pairs, N, K, E, a.stride(0), out.stride(0), {"none": 0, "relu2": 1}[act], _dt(a), _stream()),
@@ -1530,8 +1520,6 @@ def moe_grouped_glu(a: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, pai
     E, n, K = w.shape
     if a.dtype == torch.float32 or K % 32 or a.stride(0) % 8 or a.data_ptr() % 16 or w.data_ptr() % 16:
         return None
-    if order is not None and a.shape[0] * a.stride(0) >= 1 << 31:
-        a, order, row_div = _near_rows(a, pairs, order, row_div)
     out = torch.empty((pairs, n // 2), dtype=a.dtype, device=a.device)
     _check(load().sp_moe_grouped_glu(out.data_ptr(), a.data_ptr(), w.data_ptr(), offsets.data_ptr(), _ptr(order), row_div, pairs,
                                      n // 2, K, E, a.stride(0), out.stride(0), {"silu": 0, "clamped": 1}[act], limit, alpha,

@@ -344,6 +344,7 @@ struct GroupedArgs {
   int64_t a_stride, out_stride;      // elements
   int vec_out;                       // 8-byte stores of 4 columns are aligned and inside a row
   float limit, alpha;                // ACT 3
+  int32_t far;                       // entries of `order` from here on name rows that no 32-bit offset from a's first byte reaches (the ring's)
 };
 
 // (shared by the separate launch and the fused epilogue, which agree bit for bit)
@@ -566,6 +567,32 @@ __global__ void __launch_bounds__(256, 2) moe_grouped_tile_kernel(GroupedArgs p)
   }
 }
 
+// The sums of a wave's part of a ring tile straight from memory, in the ring's order: for tiles with a row that a load's 32-bit offset does not
+// reach.  (An order may name any rows of `a`, and only the device knows which; those that moe_align makes lie in its first pairs / row_div + 1,
+// which the launcher looks at.)
+template <typename Tag, typename T, bool GLU>
+__device__ __forceinline__ void far_product(f32x4_q (&acc)[T::FM][T::FN], const GroupedArgs& p, const char* we, int pos0, int rows_end, int n0, int col0,
+                                            int lane) {
+  const int r16 = lane & 15, q = lane >> 4;
+#pragma unroll 1
+  for (int k = 8 * q; k < p.K; k += 32) {
+    u32x4 wf[T::FN];
+#pragma unroll
+    for (int j = 0; j < T::FN; ++j) {
+      const int c = col0 + 16 * j;                         // (a multiple of 16)
+      const int64_t row = GLU ? min(n0 + c / 2 + r16 % 8, p.N - 1) + (r16 >= 8 ? p.N : 0) : min(n0 + c + r16, p.N - 1);
+      wf[j] = ld16(we + (row * p.K + k) * 2);
+    }
+#pragma unroll
+    for (int f = 0; f < T::FM; ++f) {
+      const int64_t row = p.order[min(pos0 + 16 * f + r16, rows_end - 1)] / p.row_div;
+      const u32x4 xf = ld16(p.a + (row * p.a_stride + k) * 2);
+#pragma unroll
+      for (int j = 0; j < T::FN; ++j) acc[f][j] = mfma32<Tag>(wf[j], xf, acc[f][j]);
+    }
+  }
+}
+
 // The same for K a multiple of 64, by ring_product's loop.  Two workgroups share a CU (of all tiles but the largest) and fill each other's beginnings
 // and ends.  GLU: 8 gate rows and the up rows of the same 8 columns in one operand, their sums 32 lanes apart.  ONCE: an expert with one row tile reads
 // its weights past the L2.  The row tiles of one column tile follow each other: the weights they share are in the L2.
@@ -593,6 +620,10 @@ __global__ void __launch_bounds__(T::W * 64, T::kWaves) moe_grouped_ring_kernel(
   uint32_t off[L];
   const char* base[L];
   const char* const we = p.w + (int64_t)e * wrows * p.K * 2;
+  bool far = false;                                        // (of the tile, the same in every wave)
+  if (p.order)
+#pragma unroll
+    for (int r = 0; r < BM; r += 64) far |= p.order[min(row0 + r + lane, rows_end - 1)] >= p.far;
 #pragma unroll
   for (int i = 0; i < L; ++i) {
     const int g = min(i * T::W + wave, T::G - 1), r = g * RPL + lane / CH, chunk = (lane % CH) ^ (r & 7);
@@ -615,7 +646,8 @@ __global__ void __launch_bounds__(T::W * 64, T::kWaves) moe_grouped_ring_kernel(
   for (int f = 0; f < FM; ++f)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[f][j] = f32x4_q{0.f, 0.f, 0.f, 0.f};
-  if (ONCE && row_tiles == 1) ring_product<Tag, T, ONCE, 2>(acc, off, base, lds, steps, wave, lane);
+  if (__any(far)) far_product<Tag, T, GLU>(acc, p, we, row0 + wm * T::TM, rows_end, n0, wn * T::TN, lane);
+  else if (ONCE && row_tiles == 1) ring_product<Tag, T, ONCE, 2>(acc, off, base, lds, steps, wave, lane);
   else ring_product<Tag, T, 0, 2>(acc, off, base, lds, steps, wave, lane);
 #pragma unroll
   for (int f = 0; f < FM; ++f) {
@@ -847,7 +879,7 @@ int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
   const int held = pairs < p.E ? pairs : p.E;                    // experts with a row, at most
   const int row_tiles = pairs / 16 + held;
   // (moe_align takes 4096 experts, 6656 tiles; more than a grid's second dimension holds go to the 64-row tiles)
-  // (a ring's loads have 32-bit offsets from the operand's first byte)
+  // (a ring's loads have 32-bit offsets from the operand's first byte; rows further on that an order names: far_product)
   const int64_t last_row = p.order ? (int64_t)pairs / p.row_div + 1 : pairs;
   const bool ring = p.K % 64 == 0 && last_row * p.a_stride < (int64_t)1 << 31 && (ACT >= 2 ? 2 : 1) * (int64_t)p.N * p.K < (int64_t)1 << 31;
   const int wide_per = ACT >= 2 ? 16 : 32, blocks_of_rows = (p.N + wide_per - 1) / wide_per;
@@ -877,6 +909,11 @@ int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
   else moe_grouped_tile_kernel<Tag, 64, ACT><<<dim3(blocks), 256, 0, st>>>(p);
   SP_LAUNCH_CHECK();
   return SP_OK;
+}
+
+// GroupedArgs::far: all of a row below 2^31 / a_stride is within 2^32 bytes of the first one's beginning
+inline int32_t far_pairs(int row_div, int64_t a_stride) {
+  return (int32_t)std::min<int64_t>((((int64_t)1 << 31) / a_stride) * row_div, INT32_MAX);
 }
 
 // ---- y = g' * sigmoid(alpha g') * (u' + 1), g' = min(g, limit), u' = clamp(u, -limit, limit); gu = [g | u] per row -----
@@ -1000,7 +1037,7 @@ extern "C" int sp_moe_grouped_gemm(void* out, const void* a, const void* w, cons
   const bool aligned = k % 32 == 0 && a_stride % 8 == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0;
   if ((dtype == SP_BF16 || dtype == SP_F16) && aligned) {
     const GroupedArgs p{(char*)out, (const char*)a, (const char*)w, offsets, order, row_div, n, k, experts, a_stride, out_stride,
-                        out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0, 0.f, 0.f};
+                        out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0, 0.f, 0.f, far_pairs(row_div, a_stride)};
     hipStream_t st = (hipStream_t)stream;
     if (dtype == SP_BF16)
       return act ? launch_grouped_mfma<bf16_tag, 1>(p, pairs, st) : launch_grouped_mfma<bf16_tag, 0>(p, pairs, st);
@@ -1022,7 +1059,7 @@ extern "C" int sp_moe_grouped_glu(void* out, const void* a, const void* w, const
   if (dtype != SP_BF16 && dtype != SP_F16) return SP_ERR_UNSUPPORTED;
   if (k % 32 || a_stride % 8 || ((uintptr_t)a & 15) || ((uintptr_t)w & 15)) return SP_ERR_UNSUPPORTED;
   const GroupedArgs p{(char*)out, (const char*)a, (const char*)w, offsets, order, row_div, ff, k, experts, a_stride, out_stride,
-                      out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0, limit, alpha};
+                      out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0, limit, alpha, far_pairs(row_div, a_stride)};
   hipStream_t st = (hipStream_t)stream;
   if (dtype == SP_BF16)
     return act ? launch_grouped_mfma<bf16_tag, 3>(p, pairs, st) : launch_grouped_mfma<bf16_tag, 2>(p, pairs, st);

@@ -174,3 +174,27 @@ def test_rows_far_from_the_first():
     near = a[-P:].clone()
     assert torch.equal(_native.moe_grouped_gemm(a, w, offsets, P, order), _native.moe_grouped_gemm(near, w, offsets, P))
     assert torch.equal(_native.moe_grouped_glu(a, w, offsets, P, order, 1, "silu"), _native.moe_grouped_glu(near, w, offsets, P, None, 1, "silu"))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("row_div", [1, 2])
+@pytest.mark.parametrize("counts", [[40, 60], [7, 0, 300, 293], [33, 1567], [70] * 16], ids=lambda c: str(sum(c)))
+def test_orders_of_near_and_far_rows(counts, row_div, dtype):
+    """an order names any rows: first ones, ones on either side of 2^31 elements and the last, in one row tile; the bits of the same rows gathered"""
+    from scratchpad_amd import _native
+    K, N, E, P = 512, 200, len(counts), sum(counts)
+    print("far", counts[:4], row_div, dtype, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(11)
+    edge = 2 ** 31 // K
+    a = torch.empty(edge + 2 * P, K, dtype=dtype, device=DEV)
+    rows = torch.cat([torch.arange(P, device=DEV), torch.arange(edge - P, edge + P, device=DEV), torch.arange(a.shape[0] - P, a.shape[0], device=DEV)])
+    a[rows] = torch.randn(len(rows), K, generator=g, device=DEV).to(dtype)
+    rows = rows[torch.randperm(len(rows), generator=g, device=DEV)[:P]]
+    order = (rows * row_div + row_div - 1).to(torch.int32)
+    w = (torch.randn(E, 2 * N, K, generator=g, device=DEV) * K ** -0.5).to(dtype)
+    offsets = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device=DEV)
+    near = a[rows].clone()
+    for act in ("none", "relu2"):
+        assert torch.equal(_native.moe_grouped_gemm(a, w, offsets, P, order, row_div, act=act), _native.moe_grouped_gemm(near, w, offsets, P, act=act))
+    for act in (("silu",), ("clamped", 2.0, 1.702)):
+        assert torch.equal(_native.moe_grouped_glu(a, w, offsets, P, order, row_div, *act), _native.moe_grouped_glu(near, w, offsets, P, None, 1, *act))
