@@ -207,6 +207,7 @@ def _not_built(name: str):
     def missing(*_a, **_k):
         raise RuntimeError(f"{name} is not in this build of {_LIB_PATH} (it was made of the sources of one model family, or of older ones): "
                            "run `python -m scratchpad_amd.build` for the whole library")
+    missing.not_built = True
     return missing
 
 
@@ -906,13 +907,18 @@ def _dense_plan(M: int, N: int, K: int, epilogue: int) -> int:
     key = (M, N, K, epilogue)
     plan = _DENSE_PLANS.get(key)
     if plan is None:
-        plan = load().sp_gemm_dense_plan(M, N >> epilogue, K, epilogue) if dense_gemm_pays(M, N, K) and N % (epilogue + 1) == 0 else -1
+        plan = -1
+        if dense_gemm_pays(M, N, K) and N % (epilogue + 1) == 0:
+            entry = load().sp_gemm_dense_plan
+            if not hasattr(entry, "not_built"):          # (a library made before it: the products are the library's)
+                plan = entry(M, N >> epilogue, K, epilogue)
         _DENSE_PLANS[key] = plan
     return plan
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _forward_ad = torch.autograd.forward_ad
+_tracing = torch._C._get_tracing_state
 _transforms = torch._C._functorch.peek_interpreter_stack
 _dispatch_modes = torch._C._len_torch_dispatch_stack
 
@@ -920,22 +926,23 @@ _dispatch_modes = torch._C._len_torch_dispatch_stack
 def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Optional[torch.Tensor]:
     """x @ weight.T (epilogue 1: silu of its first half of columns times its second) by sp_gemm_dense, or None: a product it does not run,
     or not faster than what else would.  Autograd, function transforms, tracing and dispatch modes keep the library call they can see."""
-    shape, wshape = x.shape, weight.shape
-    if not _DENSE_ON or len(shape) != 2 or len(wshape) != 2:
+    # (first what keeps tensors of the host, sizes that are no numbers and types that others bring from the library and its table of plans)
+    if not _DENSE_ON or not x.is_cuda or type(x) not in _PLAIN or type(weight) not in _PLAIN or _tracing() is not None:
+        return None
+    shape, wshape, dtype = x.shape, weight.shape, x.dtype
+    if len(shape) != 2 or len(wshape) != 2 or (dtype is not torch.bfloat16 and dtype is not torch.float16) or weight.dtype is not dtype:
         return None
     M, K = shape
     N = wshape[0]
     plan = _dense_plan(M, N, K, epilogue)
-    dtype = x.dtype
-    if plan < 0 or wshape[1] != K or (dtype is not torch.bfloat16 and dtype is not torch.float16) or weight.dtype is not dtype \
-            or not x.is_cuda or not x.get_device() == weight.get_device() == torch._C._cuda_getDevice() \
-            or type(x) not in _PLAIN or type(weight) not in _PLAIN:
-        return None          # (another device's tensors: the launch would be on the current one's stream)
+    # (another device's tensors: the launch would be on the current one's stream)
+    if plan < 0 or wshape[1] != K or not x.get_device() == weight.get_device() == torch._C._cuda_getDevice():
+        return None
     (xs, x1), (ws, w1) = x.stride(), weight.stride()
     if x1 != 1 or w1 != 1 or xs % 8 or ws % 8 or xs < K or ws < K or M * xs >= 1 << 31 or N * ws >= 1 << 31:
         return None
     if (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)) or _dispatch_modes() or _transforms() is not None \
-            or _forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None:
+            or _forward_ad._current_level >= 0:
         return None
     # a table that was calibrated on this box says how the library runs these projections
     if (N, K) in getattr(_LIBRARY_ROWS, "calibrated", ()):

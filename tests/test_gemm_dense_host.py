@@ -78,3 +78,45 @@ def test_only_tensors_of_the_current_device(monkeypatch):
     assert _own_product(monkeypatch)
     assert _own_product(monkeypatch, device=1, current=1)
     assert not _own_product(monkeypatch, device=1, current=0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows, N, K", [(8, 6144, 2048), (64, 768, 1024), (200, 1024, 1024), (800, 2048, 1024), (260, 2048, 5184)])
+def test_tensors_that_are_not_on_a_gpu_need_no_library(monkeypatch, rows, N, K, dtype):
+    from scratchpad_amd import _native
+
+    def missing():
+        raise RuntimeError("not built")
+
+    monkeypatch.setattr(_native, "load", missing)
+    monkeypatch.setattr(_native, "_DENSE_PLANS", {})
+    assert _native.dense_gemm_pays(rows, N, K)
+    x, w = torch.ones(rows, K, dtype=dtype), torch.ones(N, K, dtype=dtype)
+    assert torch.equal(_native.linear(x, w), torch.nn.functional.linear(x, w))
+    assert _native.linear(x.to("meta"), w.to("meta")).shape == (rows, N)
+    assert _native.dense_silu_mul(x, w) is None and _native.linear_silu_mul(x, w) is None
+
+
+def test_traced_and_symbolic_sizes():
+    """sizes that are no plain numbers reach neither the table of plans nor the library"""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from scratchpad_amd import _native
+    x, w = torch.randn(64, 1024), torch.randn(256, 1024)
+    want = torch.nn.functional.linear(x, w)
+    before = dict(_native._DENSE_PLANS)
+    assert torch.allclose(torch.jit.trace(_native.linear, (x, w))(x, w), want)
+    assert torch.allclose(make_fx(_native.linear, tracing_mode="symbolic")(x, w)(x, w), want)
+    assert _native._DENSE_PLANS == before
+
+
+def test_a_library_of_before_the_product():
+    """its entry is a stub that raises: the products are the library's"""
+    from scratchpad_amd import _native
+
+    class Older:
+        sp_gemm_dense_plan = staticmethod(_native._not_built("sp_gemm_dense_plan"))
+
+    with pytest.MonkeyPatch.context() as m:
+        m.setattr(_native, "load", lambda: Older)
+        m.setattr(_native, "_DENSE_PLANS", {})
+        assert _native.dense_gemm_pays(64, 1024, 1024) and _native._dense_plan(64, 1024, 1024, 0) == -1
