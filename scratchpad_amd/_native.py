@@ -925,9 +925,9 @@ _dispatch_modes = torch._C._len_torch_dispatch_stack
 
 def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Optional[torch.Tensor]:
     """x @ weight.T (epilogue 1: silu of its first half of columns times its second) by sp_gemm_dense, or None: a product it does not run,
-    or not faster than what else would.  Autograd, function transforms, tracing and dispatch modes keep the library call they can see."""
+    or not faster than what else would.  Autograd, function transforms, tracing, compilers and dispatch modes keep the library call they can see."""
     # (first what keeps tensors of the host, sizes that are no numbers and types that others bring from the library and its table of plans)
-    if not _DENSE_ON or not x.is_cuda or type(x) not in _PLAIN or type(weight) not in _PLAIN or _tracing() is not None:
+    if not _DENSE_ON or torch.compiler.is_compiling() or not x.is_cuda or type(x) not in _PLAIN or type(weight) not in _PLAIN or _tracing() is not None:
         return None
     shape, wshape, dtype = x.shape, weight.shape, x.dtype
     if len(shape) != 2 or len(wshape) != 2 or (dtype is not torch.bfloat16 and dtype is not torch.float16) or weight.dtype is not dtype:

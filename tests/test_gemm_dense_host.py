@@ -1,4 +1,6 @@
 """sp_gemm_dense_plan over the sizes that linear hands it: a tile that divides K, shares that it can serve (host code, no GPU)."""
+import contextlib
+
 import pytest
 import torch
 
@@ -50,8 +52,8 @@ class _OnDevice(torch.Tensor):
         return self.device_index
 
 
-def _own_product(monkeypatch, device=0, current=0, dtype=torch.bfloat16):
-    """whether _dense_product hands x @ w.T of 64 rows to the native product"""
+def _own_product(monkeypatch, device=0, current=0, dtype=torch.bfloat16, within=contextlib.nullcontext):
+    """whether _dense_product, called under `within`, hands x @ w.T of 64 rows to the native product"""
     from scratchpad_amd import _native
     calls = []
 
@@ -68,7 +70,8 @@ def _own_product(monkeypatch, device=0, current=0, dtype=torch.bfloat16):
         m.setattr(torch._C, "_cuda_getDevice", lambda: current, raising=False)
         x, w = (torch.zeros(rows, 1024, dtype=dtype).as_subclass(_OnDevice) for rows in (64, 1024))
         x.device_index = w.device_index = device
-        out = _native._dense_product(x, w, 0)
+        with within():
+            out = _native._dense_product(x, w, 0)
     assert (out is None) == (not calls)
     return bool(calls)
 
@@ -120,3 +123,11 @@ def test_a_library_of_before_the_product():
         m.setattr(_native, "load", lambda: Older)
         m.setattr(_native, "_DENSE_PLANS", {})
         assert _native.dense_gemm_pays(64, 1024, 1024) and _native._dense_plan(64, 1024, 1024, 0) == -1
+
+
+def test_compiled_graphs_hold_the_product():
+    """Dynamo traces linear as one graph, whatever the library would take"""
+    from scratchpad_amd import _native
+    x, w = torch.randn(64, 1024), torch.randn(1024, 1024)
+    compiled = torch.compile(_native.linear, backend="eager", fullgraph=True)
+    assert torch.equal(compiled(x, w), torch.nn.functional.linear(x, w))

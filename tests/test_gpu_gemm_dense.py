@@ -114,3 +114,12 @@ def test_replays_of_a_captured_product_are_the_eager_one():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, _native.linear(x, w)), i
+
+
+def test_compiled_graphs_hold_the_product():
+    """Dynamo traces linear of tensors on the GPU as one graph: no call into the library that it cannot see"""
+    from scratchpad_amd import _native
+    x, w = torch.randn(64, 1024, device="cuda").bfloat16(), torch.randn(1024, 1024, device="cuda").bfloat16()
+    assert _native.dense_gemm_pays(64, 1024, 1024)
+    compiled = torch.compile(_native.linear, backend="eager", fullgraph=True)
+    assert torch.equal(compiled(x, w), torch.nn.functional.linear(x, w))
