@@ -14,6 +14,7 @@ import weakref
 from typing import Optional, Tuple
 
 import torch
+from torch.utils._device import DeviceContext
 
 # SP_NATIVE_LIB names a diagnostic build under lib/ (A/B runs of a kernel variant through the whole model); unset = the product
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib",
@@ -923,9 +924,15 @@ _transforms = torch._C._functorch.peek_interpreter_stack
 _dispatch_modes = torch._C._len_torch_dispatch_stack
 
 
+def _function_modes() -> bool:
+    """under a mode that overrides torch's functions (the one that says where new tensors go, torch.device's, overrides no product)"""
+    return torch._C._len_torch_function_stack() > 0 \
+        and any(type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack())
+
+
 def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Optional[torch.Tensor]:
     """x @ weight.T (epilogue 1: silu of its first half of columns times its second) by sp_gemm_dense, or None: a product it does not run,
-    or not faster than what else would.  Autograd, function transforms, tracing, compilers and dispatch modes keep the library call they can see."""
+    or not faster than what else would.  Autograd, function transforms, tracing, compilers and modes keep the library call they can see."""
     # (first what keeps tensors of the host, sizes that are no numbers and types that others bring from the library and its table of plans)
     if not _DENSE_ON or torch.compiler.is_compiling() or not x.is_cuda or type(x) not in _PLAIN or type(weight) not in _PLAIN or _tracing() is not None:
         return None
@@ -941,8 +948,8 @@ def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Opti
     (xs, x1), (ws, w1) = x.stride(), weight.stride()
     if x1 != 1 or w1 != 1 or xs % 8 or ws % 8 or xs < K or ws < K or M * xs >= 1 << 31 or N * ws >= 1 << 31:
         return None
-    if (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)) or _dispatch_modes() or _transforms() is not None \
-            or _forward_ad._current_level >= 0:
+    if (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)) or _dispatch_modes() or _function_modes() \
+            or _transforms() is not None or _forward_ad._current_level >= 0:
         return None
     # a table that was calibrated on this box says how the library runs these projections
     if (N, K) in getattr(_LIBRARY_ROWS, "calibrated", ()):

@@ -131,3 +131,14 @@ def test_compiled_graphs_hold_the_product():
     x, w = torch.randn(64, 1024), torch.randn(1024, 1024)
     compiled = torch.compile(_native.linear, backend="eager", fullgraph=True)
     assert torch.equal(compiled(x, w), torch.nn.functional.linear(x, w))
+
+
+class _Counting(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def test_function_modes_see_the_product(monkeypatch):
+    """a mode that overrides torch's functions finds the library's product; the one that only says where new tensors go hides none"""
+    assert not _own_product(monkeypatch, within=_Counting)
+    assert _own_product(monkeypatch, within=lambda: torch.device("cpu"))

@@ -123,3 +123,18 @@ def test_compiled_graphs_hold_the_product():
     assert _native.dense_gemm_pays(64, 1024, 1024)
     compiled = torch.compile(_native.linear, backend="eager", fullgraph=True)
     assert torch.equal(compiled(x, w), torch.nn.functional.linear(x, w))
+
+
+def test_function_modes_find_the_librarys_product():
+    from scratchpad_amd import _native
+    x, w = torch.randn(64, 1024, device="cuda").bfloat16(), torch.randn(1024, 1024, device="cuda").bfloat16()
+    seen = []
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        _native.linear(x, w)
+    assert torch.nn.functional.linear in seen
