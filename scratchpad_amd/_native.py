@@ -932,7 +932,7 @@ def _function_modes() -> bool:
 
 def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Optional[torch.Tensor]:
     """x @ weight.T (epilogue 1: silu of its first half of columns times its second) by sp_gemm_dense, or None: a product it does not run,
-    or not faster than what else would.  Autograd, function transforms, tracing, compilers and modes keep the library call they can see."""
+    or not faster than what else would.  Autograd, function transforms, tracing, compilers, modes and casts keep the library call they can see."""
     # (first what keeps tensors of the host, sizes that are no numbers and types that others bring from the library and its table of plans)
     if not _DENSE_ON or torch.compiler.is_compiling() or not x.is_cuda or type(x) not in _PLAIN or type(weight) not in _PLAIN or _tracing() is not None:
         return None
@@ -949,7 +949,8 @@ def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Opti
     if x1 != 1 or w1 != 1 or xs % 8 or ws % 8 or xs < K or ws < K or M * xs >= 1 << 31 or N * ws >= 1 << 31:
         return None
     if (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)) or _dispatch_modes() or _function_modes() \
-            or _transforms() is not None or _forward_ad._current_level >= 0:
+            or _transforms() is not None or _forward_ad._current_level >= 0 \
+            or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") is not dtype):
         return None
     # a table that was calibrated on this box says how the library runs these projections
     if (N, K) in getattr(_LIBRARY_ROWS, "calibrated", ()):

@@ -142,3 +142,22 @@ def test_function_modes_see_the_product(monkeypatch):
     """a mode that overrides torch's functions finds the library's product; the one that only says where new tensors go hides none"""
     assert not _own_product(monkeypatch, within=_Counting)
     assert _own_product(monkeypatch, within=lambda: torch.device("cpu"))
+
+
+@contextlib.contextmanager
+def _autocast(dtype):
+    """torch.autocast("cuda", dtype) where there is no GPU for it to ask"""
+    enabled, before = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
+    torch.set_autocast_enabled("cuda", True)
+    torch.set_autocast_dtype("cuda", dtype)
+    try:
+        yield
+    finally:
+        torch.set_autocast_enabled("cuda", enabled)
+        torch.set_autocast_dtype("cuda", before)
+
+
+def test_autocast_to_the_other_type_is_the_librarys(monkeypatch):
+    for dtype, other in ((torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16)):
+        assert not _own_product(monkeypatch, dtype=dtype, within=lambda: _autocast(other))
+        assert _own_product(monkeypatch, dtype=dtype, within=lambda: _autocast(dtype))

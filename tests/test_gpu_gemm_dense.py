@@ -138,3 +138,10 @@ def test_function_modes_find_the_librarys_product():
     with Mode():
         _native.linear(x, w)
     assert torch.nn.functional.linear in seen
+
+
+def test_autocast_to_the_other_type_is_the_librarys():
+    from scratchpad_amd import _native
+    x, w = torch.randn(64, 1024, device="cuda").bfloat16(), torch.randn(1024, 1024, device="cuda").bfloat16()
+    with torch.autocast("cuda", torch.float16):
+        assert _native.linear(x, w).dtype == torch.float16
