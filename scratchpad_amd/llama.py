@@ -15,6 +15,7 @@ from typing import Any, Dict, Iterable, Optional, Tuple
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _native
 from .attention import RadixAttention
@@ -357,6 +358,12 @@ class LogitsProcessor(nn.Module):
 
 
 # --------------------------------------------------------------------------- decoder
+def _runs_only(module: nn.Module, cls: type) -> bool:
+    """calling the module runs cls.forward and nothing of a user's: no hooks, no other module or forward in its place"""
+    return type(module) is cls and "forward" not in module.__dict__ and not (
+        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or _has_any_global_hook())
+
+
 class LlamaMLP(nn.Module):
     def __init__(self, hidden_size: int, intermediate_size: int, hidden_act: str, dtype=None):
         super().__init__()
@@ -367,11 +374,13 @@ class LlamaMLP(nn.Module):
         self.act_fn = SiluAndMul()
 
     def forward(self, x, reduce_output: bool = True):
-        # small decode steps (<= _native.SILU_FUSED_MAX_ROWS tokens): projection and activation in one weight-streaming launch, the bits of
-        # the skinny projection followed by act_fn; steps of 17 rows and more likewise where the tiled kernel takes the projection
-        act = _native.linear_silu_mul(x, self.gate_up_proj.weight)
-        if act is None:
-            act = _native.dense_silu_mul(x, self.gate_up_proj.weight)
+        # projection and activation in one launch: small decode steps (<= _native.SILU_FUSED_MAX_ROWS tokens) by the weight-streaming
+        # kernel, 17 rows and more (5 and more over large weights) where the tiled kernel takes the projection
+        act = None
+        if _runs_only(self.gate_up_proj, MergedColumnParallelLinear) and _runs_only(self.act_fn, SiluAndMul):
+            act = _native.linear_silu_mul(x, self.gate_up_proj.weight)
+            if act is None:
+                act = _native.dense_silu_mul(x, self.gate_up_proj.weight)
         if act is None:
             gate_up, _ = self.gate_up_proj(x)
             act = self.act_fn(gate_up)

@@ -161,3 +161,57 @@ def test_autocast_to_the_other_type_is_the_librarys(monkeypatch):
     for dtype, other in ((torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16)):
         assert not _own_product(monkeypatch, dtype=dtype, within=lambda: _autocast(other))
         assert _own_product(monkeypatch, dtype=dtype, within=lambda: _autocast(dtype))
+
+
+def _touch(kind, mlp, seen):
+    """something of a user's that calling gate_up_proj or act_fn runs"""
+    note = lambda *a: seen.append(kind)                            # noqa: E731
+    if kind == "forward hook":
+        mlp.gate_up_proj.register_forward_hook(lambda m, a, out: note())
+    elif kind == "pre-hook":
+        mlp.gate_up_proj.register_forward_pre_hook(lambda m, a: note())
+    elif kind == "activation's hook":
+        mlp.act_fn.register_forward_hook(lambda m, a, out: note())
+    elif kind == "hook of all modules":
+        return torch.nn.modules.module.register_module_forward_hook(lambda m, a, out: note())
+    elif kind == "its own forward":
+        before = mlp.gate_up_proj.forward
+        mlp.gate_up_proj.forward = lambda x: (note(), before(x))[1]
+    else:                                                           # another module in its place
+        class Adapter(torch.nn.Module):
+            def __init__(self, inner):
+                super().__init__()
+                self.inner, self.weight = inner, inner.weight
+
+            def forward(self, x):
+                note()
+                return self.inner(x)
+
+        mlp.gate_up_proj = Adapter(mlp.gate_up_proj)
+
+
+@pytest.mark.parametrize("kind", ["forward hook", "pre-hook", "activation's hook", "hook of all modules", "its own forward", "adapter"])
+@pytest.mark.parametrize("rows", [5, 9, 64])
+def test_fused_mlp_passes_by_nothing_that_its_modules_would_run(monkeypatch, kind, rows):
+    from scratchpad_amd import _native, distributed
+    from scratchpad_amd.llama import LlamaMLP
+    if not distributed.model_parallel_is_initialized():
+        distributed.initialize_model_parallel(1)
+    fused = []
+    one_launch = lambda x, w: fused.append(1) or x.new_zeros(x.shape[0], w.shape[0] // 2)          # noqa: E731
+    monkeypatch.setattr(_native, "linear_silu_mul", lambda x, w: one_launch(x, w) if x.shape[0] <= 8 else None)
+    monkeypatch.setattr(_native, "dense_silu_mul", one_launch)
+    monkeypatch.setattr(_native, "silu_and_mul", lambda x: x[:, :x.shape[1] // 2])
+    mlp = LlamaMLP(64, 96, "silu", torch.float32)
+    for p in mlp.parameters():
+        p.data.zero_()
+    mlp(torch.zeros(rows, 64))
+    assert fused == [1]
+    seen = []
+    handle = _touch(kind, mlp, seen)
+    try:
+        mlp(torch.zeros(rows, 64))
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert seen and fused == [1]
