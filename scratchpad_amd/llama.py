@@ -376,14 +376,15 @@ class LlamaMLP(nn.Module):
     def forward(self, x, reduce_output: bool = True):
         # projection and activation in one launch: small decode steps (<= _native.SILU_FUSED_MAX_ROWS tokens) by the weight-streaming
         # kernel, 17 rows and more (5 and more over large weights) where the tiled kernel takes the projection
-        act = None
-        if _runs_only(self.gate_up_proj, MergedColumnParallelLinear) and _runs_only(self.act_fn, SiluAndMul):
-            act = _native.linear_silu_mul(x, self.gate_up_proj.weight)
+        project, act_fn, act = self.gate_up_proj, self.act_fn, None
+        if _runs_only(project, MergedColumnParallelLinear) and _runs_only(act_fn, SiluAndMul):
+            weight = project.weight
+            act = _native.linear_silu_mul(x, weight)
             if act is None:
-                act = _native.dense_silu_mul(x, self.gate_up_proj.weight)
+                act = _native.dense_silu_mul(x, weight)
         if act is None:
-            gate_up, _ = self.gate_up_proj(x)
-            act = self.act_fn(gate_up)
+            gate_up, _ = project(x)
+            act = act_fn(gate_up)
         x, _ = self.down_proj(act, reduce_output)
         return x
 
