@@ -1089,8 +1089,10 @@ SILU_FUSED_MAX_ROWS = 8
 def linear_silu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor, any_rows: bool = False) -> Optional[torch.Tensor]:
     """SiluAndMul(x @ gate_up_weight.T) as ONE launch (sp_gemm_skinny, epilogue 1) for a step of at most
     SILU_FUSED_MAX_ROWS tokens (any_rows: up to the kernel's 16): x [M, K], gate_up_weight [2 I, K] (gate rows first),
-    result [M, I].  Bit for bit ``linear`` followed by silu_and_mul; with any_rows the skinny projection whatever its size, else
-    sp_gemm_dense where linear would take it.  None when the shape is not taken (the caller runs the two steps)."""
+    result [M, I].  Bit for bit the sp_gemm_skinny projection followed by silu_and_mul, except that (without any_rows) a projection that
+    sp_gemm_dense runs with the activation in its epilogue is that one, bit for bit ``linear`` followed by silu_and_mul.  (``linear`` itself
+    hands some projections of few rows to other kernels: those whose K sp_gemm_dense shares out, and what skinny_gemm_pays leaves to the
+    library.)  None when the shape is not taken (the caller runs the two steps)."""
     if not any_rows and x.dim() == 2 and 4 < x.shape[0] <= SILU_FUSED_MAX_ROWS and gate_up_weight.numel() > 1 << 23:
         out = dense_silu_mul(x, gate_up_weight)
         if out is not None:
@@ -1105,8 +1107,8 @@ def dense_silu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> Optional[to
 
 
 def linear_gelu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.Tensor:
-    """gelu_tanh(x @ gate.T) * (x @ up.T) of the merged matrix [gate | up]: one launch for a step of few tokens, the product and
-    gelu_tanh_and_mul one after the other elsewhere (the same bits)"""
+    """gelu_tanh(x @ gate.T) * (x @ up.T) of the merged matrix [gate | up]: one launch for a step of few tokens (bit for bit the
+    sp_gemm_skinny projection followed by gelu_tanh_and_mul), ``linear`` and gelu_tanh_and_mul one after the other elsewhere"""
     out = _skinny_glu(x, gate_up_weight, False, 3, "sp_gemm_skinny(gelu)")
     return gelu_tanh_and_mul(linear(x, gate_up_weight)) if out is None else out
 
@@ -1186,8 +1188,8 @@ def _feeds_a_measured_shape(width: int) -> bool:
 
 
 def linear_relu_square(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """max(x @ weight.T, 0)^2: one launch where ``linear`` would take the weight-streaming kernel (the square is taken of the
-    fp32 sum), the product and the activation one after the other elsewhere"""
+    """max(x @ weight.T, 0)^2: one launch where the weight-streaming kernel takes the product and is faster than the library (the square is
+    taken of the fp32 sum), the product and the activation one after the other elsewhere"""
     if _skinny_takes(x, weight):
         M, K = x.shape
         N = weight.shape[0]

@@ -145,3 +145,21 @@ def test_autocast_to_the_other_type_is_the_librarys():
     x, w = torch.randn(64, 1024, device="cuda").bfloat16(), torch.randn(1024, 1024, device="cuda").bfloat16()
     with torch.autocast("cuda", torch.float16):
         assert _native.linear(x, w).dtype == torch.float16
+
+
+@pytest.mark.parametrize("N, K", [(4096, 6144), (6144, 8192), (18944, 14336), (6144, 2048), (4096, 4096), (28672, 4096), (2048, 1024)])
+def test_silu_of_a_projection_has_the_bits_of_two_steps(N, K):
+    """at the rows of small decode steps: of linear's product where sp_gemm_dense has the activation in its epilogue, else of sp_gemm_skinny's - also
+    where linear takes neither (K that sp_gemm_dense shares out, K past 8192 at 1 - 4 rows)"""
+    from scratchpad_amd import _native
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    w = torch.randn(N, K, generator=g, device="cuda").mul_(0.05).bfloat16()
+    for M in (1, 2, 4, 5, 7, 8):
+        x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+        if _native._dense_plan(M, N, K, 1) >= 0:
+            plain = _native.linear(x, w)
+        else:
+            plain = torch.empty(M, N, dtype=x.dtype, device="cuda")
+            _native._check(_native.load().sp_gemm_skinny(plain.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, K, K, N, 0, _native._dt(x),
+                                                         _native._stream()), "sp_gemm_skinny")
+        assert torch.equal(_native.linear_silu_mul(x, w), _native.silu_and_mul(plain)), M
