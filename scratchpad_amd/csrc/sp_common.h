@@ -141,11 +141,14 @@ __device__ __forceinline__ u32x4 pack16<f16_tag>(const float* f) {
   return v;
 }
 
-// n / (1 + expf(-z)) in 18 instructions instead of 25 (4096 x 6144 SiLUs of a convolution: 43.8 -> 38.7 us): the exponential without its
-// checks of the range, which one median makes unnecessary, and the quotient from a reciprocal and one correction, without a division's
-// scaling - the denominator is at least 1, and its reciprocal is taken of a quarter of it, so that it is no denormal.  Measured over all 2^32
+// n / (1 + expf(-z)) in 18 instructions instead of 25 (4096 x 6144 SiLUs of a convolution: 43.8 -> 38.7 us).  The exponential by Cody and Waite's
+// reduction (the argument times log2 e in two floats, its nearest whole by ldexp, the rest by the hardware's exp2), without checks of the range, which
+// one median makes unnecessary; the quotient by a reciprocal and one step of Newton's iteration on the quotient (Markstein's), without a
+// division's scaling - the denominator is at least 1, and its reciprocal is taken of a quarter of it, so that it is no denormal.  Measured over all 2^32
 // values of z: with n = z the bits of __fdiv_rn(n, __fadd_rn(1, expf(-z))) but for 15, the next float there, with n = 1 but for 14; errors against 64
-// bits the same (largest 2.72 ulp, means 0.34 - 0.49 by magnitude).  Quotients that are denormal may be the next denormal.
+// bits the same (largest 2.72 ulp, means 0.34 - 0.49 by magnitude).  Other numerators, 67 M draws of each range: at most one result in 10^6 differs, by one ulp,
+// and errors are the same to six digits (n of 2^-6 .. 2^6 and 2^-100 .. 2^126; mean 0.31 - 0.38, largest 2.66), but for n below 2^-90, whose
+// quotients come near the denormals (mean 0.2752 -> 0.2755, largest 2.099 -> 2.100).  Quotients that are denormal may be the next denormal.
 __device__ __forceinline__ float over_one_plus_exp(float n, float z) {
 #pragma clang fp contract(off)
   const float L = 1.44269502162933349609375f, Llow = 1.925963033500011079e-08f;              // log2(e) in two floats
