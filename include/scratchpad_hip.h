@@ -516,6 +516,10 @@ SP_API int sp_moe_grouped_gemm(void* out, const void* a, const void* w, const in
 SP_API int sp_moe_grouped_glu(void* out, const void* a, const void* w, const int32_t* offsets, const int32_t* order,
                               int row_div, int pairs, int ff, int k, int experts, int64_t a_stride, int64_t out_stride,
                               int act, float limit, float alpha, int dtype, void* stream);
+/* Host code: the kernel that a product of 16-bit types and aligned rows takes, by sizes alone: 0 a wave per 16 rows, 1 the same with half the
+ * weight rows, 2 / 3 tiles of 64 / 128 rows, 4 of 128 x 256, 16 + i the i-th tile of the LDS rings; -1: sizes that they do not take.  gated: n output
+ * columns of 2 n weight rows; row_div: of an order, 0 without one.                                                       */
+SP_API int sp_moe_grouped_plan(int gated, int row_div, int pairs, int n, int k, int experts, int64_t a_stride);
 /* out[p, f] = g * sigmoid(alpha g) * (u + 1), g = min(gu[p, f], limit), u = clamp(gu[p, ff + f], -limit, limit) */
 SP_API int sp_moe_glu(void* out, const void* gu, int64_t pairs, int ff, float limit, float alpha, int dtype, void* stream);
 /* out[t] = sum over k < top, in that order, of weights[t, k] * z[place[t * top + k]] */

@@ -313,7 +313,7 @@ moe_grouped_gemm_kernel(void* out, const void* a, const void* w, const int32_t* 
 // ---- the same product on the matrix cores (16-bit types, K a multiple of 32, 16-byte aligned rows) -------------------
 // v_mfma_f32_16x16x32: lane (r16 = lane & 15, q = lane >> 4) holds 8 k-values of row r16 of each operand and receives
 // D[4 q + r][r16], r < 4 - with the weights as the first operand a lane ends up with 4 neighbouring output columns of ONE
-// row.  The kernels below (tile, ring, rows, narrow rows) add the k-steps of 32 in ascending order into one accumulator, so an output
+// row.  The kernels below (tile, ring, wide, rows, narrow rows) add the k-steps of 32 in ascending order into one accumulator, so an output
 // element has the same bits whichever of them - and whichever tile height - computes it: a token's result does not depend on the
 // step's size.
 //
@@ -752,6 +752,106 @@ inline int ring_tile(int pairs, int experts, int64_t wrows, int K) {
   return best;
 }
 
+// Gated products of hundreds of rows per expert, and plain ones whose K the ring does not take: 128 rows x 256 weight rows per workgroup, a wave
+// 64 x 128 of them, k in steps of 32, any K that is a multiple of 32.  What the 128 x 128 tiles wait for is LDS (a wave reads 8 KB for 16 products of
+// 16 cycles: 128 bytes per cycle for the four of them, all there is) and the L2 (64 bytes per cycle and CU); here it is 96 and 48.  A step's operands
+// are 24 KB, double-buffered, so three workgroups share a CU and fill each other's waits.  The row tiles of one column tile follow each other: the
+// weights they share are in the L2 once.  LDS rows are 64 bytes; the chunk of a row is permuted by its number / 4, so that the 16 rows of a
+// fragment read lie in 64 banks.
+// Against the ring's tiles, gated, past a mean of 320 rows, 67 sizes (4 to 256 experts, widths 1024 to 7168), each routed evenly, by expert weights
+// of spread e^0.5 and by 1 / rank: the ring 0.67 - 1.8 of this one's speed, 2 % faster on average but more than 5 % slower in 70 of 201, where
+// counts above 192 or 384 rows cost a row tile more.  Width 2048, 32 experts of ff 1024, up product in us, ring | this, evenly and by weights: 4096 tokens
+// 170 | 186, 195 | 180; 6000: 256 | 251, 296 | 251; 8192: 323 | 318, 322 | 320.
+constexpr int kWideBM = 128, kWideBN = 256, kWideBK = 32;
+template <typename Tag, int ACT>
+__global__ void __launch_bounds__(256, 3) moe_grouped_wide_kernel(GroupedArgs p) {
+  constexpr bool GLU = ACT >= 2;
+  constexpr int CPW = kWideBN / 2, FM = 4, FN = CPW / 16, OUT_N = GLU ? kWideBN / 2 : kWideBN;
+  constexpr int LA = kWideBM / 64, LB = kWideBN / 64;            // direct loads per wave and step
+  constexpr int kBuf = (kWideBM + kWideBN) * kWideBK * 2;
+  extern __shared__ __attribute__((aligned(16))) char wide_lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+  const int ntiles = (p.N + OUT_N - 1) / OUT_N;
+  const int total = grouped_tiles(p.offsets, p.E, kWideBM, lane) * ntiles, share = (total + 7) / 8;
+  const int idx = (int)(blockIdx.x >> 3), at = (int)(blockIdx.x & 7) * share + idx;
+  if (idx >= share || at >= total) return;
+  int e = 0, row0 = 0, rows_end = 0, col = 0, row_tiles = 0;
+  if (!grouped_tile_by_column(p.offsets, p.E, kWideBM, ntiles, at, lane, e, row0, rows_end, col, row_tiles)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  const int n0 = col * OUT_N;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int wrows = GLU ? 2 * p.N : p.N;
+  // sources of this wave's direct loads: lane -> row lane / 4 of the 16 rows of a load, chunk lane % 4 of LDS
+  const int chunk = (lane & 3) ^ (lane >> 4);
+  const char* src[LA + LB];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) {
+    const int pos = min(row0 + (wave * LA + i) * 16 + (lane >> 2), rows_end - 1);     // rows past the end: never stored
+    const int64_t arow = p.order ? p.order[pos] / p.row_div : pos;
+    src[i] = p.a + arow * p.a_stride * 2 + chunk * 16;
+  }
+  const char* wbase = p.w + (int64_t)e * wrows * p.K * 2 + chunk * 16;
+#pragma unroll
+  for (int i = 0; i < LB; ++i) {
+    const int br = (wave * LB + i) * 16 + (lane >> 2);
+    int row;
+    if constexpr (GLU) {
+      const int in = br % CPW, n = n0 + (br / CPW) * (CPW / 2) + in % (CPW / 2);
+      row = min(n, p.N - 1) + (in >= CPW / 2 ? p.N : 0);
+    } else {
+      row = min(n0 + br, p.N - 1);
+    }
+    src[LA + i] = wbase + (int64_t)row * p.K * 2;
+  }
+  const int steps = p.K / kWideBK;
+  const auto stage = [&](char* lds, int step) {
+#pragma unroll
+    for (int i = 0; i < LA + LB; ++i) {
+      char* dst = lds + (i < LA ? (wave * LA + i) : (kWideBM / 16 + wave * LB + i - LA)) * 1024;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + step * (kWideBK * 2)),
+                                       (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    }
+  };
+  f32x4_q acc[FM][FN];
+#pragma unroll
+  for (int f = 0; f < FM; ++f)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[f][j] = f32x4_q{0.f, 0.f, 0.f, 0.f};
+  const int c = (q ^ (r16 >> 2)) * 16;
+  const int arow0 = (wm * 64 + r16) * 64 + c, brow0 = (kWideBM + wn * CPW + r16) * 64 + c;
+  char *now = wide_lds, *next = wide_lds + kBuf;
+  stage(now, 0);
+  for (int s = 0; s < steps; ++s) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (s + 1 < steps) stage(next, s + 1);
+    u32x4 xf[FM], wf[FN];
+#pragma unroll
+    for (int f = 0; f < FM; ++f) xf[f] = ld16(now + arow0 + f * 1024);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) wf[j] = ld16(now + brow0 + j * 1024);
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int f = 0; f < FM; ++f) acc[f][j] = mfma_q<Tag>(wf[j], xf[f], acc[f][j]);
+    char* const t = now;
+    now = next, next = t;
+  }
+  constexpr int FO = GLU ? FN / 2 : FN;
+#pragma unroll
+  for (int f = 0; f < FM; ++f) {
+    const int pos = row0 + wm * 64 + 16 * f + r16;
+    if (pos >= rows_end) continue;
+#pragma unroll
+    for (int j = 0; j < FO; ++j) {
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = grouped_act<Tag, ACT>(acc[f][j][r], GLU ? acc[f][j + FN - FO][r] : 0.f, p);
+      store4<Tag>(p, pos, n0 + wn * (GLU ? CPW / 2 : CPW) + 16 * j + 4 * q, v);
+    }
+  }
+}
+
 // Steps with a few rows per expert (decode): a stream of the chosen experts' weights.  One wave per 16 rows x 32 weight rows
 // (GLU: 16 gate rows and their 16 up rows), operands straight from global memory, kRowsUnroll k-steps of loads in flight.
 // Single waves spread evenly over the 1024 SIMDs whatever the number of chosen experts; nothing is shared between them.
@@ -870,43 +970,71 @@ static bool narrow_pays(int pairs, int experts, int blocks) {
 //     38 + 18; 32 experts of ff 1024, 3: 63 + 27 | 55 + 24, 16: 67 + 28 (64-row tiles) | 55 + 23; 128 of 512, width 1024, 4: 50 + 28 | 45 + 26;
 //   * 10 where it is at most one wave per SIMD: width 1024, 16 experts of ff 512, mean 2: 9.2 + 6.7 | 10.5 + 7.3, 10: 10.0 + 7.0 | 10.5 + 7.7; 32 experts,
 //     2 - 8: 14.5 + 9.2 | 15.0 + 9.6; 8 of 1536, width 2048, 2: 24.6 + 11.5 | 26.4 + 12.7, 10: 22.9 + 12.3 | 23.7 + 12.1 - and 12: 35 + 20 | 24 + 12;
-//   * 10 where the ring does not take the product (K no multiple of 64, 2^31 bytes of offsets), the 64-row tiles from there.
-// Else the ring tiles, the tile by ring_tile.  The mean says nothing of a skewed step.  Every pair on top_k experts, both products together, the
-// kernels and rules before -> these: 32 experts of ff 1024, 24 tokens 25.4 -> 29.2, 48: 33.3 -> 22.5, 200: 42.2 -> 31.8, 1000: 66.6 -> 72.3; 128 of 1536,
-// width 4096, 200: 114 -> 143, 800: 405 -> 316 (a tile chosen for fewer rows than there are reads an expert's weights more often).
-template <typename Tag, int ACT>
-int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
-  const int held = pairs < p.E ? pairs : p.E;                    // experts with a row, at most
+//   * 10 where the ring does not take the product (K no multiple of 64, 2^31 bytes of offsets), the 64-row tiles from there, the 128-row tiles from 56.
+// Else the ring tiles, the tile by ring_tile, and from a mean of 320 rows on the wide kernel for gated products (its comment has both sides) and for
+// what the ring does not take (K of 1056, 512 rows: 379 by the 128-row tiles, 337 by it, both of K 1024).
+// The mean says nothing of a skewed step: a row tile chosen for the mean may be taller than most experts' rows, or one row too short for some.  Over 350
+// sizes (4 to 256 experts, widths 1024 to 7168, means 1 to 2000), each routed evenly, by expert weights of spread e^0.5 and by 1 / rank, against the
+// kernels before (64 x 128, 128 x 128 and 128 x 256 tiles, one wave per 16 rows): up products 1.16 and down products 1.16 times as fast on average, one in
+// twenty more than 5 % slower (0.60 - 0.95; 16 experts, width 2560, mean 135, by 1 / rank: 18 -> 30), most of them at means just below a tile's height.
+// No choice by sizes alone does better: costs fitted to uneven routings, or expected counts spread by any width, lose as often.  Every pair on
+// top_k experts, both products together: 32 experts of ff 1024, 24 tokens 25.4 -> 29.2, 48: 33.3 -> 22.5, 200: 42.2 -> 31.8; 128 of 1536, width 4096,
+// 200: 114 -> 143, 800: 405 -> 316.
+// (sizes alone: the plan is the same for every step of them)
+enum : int { kGroupedRows = 0, kGroupedNarrow = 1, kGrouped64 = 2, kGrouped128 = 3, kGroupedWide = 4, kGroupedRing = 16 };      // + its tile
+inline int grouped_plan(bool gated, bool ordered, int row_div, int pairs, int n, int k, int experts, int64_t a_stride) {
+  const int held = pairs < experts ? pairs : experts;           // experts with a row, at most
   const int row_tiles = pairs / 16 + held;
   // (moe_align takes 4096 experts, 6656 tiles; more than a grid's second dimension holds go to the 64-row tiles)
   // (a ring's loads have 32-bit offsets from the operand's first byte; rows further on that an order names: far_product)
-  const int64_t last_row = p.order ? (int64_t)pairs / p.row_div + 1 : pairs;
-  const bool ring = p.K % 64 == 0 && last_row * p.a_stride < (int64_t)1 << 31 && (ACT >= 2 ? 2 : 1) * (int64_t)p.N * p.K < (int64_t)1 << 31;
-  const int wide_per = ACT >= 2 ? 16 : 32, blocks_of_rows = (p.N + wide_per - 1) / wide_per;
-  const double wrows = p.E * (1. - exp(-(double)pairs / p.E)) * (ACT >= 2 ? 2. : 1.) * p.N;                  // of the experts expected to be chosen
-  const bool streams = wrows * p.K >= 110e6 && wrows >= 700. * 64.;
-  const int most = !ring ? 20 : streams ? 0 : (int64_t)p.E * blocks_of_rows > 1024 ? 3 : 20;              // half rows per expert
-  if (2 * (int64_t)pairs <= most * (int64_t)p.E && row_tiles <= 65535) {
-    const bool narrow = narrow_pays(pairs, p.E, blocks_of_rows);
-    const int per = narrow ? wide_per / 2 : wide_per;
-    const dim3 grid((unsigned)((p.N + per - 1) / per), (unsigned)row_tiles);
-    if (narrow) moe_grouped_narrow_rows_kernel<Tag, ACT><<<grid, 64, 0, st>>>(p);
+  const int64_t last_row = ordered ? (int64_t)pairs / row_div + 1 : pairs, wide_rows = (gated ? 2 : 1) * (int64_t)n;
+  const bool ring = k % 64 == 0 && last_row * a_stride < (int64_t)1 << 31 && wide_rows * k < (int64_t)1 << 31;
+  const int blocks_of_rows = (n + (gated ? 15 : 31)) / (gated ? 16 : 32);
+  const double wrows = experts * (1. - exp(-(double)pairs / experts)) * wide_rows;                  // of the experts expected to be chosen
+  const bool streams = wrows * k >= 110e6 && wrows >= 700. * 64.;
+  const int most = !ring ? 20 : streams ? 0 : (int64_t)experts * blocks_of_rows > 1024 ? 3 : 20;      // half rows per expert
+  if (2 * (int64_t)pairs <= most * (int64_t)experts && row_tiles <= 65535) return narrow_pays(pairs, experts, blocks_of_rows) ? kGroupedNarrow : kGroupedRows;
+  if (pairs > 320 * (int64_t)experts && (gated || !ring)) return kGroupedWide;
+  if (ring) return kGroupedRing + ring_tile(pairs, experts, wide_rows, k);
+  return pairs > 56 * (int64_t)experts ? kGrouped128 : kGrouped64;
+}
+
+template <typename Tag, int ACT>
+int launch_grouped_mfma(const GroupedArgs& p, int pairs, hipStream_t st) {
+  const int held = pairs < p.E ? pairs : p.E;
+  const int plan = grouped_plan(ACT >= 2, p.order, p.row_div, pairs, p.N, p.K, p.E, p.a_stride);
+  if (plan == kGroupedRows || plan == kGroupedNarrow) {
+    const int per = (ACT >= 2 ? 16 : 32) / (plan == kGroupedNarrow ? 2 : 1);
+    const dim3 grid((unsigned)((p.N + per - 1) / per), (unsigned)(pairs / 16 + held));
+    if (plan == kGroupedNarrow) moe_grouped_narrow_rows_kernel<Tag, ACT><<<grid, 64, 0, st>>>(p);
     else moe_grouped_rows_kernel<Tag, ACT><<<grid, 64, 0, st>>>(p);
     SP_LAUNCH_CHECK();
     return SP_OK;
   }
-  if (ring) {
+  if (plan >= kGroupedRing) {
 #define SP_RING_CASE(I, TWO, ONE, FIXED, ONCE, ...) \
   case I: return launch_grouped_ring<Tag, RingTile<__VA_ARGS__>, ONCE, ACT>(p, pairs, held, st);
-    switch (ring_tile(pairs, p.E, (ACT >= 2 ? 2 : 1) * (int64_t)p.N, p.K)) { SP_RING_TILES(SP_RING_CASE) }
+    switch (plan - kGroupedRing) { SP_RING_TILES(SP_RING_CASE) }
     return SP_ERR_INVALID_ARG;
   }
-  const int per = ACT >= 2 ? kGroupedBN / 2 : kGroupedBN;
+  const int bm = plan == kGrouped64 ? 64 : 128, bn = plan == kGroupedWide ? kWideBN : kGroupedBN, per = ACT >= 2 ? bn / 2 : bn;
   const int64_t ntiles = (p.N + per - 1) / per;
-  const int bm = pairs > 56 * (int64_t)p.E ? 128 : 64;
-  const unsigned blocks = (unsigned)(((pairs / bm + held) * ntiles + 7) / 8 * 8);
-  if (bm == 128) moe_grouped_tile_kernel<Tag, 128, ACT><<<dim3(blocks), 256, 0, st>>>(p);
-  else moe_grouped_tile_kernel<Tag, 64, ACT><<<dim3(blocks), 256, 0, st>>>(p);
+  const dim3 blocks((unsigned)(((pairs / bm + held) * ntiles + 7) / 8 * 8));
+  if (plan == kGroupedWide) {
+    constexpr int lds = 2 * (kWideBM + kWideBN) * kWideBK * 2;
+    static PerDevice<int> raised;
+    int ok = 0;
+    raised.get(ok, [&](int) {
+      return hipFuncSetAttribute((const void*)moe_grouped_wide_kernel<Tag, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) ==
+             hipSuccess ? 1 : 0;
+    });
+    if (!ok) return SP_ERR_LAUNCH;
+    moe_grouped_wide_kernel<Tag, ACT><<<blocks, 256, lds, st>>>(p);
+  } else if (plan == kGrouped128) {
+    moe_grouped_tile_kernel<Tag, 128, ACT><<<blocks, 256, 0, st>>>(p);
+  } else {
+    moe_grouped_tile_kernel<Tag, 64, ACT><<<blocks, 256, 0, st>>>(p);
+  }
   SP_LAUNCH_CHECK();
   return SP_OK;
 }
@@ -1064,6 +1192,11 @@ extern "C" int sp_moe_grouped_glu(void* out, const void* a, const void* w, const
   if (dtype == SP_BF16)
     return act ? launch_grouped_mfma<bf16_tag, 3>(p, pairs, st) : launch_grouped_mfma<bf16_tag, 2>(p, pairs, st);
   return act ? launch_grouped_mfma<f16_tag, 3>(p, pairs, st) : launch_grouped_mfma<f16_tag, 2>(p, pairs, st);
+}
+
+extern "C" int sp_moe_grouped_plan(int gated, int row_div, int pairs, int n, int k, int experts, int64_t a_stride) {
+  if (pairs <= 0 || n <= 0 || k <= 0 || k % 32 || experts <= 0 || row_div < 0 || a_stride < k || a_stride % 8) return -1;
+  return grouped_plan(gated != 0, row_div > 0, row_div, pairs, n, k, experts, a_stride);
 }
 
 extern "C" int sp_moe_glu(void* out, const void* gu, int64_t pairs, int ff, float limit, float alpha, int dtype,
