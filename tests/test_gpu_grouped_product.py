@@ -130,15 +130,27 @@ def test_combine(T, width, top, dtype):
 
 
 # (experts, mean rows, weight rows, K): the sizes at which each of the ring kernel's ten tiles is the one taken, K of fewer steps than a ring holds and more
-RING = [(2, 16, 128, 64), (8, 30, 200, 192), (2, 8, 128, 512), (2, 100, 128, 512), (32, 300, 200, 64), (32, 200, 384, 320), (16, 800, 200, 320),
+RING = [(2, 16, 128, 64), (8, 30, 200, 192), (2, 12, 128, 512), (2, 100, 128, 512), (32, 300, 200, 64), (32, 200, 384, 320), (16, 800, 200, 320),
         (16, 800, 384, 64), (16, 150, 1024, 192), (32, 300, 200, 256), (32, 800, 200, 64), (8, 800, 1024, 64), (32, 500, 512, 64), (8, 500, 2048, 64),
-        (32, 800, 384, 64), (32, 150, 2048, 64), (16, 800, 512, 1024), (4, 800, 2048, 512)]
+        (32, 800, 384, 64), (32, 150, 2048, 64), (16, 800, 512, 1024), (4, 800, 2048, 512),
+        (2, 12, 128, 320), (2, 100, 128, 1024), (32, 40, 1000, 1024), (32, 150, 384, 1024), (2, 60, 128, 512), (32, 80, 1000, 1024),
+        (32, 120, 1000, 1024), (16, 300, 1000, 1024), (32, 180, 1000, 320)]
+
+
+def rows_kernel_share(E, N, K):
+    """of so many pairs, among the experts and as many more without rows, the rows kernel takes both forms: their weights are no stream"""
+    from scratchpad_amd import _native
+    takes = lambda n: all(_native.load().sp_moe_grouped_plan(gated, 2, n, N >> gated, K, E + n, K) in (0, 1) for gated in (0, 1))          # noqa: E731
+    share = max(n for n in (16, 32, 64, 128, 256, 512, 1024, 2048, 4096) if takes(n))
+    assert all(takes(n) for n in range(1, share))
+    return share
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("E,mean,N,K", RING)
 def test_ring_tiles_have_the_bits_of_the_rows_kernel(E, mean, N, K, dtype):
-    """the same rows among so many experts without any that the rows kernel takes them; uneven experts, one without rows and one with one"""
+    """the same rows a share at a time, among so many experts without any that the rows kernel takes them; uneven experts, one without rows and
+    one with one"""
     from scratchpad_amd import _native
     print("ring", E, mean, N, K, dtype, flush=True)
     counts = [mean] * E
@@ -146,19 +158,32 @@ def test_ring_tiles_have_the_bits_of_the_rows_kernel(E, mean, N, K, dtype):
     if E > 2:
         counts[2], counts[3] = 0, 2 * mean
     a, w, offsets, order, expert, P = grouped_inputs(counts, N, K, dtype, 2, seed=7)
-    many = torch.empty(E + P, N, K, dtype=dtype, device=DEV)                   # (experts without rows are not read)
+    plans = [_native.load().sp_moe_grouped_plan(gated, 2, P, N >> gated, K, E, K) for gated in (0, 1)]
+    assert plans[0] >= 16 and plans[1] >= (16 if mean <= 320 else 4)
+    share = rows_kernel_share(E, N, K)
+    many = torch.empty(E + share, N, K, dtype=dtype, device=DEV)               # (experts without rows are not read)
     many[:E] = w
-    more = torch.cat([offsets, offsets[-1:].expand(P)]).contiguous()
+
+    def by_rows(product):
+        out = []
+        for at in range(0, P, share):
+            n = min(share, P - at)
+            some = (offsets.clamp(at, at + n) - at).to(torch.int32)
+            out.append(product(torch.cat([some, some[-1:].expand(n)]).contiguous(), many[:E + n], n, order[at:at + n]))
+        return torch.cat(out)
+
     got = _native.moe_grouped_gemm(a, w, offsets, P, order, 2)
-    assert torch.equal(got, _native.moe_grouped_gemm(a, many, more, P, order, 2))
+    assert torch.equal(got, by_rows(lambda o, m, n, rows: _native.moe_grouped_gemm(a, m, o, n, rows, 2)))
     rows = a[(order // 2).long()].float()
     want = torch.cat([rows[expert == e] @ w[e].float().t() for e in range(E)])
     scale = rows.abs().max() * w.float().abs().sum(-1).max()
     bar = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11                  # as in test_grouped_products
     assert ((got.float() - want).abs() <= 2 * bar * want.abs() + K * 2.0 ** -22 * scale).all()
-    assert torch.equal(_native.moe_grouped_gemm(a, w, offsets, P, order, 2, act="relu2"), _native.moe_grouped_gemm(a, many, more, P, order, 2, act="relu2"))
+    assert torch.equal(_native.moe_grouped_gemm(a, w, offsets, P, order, 2, act="relu2"),
+                       by_rows(lambda o, m, n, rows: _native.moe_grouped_gemm(a, m, o, n, rows, 2, act="relu2")))
     for act in (("silu",), ("clamped", 2.0, 1.702)):
-        assert torch.equal(_native.moe_grouped_glu(a, w, offsets, P, order, 2, *act), _native.moe_grouped_glu(a, many, more, P, order, 2, *act))
+        assert torch.equal(_native.moe_grouped_glu(a, w, offsets, P, order, 2, *act),
+                           by_rows(lambda o, m, n, rows: _native.moe_grouped_glu(a, m, o, n, rows, 2, *act)))
 
 
 def test_rows_far_from_the_first():
