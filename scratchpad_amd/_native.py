@@ -971,38 +971,42 @@ _forward_ad = torch.autograd.forward_ad
 _tracing = torch._C._get_tracing_state
 _transforms = torch._C._functorch.peek_interpreter_stack
 _dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_stack = torch._C._len_torch_function_stack
+_autocasts = torch._C._is_any_autocast_enabled
+_compiling = torch.compiler.is_compiling
 
 
 def _function_modes() -> bool:
     """under a mode that overrides torch's functions (the one that says where new tensors go, torch.device's, overrides no product)"""
-    return torch._C._len_torch_function_stack() > 0 \
-        and any(type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack())
+    return any(type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack())
 
 
 def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Optional[torch.Tensor]:
     """x @ weight.T (epilogue 1: silu of its first half of columns times its second) by sp_gemm_dense, or None: a product it does not run,
     or not faster than what else would.  Autograd, function transforms, tracing, compilers, modes and casts keep the library call they can see."""
     # (first what keeps tensors of the host, sizes that are no numbers and types that others bring from the library and its table of plans)
-    if not _DENSE_ON or torch.compiler.is_compiling() or not x.is_cuda or type(x) not in _PLAIN or type(weight) not in _PLAIN or _tracing() is not None:
+    if not _DENSE_ON or _compiling() or not x.is_cuda or type(x) not in _PLAIN or type(weight) not in _PLAIN or _tracing() is not None:
         return None
     shape, wshape, dtype = x.shape, weight.shape, x.dtype
     if len(shape) != 2 or len(wshape) != 2 or (dtype is not torch.bfloat16 and dtype is not torch.float16) or weight.dtype is not dtype:
         return None
     M, K = shape
     N = wshape[0]
-    plan = _dense_plan(M, N, K, epilogue)
+    plan = _DENSE_PLANS.get((M, N, K, epilogue))
+    if plan is None:
+        plan = _dense_plan(M, N, K, epilogue)
     # (another device's tensors: the launch would be on the current one's stream)
     if plan < 0 or wshape[1] != K or not x.get_device() == weight.get_device() == torch._C._cuda_getDevice():
         return None
     (xs, x1), (ws, w1) = x.stride(), weight.stride()
     if x1 != 1 or w1 != 1 or xs % 8 or ws % 8 or xs < K or ws < K or M * xs >= 1 << 31 or N * ws >= 1 << 31:
         return None
-    if (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)) or _dispatch_modes() or _function_modes() \
+    if (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)) or _dispatch_modes() or (_function_stack() and _function_modes()) \
             or _transforms() is not None or _forward_ad._current_level >= 0 \
-            or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") is not dtype):
+            or (_autocasts() and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") is not dtype):
         return None
     # a table that was calibrated on this box says how the library runs these projections
-    if (N, K) in getattr(_LIBRARY_ROWS, "calibrated", ()):
+    if type(_LIBRARY_ROWS) is _CalibratedRows and (N, K) in _LIBRARY_ROWS.calibrated:
         return None
     xp, wp = x.data_ptr(), weight.data_ptr()
     if xp % 16 or wp % 16:
@@ -1011,7 +1015,7 @@ def _dense_product(x: torch.Tensor, weight: torch.Tensor, epilogue: int) -> Opti
     out = _rows_like(x, M, cols)
     floats = splits * M * cols if splits > 1 else 0
     sums = torch.empty(floats, dtype=torch.float32, device=x.device) if floats else None
-    _check(load().sp_gemm_dense(out.data_ptr(), xp, wp, _ptr(sums), floats, M, cols, K, xs, ws, cols, epilogue, plan, _dt(x), _stream()),
+    _check(load().sp_gemm_dense(out.data_ptr(), xp, wp, _ptr(sums), floats, M, cols, K, xs, ws, cols, epilogue, plan, _DTYPES[dtype], _stream()),
            "sp_gemm_dense")
     return out
 
