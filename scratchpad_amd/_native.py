@@ -867,63 +867,30 @@ _DENSE_ON = os.environ.get("SP_DENSE_GEMM", "1") != "0"
 _DENSE_PLANS = {}             # (M, weight rows, K, epilogue) -> _dense_plan: sizes alone, at most 1024 row counts per projection
 
 
-# Where the library of _LIBRARY_ROWS_MEASURED_ON is faster than sp_gemm_dense at 17 - 256 rows though the rules of dense_gemm_pays do not say so (its times
-# jump between rows that are multiples of 32 and those that are not).  Of another build nothing is assumed.
-# Weight rows from - to, K from - to, rows from - to, multiples of 32 too; us, library / own.
-_ALL, _BETWEEN = True, False
-_LIBRARY_KEEPS = (
-    (513, 2048, 256, 256, 17, 256, _ALL),                # 1536 x 256, 160 rows 4.3 / 4.8
-    (513, 2048, 2049, 4096, 65, 256, _ALL),              # 2048 x 4096: 64 rows 11.1 / 10.3, 128 10.6 / 11.2
-    (1281, 1984, 4224, 5376, 65, 160, _ALL),             # 1408 x 4608, 72 rows: 0.83 of the library's speed
-    (1345, 1600, 5377, 6400, 129, 160, _ALL),            # 1408 x 6144, 144: 0.84
-    (2049, 2431, 192, 448, 17, 256, _ALL),               # 2304 x 320, 80: 0.89
-    (2049, 2431, 1088, 1279, 193, 224, _ALL),            # 2304 x 1152, 200: 0.89
-    (2049, 2431, 3456, 4480, 33, 192, _ALL),             # 2112 x 4352, 96: 0.85
-    (2049, 2752, 2240, 4224, 33, 63, _ALL),              # 2304 x 3584, 48: 0.75; 2560 x 2560, 40: 0.91
-    (2049, 2752, 2944, 4224, 65, 103, _ALL),             # 2688 x 3072, 96: 0.90
-    (2049, 2752, 1280, 3456, 129, 256, _ALL),            # 2176 x 2560, 200: 0.83
-    (2753, 3456, 1088, 3200, 129, 160, _ALL),            # 2816 x 2560, 144: 0.78; 3072 x 2048 9.6 / 11.5
-    (2753, 3456, 1280, 3200, 161, 208, _BETWEEN),        # 2816 x 3072, 176: 0.87 - and 192: 1.3; 3072 x 2048, 192: 16.1 / 12.1
-    (2753, 3456, 1280, 3200, 209, 256, _ALL),            # 3072 x 2048, 256: 11.0 / 12.2
-    (2753, 3328, 3585, 4608, 129, 160, _ALL),            # 3072 x 4096, 144: 0.86
-    (3457, 4096, 1280, 2816, 129, 208, _BETWEEN),        # 3712 x 2560, 136: 0.85 - and 160: 1.3
-    (3457, 4096, 1280, 2816, 209, 256, _ALL),            # 3968 x 2304, 240: 0.89
-    (4097, 4992, 1216, 2304, 65, 191, _BETWEEN),         # 4352 x 2048, 80: 0.82, 136: 0.91 - and 160: 1.2
-    (4993, 5500, 1216, 1920, 65, 159, _BETWEEN),         # 5376 x 1536, 80: 0.87
-    (4097, 4639, 1664, 2304, 225, 255, _BETWEEN),        # 4352 x 2048, 240: 0.84 - and 256: 1.2
-    (4640, 6784, 1664, 3712, 193, 255, _BETWEEN),        # 6144 x 3072, 240: 0.88 - and 224: 1.2
-    (6785, 8448, 3328, 4352, 193, 255, _BETWEEN),        # 8192 x 4096, 240: 0.93 - and 256: 1.26
-    (8193, 10000, 576, 1152, 129, 191, _ALL),            # 8448 x 1024, 176: 0.83
-    (10001, 10240, 576, 896, 129, 191, _ALL),            # 10240 x 768, 144: 0.85
-    (8193, 10000, 1792, 3328, 129, 159, _ALL),           # 8448 x 3072, 136: 0.90
-    (32769, 53248, 0, 1 << 30, 193, 256, _ALL),          # 49152 x 4096, 256: 0.83; 192: 1.17
-    (53249, 65536, 0, 1 << 30, 161, 256, _ALL),          # 65536 x 1024, 224: 0.80; 160: 1.17
-    (65537, 1 << 30, 0, 2048, 96, 256, _ALL),            # 128256 x 2048: 96 rows 131 / 130, 128 134 / 142, 192 142 / 155
-) if library_versions_match() else ()
-
-
 def dense_gemm_pays(M: int, N: int, K: int) -> bool:
-    """Where sp_gemm_dense measured faster than hipBLASLt on MI355X (us under graph replay, cold weights, library / own).  17 - 256 rows of most
-    shapes (the table in gemm_dense.hip; 16600 pairs of 840 shapes and rows that this takes: 1.22 times as fast on average, one in ninety more than
-    5 % slower, six more than 10 %), but
-    * weight rows up to 512, where it depends on K and rows (512 x 2048 5.5 / 6.7, 512 x 4096 11.7 / 7.1 at 64 rows);
-    * K that is no multiple of 256, below 1600, of up to 2048 weight rows: only the tiles of 64 or 128 steps run and the launch is short (at 64 rows
-      1024 x 576 0.81 of the library's speed, 768 x 704 0.80, 1280 x 1408 0.7 at 48; 1024 x 1664 1.0);
-    * what the library is known to be better at (_LIBRARY_KEEPS).
+    """Where sp_gemm_dense measured faster than what else would run on MI355X: hipBLASLt (or, up to 16 rows, sp_gemm_skinny where that is faster).  us of
+    the device under graph replay, cold weights, library / own; of the host an eager call of the library takes 19.5 us and this one 9, so up to 256
+    rows, where most products take less than that, own products also stand where the device alone would be a little faster with the library's.
+    17 - 256 rows of most shapes (the table in gemm_dense.hip).  21100 pairs of 1000 shapes and rows: 1.17 times as fast on average on the device, one in
+    twelve more than 5 % slower there, by 6 us at most up to 65536 weight rows (short K that only small steps divide: 1280 x 704, 48 rows 3.5 / 5.2;
+    4352 x 2048 at 80 rows 10.1 / 12.4, 3072 x 2560 at 136 9.6 / 12.3; 152064 x 5120 at 208 rows 0.9 of its speed).  Left to the library: up to 512 weight rows, where it depends on K and rows (512 x 2048 5.5 / 6.7, 512 x 4096 11.7 / 7.1 at
+    64 rows); up to 2048 of them at K 2560 - 4096 past 64 rows (2048 x 4096 11.1 / 10.3 at 64 rows, 10.6 / 11.2 at 128, 1024 x 4096 12.2 / 8.0 and 9.4 / 9.6, 1536 x
+    4096 9.4 / 10.2 at 96); 2049 to 4096 at K 1536 - 3072 and 10 M elements, where its tiles fit the rows (3072 x 2048 at 144: 9.6 / 11.5, 192: 16.1 / 12.1,
+    256: 11.0 / 12.2, 2560 x 2560 11.0 / 10.8, 11.0 / 11.6 and 12.4 / 14.3); heads of 32769 to 53248 columns past 192 rows (49152 x 4096, 256: 0.83 of its speed, 192:
+    1.17), up to 65536 past 160 (65536 x 1024, 224: 0.80, 160: 1.17), larger ones with K <= 2048 from 96 rows on (128256 x 2048: 96 rows 131 / 130, 128
+    134 / 142, 192 142 / 155).
     More rows are the library's, whose large tiles win (320 rows: 28672 x 4096 81 / 84, 3072 x 2048 11.2 / 13.8; 1024: 28672 x 4096 169 / 208), but
     * where K is long and at least twice N, where it runs few of them: 2048 x 8192 33 / 26 at 320 rows, 45 / 36 at 640 and 50 / 45 at 1024, 4096 x 14336 76 / 52,
       111 / 78 and 134 / 118, 8192 x 28672 226 / 164 at 320; past 640 rows at least two and a half times N (4096 x 8192, 704: 57 / 60) and up to 288
-      tiles of 128 x 128 (6144 x 16384, 768: 1.3 times as fast, 1024: 189 / 200; 5504 x 14720, 832: 0.95);
-    * where 128-row tiles nearly fill the units once, K of 1024 - 4096: more than 200 of at most 256 (2048 x 2048, 777 rows 18.0 / 16.2, 4096 x 4096 41.7 / 38.6,
-      900 rows of 3328 x 3072 1.05 - 1.11 times as fast; with 192, 3072 x 3072, 0.85 - 0.98, 3584 x 4096 at 777, 196 tiles, 0.92), and more than 160 of narrow
-      tiles up to K 1536 (1536 x 1024, 777: 1.19; 1536 x 3072: 0.95).  Of wide ones from K 1536 on (3584 x 1024, 928: 0.98).  740 pairs: 1.09 on average, none
-      more than 5 % slower.
-    5 - 16 rows (against sp_gemm_skinny or the library, whichever is faster): matrices of more than 2^23 elements, where 16 rows of x beside every 16 weight
-    rows are what sp_gemm_skinny waits for (at 5 / 8 / 16 rows: 28672 x 4096 49 / 42, 54 / 43, 61 / 44; 128256 x 4096 190 / 161, 193 / 162, 193 / 164;
-    6144 x 2048 9.1 / 8.5, 9.4 / 8.5, 10.9 / 8.6); below that a launch of small workgroups is over sooner (2048 x 4096 7.9 / 8.4, 3072 x 2048 5.7 / 6.8).  Up to
-    2^24 elements only K in steps of 256 (8192 x 1088 0.67 - 0.89), and at 5 - 8 rows K past 5120 (1536 x 6144 1.2) or 1792 - 4096 of less than 8192 weight
-    rows (5120 x 2048 1.06 - 1.14; 6144 x 1536 0.91 - 0.99, 2048 x 4608 0.94 - 1.0).  Up to 4096 x 4096 from 9 rows on (3584 x 3584 1.0 - 1.14), from 13 where it
-    is 10 to 12.6 M elements (4096 x 2560 at 9 rows 0.87, at 14 1.0)."""
+      tiles of 128 x 128 (6144 x 16384, 768: 1.3 times as fast, 1024: 189 / 200; 5504 x 14720, 832: 0.95).  510 pairs: 1.25 on average, two more than 5 % slower;
+    * at 769 - 1024 rows, where 128-row tiles nearly fill the units once, K of 1024 - 4096: more than 200 of at most 256 (2048 x 2048, 777 rows 18.0 / 16.2,
+      4096 x 4096 41.7 / 38.6, 900 rows of 3328 x 3072 1.05 - 1.11 times as fast; with 192, 3072 x 3072, 0.85 - 0.98, 3584 x 4096 at 777, 196 tiles, 0.92), and
+      more than 160 up to K 2048, where the device is done before an eager call of the library is (3072 x 2048 18.7 / 19.2, 3328 x 1024 11.8 / 12.9).
+    5 - 16 rows: matrices of more than 2^23 elements, where 16 rows of x beside every 16 weight rows are what sp_gemm_skinny waits for (at 5 / 8 / 16 rows:
+    28672 x 4096 49 / 42, 54 / 43, 61 / 44; 128256 x 4096 190 / 161, 193 / 162, 193 / 164; 6144 x 2048 9.1 / 8.5, 9.4 / 8.5, 10.9 / 8.6); below that a launch of small
+    workgroups is over sooner (2048 x 4096 7.9 / 8.4, 3072 x 2048 5.7 / 6.8).  Up to 2^24 elements only K in steps of 256 (8192 x 1088 0.67 - 0.89), and at 5 - 8
+    rows K past 5120 (1536 x 6144 1.2) or 1792 - 4096 of less than 8192 weight rows (5120 x 2048 1.06 - 1.14; 6144 x 1536 0.91 - 0.99, 2048 x 4608 0.94 - 1.0).
+    Up to 4096 x 4096 from 9 rows on (3584 x 3584 1.0 - 1.14), from 13 where it is 10 to 12.6 M elements (4096 x 2560 at 9 rows 0.87, at 14 1.0)."""
     if K % 64:
         return False
     if M <= SKINNY_MAX_ROWS:
@@ -937,17 +904,19 @@ def dense_gemm_pays(M: int, N: int, K: int) -> bool:
     if M > DENSE_MAX_ROWS:
         if K <= 4096 and N <= 4096:
             tiles = -(-M // 128) * -(-N // (64 if N <= 2048 else 128))
-            return M > 768 and tiles <= 256 and ((tiles > 200 and K >= (1024 if N <= 2048 else 1536))
-                                                 or (tiles > 160 and N <= 2048 and 1024 <= K <= 1536))
+            return M > 768 and K >= 1024 and (160 if K <= 2048 else 200) < tiles <= 256
         if N < 2048 or K <= 5120:
             return False
         if M <= 640:
             return K >= 2 * N and (N <= 6144 or M <= 512)
         return 2 * K >= 5 * N and -(-M // 128) * -(-N // 128) <= 288
-    if N <= 512 or (K % 256 and K < 1600 and N <= 2048):
-        return False
-    return not any(n0 <= N <= n1 and k0 <= K <= k1 and m0 <= M <= m1 and (every or M % 32)
-                   for n0, n1, k0, k1, m0, m1, every in _LIBRARY_KEEPS)
+    if N <= 2048:
+        return N > 512 and not (2048 < K <= 4096 and M > 64)
+    if N <= 4096:
+        return not (1536 <= K <= 3072 and N * K <= 10 << 20 and (128 < M <= 160 or M > 208))
+    if N <= 32768 or K < 512:
+        return N <= 65536 or M < 96
+    return M <= 192 if N <= 53248 else M <= 160 if N <= 65536 else K > 2048 or M < 96
 
 
 def _dense_plan(M: int, N: int, K: int, epilogue: int) -> int:
