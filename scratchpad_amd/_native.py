@@ -873,12 +873,12 @@ def dense_gemm_pays(M: int, N: int, K: int) -> bool:
     rows, where most products take less than that, own products also stand where the device alone would be a little faster with the library's.
     17 - 256 rows of most shapes (the table in gemm_dense.hip).  21100 pairs of 1000 shapes and rows: 1.17 times as fast on average on the device, one in
     twelve more than 5 % slower there, by 6 us at most up to 65536 weight rows (short K that only small steps divide: 1280 x 704, 48 rows 3.5 / 5.2;
-    4352 x 2048 at 80 rows 10.1 / 12.4, 3072 x 2560 at 136 9.6 / 12.3; 152064 x 5120 at 208 rows 0.9 of its speed).  Left to the library: up to 512 weight rows, where it depends on K and rows (512 x 2048 5.5 / 6.7, 512 x 4096 11.7 / 7.1 at
-    64 rows); up to 2048 of them at K 2560 - 4096 past 64 rows (2048 x 4096 11.1 / 10.3 at 64 rows, 10.6 / 11.2 at 128, 1024 x 4096 12.2 / 8.0 and 9.4 / 9.6, 1536 x
-    4096 9.4 / 10.2 at 96); 2049 to 4096 at K 1536 - 3072 and 10 M elements, where its tiles fit the rows (3072 x 2048 at 144: 9.6 / 11.5, 192: 16.1 / 12.1,
-    256: 11.0 / 12.2, 2560 x 2560 11.0 / 10.8, 11.0 / 11.6 and 12.4 / 14.3); heads of 32769 to 53248 columns past 192 rows (49152 x 4096, 256: 0.83 of its speed, 192:
-    1.17), up to 65536 past 160 (65536 x 1024, 224: 0.80, 160: 1.17), larger ones with K <= 2048 from 96 rows on (128256 x 2048: 96 rows 131 / 130, 128
-    134 / 142, 192 142 / 155).
+    4352 x 2048 at 80 rows 10.1 / 12.4, 3072 x 2560 at 136 9.6 / 12.3; 152064 x 5120 at 208 rows 0.9 of its speed).  Left
+    to the library: up to 512 weight rows, where it depends on K and rows (512 x 2048 5.5 / 6.7, 512 x 4096 11.7 / 7.1 at 64 rows); up to 2048 of them at K
+    2560 - 4096 past 64 rows (2048 x 4096 11.1 / 10.3 at 64 rows, 10.6 / 11.2 at 128, 1024 x 4096 12.2 / 8.0 and 9.4 / 9.6, 1536 x 4096 9.4 / 10.2 at 96); 2049 to
+    4096 at K 1536 - 3072 and 10 M elements, where its tiles fit the rows (3072 x 2048 at 144: 9.6 / 11.5, 192: 16.1 / 12.1, 256: 11.0 / 12.2, 2560 x 2560
+    11.0 / 10.8, 11.0 / 11.6 and 12.4 / 14.3); heads of 32769 to 53248 columns past 192 rows (49152 x 4096, 256: 0.83 of its speed, 192: 1.17), up to 65536 past
+    160 (65536 x 1024, 224: 0.80, 160: 1.17), larger ones with K <= 2048 from 96 rows on (128256 x 2048: 96 rows 131 / 130, 128 134 / 142, 192 142 / 155).
     More rows are the library's, whose large tiles win (320 rows: 28672 x 4096 81 / 84, 3072 x 2048 11.2 / 13.8; 1024: 28672 x 4096 169 / 208), but
     * where K is long and at least twice N, where it runs few of them: 2048 x 8192 33 / 26 at 320 rows, 45 / 36 at 640 and 50 / 45 at 1024, 4096 x 14336 76 / 52,
       111 / 78 and 134 / 118, 8192 x 28672 226 / 164 at 320; past 640 rows at least two and a half times N (4096 x 8192, 704: 57 / 60) and up to 288

@@ -359,9 +359,10 @@ class LogitsProcessor(nn.Module):
 
 # --------------------------------------------------------------------------- decoder
 def _runs_only(module: nn.Module, cls: type) -> bool:
-    """calling the module runs cls.forward and nothing of a user's: no hooks, no other module or forward in its place"""
-    return type(module) is cls and "forward" not in module.__dict__ and not (
-        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or _has_any_global_hook())
+    """calling the module runs cls.forward and no hook of its own (those of all modules aside): no other module or forward in its place"""
+    own = module.__dict__
+    return type(module) is cls and "forward" not in own and not (
+        own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"])
 
 
 class LlamaMLP(nn.Module):
@@ -376,8 +377,8 @@ class LlamaMLP(nn.Module):
     def forward(self, x, reduce_output: bool = True):
         # projection and activation in one launch: small decode steps (<= _native.SILU_FUSED_MAX_ROWS tokens) by the weight-streaming
         # kernel, 17 rows and more (5 and more over large weights) where the tiled kernel takes the projection
-        project, act_fn, act = self.gate_up_proj, self.act_fn, None
-        if _runs_only(project, MergedColumnParallelLinear) and _runs_only(act_fn, SiluAndMul):
+        project, act_fn, act = self._modules["gate_up_proj"], self._modules["act_fn"], None          # (an attribute takes 1.2 us of the host)
+        if _runs_only(project, MergedColumnParallelLinear) and _runs_only(act_fn, SiluAndMul) and not _has_any_global_hook():
             weight = project.weight
             act = _native.linear_silu_mul(x, weight)
             if act is None:
