@@ -322,14 +322,15 @@ int launch_dense_kernel(const DenseArgs& p, hipStream_t st) {
   int threads;
   if constexpr (IsRing<T>::value) kernel = dense_wide_kernel<Tag, T, EPI, SPLIT>, threads = T::W * 64;
   else kernel = dense_kernel<Tag, T, EPI, SPLIT>, threads = T::kWaves * 64;
+  const int64_t groups = ((int64_t)p.mblocks * p.nblocks * p.splits + 7) / 8 * 8;
+  if (groups * threads >= (int64_t)1 << 32) return SP_ERR_UNSUPPORTED;          // (what a launch holds)
   static PerDevice<int> raised;
   int ok = 0;
   raised.get(ok, [&](int) {
     return hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, T::kLds) == hipSuccess ? 1 : 0;
   });
   if (!ok) return SP_ERR_LAUNCH;
-  const int total = p.mblocks * p.nblocks * p.splits;
-  kernel<<<dim3((total + 7) / 8 * 8), dim3(threads), T::kLds, st>>>(p);
+  kernel<<<dim3((unsigned)groups), dim3(threads), T::kLds, st>>>(p);
   SP_LAUNCH_CHECK();
   return SP_OK;
 }
@@ -342,9 +343,11 @@ int launch_dense_tile(DenseArgs p, int epilogue, hipStream_t st) {
   p.nblocks = (p.N + per - 1) / per;
   if (epilogue) return p.splits == 1 ? launch_dense_kernel<Tag, T, 1, false>(p, st) : SP_ERR_UNSUPPORTED;
   if (p.splits == 1) return launch_dense_kernel<Tag, T, 0, false>(p, st);
+  const int64_t quads = (int64_t)p.M * ((p.N + 3) / 4);
+  if (quads >= ((int64_t)1 << 32) - 256) return SP_ERR_UNSUPPORTED;
   const int rc = launch_dense_kernel<Tag, T, 0, true>(p, st);
   if (rc != SP_OK) return rc;
-  const dim3 grid((unsigned)(((int64_t)p.M * ((p.N + 3) / 4) + 255) / 256));
+  const dim3 grid((unsigned)((quads + 255) / 256));
   switch (p.splits) {
     case 2: dense_sum_kernel<Tag, 2><<<grid, 256, 0, st>>>(p); break;
     case 3: dense_sum_kernel<Tag, 3><<<grid, 256, 0, st>>>(p); break;
@@ -464,9 +467,8 @@ extern "C" int sp_gemm_dense(void* out, const void* x, const void* w, float* sum
   SP_CHECK_ARG(((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)out & 1) == 0);
   if (dtype != SP_BF16 && dtype != SP_F16) return SP_ERR_UNSUPPORTED;
   if (K % sp::kCosts[tile].bk || K / sp::kCosts[tile].bk < splits) return SP_ERR_UNSUPPORTED;
-  // a load's place is a 32-bit offset from the operand's first byte; a launch has at most 2^31 - 1 workgroups
-  if ((int64_t)M * x_stride * 2 >= (int64_t)1 << 32 || rows * w_stride * 2 >= (int64_t)1 << 32 || (int64_t)M * rows >= (int64_t)1 << 38)
-    return SP_ERR_UNSUPPORTED;
+  // a load's place is a 32-bit offset from the operand's first byte
+  if ((int64_t)M * x_stride * 2 >= (int64_t)1 << 32 || rows * w_stride * 2 >= (int64_t)1 << 32) return SP_ERR_UNSUPPORTED;
   const int vec = N % 4 == 0 && out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0;
   const sp::DenseArgs p{(char*)out, sums, (const char*)x, (const char*)w, M, N, K, splits, 0, 0, x_stride, w_stride, out_stride, vec};
   return dtype == SP_BF16 ? sp::launch_dense<sp::bf16_tag>(p, tile, epilogue, (hipStream_t)stream)

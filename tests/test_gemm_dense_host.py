@@ -231,3 +231,14 @@ def test_fused_mlp_passes_by_nothing_that_its_modules_would_run(monkeypatch, kin
         if handle is not None:
             handle.remove()
     assert seen and fused == [1]
+
+
+def test_more_work_than_a_launch_holds_is_refused():
+    """2^32 threads, though every operand is within reach of its 32-bit offsets (nothing is launched: no pointer is looked at)"""
+    from scratchpad_amd import _native
+    lib = _native.load()
+    K, bf16, unsupported = 256, 2, -2
+    for tile, M, N in ((2, 1 << 19, 1 << 18), (14, 1 << 22, 1 << 15), (2, 1 << 22, 1 << 14)):
+        assert lib.sp_gemm_dense(16, 16, 16, None, 0, M, N, K, K, K, N, 0, tile + 256, bf16, None) == unsupported
+    M, N = 1 << 22, 1 << 13                                                                       # the sum of the shares
+    assert lib.sp_gemm_dense(16, 16, 16, 16, 2 * M * N, M, N, K, K, K, N, 0, 17 + 512, bf16, None) == unsupported
