@@ -15,9 +15,10 @@
 //   * a step is one barrier, in front of its last products: the next step's first operands are read behind it, under them;
 //   * small tiles split every 64 of k over two groups of waves (WK): twice the waves to hide LDS behind, one exchange at the end.
 // From about 128 rows on the matrix cores and the stream take as long as each other, and a wave's direct loads hold its products up: there
-// dense_wide_kernel, whose waves all load both operands and spread the loads between their products (28672 x 4096 at 256 rows 74.7 us by waves of
-// either kind, 66.2 so; 4096 x 14336 48.2 and 44.2, at 640 rows 94 and 76; 2048 x 8192 24.2 and 21.4).
-// us under graph replay, cold weights, library -> this:         rows 17           64           128          256
+// dense_wide_kernel, whose waves all load both operands and spread the loads between their products (the best tile and shares of dense_kernel and
+// of it: 28672 x 4096 at 256 rows 106 and 65 us; 4096 x 14336 58.9 and 45.6, at 640 rows 113 and 78; 2048 x 8192 23.9 and 22.7).
+// us under graph replay, cold weights, library -> this, as it is planned:
+//                                                         rows 17           64           128          256
 //   3072 x 2048 (qkv, hidden 2048)                          8.9 ->  7.6   9.5 ->  7.8   12.1 ->  9.6   11.0 -> 12.2
 //   2048 x 2048                                             8.6 ->  7.4   9.2 ->  7.5    8.8 ->  7.5    9.8 ->  9.6
 //   16384 x 2048 (gate and up)                             18.6 -> 16.2  18.3 -> 17.0   22.4 -> 20.7   30.6 -> 26.1
@@ -104,7 +105,7 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
   constexpr int TM = T::BM / T::WM, TN = T::BN / T::WN, FM = TM / 16, FN = TN / 16, KS = T::BK / 32 / T::WK;
   constexpr int GX = T::BM / RPL, GW = T::BN / RPL, WW = T::kWaves - T::WX;
   constexpr int LX = (GX + T::WX - 1) / T::WX, LW = (GW + WW - 1) / WW, LM = LX > LW ? LX : LW;
-  static_assert(T::BM % RPL == 0 && T::BN % RPL == 0 && TM % 16 == 0 && TN % 16 == 0 && T::BK % (32 * T::WK) == 0 && T::WK <= 2, "tile");
+  static_assert(T::BM % RPL == 0 && T::BN % RPL == 0 && TM % 16 == 0 && TN % 16 == 0 && T::BK % (64 * T::WK) == 0 && T::WK <= 2, "tile");
   static_assert(LX * (T::SX - 1) <= 63 && LW * (T::SW - 1) <= 63 && T::SX >= 2 && T::SW >= 2 && T::kLds <= 160 * 1024, "ring");
   extern __shared__ __attribute__((aligned(1024))) char dense_lds[];
   char* const lds = dense_lds;
@@ -169,13 +170,12 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
   ring_barrier();
   read(0, 0, wk, 0);
   int cx = 0, cw = 0;
-  // One step: its products, behind the reads of the next one's first operands.  PAR: which of the two operand sets is the step's first
-  const auto body = [&](int s, auto par) {
-    constexpr int PAR = decltype(par)::value;
+  // a step's products, behind the reads of the next one's first operands
+  for (int s = 0; s < steps; ++s) {
     const int nx = cx == (T::SX - 1) * T::kX ? 0 : cx + T::kX, nw = cw == (T::SW - 1) * T::kW ? 0 : cw + T::kW;
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
-      const int at = (PAR + j) & 1;
+      const int at = j & 1;
       if (j < KS - 1) {
         read(cx, cw, (j + 1) * T::WK + wk, at ^ 1);
       } else if (s + 1 < steps) {
@@ -196,15 +196,6 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
         for (int f = 0; f < FM; ++f) acc[f][n] = mfma32<Tag>(wf[at][n], xf[at][f], acc[f][n]);
     }
     cx = nx, cw = nw;
-  };
-  const std::integral_constant<int, 0> even;
-  if constexpr (KS % 2 == 0) {
-    for (int s = 0; s < steps; ++s) body(s, even);
-  } else {
-    const std::integral_constant<int, 1> odd;
-    int s = 0;
-    for (; s + 2 <= steps; s += 2) body(s, even), body(s + 1, odd);
-    if (s < steps) body(s, even);
   }
   if constexpr (T::WK > 1) {                              // the two halves of every 64 of k meet in LDS, the first wave's plus the second's
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -228,7 +219,8 @@ __global__ void __launch_bounds__(T::kWaves * 64, T::kOcc) dense_kernel(DenseArg
 }
 
 // The same by ring_product's loop, for more rows: every wave loads both operands, its loads spread between its products.  Past the L2 only the weights of
-// an unsplit product with one row block: at 256 rows 28672 x 4096 66 us with it and 72 without, 4096 x 14336 in 8 shares 44 and 45, at 192 41 and 39.
+// an unsplit product with one row block: at 256 rows 28672 x 4096 66 us with it and 72 without, 4096 x 14336 in 8 shares (the fastest
+// there; four of 128 x 128 tiles are planned) 44 and 45, at 192 41 and 39.
 // Four row blocks share the columns they pass: their rows of x and a few columns stay in an XCD's L2.
 constexpr int kRowGroup = 4;
 
