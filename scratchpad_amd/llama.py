@@ -7,8 +7,8 @@ callers of the hot path keep the reference's tensor-parallel shard math:
 QKVParallelLinear (nn/layers/linear.py:696-760), MergedColumnParallelLinear (423-470),
 RowParallelLinear + all-reduce (1033-1155), VocabParallelEmbedding + all-reduce
 (nn/layers/vocab_parallel_embedding.py:452-472), LogitsProcessor pruning + all-gather
-(nn/layers/logits_processor.py:179-203, 344-376).  GEMMs stay on torch (hipBLASLt/rocBLAS):
-they are outside the path this package re-kernels.
+(nn/layers/logits_processor.py:179-203, 344-376).  Products go through ``_native.linear``: own kernels
+where they measured faster (few rows, decode batches, some prompts), else hipBLASLt/rocBLAS.
 """
 from typing import Any, Dict, Iterable, Optional, Tuple
 

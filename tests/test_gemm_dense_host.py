@@ -242,3 +242,13 @@ def test_more_work_than_a_launch_holds_is_refused():
         assert lib.sp_gemm_dense(16, 16, 16, None, 0, M, N, K, K, K, N, 0, tile + 256, bf16, None) == unsupported
     M, N = 1 << 22, 1 << 13                                                                       # the sum of the shares
     assert lib.sp_gemm_dense(16, 16, 16, 16, 2 * M * N, M, N, K, K, K, N, 0, 17 + 512, bf16, None) == unsupported
+
+
+def test_rows_like_a_subclass_are_plain_tensors():
+    """what the own products of few rows write into: a tensor, whatever x is, with the spare rows behind it"""
+    from scratchpad_amd import _native
+    x = torch.zeros(3, 64, dtype=torch.bfloat16)
+    for like in (x, torch.nn.Parameter(x, requires_grad=False), x.as_subclass(_OnDevice)):
+        out = _native._rows_like(like, 3, 8)
+        assert type(out) is torch.Tensor and out.shape == (3, 8) and out.stride() == (8, 1) and out.dtype == x.dtype
+        assert out.untyped_storage().nbytes() == (3 + _native.ROW_SLACK) * 8 * 2
