@@ -248,6 +248,19 @@ SP_API int sp_decode_attention(void* out, const void* q, const void* k_buffer, c
                         void* workspace, size_t workspace_bytes, const int32_t* plan, size_t plan_bytes,
                         int dtype, int kv_dtype, void* stream);
 
+/* ---- The attention of a small decode step in one launch: sp_rotary_embedding (neox pairs over the whole head) with its store of
+ *      k and v (byte pools: sp_kv_store_fp8's), then decode attention over request b's keys req_to_token[req][0 .. seq_lens[b]), of
+ *      which the one in slot out_cache_loc[b] is the step's own.  q, k and v are the projection's rows and stay as they are.
+ *      One workgroup per (request, kv head) whatever the lengths: no plan, no workspace, no merge; long requests are
+ *      sp_decode_attention's.  16-bit types over pools of the same type or of e5m2 bytes, heads of 64 or 128, at most 8 query heads per
+ *      kv head (else SP_ERR_UNSUPPORTED); rows aligned to 16 bytes, strides in multiples of 8 elements. */
+SP_API int sp_decode_small(void* out, const void* q, const void* k, const void* v, const void* cos_sin_cache,
+                    const int64_t* positions, const int64_t* out_cache_loc, void* k_buffer, void* v_buffer,
+                    const int32_t* req_to_token, int64_t req_to_token_stride, const void* req_pool_indices,
+                    const void* seq_lens, int idx64, int batch_size, int num_q_heads, int num_kv_heads, int head_dim,
+                    int64_t q_stride, int64_t k_stride, int64_t v_stride, int64_t out_stride, int64_t kv_buffer_stride,
+                    float sm_scale, float k_scale, float v_scale, int64_t max_seq_len, int dtype, int kv_dtype, void* stream);
+
 /* ---- Ragged extend (prefill) attention: replaces extend_attention_fwd (nn/attention/
  *      triton_attn/extend_attention.py:229-327; call site triton_backend.py:137-154) and the
  *      flashinfer ragged+paged+merge_state / paged-only paths (flashinfer_backend.py:400-444).

@@ -80,6 +80,8 @@ SIGNATURES = {
     "sp_decode_attention": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i32, _i32,
                                    _i32, _i32, _i32, _i64, _i64, _i64, _f32, _f32, _f32, _f32, _i64, _i32, _i64,
                                    _i32, _vp, _sz, _vp, _sz, _i32, _i32, _vp]),
+    "sp_decode_small": (_i32, [_vp] * 10 + [_i64, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _f32,
+                               _i64, _i32, _i32, _vp]),
     "sp_extend_attention_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32, _i32]),
     "sp_extend_attention": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i32, _vp, _vp,
                                    _i32, _i64, _i32, _i32, _i32, _i64, _i64, _i64, _f32, _f32, _f32, _f32,
@@ -617,6 +619,35 @@ def decode_attention(out: torch.Tensor, q: torch.Tensor, k_buffer: torch.Tensor,
         max_seq_len, chunk, max_slots, ranges if plan is not None else 0, workspace.data_ptr(),
         workspace.numel() * workspace.element_size(),
         _ptr(plan), plan_bytes, _dt(q), kv_dt, _stream()), "sp_decode_attention")
+
+
+def decode_small(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, positions: torch.Tensor, cos_sin_cache: torch.Tensor,
+                 out_cache_loc: torch.Tensor, k_buffer: torch.Tensor, v_buffer: torch.Tensor, req_to_token: torch.Tensor,
+                 req_pool_indices: torch.Tensor, seq_lens: torch.Tensor, sm_scale: float, max_seq_len: int,
+                 k_scale: Optional[float] = None, v_scale: Optional[float] = None) -> None:
+    """rotary_embedding with its store and decode_attention of a small step in one launch (sp_decode_small).  q [bs, Hq * D], k and
+    v [bs, Hkv * D]: the projection's rows, left as they are; the cos_sin_cache [positions, D] of whole-head neox pairs"""
+    _gpu(out, q, k, v, positions, cos_sin_cache, out_cache_loc, k_buffer, v_buffer, req_to_token, req_pool_indices, seq_lens)
+    if any(t.dim() != 2 or t.stride(1) != 1 or t.dtype != q.dtype for t in (out, q, k, v)):
+        raise RuntimeError("decode_small: out, q, k and v must be 2-D, row-contiguous and of one type")
+    kv_dt = _kv_dt(k_buffer, q, "decode_small")
+    _kv_layout(k_buffer, v_buffer, "decode_small")
+    bs, Hkv, D = q.shape[0], k_buffer.shape[1], k_buffer.shape[2]
+    if v_buffer.dtype != k_buffer.dtype or v_buffer.shape[2] != D or q.shape[1] % D or out.shape != q.shape or k.shape != (bs, Hkv * D) or v.shape != k.shape:
+        raise RuntimeError(f"decode_small: q {tuple(q.shape)}, k {tuple(k.shape)}, v {tuple(v.shape)}, out {tuple(out.shape)} over a pool of "
+                           f"{Hkv} heads of {D}")
+    if cos_sin_cache.dtype != q.dtype or not cos_sin_cache.is_contiguous() or cos_sin_cache.shape[1] != D:
+        raise RuntimeError("decode_small: cos_sin_cache must be contiguous, in the activation dtype and as wide as a head")
+    req, seq, idx64 = _idx_pair(req_pool_indices, seq_lens)
+    positions, out_cache_loc = positions.to(torch.int64).contiguous(), out_cache_loc.to(torch.int64).contiguous()
+    if min(req.shape[0], seq.shape[0], positions.shape[0], out_cache_loc.shape[0]) < bs:
+        raise RuntimeError("decode_small: fewer indices than rows")
+    _check(load().sp_decode_small(
+        out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), cos_sin_cache.data_ptr(), positions.data_ptr(), out_cache_loc.data_ptr(),
+        k_buffer.data_ptr(), v_buffer.data_ptr(), req_to_token.data_ptr(), req_to_token.stride(0), req.data_ptr(), seq.data_ptr(), idx64, bs,
+        q.shape[1] // D, Hkv, D, q.stride(0), k.stride(0), v.stride(0), out.stride(0), k_buffer.stride(0), sm_scale,
+        1.0 if k_scale is None else float(k_scale), 1.0 if v_scale is None else float(v_scale), max_seq_len, _dt(q), kv_dt, _stream()),
+        "sp_decode_small")
 
 
 def extend_workspace_bytes(num_tokens: int, bs: int, Hq: int, D: int, dtype: torch.dtype) -> int:

@@ -87,6 +87,9 @@ class RadixAttention(nn.Module):
         self.k_scale_float = None
         self.v_scale_float = None
         self.use_irope = use_irope
+        # the layer's model rotates q and k right in front of it, whole heads by halves: a step of few keys may then do both and the
+        # store in one launch (HipAttnBackend.rotary_store_attend)
+        self.follows_rotation = False
 
     def forward(self, q, k, v, forward_batch: "ForwardBatch", save_kv_cache: bool = True):
         if k is not None:
@@ -159,8 +162,29 @@ class HipAttnBackend(AttentionBackend):
         # plan is the range section alone and nothing of a step depends on the host's bound on sum(seq_lens).
         layers = [m for m in getattr(model_runner, "model", nn.Module()).modules() if isinstance(m, RadixAttention)]
         self.plan_items = self.decode_ranges <= 0 or any(m.logit_cap > 0 for m in layers)
+        # steps of few keys (_few_keys) run rotation, store and attention of a layer as one launch, without a plan
+        dtype = getattr(model_runner, "dtype", None)
+        self.small_steps = (not self.is_encoder_decoder and self.sliding_window_size is None and bool(layers)
+                            and dtype in (torch.float16, torch.bfloat16) and self.kv_dtype in (dtype, torch.float8_e5m2)
+                            and self.head_dim in (64, 128) and self.v_head_dim == self.head_dim
+                            and self.num_head % self.num_kv_head == 0 and self.num_head // self.num_kv_head <= 8
+                            and all(m.follows_rotation and not m.logit_cap > 0 and m.sliding_window_size == -1 and not m.is_cross_attention
+                                    for m in layers))
 
     # ---------------------------------------------------------------- launch planning
+    # One launch per layer for a small step: rows, and keys of all requests together - a workgroup walks a request's keys
+    # alone, and the host knows their sum.  us per layer, three launches / one, by keys of the one request: heads of 64 300
+    # 10.2 / 5.9, 600 10.4 / 8.5, 1200 11.4 / 10.9, 2400 13.2 / 16.3; of 128 300 12.2 / 7.9, 600 12.3 / 11.4, 1200 13.9 / 16.5.  More
+    # requests share the sum: 8 of 300 12.0 / 7.7 and 13.9 / 10.0, 32 of 64 11.7 / 5.6 and 14.5 / 7.0; what they lose where one of them has
+    # nearly all keys bounds the sum at twice the one request's.
+    SMALL_MAX_ROWS = 32
+    small_steps = False            # this model has such steps
+    small_step = False             # the step that forward_metadata is of is one
+
+    def _few_keys(self, bs: int, seq_lens_sum: int) -> bool:
+        one = 1024 if self.head_dim == 64 and self.kv_dtype != torch.float8_e5m2 else 512
+        return self.small_steps and not self.plan_items and bs <= self.SMALL_MAX_ROWS and seq_lens_sum <= min(one + (bs - 1) * one // 8, 2 * one)
+
     def _head_groups(self, dtype: torch.dtype) -> int:
         vec = 4 if dtype == torch.float32 else 8
         rpl = 64 // (self.head_dim // vec)
@@ -312,15 +336,13 @@ class HipAttnBackend(AttentionBackend):
             else:
                 max_len = min(self.max_context_len, forward_batch.seq_lens_sum - (bs - 1))
             max_len = max(max_len, enc_max, 1)
-            enc = forward_batch.encoder_lens if self.is_encoder_decoder else None
-            enc_sum = sum(forward_batch.encoder_lens_cpu) if forward_batch.encoder_lens_cpu else None
-            self._window = self._window_of(forward_batch.seq_lens)
-            plans, slots = self._build_plans(self._plans, bs, self._windows(
-                bs, forward_batch.seq_lens, forward_batch.seq_lens_sum, enc, enc_sum), max_len)
-            ws = self._ensure_workspace(_native.decode_workspace_bytes(bs, self.num_head, self.v_head_dim, max_len,
-                                                                       self.MIN_CHUNK, slots))
-            self.forward_metadata = (self.MIN_CHUNK, max_len, ws, plans)
+            self.small_step = self._few_keys(bs, forward_batch.seq_lens_sum)
+            if self.small_step:
+                self.forward_metadata = (self.MIN_CHUNK, max_len, None, None)      # (no plan: rotary_store_attend)
+            else:
+                self._plan_decode(forward_batch, max_len)
         else:
+            self.small_step = False
             max_extend = max(forward_batch.extend_seq_lens_cpu)
             if forward_batch.seq_lens_cpu is not None:
                 max_len = int(forward_batch.seq_lens_cpu.max())
@@ -337,6 +359,17 @@ class HipAttnBackend(AttentionBackend):
                                                     forward_batch.extend_num_tokens, self.num_head,
                                                     self.num_kv_head, True, self._extend_plan)
             self.forward_metadata = (max_extend, max_len, ws)
+
+    def _plan_decode(self, forward_batch: "ForwardBatch", max_len: int) -> None:
+        bs = forward_batch.batch_size
+        enc = forward_batch.encoder_lens if self.is_encoder_decoder else None
+        enc_sum = sum(forward_batch.encoder_lens_cpu) if forward_batch.encoder_lens_cpu else None
+        self._window = self._window_of(forward_batch.seq_lens)
+        plans, slots = self._build_plans(self._plans, bs, self._windows(
+            bs, forward_batch.seq_lens, forward_batch.seq_lens_sum, enc, enc_sum), max_len)
+        ws = self._ensure_workspace(_native.decode_workspace_bytes(bs, self.num_head, self.v_head_dim, max_len,
+                                                                   self.MIN_CHUNK, slots))
+        self.forward_metadata = (self.MIN_CHUNK, max_len, ws, plans)
 
     def init_cuda_graph_state(self, max_bs: int):
         """Static buffers for graph replay (triton_backend.py:70-80 allocates its static attn_logits the same
@@ -374,6 +407,7 @@ class HipAttnBackend(AttentionBackend):
                                                  encoder_lens, forward_mode, spec_info=None):
         assert forward_mode.is_decode(), "only decode is captured"
         assert spec_info is None, "speculative decoding is out of scope"
+        self.small_step = False
         self._window = self._window_of(seq_lens, self._graph_window, bs)
         self._graph_metadata(bs, seq_lens, bs * self.get_cuda_graph_seq_len_fill_value(), encoder_lens)
 
@@ -387,6 +421,18 @@ class HipAttnBackend(AttentionBackend):
         # step, from seq_lens_sum (it is plan data, not launch geometry).
         self._window = self._window_of(seq_lens[:bs], self._graph_window, bs)
         self._graph_metadata(bs, seq_lens[:bs], seq_lens_sum, None if encoder_lens is None else encoder_lens[:bs])
+
+    def captures_small_step(self, bs: int) -> bool:
+        """a step of bs rows may be one of few keys: the graph runner captures that form of it beside the general one"""
+        return self._few_keys(bs, bs)
+
+    def init_small_step_capture(self) -> None:
+        """in the place of init_forward_metadata_capture_cuda_graph"""
+        self.forward_metadata = (self.MIN_CHUNK, self.cuda_graph_max_seq_len, self._graph_ws, None)
+        self.small_step = True
+
+    def replays_small_step(self, bs: int, seq_lens_sum: int) -> bool:
+        return self._few_keys(bs, seq_lens_sum)
 
     def get_cuda_graph_seq_len_fill_value(self):
         return 1  # padded rows attend to the dummy slot 0 only (triton_backend.py:115-116)
@@ -437,6 +483,18 @@ class HipAttnBackend(AttentionBackend):
         kb, vb = pool.get_kv_buffer(layer.layer_id)
         _native.rotary_embedding(positions, q, k, rope.head_size, rope.cos_sin_cache, rope.is_neox_style,
                                  value=v, k_buffer=kb, v_buffer=vb, out_cache_loc=forward_batch.out_cache_loc)
+
+    def rotary_store_attend(self, rope, positions, q, k, v, layer: RadixAttention, forward_batch: "ForwardBatch"):
+        """rotary_and_store followed by forward_decode, for a small step (``small_step``), in one launch; q and k stay unrotated"""
+        if rope.cos_sin_cache.device != q.device or rope.cos_sin_cache.dtype != q.dtype:
+            rope.cos_sin_cache = rope.cos_sin_cache.to(q.device, dtype=q.dtype)
+        o = self._alloc_out(q, layer)
+        kb, vb = forward_batch.token_to_kv_pool.get_kv_buffer(layer.layer_id)
+        k_scale, v_scale = self._kv_scales(layer)
+        _native.decode_small(o, q, k, v, positions, rope.cos_sin_cache, forward_batch.out_cache_loc, kb, vb,
+                             forward_batch.req_to_token_pool.req_to_token, forward_batch.req_pool_indices, forward_batch.seq_lens,
+                             layer.scaling, self.forward_metadata[1], k_scale, v_scale)
+        return o
 
     def _kv_scales(self, layer: RadixAttention):
         """flashinfer_backend.py:400-401, 457-458: the layer's float scales, only for a non-"auto"
@@ -495,6 +553,11 @@ class HipAttnBackend(AttentionBackend):
         q = q.reshape(-1, layer.tp_q_head_num * layer.qk_head_dim)
         o = self._alloc_out(q, layer)
         self._store(layer, forward_batch, k, v, save_kv_cache)
+        if self.small_step and self.forward_metadata[3] is None:       # a layer of a small step that is called by itself (a hook, another caller)
+            if self.forward_metadata[2] is None:
+                self._plan_decode(forward_batch, self.forward_metadata[1])
+            else:                                                      # under capture: the plan is a launch of the graph
+                self._graph_metadata(forward_batch.batch_size, forward_batch.seq_lens, forward_batch.seq_lens_sum, None)
         chunk, max_len, ws, plans = self.forward_metadata
         k_scale, v_scale = self._kv_scales(layer)
         seq_lens, kv_start = self._kv_window(layer, forward_batch)

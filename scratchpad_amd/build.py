@@ -27,6 +27,8 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hi
 PER_FILE_FLAGS = {"elementwise.hip": ["-ffp-contract=off"], "allreduce.hip": ["-ffp-contract=off"],
                   # its epilogues repeat the roundings of elementwise.hip's activations
                   "gemm_skinny.hip": ["-ffp-contract=off"], "gemm_dense.hip": ["-ffp-contract=off"],
+                  # it rotates q and k with elementwise.hip's roundings
+                  "decode_small.hip": ["-ffp-contract=off"],
                   "extend_mfma.hip": ["-fno-honor-nans"],
                   # extend_w64.hip: every filler of its hand-placed MFMA gaps is a single instruction: no SLP packing
                   # of adjacent f32 adds / multiplies into v_pk_* (MI355X_MICROARCH.md: an anti-lever beside MFMAs).  Its

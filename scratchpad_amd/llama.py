@@ -23,7 +23,7 @@ from .distributed import (divide, get_tensor_model_parallel_rank,
                           get_tensor_model_parallel_world_size, get_tp_group, tensor_model_parallel_all_gather,
                           tensor_model_parallel_all_reduce)
 from .forward_info import ForwardBatch
-from .layers import RMSNorm, SiluAndMul, get_rope
+from .layers import RMSNorm, RotaryEmbedding, SiluAndMul, get_rope
 
 
 class LogitsProcessorOutput:
@@ -365,6 +365,13 @@ def _runs_only(module: nn.Module, cls: type) -> bool:
         own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"])
 
 
+def _plain_rotation(rope: nn.Module) -> bool:
+    """a call of the module is the rotation of whole heads by halves with the module's table, and nothing else"""
+    own = rope.__dict__
+    return (isinstance(rope, RotaryEmbedding) and type(rope).forward_hip is RotaryEmbedding.forward_hip and "forward" not in own
+            and getattr(rope._forward_method, "__func__", None) is RotaryEmbedding.forward_hip and rope.is_neox_style and rope.rotary_dim == rope.head_size and not (own["_forward_hooks"] or own["_forward_pre_hooks"]))
+
+
 class LlamaMLP(nn.Module):
     def __init__(self, hidden_size: int, intermediate_size: int, hidden_act: str, dtype=None):
         super().__init__()
@@ -422,13 +429,17 @@ class LlamaAttention(nn.Module):
                                    dtype=dtype)
         self.attn = RadixAttention(self.num_heads, self.head_dim, self.scaling,
                                    num_kv_heads=self.num_kv_heads, layer_id=layer_id)
+        self.attn.follows_rotation = _plain_rotation(self.rotary_emb)
 
     def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor,
                 forward_batch: ForwardBatch, reduce_output: bool = True) -> torch.Tensor:
         qkv, _ = self.qkv_proj(hidden_states)
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
         backend = forward_batch.attn_backend
-        if getattr(backend, "fused_rope_kv_store", False):
+        if (getattr(backend, "small_step", False) and backend.fused_rope_kv_store and _runs_only(self.attn, RadixAttention)
+                and _plain_rotation(self.rotary_emb) and not _has_any_global_hook()):
+            attn_output = backend.rotary_store_attend(self.rotary_emb, positions, q, k, v, self.attn, forward_batch)
+        elif getattr(backend, "fused_rope_kv_store", False):
             # one launch: rotate q,k in place AND scatter rotated k + v into the KV pool
             # (= rotary_emb followed by set_kv_buffer; the backend then skips its own store)
             backend.rotary_and_store(self.rotary_emb, positions, q, k, v, self.attn, forward_batch)

@@ -8,7 +8,7 @@ speculative decoding and the NVML/zmq control plane are out of scope (SURVEY.md 
 """
 import bisect
 from dataclasses import dataclass, field
-from typing import Dict, List, Optional
+from typing import Dict, List, Optional, Tuple
 
 import torch
 
@@ -324,6 +324,8 @@ class HipGraphRunner:
         self.model_runner = model_runner
         self.graphs: Dict[int, torch.cuda.CUDAGraph] = {}
         self.output_buffers: Dict[int, LogitsProcessorOutput] = {}
+        # beside them, where the backend has one, the form of a bucket whose requests hold few keys together
+        self.small_graphs: Dict[int, Tuple[torch.cuda.CUDAGraph, LogitsProcessorOutput]] = {}
         self.capture_bs = get_batch_sizes_to_capture(model_runner.server_args, model_runner.req_to_token_pool.size,
                                                      getattr(model_runner.model, "max_graph_batch", None))
         if not self.capture_bs:
@@ -365,11 +367,13 @@ class HipGraphRunner:
                     graph, out = self.capture_one_batch_size(bs)
                     self.graphs[bs] = graph
                     self.output_buffers[bs] = out
+                    if getattr(self.model_runner.attn_backend, "small_steps", False) and self.model_runner.attn_backend.captures_small_step(bs):
+                        self.small_graphs[bs] = self.capture_one_batch_size(bs, small_step=True)
         finally:
             if self.is_encoder_decoder:
                 model.capture_mode = False
 
-    def capture_one_batch_size(self, bs: int):
+    def capture_one_batch_size(self, bs: int, small_step: bool = False):
         mr = self.model_runner
         fb = ForwardBatch(
             forward_mode=ForwardMode.DECODE, batch_size=bs, input_ids=self.input_ids[:bs],
@@ -384,17 +388,20 @@ class HipGraphRunner:
             fb.encoder_lens = enc
             fb.encoder_lens_cpu = [0] * bs
             fb.encoder_cached = [True] * bs
-        mr.attn_backend.init_forward_metadata_capture_cuda_graph(
-            bs, bs, fb.req_pool_indices, fb.seq_lens, enc, ForwardMode.DECODE, None)
+        if not small_step:
+            mr.attn_backend.init_forward_metadata_capture_cuda_graph(
+                bs, bs, fb.req_pool_indices, fb.seq_lens, enc, ForwardMode.DECODE, None)
 
         def run_once():
+            if small_step:
+                mr.attn_backend.init_small_step_capture()
             return mr.model.forward(fb.input_ids, fb.positions, fb)
 
         # warm up on a side stream before capturing (cuda_graph_runner.py:400-412)
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
-            for _ in range(2):
+            for _ in range(1 if small_step else 2):        # (the bucket's general form has warmed up everything but the one launch)
                 run_once()
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
@@ -426,9 +433,13 @@ class HipGraphRunner:
         self.seq_lens[:raw_bs].copy_(forward_batch.seq_lens)
         self.out_cache_loc[:raw_bs].copy_(forward_batch.out_cache_loc)
         self.positions[:raw_bs].copy_(forward_batch.positions)
+        seq_lens_sum = forward_batch.seq_lens_sum + (bs - raw_bs) * self.seq_len_fill_value
+        if bs in self.small_graphs and self.model_runner.attn_backend.replays_small_step(bs, seq_lens_sum):
+            graph, out = self.small_graphs[bs]
+            graph.replay()
+            return out.rows(raw_bs)
         self.model_runner.attn_backend.init_forward_metadata_replay_cuda_graph(
-            bs, self.req_pool_indices, self.seq_lens,
-            forward_batch.seq_lens_sum + (bs - raw_bs) * self.seq_len_fill_value, self.encoder_lens,
+            bs, self.req_pool_indices, self.seq_lens, seq_lens_sum, self.encoder_lens,
             ForwardMode.DECODE, None, forward_batch.seq_lens_cpu)
         self.graphs[bs].replay()
         return self.output_buffers[bs].rows(raw_bs)
