@@ -1800,12 +1800,10 @@ SMALL_LINEAR_OWN_ROWS = 64      # up to this many rows a workgroup per row; abov
 
 
 def small_linear_tiles_pay(T: int, K: int, n: int) -> bool:
-    """Where the tiles for more than 64 bf16 rows measured faster than a copy of x to fp32 and the library's product (us, tiles /
-    library).  Their 8 waves share K in one workgroup, a chain that few rows of a long K do not hide (64 outputs of K 4096: 65 rows
-    17.6 / 14.2, 512 rows 17.9 / 18.8; of K 8192: 512 rows 32.5 / 28.7, 1024 rows 32.6 / 33.6).  They read x once per 32 outputs:
-    the library's larger tiles win with outputs and rows (K 2048: 4096 rows of 256 50.9 / 53.8, of 512 91 / 77, 8192 rows of 128
-    50.0 / 56.2, of 256 94.9 / 87.8; K 4096: 2048 rows of 256 49.0 / 49.7, 4096 of 256 93.7 / 87.8; few rows of many outputs: K 2048,
-    256 rows of 1024 17.5 / 18.8, of 2048 28.7 / 26.5)."""
+    """Where the tiles for more than 64 bf16 rows take the product, else a copy of x to fp32 and the library's.  The line is where the
+    tiles crossed the library when their operands came straight to registers; through LDS they are faster on both sides of it (us,
+    tiles / library: K 2048, 4096 rows of 64 outputs 8.8 / 27.8, of 256 29.2 / 48.3; 8192 of 128 33.9 / 53.9; 256 of 1024 9.5 / 17.0; past
+    the line 65 rows of K 4096 8.0 / 13.2, 512 of K 8192 12.9 / 27.7, 4096 of 512 outputs 56.0 / 74.0, 8192 of 256 59.2 / 83.1)."""
     return (K <= 2048 or 8 * T >= K) and (n <= 128 or (n <= 256 and T * K <= 1 << 23) or (K <= 2048 and T * n <= 1 << 18))
 
 

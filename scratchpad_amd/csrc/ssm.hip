@@ -8,6 +8,7 @@
 //                      per head, S [N, Dv] fp32 in the state pool; head h reads B, C of group h / (H / G)
 //   gated group norm   out = (y silu(z)) / rms_part * w      the gate BEFORE the norm, `parts` equal parts per row
 #include "chunk_scan.h"
+#include "lds_ring.h"
 
 namespace sp {
 namespace {
@@ -62,92 +63,125 @@ small_linear_f32_kernel(float* out, const void* x, int64_t x_stride, const float
 }
 
 // The same for many rows of bf16 x, on the matrix cores with nothing rounded on the way: a weight is three bf16 parts whose sum is
-// exact (split3), x is bf16 already, the sums are fp32.  A workgroup takes 32 tokens x 16 NT outputs; its 8 waves share K (a
-// stretch each, two 32-deep steps of it in flight) and add up through LDS in wave order.  4096 tokens x 2048, us, with the library's
-// fp32 product behind a copy of x to fp32 -> now: 64 outputs 29.3 -> 14.9, 32 outputs 27.0 -> 10.2; 65 rows of 64 outputs
-// 24.8 -> 9.7.  An infinity has no parts that are numbers: a sum that is not finite is formed again, element by element.
-constexpr int kLinTokens = 32, kLinWaves = 8;
-template <int NT>
-__global__ void __launch_bounds__(kLinWaves * 64)
+// exact (split3), x is bf16 already, the sums are fp32.  A workgroup takes 16 MT tokens x 16 outputs; its W waves share K (a stretch each)
+// and add up through LDS in wave order.  An infinity has no parts that are numbers: a sum that is not finite is formed again, element
+// by element.
+// What bounds it is the way of the operands to the lanes: a matrix instruction wants 16 rows in neighbouring lanes, and a load of that shape
+// asks for 16 lines a quarter (65 rows of K 2048 took 9.7 us whatever was in flight).  So rows come by direct loads of 128 or 256 neighbouring
+// bytes into LDS that is the wave's own - no barrier but the last - and the lanes take their operands from there; the next 64 of k load while
+// those are split and multiplied (more stages in flight leave room for fewer workgroups: 4096 rows of 64 outputs 12.5 with two).
+// us, K 2048, loads to registers -> this: 4096 rows of 64 outputs 15.6 -> 9.1, of 32 10.1 -> 6.7, 65 rows of 64 9.8 -> 5.5; K 1024, 4096 of 32
+// 6.8 -> 5.1.  Layers of 4096 and 3001 tokens: Mamba-2 395 -> 388, mLSTM 207 -> 202.
+constexpr int kLinOut = 16;
+template <int MT, int W>
+__global__ void __launch_bounds__(W * 64)
 linear_f32_mfma_kernel(float* out, const char* x, int64_t x_stride, const float* w, const float* bias, int64_t T, int K, int N) {
-  constexpr int MT = kLinTokens / 16, U = 2, ROW = 16 * NT + 4;
-  __shared__ __attribute__((aligned(16))) float part[kLinWaves / 2][kLinTokens][ROW];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, q = lane >> 4;
-  const int64_t t0 = (int64_t)blockIdx.x * kLinTokens;
-  const int n0 = blockIdx.y * 16 * NT;
-  const char* xp[MT];
-  const float* wp[NT];
+  constexpr int TOK = 16 * MT, LX = 2 * MT, LW = 4, kX = TOK * 128, kStage = kX + kLinOut * 256, ROW = kLinOut + 4;
+  static_assert(W / 2 * TOK * ROW * 4 <= W * kStage && W * kStage <= 160 * 1024, "LDS");
+  extern __shared__ __attribute__((aligned(1024))) char lin_lds[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, q = lane >> 4;
+  const int64_t t0 = (int64_t)blockIdx.x * TOK;
+  const int n0 = blockIdx.y * kLinOut;
+  // rows past the last: that one again, never stored; 16-byte chunks permuted by the row's number
+  uint32_t ox[LX], ow[LW];
+  const int cx = (lane & 7) ^ (lane >> 3);
 #pragma unroll
-  for (int i = 0; i < MT; ++i) xp[i] = x + ((t0 + 16 * i + r16 < T ? t0 + 16 * i + r16 : T - 1) * x_stride + 8 * q) * 2;
-#pragma unroll
-  for (int j = 0; j < NT; ++j) wp[j] = w + (int64_t)min(n0 + 16 * j + r16, N - 1) * K + 8 * q;      // (rows past N: never stored)
-  f32x4_c acc[MT][NT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_c{0.f, 0.f, 0.f, 0.f};
-  const int steps = K / 32, mine = (steps + kLinWaves - 1) / kLinWaves;
-  const int first = wave * mine, last = min(first + mine, steps);
-  const u32x4 zero = {0u, 0u, 0u, 0u};
-  for (int ks = first; ks < last; ks += U) {
-    u32x4 xf[U][MT], wf[U][NT][2];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool in = ks + u < last;
-      const int64_t k = (int64_t)(ks + u) * 32;
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) wf[u][j][h] = in ? ld16(wp[j] + k + 4 * h) : zero;
-#pragma unroll
-      for (int i = 0; i < MT; ++i) xf[u][i] = in ? ld16(xp[i] + k * 2) : zero;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        u32x4 b[3];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          uint32_t hi, mid, lo;
-          split3(as_f32(wf[u][j][e / 2][2 * (e & 1)]), as_f32(wf[u][j][e / 2][2 * (e & 1) + 1]), hi, mid, lo);
-          b[0][e] = hi, b[1][e] = mid, b[2][e] = lo;
-        }
-#pragma unroll
-        for (int c = 2; c >= 0; --c)
-#pragma unroll
-          for (int i = 0; i < MT; ++i) acc[i][j] = mfma_c(xf[u][i], b[c], acc[i][j]);
-      }
+  for (int i = 0; i < LX; ++i) {
+    const int64_t row = i * 8 + (lane >> 3), last = T - 1 - t0;
+    ox[i] = (uint32_t)((row < last ? row : last) * x_stride * 2) + cx * 16;
   }
-  // lane (r16, q): tokens 16 i + 4 q + r, output 16 j + r16; waves 4-7 first, then 0-3 add their own
+#pragma unroll
+  for (int i = 0; i < LW; ++i) {
+    const int row = i * 4 + q;
+    ow[i] = (uint32_t)min(row, N - 1 - n0) * (uint32_t)K * 4 + ((lane & 15) ^ row) * 16;
+  }
+  const char *const xb = x + t0 * x_stride * 2, *const wb = (const char*)(w + (int64_t)n0 * K);
+  char* const own = lin_lds + wave * kStage;
+  const uint32_t own0 = lds_address(own);
+  const int stages = (K + 63) / 64, first = stages * wave / W, last = stages * (wave + 1) / W;
+  const auto load = [&](int s) {
+    const bool half = s * 64 + 64 > K;                    // K ends in the middle: its second 32 are the first again, and not taken
+#pragma unroll
+    for (int i = 0; i < LX; ++i) ring_load<false>(half && cx >= 4 ? ox[i] - 64 : ox[i], xb + (int64_t)s * 128, own0 + i * 1024);
+#pragma unroll
+    for (int i = 0; i < LW; ++i)
+      ring_load<false>(half && ((lane & 15) ^ (i * 4 + q)) >= 8 ? ow[i] - 128 : ow[i], wb + (int64_t)s * 256, own0 + kX + i * 1024);
+  };
+  f32x4_c acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = f32x4_c{0.f, 0.f, 0.f, 0.f};
+  if (first < last) load(first);
+  for (int s = first; s < last; ++s) {
+    ring_wait<LX + LW, 0>(0);
+    u32x4 xf[2][MT], wf[2][2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wf[k][h] = ld16(own + kX + r16 * 256 + (((8 * k + 2 * q + h) ^ r16) * 16));
+#pragma unroll
+      for (int i = 0; i < MT; ++i) xf[k][i] = ld16(own + (16 * i + r16) * 128 + (((4 * k + q) ^ (r16 & 7)) * 16));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // in registers: the stage is free
+    if (s + 1 < last) load(s + 1);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (k && s * 64 + 64 > K) break;
+      u32x4 b[3];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t hi, mid, lo;
+        split3(as_f32(wf[k][e / 2][2 * (e & 1)]), as_f32(wf[k][e / 2][2 * (e & 1) + 1]), hi, mid, lo);
+        b[0][e] = hi, b[1][e] = mid, b[2][e] = lo;
+      }
+#pragma unroll
+      for (int c = 2; c >= 0; --c)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[i] = mfma_c(xf[k][i], b[c], acc[i]);
+    }
+  }
+  // lane (r16, q): tokens 16 i + 4 q + r, output r16; the upper half of the waves first, then the lower add their own
+  __syncthreads();
+  float* const part = (float*)lin_lds;
 #pragma unroll
   for (int half = 1; half >= 0; --half) {
-    if (wave / (kLinWaves / 2) == half) {
+    if (wave / (W / 2) == half) {
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float* to = &part[wave % (kLinWaves / 2)][16 * i + 4 * q + r][16 * j + r16];
-            *to = half ? acc[i][j][r] : acc[i][j][r] + *to;
-          }
+        for (int r = 0; r < 4; ++r) {
+          float* const to = part + (wave % (W / 2) * TOK + 16 * i + 4 * q + r) * ROW + r16;
+          *to = half ? acc[i][r] : acc[i][r] + *to;
+        }
     }
     __syncthreads();
   }
-  for (int e = tid; e < kLinTokens * 16 * NT; e += kLinWaves * 64) {
-    const int t = e / (16 * NT), n = e % (16 * NT);
+  for (int e = tid; e < TOK * kLinOut; e += W * 64) {
+    const int t = e / kLinOut, n = e % kLinOut;
     if (t0 + t >= T || n0 + n >= N) continue;
     float v = 0.f;
 #pragma unroll
-    for (int u = 0; u < kLinWaves / 2; ++u) v += part[u][t][n];
+    for (int u = 0; u < W / 2; ++u) v += part[(u * TOK + t) * ROW + n];
     if (!(fabsf(v) < INFINITY)) {
       v = 0.f;
       for (int k = 0; k < K; ++k) v += w[(int64_t)(n0 + n) * K + k] * Elem<bf16_tag>::load(x, (t0 + t) * x_stride + k);
     }
     out[(t0 + t) * N + n0 + n] = v + (bias ? bias[n0 + n] : 0.f);
   }
+}
+
+template <int MT, int W>
+int launch_linear_f32(float* out, const char* x, int64_t x_stride, const float* w, const float* bias, int64_t T, int K, int N, hipStream_t st) {
+  constexpr int lds = W * (MT * 2048 + kLinOut * 256);
+  static PerDevice<int> raised;
+  int ok = 0;
+  raised.get(ok, [&](int) {
+    return hipFuncSetAttribute((const void*)linear_f32_mfma_kernel<MT, W>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess ? 1 : 0;
+  });
+  if (!ok) return SP_ERR_LAUNCH;
+  const dim3 tiles((unsigned)((T + 16 * MT - 1) / (16 * MT)), (unsigned)((N + kLinOut - 1) / kLinOut));
+  linear_f32_mfma_kernel<MT, W><<<tiles, W * 64, lds, st>>>(out, x, x_stride, w, bias, T, K, N);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
 }
 
 // state [slot][taps - 1][C]: entry k = the input at position (tokens held) - (taps - 1) + k
@@ -647,19 +681,13 @@ extern "C" int sp_small_linear_f32(float* out, const void* x, int64_t x_stride, 
   if (num_tokens == 0) return SP_OK;
   SP_CHECK_ARG(out && x && weight && x_stride >= k);
   if (num_tokens > 64 && dtype == SP_BF16 && k % 32 == 0 && x_stride % 8 == 0 && (((uintptr_t)x | (uintptr_t)weight) & 15) == 0) {
-    // (up to 64 rows a workgroup per row has the shorter chain.)  16 outputs a workgroup while that leaves a CU one of them, 32
-    // beyond: the chain over K is half as long (4096 rows of 32 outputs: 10.2 against 14.3 us), x and the weights are read twice
-    // as often (16384 rows of 64: 59.7 against 46.7).
-    const int64_t rows = (num_tokens + kLinTokens - 1) / kLinTokens;
-    const int nt = rows * ((n + 15) / 16) <= 256 ? 1 : 2;
-    const dim3 tiles((unsigned)rows, (unsigned)((n + 16 * nt - 1) / (16 * nt)));
-#define SP_LIN(NT) \
-  linear_f32_mfma_kernel<NT><<<tiles, kLinWaves * 64, 0, (hipStream_t)stream>>>(out, (const char*)x, x_stride, weight, bias, num_tokens, k, n)
-    if (nt == 1) SP_LIN(1);
-    else SP_LIN(2);
-#undef SP_LIN
-    SP_LAUNCH_CHECK();
-    return SP_OK;
+    // (up to 64 rows a workgroup per row has the shorter chain.)  Workgroups of 32 tokens, two of which fit a CU; of 64, one a CU, which
+    // read the weights half as often, where their rounds are at least half full and not more than two (us, 32 / 64: 4096 rows of 32
+    // outputs 6.7 / 8.4, of 64 10.3 / 9.1, of 128 15.9 / 14.9; 9000 of 32 16.9 / 18.8; 16384 of 64 43.3 / 48.4).  The order of the sums is the same.
+    const int64_t nb = (n + kLinOut - 1) / kLinOut, wide = (num_tokens + 63) / 64 * nb;
+    if ((num_tokens + 31) / 32 * nb > 256 && wide <= 512 && (wide + 255) % 256 >= 127)
+      return launch_linear_f32<4, 8>(out, (const char*)x, x_stride, weight, bias, num_tokens, k, n, (hipStream_t)stream);
+    return launch_linear_f32<2, 8>(out, (const char*)x, x_stride, weight, bias, num_tokens, k, n, (hipStream_t)stream);
   }
   const dim3 grid((unsigned)num_tokens, (unsigned)((n + 15) / 16));
   if (k % 4 == 0 && ((uintptr_t)weight & 15) == 0)

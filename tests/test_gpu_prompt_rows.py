@@ -186,6 +186,19 @@ def test_fp32_products_of_many_rows(T, K, n, bias):
     assert out.shape == (T, n) and bool(((out.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("T,K,n", [(2100, 1056, 64), (4097, 96, 17), (8193, 64, 16)])       # tiles of 64 rows, the last of few; of 32 rows again
+def test_fp32_products_of_more_rows(T, K, n):
+    from scratchpad_amd import _native
+    g = torch.Generator(device=DEV).manual_seed(T + K + n)
+    x = torch.randn(T, K, generator=g, device=DEV).bfloat16()
+    w = torch.randn(n, K, generator=g, device=DEV)
+    out = _native.small_linear_f32(x, w)
+    bound = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((out.double() - x.double() @ w.double().T).abs() <= bound).all())
+    few = _native.small_linear_f32(x[T - 70:], w)                     # the order of a row's sum is K's alone
+    assert torch.equal(out[T - 70:], few)
+
+
 @pytest.mark.parametrize("T", [64, 65, 100])
 def test_fp32_products_of_infinite_inputs(T):
     """an infinity is one in the sum it enters, in every form: not NaN"""
