@@ -44,7 +44,7 @@ struct ExtendArgs {
   // keys of a row block shared by `splits` workgroups (1: none): each leaves its unnormalised O^T tile and the rows' maximum and sum
   // in 32 bits, tile ((item * gridDim.x + kv-head group) * waves + wave) * splits + split, for extend_merge_kernel
   int splits;
-  int half_blocks;      // 1: a workgroup of four waves takes half a row block (heads of 64)
+  int half_blocks;      // 1: a workgroup's eight waves take half a row block (heads of 64)
   float* part_o;        // per tile: [D / 4][32 rows][4]
   float* part_ml;       // per tile: 32 maxima (log2 domain), 32 sums
 };

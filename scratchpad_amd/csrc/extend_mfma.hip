@@ -74,10 +74,16 @@ __device__ __forceinline__ int64_t split_tile(const ExtendArgs& a, int wave) {
 
 // PLAIN: no logit cap and no sliding window (both compiled out of the tile loop)
 // SPLIT: the row block's tiles are shared by a.splits workgroups (blockIdx.z), see ExtendArgs::splits
-template <typename Tag, int D, int GK, int NW, bool KV8, bool PLAIN, bool DMA, bool SPLIT = false>
-__global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
+// FORM: the waves, 8; kPairs: half a row block by eight waves - the first four take its even tiles, the others the odd ones, and their sums
+// meet in LDS at the end
+constexpr int kPairs = 16;
+template <typename Tag, int D, int GK, int FORM, bool KV8, bool PLAIN, bool DMA, bool SPLIT = false>
+__global__ __launch_bounds__((FORM == kPairs ? 8 : FORM) * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
+  constexpr bool PAIR = FORM == kPairs;
+  constexpr int NW = PAIR ? 8 : FORM;
   static_assert(!DMA || ((D == 128 || D == 64) && !KV8), "the LDS-DMA images are laid out for 256- / 128-byte rows");
-  static_assert(NW == 8 || (NW == 4 && D == 64 && !SPLIT), "a row block of 8 waves, or one half of it");
+  static_assert(NW == 8, "a row block of 8 waves, or one half of it");
+  static_assert(!PAIR || (D == 64 && !SPLIT), "two tiles are in LDS at a time");
   constexpr int NT = NW * 64;
   constexpr int NB = 2;                // LDS tile buffers: tile t lives in buffer t & 1
   typedef ExtCfg<D, NT> C;
@@ -85,7 +91,8 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
   typedef typename std::conditional<KV8, u32x2, u32x4>::type raw_t;   // one thread's gathered chunk
   constexpr int BN = C::BN, SK = C::SK, SV = C::SV, CPR = C::CPR, RPP = C::RPP, PASSES = C::PASSES;
   constexpr int KSTEPS = C::KSTEPS, DBLK = C::DBLK;
-  constexpr int BM = 32 * (NW / GK);
+  constexpr int RW = PAIR ? NW / 2 : NW;             // waves that share the rows
+  constexpr int BM = 32 * (RW / GK);
   extern __shared__ __attribute__((aligned(16))) char lds[];
 #ifdef SP_EXTEND_WGSTAMPS
   unsigned long long wg0 = 0, wg1 = 0, wg2 = 0, wg3 = 0, wg4 = 0;
@@ -93,8 +100,8 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
 #endif
 
   int b, row0;
-  // four waves: blockIdx.z names the half of the 8-wave row block
-  constexpr int HALVES = 8 / NW;
+  // half a row block: blockIdx.z names which
+  constexpr int HALVES = 8 / RW;
   const int half = HALVES == 1 ? 0 : (int)blockIdx.z % HALVES;
   if (SPLIT || a.plan) {                           // planned: items are sorted heaviest first
     if (!extend_item(a, BM * HALVES, (int)blockIdx.y, b, row0)) return;
@@ -130,7 +137,7 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int c = lane & 31, h = lane >> 5;
-  const int g = wave % GK, rb = wave / GK;
+  const int g = wave % GK, rb = wave % RW / GK;
   const int head = hk * G + hh * GK + g;
   const int r0 = row0 + rb * 32;                   // this wave's first query row
   const int my_row = r0 + c;                       // this lane's query row (may be >= E: masked out)
@@ -189,14 +196,16 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
   // walk the same keys in step, so every tile's first touch is an HBM miss for all of them at once).
   // Slot indices of a set's NEXT tile are fetched right after its gathers are issued, so the
   // dependent req_to_token -> row chain is never waited for inside the loop.
+  constexpr int TPS = PAIR ? 2 : 1;                // tiles of a step
+  const int mine = PAIR ? __builtin_amdgcn_readfirstlane(wave / RW) : 0;      // this wave's tile of a step
   struct RegSet {
-    raw_t k[PASSES], v[PASSES];
-    int slot[PASSES];
+    raw_t k[TPS * PASSES], v[TPS * PASSES];
+    int slot[TPS * PASSES];
   };
   RegSet setA, setB;
-  auto fetch_slots = [&](RegSet& r, int tile) __attribute__((always_inline)) {
+  auto fetch_slots = [&](RegSet& r, int tile) __attribute__((always_inline)) {      // of the step that starts with `tile`
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
+    for (int p = 0; p < TPS * PASSES; ++p) {
       // rows past the end re-read the last valid key (masked in the softmax; real, finite K/V so a
       // zero probability times its V row is zero).  No conditional load and no select on the loaded
       // value: a load the wave may skip makes the compiler's count of outstanding loads ambiguous
@@ -206,21 +215,21 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
       r.slot[p] = idx_row[max(min(key, kv_len - 1), 0)];
     }
   };
-  auto prefetch = [&](RegSet& r, int tile) __attribute__((always_inline)) {   // gathers of `tile` from r.slot, then the indices of tile+2
+  auto prefetch = [&](RegSet& r, int tile) __attribute__((always_inline)) {   // gathers of a step from r.slot, then the indices of the one after the next
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
+    for (int p = 0; p < TPS * PASSES; ++p) {
       const int64_t off = (int64_t)r.slot[p] * tok_bytes + head_off;
       r.k[p] = *(const raw_t*)(a.kbuf + off);
       r.v[p] = *(const raw_t*)(a.vbuf + off);
     }
-    fetch_slots(r, tile + 2);
+    fetch_slots(r, tile + 2 * TPS);
   };
   auto stage = [&](const RegSet& r, int buf) __attribute__((always_inline)) {
-    char* dK = lds + buf * C::kTileBytes;
-    char* dV = dK + BN * SK;
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
-      const int row = p * RPP + st_row;
+    for (int p = 0; p < TPS * PASSES; ++p) {
+      char* dK = lds + (buf + p / PASSES) * C::kTileBytes;
+      char* dV = dK + BN * SK;
+      const int row = p % PASSES * RPP + st_row;
       if constexpr (KV8) {
         st16(dK + row * SK + st_ch * 16, expand_e5m2x8(r.k[p]));
         st16(dV + row * SV + st_ch * 16, expand_e5m2x8(r.v[p]));
@@ -246,11 +255,11 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
   // Four K and four V buffers (D = 128: 128 KiB; D = 64: 64 KiB).
   constexpr int kRowB = 2 * D;                       // bytes of a K / V row in LDS
   constexpr int kDmaTile = 64 * kRowB;
-  constexpr int kDmaBufs = 4;   // tile t is consumed from buffer t % 4 while t+1, t+2 and t+3 are in flight
+  constexpr int kDmaBufs = PAIR ? 8 : 4;   // tile t is consumed from buffer t % 4 while t+1, t+2 and t+3 are in flight (PAIR: pairs of tiles)
   constexpr int kCPR = kRowB / 16;                   // 16-byte chunks per row (16 / 8)
   constexpr int kRPP = 64 / kCPR;                    // rows per DMA piece (4 / 8)
   constexpr int kRPW = 64 / NW;                      // rows a wave fetches of every tile
-  constexpr int kPPW = kRPW / kRPP;                  // its pieces, each for K and for V (8 waves: 2 / 1, 4 waves: 2 at D = 64)
+  constexpr int kPPW = kRPW / kRPP;                  // its pieces, each for K and for V (2 / 1)
   const int k_swz = D == 128 ? ((c & 15) ^ h) : (((c >> 1) & 7) ^ h);
   // pipeline: the gathers of tiles t+1 and t+2 fly during compute(t); tile t+1 is written to the other
   // LDS buffer right after compute(t), and one barrier per tile both publishes tile t+1 and retires
@@ -479,6 +488,57 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
                                          (__attribute__((address_space(3))) void*)(kd + kDmaBufs * kDmaTile), 16, 0, 0);
       }
     };
+    if constexpr (PAIR) {
+      // Steps of two tiles, one for each four waves, through rings of four steps; otherwise as below: a step issues the index loads of step + 5
+      // and the four pieces of step + 3, and all but the eight youngest operations have landed at its end.
+      const int steps = (ntiles - tbeg + 1) / 2;
+      static_assert(kPPW == 1, "a piece of each tile's keys and values per wave");
+      struct Pair { Slots t[2]; };
+      Pair p0, p1, p2, p3;
+      auto load_pair = [&](Pair& r, int n) __attribute__((always_inline)) {
+        load_slots(r.t[0], tbeg + 2 * n);
+        load_slots(r.t[1], tbeg + 2 * n + 1);
+      };
+      auto dma_pair = [&](const Pair& r, int n4) __attribute__((always_inline)) {
+        dma(r.t[0], 2 * n4);
+        dma(r.t[1], 2 * n4 + 1);
+      };
+      load_pair(p0, 0);
+      load_pair(p1, 1);
+      load_pair(p2, 2);
+      dma_pair(p0, 0);
+      load_pair(p3, 3);
+      load_pair(p0, 4);
+      __builtin_amdgcn_sched_barrier(0);
+      dma_pair(p1, 1);
+      dma_pair(p2, 2);
+      __builtin_amdgcn_s_waitcnt(0x0F78);   // vmcnt(8): the first step's tiles have landed
+      asm volatile("s_barrier" ::: "memory");
+      auto step = [&](int n, int n4, Pair& refill, const Pair& next) __attribute__((always_inline)) {
+        load_pair(refill, n + 5);
+        dma_pair(next, (n4 + 3) % 4);
+        const int t = tbeg + 2 * n + mine;
+        u32x4 pf[4];
+        if (t < ntiles && qk_softmax(t, 2 * n4 + mine, pf)) pv(2 * n4 + mine, pf);
+        __builtin_amdgcn_s_waitcnt(0x0078);   // vmcnt(8) lgkmcnt(0)
+        asm volatile("s_barrier" ::: "memory");
+      };
+      int n = 0;
+      for (; n + 3 < steps; n += 4) {
+        step(n, 0, p1, p3);
+        step(n + 1, 1, p2, p0);
+        step(n + 2, 2, p3, p1);
+        step(n + 3, 3, p0, p2);
+      }
+      if (n < steps) {
+        step(n, 0, p1, p3);
+        if (n + 1 < steps) {
+          step(n + 1, 1, p2, p0);
+          if (n + 2 < steps) step(n + 2, 2, p3, p1);
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): no DMA may outlive the workgroup's LDS
+    } else {
     // The compiler does not track LDS-DMA arrivals: the waits are placed by hand.  A tile step issues
     // kPPW index loads (tile +5) and the 2 kPPW DMA pieces of tile +3 (D = 128: 2 + 4; D = 64: 1 + 2); before the
     // barrier that publishes tile +1, everything up to ITS pieces must have landed, i.e. all but the pieces of tiles
@@ -554,27 +614,29 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): no DMA may outlive the workgroup's LDS
     SP_WGSTAMP(wg3);
+    }
   } else {
   fetch_slots(setA, tbeg);
-  fetch_slots(setB, tbeg + 1);
+  fetch_slots(setB, tbeg + TPS);
   prefetch(setA, tbeg);
-  prefetch(setB, tbeg + 1);
-  stage(setA, tbeg & 1);
+  prefetch(setB, tbeg + TPS);
+  stage(setA, 0);
   __syncthreads();
-  // one tile: `fill` is the free register set (it receives tile t+2), `next` holds tile t+1
-  auto tile_step = [&](int t, RegSet& fill, const RegSet& next) __attribute__((always_inline)) {
+  // one step: `fill` is the free register set (it receives step n + 2), `next` holds step n + 1
+  auto tile_step = [&](int n, RegSet& fill, const RegSet& next) __attribute__((always_inline)) {
     SP_STAMP(ts0);
     // unconditional, also past the last tile (rows of the last valid key, never consumed): see fetch_slots
-    prefetch(fill, t + 2);
+    const int t = tbeg + n * TPS, buf = (n & 1) * TPS + mine;
+    prefetch(fill, t + 2 * TPS);
     SP_STAMP(ts1);
     u32x4 pf[4];
-    const bool visible = qk_softmax(t, t & 1, pf);
-    if (visible) pv(t & 1, pf);
+    const bool visible = (!PAIR || t + mine < ntiles) && qk_softmax(t + mine, buf, pf);
+    if (visible) pv(buf, pf);
 #ifdef SP_EXTEND_STAMPS
     if (!visible) ts2 = ts3 = ts1;
 #endif
     SP_STAMP(ts4);
-    stage(next, (t + 1) & 1);   // past the last tile: dummy rows into the buffer nobody reads again
+    stage(next, ((n + 1) & 1) * TPS);   // past the last tile: dummy rows into the buffer nobody reads again
     SP_STAMP(ts5);
     __syncthreads();
     SP_STAMP(ts6);
@@ -592,12 +654,13 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
   // whole pairs in the loop, an odd last tile after it: with the second step under a condition the
   // compiler sees a path from the first step straight to the loop head, where set A's indices would
   // be the youngest loads, and waits vmcnt(0) at the top of EVERY iteration
-  int t = tbeg;
-  for (; t + 1 < ntiles; t += 2) {
-    tile_step(t, setA, setB);
-    tile_step(t + 1, setB, setA);
+  const int steps = (ntiles - tbeg + TPS - 1) / TPS;
+  int n = 0;
+  for (; n + 1 < steps; n += 2) {
+    tile_step(n, setA, setB);
+    tile_step(n + 1, setB, setA);
   }
-  if (t < ntiles) tile_step(t, setA, setB);
+  if (n < steps) tile_step(n, setA, setB);
   }
 #ifdef SP_EXTEND_STAMPS
   if (lane == 0 && g_stamp_buf) {
@@ -605,13 +668,37 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
   }
 #endif
 
+  if constexpr (PAIR) {
+    // the second four waves' sums to the first: one share of each row, weighed by the distance of its maximum
+    __syncthreads();
+    float* const over = (float*)lds + (wave % RW) * (DBLK * 16 + 2) * 64 + lane;
+    l_part += xchg32(l_part);
+    if (mine) {
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) over[(db * 16 + r) * 64] = oacc[db][r];
+      over[DBLK * 16 * 64] = m_run;
+      over[(DBLK * 16 + 1) * 64] = l_part;
+    }
+    __syncthreads();
+    if (!mine) {
+      const float m2 = over[DBLK * 16 * 64], m_new = fmaxf(m_run, m2);
+      const float w1 = __builtin_amdgcn_exp2f(m_run - m_new), w2 = __builtin_amdgcn_exp2f(m2 - m_new);
+      l_part = __builtin_fmaf(over[(DBLK * 16 + 1) * 64], w2, l_part * w1);
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[db][r] = __builtin_fmaf(over[(db * 16 + r) * 64], w2, oacc[db][r] * w1);
+    }
+  }
   // ---- epilogue: O[row][head][d] = O^T[d][row] / l.  In the accumulator a lane holds 4 consecutive d of ITS row
   // per register quad: stored straight from there, every store instruction writes 64 pieces of 8 bytes
   // into 32 different rows, and the workgroup's last microseconds are store ISSUE (a workgroup's fixed
   // cost measured 10 - 13 us, a tile step 1.7 us).  The wave's 32 x D tile goes through LDS instead (the
   // tile ring is free by now: barrier first, every wave has left it and drained its DMA) and leaves as
   // whole rows, 16 bytes per lane, 4 rows of 256 B per store instruction.
-  const float l_run = l_part + xchg32(l_part);
+  const float l_run = PAIR ? l_part : l_part + xchg32(l_part);
   if constexpr (SPLIT) {
     // (the accumulators as they lie: every store writes two runs of 512 bytes; rows past the request's end are never read back)
     if (wave_live) {
@@ -633,7 +720,7 @@ __global__ __launch_bounds__(NW * 64, 2) void extend_mfma_kernel(ExtendArgs a) {
     return;
   }
   __syncthreads();
-  {
+  if (!PAIR || wave < RW) {
     constexpr int EPS = C::ROW_B + 8;                   // padded row: the 8-byte writes of 16 lanes hit 32 different banks
     char* ep = lds + wave * (32 * EPS);
     const float inv = l_run > 0.f ? a.out_scale / l_run : 0.f;  // no visible key (empty encoder): zeros
@@ -771,15 +858,16 @@ size_t extend_split_bytes(int64_t num_tokens, int num_q_heads, int head_dim) {
 // The form of a launch whose row blocks leave compute units idle (at most half as many workgroups as there are; plain attention).
 // A row block costs its workgroup about a + t * tiles, t = 1.05 us per 64-key tile at heads of 64 (vector work of two waves per SIMD), 1.15 - 1.35
 // at 128.  Two ways to use the idle units:
-//   * half_blocks (heads of 64): four waves take half a row block, one wave per SIMD, 0.8 us per tile, same bits, twice the workgroups -
-//     where the other half has rows: 4 requests of 17 behind 1000, heads of 64, 16 on 16: 15.4 | 16.5, of 64 behind 1000: 17.8 | 18.8;
+//   * half_blocks (heads of 64): eight waves take half a row block, four of them its even tiles and four the odd ones, and add up in LDS: 0.6 us
+//     per tile, twice the workgroups (four waves alone, one per SIMD: 0.8 us; a model step of 777 tokens behind 1500, 16 layers, 3146 -> 3033);
 //   * splits: workgroups share the block's keys, t * tiles / splits, and pay for the partial sums (5 us for the merge, and their traffic).
-// Taken is the one that this model puts ahead, in ns (us at one form for all | half blocks | two | four | eight shares; 16-bit pool):
-//   heads of 64, 32 on 8:   3 requests, 777 tokens behind 1500: 37.3 | 29.0 | 29.0        1, 64 behind 2000:  38.9 | 31.5 | 25.5 | 18.1 | 16.1
-//                           1, 1024 behind 2000: 55.3 | 49.5 | 40.7                       2, 200 behind 500:  15.8 | 13.6 | 14.6 | 14.3 | 14.7
-//                           1, 512: 13.6 | 11.6 | 13.9                                    1, 1024: 22.5 | 18.6 | 21.7
-//   heads of 128, byte pool:  1, 17 behind 2000: 41.6 | - | 28.0 | 19.9 | 17.7            3, 777 behind 1500: 54.6 | - | 44.2
-//                           1, 1024 behind 2000: 86.5 | - | 64.7                          1, 1024: 34.3 | - | 33.2 (not taken)
+// Taken is the one that this model puts ahead, in ns (us at one form for all | half blocks by four waves | by eight | two | four | eight shares; 16-bit pool):
+//   heads of 64, 32 on 8:   3 requests, 777 tokens behind 1500: 37.1 | 29.5 | 23.6 | 29.0 | 36.1     1, 64 behind 2000:  39.6 | 31.6 | 24.6 | 26.3 | 19.1 | 17.0
+//                           1, 1024 behind 2000: 56.0 | 51.0 | 35.4 | 40.8 | 47.7                    2, 200 behind 500:  17.1 | 14.1 | 12.8 | 16.2 | 15.3
+//                           1, 512: 13.4 | 11.2 | 10.4 | 13.7      1, 1024: 22.2 | 18.5 | 15.3 | 21.7      1, 128 behind 4000: 72.1 | 56.4 | 41.5 | 42.6 | 27.2 | 21.8
+//   heads of 128, byte pool:  1, 17 behind 2000: 41.6 | - | - | 28.0 | 19.9 | 17.7        3, 777 behind 1500: 54.6 | - | - | 44.2
+//                           1, 1024 behind 2000: 86.5 | - | - | 64.7                      1, 1024: 34.3 | - | - | 33.2 (not taken)
+// (Beside the other wave's vector work a wave's products gain nothing: the second four waves half a tile behind the first, 37.1 -> 40.2.)
 // What the 4 x 64-row kernel applies to stays whole: its forms and this file's agree to the bit, whichever of them a size selects.
 // With more than half of the units busy the same forms lose: 4 requests, 2048 tokens behind 1500, heads of 64: 45 | 46; 4096 tokens: 90 | 102.
 static void extend_small_form(ExtendArgs& a, int head_dim, int max_extend_len, int64_t max_seq_len, void* workspace,
@@ -796,16 +884,16 @@ static void extend_small_form(ExtendArgs& a, int head_dim, int max_extend_len, i
   int64_t s = std::min<int64_t>(std::min<int64_t>(kSplitGroups / groups, max_seq_len / 256), kMaxSplits);
   if (g_extend_small > 1) s = g_extend_small - 1;
   s = std::min(s, fit);
-  const int64_t tiles = max_seq_len / 64, alone = head_dim == 64 ? 800 : 1350, shared = head_dim == 64 ? 1050 : 1150;
+  const int64_t tiles = max_seq_len / 64, alone = head_dim == 64 ? 600 : 1350, shared = head_dim == 64 ? 1050 : 1150;
   if (tiles < 2 && !g_extend_small) return;
-  if (s > 1 && (g_extend_small > 2 || tiles * (alone - shared / s) > 5000 + (head_dim == 64 ? 20 : 40) * groups * s)) {
+  if (s > 1 && g_extend_small >= 0 && (g_extend_small > 2 || tiles * (alone - shared / s) > 5000 + (head_dim == 64 ? 20 : 40) * groups * s)) {
     a.splits = (int)s;
     a.plan_items = (int)items;
     a.part_o = (float*)workspace;
     a.part_ml = a.part_o + groups * kExtendWaves * s * 32 * head_dim;
+  } else if (head_dim == 64 && a.bs < 32768 && g_extend_small != 2 && fit > 0) {
+    a.half_blocks = 1;      // (a workspace without room for shares asks for the general form's order of the sums)
   }
-  // (portions of one half only would leave four waves to load what eight do)
-  else if (head_dim == 64 && (a.kv8 || g_extend_dma) && a.bs < 32768 && (max_extend_len > rows / 2 || g_extend_small == 2)) a.half_blocks = 1;
 }
 
 #define SP_EXT_SET_LDS(KERNEL, BYTES)                                                                              \
@@ -839,11 +927,18 @@ static int launch_splits(const ExtendArgs& a, int halves, hipStream_t st) {
 
 template <typename Tag, int GK>
 static int launch_half_blocks(const ExtendArgs& a, int max_extend_len, int halves, hipStream_t st) {
-  constexpr int D = 64, NW = 4, rows = 32 * (kExtendWaves / GK), kDma = 8 * 64 * 2 * D, kStaged = 2 * ExtCfg<D, NW * 64>::kTileBytes;
+  constexpr int D = 64, rows = 32 * (kExtendWaves / GK), kDma = 16 * 64 * 2 * D, kStaged = 4 * ExtCfg<D, 512>::kTileBytes;
   const dim3 grid(a.Hkv * halves, a.plan ? a.plan_items : (max_extend_len + rows - 1) / rows, 2 * (a.plan ? 1 : a.bs));
-  if (a.kv8) extend_mfma_kernel<Tag, D, GK, NW, true, true, false><<<grid, NW * 64, kStaged, st>>>(a);
-  else extend_mfma_kernel<Tag, D, GK, NW, false, true, true><<<grid, NW * 64, kDma, st>>>(a);
-  static_assert(kDma <= 64 * 1024 && kStaged <= 64 * 1024, "LDS without an attribute");
+#define SP_EXT_HALVES(KV8_, DMA_, BYTES)                                                                           \
+  do {                                                                                                           \
+    constexpr auto kernel = extend_mfma_kernel<Tag, D, GK, kPairs, KV8_, true, DMA_>;                            \
+    SP_EXT_SET_LDS(kernel, BYTES);                                                                               \
+    kernel<<<grid, 512, BYTES, st>>>(a);                                                                         \
+  } while (0)
+  if (a.kv8) SP_EXT_HALVES(true, false, kStaged);
+  else if (g_extend_dma) SP_EXT_HALVES(false, true, kDma);
+  else SP_EXT_HALVES(false, false, kStaged);
+#undef SP_EXT_HALVES
   SP_LAUNCH_CHECK();
   return SP_OK;
 }

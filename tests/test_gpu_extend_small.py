@@ -101,3 +101,37 @@ def test_shares_replay_in_a_graph(nat):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv", [(8, 2), (6, 3), (3, 3)])
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("pre,new", [([1000, 0, 64, 700, 5], [65, 1, 0, 130, 300]), ([0, 63, 64], [64, 1, 65]), ([511, 448], [1, 64])])
+def test_tiles_shared_by_the_halves_of_a_workgroup(nat, dt, causal, Hq, Hkv, kv8, pre, new):
+    """heads of 64: even and odd tiles by four waves each - one tile, odd counts, a half without a visible tile, no key at all"""
+    dtype, D = DTYPES[dt], 64
+    p, q, ext, start = extend_problem(17, Hq, Hkv, D, pre, new, dtype)
+    if kv8:
+        for name in ("k_buffer", "v_buffer"):
+            p[name] = p[name].float().to(torch.float8_e5m2).view(torch.uint8)
+    if not causal:
+        p["seq_lens"][0] = 0
+    ws = torch.empty(nat.extend_workspace_bytes(sum(new), len(new), Hq, D, dtype), dtype=torch.uint8, device=DEV)
+    plan = nat.extend_plan(ext, p["seq_lens"], sum(new), Hq, Hkv, causal)
+    outs = []
+    try:
+        nat.debug_set("extend_small", -1)
+        for pl in (plan, None):
+            o = torch.full_like(q, float("nan"))
+            nat.extend_attention(o, q, p["k_buffer"], p["v_buffer"], p["req_to_token"], p["req_pool_indices"], p["seq_lens"], ext, start, D ** -0.5,
+                                 0.0, causal, max(new), int(p["seq_lens"].max()), ws, plan=pl)
+            outs.append(o)
+    finally:
+        nat.debug_set("extend_small", 0)
+    c = cpu(p)
+    keys, values = (c[n].view(torch.float8_e5m2).float() if kv8 else c[n].float() for n in ("k_buffer", "v_buffer"))
+    oracle = lambda v: ops.extend_attention(q.cpu().float(), keys, v, c["req_to_token"], c["req_pool_indices"],  # noqa: E731
+                                            c["seq_lens"], ext.cpu(), start.cpu(), D ** -0.5, causal=causal)
+    assert torch.equal(outs[0], outs[1])
+    assert_attn_close(outs[0], oracle(values), oracle(values.abs()), dtype, what=f"half blocks {pre} {new}")
