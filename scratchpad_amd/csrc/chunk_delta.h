@@ -230,22 +230,30 @@ __device__ __forceinline__ f32x4_d mfma_d(float a, float b, const f32x4_d& c) {
 }
 
 // One workgroup per (request, head, range of the head's columns): a wave per 16 columns runs the products of chunk c while
-// kDcHelpers more waves form the operand rows of chunk c + 1 and have those of chunks c + 2 and c + 3 on their way into LDS; they
+// kDcHelpers more waves form the operand rows of a chunk ahead and have those of the two chunks after it on their way into LDS; they
 // meet at one barrier per chunk.  (The same waves doing both in turn left the matrix cores idle for two thirds of a chunk: 4.4 us.)
+// What bounds a chunk is the issue of vector and matrix instructions together: a fp32 matrix instruction takes the vector unit's 32 cycles, so its
+// 104 (3380 cycles of 5800) and every address, decay and conversion of both kinds of waves add up.  Hence rows by pointers that move on by a
+// step, masks in a request's last chunk alone, and reads of LDS between the products.  One request of 4096 tokens, 16 heads of 128:
+// 2.43 -> 2.25 us a chunk with a decay per channel, 2.2 -> 1.96 with one per head (the layer 850 -> 802 and 798 -> 742).  Operands two chunks ahead,
+// and helpers ahead of the products in the issue, gave nothing: the sum stays.
 constexpr int kDcHelpers = 4;
 
-template <typename Tag, int D, bool CHANNEL>
+// COLS: columns of a workgroup at the most
+template <typename Tag, int D, bool CHANNEL, int COLS>
 struct DeltaScanLds {
   static constexpr int kRow = D + 4;                                                     // floats per operand row
   static constexpr int kRaw = kDC * D * (2 * Elem<Tag>::kBytes + (CHANNEL ? 4 : 0));     // a chunk's k, q (and decay) rows
   static constexpr int kOps = (3 * kDC * kRow + D) * 4;                                  // Kd, Qd, Ke, G_end
   static constexpr int kOp = 3 * kRaw, kWork = kOp + 2 * kOps, kBytes = kWork + 4 * kDcFloats * 4;
+  static constexpr int kWaves = (COLS / 16 + kDcHelpers) / 4 * (COLS <= 64 && kBytes <= 80 * 1024 ? 2 : 1);      // per SIMD
+  static_assert(kBytes <= 160 * 1024, "LDS");
 };
 
-template <typename Tag, int D, bool CHANNEL>
-__global__ void __launch_bounds__(768) delta_chunk_scan_kernel(DeltaChunks a, SeqBatch sb) {
+template <typename Tag, int D, bool CHANNEL, int COLS>
+__global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag, D, CHANNEL, COLS>::kWaves)) delta_chunk_scan_kernel(DeltaChunks a, SeqBatch sb) {
   typedef Elem<Tag> E;
-  typedef DeltaScanLds<Tag, D, CHANNEL> L;
+  typedef DeltaScanLds<Tag, D, CHANNEL, COLS> L;
   constexpr int DT = D / 16, ROW = L::kRow, kRowBytes = D * E::kBytes, HT = kDcHelpers * 64;
   extern __shared__ __attribute__((aligned(16))) char delta_lds[];
   const int tid = threadIdx.x, waves = a.cols / 16;    // the first `waves` waves own columns
@@ -265,28 +273,50 @@ __global__ void __launch_bounds__(768) delta_chunk_scan_kernel(DeltaChunks a, Se
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                        (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
     };
-    const auto fetch = [&](int c) {
-      if (c >= chunks) return;
-      const int last = len - c * kDC - 1;              // the chunk's last row (or more)
+    constexpr int KU = (LK + kDcHelpers - 1) / kDcHelpers, WU = CHANNEL ? (LW + kDcHelpers - 1) / kDcHelpers : 1;
+    const char *kp[KU], *qp[KU], *wp[WU], *mp = (const char*)work + hw * 1024 + lane * 16;
+    const auto point = [&](int c, int last) {           // at chunk c, rows behind `last` as that one again
       const int64_t row0 = start + c * kDC;
-      char* raw = delta_lds + c % 3 * L::kRaw;
-      for (int u = hw; u < LK; u += kDcHelpers) {
-        const int byte = u * 1024 + lane * 16, t = byte / kRowBytes, x = byte % kRowBytes;
+#pragma unroll
+      for (int i = 0; i < KU; ++i) {
+        const int byte = (hw + i * kDcHelpers) * 1024 + lane * 16, t = byte / kRowBytes, x = byte % kRowBytes;
         const int64_t row = row0 + (t < last ? t : last);
-        load((const char*)a.k + (row * a.k_stride + qc) * E::kBytes + x, raw + u * 1024);
-        load((const char*)a.q + (row * a.q_stride + qc) * E::kBytes + x, raw + (LK + u) * 1024);
+        kp[i] = (const char*)a.k + (row * a.k_stride + qc) * E::kBytes + x;
+        qp[i] = (const char*)a.q + (row * a.q_stride + qc) * E::kBytes + x;
       }
-      for (int u = hw; u < LW; u += kDcHelpers) {
-        const int byte = u * 1024 + lane * 16, t = byte / (D * 4), x = byte % (D * 4);
+#pragma unroll
+      for (int i = 0; CHANNEL && i < WU; ++i) {
+        const int byte = (hw + i * kDcHelpers) * 1024 + lane * 16, t = byte / (D * 4), x = byte % (D * 4);
         const int64_t row = row0 + (t < last ? t : last);
-        load((const char*)(a.decay + row * a.H * D + (int64_t)h * D) + x, raw + (2 * LK + u) * 1024);
-      }
-      for (int u = hw; u < LM; u += kDcHelpers) {
-        const int byte = u * 1024 + lane * 16;
-        if (byte < kDcFloats * 4)
-          load((const char*)(work + (int64_t)c * a.H * kDcFloats) + byte, delta_lds + L::kWork + (c & 3) * kDcFloats * 4 + u * 1024);
+        wp[i] = (const char*)(a.decay + row * a.H * D + (int64_t)h * D) + x;
       }
     };
+    const int64_t kstep = kDC * a.k_stride * E::kBytes, qstep = kDC * a.q_stride * E::kBytes, wstep = (int64_t)kDC * a.H * D * 4,
+                  mstep = (int64_t)a.H * kDcFloats * 4;
+    static_assert(kDcFloats * 4 <= kDcHelpers * 1024, "one load of the matrices per helper");
+    const auto fetch = [&](int c) {                    // (c = 0, 1, 2 ...)
+      if (c >= chunks) return;
+      char* raw = delta_lds + c % 3 * L::kRaw;
+      if (c == chunks - 1) point(c, len - c * kDC - 1);
+#pragma unroll
+      for (int i = 0; i < KU; ++i) {
+        const int u = hw + i * kDcHelpers;
+        if (u < LK) {
+          load(kp[i], raw + u * 1024);
+          load(qp[i], raw + (LK + u) * 1024);
+        }
+        kp[i] += kstep, qp[i] += qstep;
+      }
+#pragma unroll
+      for (int i = 0; CHANNEL && i < WU; ++i) {
+        const int u = hw + i * kDcHelpers;
+        if (u < LW) load(wp[i], raw + (2 * LK + u) * 1024);
+        wp[i] += wstep;
+      }
+      if (hw * 1024 + lane * 16 < kDcFloats * 4) load(mp, delta_lds + L::kWork + (c & 3) * kDcFloats * 4 + hw * 1024);
+      mp += mstep;
+    };
+    point(0, kDC);
     // operand rows of a chunk: a thread walks a channel forward (Kd, Qd, G_end) or backward (Ke); rows behind the end are zeros
     const auto operands = [&](int c, auto whole) {
       const int n = len - c * kDC;
@@ -363,7 +393,7 @@ __global__ void __launch_bounds__(768) delta_chunk_scan_kernel(DeltaChunks a, Se
   const bool held = sb.extend_prefix_lens[b] > 0;
   const int64_t slot = load_idx(sb.req_pool_indices, b, sb.idx64);
   const int col = blockIdx.z * a.cols + 16 * wave + r16;
-  const bool live = col < a.Dv;                        // (Dv is a multiple of 16: whole waves)
+  const bool live = __builtin_amdgcn_readfirstlane(col < a.Dv);      // (Dv is a multiple of 16: whole waves)
   float* st = a.state + slot * a.state_stride + (int64_t)h * D * a.Dv + (live ? col : 0);
   const int64_t vc = (int64_t)h * a.Dv + (live ? col : 0);
   f32x4_d S[DT];
@@ -373,14 +403,27 @@ __global__ void __launch_bounds__(768) delta_chunk_scan_kernel(DeltaChunks a, Se
     for (int r = 0; r < 4; ++r) S[i][r] = held && live ? st[(int64_t)(16 * i + 4 * q + r) * a.Dv] : 0.f;
   float v[4];
   typename E::storage vn[4];                           // the next chunk's values as they lie in memory
-  const auto fetch_v = [&](int c) {
-    const int last = len - c * kDC - 1;
+  const char* vp[4];
+  char* op[4];
+  const int64_t vstep = kDC * a.v_stride * E::kBytes, ostep = (int64_t)kDC * a.H * a.Dv * 4;
+  const auto point_v = [&](int c, int last) {          // as the helpers'
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 4 * q + r;
-      vn[r] = ((const typename E::storage*)a.v)[(start + c * kDC + (t < last ? t : last)) * a.v_stride + vc];
+      vp[r] = (const char*)a.v + ((start + c * kDC + (t < last ? t : last)) * a.v_stride + vc) * E::kBytes;
     }
   };
+  const auto fetch_v = [&](int c) {
+    if (c == chunks - 1) point_v(c, len - c * kDC - 1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      vn[r] = *(const typename E::storage*)vp[r];
+      vp[r] += vstep;
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < 4; ++r) op[r] = (char*)(a.raw + (start + 4 * q + r) * (int64_t)a.H * a.Dv + vc);
+  point_v(0, kDC);
   fetch_v(0);
   lds_barrier();
   lds_barrier();
@@ -388,59 +431,65 @@ __global__ void __launch_bounds__(768) delta_chunk_scan_kernel(DeltaChunks a, Se
     const int n = len - c * kDC;
     const float* m = (const float*)(delta_lds + L::kWork + (c & 3) * kDcFloats * 4);
     const float* ops = (const float*)(delta_lds + L::kOp + (c & 1) * L::kOps);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = 4 * q + r < n ? E::load(&vn[r], 0) : 0.f;
-    if (c + 1 < chunks) fetch_v(c + 1);
-    // the operands of the next products are read while the matrix cores are on the ones before (left to itself the compiler keeps
-    // registers free and waits for each read)
-    f32x4_d kd = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f}, ak[DT], aq[DT], g[DT];
+    // Every read of LDS goes out between two products: in one piece the four waves' reads hold their products up until LDS has taken them
+    // (left to itself the compiler keeps registers free and waits for each read).
+    f32x4_d kd = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f}, ak[DT], aq[DT], g[DT], tr, pr;
     float ke[4][DT];
+    const auto read_k = [&](int i) { ak[i] = *(const f32x4_d*)&ops[r16 * ROW + 16 * i + 4 * q]; };
+    read_k(0);
+    read_k(1);
 #pragma unroll
     for (int i = 0; i < DT; ++i) {
-      ak[i] = *(const f32x4_d*)&ops[r16 * ROW + 16 * i + 4 * q];
+      if (i + 2 < DT) read_k(i + 2);
       aq[i] = *(const f32x4_d*)&ops[(kDC + r16) * ROW + 16 * i + 4 * q];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    const auto read_state = [&](int i0, int i1) {
+      if (i == DT - 1) tr = *(const f32x4_d*)&m[kDcT + r16 * kDC + 4 * q];
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = i0; i < i1; ++i)
+      for (int r = 0; r < 4; ++r) kd = mfma_d(ak[i][r], S[i][r], kd);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = E::load(&vn[r], 0);
+    if (n < kDC) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = 4 * q + r < n ? v[r] : 0.f;
+    }
+    if (c + 1 < chunks) fetch_v(c + 1);
+#pragma unroll
+    for (int i = 0; i < DT; ++i) {
+      g[i] = *(const f32x4_d*)&ops[3 * kDC * ROW + 16 * i + 4 * q];
+      if (i == 0) pr = *(const f32x4_d*)&m[kDcP + r16 * kDC + 4 * q];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        __builtin_amdgcn_sched_barrier(0);
+        ke[r][i] = ops[(2 * kDC + 4 * q + r) * ROW + 16 * i + r16];
+        __builtin_amdgcn_sched_barrier(0);
+        o = mfma_d(aq[i][r], S[i][r], o);
+      }
+      if (i == 1) {
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          kd = mfma_d(ak[i][r], S[i][r], kd);
-          o = mfma_d(aq[i][r], S[i][r], o);
+          v[r] -= kd[r];
+          u = mfma_d(tr[r], v[r], u);
         }
-    };
-    read_state(0, DT / 2);
-    __builtin_amdgcn_sched_barrier(0);
-    const f32x4_d tr = *(const f32x4_d*)&m[kDcT + r16 * kDC + 4 * q], pr = *(const f32x4_d*)&m[kDcP + r16 * kDC + 4 * q];
+      }
+      if (i > 0) {
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < DT; ++i) g[i] = *(const f32x4_d*)&ops[3 * kDC * ROW + 16 * i + 4 * q];
-    __builtin_amdgcn_sched_barrier(0);
-    read_state(DT / 2, DT);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int i = 0; i < DT; ++i) ke[r][i] = ops[(2 * kDC + 4 * q + r) * ROW + 16 * i + r16];
-    __builtin_amdgcn_sched_barrier(0);
-    f32x4_d u = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      v[r] -= kd[r];
-      u = mfma_d(tr[r], v[r], u);
+        for (int r = 0; r < 4; ++r) S[i - 1][r] *= g[i - 1][r];
+      }
     }
 #pragma unroll
-    for (int i = 0; i < DT; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S[i][r] *= g[i][r];
+    for (int r = 0; r < 4; ++r) S[DT - 1][r] *= g[DT - 1][r];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r], S[i]);
+    for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[0][i], u[0], S[i]);
     int first = kDC;                                  // the column's first token whose u is not finite
+    f32x4_d uf = u;
     const float probe = fmaf(u[0], 0.f, fmaf(u[1], 0.f, fmaf(u[2], 0.f, u[3] * 0.f)));
-    if (__ballot(probe != probe)) {
+    const bool odd = __ballot(probe != probe) != 0;
+    if (odd) {
       const auto finite = [](float x) { return fabsf(x) < INFINITY; };
 #pragma unroll
       for (int r = 3; r >= 0; --r)
@@ -448,27 +497,33 @@ __global__ void __launch_bounds__(768) delta_chunk_scan_kernel(DeltaChunks a, Se
           v[r] = 0.f;
           first = 4 * q + r;
         }
-      u = f32x4_d{0.f, 0.f, 0.f, 0.f};
+      uf = f32x4_d{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) u = mfma_d(tr[r], v[r], u);
+      for (int r = 0; r < 4; ++r) uf = mfma_d(tr[r], v[r], uf);
 #pragma unroll
       for (int r = 3; r >= 0; --r)
-        if (!finite(u[r])) first = min(first, 4 * q + r);
+        if (!finite(uf[r])) first = min(first, 4 * q + r);
       first = min(first, __shfl_xor(first, 16, 64));
       first = min(first, __shfl_xor(first, 32, 64));
 #pragma unroll
-      for (int r = 0; r < 4; ++r) u[r] = 4 * q + r < first ? u[r] : 0.f;
+      for (int r = 0; r < 4; ++r) uf[r] = 4 * q + r < first ? uf[r] : 0.f;
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o = mfma_d(pr[r], u[r], o);
-    if (__ballot(first < kDC)) {
+    for (int r = 0; r < 4; ++r) o = mfma_d(pr[r], uf[r], o);
+#pragma unroll
+    for (int r = 1; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r], S[i]);
+    if (odd) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = 4 * q + r < first ? o[r] : as_f32(0x7fc00000u);
     }
     if (live) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (4 * q + r < n) a.raw[(start + c * kDC + 4 * q + r) * (int64_t)a.H * a.Dv + vc] = o[r];
+      for (int r = 0; r < 4; ++r) {
+        if (n >= kDC || 4 * q + r < n) *(float*)op[r] = o[r];
+        op[r] += ostep;
+      }
     }
     lds_barrier();
   }
@@ -488,6 +543,24 @@ inline bool delta_chunks_take(const DeltaChunks& a, int D, int dtype, const SeqB
          (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.decay | (uintptr_t)a.work) & 15) == 0;
 }
 
+template <typename Tag, int D, bool CHANNEL, int COLS>
+int launch_delta_scan(const DeltaChunks& a, const SeqBatch& s, hipStream_t st) {
+  constexpr int lds = DeltaScanLds<Tag, D, CHANNEL, COLS>::kBytes;
+  if (lds > 64 * 1024) {
+    static PerDevice<int> raised;
+    int ok = 0;
+    raised.get(ok, [&](int) {
+      return hipFuncSetAttribute((const void*)delta_chunk_scan_kernel<Tag, D, CHANNEL, COLS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) ==
+             hipSuccess ? 1 : 0;
+    });
+    if (!ok) return SP_ERR_LAUNCH;
+  }
+  delta_chunk_scan_kernel<Tag, D, CHANNEL, COLS><<<dim3((unsigned)s.B, (unsigned)a.H, (unsigned)((a.Dv + a.cols - 1) / a.cols)),
+                                                   a.cols * 4 + kDcHelpers * 64, lds, st>>>(a, s);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
+
 template <typename Tag, int D, bool CHANNEL>
 int launch_delta_chunks(DeltaChunks a, const SeqBatch& s, hipStream_t st) {
   const int64_t chunks = a.T / kDC + s.B;              // at most: a request's last chunk may be partial
@@ -499,20 +572,7 @@ int launch_delta_chunks(DeltaChunks a, const SeqBatch& s, hipStream_t st) {
   a.cols = 128;
   while (a.cols > 64 && (int64_t)s.B * a.H * ((a.Dv + a.cols - 1) / a.cols) < 256) a.cols /= 2;
   if (a.cols > a.Dv) a.cols = a.Dv;
-  constexpr int lds = DeltaScanLds<Tag, D, CHANNEL>::kBytes;
-  if (lds > 64 * 1024) {
-    static PerDevice<int> raised;
-    int ok = 0;
-    raised.get(ok, [&](int) {
-      return hipFuncSetAttribute((const void*)delta_chunk_scan_kernel<Tag, D, CHANNEL>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) ==
-             hipSuccess ? 1 : 0;
-    });
-    if (!ok) return SP_ERR_LAUNCH;
-  }
-  delta_chunk_scan_kernel<Tag, D, CHANNEL><<<dim3((unsigned)s.B, (unsigned)a.H, (unsigned)((a.Dv + a.cols - 1) / a.cols)),
-                                             a.cols * 4 + kDcHelpers * 64, lds, st>>>(a, s);
-  SP_LAUNCH_CHECK();
-  return SP_OK;
+  return a.cols <= 64 ? launch_delta_scan<Tag, D, CHANNEL, 64>(a, s, st) : launch_delta_scan<Tag, D, CHANNEL, 128>(a, s, st);
 }
 
 }  // namespace sp
