@@ -317,7 +317,8 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
       mp += mstep;
     };
     point(0, kDC);
-    // operand rows of a chunk: a thread walks a channel forward (Kd, Qd, G_end) or backward (Ke); rows behind the end are zeros
+    // operand rows of a chunk: a thread walks a channel forward (Kd, Qd, G_end) or backward (Ke); rows behind the end are zeros.  The
+    // norms of k and q are the products': 12 multiplications of a wave that owns columns for 48 of a channel's two threads here.
     const auto operands = [&](int c, auto whole) {
       const int n = len - c * kDC;
       const char* raw = delta_lds + c % 3 * L::kRaw;
@@ -329,17 +330,11 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
         const bool fwd = role < D;                     // (D is a multiple of 64: whole waves)
         typename E::storage kr[kDC], qr[kDC];
         float w[kDC];
-        f32x4_d ik[kDC / 4], iq[kDC / 4];
 #pragma unroll
         for (int t = 0; t < kDC; ++t) {                // every read on its way before the first is used
           w[t] = CHANNEL ? wr[t * D + d] : m[kDcW + t];
           kr[t] = ((const typename E::storage*)raw)[t * D + d];
           qr[t] = ((const typename E::storage*)(raw + (fwd ? kDC * kRowBytes : 0)))[t * D + d];
-        }
-#pragma unroll
-        for (int x = 0; x < kDC / 4; ++x) {
-          ik[x] = *(const f32x4_d*)&m[kDcIk + 4 * x];
-          iq[x] = *(const f32x4_d*)&m[kDcIq + 4 * x];
         }
         __builtin_amdgcn_sched_barrier(0);
         float k[kDC];
@@ -347,7 +342,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
         for (int t = 0; t < kDC; ++t) {
           const bool on = whole || t < n;
           if (!on) w[t] = 1.f;
-          k[t] = on ? E::load(&kr[t], 0) * ik[t / 4][t % 4] : 0.f;
+          k[t] = on ? E::load(&kr[t], 0) : 0.f;
         }
         float g = 1.f;
         if (fwd) {
@@ -355,7 +350,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
           for (int t = 0; t < kDC; ++t) {
             g *= w[t];
             ops[t * ROW + d] = k[t] * g;
-            ops[(kDC + t) * ROW + d] = whole || t < n ? E::load(&qr[t], 0) * iq[t / 4][t % 4] * g : 0.f;
+            ops[(kDC + t) * ROW + d] = whole || t < n ? E::load(&qr[t], 0) * g : 0.f;
           }
           ops[3 * kDC * ROW + d] = g;
         } else {
@@ -433,7 +428,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
     const float* ops = (const float*)(delta_lds + L::kOp + (c & 1) * L::kOps);
     // Every read of LDS goes out between two products: in one piece the four waves' reads hold their products up until LDS has taken them
     // (left to itself the compiler keeps registers free and waits for each read).
-    f32x4_d kd = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f}, ak[DT], aq[DT], g[DT], tr, pr;
+    f32x4_d kd = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f}, ak[DT], aq[DT], g[DT], tr, pr, ik, iq;
     float ke[4][DT];
     const auto read_k = [&](int i) { ak[i] = *(const f32x4_d*)&ops[r16 * ROW + 16 * i + 4 * q]; };
     read_k(0);
@@ -442,6 +437,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
     for (int i = 0; i < DT; ++i) {
       if (i + 2 < DT) read_k(i + 2);
       aq[i] = *(const f32x4_d*)&ops[(kDC + r16) * ROW + 16 * i + 4 * q];
+      if (i == DT - 2) ik = *(const f32x4_d*)&m[kDcIk + 4 * q];
       if (i == DT - 1) tr = *(const f32x4_d*)&m[kDcT + r16 * kDC + 4 * q];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -459,6 +455,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
     for (int i = 0; i < DT; ++i) {
       g[i] = *(const f32x4_d*)&ops[3 * kDC * ROW + 16 * i + 4 * q];
       if (i == 0) pr = *(const f32x4_d*)&m[kDcP + r16 * kDC + 4 * q];
+      if (i == 1) iq = *(const f32x4_d*)&m[kDcIq + 4 * q];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         __builtin_amdgcn_sched_barrier(0);
@@ -470,7 +467,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          v[r] -= kd[r];
+          v[r] = fmaf(-kd[r], ik[r], v[r]);
           u = mfma_d(tr[r], v[r], u);
         }
       }
@@ -484,7 +481,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
     for (int r = 0; r < 4; ++r) S[DT - 1][r] *= g[DT - 1][r];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[0][i], u[0], S[i]);
+    for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[0][i], u[0] * ik[0], S[i]);
     int first = kDC;                                  // the column's first token whose u is not finite
     f32x4_d uf = u;
     const float probe = fmaf(u[0], 0.f, fmaf(u[1], 0.f, fmaf(u[2], 0.f, u[3] * 0.f)));
@@ -508,12 +505,13 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
 #pragma unroll
       for (int r = 0; r < 4; ++r) uf[r] = 4 * q + r < first ? uf[r] : 0.f;
     }
+    o *= iq;
 #pragma unroll
     for (int r = 0; r < 4; ++r) o = mfma_d(pr[r], uf[r], o);
 #pragma unroll
     for (int r = 1; r < 4; ++r)
 #pragma unroll
-      for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r], S[i]);
+      for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r] * ik[r], S[i]);
     if (odd) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = 4 * q + r < first ? o[r] : as_f32(0x7fc00000u);
