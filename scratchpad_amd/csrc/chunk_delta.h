@@ -1,4 +1,5 @@
-// Delta-rule recurrences with a decay per key channel (or per head), 16 tokens at a time, all of it fp32 on the matrix cores.
+// Delta-rule recurrences with a decay per key channel (or per head), 16 tokens at a time on the matrix cores: fp32 products, or those of
+// three bf16 parts of each operand (below: which, and why).
 //
 //   S = diag(w_t) S;   u_t = beta_t (v_t - S^T k_t);   S = S + k_t u_t^T;   o_t = S^T q_t        (k, q of the token, S [D, Dv])
 //
@@ -229,22 +230,53 @@ __device__ __forceinline__ f32x4_d mfma_d(float a, float b, const f32x4_d& c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+typedef __bf16 bf16x8_d __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ f32x4_d mfma_parts(const u32x4& a, const u32x4& b, const f32x4_d& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_d, a), __builtin_bit_cast(bf16x8_d, b), c, 0, 0, 0);
+}
+// two fp32 values as three pairs of bf16 whose sums they are: the upper 16 bits (which cannot overflow), then what is left, rounded, then
+// what is left of that (8 bits at the most: exact).  Not finite: the second part is NaN.
+struct Parts {
+  uint32_t p[3];
+};
+__device__ __forceinline__ Parts parts_of(float x, float y) {
+  const auto pair = [](float a, float b) {
+    bf16x2_t v;
+    v[0] = (__bf16)a, v[1] = (__bf16)b;
+    return __builtin_bit_cast(uint32_t, v);
+  };
+  const uint32_t xh = as_u32(x) & 0xffff0000u, yh = as_u32(y) & 0xffff0000u;
+  x -= as_f32(xh), y -= as_f32(yh);
+  const uint32_t mid = pair(x, y);
+  return Parts{{__builtin_amdgcn_perm(yh, xh, 0x07060302u), mid, pair(x - as_f32(mid << 16), y - as_f32(mid & 0xffff0000u))}};
+}
+
 // One workgroup per (request, head, range of the head's columns): a wave per 16 columns runs the products of chunk c while
 // kDcHelpers more waves form the operand rows of a chunk ahead and have those of the two chunks after it on their way into LDS; they
 // meet at one barrier per chunk.  (The same waves doing both in turn left the matrix cores idle for two thirds of a chunk: 4.4 us.)
-// What bounds a chunk is the issue of vector and matrix instructions together: a fp32 matrix instruction takes the vector unit's 32 cycles, so its
-// 104 (3380 cycles of 5800) and every address, decay and conversion of both kinds of waves add up.  Hence rows by pointers that move on by a
-// step, masks in a request's last chunk alone, and reads of LDS between the products.  One request of 4096 tokens, 16 heads of 128:
-// 2.43 -> 2.25 us a chunk with a decay per channel, 2.2 -> 1.96 with one per head (the layer 850 -> 802 and 798 -> 742).  Operands two chunks ahead,
-// and helpers ahead of the products in the issue, gave nothing: the sum stays.
+// With fp32 products (kParts false) a chunk is bound by the issue of vector and matrix instructions together: a fp32 matrix instruction keeps the
+// vector unit for its 32 cycles, so its 104 (3380 of 5800 cycles) and every address, decay and conversion of both kinds of waves add up.  Hence
+// rows by pointers that move on by a step, masks in a request's last chunk alone, and the norms of k and q with the products.  Operands two chunks
+// ahead, helpers ahead of the products in the issue, and stores behind the loads that are waited for gave nothing: the sum stays.
+// bf16 products run beside vector work, so heads of 128 by ranges of 64 columns (kParts) take the products with S, and Ke^T U, as six products of
+// parts with 8 bits each (the three left out are below 2^-23 of the whole, of either sign): 72 instructions of 16 cycles in the place of 96 of 32, for 280
+// more of the vector unit.  The chain is then the helpers', so each takes a quarter of the tokens (K, Q and Ke as a wave each: 4900 cycles).
+// us a chunk, one request of 4096 tokens, 16 heads of 128: decay per channel 2.43 -> 1.80, per head 2.2 -> 1.66 (the layers 854 -> 693 and 827 -> 687; of
+// 8 requests 331 -> 310 and 335 -> 312).  128 columns a workgroup, which many requests take, keep fp32: the parts do not fit 168
+// registers (16 requests of 125 tokens 212 and 243 us), nor two workgroups a unit of heads of 64.
+// S and the read-outs are as far from 64 bits as with fp32 products.
 constexpr int kDcHelpers = 4;
 
 // COLS: columns of a workgroup at the most
 template <typename Tag, int D, bool CHANNEL, int COLS>
 struct DeltaScanLds {
+  // heads of 128 by ranges of 64 columns: operands in three bf16 parts
+  static constexpr bool kParts = D == 128 && COLS <= 64;
   static constexpr int kRow = D + 4;                                                     // floats per operand row
   static constexpr int kRaw = kDC * D * (2 * Elem<Tag>::kBytes + (CHANNEL ? 4 : 0));     // a chunk's k, q (and decay) rows
-  static constexpr int kOps = (3 * kDC * kRow + D) * 4;                                  // Kd, Qd, Ke, G_end
+  // kParts: Kd and Qd three parts of 16 rows each, channels in the order that a lane takes them; Ke of a channel three parts of 16 tokens; G_end
+  static constexpr int kPartRow = 2 * D + 16, kPart = kDC * kPartRow, kKe = 6 * kPart, kKeRow = 6 * kDC + 8, kG = kKe + D * kKeRow;
+  static constexpr int kOps = kParts ? kG + 4 * D : (3 * kDC * kRow + D) * 4;            // Kd, Qd, Ke, G_end
   static constexpr int kOp = 3 * kRaw, kWork = kOp + 2 * kOps, kBytes = kWork + 4 * kDcFloats * 4;
   static constexpr int kWaves = (COLS / 16 + kDcHelpers) / 4 * (COLS <= 64 && kBytes <= 80 * 1024 ? 2 : 1);      // per SIMD
   static_assert(kBytes <= 160 * 1024, "LDS");
@@ -362,10 +394,86 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
         }
       }
     };
+    // kParts: a helper takes four tokens of every chunk, a thread two channels - the decays in front of them for Kd and Qd (and G_end), those
+    // behind them for Ke
+    struct __attribute__((aligned(2 * E::kBytes))) Two {
+      typename E::storage x[2];
+    };
+    typedef float f32x2_d __attribute__((ext_vector_type(2)));
+    const auto parts = [&](int c, auto whole) {
+      const int n = len - c * kDC, d = 2 * lane, t0 = 4 * hw;
+      const char* raw = delta_lds + c % 3 * L::kRaw;
+      const float* wr = (const float*)(raw + 2 * kDC * kRowBytes);
+      const float* m = (const float*)(delta_lds + L::kWork + (c & 3) * kDcFloats * 4);
+      char* ops = delta_lds + L::kOp + (c & 1) * L::kOps;
+      f32x2_d w[kDC];
+      Two kr[4], qr[4];
+#pragma unroll
+      for (int t = 0; t < kDC; ++t) w[t] = CHANNEL ? *(const f32x2_d*)&wr[t * D + d] : f32x2_d{m[kDcW + t], m[kDcW + t]};
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        kr[x] = *(const Two*)(raw + (t0 + x) * kRowBytes + d * E::kBytes);
+        qr[x] = *(const Two*)(raw + (kDC + t0 + x) * kRowBytes + d * E::kBytes);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!decltype(whole)::value) {
+#pragma unroll
+        for (int t = 0; t < kDC; ++t)
+          if (t >= n) w[t] = f32x2_d{1.f, 1.f};
+      }
+      float y[3][4][2];                                // k, q, and k backward
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+          const bool on = whole || t0 + x < n;
+          y[0][x][ch] = y[2][x][ch] = on ? E::load(kr[x].x, ch) : 0.f;
+          y[1][x][ch] = on ? E::load(qr[x].x, ch) : 0.f;
+        }
+#pragma unroll
+      for (int part = 0; part < kDcHelpers; ++part) {  // (hw is the wave's: one of four)
+        if (hw != part) continue;
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+          float g = 1.f, back = 1.f;
+#pragma unroll
+          for (int t = 0; t < 4 * part + 4; ++t) {
+            g *= w[t][ch];
+            if (t >= 4 * part) y[0][t - 4 * part][ch] *= g, y[1][t - 4 * part][ch] *= g;
+          }
+#pragma unroll
+          for (int t = kDC - 1; t >= 4 * part; --t) {
+            if (t < 4 * part + 4) y[2][t - 4 * part][ch] *= back;
+            back *= w[t][ch];
+          }
+          if (part == kDcHelpers - 1) *(float*)(ops + L::kG + (d + ch) * 4) = g;
+        }
+      }
+      // channels 4 q + r and 16 + 4 q + r of every 32 are a lane's eight
+      char* rows = ops + t0 * L::kPartRow + (d / 32 * 32 + d % 16 / 4 * 8 + d % 32 / 16 * 4 + d % 4) * 2;
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int which = 0; which < 2; ++which) {
+          const Parts z = parts_of(y[which][x][0], y[which][x][1]);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) *(uint32_t*)(rows + (3 * which + i) * L::kPart + x * L::kPartRow) = z.p[i];
+        }
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch) {
+        const Parts lo = parts_of(y[2][0][ch], y[2][1][ch]), hi = parts_of(y[2][2][ch], y[2][3][ch]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *(u32x2*)(ops + L::kKe + (d + ch) * L::kKeRow + i * 2 * kDC + t0 * 2) = u32x2{lo.p[i], hi.p[i]};
+      }
+    };
     const auto form = [&](int c) {
       if (c >= chunks) return;
-      if (len - c * kDC >= kDC) operands(c, std::true_type());
-      else operands(c, std::false_type());
+      const auto with = [&](auto whole) {
+        if constexpr (L::kParts) parts(c, whole);
+        else operands(c, whole);
+      };
+      if (len - c * kDC >= kDC) with(std::true_type());
+      else with(std::false_type());
     };
     // loads of one fetch that every helper issues at the least: waiting for all but so many is waiting for the fetch before it
     constexpr int kLoads = 2 * (LK / kDcHelpers) + LW / kDcHelpers + LM / kDcHelpers;
@@ -426,62 +534,141 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
     const int n = len - c * kDC;
     const float* m = (const float*)(delta_lds + L::kWork + (c & 3) * kDcFloats * 4);
     const float* ops = (const float*)(delta_lds + L::kOp + (c & 1) * L::kOps);
-    // Every read of LDS goes out between two products: in one piece the four waves' reads hold their products up until LDS has taken them
-    // (left to itself the compiler keeps registers free and waits for each read).
-    f32x4_d kd = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f}, ak[DT], aq[DT], g[DT], tr, pr, ik, iq;
-    float ke[4][DT];
-    const auto read_k = [&](int i) { ak[i] = *(const f32x4_d*)&ops[r16 * ROW + 16 * i + 4 * q]; };
-    read_k(0);
-    read_k(1);
+    f32x4_d kd = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f}, tr, pr, ik, iq;
+    float ke[L::kParts ? 1 : 4][DT];
+    const auto values = [&] {
 #pragma unroll
-    for (int i = 0; i < DT; ++i) {
-      if (i + 2 < DT) read_k(i + 2);
-      aq[i] = *(const f32x4_d*)&ops[(kDC + r16) * ROW + 16 * i + 4 * q];
-      if (i == DT - 2) ik = *(const f32x4_d*)&m[kDcIk + 4 * q];
-      if (i == DT - 1) tr = *(const f32x4_d*)&m[kDcT + r16 * kDC + 4 * q];
+      for (int r = 0; r < 4; ++r) v[r] = E::load(&vn[r], 0);
+      if (n < kDC) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = 4 * q + r < n ? v[r] : 0.f;
+      }
+      if (c + 1 < chunks) fetch_v(c + 1);
+    };
+    if constexpr (L::kParts) {
+      // Products of parts, the small ones first (those of two last parts, or a middle and a last one, are below fp32's rounding).  The parts of
+      // a block's state are formed between the products of the block before, whose operands are read a block ahead.
+      constexpr int BLOCKS = D / 32;
+      f32x4_d g[DT];
+      const char* rows = (const char*)ops;
+      u32x4 ak[2][3], aq[2][3], sp[2][3];
+      u32x2 kp[DT][3];
+      const auto read = [&](int x) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          ak[x & 1][p] = ld16(rows + p * L::kPart + r16 * L::kPartRow + 64 * x + 16 * q);
+          aq[x & 1][p] = ld16(rows + (3 + p) * L::kPart + r16 * L::kPartRow + 64 * x + 16 * q);
+        }
+#pragma unroll
+        for (int i = 2 * x; i < 2 * x + 2; ++i) g[i] = *(const f32x4_d*)(rows + L::kG + (16 * i + 4 * q) * 4);
+      };
+      const auto split = [&](int x) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const Parts y = parts_of(S[2 * x + e / 2][2 * (e & 1)], S[2 * x + e / 2][2 * (e & 1) + 1]);
+#pragma unroll
+          for (int p = 0; p < 3; ++p) sp[x & 1][p][e] = y.p[p];
+        }
+      };
+      constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+      read(0);
+      split(0);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) kd = mfma_d(ak[i][r], S[i][r], kd);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+      for (int x = 0; x < BLOCKS; ++x) {
+        if (x + 1 < BLOCKS) read(x + 1);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = E::load(&vn[r], 0);
-    if (n < kDC) {
+        for (int i = 2 * x; i < 2 * x + 2; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = 4 * q + r < n ? v[r] : 0.f;
-    }
-    if (c + 1 < chunks) fetch_v(c + 1);
+          for (int p = 0; p < 3; ++p) kp[i][p] = *(const u32x2*)(rows + L::kKe + (16 * i + r16) * L::kKeRow + p * 2 * kDC + 8 * q);
 #pragma unroll
-    for (int i = 0; i < DT; ++i) {
-      g[i] = *(const f32x4_d*)&ops[3 * kDC * ROW + 16 * i + 4 * q];
-      if (i == 0) pr = *(const f32x4_d*)&m[kDcP + r16 * kDC + 4 * q];
-      if (i == 1) iq = *(const f32x4_d*)&m[kDcIq + 4 * q];
+        for (int y = 0; y < 6; ++y) {
+          kd = mfma_parts(ak[x & 1][PA[y]], sp[x & 1][PB[y]], kd);
+          o = mfma_parts(aq[x & 1][PA[y]], sp[x & 1][PB[y]], o);
+        }
+        if (x + 1 < BLOCKS) split(x + 1);
+#pragma unroll
+        for (int i = 2 * x; i < 2 * x + 2; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[i][r] *= g[i][r];
+#pragma unroll
+        for (int y = 0; y < 12; ++y) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // a read of LDS, a product, four vector instructions
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      tr = *(const f32x4_d*)&m[kDcT + r16 * kDC + 4 * q], pr = *(const f32x4_d*)&m[kDcP + r16 * kDC + 4 * q];
+      ik = *(const f32x4_d*)&m[kDcIk + 4 * q], iq = *(const f32x4_d*)&m[kDcIq + 4 * q];
+      values();
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        __builtin_amdgcn_sched_barrier(0);
-        ke[r][i] = ops[(2 * kDC + 4 * q + r) * ROW + 16 * i + r16];
-        __builtin_amdgcn_sched_barrier(0);
-        o = mfma_d(aq[i][r], S[i][r], o);
+        v[r] = fmaf(-kd[r], ik[r], v[r]);
+        u = mfma_d(tr[r], v[r], u);
       }
-      if (i == 1) {
+      const Parts u0 = parts_of(u[0] * ik[0], u[1] * ik[1]), u1 = parts_of(u[2] * ik[2], u[3] * ik[3]);
+      const u32x4 ub[3] = {u32x4{u0.p[2], u1.p[2], u0.p[0], u1.p[0]}, u32x4{u0.p[1], u1.p[1], u0.p[1], u1.p[1]},
+                           u32x4{u0.p[0], u1.p[0], u0.p[0], u1.p[0]}};
+      // Ke's first part beside the last against U's last and first, then its first beside the second against U's second twice and first twice
+#pragma unroll
+      for (int y = 0; y < 3; ++y)
+#pragma unroll
+        for (int i = 0; i < DT; ++i) {
+          const int p = y == 0 ? 2 : 1;
+          S[i] = mfma_parts(u32x4{kp[i][0][0], kp[i][0][1], kp[i][p][0], kp[i][p][1]}, ub[y], S[i]);
+        }
+    } else {
+      // Every read of LDS goes out between two products: in one piece the four waves' reads hold their products up until LDS has taken them
+      // (left to itself the compiler keeps registers free and waits for each read).
+      f32x4_d ak[DT], aq[DT], g[DT];
+      const auto read_k = [&](int i) { ak[i] = *(const f32x4_d*)&ops[r16 * ROW + 16 * i + 4 * q]; };
+      read_k(0);
+      read_k(1);
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        if (i + 2 < DT) read_k(i + 2);
+        aq[i] = *(const f32x4_d*)&ops[(kDC + r16) * ROW + 16 * i + 4 * q];
+        if (i == DT - 2) ik = *(const f32x4_d*)&m[kDcIk + 4 * q];
+        if (i == DT - 1) tr = *(const f32x4_d*)&m[kDcT + r16 * kDC + 4 * q];
         __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) kd = mfma_d(ak[i][r], S[i][r], kd);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      values();
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        g[i] = *(const f32x4_d*)&ops[3 * kDC * ROW + 16 * i + 4 * q];
+        if (i == 0) pr = *(const f32x4_d*)&m[kDcP + r16 * kDC + 4 * q];
+        if (i == 1) iq = *(const f32x4_d*)&m[kDcIq + 4 * q];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          v[r] = fmaf(-kd[r], ik[r], v[r]);
-          u = mfma_d(tr[r], v[r], u);
+          __builtin_amdgcn_sched_barrier(0);
+          ke[r][i] = ops[(2 * kDC + 4 * q + r) * ROW + 16 * i + r16];
+          __builtin_amdgcn_sched_barrier(0);
+          o = mfma_d(aq[i][r], S[i][r], o);
+        }
+        if (i == 1) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            v[r] = fmaf(-kd[r], ik[r], v[r]);
+            u = mfma_d(tr[r], v[r], u);
+          }
+        }
+        if (i > 0) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[i - 1][r] *= g[i - 1][r];
         }
       }
-      if (i > 0) {
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) S[i - 1][r] *= g[i - 1][r];
-      }
+      for (int r = 0; r < 4; ++r) S[DT - 1][r] *= g[DT - 1][r];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[0][i], u[0] * ik[0], S[i]);
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) S[DT - 1][r] *= g[DT - 1][r];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[0][i], u[0] * ik[0], S[i]);
     int first = kDC;                                  // the column's first token whose u is not finite
     f32x4_d uf = u;
     const float probe = fmaf(u[0], 0.f, fmaf(u[1], 0.f, fmaf(u[2], 0.f, u[3] * 0.f)));
@@ -508,10 +695,12 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
     o *= iq;
 #pragma unroll
     for (int r = 0; r < 4; ++r) o = mfma_d(pr[r], uf[r], o);
+    if constexpr (!L::kParts) {
 #pragma unroll
-    for (int r = 1; r < 4; ++r)
+      for (int r = 1; r < 4; ++r)
 #pragma unroll
-      for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r] * ik[r], S[i]);
+        for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r] * ik[r], S[i]);
+    }
     if (odd) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = 4 * q + r < first ? o[r] : as_f32(0x7fc00000u);

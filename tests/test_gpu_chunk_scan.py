@@ -241,6 +241,44 @@ def test_head_delta_chunks_where_the_other_form_pays(lens, H, G, D, Dv, dtype, m
     test_head_delta_chunks_against_the_per_token_kernel(lens, H, G, D, Dv, dtype)
 
 
+MANY = [17, 5, 33, 16] * 24      # 288 workgroups of 3 heads: the widest range of columns per workgroup
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D", [64, 128])
+def test_delta_chunks_of_many_requests(D, dtype, monkeypatch):
+    from scratchpad_amd import _native
+    monkeypatch.setattr(_native, "delta_chunks_pay", lambda *a: True)
+    test_gated_delta_chunks(MANY, 3, 1, D, 128, dtype)
+    test_head_delta_chunks_against_the_per_token_kernel([n + 16 for n in MANY], 3, 1, D, 128, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,Dv", [(128, 128), (64, 48)])
+def test_gated_delta_chunks_of_rows_of_any_length(D, Dv, dtype, monkeypatch):
+    """q and k are of unit length whatever they come as: the chunks' products of rows of 1e-6 to 1e6 against the per-token kernel's, both
+    orders of the same fp32 sums (bars as above)"""
+    from scratchpad_amd import _native
+    announce("gated delta rows of any length", dtype, D, Dv)
+    g = torch.Generator(device=DEV).manual_seed(9)
+    lens, H = [50, 17, 32], 2
+    T, slots = sum(lens), slots_of(lens)
+    size = lambda: 10.0 ** (12 * torch.rand(T, 1, generator=g, device=DEV) - 6)  # noqa: E731
+    q, k = ((torch.randn(T, H * D, generator=g, device=DEV) * size()).to(dtype) for _ in range(2))
+    v, bp = (torch.randn(T, n, generator=g, device=DEV).to(dtype) for n in (H * Dv, H))
+    decay, gate = (torch.rand(T, n, generator=g, device=DEV) for n in (H * D, H * Dv))
+    nw, states, outs = torch.rand(Dv, generator=g, device=DEV) + 0.5, [], []
+    for chunks in (True, False):
+        monkeypatch.setattr(_native, "delta_chunks_pay", lambda *a, chunks=chunks: chunks)
+        states.append(torch.zeros(2 * len(lens) + 1, H, D, Dv, device=DEV))
+        outs.append(_native.gated_delta_scan(q, k, v, bp, decay, gate, nw, states[-1], seq_extend(lens, [0] * len(lens), slots), H, H, D, Dv, 1e-5))
+    for slot in slots:
+        near(states[0][slot], states[1][slot].double(), 2e-5)
+    bar = {torch.bfloat16: 2.0 ** -7, torch.float32: 1e-4}[dtype]
+    # (1e-3: as in test_gated_delta_chunks)
+    assert ((outs[0].double() - outs[1].double()).abs() <= bar * outs[1].double().abs() + 1e-3).all()
+
+
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.bfloat16, 32), (torch.float32, 64)])
 @pytest.mark.parametrize("lens", [[1, 1, 1], [70, 3]], ids=lambda l: "-".join(map(str, l)))
 def test_mlstm_gates_as_halves_of_one_product(dtype, D, lens):
