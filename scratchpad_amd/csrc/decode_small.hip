@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kSmallWaves * 64, 2) void decode_small_kernel(Small
     for (int t = 0; t < T; ++t)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        x[t][j] = __builtin_amdgcn_exp2f(x[t][j] - top);
+        x[t][j] = Elem<CT>::round(__builtin_amdgcn_exp2f(x[t][j] - top));      // (as the products take it: the weights sum to one)
         sum += x[t][j];
       }
     l = __builtin_fmaf(l, keep, sum_quarters(sum));
