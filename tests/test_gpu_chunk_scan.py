@@ -530,6 +530,44 @@ def test_delta_values_that_are_not_finite_reach_no_earlier_token(channel, at, wh
         assert torch.equal(S1[1, 1][:, ~hit], S0[1, 1][:, ~hit]) and not torch.isfinite(S1[1, 1][:, hit]).any()
 
 
+@pytest.mark.parametrize("where,bad", [(w, b) for w in "qkv" for b in BAD] + [("beta", BAD[0]), ("decay", BAD[0])])
+@pytest.mark.parametrize("at", [0, 9, 15, 40])
+@pytest.mark.parametrize("channel", [True, False], ids=["gated", "head"])
+def test_delta_products_of_parts_and_values_that_are_not_finite(channel, at, where, bad, monkeypatch):
+    """heads of 128: what is not finite reaches its own token's rows and the ones behind it, of its own head"""
+    from scratchpad_amd import _native
+    monkeypatch.setattr(_native, "delta_chunks_pay", lambda *a: True)
+    announce("delta parts not finite", channel, where, bad, at)
+    g = torch.Generator(device=DEV).manual_seed(19)
+    lens, H, D, Dv = [61, 30], 2, 128, 128
+    T = sum(lens)
+    rn = lambda n: torch.randn(T, n, generator=g, device=DEV)  # noqa: E731
+    x = {"q": rn(H * D).bfloat16(), "k": rn(H * D).bfloat16(), "v": rn(H * Dv).bfloat16(), "beta": rn(H).bfloat16(),
+         "decay": torch.rand(T, H * D, generator=g, device=DEV), "pre": rn(2 * H)}
+    gate, nw, dt_bias, A_log = rn(H * Dv).bfloat16(), *(torch.rand(n, generator=g, device=DEV) for n in (Dv, H, H))
+    seq, got = seq_extend(lens, [0, 0], [1, 3]), []
+    for dirty in (False, True):
+        if dirty and not channel and where in ("beta", "decay"):
+            x["pre"][at, 1 + (H if where == "decay" else 0)] = bad
+        elif dirty:
+            x[where][at, 1 if where == "beta" else D + 7] = bad
+        S = torch.zeros(5, H, D, Dv, device=DEV)
+        assert _native._delta_chunks_take(x["q"], x["k"], x["v"], x["decay"] if channel else None, seq, D, Dv)
+        if channel:
+            y = _native.gated_delta_scan(x["q"], x["k"], x["v"], x["beta"], x["decay"], gate.float().abs(), nw, S, seq, H, H, D, Dv, 1e-5)
+        else:
+            y = _native.head_delta_scan(x["q"], x["k"], x["v"], gate, x["pre"], dt_bias, A_log, nw, S, seq, H, H, D, Dv, 1e-5)
+        got.append((y.view(T, H, Dv), S))
+    (y0, S0), (y1, S1) = got
+    hit = torch.zeros(T, H, Dv, dtype=torch.bool, device=DEV)
+    hit[at:at + 1 if where == "q" else 61, 1] = True
+    assert torch.equal(y1[~hit], y0[~hit]) and not torch.isfinite(y1[hit]).any()
+    assert torch.equal(S1[:, 0], S0[:, 0]) and torch.equal(S1[3], S0[3])
+    if where == "v":
+        hit = torch.arange(Dv, device=DEV) == 7
+        assert torch.equal(S1[1, 1][:, ~hit], S0[1, 1][:, ~hit]) and not torch.isfinite(S1[1, 1][:, hit]).any()
+
+
 @pytest.mark.parametrize("T", [40, 64, 129])
 def test_lowrank_decays_of_all_rates(T):
     """exp(-rate softplus(z)) at the accuracy of fp32 functions - the product's, an ulp or two of softplus, rate and exponential -
