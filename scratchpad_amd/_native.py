@@ -1807,15 +1807,19 @@ def small_linear_tiles_pay(T: int, K: int, n: int) -> bool:
     return (K <= 2048 or 8 * T >= K) and (n <= 128 or (n <= 256 and T * K <= 1 << 23) or (K <= 2048 and T * n <= 1 << 18))
 
 
+def _small_linear_tiles_take(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    # (2^25 elements: 64 rows of a tile within the 32 bits that its loads count in; sp_small_linear_f32 takes rows further apart one at a time)
+    return (x.dtype == torch.bfloat16 and x.shape[1] % 32 == 0 and x.stride(0) % 8 == 0 and x.stride(0) <= 1 << 25
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and small_linear_tiles_pay(x.shape[0], x.shape[1], weight.shape[0]))
+
+
 def small_linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """fp32 [T, n] = x @ weight.T + bias with fp32 weights, accumulation and output (gates and step sizes of recurrences)"""
     _mat(x, "x"), _f32(weight, "weight")
     if weight.dim() != 2 or weight.shape[1] != x.shape[1] or (bias is not None and _f32(bias, "bias").shape[0] != weight.shape[0]):
         raise RuntimeError("small_linear_f32: weight [n, k], bias [n]")
-    if x.shape[0] > SMALL_LINEAR_OWN_ROWS and not (x.dtype == torch.bfloat16 and x.shape[1] % 32 == 0 and x.stride(0) % 8 == 0
-                                                   and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
-                                                   and small_linear_tiles_pay(x.shape[0], x.shape[1], weight.shape[0])):
-        # many rows where sp_small_linear_f32's tiles do not pay, or of types or lengths without them: the kernel for few rows reads
+    if x.shape[0] > SMALL_LINEAR_OWN_ROWS and not _small_linear_tiles_take(x, weight):
+        # many rows where sp_small_linear_f32's tiles do not pay, or of types, lengths or distances without them: the kernel for few rows reads
         # the weight rows again for every token, the library's fp32 product tiles them
         return torch.nn.functional.linear(x.to(torch.float32), weight, bias)
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=x.device)

@@ -680,12 +680,17 @@ extern "C" int sp_small_linear_f32(float* out, const void* x, int64_t x_stride, 
   SP_CHECK_ARG(num_tokens >= 0 && k > 0 && n > 0);
   if (num_tokens == 0) return SP_OK;
   SP_CHECK_ARG(out && x && weight && x_stride >= k);
-  if (num_tokens > 64 && dtype == SP_BF16 && k % 32 == 0 && x_stride % 8 == 0 && (((uintptr_t)x | (uintptr_t)weight) & 15) == 0) {
+  // the tiles' loads name a row by its distance from the tile's first in 32 bits, of x and of the weights
+  const auto near = [&](int64_t rows) {
+    const int64_t most = (int64_t)1 << 32;
+    return k <= most / (4 * kLinOut) && x_stride <= most / (2 * rows);
+  };
+  if (num_tokens > 64 && dtype == SP_BF16 && k % 32 == 0 && x_stride % 8 == 0 && (((uintptr_t)x | (uintptr_t)weight) & 15) == 0 && near(32)) {
     // (up to 64 rows a workgroup per row has the shorter chain.)  Workgroups of 32 tokens, two of which fit a CU; of 64, one a CU, which
     // read the weights half as often, where their rounds are at least half full and not more than two (us, 32 / 64: 4096 rows of 32
     // outputs 6.7 / 8.4, of 64 10.3 / 9.1, of 128 15.9 / 14.9; 9000 of 32 16.9 / 18.8; 16384 of 64 43.3 / 48.4).  The order of the sums is the same.
     const int64_t nb = (n + kLinOut - 1) / kLinOut, wide = (num_tokens + 63) / 64 * nb;
-    if ((num_tokens + 31) / 32 * nb > 256 && wide <= 512 && (wide + 255) % 256 >= 127)
+    if (near(64) && (num_tokens + 31) / 32 * nb > 256 && wide <= 512 && (wide + 255) % 256 >= 127)
       return launch_linear_f32<4, 8>(out, (const char*)x, x_stride, weight, bias, num_tokens, k, n, (hipStream_t)stream);
     return launch_linear_f32<2, 8>(out, (const char*)x, x_stride, weight, bias, num_tokens, k, n, (hipStream_t)stream);
   }

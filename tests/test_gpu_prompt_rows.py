@@ -199,6 +199,25 @@ def test_fp32_products_of_more_rows(T, K, n):
     assert torch.equal(out[T - 70:], few)
 
 
+# tiles of 64 rows: the widest stride that they take, the first past 32 bits; the same of 32
+@pytest.mark.parametrize("stride,n", [(1 << 25, 1376), (34087048, 1376), (1 << 26, 16), (69273672, 16)])
+def test_fp32_products_of_far_apart_rows(stride, n):
+    """the entry and its wrapper take rows any distance apart"""
+    from scratchpad_amd import _native
+    T, K = 65, 64
+    announce("fp32 products of far rows", stride, n)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.empty(stride * (T - 1) + K, dtype=torch.bfloat16, device=DEV).as_strided((T, K), (stride, 1))
+    x.copy_(torch.randn(T, K, generator=g, device=DEV))
+    w = torch.randn(n, K, generator=g, device=DEV)
+    want, bound = x.double() @ w.double().T, (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    out = torch.empty(T, n, device=DEV)
+    _native._check(_native.load().sp_small_linear_f32(out.data_ptr(), x.data_ptr(), stride, w.data_ptr(), None, T, K, n, _native._dt(x),
+                                                      _native._stream()), "sp_small_linear_f32")
+    for got in (out, _native.small_linear_f32(x, w)):
+        assert bool(((got.double() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("T", [64, 65, 100])
 def test_fp32_products_of_infinite_inputs(T):
     """an infinity is one in the sum it enters, in every form: not NaN"""

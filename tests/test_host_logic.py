@@ -262,6 +262,16 @@ def test_fp32_product_dispatch_rule():
     assert not pays(256, 2048, 2048) and not pays(65, 4096, 2048)
 
 
+def test_fp32_products_of_far_apart_rows_leave_the_tiles():
+    """a tile's loads count in 32 bits from its first row: 64 rows of the widest stride that takes tiles lie within them"""
+    from scratchpad_amd import _native
+    w = torch.empty(64, 2048, device="meta")
+    rows = lambda stride: torch.empty_strided((65, 2048), (stride, 1), dtype=torch.bfloat16, device="meta")  # noqa: E731
+    widest = max(s for s in (2048, 1 << 20, 1 << 25, (1 << 25) + 8, 34087048, 69273672) if _native._small_linear_tiles_take(rows(s), w))
+    assert widest >= 1 << 20 and 63 * widest * 2 + 128 <= 1 << 32
+    assert not _native._small_linear_tiles_take(rows(34087048), w) and not _native._small_linear_tiles_take(rows(69273672), w)
+
+
 def test_scan_segments_keep_to_one_round_and_to_long_requests():
     """a step is cut only where its longest request is likely to be several segments, into multiples of 64 tokens whose workgroups the
     chip holds at a time"""
