@@ -256,13 +256,13 @@ __device__ __forceinline__ Parts parts_of(float x, float y) {
 // meet at one barrier per chunk.  (The same waves doing both in turn left the matrix cores idle for two thirds of a chunk: 4.4 us.)
 // With fp32 products (kParts false) a chunk is bound by the issue of vector and matrix instructions together: a fp32 matrix instruction keeps the
 // vector unit for its 32 cycles, so its 104 (3380 of 5800 cycles) and every address, decay and conversion of both kinds of waves add up.  Hence
-// rows by pointers that move on by a step, masks in a request's last chunk alone, and the norms of k and q with the products.  Operands two chunks
+// rows by pointers that move on by a step, and masks in a request's last chunk alone.  Operands two chunks
 // ahead, helpers ahead of the products in the issue, and stores behind the loads that are waited for gave nothing: the sum stays.
 // bf16 products run beside vector work, so heads of 128 by ranges of 64 columns (kParts) take the products with S, and Ke^T U, as six products of
 // parts with 8 bits each (the three left out are below 2^-23 of the whole, of either sign): 72 instructions of 16 cycles in the place of 96 of 32, for 280
 // more of the vector unit.  The chain is then the helpers', so each takes a quarter of the tokens (K, Q and Ke as a wave each: 4900 cycles).
-// us a chunk, one request of 4096 tokens, 16 heads of 128: decay per channel 2.43 -> 1.80, per head 2.2 -> 1.66 (the layers 854 -> 693 and 827 -> 687; of
-// 8 requests 331 -> 310 and 335 -> 312).  128 columns a workgroup, which many requests take, keep fp32: the parts do not fit 168
+// us a chunk, one request of 4096 tokens, 16 heads of 128: decay per channel 2.43 -> 1.86, per head 2.2 -> 1.66 (the layers 855 -> 708 and 823 -> 685; of
+// 8 requests 334 -> 309 and 333 -> 307).  128 columns a workgroup, which many requests take, keep fp32: the parts do not fit 168
 // registers (16 requests of 125 tokens 212 and 243 us), nor two workgroups a unit of heads of 64.
 // S and the read-outs are as far from 64 bits as with fp32 products.
 constexpr int kDcHelpers = 4;
@@ -349,8 +349,9 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
       mp += mstep;
     };
     point(0, kDC);
-    // operand rows of a chunk: a thread walks a channel forward (Kd, Qd, G_end) or backward (Ke); rows behind the end are zeros.  The
-    // norms of k and q are the products': 12 multiplications of a wave that owns columns for 48 of a channel's two threads here.
+    // operand rows of a chunk: a thread walks a channel forward (Kd, Qd, G_end) or backward (Ke); rows behind the end are zeros.  Rows
+    // become unit rows here and not in the products, where their lengths would be fewer multiplications (12 of a wave for 48 of a
+    // channel's two threads): a product with a row that is not of unit length can be past fp32 where the state is not, and zeros have a factor of 1000.
     const auto operands = [&](int c, auto whole) {
       const int n = len - c * kDC;
       const char* raw = delta_lds + c % 3 * L::kRaw;
@@ -362,11 +363,17 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
         const bool fwd = role < D;                     // (D is a multiple of 64: whole waves)
         typename E::storage kr[kDC], qr[kDC];
         float w[kDC];
+        f32x4_d ik[kDC / 4], iq[kDC / 4];
 #pragma unroll
         for (int t = 0; t < kDC; ++t) {                // every read on its way before the first is used
           w[t] = CHANNEL ? wr[t * D + d] : m[kDcW + t];
           kr[t] = ((const typename E::storage*)raw)[t * D + d];
           qr[t] = ((const typename E::storage*)(raw + (fwd ? kDC * kRowBytes : 0)))[t * D + d];
+        }
+#pragma unroll
+        for (int x = 0; x < kDC / 4; ++x) {
+          ik[x] = *(const f32x4_d*)&m[kDcIk + 4 * x];
+          iq[x] = *(const f32x4_d*)&m[kDcIq + 4 * x];
         }
         __builtin_amdgcn_sched_barrier(0);
         float k[kDC];
@@ -374,7 +381,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
         for (int t = 0; t < kDC; ++t) {
           const bool on = whole || t < n;
           if (!on) w[t] = 1.f;
-          k[t] = on ? E::load(&kr[t], 0) : 0.f;
+          k[t] = on ? E::load(&kr[t], 0) * ik[t / 4][t % 4] : 0.f;
         }
         float g = 1.f;
         if (fwd) {
@@ -382,7 +389,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
           for (int t = 0; t < kDC; ++t) {
             g *= w[t];
             ops[t * ROW + d] = k[t] * g;
-            ops[(kDC + t) * ROW + d] = whole || t < n ? E::load(&qr[t], 0) * g : 0.f;
+            ops[(kDC + t) * ROW + d] = whole || t < n ? E::load(&qr[t], 0) * iq[t / 4][t % 4] * g : 0.f;
           }
           ops[3 * kDC * ROW + d] = g;
         } else {
@@ -415,6 +422,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
         kr[x] = *(const Two*)(raw + (t0 + x) * kRowBytes + d * E::kBytes);
         qr[x] = *(const Two*)(raw + (kDC + t0 + x) * kRowBytes + d * E::kBytes);
       }
+      const f32x4_d ik = *(const f32x4_d*)&m[kDcIk + t0], iq = *(const f32x4_d*)&m[kDcIq + t0];
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (!decltype(whole)::value) {
 #pragma unroll
@@ -427,8 +435,8 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
 #pragma unroll
         for (int ch = 0; ch < 2; ++ch) {
           const bool on = whole || t0 + x < n;
-          y[0][x][ch] = y[2][x][ch] = on ? E::load(kr[x].x, ch) : 0.f;
-          y[1][x][ch] = on ? E::load(qr[x].x, ch) : 0.f;
+          y[0][x][ch] = y[2][x][ch] = on ? E::load(kr[x].x, ch) * ik[x] : 0.f;
+          y[1][x][ch] = on ? E::load(qr[x].x, ch) * iq[x] : 0.f;
         }
 #pragma unroll
       for (int part = 0; part < kDcHelpers; ++part) {  // (hw is the wave's: one of four)
@@ -534,7 +542,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
     const int n = len - c * kDC;
     const float* m = (const float*)(delta_lds + L::kWork + (c & 3) * kDcFloats * 4);
     const float* ops = (const float*)(delta_lds + L::kOp + (c & 1) * L::kOps);
-    f32x4_d kd = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f}, tr, pr, ik, iq;
+    f32x4_d kd = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f}, tr, pr;
     float ke[L::kParts ? 1 : 4][DT];
     const auto values = [&] {
 #pragma unroll
@@ -600,14 +608,13 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
         __builtin_amdgcn_sched_barrier(0);
       }
       tr = *(const f32x4_d*)&m[kDcT + r16 * kDC + 4 * q], pr = *(const f32x4_d*)&m[kDcP + r16 * kDC + 4 * q];
-      ik = *(const f32x4_d*)&m[kDcIk + 4 * q], iq = *(const f32x4_d*)&m[kDcIq + 4 * q];
       values();
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        v[r] = fmaf(-kd[r], ik[r], v[r]);
+        v[r] -= kd[r];
         u = mfma_d(tr[r], v[r], u);
       }
-      const Parts u0 = parts_of(u[0] * ik[0], u[1] * ik[1]), u1 = parts_of(u[2] * ik[2], u[3] * ik[3]);
+      const Parts u0 = parts_of(u[0], u[1]), u1 = parts_of(u[2], u[3]);
       const u32x4 ub[3] = {u32x4{u0.p[2], u1.p[2], u0.p[0], u1.p[0]}, u32x4{u0.p[1], u1.p[1], u0.p[1], u1.p[1]},
                            u32x4{u0.p[0], u1.p[0], u0.p[0], u1.p[0]}};
       // Ke's first part beside the last against U's last and first, then its first beside the second against U's second twice and first twice
@@ -629,7 +636,6 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
       for (int i = 0; i < DT; ++i) {
         if (i + 2 < DT) read_k(i + 2);
         aq[i] = *(const f32x4_d*)&ops[(kDC + r16) * ROW + 16 * i + 4 * q];
-        if (i == DT - 2) ik = *(const f32x4_d*)&m[kDcIk + 4 * q];
         if (i == DT - 1) tr = *(const f32x4_d*)&m[kDcT + r16 * kDC + 4 * q];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -641,7 +647,6 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
       for (int i = 0; i < DT; ++i) {
         g[i] = *(const f32x4_d*)&ops[3 * kDC * ROW + 16 * i + 4 * q];
         if (i == 0) pr = *(const f32x4_d*)&m[kDcP + r16 * kDC + 4 * q];
-        if (i == 1) iq = *(const f32x4_d*)&m[kDcIq + 4 * q];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           __builtin_amdgcn_sched_barrier(0);
@@ -653,7 +658,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            v[r] = fmaf(-kd[r], ik[r], v[r]);
+            v[r] -= kd[r];
             u = mfma_d(tr[r], v[r], u);
           }
         }
@@ -667,7 +672,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
       for (int r = 0; r < 4; ++r) S[DT - 1][r] *= g[DT - 1][r];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[0][i], u[0] * ik[0], S[i]);
+      for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[0][i], u[0], S[i]);
     }
     int first = kDC;                                  // the column's first token whose u is not finite
     f32x4_d uf = u;
@@ -692,14 +697,13 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
 #pragma unroll
       for (int r = 0; r < 4; ++r) uf[r] = 4 * q + r < first ? uf[r] : 0.f;
     }
-    o *= iq;
 #pragma unroll
     for (int r = 0; r < 4; ++r) o = mfma_d(pr[r], uf[r], o);
     if constexpr (!L::kParts) {
 #pragma unroll
       for (int r = 1; r < 4; ++r)
 #pragma unroll
-        for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r] * ik[r], S[i]);
+        for (int i = 0; i < DT; ++i) S[i] = mfma_d(ke[r][i], u[r], S[i]);
     }
     if (odd) {
 #pragma unroll

@@ -279,6 +279,36 @@ def test_gated_delta_chunks_of_rows_of_any_length(D, Dv, dtype, monkeypatch):
     assert ((outs[0].double() - outs[1].double()).abs() <= bar * outs[1].double().abs() + 1e-3).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("channel", [True, False], ids=["gated", "head"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("rows,values", [(1e18, 1e21), (0.0, 1e36)])
+def test_delta_chunks_of_states_at_the_end_of_fp32(rows, values, D, channel, dtype, monkeypatch):
+    """q and k enter every product with unit length: long rows beside large states, and rows of zeros beside the largest values, leave the states
+    that the per-token kernels leave, two orders of the same fp32 sums (bar as above)"""
+    from scratchpad_amd import _native
+    announce("delta states at the end of fp32", dtype, D, channel, rows, values)
+    g = torch.Generator(device=DEV).manual_seed(21)
+    lens, H, Dv = [50, 17, 32], 2, 128
+    T, slots = sum(lens), slots_of(lens)
+    size = torch.where(torch.arange(T, device=DEV) % 3 == 1, rows, 1.0)[:, None]
+    q, k = ((torch.randn(T, H * D, generator=g, device=DEV) * size).to(dtype) for _ in range(2))
+    v, bp = (torch.randn(T, H * Dv, generator=g, device=DEV) * values).to(dtype), torch.randn(T, H, generator=g, device=DEV).to(dtype)
+    decay, gate, pre = (torch.rand(T, n, generator=g, device=DEV) for n in (H * D, H * Dv, 2 * H))
+    nw, dt_bias, A_log, states = torch.ones(Dv, device=DEV), *(torch.rand(H, generator=g, device=DEV) for _ in range(2)), []
+    seq = seq_extend(lens, [0] * len(lens), slots)
+    for chunks in (True, False):
+        monkeypatch.setattr(_native, "delta_chunks_pay", lambda *a, chunks=chunks: chunks)
+        S = torch.zeros(2 * len(lens) + 1, H, D, Dv, device=DEV)
+        if channel:
+            _native.gated_delta_scan(q, k, v, bp, decay, gate, nw, S, seq, H, H, D, Dv, 1e-5)
+        else:
+            _native.head_delta_scan(q, k, v, gate.to(dtype), pre, dt_bias, A_log, nw, S, seq, H, H, D, Dv, 1e-5)
+        states.append(S)
+    for slot in slots:
+        near(states[0][slot], states[1][slot].double(), 2e-5)
+
+
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.bfloat16, 32), (torch.float32, 64)])
 @pytest.mark.parametrize("lens", [[1, 1, 1], [70, 3]], ids=lambda l: "-".join(map(str, l)))
 def test_mlstm_gates_as_halves_of_one_product(dtype, D, lens):
