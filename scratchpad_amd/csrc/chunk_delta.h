@@ -258,13 +258,16 @@ __device__ __forceinline__ Parts parts_of(float x, float y) {
 // vector unit for its 32 cycles, so its 104 (3380 of 5800 cycles) and every address, decay and conversion of both kinds of waves add up.  Hence
 // rows by pointers that move on by a step, and masks in a request's last chunk alone.  Operands two chunks
 // ahead, helpers ahead of the products in the issue, and stores behind the loads that are waited for gave nothing: the sum stays.
-// bf16 products run beside vector work, so heads of 128 by ranges of 64 columns (kParts) take the products with S, and Ke^T U, as six products of
-// parts with 8 bits each (the three left out are below 2^-23 of the whole, of either sign): 72 instructions of 16 cycles in the place of 96 of 32, for 280
-// more of the vector unit.  The chain is then the helpers', so each takes a quarter of the tokens (K, Q and Ke as a wave each: 4900 cycles).
-// us a chunk, one request of 4096 tokens, 16 heads of 128: decay per channel 2.43 -> 1.86, per head 2.2 -> 1.66 (the layers 855 -> 708 and 823 -> 685; of
-// 8 requests 334 -> 309 and 333 -> 307).  128 columns a workgroup, which many requests take, keep fp32: the parts do not fit 168
+// bf16 products run beside vector work, so heads of 128 by ranges of 64 columns (kParts) take the products with S, and Ke^T U, as eight products of
+// parts with 8 bits each: 96 instructions of 16 cycles in the place of 96 of 32, for 280 more of the vector unit.  The one left out, of both last
+// parts, is at most 2^-32 of the whole.  (Without the two of a second and a last part as well, up to 2^-22 is left out where mantissas lie just below a
+// cut, and a sum that one channel makes up is four times as far from 64 bits as fp32's; 25 us of the layers below.)  bf16 ends at 2^-133 where fp32
+// ends at 2^-149: of states below 2^-109 the last part is cut there (300 tokens of values around 2^-120: 7e-5 of them, 1.3e-7 down to 2^-105).
+// The helpers' chain is then about as long, so each takes a quarter of the tokens (K, Q and Ke as a wave each: 4900 cycles).
+// us a chunk, one request of 4096 tokens, 16 heads of 128: decay per channel 2.44 -> 1.96, per head 2.2 -> 1.79 (the layers 855 -> 733 and 823 -> 717, 797 and
+// 767 with fp32 products; of 8 requests 334 -> 316 and 333 -> 314, 323 and 320).  128 columns a workgroup, which many requests take, keep fp32: the parts do not fit 168
 // registers (16 requests of 125 tokens 212 and 243 us), nor two workgroups a unit of heads of 64.
-// S and the read-outs are as far from 64 bits as with fp32 products.
+// S and the read-outs are otherwise no further from 64 bits than with fp32 products (S of those tokens 1.26e-7, 1.37e-7 with fp32).
 constexpr int kDcHelpers = 4;
 
 // COLS: columns of a workgroup at the most
@@ -554,7 +557,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
       if (c + 1 < chunks) fetch_v(c + 1);
     };
     if constexpr (L::kParts) {
-      // Products of parts, the small ones first (those of two last parts, or a middle and a last one, are below fp32's rounding).  The parts of
+      // Products of parts, the small ones first (those of two last parts are far below fp32's rounding).  The parts of
       // a block's state are formed between the products of the block before, whose operands are read a block ahead.
       constexpr int BLOCKS = D / 32;
       f32x4_d g[DT];
@@ -578,7 +581,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
           for (int p = 0; p < 3; ++p) sp[x & 1][p][e] = y.p[p];
         }
       };
-      constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+      constexpr int PA[8] = {2, 1, 2, 0, 1, 1, 0, 0}, PB[8] = {1, 2, 0, 2, 1, 0, 1, 0};
       read(0);
       split(0);
       __builtin_amdgcn_sched_barrier(0);
@@ -590,7 +593,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
 #pragma unroll
           for (int p = 0; p < 3; ++p) kp[i][p] = *(const u32x2*)(rows + L::kKe + (16 * i + r16) * L::kKeRow + p * 2 * kDC + 8 * q);
 #pragma unroll
-        for (int y = 0; y < 6; ++y) {
+        for (int y = 0; y < 8; ++y) {
           kd = mfma_parts(ak[x & 1][PA[y]], sp[x & 1][PB[y]], kd);
           o = mfma_parts(aq[x & 1][PA[y]], sp[x & 1][PB[y]], o);
         }
@@ -600,7 +603,7 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
 #pragma unroll
           for (int r = 0; r < 4; ++r) S[i][r] *= g[i][r];
 #pragma unroll
-        for (int y = 0; y < 12; ++y) {
+        for (int y = 0; y < 16; ++y) {
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // a read of LDS, a product, four vector instructions
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
@@ -615,16 +618,15 @@ __global__ void __launch_bounds__(COLS * 4 + kDcHelpers * 64, (DeltaScanLds<Tag,
         u = mfma_d(tr[r], v[r], u);
       }
       const Parts u0 = parts_of(u[0], u[1]), u1 = parts_of(u[2], u[3]);
-      const u32x4 ub[3] = {u32x4{u0.p[2], u1.p[2], u0.p[0], u1.p[0]}, u32x4{u0.p[1], u1.p[1], u0.p[1], u1.p[1]},
-                           u32x4{u0.p[0], u1.p[0], u0.p[0], u1.p[0]}};
-      // Ke's first part beside the last against U's last and first, then its first beside the second against U's second twice and first twice
+      const u32x4 ub[4] = {u32x4{u0.p[2], u1.p[2], u0.p[1], u1.p[1]}, u32x4{u0.p[2], u1.p[2], u0.p[0], u1.p[0]},
+                           u32x4{u0.p[1], u1.p[1], u0.p[1], u1.p[1]}, u32x4{u0.p[0], u1.p[0], u0.p[0], u1.p[0]}};
+      // Ke's parts second and last, first and last, and first and second twice, against U's last and second, last and first, second twice, first twice
+      constexpr int KA[4] = {1, 0, 0, 0}, KB[4] = {2, 2, 1, 1};
 #pragma unroll
-      for (int y = 0; y < 3; ++y)
+      for (int y = 0; y < 4; ++y)
 #pragma unroll
-        for (int i = 0; i < DT; ++i) {
-          const int p = y == 0 ? 2 : 1;
-          S[i] = mfma_parts(u32x4{kp[i][0][0], kp[i][0][1], kp[i][p][0], kp[i][p][1]}, ub[y], S[i]);
-        }
+        for (int i = 0; i < DT; ++i)
+          S[i] = mfma_parts(u32x4{kp[i][KA[y]][0], kp[i][KA[y]][1], kp[i][KB[y]][0], kp[i][KB[y]][1]}, ub[y], S[i]);
     } else {
       // Every read of LDS goes out between two products: in one piece the four waves' reads hold their products up until LDS has taken them
       // (left to itself the compiler keeps registers free and waits for each read).

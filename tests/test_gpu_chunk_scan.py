@@ -309,6 +309,59 @@ def test_delta_chunks_of_states_at_the_end_of_fp32(rows, values, D, channel, dty
         near(states[0][slot], states[1][slot].double(), 2e-5)
 
 
+def _unit_parts_just_below_a_cut(lo, factor, n, seed):
+    """n pairs (a, b) of fp32 whose unit row's a, times `factor`, lies in [lo, 1.06 lo] with mantissas that split badly into 8 + 8 + 8 bits:
+    below a cut of the first, half of one of the second left over"""
+    g, out = torch.Generator().manual_seed(seed), []
+    while len(out) < n:
+        a = lo / factor * (1 + 0.06 * torch.rand(1 << 20, generator=g))
+        b = torch.sqrt(1 - a * a)
+        x = a * (factor / torch.sqrt(a * a + b * b + 1e-6))
+        low = x.view(torch.int32) & 0xffff
+        hit = ((low >= 0xff60) & (low <= 0xff7e)).nonzero()[:, 0]
+        out += [(float(a[i]), float(b[i])) for i in hit]
+    return torch.tensor(out[:n])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_delta_products_of_one_channel_are_products_in_fp32(D, monkeypatch):
+    """Sums that one channel makes up: a product k v of the state and a product q S of the read-out, of mantissas whose parts of 8 bits leave the
+    most behind.  fp32 rounds the product (at most 2^-24 of it, 2^-24 / sqrt(3) in the mean), the read-out's norm once more for each of two columns."""
+    from scratchpad_amd import _native
+    announce("delta products of one channel", D)
+    monkeypatch.setattr(_native, "delta_chunks_pay", lambda *a: True)
+    H, Dv, T, ulp = 2, 64, 16, 2.0 ** -24
+    g = torch.Generator().manual_seed(7)
+    # columns: 1, then numbers just below a cut over some exponents and signs
+    low = 0xff60 + torch.randint(0, 0x1f, (T, Dv), generator=g)
+    bits = (torch.randint(125, 130, (T, Dv), generator=g) << 23) | (torch.randint(0, 8, (T, Dv), generator=g) << 16) | low
+    numbers = bits.int().view(torch.float32) * (1 - 2 * torch.randint(0, 2, (T, Dv), generator=g))
+    numbers[:, 0] = 1.0
+    seq = lambda held: seq_extend([T], [held], [1])  # noqa: E731
+    ones = lambda n: torch.ones(T, n, device=DEV)  # noqa: E731
+    rows = lambda pairs: torch.stack([torch.nn.functional.pad(p, (2 * t, D - 2 * t - 2)) for t, p in enumerate(pairs)]).repeat(1, H).to(DEV)  # noqa: E731
+
+    def error(got, want):
+        return float(((got / want - 1) ** 2).mean().sqrt() / ulp)
+
+    # S = k v: token t has the channels 2 t and 2 t + 1 to itself, steps of 1, no decay; the column of ones is k
+    S = torch.zeros(2, H, D, Dv, device=DEV)
+    k = rows(_unit_parts_just_below_a_cut(0.5, 1.0, T, 1))
+    v = numbers.repeat(1, H).to(DEV)
+    _native.gated_delta_scan(k, k, v, ones(H) * 100, ones(H * D), ones(H * Dv), torch.ones(Dv, device=DEV), S, seq(0), H, H, D, Dv, 1e-5)
+    got = S[1, :, 0:2 * T:2].double().cpu()                                       # [H, T, Dv]
+    assert error(got[:, :, 1:], got[:, :, :1] * numbers[:, 1:].double()) <= 1.0
+
+    # o = q S of a held state whose rows 2 t are the numbers and rows 2 t + 1 zeros; keys of zeros leave it
+    S = torch.zeros(2, H, D, Dv, device=DEV)
+    S[1, :, 0:2 * T:2] = numbers.to(DEV)
+    q = rows(_unit_parts_just_below_a_cut(2.0 ** -4, D ** -0.5, T, 2))
+    out = _native.gated_delta_scan(q, torch.zeros_like(q), torch.zeros_like(v), ones(H), ones(H * D), ones(H * Dv), torch.ones(Dv, device=DEV), S, seq(16),
+                                   H, H, D, Dv, 1e-5)
+    got = out.view(T, H, Dv).double().cpu()
+    assert error(got[:, :, 1:], got[:, :, :1] * numbers[:, None, 1:].double()) <= 1.5
+
+
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.bfloat16, 32), (torch.float32, 64)])
 @pytest.mark.parametrize("lens", [[1, 1, 1], [70, 3]], ids=lambda l: "-".join(map(str, l)))
 def test_mlstm_gates_as_halves_of_one_product(dtype, D, lens):
