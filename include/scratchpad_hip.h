@@ -62,8 +62,8 @@ SP_API const char* sp_status_string(int status);
  * tokens; the two forms agree bit for bit), "decode_ranges" (0 = decode launches never take the range geometry of
  * their plan: the (request, split) items everywhere; -1 = the default, wherever the range kernel applies),
  * "extend_small" (16-bit extend launches that leave compute units idle: 0 = the form by their size, the default; 1 = as all others;
- * 2 = as 1 where nothing else is asked for; -1 = half row blocks where that form exists; n > 2 = every row block's keys shared by n - 1 workgroups where the
- * workspace allows it), "decode_nt_min_mb" (see sp_decode_attention), "ar_fused_blocks".  Nothing on the call path reads the environment.  Returns
+ * 2 = half row blocks where that form exists; n > 2 = every row block's keys shared by n - 1 workgroups where the
+ * workspace allows it, else as 2), "decode_nt_min_mb" (see sp_decode_attention), "ar_fused_blocks".  Nothing on the call path reads the environment.  Returns
  * SP_ERR_INVALID_ARG for an unknown key.                                                          */
 SP_API int sp_debug_set(const char* key, int value);
 /* Read-only counterpart (ABI 6): "w64_descriptor_patched" (1 = extend_w64.hip was built in stages with its kernels'

@@ -870,8 +870,7 @@ size_t extend_split_bytes(int64_t num_tokens, int num_q_heads, int head_dim) {
 // (Beside the other wave's vector work a wave's products gain nothing: the second four waves half a tile behind the first, 37.1 -> 40.2.)
 // What the 4 x 64-row kernel applies to stays whole: its forms and this file's agree to the bit, whichever of them a size selects.
 // With more than half of the units busy the same forms lose: 4 requests, 2048 tokens behind 1500, heads of 64: 45 | 46; 4096 tokens: 90 | 102.
-static void extend_small_form(ExtendArgs& a, int head_dim, int max_extend_len, int64_t max_seq_len, void* workspace,
-                              size_t workspace_bytes) {
+static void extend_small_form(ExtendArgs& a, int head_dim, int64_t max_seq_len, void* workspace, size_t workspace_bytes) {
   a.splits = 1;
   a.half_blocks = 0;
   const int G = a.Hq / a.Hkv, gk = extend_gk(G), gx = a.Hkv * (G / gk), rows = 32 * (kExtendWaves / gk);
@@ -886,13 +885,13 @@ static void extend_small_form(ExtendArgs& a, int head_dim, int max_extend_len, i
   s = std::min(s, fit);
   const int64_t tiles = max_seq_len / 64, alone = head_dim == 64 ? 600 : 1350, shared = head_dim == 64 ? 1050 : 1150;
   if (tiles < 2 && !g_extend_small) return;
-  if (s > 1 && g_extend_small >= 0 && (g_extend_small > 2 || tiles * (alone - shared / s) > 5000 + (head_dim == 64 ? 20 : 40) * groups * s)) {
+  if (s > 1 && (g_extend_small > 2 || tiles * (alone - shared / s) > 5000 + (head_dim == 64 ? 20 : 40) * groups * s)) {
     a.splits = (int)s;
     a.plan_items = (int)items;
     a.part_o = (float*)workspace;
     a.part_ml = a.part_o + groups * kExtendWaves * s * 32 * head_dim;
-  } else if (head_dim == 64 && a.bs < 32768 && g_extend_small != 2 && fit > 0) {
-    a.half_blocks = 1;      // (a workspace without room for shares asks for the general form's order of the sums)
+  } else if (head_dim == 64 && a.bs < 32768) {
+    a.half_blocks = 1;      // (whatever room the workspace has: it takes none of it)
   }
 }
 
@@ -1019,7 +1018,7 @@ int run_extend_mfma(void* out, const void* q, const void* k_buffer, const void* 
   a.plan_items = plan_items;
   if (plan && (plan_items <= 0 || plan_items > 65535)) a.plan = nullptr;   // grid.y limit: unplanned launch
   a.part_o = a.part_ml = nullptr;
-  extend_small_form(a, head_dim, max_extend_len, max_seq_len, workspace, workspace_bytes);
+  extend_small_form(a, head_dim, max_seq_len, workspace, workspace_bytes);
   const int G = num_q_heads / num_kv_heads;
   if (max_extend_len <= 0) return SP_OK;
   if (const int form = a.splits > 1 ? 0 : try_extend_w64(a, head_dim, dtype, max_extend_len, max_seq_len, st)) {
