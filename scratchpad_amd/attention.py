@@ -16,6 +16,7 @@ import torch
 from torch import nn
 
 from . import _native
+from .pool import MHATokenToKVPool
 
 if TYPE_CHECKING:
     from .forward_info import ForwardBatch, ForwardMode
@@ -99,6 +100,10 @@ class RadixAttention(nn.Module):
         return forward_batch.attn_backend.forward(q, k, v, self, forward_batch, save_kv_cache)
 
 
+def _plain_store(pool) -> bool:
+    return getattr(getattr(pool, "set_kv_buffer", None), "__func__", None) is MHATokenToKVPool.set_kv_buffer
+
+
 def _pow2_floor(x: int) -> int:
     return 1 << (max(int(x), 1).bit_length() - 1)
 
@@ -168,6 +173,8 @@ class HipAttnBackend(AttentionBackend):
                             and dtype in (torch.float16, torch.bfloat16) and self.kv_dtype in (dtype, torch.float8_e5m2)
                             and self.head_dim in (64, 128) and self.v_head_dim == self.head_dim
                             and self.num_head % self.num_kv_head == 0 and self.num_head // self.num_kv_head <= 8
+                            # (a byte pool stores through its method, which a small step does not call)
+                            and (self.kv_dtype == dtype or _plain_store(model_runner.token_to_kv_pool))
                             and all(m.follows_rotation and not m.logit_cap > 0 and m.sliding_window_size == -1 and not m.is_cross_attention
                                     for m in layers))
 
@@ -183,7 +190,13 @@ class HipAttnBackend(AttentionBackend):
     small_steps = False            # this model has such steps
     small_step = False             # the step that forward_metadata is of is one
 
+    # what a small step does not call: a backend with an own form of one of them has no such steps
+    PASSED_BY = ("init_forward_metadata", "init_forward_metadata_capture_cuda_graph", "init_forward_metadata_replay_cuda_graph",
+                 "forward", "forward_decode", "rotary_and_store")
+
     def _few_keys(self, bs: int, seq_lens_sum: int) -> bool:
+        if not all(getattr(getattr(self, n), "__func__", None) is getattr(HipAttnBackend, n) for n in self.PASSED_BY):
+            return False
         one = 1024 if self.head_dim == 64 and self.kv_dtype != torch.float8_e5m2 else 512
         return self.small_steps and not self.plan_items and bs <= self.SMALL_MAX_ROWS and seq_lens_sum <= min(one + (bs - 1) * one // 8, 2 * one)
 

@@ -613,6 +613,27 @@ def test_decode_split_size_policy_and_where_items_are_planned():
     assert b._ranges_for(256, 2 ** 24) == 0 and b._graph_slots(256) > 0
 
 
+def test_small_steps_pass_by_no_backend_of_its_own():
+    """a small step runs neither the backend's decode methods nor, over a byte pool, the pool's store: where one of them is another's, there is none"""
+    from scratchpad_amd.attention import HipAttnBackend, _plain_store
+    from scratchpad_amd.pool import MHATokenToKVPool
+
+    def few(cls, **own):
+        b = cls.__new__(cls)
+        b.head_dim, b.kv_dtype, b.small_steps, b.plan_items = 64, torch.bfloat16, True, False
+        b.__dict__.update(own)
+        return b._few_keys(1, 300)
+    assert few(HipAttnBackend) and few(type("Same", (HipAttnBackend,), {"forward_extend": lambda *a, **k: None}))
+    for name in ("forward", "forward_decode", "rotary_and_store", "init_forward_metadata", "init_forward_metadata_replay_cuda_graph"):
+        assert not few(type("Own", (HipAttnBackend,), {name: lambda *a, **k: None})), name
+        assert not few(HipAttnBackend, **{name: lambda *a, **k: None}), name
+    pool = MHATokenToKVPool.__new__(MHATokenToKVPool)
+    own = type("Own", (MHATokenToKVPool,), {"set_kv_buffer": lambda *a: None})
+    assert _plain_store(pool) and not _plain_store(own.__new__(own))
+    pool.set_kv_buffer = lambda *a: None
+    assert not _plain_store(pool)
+
+
 def test_plan_registry_trusts_only_live_plan_buffers():
     """_native remembers what each decode plan buffer was built with (data_ptr -> (bs, max_slots, ranges)) so that a launch
     given other values raises on the host (ABI 9).  A view of the buffer is the same plan; an entry whose tensor has died is
