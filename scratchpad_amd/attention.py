@@ -182,10 +182,9 @@ class HipAttnBackend(AttentionBackend):
     # One launch per layer for a small step: rows, and keys of all requests together - a workgroup walks a request's keys
     # alone, and the host knows their sum.  us per layer, three launches / one, by keys of the one request: heads of 64 300
     # 10.2 / 5.9, 600 10.4 / 8.5, 1200 11.4 / 10.9, 2400 13.2 / 16.3; of 128 300 12.2 / 7.9, 600 12.3 / 11.4, 1200 13.9 / 16.5.  More
-    # requests share the sum: 8 of 300 12.0 / 7.7 and 13.9 / 10.0, 32 of 64 11.7 / 5.6 and 14.5 / 7.0; what they lose where one of them has
-    # nearly all keys bounds the sum at twice the one request's.  Four rows: more of them would gain too, but each bucket's second form takes 3.4 ms and
-    # a graph's memory at a server's start, and steps of 8 and 16 rows add their sums in another order than the results that they are compared with
-    # (rms of logits against fp32 1.000 of torch's own 16-bit evaluation here, 1.003 in three launches; the largest of 500 000 is either's).
+    # requests share the sum, an eighth of the one's for each: all but a few of the keys may still be one request's.
+    # Four rows: not where the one launch stops being faster (8 requests of 300 keys 12.0 / 7.7 and 13.9 / 10.0, 32 of 64 11.7 / 5.6 and
+    # 14.5 / 7.0), but what a server's start is given to it - a bucket's second form takes 4 ms for 16 layers (its first 6), and a graph's memory.
     SMALL_MAX_ROWS = 4
     small_steps = False            # this model has such steps
     small_step = False             # the step that forward_metadata is of is one
@@ -198,7 +197,7 @@ class HipAttnBackend(AttentionBackend):
         if not all(getattr(getattr(self, n), "__func__", None) is getattr(HipAttnBackend, n) for n in self.PASSED_BY):
             return False
         one = 1024 if self.head_dim == 64 and self.kv_dtype != torch.float8_e5m2 else 512
-        return self.small_steps and not self.plan_items and bs <= self.SMALL_MAX_ROWS and seq_lens_sum <= min(one + (bs - 1) * one // 8, 2 * one)
+        return self.small_steps and not self.plan_items and bs <= self.SMALL_MAX_ROWS and seq_lens_sum <= one + (bs - 1) * one // 8
 
     def _head_groups(self, dtype: torch.dtype) -> int:
         vec = 4 if dtype == torch.float32 else 8
