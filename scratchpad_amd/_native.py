@@ -1800,11 +1800,20 @@ SMALL_LINEAR_OWN_ROWS = 64      # up to this many rows a workgroup per row; abov
 
 
 def small_linear_tiles_pay(T: int, K: int, n: int) -> bool:
-    """Where the tiles for more than 64 bf16 rows take the product, else a copy of x to fp32 and the library's.  The line is where the
-    tiles crossed the library when their operands came straight to registers; through LDS they are faster on both sides of it (us,
-    tiles / library: K 2048, 4096 rows of 64 outputs 8.8 / 27.8, of 256 29.2 / 48.3; 8192 of 128 33.9 / 53.9; 256 of 1024 9.5 / 17.0; past
-    the line 65 rows of K 4096 8.0 / 13.2, 512 of K 8192 12.9 / 27.7, 4096 of 512 outputs 56.0 / 74.0, 8192 of 256 59.2 / 83.1)."""
-    return (K <= 2048 or 8 * T >= K) and (n <= 128 or (n <= 256 and T * K <= 1 << 23) or (K <= 2048 and T * n <= 1 << 18))
+    """Where the tiles for more than 64 bf16 rows are faster than a copy of x to fp32 and the library's product.  They save the copy and a launch,
+    and read x once per 16 outputs, exactly split on the way: the library's larger tiles win with outputs times rows.  Of 1690 sizes (T 65 - 40 000, K 64 -
+    16 384, n 4 - 4096) the tiles are faster at 1490; the line gives them 1320, one of them at 0.9 of the library's speed, and 2.4 times its speed in the mean.
+    us, tiles / library, on this side: K 2048, 4096 rows of 64 outputs 7.9 / 27.6, of 512 50 / 76, 8192 of 256 52 / 85, 256 of 2048 16.3 / 24.8; K 4096,
+    65 rows of 64 6.7 / 12.5, of 4096 25 / 37; K 8192, 512 rows of 64 10.8 / 27.5.  Beyond it: K 64, 16 384 rows of 256 28 / 15; K 256,
+    32 768 of 512 116 / 88; K 4096, 8192 of 512 292 / 268, 777 of 2048 137 / 119; K 16 384, 16 384 of 100 820 / 723.  (Some sizes beyond it would
+    gain too, 1.2 - 1.6 times, beside others of the same T n that lose: the library's choice of tile changes there.)"""
+    if n <= 32:
+        return True
+    if K <= 2048:
+        return T * n <= 1 << (22 if K >= 1024 or (K >= 128 and n <= 128) else 20 if K >= 128 or n <= 64 else 19)
+    if n <= 128:
+        return T * n * K <= 1 << 34
+    return T * n <= 1 << (20 if n <= 512 else 19)
 
 
 def _small_linear_tiles_take(x: torch.Tensor, weight: torch.Tensor) -> bool:

@@ -186,7 +186,8 @@ def test_fp32_products_of_many_rows(T, K, n, bias):
     assert out.shape == (T, n) and bool(((out.double() - want).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("T,K,n", [(2100, 1056, 64), (4097, 96, 17), (8193, 64, 16)])       # tiles of 64 rows, the last of few; of 32 rows again
+# tiles of 64 rows, the last of few; of 32 rows again; few rows of a long K and of many outputs
+@pytest.mark.parametrize("T,K,n", [(2100, 1056, 64), (4097, 96, 17), (8193, 64, 16), (100, 16384, 40), (71, 4096, 2050)])
 def test_fp32_products_of_more_rows(T, K, n):
     from scratchpad_amd import _native
     g = torch.Generator(device=DEV).manual_seed(T + K + n)

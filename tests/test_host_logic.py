@@ -252,14 +252,15 @@ def test_delta_chunk_dispatch_rule():
 
 
 def test_fp32_product_dispatch_rule():
-    """the tiles for many bf16 rows where they measured faster than the library, the library elsewhere"""
+    """the tiles for many bf16 rows where they measured faster than the library, the library where it did"""
     from scratchpad_amd import _native
     pays = _native.small_linear_tiles_pay
     assert pays(65, 2048, 32) and pays(16384, 2048, 64) and pays(8192, 2048, 128) and pays(4096, 2048, 256) and pays(256, 2048, 1024)
     assert pays(512, 4096, 64) and pays(2048, 4096, 256) and pays(1024, 8192, 64)
-    assert not pays(65, 4096, 64) and not pays(256, 4096, 16) and not pays(512, 8192, 64)             # a long chain, few rows
-    assert not pays(8192, 2048, 256) and not pays(4096, 2048, 512) and not pays(4096, 4096, 256)      # many outputs of many rows
-    assert not pays(256, 2048, 2048) and not pays(65, 4096, 2048)
+    assert pays(65, 4096, 64) and pays(256, 4096, 16) and pays(512, 8192, 64) and pays(65, 4096, 2048)       # a long chain, few rows
+    assert pays(8192, 2048, 256) and pays(4096, 2048, 512) and pays(4096, 4096, 256) and pays(256, 2048, 2048)
+    assert not pays(16384, 64, 256) and not pays(32768, 64, 64) and not pays(32768, 256, 512)                # many outputs of many rows, short and
+    assert not pays(8192, 4096, 512) and not pays(777, 4096, 2048) and not pays(16384, 16384, 100)           # long
 
 
 def test_fp32_products_of_far_apart_rows_leave_the_tiles():
