@@ -111,3 +111,66 @@ def test_small_steps_of_a_model(graph, monkeypatch):
     for x in (got, want_hook):
         # two orders of the same sums: a few roundings of 2^-9 through two layers
         assert float((x - want).norm() / want.norm()) < 0.01
+
+
+# lengths of three requests, and whether the step is small, eagerly and replayed in the bucket of four (whose padded row holds one key): at the bounds
+# 1280 and 1408 of heads of 64, past them, and back
+WALK = [((400, 430, 450), True, True), ((401, 431, 451), False, True), ((440, 480, 487), False, True), ((441, 481, 488), False, False),
+        ((5, 17, 9), True, True), ((700, 600, 600), False, False), ((6, 18, 10), True, True)]
+
+
+@pytest.mark.parametrize("hooked", [None, 0, 1])
+@pytest.mark.parametrize("graph", [None, [2, 4]])
+def test_steps_cross_the_bound_of_keys(graph, hooked, monkeypatch):
+    """a model's steps go from one form to the other and back as its requests grow, are served and start anew: which form ran, and that every
+    step's logits are the general form's.  With a hook on a layer (there before the graphs are captured) that layer is called by itself: its
+    plan is built once a step, under capture as a launch of the graph."""
+    from scratchpad_amd import attention
+    from scratchpad_amd.forward_info import ForwardMode, ModelWorkerBatch
+    from scratchpad_amd.model_runner import ModelConfig, ModelRunner, ServerArgs, TpModelWorker
+
+    def walk(hooked):
+        cfg = ModelConfig(256, 512, 2, 4, 2, 640, context_len=800)
+        mr = ModelRunner(cfg, ServerArgs(max_total_tokens=2500, max_running_requests=3, disable_cuda_graph=graph is None, cuda_graph_bs=graph),
+                         dtype=torch.bfloat16, seed=3, init_weights=True)
+        forms, calls, out = [], [], []
+        if hooked is not None:
+            mr.model.model.layers[hooked].self_attn.attn.register_forward_hook(lambda *_: calls.append(1))
+        if graph:
+            mr.init_cuda_graphs()
+
+            class Noted:
+                def __init__(self, graph, small):
+                    self.graph, self.small = graph, small
+
+                def replay(self):
+                    forms.append(self.small)
+                    self.graph.replay()
+            runner = mr.graph_runner
+            runner.graphs = {b: Noted(g, False) for b, g in runner.graphs.items()}
+            runner.small_graphs = {b: (Noted(g, True), o) for b, (g, o) in runner.small_graphs.items()}
+        gen = torch.Generator(device=mr.device).manual_seed(5)
+        for layer in range(2):
+            for buf in mr.token_to_kv_pool.get_kv_buffer(layer):
+                buf.copy_(torch.randn(buf.shape, generator=gen, device=mr.device).to(buf.dtype))
+        req = torch.arange(1, 4, device=mr.device)
+        for i, row in enumerate(req.tolist()):
+            mr.req_to_token_pool.req_to_token[row, :800] = torch.arange(1 + 800 * i, 801 + 800 * i, device=mr.device, dtype=torch.int32)
+        worker = TpModelWorker(mr)
+        for s, (lens, *_) in enumerate(WALK):
+            seq = torch.tensor(lens, device=mr.device)
+            batch = ModelWorkerBatch(bid=s, forward_mode=ForwardMode.DECODE, input_ids=torch.arange(3, 6, device=mr.device) + s, req_pool_indices=req,
+                                     seq_lens=seq, out_cache_loc=mr.req_to_token_pool.req_to_token[req, seq - 1].long(), seq_lens_sum=sum(lens))
+            out.append(worker.forward_batch_generation(batch)[0].next_token_logits.float().cpu())
+            if not graph:
+                forms.append(mr.attn_backend.small_step)
+        return out, forms, calls
+
+    got, forms, calls = walk(hooked)
+    assert forms == [w[2 if graph else 1] for w in WALK] and (hooked is None) == (not calls)
+    monkeypatch.setattr(attention.HipAttnBackend, "SMALL_MAX_ROWS", 0)
+    want, general, _ = walk(None)
+    assert not any(general)
+    for s, (x, y) in enumerate(zip(got, want)):
+        # two orders of the same sums: a few roundings of 2^-9 through two layers
+        assert float((x - y).norm() / y.norm()) < 0.01, f"step {s}, {WALK[s]}"
