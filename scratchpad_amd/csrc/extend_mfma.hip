@@ -897,11 +897,13 @@ static void extend_small_form(ExtendArgs& a, int head_dim, int64_t max_seq_len, 
 
 #define SP_EXT_SET_LDS(KERNEL, BYTES)                                                                              \
   do {                                                                                                           \
-    static bool attr_set = false; /* benign race: idempotent */                                                  \
-    if (!attr_set && (BYTES) > 64 * 1024) {                                                                      \
-      (void)hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);         \
-      attr_set = true;                                                                                           \
-    }                                                                                                            \
+    static PerDevice<int> raised;                                                                                \
+    int ok = 1;                                                                                                  \
+    if ((BYTES) > 64 * 1024)                                                                                     \
+      raised.get(ok, [&](int) {                                                                                  \
+        return hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, BYTES) == hipSuccess ? 1 : 0; \
+      });                                                                                                        \
+    if (!ok) return SP_ERR_LAUNCH;                                                                               \
   } while (0)
 
 template <typename Tag, int D, int GK>
