@@ -181,10 +181,10 @@ class HipAttnBackend(AttentionBackend):
     # ---------------------------------------------------------------- launch planning
     # One launch per layer for a small step: rows, and keys of all requests together - a workgroup walks a request's keys
     # alone, and the host knows their sum.  us per layer, three launches / one, by keys of the one request: heads of 64 300
-    # 10.2 / 5.9, 600 10.4 / 8.5, 1200 11.4 / 10.9, 2400 13.2 / 16.3; of 128 300 12.2 / 7.9, 600 12.3 / 11.4, 1200 13.9 / 16.5.  More
+    # 10.2 / 6.2, 600 10.4 / 9.0, 1200 11.4 / 11.8, 2400 13.2 / 17.8; of 128 300 12.2 / 8.3, 600 12.3 / 11.9, 1200 13.9 / 17.6.  More
     # requests share the sum, an eighth of the one's for each: all but a few of the keys may still be one request's.
-    # Four rows: not where the one launch stops being faster (8 requests of 300 keys 12.0 / 7.7 and 13.9 / 10.0, 32 of 64 11.7 / 5.6 and
-    # 14.5 / 7.0), but what a server's start is given to it - a bucket's second form takes 4 ms for 16 layers (its first 6), and a graph's memory.
+    # Four rows: not where the one launch stops being faster (8 requests of 300 keys 12.0 / 8.0 and 13.9 / 10.4, 32 of 64 11.7 / 5.8 and
+    # 14.5 / 7.1), but what a server's start is given to it - a bucket's second form takes 4 ms for 16 layers (its first 6), and a graph's memory.
     SMALL_MAX_ROWS = 4
     small_steps = False            # this model has such steps
     small_step = False             # the step that forward_metadata is of is one

@@ -9,8 +9,8 @@
 // of 64, 32 at 128) while q is rotated; the sums of the eight waves meet in LDS.  A workgroup has a request's keys of one kv head to itself, so nothing
 // is left to merge - and long requests are slower than where many share them (SMALL_MAX_ROWS' line in attention.py has both sides).
 // us under graph replay, rotation + attention + merge -> this, bf16, 32 query and 8 kv heads: heads of 64, 1 request of 64 / 300 / 600 keys 8.7 ->
-// 4.6, 10.2 -> 5.9, 10.4 -> 8.5; 8 of 300 12.0 -> 7.7; heads of 128, 1 of 300 12.2 -> 7.9; byte pools 12.8 -> 9.4 and 14.5 -> 12.9.  A decode step of 1
-// row (16 layers, hidden 2048): 846 -> 759.
+// 4.6, 10.2 -> 6.2, 10.4 -> 9.0; heads of 128, 1 of 300 12.2 -> 8.3; byte pools 12.8 -> 9.2 and 14.5 -> 12.0.  A decode step of 1
+// row (16 layers, hidden 2048): 843 -> 763.
 #include "sp_common.h"
 
 #include <type_traits>
@@ -120,6 +120,10 @@ __global__ __launch_bounds__(kSmallWaves * 64, 2) void decode_small_kernel(Small
   typedef typename std::conditional<KV8, u32x2, u32x4>::type raw_t;       // 8 elements of the pool
   constexpr int S = D / 32, CPR = D / 8, RPL = 64 / CPR, NV = 16 / RPL, DB = D / 16, EB = KV8 ? 1 : 2, ROW = D * 2;
   constexpr int T = kSmallTiles<D>, kKeys = kSmallWaves * T * 16;         // keys of a pass
+  // The weights of a tile of 16 keys are rounded against the tile's own largest, which is 1 then and exact, and its sums join the others' in fp32: with
+  // one reference for all tiles of a wave a request of 600 - 1000 keys came out 1.01 - 1.03 times as far from 64 bits as in sp_decode_attention, whose
+  // pieces are that short; now 0.96 - 0.98, for 0.3 - 0.8 us.  bf16 queries of a byte pool: their weights are fp16, far below what the output rounds.
+  constexpr bool OWN_TOP = std::is_same<CT, Tag>::value;
   __shared__ __attribute__((aligned(16))) char tiles[kSmallWaves][16 * ROW];
   __shared__ float ml[kSmallWaves][8][2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, col = lane & 15, kq = lane >> 4;
@@ -234,24 +238,33 @@ __global__ __launch_bounds__(kSmallWaves * 64, 2) void decode_small_kernel(Small
     }
     const bool more = base + kKeys < seq;
     if (more) gather_k(next);
-    float top = m;
+    float top = m, tops[T], part[T];
 #pragma unroll
-    for (int t = 0; t < T; ++t)
+    for (int t = 0; t < T; ++t) {
+      tops[t] = kNegBigS;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         x[t][j] = base + t * kSmallWaves * 16 + 4 * kq + j < seq ? x[t][j] * a.qk_scale : -INFINITY;
-        top = fmaxf(top, x[t][j]);
+        tops[t] = fmaxf(tops[t], x[t][j]);
       }
-    top = max_quarters(top);
+      if constexpr (OWN_TOP) tops[t] = max_quarters(tops[t]);
+      top = fmaxf(top, tops[t]);
+    }
+    if constexpr (!OWN_TOP) top = max_quarters(top);
     const float keep = __builtin_amdgcn_exp2f(m - top);
     float sum = 0.f;
 #pragma unroll
-    for (int t = 0; t < T; ++t)
+    for (int t = 0; t < T; ++t) {
+      if constexpr (!OWN_TOP) tops[t] = top;
+      part[t] = OWN_TOP ? __builtin_amdgcn_exp2f(tops[t] - top) : 1.f;
+      float of = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        x[t][j] = Elem<CT>::round(__builtin_amdgcn_exp2f(x[t][j] - top));      // (as the products take it: the weights sum to one)
-        sum += x[t][j];
+        x[t][j] = Elem<CT>::round(__builtin_amdgcn_exp2f(x[t][j] - tops[t]));      // (as the products take it: the weights sum to one)
+        of += x[t][j];
       }
+      sum = __builtin_fmaf(of, part[t], sum);
+    }
     l = __builtin_fmaf(l, keep, sum_quarters(sum));
     m = top;
 #pragma unroll
@@ -278,7 +291,13 @@ __global__ __launch_bounds__(kSmallWaves * 64, 2) void decode_small_kernel(Small
         const int cg = 2 * d + ((col & 3) >> 1);
         const char* const p = tile + tr * ROW + ((cg ^ (tr & (CPR - 1))) * 16) + 8 * (col & 1);
         const u32x2 vf = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_s*)p));
-        o[d] = dot16<CT>(vf, pf, o[d]);
+        if constexpr (OWN_TOP) {
+          const f32x4_s c = dot16<CT>(vf, pf, f32x4_s{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[d][r] = __builtin_fmaf(c[r], part[t], o[d][r]);
+        } else {
+          o[d] = dot16<CT>(vf, pf, o[d]);
+        }
       }
     }
     if (more) gather_v(next);
