@@ -184,7 +184,7 @@ class HipAttnBackend(AttentionBackend):
     # 10.2 / 6.2, 600 10.4 / 9.0, 1200 11.4 / 11.8, 2400 13.2 / 17.8; of 128 300 12.2 / 8.3, 600 12.3 / 11.9, 1200 13.9 / 17.6.  More
     # requests share the sum, an eighth of the one's for each: all but a few of the keys may still be one request's.
     # Four rows: not where the one launch stops being faster (8 requests of 300 keys 12.0 / 8.0 and 13.9 / 10.4, 32 of 64 11.7 / 5.8 and
-    # 14.5 / 7.1), but what a server's start is given to it - a bucket's second form takes 4 ms for 16 layers (its first 6), and a graph's memory.
+    # 14.5 / 7.1), but what a server's start is given to it - a bucket's second form takes 2 ms for 16 layers (its first 6), and a graph's memory.
     SMALL_MAX_ROWS = 4
     small_steps = False            # this model has such steps
     small_step = False             # the step that forward_metadata is of is one
@@ -444,6 +444,14 @@ class HipAttnBackend(AttentionBackend):
         """in the place of init_forward_metadata_capture_cuda_graph"""
         self.forward_metadata = (self.MIN_CHUNK, self.cuda_graph_max_seq_len, self._graph_ws, None)
         self.small_step = True
+
+    def warm_small_step(self, model_runner) -> None:
+        """the one launch, once, over the dummy slot: before a first capture of it, where everything else of a step has run"""
+        pool = model_runner.token_to_kv_pool
+        zeros = lambda *shape, dtype=torch.int64: torch.zeros(shape, dtype=dtype, device=self.device)  # noqa: E731
+        q, kv = zeros(1, self.num_head * self.head_dim, dtype=model_runner.dtype), zeros(1, self.num_kv_head * self.head_dim, dtype=model_runner.dtype)
+        _native.decode_small(torch.empty_like(q), q, kv, kv, zeros(1), zeros(1, self.head_dim, dtype=q.dtype), zeros(1), *pool.get_kv_buffer(0),
+                             model_runner.req_to_token_pool.req_to_token, zeros(1), zeros(1) + 1, 1.0, 1)
 
     def replays_small_step(self, bs: int, seq_lens_sum: int) -> bool:
         return self._few_keys(bs, seq_lens_sum)

@@ -401,8 +401,11 @@ class HipGraphRunner:
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
-            for _ in range(1 if small_step else 2):        # (the bucket's general form has warmed up everything but the one launch)
-                run_once()
+            if small_step:          # (the bucket's general form has warmed up everything but the one launch)
+                mr.attn_backend.warm_small_step(mr)
+            else:
+                for _ in range(2):
+                    run_once()
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
