@@ -194,10 +194,9 @@ class HipAttnBackend(AttentionBackend):
                  "forward", "forward_decode", "rotary_and_store")
 
     def _few_keys(self, bs: int, seq_lens_sum: int) -> bool:
-        if not all(getattr(getattr(self, n), "__func__", None) is getattr(HipAttnBackend, n) for n in self.PASSED_BY):
-            return False
         one = 1024 if self.head_dim == 64 and self.kv_dtype != torch.float8_e5m2 else 512
-        return self.small_steps and not self.plan_items and bs <= self.SMALL_MAX_ROWS and seq_lens_sum <= one + (bs - 1) * one // 8
+        return (self.small_steps and not self.plan_items and bs <= self.SMALL_MAX_ROWS and seq_lens_sum <= one + (bs - 1) * one // 8
+                and all(getattr(getattr(self, n), "__func__", None) is getattr(HipAttnBackend, n) for n in self.PASSED_BY))
 
     def _head_groups(self, dtype: torch.dtype) -> int:
         vec = 4 if dtype == torch.float32 else 8
